@@ -1,0 +1,989 @@
+"""The work whose speed counts here, as cases that can be timed and checked.
+
+A case is one call (or a short run of calls) of the framework's public entry
+points with inputs as its users have them:
+
+  train       one micro-step of a LoRA update: forward, token log-probabilities,
+              backward, AdamW (models, ops.token_logprob_entropy, ops.FusedAdamW)
+  score       log-probabilities of given responses under a frozen policy, or the
+              reward model's scores of whole sequences
+  attention   ops.flash_attn_varlen over packed sequences, with its backward
+  decode      ops.paged_attn_decode, one new token of every sequence
+  sample      ops.sample_tokens from a batch of logits
+  generate    SamplerEngine.generate: prompts in, sampled tokens out
+  prompt      SamplerEngine.step over prompts, in one or several portions
+  experts     ops.moe_route and ops.moe_experts
+  latent      ops.latent_attn, one new token of every sequence
+
+Whole models run at the presets' widths with a few layers; the vocabulary is cut
+with the depth, so that the head keeps its share of the work.  Weights are
+random.  exact() is plain torch in 64 bits."""
+import math
+import random
+
+import torch
+
+from nanorlhf_amd import ops
+from nanorlhf_amd.models import CausalLM, ScalarHeadModel, build_model, get_config
+from nanorlhf_amd.models.config import _bedalorn_layers, _gonurax_layers
+from nanorlhf_amd.models.bedalorn import BedalornConfig
+from nanorlhf_amd.models.gonurax import GonuraxConfig
+from nanorlhf_amd.models.lora import LoraConfig, apply_lora
+from nanorlhf_amd.models.qwen2 import AttnContext, pack_sequences
+from nanorlhf_amd.sampler import SamplerEngine, SamplingParams, SeqState
+
+#            width   ff   heads  kv  head width
+SHAPES = {
+    "0.5b": (896, 4864, 14, 2, 64),
+    "1.5b": (1536, 8960, 12, 2, 128),
+    "7b": (3584, 18944, 28, 4, 128),
+}
+#          query heads, kv heads, head width, causal: the presets' attention
+HEADS = {"0.5b": (14, 2, 64, True), "1.5b": (12, 2, 128, True), "7b": (28, 4, 128, True),
+         "reward": (16, 16, 64, False)}
+#           width, expert width: a quarter of the dense feed-forward each
+EXPERTS = {"1.5b": (1536, 2240), "3b": (2048, 2752), "8b": (4096, 3584)}
+N_EXPERTS, TOP = 16, 4
+PAGE = 16
+LAYERS = 6                                   # of served models, as the serving benchmark has
+VOCABS = (32768, 128100, 151936, 152064)     # the serving benchmark's and the presets'
+
+
+def listed():
+    return [
+        # four short rows of the small policy: what a first try or a unit of a sparse batch costs
+        dict(name="train_short", kind="train", shape="0.5b", layers=3, vocab=8192, rows=4, mean=60),
+        # a full micro-batch of the default update (its token budget is 49152)
+        dict(name="train_bucket", kind="train", shape="1.5b", layers=3, vocab=16384, rows=56,
+             mean=870),
+        # the reward model over a bucket of finished episodes
+        dict(name="score_reward", kind="score", model="reward", layers=6, vocab=32768, rows=80,
+             mean=800),
+        # long reasoning responses (up to 8000 tokens): attention of the update
+        dict(name="attention_long", kind="attention", shape="1.5b", rows=5, mean=6500,
+             backward=True),
+        # decoding in the middle of a rollout, cache in 8 bits
+        dict(name="decode_rollout", kind="decode", shape="1.5b", rows=2048, mean=850, cache="fp8"),
+        # decoding for a few users
+        dict(name="decode_serving", kind="decode", shape="1.5b", rows=32, mean=2000, cache="bf16"),
+        # sampling for a few users
+        dict(name="sample_serving", kind="sample", rows=8, vocab=151936, temperature=0.7,
+             top_p=0.95, dtype="bf16"),
+        # a small rollout, four samples of each prompt
+        dict(name="generate_rollout", kind="generate", shape="1.5b", layers=LAYERS, prompts=16,
+             samples=4, mean=120, tokens=96, cache="fp8"),
+        # a batch of prompts of the two served designs; one long prompt in portions
+        dict(name="prompts_gonurax", kind="prompt", model="gonurax", rows=8, mean=2040, steps=1),
+        dict(name="prompt_bedalorn", kind="prompt", model="bedalorn", rows=1, mean=12000, steps=3),
+        # the experts of a decode step
+        dict(name="experts_decode", kind="experts", size="1.5b", rows=32),
+        # latent attention of a decode step
+        dict(name="latent_decode", kind="latent", rows=128, mean=2000, rank=512),
+    ]
+
+
+def _log(rng, a, b):
+    return min(b, max(a, int(round(math.exp(rng.uniform(math.log(a), math.log(b)))))))
+
+
+def draw(rng):
+    kind = rng.choice(["train", "score", "attention", "decode", "sample", "generate", "prompt",
+                       "experts", "latent"])
+    c = dict(kind=kind)
+    if kind == "train":
+        c.update(shape=rng.choice(["0.5b", "1.5b"]), layers=rng.randint(1, 3),
+                 vocab=rng.choice([8192, 16384]), rows=_log(rng, 1, 64), mean=_log(rng, 40, 1500))
+        c["rows"] = max(1, min(c["rows"], 48000 // c["mean"]))
+    elif kind == "score":
+        c.update(model=rng.choice(["0.5b", "1.5b", "reward"]), layers=rng.randint(1, 6),
+                 vocab=rng.choice([16384, 32768]), rows=_log(rng, 1, 96), mean=_log(rng, 40, 1500))
+        c["rows"] = max(1, min(c["rows"], 62000 // c["mean"]))
+    elif kind == "attention":
+        c.update(shape=rng.choice(sorted(HEADS)), rows=_log(rng, 1, 64), mean=_log(rng, 30, 6500),
+                 backward=rng.random() < 0.7)
+        c["rows"] = max(1, min(c["rows"], (8000 if c["shape"] == "7b" else 24000) // c["mean"]))
+    elif kind == "decode":
+        c.update(shape=rng.choice(sorted(SHAPES)), rows=_log(rng, 1, 2048),
+                 mean=_log(rng, 40, 8000), cache=rng.choice(["fp8", "bf16"]))
+        c["rows"] = max(1, min(c["rows"], 400000 // c["mean"]))
+    elif kind == "sample":
+        c.update(rows=_log(rng, 1, 2048), vocab=rng.choice(VOCABS),
+                 temperature=rng.choice([0.0, 0.7, 1.0]), top_p=rng.choice([0.9, 0.95, 1.0]),
+                 dtype=rng.choice(["bf16", "bf16", "float32"]))
+    elif kind == "generate":
+        c.update(shape=rng.choice(["0.5b", "1.5b"]), layers=rng.randint(2, LAYERS),
+                 prompts=_log(rng, 1, 24), samples=rng.choice([1, 4]), mean=_log(rng, 20, 400),
+                 tokens=rng.randint(16, 96), cache=rng.choice(["fp8", "bf16"]))
+    elif kind == "prompt":
+        c.update(model=rng.choice(["gonurax", "bedalorn", "qwen2"]), rows=_log(rng, 1, 16),
+                 mean=_log(rng, 60, 12000), steps=rng.choice([1, 1, 2, 4]))
+        c["rows"] = max(1, min(c["rows"], 12000 // c["mean"]))
+    elif kind == "experts":
+        c.update(size=rng.choice(["1.5b", "3b"]), rows=_log(rng, 1, 8192))
+    else:
+        c.update(rows=_log(rng, 1, 256), mean=_log(rng, 60, 8000), rank=rng.choice([256, 512]))
+        c["rows"] = max(1, min(c["rows"], 260000 // c["mean"]))
+    return c
+
+
+# ------------------------------------------------------------------- inputs
+def _gen(seed):
+    return torch.Generator(device="cuda").manual_seed(int(seed) * 7919 + 17)
+
+
+def _randn(g, *shape, std=1.0, dtype=torch.bfloat16):
+    return (torch.randn(*shape, generator=g, device="cuda") * std).to(dtype)
+
+
+def _lengths(case, seed, least=8):
+    """Ragged lengths: a third of the mean up to five thirds, odd ones among them.
+    The seed orders them."""
+    r, m = random.Random(case["rows"] * 7919 + case["mean"]), case["mean"]
+    lens = [max(least, int(m * (0.34 + 1.33 * r.random()))) for _ in range(case["rows"])]
+    random.Random(int(seed) * 31 + 7).shuffle(lens)
+    return lens
+
+
+def _lens_total(case):
+    return case["rows"] * case["mean"]
+
+
+def _qwen_config(case, shape):
+    W, ff, H, G, D = SHAPES[shape]
+    return dict(hidden_size=W, intermediate_size=ff, num_heads=H, num_kv_heads=G, head_dim=D,
+                num_layers=case["layers"], vocab_size=case["vocab"], max_position=8192)
+
+
+def _reward_config(case):
+    return dict(num_layers=case["layers"], vocab_size=case["vocab"], max_position=4096)
+
+
+def _qwen_weights(cfg, seed, small=1.0):
+    """Base weights by their names in the framework's model; `small` scales
+    what the layers add to the embedding."""
+    g, w = _gen(seed), {}
+    W, ff = cfg.hidden_size, cfg.intermediate_size
+    q, kv = cfg.num_heads * cfg.head_dim, cfg.num_kv_heads * cfg.head_dim
+    w["model.embed_tokens.weight"] = _randn(g, cfg.vocab_size, W, std=0.02)
+    for i in range(cfg.num_layers):
+        p = f"model.layers.{i}."
+        w[p + "self_attn.qkv_proj.weight"] = _randn(g, q + 2 * kv, W, std=0.02)
+        w[p + "self_attn.qkv_proj.bias"] = _randn(g, q + 2 * kv, std=0.3)
+        w[p + "self_attn.o_proj.weight"] = _randn(g, W, q, std=0.02 * small)
+        w[p + "mlp.gate_up_proj.weight"] = _randn(g, 2 * ff, W, std=0.02)
+        w[p + "mlp.down_proj.weight"] = _randn(g, W, ff, std=0.02 * small)
+        for n in ("input_layernorm", "post_attention_layernorm"):
+            w[p + n + ".weight"] = 1 + _randn(g, W, std=0.1)
+    w["model.norm.weight"] = 1 + _randn(g, W, std=0.1)
+    return w
+
+
+def _built(make):
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        with torch.device("cuda"):
+            return make()
+    finally:
+        torch.set_default_dtype(torch.float32)
+
+
+def _qwen(cfg, w):
+    m = _built(lambda: CausalLM(cfg))
+    m.load_state_dict(w, strict=True)
+    return m
+
+
+LORA = LoraConfig(r=64, alpha=16)
+
+
+def _lora_weights(cfg, seed):
+    g, out = _gen(seed + 1000003), {}
+    for n, t in _qwen_weights_shapes(cfg).items():
+        N, K = t
+        out[n + ".lora_A"] = _randn(g, 64, K, std=K ** -0.5)
+        out[n + ".lora_B"] = _randn(g, N, 64, std=0.01)
+    return out
+
+
+def _qwen_weights_shapes(cfg):
+    W, ff = cfg.hidden_size, cfg.intermediate_size
+    q, kv = cfg.num_heads * cfg.head_dim, cfg.num_kv_heads * cfg.head_dim
+    out = {}
+    for i in range(cfg.num_layers):
+        p = f"model.layers.{i}."
+        out[p + "self_attn.qkv_proj"] = (q + 2 * kv, W)
+        out[p + "self_attn.o_proj"] = (W, q)
+        out[p + "mlp.gate_up_proj"] = (2 * ff, W)
+        out[p + "mlp.down_proj"] = (W, ff)
+    return out
+
+
+def _episodes(case, seed):
+    """Packed rows of prompt and response, and which hidden states predict
+    which response tokens."""
+    lens = _lengths(case, seed, least=24)
+    g = _gen(seed + 2000003)
+    seqs = [torch.randint(2, case["vocab"], (n,), generator=g, device="cuda") for n in lens]
+    plen = [max(8, int(n * (0.1 + n % 17 / 50))) for n in lens]     # the prompt's part
+    first, rows = 0, []
+    for n, p in zip(lens, plen):
+        rows.append(torch.arange(first + p - 1, first + n - 1))
+        first += n
+    return seqs, lens, torch.cat(rows).cuda()
+
+
+def _prepare_train(case, seed):
+    cfg = get_config("qwen2.5-1.5b", **_qwen_config(case, case["shape"]))
+    model = _qwen(cfg, _qwen_weights(cfg, seed))
+    apply_lora(model, LORA)
+    lora = _lora_weights(cfg, seed)
+    with torch.no_grad():
+        for n, p in model.named_parameters():
+            if n in lora:
+                p.copy_(lora[n])
+    seqs, _, rows = _episodes(case, seed)
+    ids, cu, mx, pos = pack_sequences(seqs, device="cuda")
+    adv = _randn(_gen(seed + 5), len(rows), dtype=torch.float32)
+    names = [(n, p) for n, p in model.named_parameters() if p.requires_grad]
+    opt = ops.FusedAdamW([p for _, p in names], lr=1e-4)
+    return dict(case=case, model=model.train(), opt=opt, names=names, ids=ids, cu=cu, mx=mx,
+                pos=pos, rows=rows, labels=ids[rows + 1], adv=adv)
+
+
+def _run_train(s):
+    s["opt"].zero_grad(set_to_none=True)
+    hidden = s["model"](s["ids"], CausalLM.train_ctx(s["cu"], s["mx"], s["pos"]))
+    lp, ent = ops.token_logprob_entropy(hidden[s["rows"]], s["model"].lm_head_weight, s["labels"],
+                                        0.7)
+    loss = -(lp * s["adv"]).sum() / lp.numel()
+    loss.backward()
+    s["opt"].step()
+    return dict(logprob=lp.detach(), entropy=ent, grads={n: p.grad for n, p in s["names"]},
+                weights={n: p.detach() for n, p in s["names"]})
+
+
+def _prepare_score(case, seed):
+    seqs, _, rows = _episodes(case, seed)
+    ids, cu, mx, pos = pack_sequences(seqs, device="cuda")
+    s = dict(case=case, ids=ids, cu=cu, mx=mx, pos=pos, rows=rows, labels=ids[rows + 1])
+    if case["model"] == "reward":
+        cfg = get_config("rm-large", **_reward_config(case))
+        s["model"] = _built(lambda: ScalarHeadModel(cfg))
+        w = _qwen_weights(cfg, seed)
+        w["score.weight"] = _randn(_gen(seed + 9), 1, cfg.hidden_size, std=0.03)
+        s["model"].load_state_dict(w, strict=True)
+    else:
+        cfg = get_config("qwen2.5-1.5b", **_qwen_config(case, case["model"]))
+        s["model"] = _qwen(cfg, _qwen_weights(cfg, seed))
+    s["model"].eval()
+    return s
+
+
+@torch.no_grad()
+def _run_score(s):
+    if s["case"]["model"] == "reward":
+        return dict(scores=s["model"].sequence_scores(s["ids"], s["cu"], s["mx"]))
+    hidden = s["model"](s["ids"], CausalLM.train_ctx(s["cu"], s["mx"], s["pos"]))
+    lp, ent = ops.token_logprob_entropy(hidden[s["rows"]], s["model"].lm_head_weight, s["labels"],
+                                        0.7)
+    return dict(logprob=lp, entropy=ent)
+
+
+def _prepare_attention(case, seed):
+    H, G, D, causal = HEADS[case["shape"]]
+    lens = _lengths(case, seed)
+    T, g = sum(lens), _gen(seed)
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    # scores of a standard deviation of about 1.5; values around a mean per channel
+    q, k = _randn(g, T, H, D, std=1.5), _randn(g, T, G, D)
+    v = (torch.randn(T, G, D, generator=g, device="cuda")
+         + torch.randn(1, G, D, generator=g, device="cuda")).bfloat16()
+    do = _randn(g, T, H, D)
+    for t in (q, k, v):
+        t.requires_grad_(case["backward"])
+    return dict(case=case, q=q, k=k, v=v, do=do, cu=cu, lens=lens, causal=causal)
+
+
+def _run_attention(s):
+    q, k, v = s["q"], s["k"], s["v"]
+    o = ops.flash_attn_varlen(q, k, v, s["cu"], max(s["lens"]), causal=s["causal"])
+    if not s["case"]["backward"]:
+        return dict(o=o)
+    dq, dk, dv = torch.autograd.grad(o, (q, k, v), s["do"])
+    return dict(o=o.detach(), dq=dq, dk=dk, dv=dv)
+
+
+def _pages(lens, seed):
+    """Block tables of sequences whose pages lie in no order, as they do after
+    some have finished and others were let in."""
+    n = [-(-l // PAGE) for l in lens]
+    order = torch.randperm(sum(n), generator=torch.Generator().manual_seed(int(seed)))
+    bt, at = torch.zeros(len(lens), max(n), dtype=torch.int32), 0
+    for i, m in enumerate(n):
+        bt[i, :m] = order[at:at + m]
+        at += m
+    return bt, sum(n)
+
+
+def _prepare_decode(case, seed):
+    W, ff, H, G, D = SHAPES[case["shape"]]
+    lens = _lengths(case, seed, least=1)
+    bt, P = _pages(lens, seed)
+    g = _gen(seed)
+    dt = torch.float8_e4m3fn if case["cache"] == "fp8" else torch.bfloat16
+    k = _randn(g, P, PAGE, G, D, dtype=dt)
+    v = (torch.randn(P, G, D, PAGE, generator=g, device="cuda")
+         + torch.randn(1, G, D, 1, generator=g, device="cuda")).to(dt)
+    return dict(case=case, q=_randn(g, len(lens), H, D, std=1.5), k=k, v=v, bt=bt.cuda(),
+                lens=torch.tensor(lens, dtype=torch.int32).cuda(), scale=D ** -0.5)
+
+
+def _run_decode(s):
+    return dict(o=ops.paged_attn_decode(s["q"], s["k"], s["v"], s["bt"], s["lens"], s["scale"]))
+
+
+def _prepare_sample(case, seed):
+    """Peaked logits over a long tail, as language models have them: the n-th
+    most likely token has about n^-1.4 of the weight of the first."""
+    g, V, B = _gen(seed), case["vocab"], case["rows"]
+    tail = -1.4 * torch.arange(1, V + 1, device="cuda").log()
+    x = torch.empty(B, V, dtype=torch.bfloat16 if case["dtype"] == "bf16" else torch.float32,
+                    device="cuda")
+    for i in range(B):
+        if i % 64 == 0:
+            place = torch.randperm(V, generator=g, device="cuda")
+        x[i] = (tail[place.roll(i * 37)] + 18 + 0.6 * torch.randn(V, generator=g, device="cuda"))
+    return dict(case=case, logits=x, seed=int(seed))
+
+
+def _run_sample(s):
+    c = s["case"]
+    return ops.sample_tokens(s["logits"], c["temperature"], c["top_p"], s["seed"], 1)
+
+
+def _prepare_generate(case, seed):
+    """A policy that is sure of its next token at most steps: its layers add
+    little to the embedding, which the head reads back."""
+    cfg = get_config("qwen2.5-1.5b", **_qwen_config(dict(case, vocab=151936), case["shape"]))
+    model = _qwen(cfg, _qwen_weights(cfg, seed, small=0.01)).eval()
+    r = random.Random(int(seed))
+    prompts = [[r.randrange(2, 151000) for _ in range(n)]
+               for n in _lengths(dict(case, rows=case["prompts"]), seed)]
+    pool = case["samples"] * sum(len(p) + case["tokens"] + PAGE for p in prompts)
+    eng = SamplerEngine(model, kv_pool_tokens=pool,
+                        kv_cache_dtype="fp8_e4m3" if case["cache"] == "fp8" else "bf16")
+    par = SamplingParams(n=case["samples"], temperature=0.7, top_p=0.95,
+                         max_tokens=case["tokens"], seed=int(seed), stop_token_id=1)
+    return dict(case=case, eng=eng, prompts=prompts, params=par)
+
+
+def _run_generate(s):
+    return s["eng"].generate(s["prompts"], s["params"])
+
+
+# -- served models, as serving_bench shapes them at width 1536
+W15, FF15, H15, G15 = 1536, 8960, 12, 2
+SERVED_VOCAB = 32768
+
+
+def _served_config(model):
+    if model == "qwen2":
+        return get_config("qwen2.5-1.5b", num_layers=LAYERS, vocab_size=SERVED_VOCAB)
+    if model == "bedalorn":
+        return BedalornConfig(vocab_size=SERVED_VOCAB, hidden_size=W15, logit_scale=0.5,
+                              **_bedalorn_layers(4, heads=H15, dim=128, vdim=128, kv_rank=512,
+                                                 wkv_heads=W15 // 64, wkv_dim=64, decay_rank=64,
+                                                 ff=FF15, experts=N_EXPERTS, top=TOP,
+                                                 expert_ff=FF15 // 4, loop=(1, 3, 2)))
+    return GonuraxConfig(vocab_size=SERVED_VOCAB, hidden_size=W15, norm_groups=4,
+                         residual_mult=0.5,
+                         **_gonurax_layers(LAYERS, heads=H15, dim=128, vdim=128, attn_heads=H15,
+                                           kv_heads=G15, attn_dim=128, ff=FF15, window=1024,
+                                           keep_first=4))
+
+
+def _gonurax_weights(cfg, seed):
+    g, w = _gen(seed), {}
+    W = cfg.hidden_size
+
+    def lin(name, n, k):
+        w[name] = _randn(g, n, k, std=k ** -0.5)
+
+    w["embed"] = _randn(g, cfg.vocab_size, W)
+    for i, l in enumerate(cfg.layers):
+        m, p = l["mixer"], f"l{i}.mix."
+        H, D, V, G = m["heads"], m["dim"], m["vdim"], m.get("kv_heads", m["heads"])
+        w[f"l{i}.norm1"] = 1 + _randn(g, W, std=0.2)
+        lin(p + "q", H * D, W), lin(p + "k", G * D, W), lin(p + "v", G * V, W)
+        if l["type"] == "attention":
+            w[p + "q.norm"] = 1.3 + _randn(g, D, std=0.2)
+            w[p + "k.norm"] = 1.3 + _randn(g, D, std=0.2)
+        else:
+            lin(p + "g", H * V, W)
+        if l["type"] == "lightning":
+            w[p + "norm"] = 1 + _randn(g, H * V, std=0.2)
+        lin(p + "o", W, H * V)
+        ff = l["mlp"]["ff"]
+        p = f"l{i}.mlp."
+        lin(p + "gate", ff, W), lin(p + "up", ff, W), lin(p + "down", W, ff)
+    w["final.norm"] = 1 + _randn(g, W, std=0.2)
+    return w
+
+
+def _bedalorn_weights(cfg, seed):
+    g, w = _gen(seed), {}
+    W = cfg.hidden_size
+
+    def lin(name, n, k, std=1.0):
+        w[name] = _randn(g, n, k, std=std * k ** -0.5)
+
+    w["embed"], w["final.norm"] = _randn(g, cfg.vocab_size, W), _randn(g, W, std=0.3)
+    lin("loop.in", W, 2 * W)
+    w["loop.step"] = _randn(g, cfg.loop["times"], W, std=0.5)
+    for i, l in enumerate(cfg.layers):
+        m, p = l["mixer"], f"l{i}.mix."
+        w[f"l{i}.norm1"], w[f"l{i}.norm2"] = _randn(g, W, std=0.3), _randn(g, W, std=0.3)
+        H, D = m["heads"], m["dim"]
+        if l["type"] == "wkv":
+            for x in "rkvgw":
+                w[p + "mu." + x] = torch.rand(W, generator=g, device="cuda").bfloat16()
+            for x in "rkvg":
+                lin(p + x, H * D, W)
+            lin(p + "w1", m["decay_rank"], W), lin(p + "w2", H * D, m["decay_rank"])
+            w[p + "w0"] = -2.5 + _randn(g, H * D, std=1.5)
+            w[p + "u"], w[p + "norm"] = _randn(g, H, D), 1 + _randn(g, H * D, std=0.3)
+            lin(p + "o", W, H * D)
+        else:
+            R, V = m["kv_rank"], m["vdim"]
+            lin(p + "q", H * D, W), lin(p + "dkv", R, W)
+            w[p + "dkv.norm"] = 1 + _randn(g, R, std=0.3)
+            lin(p + "uk", H * D, R), lin(p + "uv", H * V, R), lin(p + "o", W, H * V)
+        mlp, p = l["mlp"], f"l{i}.mlp."
+        if mlp["kind"] == "dense":
+            lin(p + "up", mlp["ff"], W), lin(p + "down", W, mlp["ff"])
+        else:
+            E, ff = mlp["router"]["experts"], mlp["expert"]["ff"]
+            lin(p + "router", E, W, 2.0)
+            w[p + "router.b"] = _randn(g, E, std=0.3)
+            for e in range(E):
+                lin(f"{p}e{e}.gate", ff, W), lin(f"{p}e{e}.up", ff, W)
+                lin(f"{p}e{e}.down", W, ff)
+    return w
+
+
+def _prepare_prompt(case, seed):
+    cfg = _served_config(case["model"])
+    if case["model"] == "qwen2":
+        model = _qwen(cfg, _qwen_weights(cfg, seed)).eval()
+    else:
+        make = _gonurax_weights if case["model"] == "gonurax" else _bedalorn_weights
+        model = _built(lambda: build_model(cfg)).eval()
+        model.load(make(cfg, seed))
+    lens = _lengths(case, seed, least=case["steps"])
+    r = random.Random(int(seed))
+    seqs = [SeqState(i, [r.randrange(2, SERVED_VOCAB) for _ in range(n)], i)
+            for i, n in enumerate(lens)]
+    eng = SamplerEngine(model, kv_pool_tokens=sum(n + PAGE for n in lens), kv_cache_dtype="bf16",
+                        state_slots=len(lens))
+    return dict(case=case, eng=eng, seqs=seqs, model=model)
+
+
+@torch.no_grad()
+def _run_prompt(s):
+    steps, outs = s["case"]["steps"], []
+    for q in s["seqs"]:
+        q.computed = 0
+    for k in range(steps):
+        entries = [(q, len(q) * (k + 1) // steps - q.computed) for q in s["seqs"]]
+        hidden, first = s["eng"].step(entries)
+        outs.append(hidden)
+    last = torch.tensor([a + n - 1 for a, (_, n) in zip(first, entries)], device="cuda")
+    return dict(hidden=outs, logits=s["model"].logits(hidden[last]))
+
+
+def _prepare_experts(case, seed):
+    W, ff = EXPERTS[case["size"]]
+    g, E = _gen(seed), N_EXPERTS
+    return dict(case=case, h=_randn(g, case["rows"], W), router=_randn(g, E, W, std=2 * W ** -0.5),
+                bias=_randn(g, E, std=0.3), gate_up=_randn(g, E, 2, ff, W, std=W ** -0.5),
+                down=_randn(g, E, W, ff, std=ff ** -0.5))
+
+
+def _run_experts(s):
+    routing = ops.moe_route(s["h"], s["router"], s["bias"], TOP)
+    y = ops.moe_experts(s["h"], s["gate_up"], s["down"], routing)
+    return dict(y=y, chosen=routing[0], weights=routing[1])
+
+
+LATENT_HEADS, LATENT_DIM = 12, 128
+
+
+def _prepare_latent(case, seed):
+    H, D, R = LATENT_HEADS, LATENT_DIM, case["rank"]
+    lens = _lengths(case, seed, least=1)
+    bt, P = _pages(lens, seed)
+    g = _gen(seed)
+    L = torch.tensor(lens, dtype=torch.int32).cuda()
+    uk = _randn(g, H, D, R, std=R ** -0.5)
+    ctx = AttnContext(mode="decode", positions=L.long() - 1, block_tables=bt.cuda(), seq_lens=L)
+    return dict(case=case, q=_randn(g, len(lens), H * D, std=1.5), cache=_randn(g, P, PAGE, R),
+                ctx=ctx, uk=uk, uk_t=uk.transpose(1, 2).contiguous(),
+                uv=_randn(g, H, D, R, std=R ** -0.5))
+
+
+def _run_latent(s):
+    out = torch.empty(s["q"].shape[0], LATENT_HEADS * LATENT_DIM, dtype=torch.bfloat16,
+                      device="cuda")
+    ops.latent_attn(s["q"], s["cache"], s["ctx"], s["uk"], s["uk_t"], s["uv"], out,
+                    LATENT_DIM ** -0.5)
+    return dict(o=out)
+
+
+_PREPARE = dict(train=_prepare_train, score=_prepare_score, attention=_prepare_attention,
+                decode=_prepare_decode, sample=_prepare_sample, generate=_prepare_generate,
+                prompt=_prepare_prompt, experts=_prepare_experts, latent=_prepare_latent)
+_RUN = dict(train=_run_train, score=_run_score, attention=_run_attention, decode=_run_decode,
+            sample=_run_sample, generate=_run_generate, prompt=_run_prompt, experts=_run_experts,
+            latent=_run_latent)
+
+
+def prepare(case, seed):
+    return _PREPARE[case["kind"]](case, seed)
+
+
+def run(state):
+    return _RUN[state["case"]["kind"]](state)
+
+
+# --------------------------------------------------------------------- work
+def _dense_params(shape):
+    W, ff, H, G, D = shape
+    return W * (H + 2 * G) * D + H * D * W + 3 * W * ff
+
+
+def work(case):
+    kind = case["kind"]
+    if kind in ("train", "score"):
+        reward = case.get("model") == "reward"
+        shape = (1024, 4096, 16, 16, 64) if reward else SHAPES[case.get("shape") or case["model"]]
+        W, ff, H, G, D = shape
+        T, n = _lens_total(case), _dense_params(shape) * case["layers"]
+        pairs = case["rows"] * case["mean"] ** 2 * (1.15 if reward else 0.575)
+        attn = 4 * pairs * H * D * case["layers"]
+        head = 0 if reward else 2 * 0.75 * T * W * case["vocab"]
+        if kind == "score":
+            return dict(flops=2 * T * n + attn + head,
+                        bytes=2 * n + 2 * case["vocab"] * W + 4 * T * W)
+        # frozen weights: no gradient of theirs; the head's logits are made once
+        adapters = case["layers"] * 64 * (2 * W + 2 * H * D + 2 * G * D + 3 * ff + 2 * W)
+        trained = case["vocab"] * W + adapters
+        return dict(flops=4 * T * n + 6 * T * adapters + 3.5 * attn + 3 * head,
+                    bytes=2 * n + 22 * trained + 4 * T * W)
+    if kind == "attention":
+        H, G, D, causal = HEADS[case["shape"]]
+        T = _lens_total(case)
+        pairs = case["rows"] * case["mean"] ** 2 * 1.15 * (0.5 if causal else 1.0)
+        io = 2 * T * D * (2 * H + 2 * G)
+        return dict(flops=4 * pairs * H * D * (3.5 if case["backward"] else 1.0),
+                    bytes=io * (3 if case["backward"] else 1))
+    if kind == "decode":
+        W, ff, H, G, D = SHAPES[case["shape"]]
+        T, size = _lens_total(case), 1 if case["cache"] == "fp8" else 2
+        return dict(bytes=T * 2 * G * D * size + 4 * case["rows"] * H * D, flops=4 * T * H * D)
+    if kind == "sample":
+        n = case["rows"] * case["vocab"]
+        return dict(bytes=n * (2 if case["dtype"] == "bf16" else 4), flops=6 * n)
+    if kind == "generate":
+        shape = SHAPES[case["shape"]]
+        n, head = _dense_params(shape) * case["layers"], 151936 * shape[0]
+        rows, size = case["prompts"] * case["samples"], 1 if case["cache"] == "fp8" else 2
+        kv = 2 * shape[3] * shape[4] * size * case["layers"]
+        steps = case["tokens"]
+        tokens = rows * (case["mean"] + steps)
+        return dict(bytes=2 * (n + head) * steps + rows * kv * steps * (case["mean"] + steps / 2),
+                    flops=2 * n * tokens + 2 * head * rows * steps)
+    if kind == "prompt":
+        T = _lens_total(case)
+        if case["model"] == "bedalorn":
+            n = 4 * (2 * W15 * W15 + 3 * 512 * W15) + 2 * 5 * W15 * W15 \
+                + 3 * 2 * W15 * FF15 + 3 * 3 * W15 * FF15 + 4 * W15 * W15
+            pairs = case["rows"] * case["mean"] ** 2 * 0.575 * 4
+            weights = n + 3 * 3 * W15 * FF15 * 3
+        else:
+            n = LAYERS * _dense_params(SHAPES["1.5b"])
+            pairs = case["rows"] * case["mean"] ** 2 * 0.575 * LAYERS
+            if case["model"] == "gonurax":
+                n += 4 * W15 * W15 * 2
+                pairs = 2 * case["rows"] * case["mean"] * min(case["mean"] / 2, 1024)
+            weights = n
+        return dict(flops=2 * T * n + 4 * pairs * H15 * 128, bytes=2 * weights + 4 * T * W15)
+    if kind == "experts":
+        W, ff = EXPERTS[case["size"]]
+        used = N_EXPERTS * (1 - (1 - TOP / N_EXPERTS) ** case["rows"])
+        return dict(flops=6 * W * ff * TOP * case["rows"],
+                    bytes=used * 6 * W * ff + 2 * case["rows"] * W * (1 + TOP))
+    H, D, R = LATENT_HEADS, LATENT_DIM, case["rank"]
+    return dict(bytes=2 * _lens_total(case) * R + 4 * H * D * R + 4 * case["rows"] * H * D,
+                flops=4 * _lens_total(case) * H * R + 4 * case["rows"] * H * D * R)
+
+
+def tolerance(case):
+    """About four times what bf16 leaves between run() and exact()."""
+    kind = case["kind"]
+    if kind == "train":           # gradients through the layers: 0.01 measured
+        return {"rel": 0.03, "max": 0.9}
+    if kind == "score":           # 0.001 (log-probabilities) to 0.006 (scores)
+        return {"rel": 0.024, "max": 0.3}
+    if kind == "attention":       # 0.002 to 0.004
+        return {"rel": 0.015, "max": 0.3}
+    if kind == "decode":          # 0.002; in 8 bits the weights are rounded to 3 bits: 0.005
+        return {"rel": 0.02 if case["cache"] == "fp8" else 0.007, "max": 0.2}
+    if kind in ("sample", "generate"):      # a draw at the border of two tokens may tip over
+        return {"rel": 0.0, "differ": 0.01}
+    if kind == "prompt":          # 0.005; 0.015 where a router's near ties pick other experts
+        return {"rel": 0.03, "max": 0.9}
+    if kind == "experts":         # 0.0024
+        return {"rel": 0.01, "max": 0.1, "differ": 0.001}
+    return {"rel": 0.013, "max": 0.15}      # latent: 0.0032
+
+
+# -------------------------------------------------------------------- exact
+def _rms(x, eps):
+    return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + eps)
+
+
+def _attend(q, k, v, scale, causal=True, size=1 << 30, keep=0):
+    """One sequence, 64 bits: q [T, H, D], k [T, G, D], v [T, G, V], rows in blocks."""
+    T, H, _ = q.shape
+    rep, out, step = H // k.shape[1], [], 1024
+    kt, vt = (t.transpose(0, 1).repeat_interleave(rep, 0) for t in (k, v))
+    for a in range(0, T, step):
+        b = min(a + step, T)
+        n = b if causal else T
+        s = (q[a:b].transpose(0, 1) @ kt[:, :n].transpose(1, 2)) * scale
+        if causal:
+            i = torch.arange(a, b, device=q.device)[:, None]
+            j = torch.arange(n, device=q.device)[None, :]
+            s = s.masked_fill((j > i) | ((i - j >= size) & (j >= keep)), -math.inf)
+        out.append((torch.softmax(s, -1) @ vt[:, :n]).transpose(0, 1))
+    return torch.cat(out)
+
+
+def _turn_half(x, pos, base):
+    D = x.shape[-1]
+    a = pos[:, None, None] * base ** (-torch.arange(0, D, 2, device=x.device).double() / D)
+    u, v = x[..., :D // 2], x[..., D // 2:]
+    return torch.cat([u * a.cos() - v * a.sin(), v * a.cos() + u * a.sin()], -1)
+
+
+def _turn_pairs(x, pos, base, sign=1.0):
+    D = x.shape[-1]
+    a = sign * pos[:, None, None] * base ** (-torch.arange(0, D, 2, device=x.device).double() / D)
+    u, v = x[..., 0::2], x[..., 1::2]
+    return torch.stack([u * a.cos() - v * a.sin(), v * a.cos() + u * a.sin()], -1).flatten(-2)
+
+
+def _qwen64(cfg, w, ids, lens, lora=None):
+    """Final normed hidden states of packed rows."""
+    from torch.utils.checkpoint import checkpoint
+    H, G, D = cfg.num_heads, cfg.num_kv_heads, cfg.head_dim
+    pos = torch.cat([torch.arange(n, device="cuda") for n in lens]).double()
+
+    def lin(name, x, bias=None):
+        y = x @ w[name + ".weight"].double().t()
+        if lora is not None:
+            y = y + 0.25 * (x @ lora[name + ".lora_A"].t()) @ lora[name + ".lora_B"].t()
+        return y if bias is None else y + bias.double()
+
+    def attend(q, k, v):
+        return torch.cat([_attend(a, b, c, D ** -0.5, not cfg.bidirectional)
+                          for a, b, c in zip(q.split(lens), k.split(lens), v.split(lens))])
+
+    x = w["model.embed_tokens.weight"].double()[ids]
+    for i in range(cfg.num_layers):
+        p = f"model.layers.{i}."
+        h = _rms(x, cfg.rms_eps) * w[p + "input_layernorm.weight"].double()
+        qkv = lin(p + "self_attn.qkv_proj", h, w[p + "self_attn.qkv_proj.bias"])
+        q, k, v = (t.unflatten(1, (-1, D)) for t in qkv.split([H * D, G * D, G * D], 1))
+        q, k = _turn_half(q, pos, cfg.rope_theta), _turn_half(k, pos, cfg.rope_theta)
+        if torch.is_grad_enabled():
+            o = checkpoint(attend, q, k, v, use_reentrant=False)
+        else:
+            o = attend(q, k, v)
+        x = x + lin(p + "self_attn.o_proj", o.flatten(1))
+        h = _rms(x, cfg.rms_eps) * w[p + "post_attention_layernorm.weight"].double()
+        gate, up = lin(p + "mlp.gate_up_proj", h).chunk(2, 1)
+        x = x + lin(p + "mlp.down_proj", torch.nn.functional.silu(gate) * up)
+    return _rms(x, cfg.rms_eps) * w["model.norm.weight"].double()
+
+
+def _logprob64(hidden, head, labels):
+    lps, ents = [], []
+    for a in range(0, len(labels), 8192):
+        z = torch.log_softmax(hidden[a:a + 8192] @ head.t() / (0.7 + 1e-7), -1)
+        lps.append(z.gather(1, labels[a:a + 8192, None])[:, 0])
+        ents.append(-(z.detach().exp() * z.detach()).sum(-1))
+    return torch.cat(lps), torch.cat(ents)
+
+
+def _exact_train(case, seed):
+    cfg = get_config("qwen2.5-1.5b", **_qwen_config(case, case["shape"]))
+    w = _qwen_weights(cfg, seed)
+    lora = {n: t.double().requires_grad_() for n, t in _lora_weights(cfg, seed).items()}
+    emb = "model.embed_tokens.weight"
+    w[emb] = w[emb].double().requires_grad_()
+    seqs, lens, rows = _episodes(case, seed)
+    ids = torch.cat(seqs)
+    adv = _randn(_gen(seed + 5), len(rows), dtype=torch.float32).double()
+    lp, ent = _logprob64(_qwen64(cfg, w, ids, lens, lora)[rows], w[emb], ids[rows + 1])
+    (-(lp * adv).sum() / lp.numel()).backward()
+    leaves = {emb: w[emb], **lora}
+    grads = {n: t.grad for n, t in leaves.items()}
+    new = {n: t.detach() - 1e-4 * t.grad / (t.grad.abs() + 1e-8) for n, t in leaves.items()}
+    return dict(logprob=lp.detach(), entropy=ent, grads=grads, weights=new)
+
+
+@torch.no_grad()
+def _exact_score(case, seed):
+    seqs, lens, rows = _episodes(case, seed)
+    ids = torch.cat(seqs)
+    if case["model"] == "reward":
+        cfg = get_config("rm-large", **_reward_config(case))
+        h = _qwen64(cfg, _qwen_weights(cfg, seed), ids, lens)
+        head = _randn(_gen(seed + 9), 1, cfg.hidden_size, std=0.03).double()
+        last = torch.tensor(lens, device="cuda").cumsum(0) - 1
+        return dict(scores=(h[last] @ head.t())[:, 0])
+    cfg = get_config("qwen2.5-1.5b", **_qwen_config(case, case["model"]))
+    w = _qwen_weights(cfg, seed)
+    lp, ent = _logprob64(_qwen64(cfg, w, ids, lens)[rows],
+                         w["model.embed_tokens.weight"].double(), ids[rows + 1])
+    return dict(logprob=lp, entropy=ent)
+
+
+def _exact_attention(case, seed):
+    """Forward by blocks of rows, and the backward written out the same way."""
+    s = _prepare_attention(case, seed)
+    q, k, v, do = (s[n].detach().double() for n in ("q", "k", "v", "do"))
+    G, D = k.shape[1:]
+    rep, scale = q.shape[1] // G, D ** -0.5
+    o = torch.empty_like(q)
+    dq, dk, dv = (torch.zeros_like(t) for t in (q, k, v))
+    first = 0
+    for n in s["lens"]:
+        for g in range(G):
+            kk, vv = k[first:first + n, g], v[first:first + n, g]
+            for a in range(0, n, 1024):
+                b = min(a + 1024, n)
+                m = b if s["causal"] else n
+                rows, heads = slice(first + a, first + b), slice(g * rep, (g + 1) * rep)
+                qq = q[rows, heads].transpose(0, 1)
+                z = (qq @ kk[:m].t()) * scale
+                if s["causal"]:
+                    i = torch.arange(a, b, device="cuda")[:, None]
+                    z = z.masked_fill(torch.arange(m, device="cuda")[None, :] > i, -math.inf)
+                p = torch.softmax(z, -1)
+                oo = p @ vv[:m]
+                o[rows, heads] = oo.transpose(0, 1)
+                if not case["backward"]:
+                    continue
+                dd = do[rows, heads].transpose(0, 1)
+                dz = p * (dd @ vv[:m].t() - (dd * oo).sum(-1, keepdim=True)) * scale
+                dq[rows, heads] = (dz @ kk[:m]).transpose(0, 1)
+                dk[first:first + m, g] += (dz.transpose(1, 2) @ qq).sum(0)
+                dv[first:first + m, g] += (p.transpose(1, 2) @ dd).sum(0)
+        first += n
+    return dict(o=o, dq=dq, dk=dk, dv=dv) if case["backward"] else dict(o=o)
+
+
+def _exact_decode(case, seed):
+    s = _prepare_decode(case, seed)
+    H, D = s["q"].shape[1:]
+    G = s["k"].shape[2]
+    place = torch.arange(D, device="cuda")
+    if case["cache"] == "fp8":      # each key's groups of 8 are stored (d % 32) / 8 first
+        place = (place % 32) // 8 * (D // 4) + place // 32 * 8 + place % 8
+    out = torch.empty(len(s["lens"]), H, D, dtype=torch.float64, device="cuda")
+    for b, n in enumerate(s["lens"].tolist()):
+        pages = s["bt"][b, :-(-n // PAGE)].long()
+        k = s["k"][pages].double().flatten(0, 1)[:n][..., place]
+        v = s["v"][pages].double().permute(0, 3, 1, 2).flatten(0, 1)[:n]
+        q = s["q"][b].double().unflatten(0, (G, -1))
+        z = torch.softmax(q @ k.permute(1, 2, 0) * s["scale"], -1)
+        out[b] = (z @ v.transpose(0, 1)).flatten(0, 1)
+    return dict(o=out)
+
+
+def _exact_latent(case, seed):
+    s = _prepare_latent(case, seed)
+    uk, uv = s["uk"].double(), s["uv"].double()
+    out = torch.empty(s["q"].shape, dtype=torch.float64, device="cuda")
+    for b, n in enumerate(s["ctx"].seq_lens.tolist()):
+        pages = s["ctx"].block_tables[b, :-(-n // PAGE)].long()
+        c = s["cache"][pages].double().flatten(0, 1)[:n]
+        q = s["q"][b].double().unflatten(0, (LATENT_HEADS, -1))
+        qc = (q[:, None] @ uk)[:, 0]
+        z = torch.softmax(qc @ c.t() * LATENT_DIM ** -0.5, -1)
+        out[b] = ((z @ c)[:, None] @ uv.transpose(1, 2)).flatten()
+    return dict(o=out)
+
+
+def _exact_experts(case, seed):
+    s = _prepare_experts(case, seed)
+    h = s["h"].double()
+    z, chosen = torch.sort(h @ s["router"].double().t() + s["bias"].double(), dim=-1,
+                           descending=True, stable=True)
+    chosen, weights = chosen[:, :TOP], torch.softmax(z[:, :TOP], -1)
+    y = torch.zeros(h.shape[0], TOP, h.shape[1], dtype=torch.float64, device="cuda")
+    for e in range(N_EXPERTS):
+        r, c = (chosen == e).nonzero(as_tuple=True)
+        gate, up = (h[r] @ s["gate_up"][e, i].double().t() for i in (0, 1))
+        y[r, c] = weights[r, c, None] * ((torch.nn.functional.silu(gate) * up)
+                                         @ s["down"][e].double().t())
+    return dict(y=y, chosen=chosen.int(), weights=weights)
+
+
+def _decayed64(q, k, v, decay):
+    """S <- decay S + k v^T, o = S^T q in blocks of 512: [T, H, .]"""
+    T, H, D = q.shape
+    lg = torch.tensor(decay, dtype=torch.float64, device="cuda").log()[:, None]
+    S = torch.zeros(H, D, v.shape[-1], dtype=torch.float64, device="cuda")
+    out = []
+    for a in range(0, T, 512):
+        qq, kk, vv = (t[a:a + 512].transpose(0, 1) for t in (q, k, v))
+        n = qq.shape[1]
+        i = torch.arange(n, device="cuda").double()
+        gap = i[:, None] - i[None, :]
+        m = torch.where(gap >= 0, (lg[..., None] * gap.clamp(min=0)).exp(), 0.0)
+        o = ((qq @ kk.transpose(1, 2)) * m) @ vv + (lg * (i + 1)).exp()[..., None] * (qq @ S)
+        S = (lg * n).exp()[..., None] * S \
+            + (kk * (lg * (n - 1 - i)).exp()[..., None]).transpose(1, 2) @ vv
+        out.append(o.transpose(0, 1))
+    return torch.cat(out)
+
+
+def _gonurax64(cfg, w, ids):
+    eps, silu = cfg.norm_eps, torch.nn.functional.silu
+    T = len(ids)
+    pos = torch.arange(T, device="cuda").double()
+
+    def lin(name, x):
+        return x @ w[name].double().t()
+
+    def norm(name, x):
+        return _rms(x.unflatten(-1, (cfg.norm_groups, -1)), eps).flatten(-2) * w[name].double()
+
+    x = w["embed"].double()[ids]
+    for i, l in enumerate(cfg.layers):
+        m, p = l["mixer"], f"l{i}.mix."
+        h = norm(f"l{i}.norm1", x)
+        q, k = (lin(p + n, h).unflatten(1, (-1, m["dim"])) for n in "qk")
+        v = lin(p + "v", h).unflatten(1, (-1, m["vdim"]))
+        if l["type"] == "attention":
+            base = m["rot"]["base"]
+            q = _turn_pairs(_rms(q, eps) * w[p + "q.norm"].double(), pos, base)
+            k = _turn_pairs(_rms(k, eps) * w[p + "k.norm"].double(), pos, base)
+            o = _attend(q, k, _turn_pairs(v, pos, base), m["scale"], True, m["mask"]["size"],
+                        m["mask"]["keep_first"])
+            o = _turn_pairs(o, pos, base, -1.0).flatten(1)
+        elif l["type"] == "retention":
+            base = m["rot"]["base"]
+            o = _decayed64(_turn_half(q, pos, base), _turn_half(k, pos, base) * m["dim"] ** -0.5,
+                           v, m["decay"])
+            o = _rms(o, eps).flatten(1) * silu(lin(p + "g", h))
+        else:
+            o = _decayed64(silu(q), silu(k), silu(v), m["decay"]).flatten(1)
+            o = _rms(o, eps) * w[p + "norm"].double() * torch.sigmoid(lin(p + "g", h))
+        p2 = f"l{i}.mlp."
+        ff = torch.nn.functional.gelu(lin(p2 + "gate", h), approximate="tanh") * lin(p2 + "up", h)
+        x = x + cfg.residual_mult * (lin(p + "o", o) + lin(p2 + "down", ff))
+    return norm("final.norm", x)
+
+
+def _bedalorn64(cfg, w, ids):
+    eps, silu = cfg.norm_eps, torch.nn.functional.silu
+
+    def lin(name, x):
+        return x @ w[name].double().t()
+
+    def norm(name, x):
+        return _rms(x, eps) * (1 + w[name].double())
+
+    def wkv(p, m, h):
+        H, D = m["heads"], m["dim"]
+        gap = torch.cat([torch.zeros_like(h[:1]), h[:-1]]) - h
+        mix = {s: h + gap * w[p + "mu." + s].double() for s in "rkvgw"}
+        r, k, v = (lin(p + s, mix[s]).unflatten(1, (H, D)) for s in "rkv")
+        dec = torch.exp(-torch.exp(lin(p + "w2", torch.tanh(lin(p + "w1", mix["w"])))
+                                   + w[p + "w0"].double())).unflatten(1, (H, D))
+        u = w[p + "u"].double()
+        S = torch.zeros(H, D, D, dtype=torch.float64, device="cuda")
+        o = torch.empty_like(r)
+        ru = (r * u * k).sum(-1, keepdim=True) * v        # the bonus of the token itself
+        for t in range(len(h)):
+            o[t] = torch.bmm(r[t][:, None], S)[:, 0]
+            S = torch.baddbmm(dec[t][:, :, None] * S, k[t][:, :, None], v[t][:, None])
+        o = _rms(o + ru, eps).flatten(1) * w[p + "norm"].double() * silu(lin(p + "g", mix["g"]))
+        return lin(p + "o", o)
+
+    def latent(p, m, h):
+        q = lin(p + "q", h).unflatten(1, (-1, m["dim"]))
+        c = _rms(lin(p + "dkv", h), eps) * w[p + "dkv.norm"].double()
+        k = lin(p + "uk", c).unflatten(1, (-1, m["dim"]))
+        v = lin(p + "uv", c).unflatten(1, (-1, m["vdim"]))
+        return lin(p + "o", _attend(q, k, v, m["scale"]).flatten(1))
+
+    def experts(p, m, h):
+        z, best = torch.sort(lin(p + "router", h) + w[p + "router.b"].double(), -1,
+                             descending=True)
+        top = m["router"]["top"]
+        best, weight, y = best[:, :top], torch.softmax(z[:, :top], -1), torch.zeros_like(h)
+        for e in range(m["router"]["experts"]):
+            r, c = (best == e).nonzero(as_tuple=True)
+            a = silu(lin(f"{p}e{e}.gate", h[r])) * lin(f"{p}e{e}.up", h[r])
+            y[r] += weight[r, c, None] * lin(f"{p}e{e}.down", a)
+        return y
+
+    x0 = x = w["embed"].double()[ids]
+    for kind, i in cfg.plan():
+        if kind == "pass":
+            x = lin("loop.in", torch.cat([x, x0], -1)) + w["loop.step"][i].double()
+            continue
+        l, p = cfg.layers[i], f"l{i}."
+        x = x + (wkv if l["type"] == "wkv" else latent)(p + "mix.", l["mixer"],
+                                                        norm(p + "norm1", x))
+        h = norm(p + "norm2", x)
+        if l["mlp"]["kind"] == "dense":
+            x = x + lin(p + "mlp.down", torch.relu(lin(p + "mlp.up", h)).pow(2))
+        else:
+            x = x + experts(p + "mlp.", l["mlp"], h)
+    return norm("final.norm", x) * cfg.logit_scale
+
+
+@torch.no_grad()
+def _exact_prompt(case, seed):
+    cfg = _served_config(case["model"])
+    lens = _lengths(case, seed, least=case["steps"])
+    r = random.Random(int(seed))
+    rows = [torch.tensor([r.randrange(2, SERVED_VOCAB) for _ in range(n)], device="cuda")
+            for n in lens]
+    if case["model"] == "qwen2":
+        w = _qwen_weights(cfg, seed)
+        h, head = [_qwen64(cfg, w, x, [len(x)]) for x in rows], w["model.embed_tokens.weight"]
+    else:
+        make, model = ((_gonurax_weights, _gonurax64) if case["model"] == "gonurax"
+                       else (_bedalorn_weights, _bedalorn64))
+        w = make(cfg, seed)
+        h, head = [model(cfg, w, x) for x in rows], w["embed"]
+    steps, outs = case["steps"], []
+    for k in range(steps):      # a step lays single tokens first, then the longer portions
+        parts = [x[n * k // steps:n * (k + 1) // steps] for x, n in zip(h, lens)]
+        outs.append(torch.cat([p for p in parts if len(p) == 1]
+                              + [p for p in parts if len(p) != 1]))
+    return dict(hidden=outs, logits=torch.stack([x[-1] for x in h]) @ head.double().t())
+
+
+def exact(case, seed):
+    fn = dict(train=_exact_train, score=_exact_score, attention=_exact_attention,
+              decode=_exact_decode, latent=_exact_latent, experts=_exact_experts,
+              prompt=_exact_prompt).get(case["kind"])
+    return None if fn is None else fn(case, seed)   # sampled tokens have no 64-bit value
