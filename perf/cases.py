@@ -97,6 +97,8 @@ def draw(rng):
     elif kind == "score":
         c.update(model=rng.choice(["0.5b", "1.5b", "reward"]), layers=rng.randint(1, 6),
                  vocab=rng.choice([16384, 32768]), rows=_log(rng, 1, 96), mean=_log(rng, 40, 1500))
+        if c["model"] == "reward":      # one score a row: a few alone say little
+            c["rows"] = max(24, c["rows"])
         c["rows"] = max(1, min(c["rows"], 62000 // c["mean"]))
     elif kind == "attention":
         c.update(shape=rng.choice(sorted(HEADS)), rows=_log(rng, 1, 64), mean=_log(rng, 30, 6500),
@@ -158,13 +160,13 @@ def _reward_config(case):
     return dict(num_layers=case["layers"], vocab_size=case["vocab"], max_position=4096)
 
 
-def _qwen_weights(cfg, seed, small=1.0):
+def _qwen_weights(cfg, seed, small=1.0, embed=0.02):
     """Base weights by their names in the framework's model; `small` scales
     what the layers add to the embedding."""
     g, w = _gen(seed), {}
     W, ff = cfg.hidden_size, cfg.intermediate_size
     q, kv = cfg.num_heads * cfg.head_dim, cfg.num_kv_heads * cfg.head_dim
-    w["model.embed_tokens.weight"] = _randn(g, cfg.vocab_size, W, std=0.02)
+    w["model.embed_tokens.weight"] = _randn(g, cfg.vocab_size, W, std=embed)
     for i in range(cfg.num_layers):
         p = f"model.layers.{i}."
         w[p + "self_attn.qkv_proj.weight"] = _randn(g, q + 2 * kv, W, std=0.02)
@@ -269,7 +271,7 @@ def _prepare_score(case, seed):
     if case["model"] == "reward":
         cfg = get_config("rm-large", **_reward_config(case))
         s["model"] = _built(lambda: ScalarHeadModel(cfg))
-        w = _qwen_weights(cfg, seed)
+        w = _qwen_weights(cfg, seed, embed=0.5)     # scores tell the sequences apart
         w["score.weight"] = _randn(_gen(seed + 9), 1, cfg.hidden_size, std=0.03)
         s["model"].load_state_dict(w, strict=True)
     else:
@@ -632,8 +634,8 @@ def tolerance(case):
     kind = case["kind"]
     if kind == "train":           # gradients through the layers: 0.01 measured
         return {"rel": 0.03, "max": 0.9}
-    if kind == "score":           # 0.001 (log-probabilities) to 0.006 (scores)
-        return {"rel": 0.024, "max": 0.3}
+    if kind == "score":           # 0.001 (log-probabilities) to 0.011 (scores)
+        return {"rel": 0.03, "max": 0.3}
     if kind == "attention":       # 0.002 to 0.004
         return {"rel": 0.015, "max": 0.3}
     if kind == "decode":          # 0.002; in 8 bits the weights are rounded to 3 bits: 0.005
@@ -749,7 +751,7 @@ def _exact_score(case, seed):
     ids = torch.cat(seqs)
     if case["model"] == "reward":
         cfg = get_config("rm-large", **_reward_config(case))
-        h = _qwen64(cfg, _qwen_weights(cfg, seed), ids, lens)
+        h = _qwen64(cfg, _qwen_weights(cfg, seed, embed=0.5), ids, lens)
         head = _randn(_gen(seed + 9), 1, cfg.hidden_size, std=0.03).double()
         last = torch.tensor(lens, device="cuda").cumsum(0) - 1
         return dict(scores=(h[last] @ head.t())[:, 0])
