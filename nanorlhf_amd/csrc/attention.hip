@@ -1,20 +1,35 @@
 // Varlen causal flash attention, forward + backward, MFMA bf16 for gfx950.
 //
-// Forward (fa_fwd_varlen): one 256-thread workgroup (4 waves) per
-// (sequence, q-head, 64-row q-tile); each wave owns 16 q rows.  KV walks in
-// 32-token tiles staged cooperatively in LDS (K row-major for the QK^T
-// B-fragment, V transposed so the PV B-fragment is a contiguous
-// ds_read_b128).  QK^T and PV are v_mfma_f32_16x16x32_bf16; softmax is
-// online in fp32 with per-row running (m, s); P round-trips through a
-// per-wave LDS buffer to convert the C-layout into an A-fragment.
-// Returns (o, lse[T, Hq] fp32) — lse feeds the backward's P recompute.
+// Sequences are packed ([T, H, D] with cu_seqlens); a workgroup of four waves
+// owns 128 rows of one sequence and head, 32 per wave, and walks the other side
+// in tiles of 64 rows, which two LDS buffers receive by direct loads
+// (global_load_lds) while the tile before is computed on.
 //
-// Backward (fa_bwd_varlen): FA2 structure — one workgroup per (sequence,
-// kv-head, 32-token kv-tile); the G grouped q-heads x overlapping q-tiles
-// are strided across the 4 waves; dK/dV accumulate in AGPRs across the pair
-// loop and leave via fp32 atomics (workgroup-exclusive per kv tile, so only
-// the 4 waves contend); dQ contributions leave via fp32 atomics as in FA2.
-// dV/dK use v_mfma_f32_32x32x16_bf16 with P^T / dS^T staged per-wave.
+//   fa_fwd_kernel   rows of q; S^T = K Q^T, so a lane holds scores of ONE q
+//                   row and the online softmax is lane-local; O^T += V^T P^T
+//   fa_bwd_dq       rows of q; S^T and dP^T = V dO^T the same way, then
+//                   dQ^T += K^T dS^T
+//   fa_bwd_dkv      rows of k and v; S = Q K^T and dP = dO V^T, then
+//                   dV += P^T dO and dK += dS^T Q over all q heads of the group
+//
+// The backward runs S and dP twice (7 products instead of 5) and in return
+// has no atomics: dq, dk and dv are summed in registers in a fixed order and
+// written once.
+//
+// What bounds them: 16 MFMAs' worth of LDS reads (16 KB of fragments per 32 x 32
+// scores and two products) keep LDS as busy as the matrix cores, and the
+// exponentials take half as long as the products; two waves per SIMD overlap the
+// three.  5 causal sequences of about 6500 tokens, 12 heads over 2, width 128:
+// forward 1.1 ms (760 TFLOP/s), dq 1.3 ms, dk and dv 2.2 ms; before, with V
+// transposed by scalar LDS writes, 2.9 ms, and with dq added up by float atomics
+// over 32-row kv tiles, 21.5 ms for the backward.  Twice the rows per wave (half
+// the LDS reads, one wave per SIMD) was slower everywhere: forward 1.6 ms.
+//
+// Products contract over the MFMA's k index in any order as long as both
+// operands agree.  The C layout gives a lane the rows {0-3, 8-11} + 4 * half of
+// each 16, so a P or dS fragment is those registers converted in place, and the
+// other operand, a transposed LDS read of a row-major tile (ds_read_tr16_b64:
+// 16 lanes, 4 rows x 16 columns), simply starts at the same rows.
 //
 // Replaces the reference's flash_attention_2 dependency
 // (GRPO/grpo.py:219,223); packed varlen replaces its pad-mask forward
@@ -27,29 +42,8 @@
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-DEVINL f32x4 mfma16x16x32(bf16x8 a, bf16x8 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
 DEVINL f32x16_t mfma32x32x16(bf16x8 a, bf16x8 b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-
-DEVINL void lds_fence_wave() { lds_fence_wave_kv(); }
-
-// XOR-swizzled LDS element index for a [row][bytes-per-row] bf16 tile:
-// spreads each 16-B slot across bank columns (row-major D=128 tiles read
-// with ds_read_b128 are otherwise up to 16-way bank conflicts —
-// cdna_hip_programming.md §6 G4).  ROWBYTES must be a power of two >= 32.
-template <int ROWBYTES>
-DEVINL int swz_idx(int row, int byte_in_row) {
-  constexpr int MASK = (ROWBYTES / 16) - 1;
-  return row * (ROWBYTES / 2) + ((byte_in_row ^ ((row & MASK) << 4)) >> 1);
-}
-
-DEVINL __bf16 f2bf16t(float f) {
-  union { short s; __bf16 b; } u;
-  u.s = f2bf(f);
-  return u.b;
 }
 
 // pack two f32 into one dword of 2xbf16 (compiler emits v_cvt_pk_bf16_f32)
@@ -58,467 +52,493 @@ DEVINL unsigned pack2bf(float lo, float hi) {
   return *reinterpret_cast<unsigned*>(&h2);
 }
 
-// ======================================================= FORWARD (v2) ====
-// 8-wave structure (cdna_hip_programming.md Appendix B "fused attention
-// prefill" ladder): each of 8 waves owns QBLK=32 q rows; KV walks in
-// 64-token LDS tiles (double-buffered, XOR-swizzled, async-STAGE split).
-// QK^T is computed SWAPPED — S^T = mfma(K, Q^T) — so each lane holds the
-// whole 64-score P-row of ONE q row (split with its half-partner lane),
-// making the online softmax fully lane-local: 31 fmax + one
-// permlane32_swap per tile, no LDS round trip for P, defer-max rescale
-// (RESCALE_THRESHOLD=8; P bounded by e^8, bf16-safe; decision taken
-// BEFORE this tile's exponentiation — the textbook-safe order).
-// P→bf16 via v_cvt_pk packing + permlane32_swap builds the PV fragments
-// in registers, and PV is ALSO computed transposed — O^T = mfma(V^T, P^T)
-// — which lands each lane's O accumulator in its OWN q-row column, so the
-// rescale and the 1/s epilogue are lane-local too.
-template <int D, bool CAUSAL, int NW = 8>
-__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2)
-void fa_fwd_kernel8(const short* __restrict__ q,
-                    const short* __restrict__ k,
-                    const short* __restrict__ v,
-                    const int* __restrict__ cu,
-                    short* __restrict__ o,
-                    float* __restrict__ lse,
-                    int Hq, int Hkv, float scale) {
-  constexpr int QBLK = 32;            // q rows per wave
-  constexpr int QTILE = NW * QBLK;    // rows per workgroup
-  constexpr int NT = NW * 64;         // threads
-  constexpr int KVBLK = 64;
-  constexpr int NDS = D / 16;         // d-slots per QK^T chain
-  constexpr int NDT = D / 32;         // O d-tiles
-  constexpr float THR = 11.54f;       // defer-max threshold (8 nats, log2 units)
-  const int seq = blockIdx.y;
-  const int h = blockIdx.z;
-  const int kvh = h / (Hq / Hkv);
-  const int s0 = cu[seq], s1 = cu[seq + 1];
-  const int len = s1 - s0;
-  const int q0 = blockIdx.x * QTILE;
-  if (q0 >= len) return;
-  const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  const int col = lane & 31;          // this lane's q row within the wave blk
-  const int hi = lane >> 5;           // half-wave: which 8-kv slot of frags
-  const int qw0 = q0 + wid * QBLK;
-  const int qi = qw0 + col;           // lane's q row (sequence-local)
-  const bool row_ok = qi < len;
-  const bool wave_active = qw0 < len;
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr int TILE = 64;     // rows of the walked side per LDS tile
+constexpr int ROWS = 128;    // rows that a workgroup owns, 32 per wave
 
-  __shared__ short Kt[2][KVBLK * D];   // [tok][d], XOR-swizzled rows
-  __shared__ short Vt[2][D * KVBLK];   // [d][tok], XOR-swizzled rows
+// ---- LDS tiles: [row][D] bf16, 16-byte chunks XOR-swizzled by row ----------
+// 16 rows x one chunk (a fragment read along D) and 4 rows x 4 chunks (half a
+// transposed read) both have to touch all 64 banks once.  Rows 256 bytes apart
+// start at the same bank, so the row's low two bits move a chunk between the
+// groups of four that a transposed read takes, the next two within a group.
+template <int D>
+DEVINL int swz(int row) {
+  if constexpr (D == 128) return ((row & 3) << 2) | ((row >> 2) & 3);
+  else if constexpr (D == 64) return (((row >> 1) & 1) << 2) | ((row >> 2) & 3);
+  else return (row >> 2) & 3;
+}
 
-  // Q fragments (B-operand of the swapped QK^T): lane holds
-  // Q[qi][16*ds + 8*hi + j], j=0..7 — contiguous d, straight from global.
-  bf16x8 qf[NDS];
-  {
-    const long base = ((long)(s0 + min(qi, len - 1)) * Hq + h) * D;
+// 16 (or 4) bytes per lane from base + offset to LDS, lane after lane from `at`.
+// As assembly, because the compiler waits for a load that it knows to write LDS
+// before the next LDS read, whichever buffer that reads, and so undoes the
+// prefetch; there is no output register.  tiles_ready() does the waiting.
+DEVINL void load_to_lds16(const void* base, unsigned offset, const void* at) {
+  const unsigned l = __builtin_amdgcn_readfirstlane(
+      (unsigned)(size_t)(const __attribute__((address_space(3))) void*)at);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               ::"s"(l), "v"(offset), "s"(base) : "memory", "m0");
+}
+DEVINL void load_to_lds4(const void* base, unsigned offset, const void* at) {
+  const unsigned l = __builtin_amdgcn_readfirstlane(
+      (unsigned)(size_t)(const __attribute__((address_space(3))) void*)at);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+               ::"s"(l), "v"(offset), "s"(base) : "memory", "m0");
+}
+
+// All waves' loads into LDS have arrived, and nobody reads the buffer that is
+// filled next.
+DEVINL void tiles_ready() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
+// the TILE rows from src on (row stride `ld` elements; rows from `left` on
+// repeat the last) into a tile; a lane fetches the chunk that its 16 bytes of
+// the tile hold
+template <int D>
+DEVINL void stage_tile(const short* src, int ld, int left, const short* tile) {
+  constexpr int SLOTS = TILE * D / 8;
+  const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x) & ~63;
 #pragma unroll
-    for (int ds = 0; ds < NDS; ds++) {
-      s16x8 raw = *reinterpret_cast<const s16x8*>(q + base + 16 * ds + 8 * hi);
-      qf[ds] = *reinterpret_cast<bf16x8*>(&raw);
-    }
+  for (int i = 0; i < SLOTS; i += 256) {
+    const int idx = i + threadIdx.x;
+    const int row = idx / (D / 8), c = (idx % (D / 8)) ^ swz<D>(row);
+    load_to_lds16(src, (unsigned)(min(row, left - 1) * ld + c * 8) * 2, tile + (i + wave0) * 8);
   }
+}
 
-  float m = -INFINITY, s_ = 0.f;
-  f32x16_t acc_o[NDT];
+// 8 consecutive d (from 16 * ds + 8 * half) of row r0 + lane % 32
+template <int D>
+DEVINL bf16x8 row_frag(const short* tile, int r0, int ds, int lane) {
+  const int row = r0 + (lane & 31);
+  return *reinterpret_cast<const bf16x8*>(
+      tile + row * D + (((2 * ds + (lane >> 5)) ^ swz<D>(row)) << 3));
+}
+
+// column d0 + lane % 32, rows r0 + {0-3, 8-11} + 4 * half (r0 a multiple of 16)
+template <int D>
+DEVINL bf16x8 col_frag(const short* tile, int r0, int d0, int lane) {
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  const int i = lane & 15;
+  const int col = d0 + (lane & 16) + (i & 3) * 4;
+  union { s16x4 h[2]; bf16x8 f; } u;
 #pragma unroll
-  for (int t = 0; t < NDT; t++) acc_o[t] = f32x16_t{};
+  for (int p = 0; p < 2; p++) {
+    const int row = r0 + 8 * p + 4 * (lane >> 5) + (i >> 2);
+    const short* a = tile + row * D + (((col >> 3) ^ swz<D>(row)) << 3) + (col & 7);
+    u.h[p] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)a);
+  }
+  return u.f;
+}
 
-  const int kv_end = CAUSAL ? min(len, q0 + QTILE) : len;       // WG bound
-  const int kv_end_w = CAUSAL ? min(len, qw0 + QBLK) : len;     // wave bound
-
-  // async-STAGE split staging (issue-early / write-late): 16 B per thread
-  // per slice, 512 threads.
-  constexpr int CHUNKS = KVBLK * D / 8;          // 16-B chunks per K (or V) tile
-  constexpr int NSLICE = (CHUNKS + NT - 1) / NT;
-  s16x8 pk_[NSLICE], pv_[NSLICE];
-  auto issue_tile_loads = [&](int kv0) {
+// registers 8 * ks .. 8 * ks + 7 of a 32x32 result as a fragment of 16 rows
+DEVINL bf16x8 pack_frag(const float* p) {
+  union { unsigned u[4]; bf16x8 f; } fr;
 #pragma unroll
-    for (int sl = 0; sl < NSLICE; sl++) {
-      const int idx = threadIdx.x + sl * NT;
-      if (CHUNKS < NT && idx >= CHUNKS) continue;
-      const int tok = idx / (D / 8);
-      const int d0 = (idx % (D / 8)) * 8;
-      const int kvi = min(kv0 + tok, len - 1);
-      const long b = ((long)(s0 + kvi) * Hkv + kvh) * D + d0;
-      pk_[sl] = *reinterpret_cast<const s16x8*>(k + b);
-      pv_[sl] = *reinterpret_cast<const s16x8*>(v + b);
+  for (int j = 0; j < 4; j++) fr.u[j] = pack2bf(p[2 * j], p[2 * j + 1]);
+  return fr.f;
+}
+
+// row of register r of a 32x32 result in lane half `hi`
+DEVINL int crow(int r, int hi) { return (r & 3) + 8 * (r >> 2) + 4 * hi; }
+
+// fragments of a row that stays in registers, along D
+template <int D>
+DEVINL void load_row(const short* __restrict__ p, int hi, bf16x8* f) {
+#pragma unroll
+  for (int ds = 0; ds < D / 16; ds++)
+    f[ds] = *reinterpret_cast<const bf16x8*>(p + 16 * ds + 8 * hi);
+}
+
+DEVINL float other_half(float x, int hi) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(hi ? r[0] : r[1]);
+}
+
+// a lane's column of a transposed [D, 32] result as a bf16 row
+template <int D>
+DEVINL void store_row(short* __restrict__ dst, const f32x16_t* acc, float mul, int hi) {
+#pragma unroll
+  for (int c = 0; c < D / 32; c++)
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      union { unsigned u[2]; unsigned long long w; } o;
+      o.u[0] = pack2bf(acc[c][4 * g] * mul, acc[c][4 * g + 1] * mul);
+      o.u[1] = pack2bf(acc[c][4 * g + 2] * mul, acc[c][4 * g + 3] * mul);
+      *reinterpret_cast<unsigned long long*>(dst + 32 * c + 8 * g + 4 * hi) = o.w;
     }
-  };
-  auto write_tile_lds = [&](int buf) {
-#pragma unroll
-    for (int sl = 0; sl < NSLICE; sl++) {
-      const int idx = threadIdx.x + sl * NT;
-      if (CHUNKS < NT && idx >= CHUNKS) continue;
-      const int tok = idx / (D / 8);
-      const int d0 = (idx % (D / 8)) * 8;
-      *reinterpret_cast<s16x8*>(&Kt[buf][swz_idx<2 * D>(tok, d0 * 2)]) = pk_[sl];
-      // V fragment-major: slot (kv>>3, d) = V^T[d][8 contiguous kv] — PV
-      // reads walk consecutive slots per lane (conflict-free).  Measured
-      // wall-neutral vs the swizzled [d][kv] row image (288 vs 287 TF —
-      // the fwd is barrier/imbalance-bound, not LDS-bound); kept for the
-      // simpler addressing
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-        Vt[buf][(((tok >> 3) * D) + d0 + j) * 8 + (tok & 7)] = pv_[sl][j];
-    }
-  };
+}
 
-  if (kv_end > 0) issue_tile_loads(0);
+// Workgroups are ordered by tile first, the longest walks first: a causal
+// row tile's work grows with its index, a kv tile's shrinks.
+struct Place { int seq, head, s0, len, tile; };
+template <bool LAST_FIRST>
+DEVINL Place place(const int* __restrict__ cu, int heads) {
+  Place p;
+  p.seq = blockIdx.x / heads;
+  p.head = blockIdx.x % heads;
+  p.s0 = cu[p.seq];
+  p.len = cu[p.seq + 1] - p.s0;
+  p.tile = LAST_FIRST ? gridDim.y - 1 - blockIdx.y : blockIdx.y;
+  return p;
+}
+
+// ================================================================ FORWARD ==
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(256, 2)
+void fa_fwd_kernel(const short* __restrict__ q, const short* __restrict__ k,
+                   const short* __restrict__ v, const int* __restrict__ cu,
+                   short* __restrict__ o, float* __restrict__ lse, int Hq, int Hkv, float scale) {
+  constexpr int NDS = D / 16, NDT = D / 32;
+  constexpr float THR = 11.54f;       // rescale when a row grows past 8 nats (log2 units)
+  const Place pl = place<CAUSAL>(cu, Hq);
+  const int len = pl.len, h = pl.head, kvh = h / (Hq / Hkv);
+  const int q0 = pl.tile * ROWS;
+  if (q0 >= len) return;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hi = lane >> 5;
+  const int qw0 = q0 + wid * 32, qi = qw0 + (lane & 31);
+
+  __shared__ short lds[2][2][TILE * D];   // [buffer][K, V]
+
+  bf16x8 qf[NDS];
+  load_row<D>(q + ((long)(pl.s0 + min(qi, len - 1)) * Hq + h) * D, hi, qf);
+  float m = -INFINITY, sum = 0.f;
+  f32x16_t acc[NDT];
+#pragma unroll
+  for (int c = 0; c < NDT; c++) acc[c] = f32x16_t{};
+  const int ld = Hkv * D;
+  const short* kb = k + (long)pl.s0 * ld + kvh * D;
+  const short* vb = v + (long)pl.s0 * ld + kvh * D;
+  const int kv_end = CAUSAL ? min(len, q0 + ROWS) : len;
+  const int kv_end_w = qw0 >= len ? 0 : CAUSAL ? min(len, qw0 + 32) : len;
+  const float sl2 = scale * LOG2E;
+
+  stage_tile<D>(kb, ld, len, lds[0][0]);
+  stage_tile<D>(vb, ld, len, lds[0][1]);
   int buf = 0;
-  for (int kv0 = 0; kv0 < kv_end; kv0 += KVBLK, buf ^= 1) {
-    __syncthreads();          // prior readers of `buf` are done
-    write_tile_lds(buf);
-    __syncthreads();          // tile visible to all waves
-    if (kv0 + KVBLK < kv_end) issue_tile_loads(kv0 + KVBLK);
-    if (!wave_active || kv0 >= kv_end_w) continue;
+  for (int kv0 = 0; kv0 < kv_end; kv0 += TILE, buf ^= 1) {
+    tiles_ready();
+    if (kv0 + TILE < kv_end) {
+      stage_tile<D>(kb + (long)(kv0 + TILE) * ld, ld, len - kv0 - TILE, lds[buf ^ 1][0]);
+      stage_tile<D>(vb + (long)(kv0 + TILE) * ld, ld, len - kv0 - TILE, lds[buf ^ 1][1]);
+    }
+    if (kv0 >= kv_end_w) continue;
+    const short* Kt = lds[buf][0];
+    const short* Vt = lds[buf][1];
 
-    // ---- S^T = K · Q^T : two 32-kv subtiles, C col = own q row ----------
     f32x16_t st[2];
 #pragma unroll
     for (int sub = 0; sub < 2; sub++) {
       st[sub] = f32x16_t{};
 #pragma unroll
-      for (int ds = 0; ds < NDS; ds++) {
-        s16x8 rk = *reinterpret_cast<const s16x8*>(
-            &Kt[buf][swz_idx<2 * D>(sub * 32 + col, (16 * ds + 8 * hi) * 2)]);
-        st[sub] = mfma32x32x16(*reinterpret_cast<bf16x8*>(&rk), qf[ds], st[sub]);
+      for (int ds = 0; ds < NDS; ds++)
+        st[sub] = mfma32x32x16(row_frag<D>(Kt, 32 * sub, ds, lane), qf[ds], st[sub]);
+    }
+    // Scores stay as they are and meet scale * log2(e) in the exponent's fma
+    // (the softmax runs in base 2), which needs a positive scale.
+    float mul = sl2;
+    if (!(sl2 > 0.f)) {
+#pragma unroll
+      for (int r = 0; r < 32; r++) st[r >> 4][r & 15] *= sl2;
+      mul = 1.f;
+    }
+    if (!(kv0 + TILE <= len && (!CAUSAL || kv0 + TILE - 1 <= qw0))) {
+#pragma unroll
+      for (int r = 0; r < 32; r++) {
+        const int ki = kv0 + 32 * (r >> 4) + crow(r & 15, hi);
+        if (!(ki < len && (!CAUSAL || ki <= qi))) st[r >> 4][r & 15] = -INFINITY;
       }
     }
-    // ---- mask + scale: p[sub*16+r] is score for kv = kv0 + 32*sub +
-    //      crow(r,hi), crow = (r&3) + 8*(r>>2) + 4*hi, all for q row qi.
-    //      Scores carry scale*log2(e) so the softmax runs in base-2
-    //      (v_exp_f32 directly; saves one VALU mul per element) ---------
-    const float sl2 = scale * 1.4426950408889634f;
-    float p[32];
-    const bool full = row_ok && (kv0 + KVBLK <= len)
-                      && (!CAUSAL || kv0 + KVBLK - 1 <= qw0);
-    if (full) {
+    float top = st[0][0];
 #pragma unroll
-      for (int sub = 0; sub < 2; sub++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) p[sub * 16 + r] = st[sub][r] * sl2;
-    } else {
-#pragma unroll
-      for (int sub = 0; sub < 2; sub++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int ki = kv0 + 32 * sub + (r & 3) + 8 * (r >> 2) + 4 * hi;
-          const bool ok = row_ok && (ki < len) && (!CAUSAL || ki <= qi);
-          p[sub * 16 + r] = ok ? st[sub][r] * sl2 : -INFINITY;
-        }
-    }
-    // ---- lane-local row max (+ half-partner combine) --------------------
-    float pmax = p[0];
-#pragma unroll
-    for (int i = 1; i < 32; i++) pmax = fmaxf(pmax, p[i]);
-    {
-      auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(pmax),
-                                                 __float_as_uint(pmax), false, false);
-      const float partner = __uint_as_float(hi ? r2[0] : r2[1]);
-      pmax = fmaxf(pmax, partner);
-    }
-    // ---- defer-max: rescale only when some row grew past THR ------------
+    for (int r = 1; r < 32; r++) top = fmaxf(top, st[r >> 4][r & 15]);
+    top = fmaxf(top, other_half(top, hi)) * mul;
+    // rescale only when some row grew past THR (or has no maximum yet)
     float alpha = 1.f;
-    const bool need = row_ok && !(pmax - m <= THR);   // true on first tile (m=-inf)
-    if (__any(need)) {
-      const float mn = fmaxf(m, pmax);
+    if (__any(!(top - m <= THR))) {
+      const float mn = fmaxf(m, top);
       alpha = (m == -INFINITY) ? 0.f : exp2f(m - mn);
       m = mn;
 #pragma unroll
-      for (int t = 0; t < NDT; t++)
+      for (int c = 0; c < NDT; c++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc_o[t][r] *= alpha;
+        for (int r = 0; r < 16; r++) acc[c][r] *= alpha;
     }
-    // ---- P = exp(score - m), row sum ------------------------------------
-    float rs = 0.f;
+    const float mm = m == -INFINITY ? 0.f : m;   // a row that sees nothing so far
+    float p[32], rs = 0.f;
 #pragma unroll
-    for (int i = 0; i < 32; i++) {
-      p[i] = (p[i] > -INFINITY) ? exp2f(p[i] - m) : 0.f;
-      rs += p[i];
+    for (int r = 0; r < 32; r++) {
+      p[r] = __builtin_amdgcn_exp2f(fmaf(st[r >> 4][r & 15], mul, -mm));
+      rs += p[r];
     }
-    {
-      auto r2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(rs),
-                                                 __float_as_uint(rs), false, false);
-      rs += __uint_as_float(hi ? r2[0] : r2[1]);
-    }
-    s_ = s_ * alpha + rs;
-    // ---- P → bf16 PV fragments in registers (cvt_pk + permlane32_swap) --
-    // pa[ks] = P^T B-operand for kv slot ks: lane holds
-    // P[qi][16*ks + 8*hi + j], j=0..7.
-    bf16x8 pa[4];
+    sum = sum * alpha + rs + other_half(rs, hi);
 #pragma unroll
     for (int ks = 0; ks < 4; ks++) {
-      const int b0 = ks * 8;  // p-index base of this 8-kv group (own half)
-      unsigned w01 = pack2bf(p[b0 + 0], p[b0 + 1]);
-      unsigned w23 = pack2bf(p[b0 + 2], p[b0 + 3]);
-      unsigned w45 = pack2bf(p[b0 + 4], p[b0 + 5]);
-      unsigned w67 = pack2bf(p[b0 + 6], p[b0 + 7]);
-      auto rA = __builtin_amdgcn_permlane32_swap(w01, w45, false, false);
-      auto rB = __builtin_amdgcn_permlane32_swap(w23, w67, false, false);
-      union { unsigned u[4]; bf16x8 f; } fr;
-      fr.u[0] = (unsigned)rA[0];
-      fr.u[1] = (unsigned)rB[0];
-      fr.u[2] = (unsigned)rA[1];
-      fr.u[3] = (unsigned)rB[1];
-      pa[ks] = fr.f;
-    }
-    // ---- O^T += V^T · P^T : NDT d-tiles × 4 kv slots --------------------
+      const bf16x8 pf = pack_frag(p + 8 * ks);
 #pragma unroll
-    for (int t = 0; t < NDT; t++) {
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++) {
-        s16x8 rv = *reinterpret_cast<const s16x8*>(
-            &Vt[buf][((2 * ks + hi) * D + t * 32 + col) * 8]);
-        acc_o[t] = mfma32x32x16(*reinterpret_cast<bf16x8*>(&rv), pa[ks], acc_o[t]);
-      }
+      for (int c = 0; c < NDT; c++)
+        acc[c] = mfma32x32x16(col_frag<D>(Vt, 16 * ks, 32 * c, lane), pf, acc[c]);
     }
   }
-
-  if (!wave_active || !row_ok) return;
-  // ---- epilogue: O = O^T column / s, packed 8-B stores ------------------
-  const float inv = s_ > 0.f ? 1.f / s_ : 0.f;
-  const long obase = ((long)(s0 + qi) * Hq + h) * D;
-#pragma unroll
-  for (int t = 0; t < NDT; t++) {
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-      // regs 4g..4g+3 are d = t*32 + 8*g + 4*hi + (0..3) — contiguous
-      const int d0 = t * 32 + 8 * g + 4 * hi;
-      short pack[4];
-#pragma unroll
-      for (int j = 0; j < 4; j++) pack[j] = f2bf(acc_o[t][4 * g + j] * inv);
-      *reinterpret_cast<unsigned long long*>(o + obase + d0) =
-          *reinterpret_cast<const unsigned long long*>(pack);
-    }
-  }
+  if (qi >= len) return;
+  store_row<D>(o + ((long)(pl.s0 + qi) * Hq + h) * D, acc, sum > 0.f ? 1.f / sum : 0.f, hi);
   if (hi == 0)   // m is in log2 units: lse = ln2 * (m + log2 s)
-    lse[(long)(s0 + qi) * Hq + h] =
-        0.6931471805599453f * (m + log2f(fmaxf(s_, 1e-30f)));
+    lse[(long)(pl.s0 + qi) * Hq + h] = 0.6931471805599453f * (m + log2f(fmaxf(sum, 1e-30f)));
 }
 
-// ====================================================== BWD: D = rowsum ==
-__global__ void fa_bwd_preprocess_kernel(const short* __restrict__ dout,
-                                         const short* __restrict__ o,
-                                         float* __restrict__ drow,
-                                         int Hq, int D) {
-  const long row = blockIdx.x;  // t * Hq + h
-  const int lane = threadIdx.x;
-  const long base = row * D;
+// =============================================================== BACKWARD ==
+// rows [Hq, T]: -sum(dO * O), which dP starts from in the matrix product's
+// accumulator, and lse in log2 units.  16 lanes per row.
+template <int D>
+__global__ __launch_bounds__(256)
+void fa_bwd_rows_kernel(const short* __restrict__ dout, const short* __restrict__ o,
+                        const float* __restrict__ lse, float* __restrict__ drow,
+                        float* __restrict__ lse2, long T, int Hq) {
+  const long row = (long)blockIdx.x * 16 + (threadIdx.x >> 4);   // t * Hq + h
+  const int i = threadIdx.x & 15;
   float acc = 0.f;
-  for (int d = lane; d < D; d += 64)
-    acc += bf2f(dout[base + d]) * bf2f(o[base + d]);
-  acc = wave_sum(acc);
-  if (lane == 0) drow[row] = acc;
+  if (row < T * Hq) {
+    float a[D / 16], b[D / 16];
+    ldv<D / 16>(dout + row * D + i * (D / 16), a);
+    ldv<D / 16>(o + row * D + i * (D / 16), b);
+#pragma unroll
+    for (int j = 0; j < D / 16; j++) acc += a[j] * b[j];
+  }
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+  if (i == 0 && row < T * Hq) {
+    const long at = (row % Hq) * T + row / Hq;
+    drow[at] = -acc;
+    lse2[at] = lse[row] * LOG2E;
+  }
 }
 
-// =========================================================== BACKWARD ====
 template <int D, bool CAUSAL>
-__global__ __launch_bounds__(256, 2) void fa_bwd_kernel(const short* __restrict__ dout,
-                              const short* __restrict__ q,
-                              const short* __restrict__ k,
-                              const short* __restrict__ v,
-                              const float* __restrict__ lse,
-                              const float* __restrict__ drow,
-                              const int* __restrict__ cu,
-                              float* __restrict__ dqf,   // [T,Hq,D] f32
-                              float* __restrict__ dkf,   // [T,Hkv,D] f32
-                              float* __restrict__ dvf,
-                              int Hq, int Hkv, float scale) {
-  constexpr int KTILE = 32;
-  constexpr int NC = D / 32;
-  const int seq = blockIdx.y;
-  const int kvh = blockIdx.z;
-  const int G = Hq / Hkv;
-  const int s0 = cu[seq], s1 = cu[seq + 1];
-  const int len = s1 - s0;
-  const int kv0 = blockIdx.x * KTILE;
+__global__ __launch_bounds__(256, 2)
+void fa_bwd_dq_kernel(const short* __restrict__ dout, const short* __restrict__ q,
+                      const short* __restrict__ k, const short* __restrict__ v,
+                      const float* __restrict__ lse2, const float* __restrict__ drow,
+                      const int* __restrict__ cu, short* __restrict__ dq, long T, int Hq,
+                      int Hkv, float scale) {
+  constexpr int NDS = D / 16, NDT = D / 32;
+  const Place pl = place<CAUSAL>(cu, Hq);
+  const int len = pl.len, h = pl.head, kvh = h / (Hq / Hkv);
+  const int q0 = pl.tile * ROWS;
+  if (q0 >= len) return;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hi = lane >> 5;
+  const int qw0 = q0 + wid * 32, qi = qw0 + (lane & 31), qc = min(qi, len - 1);
+
+  __shared__ short lds[2][2][TILE * D];   // [buffer][K, V]
+
+  bf16x8 qf[NDS], dof[NDS];
+  const long base = ((long)(pl.s0 + qc) * Hq + h) * D;
+  load_row<D>(q + base, hi, qf);
+  load_row<D>(dout + base, hi, dof);
+  const float l2 = lse2[(long)h * T + pl.s0 + qc], dr = drow[(long)h * T + pl.s0 + qc];
+  f32x16_t acc[NDT];
+#pragma unroll
+  for (int c = 0; c < NDT; c++) acc[c] = f32x16_t{};
+  const int ld = Hkv * D;
+  const short* kb = k + (long)pl.s0 * ld + kvh * D;
+  const short* vb = v + (long)pl.s0 * ld + kvh * D;
+  const int kv_end = CAUSAL ? min(len, q0 + ROWS) : len;
+  const int kv_end_w = qw0 >= len ? 0 : CAUSAL ? min(len, qw0 + 32) : len;
+  const float sl2 = scale * LOG2E;
+
+  stage_tile<D>(kb, ld, len, lds[0][0]);
+  stage_tile<D>(vb, ld, len, lds[0][1]);
+  int buf = 0;
+  for (int kv0 = 0; kv0 < kv_end; kv0 += TILE, buf ^= 1) {
+    tiles_ready();
+    if (kv0 + TILE < kv_end) {
+      stage_tile<D>(kb + (long)(kv0 + TILE) * ld, ld, len - kv0 - TILE, lds[buf ^ 1][0]);
+      stage_tile<D>(vb + (long)(kv0 + TILE) * ld, ld, len - kv0 - TILE, lds[buf ^ 1][1]);
+    }
+    const short* Kt = lds[buf][0];
+    const short* Vt = lds[buf][1];
+#pragma unroll
+    for (int sub = 0; sub < 2; sub++) {
+      const int kv1 = kv0 + 32 * sub;
+      if (kv1 >= kv_end_w) continue;
+      f32x16_t st{}, dp;
+#pragma unroll
+      for (int r = 0; r < 16; r++) dp[r] = dr;
+#pragma unroll
+      for (int ds = 0; ds < NDS; ds++) {
+        st = mfma32x32x16(row_frag<D>(Kt, 32 * sub, ds, lane), qf[ds], st);
+        dp = mfma32x32x16(row_frag<D>(Vt, 32 * sub, ds, lane), dof[ds], dp);
+      }
+      float s[16];
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+        s[r] = __builtin_amdgcn_exp2f(fmaf(st[r], sl2, -l2)) * dp[r];
+      if (!(kv1 + 32 <= len && (!CAUSAL || kv1 + 31 <= qw0))) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int ki = kv1 + crow(r, hi);
+          if (!(ki < len && (!CAUSAL || ki <= qi))) s[r] = 0.f;
+        }
+      }
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++) {
+        const bf16x8 sf = pack_frag(s + 8 * ks);
+#pragma unroll
+        for (int c = 0; c < NDT; c++)
+          acc[c] = mfma32x32x16(col_frag<D>(Kt, 32 * sub + 16 * ks, 32 * c, lane), sf, acc[c]);
+      }
+    }
+  }
+  if (qi < len) store_row<D>(dq + ((long)(pl.s0 + qi) * Hq + h) * D, acc, scale, hi);
+}
+
+// blockIdx.x = (sequence, kv head, part); part p of `parts` sums over its share
+// of the group's q heads.  One part writes bf16 (dk, dv); several write float
+// partial sums [parts, T, Hkv, D] into dk, dv.
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(256, 2)
+void fa_bwd_dkv_kernel(const short* __restrict__ dout, const short* __restrict__ q,
+                       const short* __restrict__ k, const short* __restrict__ v,
+                       const float* __restrict__ lse2, const float* __restrict__ drow,
+                       const int* __restrict__ cu, void* __restrict__ dk,
+                       void* __restrict__ dv, long T, int Hq, int Hkv, int parts, float scale) {
+  constexpr int NDS = D / 16, NDT = D / 32;
+  const Place pl = place<false>(cu, Hkv * parts);
+  const int len = pl.len, kvh = pl.head / parts, part = pl.head % parts;
+  const int heads = Hq / Hkv / parts, h0 = kvh * (Hq / Hkv) + part * heads;
+  const int kv0 = pl.tile * ROWS;
   if (kv0 >= len) return;
-  const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  const int hi = lane >> 4, lo = lane & 15;
-  const int hi5 = lane >> 5, lo5 = lane & 31;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hi = lane >> 5;
+  const int kw0 = kv0 + wid * 32, ki = kw0 + (lane & 31);
 
-  // Staging layouts are FRAGMENT-MAJOR: each MFMA B/A fragment's 8
-  // contiguous elements are one 16-B LDS slot and the 32 (or 16) lanes of
-  // a fragment read CONSECUTIVE slots — the round-1 [row][col] images put
-  // 16-B reads at 32-B row strides, a 4-way bank conflict on every read
-  // (PMC: SQ_LDS_BANK_CONFLICT/SQ_LDS_IDX_ACTIVE = 0.505).
-  //   KT  [kv>>3][d][kv&7]      — dQ's B operand (8 kv per d row)
-  //   QT/dOT keep the [d][q] row image (scalar-transpose writes outnumber
-  //   the b128 reads 8:1 there — frag-major measured SLOWER from 8-way
-  //   write conflicts; A/B 2.32→3.01 ms)
-  //   PT/dST [q>>3][kv][q&7]    — dV/dK's A operands
-  //   dSb [kv>>3][q][kv&7]      — dQ's A operand
-  __shared__ short Kt[KTILE * D];     // [tok][d] (row-contig reads, swizzled)
-  __shared__ short KT[4 * D * 8];     // frag-major, dQ B operand
-  __shared__ short Vt[KTILE * D];     // [tok][d]
-  __shared__ short QT[4][D * 16];     // per-wave, frag-major
-  __shared__ short dOT[4][D * 16];    // per-wave, frag-major
-  __shared__ short PT[4][KTILE * 16];   // per-wave, frag-major
-  __shared__ short dSb[4][16 * KTILE];  // per-wave, frag-major
-  __shared__ short dST[4][KTILE * 16];  // per-wave, frag-major
+  __shared__ short lds[2][2][TILE * D];   // [buffer][Q, dO]
+  __shared__ float rows[2][2][TILE];      // [buffer][lse2, -sum(dO * O)]
 
-  // cooperative stage of K (both layouts) and V
-  for (int idx = threadIdx.x; idx < KTILE * D / 8; idx += 256) {
-    const int tok = idx / (D / 8);
-    const int d0 = (idx % (D / 8)) * 8;
-    const int kvi = kv0 + tok;
-    s16x8 kk{}, vv{};
-    if (kvi < len) {
-      const long b = ((long)(s0 + kvi) * Hkv + kvh) * D + d0;
-      kk = *reinterpret_cast<const s16x8*>(k + b);
-      vv = *reinterpret_cast<const s16x8*>(v + b);
-    }
-    *reinterpret_cast<s16x8*>(&Kt[swz_idx<2 * D>(tok, d0 * 2)]) = kk;
-    *reinterpret_cast<s16x8*>(&Vt[swz_idx<2 * D>(tok, d0 * 2)]) = vv;
+  bf16x8 kf[NDS], vf[NDS];
+  const long base = ((long)(pl.s0 + min(ki, len - 1)) * Hkv + kvh) * D;
+  load_row<D>(k + base, hi, kf);
+  load_row<D>(v + base, hi, vf);
+  f32x16_t adk[NDT], adv[NDT];
 #pragma unroll
-    for (int j = 0; j < 8; j++)
-      KT[(((tok >> 3) * D) + d0 + j) * 8 + (tok & 7)] = kk[j];
+  for (int c = 0; c < NDT; c++) adk[c] = adv[c] = f32x16_t{};
+  const int ld = Hq * D;
+  const int qstart = CAUSAL ? kv0 / TILE * TILE : 0;
+  const float sl2 = scale * LOG2E;
+  const bool wave_active = kw0 < len;
+
+  // (lse2 and drow too: through a register they would be waited for behind the tiles)
+  auto stage = [&](int h, int r0, int buf) {
+    const long at = (long)(pl.s0 + r0) * ld + h * D;
+    stage_tile<D>(q + at, ld, len - r0, lds[buf][0]);
+    stage_tile<D>(dout + at, ld, len - r0, lds[buf][1]);
+    if (wid < 2)
+      load_to_lds4((wid ? drow : lse2) + (long)h * T + pl.s0 + r0, 4 * min(lane, len - r0 - 1),
+                   rows[buf][wid]);
+  };
+  stage(h0, qstart, 0);
+  int h = h0, r0 = qstart, buf = 0;
+  for (; h < h0 + heads; buf ^= 1) {
+    tiles_ready();
+    int hn = h, rn = r0 + TILE;
+    if (rn >= len) { hn++; rn = qstart; }
+    if (hn < h0 + heads) stage(hn, rn, buf ^ 1);
+    const short* Qt = lds[buf][0];
+    const short* Ot = lds[buf][1];
+#pragma unroll
+    for (int sub = 0; sub < 2; sub++) {
+      const int q1 = r0 + 32 * sub;
+      if (!wave_active || q1 >= len || (CAUSAL && q1 + 31 < kw0)) continue;
+      const bool whole = q1 + 32 <= len && (!CAUSAL || kw0 + 31 <= q1);
+      // K, V and the sums fill the registers: addresses are made anew each time
+      // and phases kept apart, or fragments of K and V go to scratch memory
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      f32x16_t st{}, dp;
+#pragma unroll
+      for (int g = 0; g < 4; g++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) dp[4 * g + j] = rows[buf][1][32 * sub + 8 * g + 4 * hi + j];
+#pragma unroll
+      for (int ds = 0; ds < NDS; ds++) st = mfma32x32x16(row_frag<D>(Qt, 32 * sub, ds, ln), kf[ds], st);
+#pragma unroll
+      for (int ds = 0; ds < NDS; ds++) dp = mfma32x32x16(row_frag<D>(Ot, 32 * sub, ds, ln), vf[ds], dp);
+      __builtin_amdgcn_sched_barrier(0);
+      float p[16], s[16];
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const int at = 32 * sub + 8 * g + 4 * hi;
+        const f32x4 l4 = *reinterpret_cast<const f32x4*>(&rows[buf][0][at]);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int r = 4 * g + j;
+          p[r] = __builtin_amdgcn_exp2f(fmaf(st[r], sl2, -l4[j]));
+          s[r] = p[r] * dp[r];
+        }
+      }
+      if (!whole) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int qi = q1 + crow(r, hi);
+          if (!(qi < len && (!CAUSAL || ki <= qi))) p[r] = s[r] = 0.f;
+        }
+      }
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++) {
+        __builtin_amdgcn_sched_barrier(0);
+        const bf16x8 pf = pack_frag(p + 8 * ks), sf = pack_frag(s + 8 * ks);
+#pragma unroll
+        for (int c = 0; c < NDT; c++) {
+          adv[c] = mfma32x32x16(pf, col_frag<D>(Ot, 32 * sub + 16 * ks, 32 * c, ln), adv[c]);
+          adk[c] = mfma32x32x16(sf, col_frag<D>(Qt, 32 * sub + 16 * ks, 32 * c, ln), adk[c]);
+        }
+      }
+    }
+    h = hn;
+    r0 = rn;
   }
-  __syncthreads();
-
-  // dV/dK accumulators: 32x32 C tiles over D/32 column chunks
-  f32x16_t acc_dv[NC], acc_dk[NC];
 #pragma unroll
-  for (int c = 0; c < NC; c++) {
-    acc_dv[c] = f32x16_t{};
-    acc_dk[c] = f32x16_t{};
-  }
-
-  const int qt0 = CAUSAL ? (kv0 / 16) : 0;
-  const int nqt = (len + 15) / 16;
-  const int npairs = G * (nqt - qt0);
-
-  for (int p = wid; p < npairs; p += 4) {
-    const int g = p % G;
-    const int qt = qt0 + p / G;
-    const int h = kvh * G + g;
-    const int r0 = qt * 16;
-
-    // ---- load Q / dO fragments + stage transposed copies --------------
-    bf16x8 qfr[NC], dofr[NC];
-    {
-      const int qrow = r0 + lo;
-      const long base = ((long)(s0 + min(qrow, len - 1)) * Hq + h) * D;
-      const bool ok = qrow < len;
+  for (int r = 0; r < 16; r++) {
+    const int kr = kw0 + crow(r, hi);
+    if (kr >= len) continue;
+    const long at = (((long)part * T + pl.s0 + kr) * Hkv + kvh) * D + (lane & 31);
 #pragma unroll
-      for (int c = 0; c < NC; c++) {
-        s16x8 rq{}, rd{};
-        if (ok) {
-          rq = *reinterpret_cast<const s16x8*>(q + base + 32 * c + 8 * hi);
-          rd = *reinterpret_cast<const s16x8*>(dout + base + 32 * c + 8 * hi);
-        }
-        qfr[c] = *reinterpret_cast<bf16x8*>(&rq);
-        dofr[c] = *reinterpret_cast<bf16x8*>(&rd);
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-          QT[wid][swz_idx<32>(32 * c + 8 * hi + j, lo * 2)] = rq[j];
-          dOT[wid][swz_idx<32>(32 * c + 8 * hi + j, lo * 2)] = rd[j];
-        }
-      }
-    }
-
-    // ---- S and dP (both 16x32, C layout row=q col=kv) ------------------
-    f32x4 sc[2], dp[2];
-#pragma unroll
-    for (int n = 0; n < 2; n++) {
-      sc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-      dp[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        s16x8 rk = *reinterpret_cast<const s16x8*>(
-            &Kt[swz_idx<2 * D>(16 * n + lo, 64 * c + 16 * hi)]);
-        s16x8 rv = *reinterpret_cast<const s16x8*>(
-            &Vt[swz_idx<2 * D>(16 * n + lo, 64 * c + 16 * hi)]);
-        sc[n] = mfma16x16x32(qfr[c], *reinterpret_cast<bf16x8*>(&rk), sc[n]);
-        dp[n] = mfma16x16x32(dofr[c], *reinterpret_cast<bf16x8*>(&rv), dp[n]);
-      }
-    }
-
-    // ---- P, dS (fp32, C layout) + stage P^T / dS / dS^T ----------------
-    // base-2 domain: P = 2^(S·scale·log2e − lse·log2e) (v_exp_f32 direct)
-    const float sl2 = scale * 1.4426950408889634f;
-#pragma unroll
-    for (int n = 0; n < 2; n++) {
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int qi = r0 + 4 * hi + r;
-        const int ki = kv0 + 16 * n + lo;
-        const bool ok = (qi < len) && (ki < len) && (!CAUSAL || ki <= qi);
-        float pv = 0.f, dsv = 0.f;
-        if (ok) {
-          const long li = (long)(s0 + qi) * Hq + h;
-          pv = exp2f(fmaf(sc[n][r], sl2, -lse[li] * 1.4426950408889634f));
-          dsv = pv * (dp[n][r] - drow[li]) * scale;
-        }
-        {
-          const int qq = 4 * hi + r, kv = 16 * n + lo;
-          const int pt_off = ((qq >> 3) * KTILE + kv) * 8 + (qq & 7);
-          PT[wid][pt_off] = f2bf(pv);
-          dST[wid][pt_off] = f2bf(dsv);
-          dSb[wid][((kv >> 3) * 16 + qq) * 8 + (kv & 7)] = f2bf(dsv);
-        }
-      }
-    }
-    lds_fence_wave();
-
-    // ---- dV += P^T dO ; dK += dS^T Q (32x32x16, K = 16 q rows) ---------
-    {
-      s16x8 rp = *reinterpret_cast<const s16x8*>(
-          &PT[wid][(hi5 * KTILE + lo5) * 8]);
-      s16x8 rs = *reinterpret_cast<const s16x8*>(
-          &dST[wid][(hi5 * KTILE + lo5) * 8]);
-      bf16x8 pA = *reinterpret_cast<bf16x8*>(&rp);
-      bf16x8 sA = *reinterpret_cast<bf16x8*>(&rs);
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        s16x8 rdo = *reinterpret_cast<const s16x8*>(
-            &dOT[wid][swz_idx<32>(32 * c + lo5, 16 * hi5)]);
-        s16x8 rqt = *reinterpret_cast<const s16x8*>(
-            &QT[wid][swz_idx<32>(32 * c + lo5, 16 * hi5)]);
-        acc_dv[c] = mfma32x32x16(pA, *reinterpret_cast<bf16x8*>(&rdo), acc_dv[c]);
-        acc_dk[c] = mfma32x32x16(sA, *reinterpret_cast<bf16x8*>(&rqt), acc_dk[c]);
-      }
-    }
-
-    // ---- dQ = dS K (16x16x32 over d tiles) -----------------------------
-    {
-      s16x8 rds = *reinterpret_cast<const s16x8*>(
-          &dSb[wid][(hi * 16 + lo) * 8]);
-      bf16x8 dsA = *reinterpret_cast<bf16x8*>(&rds);
-#pragma unroll
-      for (int t = 0; t < D / 16; t++) {
-        s16x8 rkt = *reinterpret_cast<const s16x8*>(
-            &KT[(hi * D + t * 16 + lo) * 8]);
-        f32x4 dq = mfma16x16x32(dsA, *reinterpret_cast<bf16x8*>(&rkt), f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int qi = r0 + 4 * hi + r;
-          if (qi < len)
-            atomicAdd(&dqf[((long)(s0 + qi) * Hq + h) * D + t * 16 + lo], dq[r]);
-        }
+    for (int c = 0; c < NDT; c++) {
+      if (parts == 1) {
+        ((short*)dk)[at + 32 * c] = f2bf(adk[c][r] * scale);
+        ((short*)dv)[at + 32 * c] = f2bf(adv[c][r]);
+      } else {
+        ((float*)dk)[at + 32 * c] = adk[c][r] * scale;
+        ((float*)dv)[at + 32 * c] = adv[c][r];
       }
     }
   }
+}
 
-  // ---- drain dV/dK (32x32 C layout: row=kv, col=d) ----------------------
+// sums of the parts, in order; n elements each, 4 per thread; y = 0: dk, 1: dv
+__global__ void fa_bwd_sum_kernel(const float* __restrict__ part, short* __restrict__ dk,
+                                  short* __restrict__ dv, long n, int parts) {
+  const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (i >= n) return;
+  const float* p = part + (blockIdx.y ? (long)parts * n : 0) + i;
+  f32x4 s = *reinterpret_cast<const f32x4*>(p);
+  for (int k = 1; k < parts; k++) s += *reinterpret_cast<const f32x4*>(p + k * n);
+  s16x4 o;
 #pragma unroll
-  for (int c = 0; c < NC; c++) {
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int kvi = kv0 + (r & 3) + 8 * (r >> 2) + 4 * hi5;
-      const int d = 32 * c + lo5;
-      if (kvi < len) {
-        const long b = ((long)(s0 + kvi) * Hkv + kvh) * D + d;
-        atomicAdd(&dvf[b], acc_dv[c][r]);
-        atomicAdd(&dkf[b], acc_dk[c][r]);
-      }
-    }
-  }
+  for (int j = 0; j < 4; j++) o[j] = f2bf(s[j]);
+  *reinterpret_cast<s16x4*>((blockIdx.y ? dv : dk) + i) = o;
 }
 
 // ======================================================== host wrappers ==
+#define FA_BY_WIDTH(CALL)                                                  \
+  do {                                                                     \
+    if (D == 128) { if (causal) CALL(128, true); else CALL(128, false); }  \
+    else if (D == 64) { if (causal) CALL(64, true); else CALL(64, false); } \
+    else if (D == 32) { if (causal) CALL(32, true); else CALL(32, false); } \
+    else TORCH_CHECK(false, "unsupported head_dim ", D);                   \
+  } while (0)
+
 std::vector<torch::Tensor> fa_fwd_varlen(torch::Tensor q, torch::Tensor k,
                                          torch::Tensor v, torch::Tensor cu_seqlens,
                                          long max_seqlen, double scale, bool causal) {
@@ -530,30 +550,15 @@ std::vector<torch::Tensor> fa_fwd_varlen(torch::Tensor q, torch::Tensor k,
   auto o = torch::empty_like(q);
   auto lse = torch::empty({T, Hq}, q.options().dtype(torch::kFloat32));
   if (T == 0) return {o, lse};
-  // 8-wave default: the 4-wave/2-block variant A/B-measured SLOWER at
-  // every shape (244 vs 287 TF at the scoring bucket) — cross-block
-  // overlap does not make up for the extra per-thread staging work.
-  static const int NW = [] {
-    const char* e = getenv("NANORLHF_FA_NW");
-    return (e && atoi(e) == 4) ? 4 : 8;
-  }();
-  const int qtile = NW * 32;
-  const int qtiles = (int)((max_seqlen + qtile - 1) / qtile);
-  dim3 grid(qtiles, B, Hq), block(NW * 64);
   auto stream = at::hip::getCurrentHIPStream();
-#define FWD_LAUNCH(DD, CC, NWW)                                                \
-  hipLaunchKernelGGL((fa_fwd_kernel8<DD, CC, NWW>), grid, block, 0, stream,    \
+  const dim3 grid(B * Hq, (max_seqlen + ROWS - 1) / ROWS);
+#define CALL(DD, CC)                                                           \
+  hipLaunchKernelGGL((fa_fwd_kernel<DD, CC>), grid, dim3(256), 0, stream,      \
                      (const short*)q.data_ptr(), (const short*)k.data_ptr(),   \
                      (const short*)v.data_ptr(), cu_seqlens.data_ptr<int>(),   \
-                     (short*)o.data_ptr(), lse.data_ptr<float>(), Hq, Hkv,     \
-                     (float)scale)
-#define FWD_D(DD, CC) do { if (NW == 8) FWD_LAUNCH(DD, CC, 8); else FWD_LAUNCH(DD, CC, 4); } while (0)
-  if (D == 128) { if (causal) FWD_D(128, true); else FWD_D(128, false); }
-  else if (D == 64) { if (causal) FWD_D(64, true); else FWD_D(64, false); }
-  else if (D == 32) { if (causal) FWD_D(32, true); else FWD_D(32, false); }
-  else TORCH_CHECK(false, "unsupported head_dim ", D);
-#undef FWD_D
-#undef FWD_LAUNCH
+                     (short*)o.data_ptr(), lse.data_ptr<float>(), Hq, Hkv, (float)scale)
+  FA_BY_WIDTH(CALL);
+#undef CALL
   HIP_CHECK_LAST();
   return {o, lse};
 }
@@ -565,34 +570,51 @@ std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
                                          double scale, bool causal) {
   TORCH_CHECK(dout.scalar_type() == torch::kBFloat16 && dout.is_contiguous());
   const long T = q.size(0);
-  const int Hq = q.size(1), D = q.size(2), Hkv = k.size(1);
+  const int Hq = q.size(1), D = q.size(2), Hkv = k.size(1), G = Hq / Hkv;
   const int B = cu_seqlens.size(0) - 1;
-  auto opts = q.options().dtype(torch::kFloat32);
-  auto dqf = torch::zeros({T, (long)Hq, (long)D}, opts);
-  auto dkf = torch::zeros({T, (long)Hkv, (long)D}, opts);
-  auto dvf = torch::zeros({T, (long)Hkv, (long)D}, opts);
-  if (T == 0) return {dqf.to(torch::kBFloat16), dkf.to(torch::kBFloat16),
-                      dvf.to(torch::kBFloat16)};
-  auto drow = torch::empty({T, (long)Hq}, opts);
+  auto dq = torch::empty_like(q), dk = torch::empty_like(k), dv = torch::empty_like(v);
+  if (T == 0) return {dq, dk, dv};
+  auto f32 = q.options().dtype(torch::kFloat32);
+  auto rows = torch::empty({2, (long)Hq, T}, f32);    // -sum(dO * O), lse in log2 units
+  float* drow = rows.data_ptr<float>();
+  float* lse2 = drow + (long)Hq * T;
+  // A workgroup of dk and dv walks the group's q heads one after the other.
+  // Where that leaves too few to fill 256 CUs twice, with spare to even out
+  // causal tiles, they are divided among `parts`.  Whole backward, 12 heads over
+  // 2: 5 x 6500 tokens (518 workgroups undivided) 4.23 ms with 1 part, 3.15 with
+  // 2, 3.07 with 3; 56 x 870 (872) 0.77 with 1, 0.81 with 2, 0.95 with 6.
+  int parts = 1;
+  const long tiles = (T / ROWS + B) * Hkv;
+  while (parts < G && (G % parts || tiles * parts < 768)) parts++;
+  const long n = T * Hkv * D;
+  torch::Tensor sums;
+  if (parts > 1) sums = torch::empty({2, (long)parts, n}, f32);
+  void* dkp = parts > 1 ? (void*)sums.data_ptr<float>() : dk.data_ptr();
+  void* dvp = parts > 1 ? (void*)(sums.data_ptr<float>() + parts * n) : dv.data_ptr();
   auto stream = at::hip::getCurrentHIPStream();
-  hipLaunchKernelGGL(fa_bwd_preprocess_kernel, dim3(T * Hq), dim3(64), 0, stream,
-                     (const short*)dout.data_ptr(), (const short*)o.data_ptr(),
-                     drow.data_ptr<float>(), Hq, D);
-  const int kvtiles = (int)((max_seqlen + 31) / 32);
-  dim3 grid(kvtiles, B, Hkv), block(256);
-#define BWD_LAUNCH(DD, CC)                                                     \
-  hipLaunchKernelGGL((fa_bwd_kernel<DD, CC>), grid, block, 0, stream,          \
-                     (const short*)dout.data_ptr(), (const short*)q.data_ptr(),\
-                     (const short*)k.data_ptr(), (const short*)v.data_ptr(),   \
-                     lse.data_ptr<float>(), drow.data_ptr<float>(),            \
-                     cu_seqlens.data_ptr<int>(), dqf.data_ptr<float>(),        \
-                     dkf.data_ptr<float>(), dvf.data_ptr<float>(), Hq, Hkv,    \
-                     (float)scale)
-  if (D == 128) { if (causal) BWD_LAUNCH(128, true); else BWD_LAUNCH(128, false); }
-  else if (D == 64) { if (causal) BWD_LAUNCH(64, true); else BWD_LAUNCH(64, false); }
-  else if (D == 32) { if (causal) BWD_LAUNCH(32, true); else BWD_LAUNCH(32, false); }
-  else TORCH_CHECK(false, "unsupported head_dim ", D);
-#undef BWD_LAUNCH
+  const int row_tiles = (max_seqlen + ROWS - 1) / ROWS;
+#define CALL(DD, CC)                                                           \
+  do {                                                                         \
+    hipLaunchKernelGGL(fa_bwd_rows_kernel<DD>, dim3((T * Hq + 15) / 16), dim3(256), 0, stream, \
+                       (const short*)dout.data_ptr(), (const short*)o.data_ptr(), \
+                       lse.data_ptr<float>(), drow, lse2, T, Hq);              \
+    hipLaunchKernelGGL((fa_bwd_dq_kernel<DD, CC>), dim3(B * Hq, row_tiles), dim3(256), 0, stream, \
+                       (const short*)dout.data_ptr(), (const short*)q.data_ptr(), \
+                       (const short*)k.data_ptr(), (const short*)v.data_ptr(), \
+                       lse2, drow, cu_seqlens.data_ptr<int>(), (short*)dq.data_ptr(), \
+                       T, Hq, Hkv, (float)scale);                              \
+    hipLaunchKernelGGL((fa_bwd_dkv_kernel<DD, CC>), dim3(B * Hkv * parts, row_tiles), dim3(256), \
+                       0, stream, (const short*)dout.data_ptr(),               \
+                       (const short*)q.data_ptr(), (const short*)k.data_ptr(), \
+                       (const short*)v.data_ptr(), lse2, drow,                 \
+                       cu_seqlens.data_ptr<int>(), dkp, dvp, T, Hq, Hkv, parts, (float)scale); \
+  } while (0)
+  FA_BY_WIDTH(CALL);
+#undef CALL
+  if (parts > 1)
+    hipLaunchKernelGGL(fa_bwd_sum_kernel, dim3((n / 4 + 255) / 256, 2), dim3(256), 0, stream,
+                       sums.data_ptr<float>(), (short*)dk.data_ptr(), (short*)dv.data_ptr(), n,
+                       parts);
   HIP_CHECK_LAST();
-  return {dqf.to(torch::kBFloat16), dkf.to(torch::kBFloat16), dvf.to(torch::kBFloat16)};
+  return {dq, dk, dv};
 }
