@@ -5,13 +5,12 @@
 // tokens) is a contiguous 16-B load.  page_size MUST be 16 (one MFMA
 // half-K per page half).
 //
-// paged_attn_decode: one 256-thread workgroup (4 waves) per (sequence,
-// kv-head).  The G <= 16 grouped query heads form the 16-row M dimension of
-// v_mfma_f32_16x16x32_bf16 tiles; each wave walks 32-token KV tiles with
-// stride 4, doing QK^T and PV on matrix cores with fp32 online softmax
-// (the first rocprof profile showed the scalar-dot version VALU-bound at
-// ~0.3 TB/s — MFMA moves the arithmetic off the VALU so the kernel can run
-// at the KV stream's memory bound).  Cross-wave states merge through LDS.
+// paged_attn_decode: one 256-thread workgroup (4 waves) per (sequence, kv-head,
+// split of the context).  The G <= 16 grouped query heads are the 16 columns of
+// v_mfma_f32_16x16x32 tiles (S^T = K Q^T, O^T += V^T P^T), so a lane's scores
+// are all of one head and the online softmax needs two exchanges between lanes;
+// each wave walks 32-token KV tiles with stride 4.  Waves merge through LDS,
+// splits through a second small kernel.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -35,34 +34,6 @@ DEVINL unsigned char f32_to_fp8(float x) {
   return (unsigned char)(__builtin_amdgcn_cvt_pk_fp8_f32(x, x, 0, false) & 0xff);
 }
 
-// load 8 cache elements starting at element index `idx` as a bf16 MFMA frag
-DEVINL bf16x8k load_frag_bf16(const short* base, long idx) {
-  s16x8 raw = *reinterpret_cast<const s16x8*>(base + idx);
-  return *reinterpret_cast<bf16x8k*>(&raw);
-}
-
-DEVINL bf16x8k load_frag_fp8(const unsigned char* base, long idx) {
-  i32x2k w = *reinterpret_cast<const i32x2k*>(base + idx);  // 8 bytes
-  float f[8];
-  f[0] = __builtin_amdgcn_cvt_f32_fp8(w[0], 0);
-  f[1] = __builtin_amdgcn_cvt_f32_fp8(w[0], 1);
-  f[2] = __builtin_amdgcn_cvt_f32_fp8(w[0], 2);
-  f[3] = __builtin_amdgcn_cvt_f32_fp8(w[0], 3);
-  f[4] = __builtin_amdgcn_cvt_f32_fp8(w[1], 0);
-  f[5] = __builtin_amdgcn_cvt_f32_fp8(w[1], 1);
-  f[6] = __builtin_amdgcn_cvt_f32_fp8(w[1], 2);
-  f[7] = __builtin_amdgcn_cvt_f32_fp8(w[1], 3);
-  s16x8 raw;
-#pragma unroll
-  for (int j = 0; j < 8; j++) raw[j] = f2bf(f[j]);
-  return *reinterpret_cast<bf16x8k*>(&raw);
-}
-
-DEVINL long load_frag8_raw(const unsigned char* base, long idx) {
-  i32x2k w = *reinterpret_cast<const i32x2k*>(base + idx);
-  return *reinterpret_cast<long*>(&w);
-}
-
 // quantize 8 f32 to 8 packed fp8 bytes (for Q / P operands on the fp8 path)
 DEVINL long pack8_fp8(const float* f) {
   int w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
@@ -73,17 +44,6 @@ DEVINL long pack8_fp8(const float* f) {
   w[0] = w0;
   w[1] = w1;
   return *reinterpret_cast<long*>(&w);
-}
-
-template <typename CT>
-DEVINL bf16x8k load_kv_frag(const CT* base, long idx);
-template <>
-DEVINL bf16x8k load_kv_frag<short>(const short* base, long idx) {
-  return load_frag_bf16(base, idx);
-}
-template <>
-DEVINL bf16x8k load_kv_frag<unsigned char>(const unsigned char* base, long idx) {
-  return load_frag_fp8(base, idx);
 }
 
 // ------------------------------------------------------------- kv append
@@ -172,246 +132,347 @@ struct DecodeExt {
   int gchunks;       // query-head groups of 16 per kv head
 };
 
-template <int D, int DV, typename CT, bool EXT>
-__global__ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
-                                    const CT* __restrict__ kc,      // [P, 16, Hkv, D]
-                                    const CT* __restrict__ vc,      // [P, Hkv, DV, 16]
-                                    const int* __restrict__ bt,     // [B, maxP]
-                                    const int* __restrict__ seq_lens,
-                                    short* __restrict__ out,        // [B, Hq, DV]
-                                    int Hq, int Hkv, int maxP, int Gq, float scale,
-                                    DecodeExt ext) {
-  constexpr int NC = D / 32;
-  constexpr int PS = 16;
-  const int unit = EXT ? blockIdx.x / ext.gchunks : blockIdx.x;
-  const int gc = EXT ? blockIdx.x % ext.gchunks : 0;
-  const int b = unit / Hkv;
-  const int kvh = unit % Hkv;
-  const int G = EXT ? min(16, Gq - 16 * gc) : Gq;   // heads of this workgroup
-  const int L = seq_lens[b];
-  const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  const int hi = lane >> 4, lo = lane & 15;
-  const int h0 = kvh * Gq + 16 * gc;
-
-  __shared__ short Pb[4][16 * 32];          // per-wave P [g][tok] (bf16)
-  __shared__ unsigned char Pb8[4][16 * 32]; // per-wave P (fp8 path)
-  __shared__ float Lm[4][16], Ls[4][16];    // per-wave (m, s) per row
-  __shared__ float Lacc[4][16][DV];         // per-wave O accumulators
-
-  // Q fragment: lane holds Q[g = lo][32c + 8hi + j]; zero for g >= G.
-  // On the fp8 cache path Q is quantized to e4m3 once here and the QK^T
-  // runs on mfma_f32_16x16x32_fp8_fp8 — K-cache bytes feed the MFMA
-  // directly (no dequant pass), doubling matrix throughput on top of the
-  // halved KV stream.
-  constexpr bool FP8 = sizeof(CT) == 1;
-  bf16x8k qf[NC];
-  long qf8[NC];
-  {
-    const int g = lo;
-    const long base = ((long)b * Hq + h0 + min(g, G - 1)) * D;
+// What bounds it: reading the cache.  K of the next tile and V of this one are
+// in flight while a tile's scores are worked on; a wave that asked for its page,
+// its K and its V one after the other had 5 us per tile of 32 tokens to wait.
+// 16 tokens of two pages, as MFMA fragments
+template <int D, typename CT>
+struct KTile {
+  static constexpr int BYTES = D * (int)sizeof(CT) / 4;          // per lane and 16 tokens
+  static constexpr int NV = BYTES >= 16 ? BYTES / 16 : 1;
+  i32x4k r[2][NV];
+  // lane (hi, lo): token lo of page n; bf16: elements 32c + 8hi .. + 7 of every
+  // c, fp8: the fragment-major D / 4 bytes of hi
+  DEVINL void load(const CT* kc, int page0, int page1, int Hkv, int kvh, int lo, int hi) {
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-      s16x8 raw{};
-      if (g < G)
-        raw = *reinterpret_cast<const s16x8*>(q + base + 32 * c + 8 * hi);
-      qf[c] = *reinterpret_cast<bf16x8k*>(&raw);
-      if (FP8) {
-        float f[8];
+    for (int n = 0; n < 2; n++) {
+      const CT* row = kc + (((long)(n ? page1 : page0) * 16 + lo) * Hkv + kvh) * D;
+      if constexpr (sizeof(CT) == 2) {
 #pragma unroll
-        for (int j = 0; j < 8; j++) f[j] = bf2f(raw[j]);
-        qf8[c] = pack8_fp8(f);
+        for (int c = 0; c < NV; c++)
+          r[n][c] = *reinterpret_cast<const i32x4k*>(row + 32 * c + 8 * hi);
+      } else if constexpr (BYTES >= 16) {
+#pragma unroll
+        for (int c = 0; c < NV; c++)
+          r[n][c] = *reinterpret_cast<const i32x4k*>(row + hi * (D / 4) + 16 * c);
+      } else {
+        const i32x2k w = *reinterpret_cast<const i32x2k*>(row + hi * (D / 4));
+        r[n][0] = i32x4k{w[0], w[1], 0, 0};
       }
     }
   }
+};
 
-  float m[4], s_[4];
-  f32x4 acc_o[DV / 16];
-#pragma unroll
-  for (int r = 0; r < 4; r++) { m[r] = -INFINITY; s_[r] = 0.f; }
-#pragma unroll
-  for (int t = 0; t < DV / 16; t++) acc_o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+// a, b hold, in the lanes of group hi (of four), something of tokens 4 * hi ..
+// + 3 of the first and of the second page; afterwards of tokens 8 * hi .. + 3 and
+// 8 * hi + 4 .. + 7 of the 32
+DEVINL void tokens_to_k(unsigned& a, unsigned& b) {
+  auto x = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  auto y = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+  a = y[0];
+  b = y[1];
+}
 
-  // tiles with a visible key: those of the kept first tokens, then the window's
-  const int win_lo = EXT ? max(0, L - ext.size) : 0;
-  const int win_tile = win_lo / 32;
-  const int kept_tiles = EXT ? min((ext.keep + 31) / 32, win_tile) : 0;
-  const int ntiles = kept_tiles + (L + 31) / 32 - win_tile;
+// over the four groups of 16 lanes
+DEVINL float max_groups(float x) {
+  x = fmaxf(x, __shfl_xor(x, 16));
+  return fmaxf(x, __shfl_xor(x, 32));
+}
+DEVINL float sum_groups(float x) {
+  x += __shfl_xor(x, 16);
+  return x + __shfl_xor(x, 32);
+}
+
+// tiles of 32 tokens with a visible key: those of the kept first tokens, then
+// the window's
+struct TileRange { int win_lo, win_tile, kept, n; };
+template <bool EXT>
+DEVINL TileRange tile_range(int L, const DecodeExt& ext) {
+  TileRange t;
+  t.win_lo = EXT ? max(0, L - ext.size) : 0;
+  t.win_tile = t.win_lo / 32;
+  t.kept = EXT ? min((ext.keep + 31) / 32, t.win_tile) : 0;
+  t.n = t.kept + (L + 31) / 32 - t.win_tile;
+  return t;
+}
+
+// o[0], o[1] at columns d, d + 1 of head h of row b, times inv, turned back if asked
+template <bool EXT>
+DEVINL void write_pair(short* out, float o0, float o1, int b, int h, int d, int Hq, int DV,
+                       const DecodeExt& ext) {
+  if constexpr (EXT) {
+    if (ext.uncs && d < ext.V) {
+      const float* cs = ext.uncs + (long)b * ext.V;
+      const float c = cs[d >> 1], s = cs[ext.V / 2 + (d >> 1)];
+      const float t = o0 * c + o1 * s;
+      o1 = o1 * c - o0 * s;
+      o0 = t;
+    }
+    short* op = out + (long)b * ext.ldo + (long)h * ext.V + d;
+    if (d < ext.V) op[0] = f2bf(o0);
+    if (d + 1 < ext.V) op[1] = f2bf(o1);
+  } else {
+    const unsigned w = (unsigned)(unsigned short)f2bf(o0) | (unsigned)(unsigned short)f2bf(o1) << 16;
+    *reinterpret_cast<unsigned*>(out + ((long)b * Hq + h) * DV + d) = w;
+  }
+}
+
+// blockIdx.x = (sequence, kv head, head group), blockIdx.y = split: tiles from
+// y * per_split on.  The result of a sequence that fits one split goes to `out`,
+// else the sums and (m, s) of each head to part [x, splits, 16, DV] and
+// ms [x, splits, 16, 2].
+template <int D, int DV, typename CT, bool EXT>
+__global__ __launch_bounds__(256)
+void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
+                         const CT* __restrict__ kc,      // [P, 16, Hkv, D]
+                         const CT* __restrict__ vc,      // [P, Hkv, DV, 16]
+                         const int* __restrict__ bt,     // [B, maxP]
+                         const int* __restrict__ seq_lens,
+                         short* __restrict__ out,        // [B, Hq, DV]
+                         float* __restrict__ part, float* __restrict__ ms,
+                         int Hq, int Hkv, int maxP, int Gq, int per_split, float scale,
+                         DecodeExt ext) {
+  constexpr int NC = D / 32, NT = DV / 16;
+  constexpr bool FP8 = sizeof(CT) == 1;
+  const int unit = EXT ? blockIdx.x / ext.gchunks : blockIdx.x;
+  const int gc = EXT ? blockIdx.x % ext.gchunks : 0;
+  const int b = unit / Hkv, kvh = unit % Hkv;
+  const int G = EXT ? min(16, Gq - 16 * gc) : Gq;   // heads of this workgroup
+  const int L = seq_lens[b];
+  const TileRange tr = tile_range<EXT>(L, ext);
+  const int it0 = blockIdx.y * per_split, it1 = min(tr.n, it0 + per_split);
+  if (blockIdx.y > 0 && it0 >= tr.n) return;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hi = lane >> 4, lo = lane & 15;
+  const int h0 = kvh * Gq + 16 * gc;
   const int* btb = bt + (long)b * maxP;
-  for (int it = wid; it < ntiles; it += 4) {
-    const int tile = it < kept_tiles ? it : it - kept_tiles + win_tile;
-    const int t0 = tile * 32;
-    // ---- scores: S[g][tok] over two 16-token subtiles ------------------
+
+  constexpr int LD = DV + 4;               // rows of 16 lanes start at different banks
+  __shared__ float Lm[4][16], Ls[4][16];   // per-wave (m, s) of each head
+  __shared__ float Lacc[4][16 * LD];       // per-wave sums
+
+  // Q^T fragment: lane holds Q[g = lo][32c + 8hi + j], zero from G on; e4m3 on
+  // an fp8 cache, whose bytes feed the MFMA directly
+  bf16x8k qf[NC];
+  long qf8[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    s16x8 raw{};
+    if (lo < G)
+      raw = *reinterpret_cast<const s16x8*>(q + ((long)b * Hq + h0 + lo) * D + 32 * c + 8 * hi);
+    qf[c] = *reinterpret_cast<bf16x8k*>(&raw);
+    if (FP8) {
+      float f[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) f[j] = bf2f(raw[j]);
+      qf8[c] = pack8_fp8(f);
+    }
+  }
+
+  float m = -INFINITY, sum = 0.f;          // log2 units; of head lo
+  f32x4 acc[NT];                           // O^T: rows d = 16t + 4hi + r, column lo
+#pragma unroll
+  for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float sl2 = scale * 1.4426950408889634f;
+
+  auto tile_of = [&](int it) { return it < tr.kept ? it : it - tr.kept + tr.win_tile; };
+  auto page = [&](int it, int n) {
+    return btb[min(2 * tile_of(min(it, it1 - 1)) + n, maxP - 1)];
+  };
+  int it = it0 + wid;
+  KTile<D, CT> kt;
+  int p0 = 0, p1 = 0, p0n = 0, p1n = 0;
+  if (it < it1) {
+    p0 = page(it, 0);
+    p1 = page(it, 1);
+    p0n = page(it + 4, 0);
+    p1n = page(it + 4, 1);
+    kt.load(kc, p0, p1, Hkv, kvh, lo, hi);
+  }
+  for (; it < it1; it += 4) {
+    const int t0 = tile_of(it) * 32;
+    // V^T fragments: row d = 16t + lo, tokens 8hi .. + 7 of the two pages
+    const CT* vp = vc + (((long)(hi < 2 ? p0 : p1) * Hkv + kvh) * DV + lo) * 16 + 8 * (hi & 1);
+    i32x4k v[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      if constexpr (FP8) {
+        const i32x2k w = *reinterpret_cast<const i32x2k*>(vp + 256 * t);
+        v[t] = i32x4k{w[0], w[1], 0, 0};
+      } else {
+        v[t] = *reinterpret_cast<const i32x4k*>(vp + 256 * t);
+      }
+    }
     f32x4 sc[2];
 #pragma unroll
     for (int n = 0; n < 2; n++) {
       sc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const int page = btb[min(2 * tile + n, maxP - 1)];
-      const long krow = (((long)page * PS + lo) * Hkv + kvh) * D;
-      if (FP8) {
-        // fragment-major K layout: this lane's NC fragments are NC*8
-        // contiguous bytes at hi*(D/4) — read them 16 B at a time
-        const long kbase = krow + hi * (D >> 2);
-        if (NC >= 2) {
 #pragma unroll
-          for (int c2 = 0; c2 < NC / 2; c2++) {
-            i32x4k w = *reinterpret_cast<const i32x4k*>(
-                (const unsigned char*)kc + kbase + c2 * 16);  // one b128 load
-            i32x2k lo2{w[0], w[1]}, hi2{w[2], w[3]};
-            sc[n] = mfma16k_fp8(qf8[2 * c2], *reinterpret_cast<const long*>(&lo2), sc[n]);
-            sc[n] = mfma16k_fp8(qf8[2 * c2 + 1], *reinterpret_cast<const long*>(&hi2), sc[n]);
-          }
+      for (int c = 0; c < NC; c++) {
+        if constexpr (FP8) {
+          const i32x4k w = kt.r[n][c / 2];
+          const i32x2k w2 = c & 1 ? i32x2k{w[2], w[3]} : i32x2k{w[0], w[1]};
+          sc[n] = mfma16k_fp8(*reinterpret_cast<const long*>(&w2), qf8[c], sc[n]);
         } else {
-          const long kf8 = load_frag8_raw((const unsigned char*)kc, kbase);
-          sc[n] = mfma16k_fp8(qf8[0], kf8, sc[n]);
-        }
-      } else {
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-          bf16x8k kf = load_kv_frag<CT>(kc, krow + 32 * c + 8 * hi);
-          sc[n] = mfma16k(qf[c], kf, sc[n]);
+          sc[n] = mfma16k(*reinterpret_cast<const bf16x8k*>(&kt.r[n][c]), qf[c], sc[n]);
         }
       }
     }
-    // ---- mask + online softmax (rows = q heads g = 4*hi + r) ----------
-    float pm[2][4];
+    p0 = p0n;
+    p1 = p1n;
+    p0n = page(it + 8, 0);
+    p1n = page(it + 8, 1);
+    kt.load(kc, p0, p1, Hkv, kvh, lo, hi);
+    // ---- online softmax of head lo: 8 of the tile's tokens in this lane ------
+    float x[8], top = -INFINITY;
 #pragma unroll
-    for (int n = 0; n < 2; n++) {
-      const int ki = t0 + 16 * n + lo;
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-        pm[n][r] = (ki < L && (!EXT || ki >= win_lo || ki < ext.keep))
-                       ? sc[n][r] * scale : -INFINITY;
+    for (int i = 0; i < 8; i++) {
+      const int ki = t0 + 16 * (i >> 2) + 4 * hi + (i & 3);
+      x[i] = (ki < L && (!EXT || ki >= tr.win_lo || ki < ext.keep)) ? sc[i >> 2][i & 3] * sl2
+                                                                    : -INFINITY;
+      top = fmaxf(top, x[i]);
     }
-    float rowmax[4], fac[4];
+    top = max_groups(top);
+    float alpha = 1.f;
+    if (__any(top > m)) {
+      const float mn = fmaxf(m, top);
+      alpha = m == -INFINITY ? 0.f : exp2f(m - mn);
+      m = mn;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      float x = fmaxf(pm[0][r], pm[1][r]);
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) x = fmaxf(x, __shfl_xor(x, off));
-      const float mn = fmaxf(m[r], x);
-      fac[r] = (m[r] == -INFINITY) ? 0.f : __expf(m[r] - mn);
-      m[r] = mn;
+      for (int t = 0; t < NT; t++) acc[t] *= alpha;
     }
-    float rowsum[4] = {0.f, 0.f, 0.f, 0.f};
+    const float mm = m == -INFINITY ? 0.f : m;
+    float rs = 0.f;
 #pragma unroll
-    for (int n = 0; n < 2; n++) {
+    for (int i = 0; i < 8; i++) {
+      x[i] = exp2f(x[i] - mm);
+      rs += x[i];
+    }
+    sum = sum * alpha + sum_groups(rs);
+    // ---- O^T += V^T P^T ----------------------------------------------------
+    if constexpr (FP8) {
+      unsigned a = __builtin_amdgcn_cvt_pk_fp8_f32(x[0], x[1], 0, false);
+      a = __builtin_amdgcn_cvt_pk_fp8_f32(x[2], x[3], a, true);
+      unsigned c = __builtin_amdgcn_cvt_pk_fp8_f32(x[4], x[5], 0, false);
+      c = __builtin_amdgcn_cvt_pk_fp8_f32(x[6], x[7], c, true);
+      tokens_to_k(a, c);
+      const i32x2k w{(int)a, (int)c};
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const float p = (pm[n][r] == -INFINITY) ? 0.f : __expf(pm[n][r] - m[r]);
-        rowsum[r] += p;
-        if (FP8)
-          Pb8[wid][(4 * hi + r) * 32 + 16 * n + lo] = f32_to_fp8(p);
-        else
-          Pb[wid][(4 * hi + r) * 32 + 16 * n + lo] = f2bf(p);
+      for (int t = 0; t < NT; t++) {
+        const i32x2k vv{v[t][0], v[t][1]};
+        acc[t] = mfma16k_fp8(*reinterpret_cast<const long*>(&vv),
+                             *reinterpret_cast<const long*>(&w), acc[t]);
       }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      float x = rowsum[r];
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) x += __shfl_xor(x, off);
-      s_[r] = s_[r] * fac[r] + x;
-    }
-#pragma unroll
-    for (int t = 0; t < DV / 16; t++) {
-#pragma unroll
-      for (int r = 0; r < 4; r++) acc_o[t][r] *= fac[r];
-    }
-    lds_fence_wave_kv();
-    // ---- PV: A = P [g][tok], B = V^T (d-major pages) -------------------
-    bf16x8k pf;
-    long pf8 = 0;
-    if (FP8) {
-      pf8 = load_frag8_raw(&Pb8[wid][0], lo * 32 + 8 * hi);
     } else {
-      s16x8 raw = *reinterpret_cast<const s16x8*>(&Pb[wid][lo * 32 + 8 * hi]);
-      pf = *reinterpret_cast<bf16x8k*>(&raw);
-    }
-    const int pv_page = btb[min(2 * tile + (hi >> 1), maxP - 1)];
-    const int tokoff = 8 * (hi & 1);
+      unsigned w[4];
 #pragma unroll
-    for (int t = 0; t < DV / 16; t++) {
-      const long vaddr = (((long)pv_page * Hkv + kvh) * DV + 16 * t + lo) * PS + tokoff;
-      if (FP8) {
-        const long vf8 = load_frag8_raw((const unsigned char*)vc, vaddr);
-        acc_o[t] = mfma16k_fp8(pf8, vf8, acc_o[t]);
-      } else {
-        bf16x8k vf = load_kv_frag<CT>(vc, vaddr);
-        acc_o[t] = mfma16k(pf, vf, acc_o[t]);
-      }
+      for (int i = 0; i < 4; i++)
+        w[i] = (unsigned)(unsigned short)f2bf(x[2 * i]) |
+               (unsigned)(unsigned short)f2bf(x[2 * i + 1]) << 16;
+      tokens_to_k(w[0], w[2]);
+      tokens_to_k(w[1], w[3]);
+      const i32x4k pw{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+        acc[t] = mfma16k(*reinterpret_cast<const bf16x8k*>(&v[t]),
+                         *reinterpret_cast<const bf16x8k*>(&pw), acc[t]);
     }
   }
 
   // ---- cross-wave merge through LDS -----------------------------------
-  if (lo < 16) {
-    // lane (hi, lo): writes rows 4*hi..4*hi+3 at cols d = 16t + lo
+  if (hi == 0) { Lm[wid][lo] = m; Ls[wid][lo] = sum; }
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      if (lo == 0) { Lm[wid][4 * hi + r] = m[r]; Ls[wid][4 * hi + r] = s_[r]; }
-#pragma unroll
-      for (int t = 0; t < DV / 16; t++)
-        Lacc[wid][4 * hi + r][16 * t + lo] = acc_o[t][r];
-    }
-  }
+  for (int t = 0; t < NT; t++)
+    *reinterpret_cast<f32x4*>(&Lacc[wid][lo * LD + 16 * t + 4 * hi]) = acc[t];
   __syncthreads();
-  if (wid == 0) {
-    constexpr int OV = DV / 64;
-    for (int g = 0; g < G; g++) {
-      float M = Lm[0][g];
-      for (int w = 1; w < 4; w++) M = fmaxf(M, Lm[w][g]);
-      if (M == -INFINITY) M = 0.f;
-      float S = 0.f;
-      float o[OV > 0 ? OV : 1];
+  for (int i = threadIdx.x; i < G * (DV / 2); i += 256) {
+    const int g = i / (DV / 2), d = 2 * (i % (DV / 2));
+    const float M = fmaxf(fmaxf(Lm[0][g], Lm[1][g]), fmaxf(Lm[2][g], Lm[3][g]));
+    const float Mf = M == -INFINITY ? 0.f : M;
+    float S = 0.f, o0 = 0.f, o1 = 0.f;
 #pragma unroll
-      for (int j = 0; j < (OV > 0 ? OV : 1); j++) o[j] = 0.f;
-      for (int w = 0; w < 4; w++) {
-        const float c = (Lm[w][g] == -INFINITY) ? 0.f : __expf(Lm[w][g] - M);
-        S += Ls[w][g] * c;
-        if (OV > 0) {
+    for (int w = 0; w < 4; w++) {
+      const float c = exp2f(Lm[w][g] - Mf);
+      S += Ls[w][g] * c;
+      o0 += Lacc[w][g * LD + d] * c;
+      o1 += Lacc[w][g * LD + d + 1] * c;
+    }
+    if (tr.n <= per_split) {      // nothing to merge
+      const float inv = S > 0.f ? 1.f / S : 0.f;
+      write_pair<EXT>(out, o0 * inv, o1 * inv, b, h0 + g, d, Hq, DV, ext);
+    } else {
+      const long row = ((long)blockIdx.x * gridDim.y + blockIdx.y) * 16 + g;
+      *reinterpret_cast<float2*>(part + row * DV + d) = make_float2(o0, o1);
+      if (d == 0) *reinterpret_cast<float2*>(ms + row * 2) = make_float2(M, S);
+    }
+  }
+}
+
+// one wave per (sequence, kv head, head group, head): the splits' sums into out
+template <int DV, bool EXT>
+__global__ __launch_bounds__(64)
+void paged_decode_merge_kernel(const float* __restrict__ part, const float* __restrict__ ms,
+                               const int* __restrict__ seq_lens, short* __restrict__ out, int Hq,
+                               int Hkv, int Gq, int per_split, int splits, DecodeExt ext) {
+  const int x = blockIdx.x, g = blockIdx.y;
+  const int unit = EXT ? x / ext.gchunks : x, gc = EXT ? x % ext.gchunks : 0;
+  const int b = unit / Hkv, kvh = unit % Hkv;
+  if (16 * gc + g >= Gq) return;
+  const int n = (tile_range<EXT>(seq_lens[b], ext).n + per_split - 1) / per_split;
+  if (n <= 1) return;
+  const long row0 = (long)x * splits * 16 + g;
+  const int lane = threadIdx.x;
+  float M = -INFINITY;
+  for (int k = lane; k < n; k += 64) M = fmaxf(M, ms[(row0 + 16L * k) * 2]);
+  M = wave_max(M);
+  if (M == -INFINITY) M = 0.f;
+  constexpr int NP = DV > 128 ? 2 : 1;      // pairs per lane
+  float S = 0.f, o[NP][2] = {};
+#pragma unroll 8
+  for (int k = 0; k < n; k++) {
+    const long row = row0 + 16L * k;
+    const float c = exp2f(ms[row * 2] - M);
+    S += ms[row * 2 + 1] * c;
 #pragma unroll
-          for (int j = 0; j < (OV > 0 ? OV : 1); j++)
-            o[j] += Lacc[w][g][lane * OV + j] * c;
-        } else if (lane < DV) {
-          o[0] += Lacc[w][g][lane] * c;
-        }
-      }
-      const float invS = S > 0.f ? 1.f / S : 0.f;
-      if constexpr (EXT) {
-        short* op = out + (long)b * ext.ldo + (long)(h0 + g) * ext.V;
-        const float* cs = ext.uncs ? ext.uncs + (long)b * ext.V : nullptr;
-        constexpr int NO = OV > 0 ? OV : 1;
-#pragma unroll
-        for (int j = 0; j < NO; j++) o[j] *= invS;
-        if (cs) {
-          const int half = ext.V / 2;
-          float tw[NO];
-#pragma unroll
-          for (int j = 0; j < NO; j++) {
-            const int d = lane * NO + j;
-            const float other = NO > 1 ? o[j ^ 1] : __shfl_xor(o[j], 1);
-            const int pr = min(d >> 1, half - 1);
-            const float c = cs[pr], s = cs[half + pr];
-            tw[j] = o[j] * c + ((d & 1) ? -other : other) * s;
-          }
-#pragma unroll
-          for (int j = 0; j < NO; j++) o[j] = tw[j];
-        }
-#pragma unroll
-        for (int j = 0; j < NO; j++)
-          if (lane * NO + j < ext.V) op[lane * NO + j] = f2bf(o[j]);
-        continue;
-      }
-      short* op = out + ((long)b * Hq + h0 + g) * DV;
-      if (OV > 0) {
-#pragma unroll
-        for (int j = 0; j < (OV > 0 ? OV : 1); j++)
-          op[lane * OV + j] = f2bf(o[j] * invS);
-      } else if (lane < DV) {
-        op[lane] = f2bf(o[0] * invS);
+    for (int j = 0; j < NP; j++) {
+      const int d = 2 * (lane + 64 * j);
+      if (d < DV) {
+        o[j][0] += part[row * DV + d] * c;
+        o[j][1] += part[row * DV + d + 1] * c;
       }
     }
   }
+  const float inv = S > 0.f ? 1.f / S : 0.f;
+#pragma unroll
+  for (int j = 0; j < NP; j++) {
+    const int d = 2 * (lane + 64 * j);
+    if (d < DV)
+      write_pair<EXT>(out, o[j][0] * inv, o[j][1] * inv, b, kvh * Gq + 16 * gc + g, d, Hq, DV, ext);
+  }
+}
+
+// How a batch of `units` workgroups with at most `tiles` tiles each is split:
+// until there is one per CU, each with at least two tiles for every wave.  Four
+// per sequence read 32 x 2000 tokens (12 heads over 2, bf16) in 17.4 us with the
+// merge, two in 22.5, eight in 22.4 (the first tile's page, key and value
+// latencies then outweigh the rest); unsplit it took 135.  At 256 sequences and
+// more nothing is split: 2048 x 850 in fp8 take 172 us, 5.1 TB/s.
+constexpr long DECODE_FILL = 256;
+struct Splits { int n, per; torch::Tensor part, ms; };
+static Splits decode_splits(long units, long tiles, int DV, const torch::Tensor& like) {
+  Splits s{1, (int)std::max(tiles, 1L), {}, {}};
+  const long want = std::min((DECODE_FILL + units - 1) / units, (tiles + 7) / 8);
+  if (want > 1) {
+    s.per = (int)((tiles + want - 1) / want + 3) / 4 * 4;
+    s.n = (int)((tiles + s.per - 1) / s.per);
+  }
+  if (s.n > 1) {
+    auto f32 = like.options().dtype(torch::kFloat32);
+    s.part = torch::empty({units * s.n * 16, (long)DV}, f32);
+    s.ms = torch::empty({units * s.n * 16, 2L}, f32);
+  }
+  return s;
 }
 
 torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor k_cache,
@@ -432,16 +493,25 @@ torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor k_cache,
   auto out = torch::empty_like(q);
   if (B == 0) return out;
   auto stream = at::hip::getCurrentHIPStream();
-  dim3 grid(B * Hkv), block(256);
+  const Splits sp = decode_splits((long)B * Hkv, (maxP + 1) / 2, D, q);
+  float* part = sp.n > 1 ? sp.part.data_ptr<float>() : nullptr;
+  float* ms = sp.n > 1 ? sp.ms.data_ptr<float>() : nullptr;
+  dim3 grid(B * Hkv, sp.n), block(256);
   const bool fp8 = k_cache.scalar_type() == torch::kFloat8_e4m3fn;
   TORCH_CHECK(fp8 || k_cache.scalar_type() == torch::kBFloat16,
               "kv cache must be bf16 or fp8_e4m3fn");
 #define LAUNCH_D(DD, CT)                                                        \
-  hipLaunchKernelGGL((paged_decode_kernel<DD, DD, CT, false>), grid, block, 0, stream, \
-                     (const short*)q.data_ptr(), (const CT*)k_cache.data_ptr(), \
-                     (const CT*)v_cache.data_ptr(), block_tables.data_ptr<int>(), \
-                     seq_lens.data_ptr<int>(), (short*)out.data_ptr(),          \
-                     Hq, Hkv, maxP, G, (float)scale, DecodeExt{})
+  do {                                                                          \
+    hipLaunchKernelGGL((paged_decode_kernel<DD, DD, CT, false>), grid, block, 0, stream, \
+                       (const short*)q.data_ptr(), (const CT*)k_cache.data_ptr(), \
+                       (const CT*)v_cache.data_ptr(), block_tables.data_ptr<int>(), \
+                       seq_lens.data_ptr<int>(), (short*)out.data_ptr(), part, ms, \
+                       Hq, Hkv, maxP, G, sp.per, (float)scale, DecodeExt{});    \
+    if (sp.n > 1)                                                               \
+      hipLaunchKernelGGL((paged_decode_merge_kernel<DD, false>), dim3(B * Hkv, G), dim3(64), 0, \
+                         stream, part, ms, seq_lens.data_ptr<int>(), (short*)out.data_ptr(), \
+                         Hq, Hkv, G, sp.per, sp.n, DecodeExt{});                \
+  } while (0)
   if (D == 128) { if (fp8) LAUNCH_D(128, unsigned char); else LAUNCH_D(128, short); }
   else if (D == 64) { if (fp8) LAUNCH_D(64, unsigned char); else LAUNCH_D(64, short); }
   else if (D == 32) { if (fp8) LAUNCH_D(32, unsigned char); else LAUNCH_D(32, short); }
@@ -483,13 +553,25 @@ void paged_attn_decode_window(torch::Tensor q, torch::Tensor k_cache, torch::Ten
   DecodeExt e{(int)std::min<long>(size, 1 << 30), (int)std::min<long>(keep, 1 << 30), V,
               out.stride(0), uncs.has_value() ? uncs->data_ptr<float>() : nullptr, (G + 15) / 16};
   auto stream = at::hip::getCurrentHIPStream();
-  dim3 grid(B * Hkv * e.gchunks), block(256);
+  const long units = (long)B * Hkv * e.gchunks;
+  // at most: the whole context, or the window and the kept tokens with their ends
+  const long tiles = std::min<long>((maxP + 1) / 2, ((long)e.size + e.keep + 31) / 32 + 2);
+  const Splits sp = decode_splits(units, tiles, DV, q);
+  float* part = sp.n > 1 ? sp.part.data_ptr<float>() : nullptr;
+  float* ms = sp.n > 1 ? sp.ms.data_ptr<float>() : nullptr;
+  dim3 grid(units, sp.n), block(256);
 #define LAUNCH_KV(KK, VV)                                                                  \
-  hipLaunchKernelGGL((paged_decode_kernel<KK, VV, short, true>), grid, block, 0, stream,   \
-                     (const short*)q.data_ptr(), (const short*)k_cache.data_ptr(),         \
-                     (const short*)v_cache.data_ptr(), block_tables.data_ptr<int>(),       \
-                     seq_lens.data_ptr<int>(), (short*)out.data_ptr(), Hq, Hkv, maxP, G,   \
-                     (float)scale, e)
+  do {                                                                                     \
+    hipLaunchKernelGGL((paged_decode_kernel<KK, VV, short, true>), grid, block, 0, stream, \
+                       (const short*)q.data_ptr(), (const short*)k_cache.data_ptr(),       \
+                       (const short*)v_cache.data_ptr(), block_tables.data_ptr<int>(),     \
+                       seq_lens.data_ptr<int>(), (short*)out.data_ptr(), part, ms, Hq, Hkv, \
+                       maxP, G, sp.per, (float)scale, e);                                  \
+    if (sp.n > 1)                                                                          \
+      hipLaunchKernelGGL((paged_decode_merge_kernel<VV, true>), dim3(units, std::min(G, 16)), \
+                         dim3(64), 0, stream, part, ms, seq_lens.data_ptr<int>(),          \
+                         (short*)out.data_ptr(), Hq, Hkv, G, sp.per, sp.n, e);             \
+  } while (0)
 #define LAUNCH_V(KK)                                                                       \
   do {                                                                                     \
     if (DV == 32) LAUNCH_KV(KK, 32);                                                       \

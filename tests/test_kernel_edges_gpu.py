@@ -54,3 +54,72 @@ def test_flash_attention_negative_and_zero_scale():
     for scale in (-0.2, 0.0):
         o = ops.flash_attn_varlen(q, k, v, cu, max(lens), scale=scale)
         assert rel(o, _sdpa_ref(q.float(), k.float(), v.float(), cu.cpu(), scale)) < FA_REL
+
+
+# ------------------------------------------------------------- paged decode
+def _paged(lens, capacity, hkv, dk, dv, dtype, seed):
+    """Caches and block tables whose pages lie in no order."""
+    pages = [-(-max(n, 1) // 16) for n in lens]
+    order = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(seed))
+    bt, at = torch.zeros(len(lens), capacity, dtype=torch.int32), 0
+    for i, n in enumerate(pages):
+        bt[i, :n] = order[at:at + n]
+        at += n
+    k = rnd(at, 16, hkv, dk, seed=seed).to(dtype)
+    v = (rnd(at, hkv, dv, 16, seed=seed + 1) + rnd(1, hkv, dv, 1, seed=seed + 2)).to(dtype)
+    return k, v, bt.to(DEV), torch.tensor(lens, dtype=torch.int32, device=DEV)
+
+
+def _attend64(q, k, v, bt, n, scale, seen=None):
+    """One sequence's decode attention in 64 bits; k in plain order."""
+    pages = bt[:-(-n // 16)].long()
+    kk = k[pages].double().flatten(0, 1)[:n]
+    vv = v[pages].double().permute(0, 3, 1, 2).flatten(0, 1)[:n]
+    qq = q.double().unflatten(0, (k.shape[2], -1))
+    z = qq @ kk.permute(1, 2, 0) * scale
+    if seen is not None:
+        z = z.masked_fill(~seen, float("-inf"))
+    return (torch.softmax(z, -1) @ vv.transpose(0, 1)).flatten(0, 1)
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(12, 2, 128), (16, 1, 64), (4, 4, 32)])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("lens,capacity", [
+    ([1], 1), ([16, 17, 31, 32, 33], 3), ([255, 256, 257, 0, 513, 1000], 80),
+    ([5, 128, 2047, 2048, 2049, 3000], 200), ([40 + i for i in range(300)], 30)])
+def test_paged_decode_split_edges(lens, capacity, hq, hkv, d, fp8):
+    from nanorlhf_amd.ops.kvcache import depermute_fp8_k
+    k, v, bt, sl = _paged(lens, capacity, hkv, d, d,
+                          torch.float8_e4m3fn if fp8 else torch.bfloat16, 11)
+    q = rnd(len(lens), hq, d, seed=5, scale=1.5)
+    got = ops.paged_attn_decode(q, k, v, bt, sl, d ** -0.5)
+    kp = depermute_fp8_k(k.float()) if fp8 else k
+    # bf16: P and the result rounded to 2^-9.  fp8: q and P to 2^-4 (0.026 in the
+    # root mean square); values around a mean per channel as large as their
+    # spread take about three quarters of P's error out of the average.
+    bound = 0.03 if fp8 else 0.006
+    want = torch.stack([_attend64(q[i], kp, v, bt[i], n, d ** -0.5) if n else
+                        torch.zeros(hq, d, dtype=torch.float64, device=DEV)
+                        for i, n in enumerate(lens)])
+    assert rel(got, want) < bound
+
+
+@pytest.mark.parametrize("dk,dv,V", [(128, 128, 128), (64, 32, 24), (32, 256, 200)])
+@pytest.mark.parametrize("size,keep", [(1 << 30, 0), (70, 5), (1000, 40)])
+@pytest.mark.parametrize("hq,hkv", [(12, 2), (40, 2)])
+def test_paged_decode_window_splits(dk, dv, V, size, keep, hq, hkv):
+    from nanorlhf_amd.ops.rope import rotate_pairs
+    lens = [1, 33, 700, 1500, 2999]
+    k, v, bt, sl = _paged(lens, 200, hkv, dk, dv, torch.bfloat16, 21)
+    q = rnd(len(lens), hq, dk, seed=6, scale=1.5)
+    a = torch.rand(len(lens), V // 2, generator=torch.Generator().manual_seed(3)).to(DEV) * 6
+    cs = torch.cat([a.cos(), a.sin()], 1).contiguous()
+    out = torch.full((len(lens), hq * V + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.serve_ext().paged_attn_decode_window(q, k, v, bt, sl, out[:, :hq * V], dk ** -0.5, size,
+                                             keep, cs)
+    for i, n in enumerate(lens):
+        j = torch.arange(n, device=DEV)
+        want = _attend64(q[i], k, v, bt[i], n, dk ** -0.5, (n - 1 - j < size) | (j < keep))
+        want = rotate_pairs(want[None, :, :V].float(), cs[i:i + 1], True, sign=-1.0)[0]
+        assert rel(out[i, :hq * V].view(hq, V), want) < 0.006
+    assert bool((out[:, hq * V:] == 7).all())
