@@ -1,312 +1,431 @@
 // Temperature / top-p token sampling over [B, V] bf16 or float32 logits.
-// One 256-thread workgroup per row, four vectorized passes (s16x8 16-B
-// loads — the scalar version measured 2.7 ms/row-batch, ~6x off BW):
-//   1. fused online (max, exp-sum) + argmax
-//   2. coarse LDS histogram of prob mass over u = (l - m)/T (1024 bins)
-//   3. one refinement histogram inside the threshold bin (no 151k sort)
-//   4. per-thread kept-mass + one block scan + inverse-CDF walk by the
-//      owning thread (counter-hash uniform: deterministic in (seed, step,
-//      row), replay-safe via a device-side step counter for hipGraphs).
+// One workgroup of 1024 threads per row, which holds the whole row in registers
+// (a CU's register file is 512 KB, a row of 151936 bf16 logits 304 KB) and reads
+// it once:
+//   1. row maximum
+//   2. sum of exp(u), u = (l - max) / T, and its histogram over 32 bins of 1 nat
+//   3. the bin in which the kept mass reaches top_p, refined into 32 parts once or
+//      twice (no sort)
+//   4. kept mass per thread + one block scan + inverse-CDF walk over the owner's
+//      elements (counter-hash uniform: deterministic in (seed, step, row),
+//      replay-safe via a device-side step counter for hipGraphs).
+// Rows too long for the registers are read again for every pass.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
 #include "common.h"
 
-#define SBLOCK 256
-#define NBINS 1024
-#define URANGE 32.0f  // histogram covers u in [-URANGE, 0]
+#define SBLOCK 1024
+#define SWAVES (SBLOCK / 64)
+#define OWNERS 256     // the order of the categories: vectors of 8 elements, by index % OWNERS, then index
+#define BINS 32
+#define URANGE 32.0f   // the histogram covers u in [-URANGE, 0]; smaller ones fall into bin 0
 
-DEVINL float warp_incl_scan(float v, int lane) {
+template <typename LT> struct Vec8;
+template <> struct Vec8<short> { s16x8 r; };
+template <> struct Vec8<float> { f32x4 r[2]; };
+DEVINL void load8(const short* p, Vec8<short>& v) { v.r = *reinterpret_cast<const s16x8*>(p); }
+DEVINL void load8(const float* p, Vec8<float>& v) {
+  v.r[0] = *reinterpret_cast<const f32x4*>(p);
+  v.r[1] = *reinterpret_cast<const f32x4*>(p + 4);
+}
+DEVINL void fill8(Vec8<short>& v) {
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    float x = __shfl_up(v, off);
-    if (lane >= off) v += x;
-  }
-  return v;
+  for (int j = 0; j < 8; j++) v.r[j] = (short)0xff80;   // -inf
+}
+DEVINL void fill8(Vec8<float>& v) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) v.r[0][j] = v.r[1][j] = -INFINITY;
+}
+DEVINL void get8(const Vec8<short>& v, float* o) {
+#pragma unroll
+  for (int j = 0; j < 8; j++) o[j] = bf2f(v.r[j]);
+}
+DEVINL void get8(const Vec8<float>& v, float* o) {
+#pragma unroll
+  for (int j = 0; j < 8; j++) o[j] = v.r[j >> 2][j & 3];
+}
+// the compiler may not keep what an earlier pass made of v: unpacked, a row does
+// not fit the registers
+DEVINL void anew(Vec8<short>& v) { asm volatile("" : "+v"(v.r)); }
+DEVINL void anew(Vec8<float>& v) { asm volatile("" : "+v"(v.r[0]), "+v"(v.r[1])); }
+DEVINL float max8(const float* v) {
+  float m = v[0];
+#pragma unroll
+  for (int j = 1; j < 8; j++) m = fmaxf(m, v[j]);
+  return m;
 }
 
-template <typename LT>
-__global__ void sample_topp_kernel(const LT* __restrict__ logits,
-                                   long* __restrict__ out,
-                                   float* __restrict__ out_lp,  // nullable
-                                   int V, float temperature, float top_p,
-                                   unsigned long long seed,
-                                   unsigned long long step_imm,
-                                   const long* __restrict__ step_ptr) {
-  const unsigned long long step = step_ptr ? (unsigned long long)*step_ptr : step_imm;
-  __shared__ float sm[SBLOCK / 64];
-  __shared__ float wm_[SBLOCK / 64];
-  __shared__ int wa_[SBLOCK / 64];
-  __shared__ int argmax_sh;
-  __shared__ int found_sh;
-  __shared__ float wsum[SBLOCK / 64];
-  const long row = blockIdx.x;
-  const LT* lr = logits + row * (long)V;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int nvec = V / 8;
+// A row as its thread's vectors tid, tid + SBLOCK, ...: NV of them in registers,
+// or (NV = 0) read anew by every pass.  The V % 8 last elements belong to the
+// first threads, behind their vectors.
+template <typename LT, int NV>
+struct Row {
+  const LT* p;
+  int nvec, V;
+  Vec8<LT> c[NV ? NV : 1];
 
-  // ---- pass 1: plain row max + argmax ----------------------------------
-  // (an online (m,s) update would carry m,s ACROSS loop iterations —
-  // a serial exp/fma dependency chain per wave; plain fmax has none, and
-  // the exp-sum folds into the histogram pass below, which also drops one
-  // full read of the row)
-  float lmax = -INFINITY;
-  int am = 0;
-  const float invT = temperature > 0.f ? 1.f / temperature : 1.f;
-  for (int i = threadIdx.x; i < nvec; i += SBLOCK) {
-    float v[8];
-      ldv<8>(lr + i * 8, v);
+  DEVINL void load() {
+    if (nvec == 0) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const float l = v[j];
-      if (l > lmax) { lmax = l; am = i * 8 + j; }
+      for (int k = 0; k < NV; k++) fill8(c[k]);
+      return;
     }
-  }
-  for (int i = nvec * 8 + threadIdx.x; i < V; i += SBLOCK) {
-    const float l = ldf(lr + i);
-    if (l > lmax) { lmax = l; am = i; }
-  }
-  {  // merge argmax across the block
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      float mx2 = __shfl_xor(lmax, off);
-      int a2 = __shfl_xor(am, off);
-      if (mx2 > lmax || (mx2 == lmax && a2 < am)) { lmax = mx2; am = a2; }
-    }
-    if (lane == 0) { wm_[wid] = lmax; wa_[wid] = am; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      float MX = wm_[0];
-      int A = wa_[0];
-      for (int w = 1; w < SBLOCK / 64; w++)
-        if (wm_[w] > MX || (wm_[w] == MX && wa_[w] < A)) { MX = wm_[w]; A = wa_[w]; }
-      wm_[0] = MX; argmax_sh = A;
-    }
-    __syncthreads();
+    for (int k = 0; k < NV; k++)
+      load8(p + 8L * min((int)threadIdx.x + SBLOCK * k, nvec - 1), c[k]);
+#pragma unroll
+    for (int k = 0; k < NV; k++)
+      if ((int)threadIdx.x + SBLOCK * k >= nvec) fill8(c[k]);
   }
-  const float M = wm_[0] * invT;        // max of temperature-scaled logits
-  if (temperature == 0.f) {
-    // greedy: one extra pass only to report the T=1-softmax logprob
-    if (out_lp) {
-      float se = 0.f;
-      const float M1 = wm_[0];
-      for (int i = threadIdx.x; i < nvec; i += SBLOCK) {
+  // f(first element's index, 8 logits, -inf where there are none)
+  template <typename F> DEVINL void vectors(F f) {
+    if constexpr (NV > 0) {
+#pragma unroll
+      for (int k = 0; k < NV; k++) {
         float v[8];
-      ldv<8>(lr + i * 8, v);
-#pragma unroll
-        for (int j = 0; j < 8; j++) se += __expf(v[j] - M1);
+        anew(c[k]);
+        get8(c[k], v);
+        f(8 * (threadIdx.x + SBLOCK * k), v);
+        __builtin_amdgcn_sched_barrier(0);     // registers for one vector at a time
       }
-      for (int i = nvec * 8 + threadIdx.x; i < V; i += SBLOCK)
-        se += __expf(ldf(lr + i) - M1);
-      se = block_sum<SBLOCK>(se, sm);
-      if (threadIdx.x == 0) {
-        out[row] = argmax_sh;
-        out_lp[row] = ldf(lr + argmax_sh) - (M1 + __logf(se));
+    } else {
+      for (int i = threadIdx.x; i < nvec; i += SBLOCK) {
+        Vec8<LT> w;
+        load8(p + 8L * i, w);
+        float v[8];
+        get8(w, v);
+        f(8 * i, v);
       }
-    } else if (threadIdx.x == 0) {
-      out[row] = argmax_sh;
     }
-    return;
   }
+  DEVINL bool has_tail() const { return 8 * nvec + (int)threadIdx.x < V; }
+  DEVINL float tail() const { return ldf(p + 8 * nvec + threadIdx.x); }
+};
 
-  // ---- pass 2: coarse histogram of prob mass (wave-privatized: 4 waves
-  // hammering one 1024-bin histogram serialize on LDS atomics; a private
-  // histogram per wave merged once removes the cross-wave conflicts) ----
-  // Threshold search WITHOUT LDS atomics.  Ablation (tools/topp_ablate.hip)
-  // showed the 1024-bin atomicAdd histogram was 75% of the kernel — LDS
-  // f32 atomics are throughput-bound regardless of conflict spreading
-  // (lane-keyed slots measured no better).  Instead: a 32-bin REGISTER
-  // histogram per thread (no atomics), block-reduced through LDS once,
-  // then the boundary bin is refined by re-binning only its interior on
-  // additional streaming passes (each pass is pure reads + VALU at ~6 TB/s).
-  __shared__ float Hist32[32 * (SBLOCK / 64)];
-  __shared__ float S_sh, lo_sh, span_sh, above_sh;
-  __shared__ int done_sh;
-  float sacc = 0.f;
+// Histogram columns are private to a lane of a wave, so that the adds meet no
+// other thread's: conflict-free, and in a fixed order.  (A histogram of 32
+// registers per thread costs 32 selects per element, which was most of the
+// kernel; one shared by the block serialises on its bins.)
+struct Scratch {
+  float hist[SWAVES][BINS][64];
+  float red[SWAVES];
+  float mass[BINS];
+  float own[SBLOCK];
+  float lo, above, excl;
+  int index[SWAVES];
+  int done, found, owner;
+};
+
+DEVINL void clear_hist(Scratch& s) {
+  f32x4* h = reinterpret_cast<f32x4*>(s.hist);
+  for (int i = threadIdx.x; i < SWAVES * BINS * 16; i += SBLOCK) h[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+}
+DEVINL void add_hist(Scratch& s, float bin, float e) {
+  const int b = max(0, min(BINS - 1, (int)bin));
+  s.hist[threadIdx.x >> 6][b][threadIdx.x & 63] += e;
+}
+// The first wave finds the highest bin at which the mass from the top, `above`
+// included, reaches `target` (or bin 0), and moves lo, above and done there.
+DEVINL void choose_bin(Scratch& s, float above, float target, float lo, float width, float S,
+                       bool refined) {
+  __syncthreads();
   {
-    float hb[32];
+    const int b = threadIdx.x >> 5, l = threadIdx.x & 31;   // 32 threads per bin
+    float x = 0.f;
+#pragma unroll 4
+    for (int w = 0; w < SWAVES; w++) x += s.hist[w][b][l] + s.hist[w][b][l + 32];
 #pragma unroll
-    for (int b = 0; b < 32; b++) hb[b] = 0.f;
-    for (int i = threadIdx.x; i < nvec; i += SBLOCK) {
-      float v[8];
-      ldv<8>(lr + i * 8, v);
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const float u = v[j] * invT - M;
-        const float e = __expf(u);
-        sacc += e;
-        int b = (int)(u + URANGE);
-        b = max(0, min(31, b));
-        hb[b] += e;
-      }
-    }
-    for (int i = nvec * 8 + threadIdx.x; i < V; i += SBLOCK) {
-      const float u = ldf(lr + i) * invT - M;
-      const float e = __expf(u);
-      sacc += e;
-      int b = (int)(u + URANGE);
-      b = max(0, min(31, b));
-      hb[b] += e;
-    }
-    // wave-reduce each bin, then one slot per (bin, wave) in LDS
-#pragma unroll
-    for (int b = 0; b < 32; b++) {
-      float x = hb[b];
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
-      if (lane == 0) Hist32[b * (SBLOCK / 64) + wid] = x;
-    }
-    sacc = block_sum<SBLOCK>(sacc, sm);
-    if (threadIdx.x == 0) S_sh = sacc;
-    __syncthreads();
-  }
-  const float S = S_sh;
-  const float ptarget = top_p * S;
-  // coarse bin select (bins are 1 nat wide, u in [-URANGE, 0])
-  if (threadIdx.x == 0) {
-    float acc = 0.f;
-    int bstar = 0;
-    float above = 0.f;
-    for (int b = 31; b >= 0; b--) {
-      float h = 0.f;
-      for (int w = 0; w < SBLOCK / 64; w++) h += Hist32[b * (SBLOCK / 64) + w];
-      const float nacc = acc + h;
-      if (nacc >= ptarget || b == 0) { bstar = b; above = acc; break; }
-      acc = nacc;
-    }
-    lo_sh = (float)bstar - URANGE;
-    span_sh = 1.0f;
-    above_sh = above;
-    done_sh = 0;
-    found_sh = -1;
+    for (int off = 16; off > 0; off >>= 1) x += __shfl_xor(x, off);
+    if (l == 0) s.mass[b] = x;
   }
   __syncthreads();
-  // refine the boundary bin: re-bin its interior into 32 sub-bins per pass
-  // until the bin is narrow (1/1024 nat) or holds negligible mass
-  for (int it = 0; it < 2 && !done_sh; it++) {
-    const float lo = lo_sh, span = span_sh;
-    float hb[32];
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    const float h = lane < BINS ? s.mass[BINS - 1 - lane] : 0.f;   // from the top down
+    float incl = h;
 #pragma unroll
-    for (int b = 0; b < 32; b++) hb[b] = 0.f;
-    const float sub = 32.0f / span;
-    for (int i = threadIdx.x; i < nvec; i += SBLOCK) {
-      float v[8];
-      ldv<8>(lr + i * 8, v);
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const float u = v[j] * invT - M;
-        if (u >= lo && u < lo + span) {
-          int b = (int)((u - lo) * sub);
-          b = max(0, min(31, b));
-          hb[b] += __expf(u);
-        }
-      }
+    for (int off = 1; off < BINS; off <<= 1) {
+      const float x = __shfl_up(incl, off);
+      if (lane >= off) incl += x;
     }
-    for (int i = nvec * 8 + threadIdx.x; i < V; i += SBLOCK) {
-      const float u = ldf(lr + i) * invT - M;
-      if (u >= lo && u < lo + span) {
-        int b = (int)((u - lo) * sub);
-        b = max(0, min(31, b));
-        hb[b] += __expf(u);
-      }
+    const unsigned long long hit = __ballot(lane < BINS && above + incl >= target);
+    const int at = hit ? __ffsll((unsigned long long)hit) - 1 : BINS - 1;
+    if (lane == at) {
+      s.lo = lo + (float)(BINS - 1 - at) * width;
+      s.above = above + (incl - h);
+      // over-keeping a sliver of the boundary bin changes the nucleus by < 2% of S
+      s.done = refined && h <= 0.02f * S;
     }
-#pragma unroll
-    for (int b = 0; b < 32; b++) {
-      float x = hb[b];
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
-      if (lane == 0) Hist32[b * (SBLOCK / 64) + wid] = x;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      float acc = above_sh;
-      int bstar = 0;
-      float above = above_sh;
-      for (int b = 31; b >= 0; b--) {
-        float h = 0.f;
-        for (int w = 0; w < SBLOCK / 64; w++) h += Hist32[b * (SBLOCK / 64) + w];
-        const float nacc = acc + h;
-        if (nacc >= ptarget || b == 0) { bstar = b; above = acc; break; }
-        acc = nacc;
-      }
-      lo_sh = lo + (float)bstar * (span / 32.0f);
-      span_sh = span / 32.0f;
-      above_sh = above;
-      // stop when the boundary sliver is negligible (over-keeping the
-      // whole sliver changes the nucleus by < 2% of S)
-      float bmass = 0.f;
-      for (int w = 0; w < SBLOCK / 64; w++)
-        bmass += Hist32[bstar * (SBLOCK / 64) + w];
-      if (bmass <= 0.02f * S) done_sh = 1;
-    }
-    __syncthreads();
   }
-  const float u_thresh = lo_sh;
+  __syncthreads();
+}
 
-  // ---- pass 4: per-thread kept mass + block scan + owner walk ----------
-  float own = 0.f;
-  for (int i = threadIdx.x; i < nvec; i += SBLOCK) {
+// largest element and its lowest index (0 where nothing is above -inf)
+template <typename LT>
+DEVINL int row_argmax(const LT* __restrict__ p, int V, float& best, float* red, int* index) {
+  float top = -INFINITY;
+  int at = 0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < V / 8; i += SBLOCK) {
     float v[8];
-      ldv<8>(lr + i * 8, v);
+    ldv<8>(p + 8L * i, v);
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const float u = v[j] * invT - M;
-      if (u >= u_thresh) own += __expf(u);
-    }
+    for (int j = 0; j < 8; j++)
+      if (v[j] > top) { top = v[j]; at = 8 * i + j; }
   }
-  for (int i = nvec * 8 + threadIdx.x; i < V; i += SBLOCK) {
-    const float u = ldf(lr + i) * invT - M;
-    if (u >= u_thresh) own += __expf(u);
+  const int t = V / 8 * 8 + threadIdx.x;
+  if (t < V && ldf(p + t) > top) { top = ldf(p + t); at = t; }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const float top2 = __shfl_xor(top, off);
+    const int at2 = __shfl_xor(at, off);
+    if (top2 > top || (top2 == top && at2 < at)) { top = top2; at = at2; }
   }
-  float incl = warp_incl_scan(own, lane);
-  if (lane == 63) wsum[wid] = incl;
+  if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6] = top; index[threadIdx.x >> 6] = at; }
   __syncthreads();
-  float wbase = 0.f;
-  for (int w = 0; w < wid; w++) wbase += wsum[w];
-  float total = 0.f;
-  for (int w = 0; w < SBLOCK / 64; w++) total += wsum[w];
-  const float excl = wbase + incl - own;
-  const float r = hash_uniform(seed, step, (unsigned long long)row);
-  const float target = r * total;
-  if (own > 0.f && target >= excl && target < excl + own) {
-    // this thread owns the crossing: re-walk its strided chunks (the
-    // sampled category order is thread-strided — a fixed permutation,
-    // which leaves the sampled distribution exactly the kept softmax)
-    // scan ALL chunks with no data-dependent loop exit: an early-out on
-    // `found` makes every iteration's branch wait on the previous load
-    // (~594 serial HBM latencies); unconditional scan lets the loads
-    // pipeline and costs only the owner thread's single stride
-    float acc = excl;
-    int found = -1;
-    for (int i = threadIdx.x; i < nvec; i += SBLOCK) {
-      float v[8];
-      ldv<8>(lr + i * 8, v);
+  top = red[0];
+  at = index[0];
+  for (int w = 1; w < SWAVES; w++)
+    if (red[w] > top || (red[w] == top && index[w] < at)) { top = red[w]; at = index[w]; }
+  __syncthreads();
+  best = top;
+  return at;
+}
+
+// temperature 0: the most likely token, and its logprob under the softmax at T = 1.
+// A kernel of its own, because two rows to a CU hide each other's loads, which
+// the other's histogram leaves no LDS for.
+template <typename LT>
+__global__ __launch_bounds__(SBLOCK)
+void sample_greedy_kernel(const LT* __restrict__ logits, long* __restrict__ out,
+                          float* __restrict__ out_lp, int V) {
+  __shared__ float red[SWAVES];
+  __shared__ int index[SWAVES];
+  const long row = blockIdx.x;
+  const LT* p = logits + row * (long)V;
+  float top;
+  const int at = row_argmax(p, V, top, red, index);
+  if (threadIdx.x == 0) out[row] = at;
+  if (!out_lp) return;
+  float se = 0.f;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < V / 8; i += SBLOCK) {
+    float v[8];
+    ldv<8>(p + 8L * i, v);
+#pragma unroll
+    for (int j = 0; j < 8; j++) se += __expf(v[j] - top);
+  }
+  const int t = V / 8 * 8 + threadIdx.x;
+  if (t < V) se += __expf(ldf(p + t) - top);
+  se = block_sum<SBLOCK>(se, red);
+  if (threadIdx.x == 0) out_lp[row] = ldf(p + at) - (top + __logf(se));
+}
+
+template <typename LT, int NV>
+__global__ __launch_bounds__(SBLOCK)
+void sample_topp_kernel(const LT* __restrict__ logits,
+                        long* __restrict__ out,
+                        float* __restrict__ out_lp,  // nullable
+                        int V, float temperature, float top_p,
+                        unsigned long long seed,
+                        unsigned long long step_imm,
+                        const long* __restrict__ step_ptr) {
+  __shared__ Scratch s;
+  const unsigned long long step = step_ptr ? (unsigned long long)*step_ptr : step_imm;
+  const long row = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  Row<LT, NV> r;
+  r.p = logits + row * (long)V;
+  r.nvec = V / 8;
+  r.V = V;
+  r.load();
+
+  // ---- 1: row maximum ---------------------------------------------------
+  float top = -INFINITY;
+  r.vectors([&](int, const float* v) { top = fmaxf(top, max8(v)); });
+  if (r.has_tail()) top = fmaxf(top, r.tail());
+  top = block_max<SBLOCK>(top, s.red);
+
+  const float invT = temperature > 0.f ? 1.f / temperature : 1.f;
+  const float M = top * invT;           // max of temperature-scaled logits
+
+  // ---- 2: sum and coarse histogram ---------------------------------------
+  clear_hist(s);
+  float sum = 0.f;
+  auto coarse = [&](float l) {
+    const float u = l * invT - M, e = __expf(u);
+    sum += e;
+    add_hist(s, u + URANGE, e);
+  };
+  r.vectors([&](int, const float* v) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) coarse(v[j]);
+  });
+  if (r.has_tail()) coarse(r.tail());
+  const float S = block_sum<SBLOCK>(sum, s.red);
+  const float target = top_p * S;
+  choose_bin(s, 0.f, target, -URANGE, 1.f, S, false);
+
+  // ---- 3: refine the boundary bin until it is narrow (1/1024 nat) or holds
+  // negligible mass; vectors without an element in it are passed over ---------
+  float width = 1.f;
+  for (int it = 0; it < 2 && !s.done; it++) {
+    const float lo = s.lo, above = s.above, scale = BINS / width;
+    clear_hist(s);
+    auto fine = [&](float l) {
+      const float u = l * invT - M;
+      if (u >= lo && u < lo + width) add_hist(s, (u - lo) * scale, __expf(u));
+    };
+    r.vectors([&](int, const float* v) {
+      if (!__any(max8(v) * invT - M >= lo)) return;
+#pragma unroll
+      for (int j = 0; j < 8; j++) fine(v[j]);
+    });
+    if (r.has_tail()) fine(r.tail());
+    choose_bin(s, above, target, lo, width / BINS, S, true);
+    width /= BINS;
+  }
+  const float lowest = s.lo;
+
+  // ---- 4: kept mass, scan over the owners, walk --------------------------
+  auto kept = [&](float l) {
+    const float u = l * invT - M;
+    return u >= lowest ? __expf(u) : 0.f;
+  };
+  float own = 0.f;
+  r.vectors([&](int, const float* v) {
+    if (!__any(max8(v) * invT - M >= lowest)) return;
+#pragma unroll
+    for (int j = 0; j < 8; j++) own += kept(v[j]);
+  });
+  if (r.has_tail()) own += kept(r.tail());
+  s.own[tid] = own;
+  if (tid == 0) { s.owner = OWNERS; s.found = -1; }
+  __syncthreads();
+  own = 0.f;
+  if (tid < OWNERS) {
+#pragma unroll
+    for (int k = 0; k < SBLOCK / OWNERS; k++) own += s.own[tid + OWNERS * k];
+  }
+  float incl = own;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const float x = __shfl_up(incl, off);
+    if (lane >= off) incl += x;
+  }
+  if (lane == 63) s.red[wid] = incl;
+  __syncthreads();
+  float base = 0.f, total = 0.f;
+  for (int w = 0; w < OWNERS / 64; w++) {
+    if (w < wid) base += s.red[w];
+    total += s.red[w];
+  }
+  const float goal = hash_uniform(seed, step, (unsigned long long)row) * total;
+  const float excl = base + incl - own;
+  // rounding may leave two at a border: the first
+  if (tid < OWNERS && own > 0.f && goal >= excl && goal < excl + own) atomicMin(&s.owner, tid);
+  __syncthreads();
+  if (tid == s.owner) s.excl = excl;
+  __syncthreads();
+  if (wid == 0 && s.owner < OWNERS) {
+    // the owner's vectors in order, 64 at a time, one per lane
+    float acc = s.excl;
+    bool found = false;
+    for (int i0 = s.owner; i0 < r.nvec && !found; i0 += OWNERS * 64) {
+      const int i = i0 + OWNERS * lane;
+      float e[8], m = 0.f;
+      Vec8<LT> w;
+      if (i < r.nvec) load8(r.p + 8L * i, w);
+      else fill8(w);
+      get8(w, e);
 #pragma unroll
       for (int j = 0; j < 8; j++) {
-        const float u = v[j] * invT - M;
-        if (u >= u_thresh) {
-          acc += __expf(u);
-          if (target < acc && found < 0) found = i * 8 + j;
+        e[j] = kept(e[j]);
+        m += e[j];
+      }
+      float upto = m;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const float x = __shfl_up(upto, off);
+        if (lane >= off) upto += x;
+      }
+      const unsigned long long hit = __ballot(m > 0.f && goal < acc + upto);
+      if (hit) {
+        found = true;
+        if (lane == __ffsll((unsigned long long)hit) - 1) {
+          float at = acc + (upto - m);
+          int last = -1, pick = -1;
+#pragma unroll
+          for (int j = 0; j < 8; j++) {
+            at += e[j];
+            if (e[j] > 0.f) last = j;
+            if (pick < 0 && e[j] > 0.f && goal < at) pick = j;
+          }
+          s.found = 8 * i + (pick >= 0 ? pick : last);
         }
       }
+      acc += __shfl(upto, 63);
     }
-    for (int i = nvec * 8 + threadIdx.x; i < V; i += SBLOCK) {
-      const float u = ldf(lr + i) * invT - M;
-      if (u >= u_thresh) {
-        acc += __expf(u);
-        if (target < acc && found < 0) found = i;
-      }
-    }
-    if (found >= 0) atomicCAS(&found_sh, -1, found);
+    const int t = 8 * r.nvec + s.owner;
+    if (!found && lane == 0 && t < V && goal < acc + kept(ldf(r.p + t))) s.found = t;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const int f = (found_sh >= 0) ? found_sh : argmax_sh;  // rounding fallback
-    out[row] = f;
+  int pick = s.found;
+  if (pick < 0) {                       // rounding: no element crosses the goal
+    float best;
+    pick = row_argmax(r.p, V, best, s.red, s.index);
+  }
+  if (tid == 0) {
+    out[row] = pick;
     // logprob of the chosen token under the temperature-scaled softmax
     // (matches the scoring pass's logits/temperature quirk, grpo_trainer.py:547)
-    if (out_lp) out_lp[row] = ldf(lr + f) * invT - (M + __logf(S));
+    if (out_lp) out_lp[row] = ldf(r.p + pick) * invT - (M + __logf(S));
   }
+}
+
+// Vectors per thread that are held in registers; 1024 threads have 128 each, so
+// 19 of bf16 (155648 logits) and 8 of float32 (65536) fit beside the rest.
+//
+// What bounds a row: the histogram's read-add-write chains and the exponentials,
+// on one CU.  151936 bf16 logits at T = 0.7, top-p 0.95, us: 8 rows 29 (with 256
+// threads, five passes over memory and histograms in registers 215), 256 rows 56
+// (325), 2048 rows 299 (1608); LDS float atomics in place of the private
+// columns' plain adds took 221 for 8 rows.
+static void launch_sampler(const torch::Tensor& logits, torch::Tensor& out, float* lp,
+                           double temperature, double top_p, long seed, long step,
+                           const long* step_ptr) {
+  const long B = logits.size(0);
+  const int V = logits.size(1), n = (V / 8 + SBLOCK - 1) / SBLOCK;
+  auto stream = at::hip::getCurrentHIPStream();
+  const bool half = logits.scalar_type() == torch::kBFloat16;
+  if ((float)temperature == 0.f) {
+    if (half)
+      hipLaunchKernelGGL(sample_greedy_kernel<short>, dim3(B), dim3(SBLOCK), 0, stream,
+                         (const short*)logits.data_ptr(), out.data_ptr<long>(), lp, V);
+    else
+      hipLaunchKernelGGL(sample_greedy_kernel<float>, dim3(B), dim3(SBLOCK), 0, stream,
+                         logits.data_ptr<float>(), out.data_ptr<long>(), lp, V);
+    HIP_CHECK_LAST();
+    return;
+  }
+#define LAUNCH(LT, NV)                                                                       \
+  hipLaunchKernelGGL((sample_topp_kernel<LT, NV>), dim3(B), dim3(SBLOCK), 0, stream,         \
+                     (const LT*)logits.data_ptr(), out.data_ptr<long>(), lp, V,              \
+                     (float)temperature, (float)top_p, (unsigned long long)seed,             \
+                     (unsigned long long)step, step_ptr)
+  if (half) {
+    if (n <= 4) LAUNCH(short, 4);
+    else if (n <= 16) LAUNCH(short, 16);
+    else if (n <= 19) LAUNCH(short, 19);
+    else LAUNCH(short, 0);
+  } else {
+    if (n <= 8) LAUNCH(float, 8);
+    else LAUNCH(float, 0);
+  }
+#undef LAUNCH
+  HIP_CHECK_LAST();
 }
 
 torch::Tensor sample_topp(torch::Tensor logits, double temperature, double top_p,
@@ -315,18 +434,9 @@ torch::Tensor sample_topp(torch::Tensor logits, double temperature, double top_p
   const bool half = logits.scalar_type() == torch::kBFloat16;
   TORCH_CHECK(half || logits.scalar_type() == torch::kFloat32, "logits must be bf16 or float32");
   const long B = logits.size(0);
-  const int V = logits.size(1);
   auto out = torch::empty({B}, logits.options().dtype(torch::kLong));
   if (B == 0) return out;
-  auto stream = at::hip::getCurrentHIPStream();
-#define LAUNCH(LT)                                                              \
-  hipLaunchKernelGGL(sample_topp_kernel<LT>, dim3(B), dim3(SBLOCK), 0, stream,  \
-                     (const LT*)logits.data_ptr(), out.data_ptr<long>(),        \
-                     nullptr, V, (float)temperature, (float)top_p,            \
-                     (unsigned long long)seed, (unsigned long long)step, nullptr)
-  if (half) LAUNCH(short); else LAUNCH(float);
-#undef LAUNCH
-  HIP_CHECK_LAST();
+  launch_sampler(logits, out, nullptr, temperature, top_p, seed, step, nullptr);
   return out;
 }
 
@@ -340,18 +450,10 @@ std::vector<torch::Tensor> sample_topp_dev(torch::Tensor logits, double temperat
   TORCH_CHECK(half || logits.scalar_type() == torch::kFloat32, "logits must be bf16 or float32");
   TORCH_CHECK(step.scalar_type() == torch::kLong && step.is_cuda());
   const long B = logits.size(0);
-  const int V = logits.size(1);
   auto out = torch::empty({B}, logits.options().dtype(torch::kLong));
   auto lp = torch::empty({B}, logits.options().dtype(torch::kFloat32));
   if (B == 0) return {out, lp};
-  auto stream = at::hip::getCurrentHIPStream();
-#define LAUNCH(LT)                                                              \
-  hipLaunchKernelGGL(sample_topp_kernel<LT>, dim3(B), dim3(SBLOCK), 0, stream,  \
-                     (const LT*)logits.data_ptr(), out.data_ptr<long>(),        \
-                     lp.data_ptr<float>(), V, (float)temperature, (float)top_p,            \
-                     (unsigned long long)seed, 0ull, step.data_ptr<long>())
-  if (half) LAUNCH(short); else LAUNCH(float);
-#undef LAUNCH
-  HIP_CHECK_LAST();
+  launch_sampler(logits, out, lp.data_ptr<float>(), temperature, top_p, seed, 0,
+                 step.data_ptr<long>());
   return {out, lp};
 }

@@ -123,3 +123,78 @@ def test_paged_decode_window_splits(dk, dv, V, size, keep, hq, hkv):
         want = rotate_pairs(want[None, :, :V].float(), cs[i:i + 1], True, sign=-1.0)[0]
         assert rel(out[i, :hq * V].view(hq, V), want) < 0.006
     assert bool((out[:, hq * V:] == 7).all())
+
+
+# ----------------------------------------------------------------- sampling
+def _splitmix(x):
+    x = (x + 0x9E3779B97F4A7C15) % 2 ** 64
+    x = ((x ^ (x >> 30)) * 0xBF58476D1CE4E5B9) % 2 ** 64
+    x = ((x ^ (x >> 27)) * 0x94D049BB133111EB) % 2 ** 64
+    return x ^ (x >> 31)
+
+
+def _sample64(row, temperature, top_p, seed, step, index):
+    """The sampler's definition in 64 bits: bins of one nat below the maximum,
+    the boundary bin refined twice by 32, categories ordered by vector of 8
+    modulo 256."""
+    V = len(row)
+    # u itself is 32-bit (one fma from a rounded maximum): whether the maximum lies
+    # inside the topmost bin, [-1, 0), depends on it
+    inv = torch.tensor(1 / temperature, dtype=torch.float32)
+    u = (row.double() * inv.double() - (row.max() * inv).double()).float().double()
+    e = torch.exp(u)
+    goal, above, lo, width = top_p * float(e.sum()), 0.0, -32.0, 1.0
+    inside = torch.ones_like(u, dtype=torch.bool)
+    for it in range(3):
+        b = ((u - lo) / width).long().clamp(0, 31) if it else (u + 32).long().clamp(0, 31)
+        mass = torch.zeros(32, dtype=torch.float64).index_add_(0, b[inside], e[inside])
+        acc, at = above, 0
+        for k in range(31, -1, -1):
+            if acc + float(mass[k]) >= goal or k == 0:
+                at = k
+                break
+            acc += float(mass[k])
+        above, lo = acc, lo + at * width
+        if it and float(mass[at]) <= 0.02 * float(e.sum()):
+            break
+        inside = (u >= lo) & (u < lo + width)
+        width /= 32
+    i = torch.arange(V)
+    vec = i // 8
+    owner = torch.where(vec < V // 8, vec % 256, i - V // 8 * 8)
+    order = torch.argsort(owner * (V + 8) + i)
+    cdf = torch.cumsum(torch.where(u >= lo, e, 0.0)[order], 0)
+    h = _splitmix(seed ^ _splitmix(step ^ _splitmix(index)))
+    r = (h >> 40) / 2.0 ** 24 * float(cdf[-1])
+    return int(order[int((cdf <= r).sum())])
+
+
+@pytest.mark.parametrize("V", [1, 7, 8, 9, 1000, 1023, 2049, 32768, 65544, 131080, 151936, 155648,
+                               155656])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("temperature,top_p", [(0.7, 0.95), (1.0, 1.0), (1.3, 0.5)])
+def test_sampler_matches_its_definition(V, dtype, temperature, top_p):
+    B = 6
+    g = torch.Generator().manual_seed(V)
+    rank = torch.argsort(torch.rand(B, V, generator=g), 1).double() + 1
+    logits = (-1.4 * rank.log() + 0.5 * torch.randn(B, V, generator=g)).to(dtype)
+    got = ops.sample_tokens(logits.to(DEV), temperature, top_p, 77, 3).cpu()
+    want = [_sample64(logits[i].float(), temperature, top_p, 77, 3, i) for i in range(B)]
+    # A 32-bit sum may move a border past the draw: about 1e-7 of the mass per
+    # kept token, some thousands of tokens.
+    assert sum(int(a) != b for a, b in zip(got.tolist(), want)) == 0
+
+
+def test_sampler_greedy_ties_and_odd_rows():
+    x = torch.full((6, 3001), -3.0)
+    x[0, [2999, 17]] = 1.0                      # the lower index wins
+    x[1, 3000] = 2.0                            # behind the last whole vector
+    x[2] = float("-inf")
+    x[3, :], x[3, 5] = float("-inf"), 0.0
+    x[4, 9] = float("inf")
+    x[5, 40], x[5, 41] = float("nan"), 0.5
+    for dtype in (torch.bfloat16, torch.float32):
+        g = ops.sample_tokens(x.to(dtype).to(DEV), 0.0, 1.0, 1, 1).tolist()
+        assert g == [17, 3000, 0, 5, 9, 41]
+        s = ops.sample_tokens(x.to(dtype).to(DEV), 1.0, 0.9, 1, 1).tolist()
+        assert s[2] == 0 and s[3] == 5 and s[4] == 9 and 0 <= s[5] < 3001 and s[5] != 40
