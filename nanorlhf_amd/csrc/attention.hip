@@ -68,23 +68,6 @@ DEVINL int swz(int row) {
   else return (row >> 2) & 3;
 }
 
-// 16 (or 4) bytes per lane from base + offset to LDS, lane after lane from `at`.
-// As assembly, because the compiler waits for a load that it knows to write LDS
-// before the next LDS read, whichever buffer that reads, and so undoes the
-// prefetch; there is no output register.  tiles_ready() does the waiting.
-DEVINL void load_to_lds16(const void* base, unsigned offset, const void* at) {
-  const unsigned l = __builtin_amdgcn_readfirstlane(
-      (unsigned)(size_t)(const __attribute__((address_space(3))) void*)at);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               ::"s"(l), "v"(offset), "s"(base) : "memory", "m0");
-}
-DEVINL void load_to_lds4(const void* base, unsigned offset, const void* at) {
-  const unsigned l = __builtin_amdgcn_readfirstlane(
-      (unsigned)(size_t)(const __attribute__((address_space(3))) void*)at);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
-               ::"s"(l), "v"(offset), "s"(base) : "memory", "m0");
-}
-
 // All waves' loads into LDS have arrived, and nobody reads the buffer that is
 // filled next.
 DEVINL void tiles_ready() {

@@ -196,6 +196,37 @@ DEVINL void split8(const float* x, s16x8& hi, s16x8& lo) {
 }
 DEVINL bf16x8l as_frag(const s16x8& x) { return *reinterpret_cast<const bf16x8l*>(&x); }
 
+// 16 (or 4) bytes per lane from base + offset to LDS, lane after lane from `at`;
+// base and at are the same in the whole wave.  As assembly, because the compiler
+// waits for a load that it knows to write LDS before the next LDS read, whichever
+// buffer that reads, and so undoes a prefetch; there is no output register, and
+// nothing else on this part uses m0.  The caller waits (wait_loads).
+DEVINL const void* in_sgprs(const void* p) {
+  const unsigned long long x = (unsigned long long)p;
+  return (const void*)((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(x >> 32)) << 32 |
+                       (unsigned)__builtin_amdgcn_readfirstlane((unsigned)x));
+}
+DEVINL unsigned lds_address(const void* p) {
+  return __builtin_amdgcn_readfirstlane(
+      (unsigned)(size_t)(const __attribute__((address_space(3))) void*)p);
+}
+DEVINL void load_to_lds16(const void* base, unsigned offset, const void* at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               ::"s"(lds_address(at)), "v"(offset), "s"(in_sgprs(base)) : "memory");
+}
+DEVINL void load_to_lds4(const void* base, unsigned offset, const void* at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+               ::"s"(lds_address(at)), "v"(offset), "s"(in_sgprs(base)) : "memory");
+}
+
+// until at most N loads of this wave are outstanding
+template <int N>
+DEVINL void wait_loads() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4) << 14 | 0x0f70);   // vmcnt alone
+  asm volatile("" ::: "memory");
+}
+
 // wave-private LDS write->read ordering (staging buffers written and read
 // by the same wave between barriers)
 DEVINL void lds_fence_wave_kv() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }

@@ -3,14 +3,14 @@
 // head's key map (qa, R wide), so a score is qa . c, and what leaves is the
 // softmax-weighted sum of c, which the caller passes through the value maps.
 //
-// latent_attn (bf16, MFMA): one workgroup of 4 or 8 waves per (sequence, 16 rows);
-// a row is a (token, head) pair, tokens outermost.  Latents walk in tiles of 64
-// tokens, read once from memory: 8 x 8 blocks go to LDS as they are (for the
-// scores) and turned around in registers (for the weighted sum).  A wave scores
-// 16 tokens, with 8 waves over half of the latent's columns; every wave then does
-// the softmax of all 16 rows (32-bit) in its own registers and sums its share of
-// the latent's columns.  Few rows and long contexts are split over the context;
-// latent_merge joins the parts.
+// latent_attn (bf16, MFMA): one workgroup of 4 waves per (sequence, 16 rows, part
+// of the context); a row is a (token, head) pair, tokens outermost.  Every wave
+// walks pages of its own (16 tokens, contiguous in memory) with a running maximum
+// and sum of its own and shares nothing with the others until the end: pages come
+// to its part of LDS by direct loads, up to three ahead, S^T = C Q^T reads them
+// along the latent and O^T += C^T P^T turned around (ds_read_tr16_b64).  Scores of
+// one row lie in one lane's column, and as they come out of the first product
+// they are the second's operand.  latent_merge joins parts of a split context.
 //
 // latent_attn_plain: one wave per (token, head), scalar products in 32-bit.
 #include <torch/extension.h>
@@ -79,160 +79,165 @@ struct LatentArgs {
   float scale;
 };
 
-template <int RP, int NW>
-__global__ __launch_bounds__(64 * NW) void latent_attn_kernel(LatentArgs a) {
-  constexpr int KH = NW / 4, NC = RP / 32 / KH, NT = RP / 16 / NW, CS = RP + 8, SS = 68;
-  constexpr int NG = RP / 8;                  // groups of 8 columns
-  constexpr int NB = (RP + 64 * NW - 1) / (64 * NW);   // 8 x 8 blocks per thread
-  __shared__ __attribute__((aligned(16))) short cs[64 * CS], ct[64 * RP];
-  __shared__ __attribute__((aligned(16))) float sc[KH][16 * SS];
+// A page's 16-byte chunks are exchanged (xor) by row, so that 16 rows at one
+// column (scores) and 4 rows at 4 columns (turned around) meet all banks.
+template <int RP>
+DEVINL int page_swz(int row) {
+  if constexpr (RP == 64)        // two rows per 256 bytes
+    return ((row >> 1) & 1) << 1 | ((row >> 2) & 1) << 2 | (row >> 3);
+  else
+    return (row & 3) << 2 | ((row >> 2) & 1) << 1 | (row >> 3);
+}
+
+// What bounds it: reading the latents, and their uneven lengths.  128 contexts of
+// about 2000 latents of 512, 12 heads: 65 us (4.3 TB/s) with two parts each, one
+// workgroup per CU; with whole tiles of 64 tokens going through registers and
+// four barriers per tile it took 116.  Four parts took 74 us (a part costs about
+// 9 us beside its pages: first loads, sums), two waves per workgroup 67 at best.
+template <int RP>
+__global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
+  constexpr int NW = 4, NC = RP / 32, NT = RP / 16, CH = RP / 8;
+  constexpr int PAGE = 16 * RP;                          // elements
+  constexpr int LOADS = PAGE / 512;                      // direct loads per page
+  constexpr int NBUF = RP >= 512 ? 2 : 4;
+  // pages of each wave; at the end its sums, 16 x RP floats
+  __shared__ __attribute__((aligned(16))) short buf[NW][NBUF * PAGE];
+  __shared__ float Lm[NW][16], Ls[NW][16];
   const int seq = blockIdx.y;
   const int t0 = a.cu ? a.cu[seq] : seq;
   const int nq = a.cu ? a.cu[seq + 1] - t0 : 1;
   const int R = nq * a.H, r0 = blockIdx.x * 16;
   if (r0 >= R) return;
-  const int L = a.seq_lens[seq], start = L - nq;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int start = a.seq_lens[seq] - nq;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lo = lane & 15, hi = lane >> 4;
-  const int tw = wid & 3, c0 = (wid >> 2) * NC * 32;   // its tokens and columns when scoring
   const int row = min(r0 + lo, R - 1);
   const int qpos = start + row / a.H;         // of this lane's row
-  const int ntiles = (start + min(r0 + 15, R - 1) / a.H) / 64 + 1;
-  const int per = (ntiles + a.splits - 1) / a.splits;
-  const int it0 = blockIdx.z * per, it1 = min(ntiles, it0 + per);
-  const int* btb = a.bt + (long)seq * a.maxP;
-  const int last_page = (L - 1) >> 4;
+  const int npages = (start + min(r0 + 15, R - 1) / a.H) / 16 + 1;
+  const int per = (npages + a.splits - 1) / a.splits;
+  const int p0 = blockIdx.z * per, p1 = min(npages, p0 + per);
+  // scalar loads: a vector load would be waited for behind the pages under way
+  typedef const __attribute__((address_space(4))) int* const_ints;
+  const const_ints btb = (const_ints)(size_t)(a.bt + (long)seq * a.maxP);
+
+  auto fetch = [&](int page, int slot) {
+    const short* src = a.cache + (long)btb[page] * PAGE;
+#pragma unroll
+    for (int j = 0; j < LOADS; j++) {
+      const int idx = 64 * j + lane, r = idx / CH, c = (idx % CH) ^ page_swz<RP>(r);
+      load_to_lds16(src, (r * CH + c) * 16, &buf[wid][slot * PAGE + 512 * j]);
+    }
+  };
+  int ahead = p0 + wid;
+#pragma unroll
+  for (int b = 0; b < NBUF; b++, ahead += NW)
+    if (ahead < p1) fetch(ahead, b);
 
   bf16x8l qf[NC];
 #pragma unroll
   for (int q = 0; q < NC; q++)
-    qf[q] = frag(a.qa + ((long)t0 * a.H + row) * RP + c0 + 32 * q + 8 * hi);
-
-  s16x8 in[NB][8];
-  auto load_tile = [&](int tile) {
+    qf[q] = frag(a.qa + ((long)t0 * a.H + row) * RP + 32 * q + 8 * hi);
+  // waited for here, once: in the loop the wait would take the pages' loads along
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-      const int blk = threadIdx.x + 64 * NW * b;
-      if (blk >= 8 * NG) break;
-      const int dg = blk % NG, tg = blk / NG;
-      const int page = btb[min(tile * 4 + (tg >> 1), last_page)];
-      const short* src = a.cache + ((long)page * 16 + (tg & 1) * 8) * RP + 8 * dg;
-#pragma unroll
-      for (int i = 0; i < 8; i++) in[b][i] = *reinterpret_cast<const s16x8*>(src + i * RP);
-    }
-  };
-  // turned around, columns of a group are exchanged (xor) by group: otherwise
-  // neighbouring lanes' stores would meet in the same banks
-  auto store_tile = [&] {
-#pragma unroll
-    for (int b = 0; b < NB; b++) {
-      const int blk = threadIdx.x + 64 * NW * b;
-      if (blk >= 8 * NG) break;
-      const int dg = blk % NG, tg = blk / NG;
-#pragma unroll
-      for (int i = 0; i < 8; i++)
-        *reinterpret_cast<s16x8*>(&cs[(8 * tg + i) * CS + 8 * dg]) = in[b][i];
-#pragma unroll
-      for (int d = 0; d < 8; d++) {
-        s16x8 col;
-#pragma unroll
-        for (int i = 0; i < 8; i++) col[i] = in[b][i][d];
-        *reinterpret_cast<s16x8*>(&ct[(tg * RP + 8 * dg + (d ^ (dg & 7))) * 8]) = col;
-      }
-    }
-  };
+  for (int q = 0; q < NC; q++) asm volatile("" : "+v"(qf[q]));
 
   float m = -INFINITY, sum = 0.f;             // of row lo
-  f32x4 acc[NT];                              // rows 4 hi + r, column lo of each tile
+  f32x4 acc[NT];                              // O^T: latent columns 16 t + 4 hi + r, row lo
 #pragma unroll
   for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const float sl2 = a.scale * 1.4426950408889634f;
-  if (it0 < it1) load_tile(it0);
-  for (int it = it0; it < it1; it++) {
-    store_tile();
-    __syncthreads();
-    if (it + 1 < it1) load_tile(it + 1);
-    f32x4 s{0.f, 0.f, 0.f, 0.f};
+  int slot = 0;
+  for (int pg = p0 + wid; pg < p1; pg += NW) {
+    // pages behind this one that are on their way
+    if (pg + NW * (NBUF - 1) < p1) wait_loads<LOADS * (NBUF - 1)>();
+    else wait_loads<0>();
+    const short* C = &buf[wid][slot * PAGE];
+    f32x4 s2[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int q = 0; q < NC; q++)
-      s = mfma16l(qf[q], frag(&cs[(16 * tw + lo) * CS + c0 + 32 * q + 8 * hi]), s);
+      s2[q & 1] = mfma16l(frag(C + lo * RP + (((4 * q + hi) ^ page_swz<RP>(lo)) << 3)), qf[q],
+                          s2[q & 1]);
+    float x[4], top = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 4; r++) sc[wid >> 2][(4 * hi + r) * SS + 16 * tw + lo] = s[r] * sl2;
-    __syncthreads();
-    float p[16];
-    float best = -INFINITY;
-#pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-      ldv<8>(&sc[0][lo * SS + 32 * ks + 8 * hi], p + 8 * ks);
-      if constexpr (KH == 2) {
-        float other[8];
-        ldv<8>(&sc[1][lo * SS + 32 * ks + 8 * hi], other);
-#pragma unroll
-        for (int j = 0; j < 8; j++) p[8 * ks + j] += other[j];
-      }
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        if (it * 64 + 32 * ks + 8 * hi + j > qpos) p[8 * ks + j] = -INFINITY;
-        best = fmaxf(best, p[8 * ks + j]);
-      }
+    for (int r = 0; r < 4; r++) {
+      x[r] = 16 * pg + 4 * hi + r > qpos ? -INFINITY : (s2[0][r] + s2[1][r]) * sl2;
+      top = fmaxf(top, x[r]);
     }
-    best = fmaxf(best, __shfl_xor(best, 16));
-    best = fmaxf(best, __shfl_xor(best, 32));
-    const float mn = fmaxf(m, best);
-    const float alpha = m == -INFINITY ? 0.f : exp2f(m - mn);
-    float rs = 0.f;
-    s16x8 pf[2];
+    top = fmaxf(top, __shfl_xor(top, 16));
+    top = fmaxf(top, __shfl_xor(top, 32));
+    float alpha = 1.f;
+    // rescale only when a row grew by 8 nats (or has no maximum yet)
+    if (__any(!(top - m <= 11.54f))) {
+      const float mn = fmaxf(m, top);
+      alpha = m == -INFINITY ? 0.f : exp2f(m - mn);
+      m = mn;
 #pragma unroll
-    for (int j = 0; j < 16; j++) {
-      // normed by the sum of the weights as rounded
-      const short x = f2bf(p[j] == -INFINITY ? 0.f : exp2f(p[j] - mn));
-      rs += bf2f(x);
-      pf[j >> 3][j & 7] = x;
+      for (int t = 0; t < NT; t++) acc[t] *= alpha;
+    }
+    const float mm = m == -INFINITY ? 0.f : m;
+    s16x4 pf;
+    float rs = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      pf[r] = f2bf(exp2f(x[r] - mm));         // normed by the sum of the weights as rounded
+      rs += bf2f(pf[r]);
     }
     rs += __shfl_xor(rs, 16);
     rs += __shfl_xor(rs, 32);
     sum = sum * alpha + rs;
-    if (__any(mn != m)) {
+    {
+      typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+      const int tr = 4 * hi + (lo >> 2), sw = page_swz<RP>(tr);
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const float al = __shfl(alpha, 4 * hi + r);
-#pragma unroll
-        for (int t = 0; t < NT; t++) acc[t][r] *= al;
+      for (int t = 0; t < NT; t++) {
+        const short* at = C + tr * RP + (((2 * t + ((lo & 3) >> 1)) ^ sw) << 3) + (lo & 1) * 4;
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at), pf, acc[t], 0, 0, 0);
       }
     }
-    m = mn;
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-      const int d = (wid * NT + t) * 16 + lo;
-      const int at = (d & ~7) + ((d & 7) ^ (d >> 3 & 7));
-#pragma unroll
-      for (int ks = 0; ks < 2; ks++)
-        acc[t] = mfma16l(as_frag(pf[ks]), frag(&ct[((4 * ks + hi) * RP + at) * 8]), acc[t]);
+    if (ahead < p1) {
+      lds_fence_wave_kv();                    // this page's reads are done
+      fetch(ahead, slot);
+      ahead += NW;
     }
-    __syncthreads();
+    slot = slot + 1 == NBUF ? 0 : slot + 1;
   }
 
-  if (a.splits > 1) {
-    const long unit = ((long)blockIdx.y * gridDim.x + blockIdx.x) * a.splits + blockIdx.z;
-    if (wid == 0 && hi == 0) {
-      a.ms[(unit * 16 + lo) * 2] = m;
-      a.ms[(unit * 16 + lo) * 2 + 1] = sum;
+  // ---- the four waves' sums, in their own LDS (chunks of 4 exchanged by row)
+  lds_fence_wave_kv();
+  float* own = reinterpret_cast<float*>(buf[wid]);
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+    *reinterpret_cast<f32x4*>(own + lo * RP + (((4 * t + hi) ^ lo) << 2)) = acc[t];
+  if (hi == 0) { Lm[wid][lo] = m; Ls[wid][lo] = sum; }
+  __syncthreads();
+  const long unit = ((long)blockIdx.y * gridDim.x + blockIdx.x) * a.splits + blockIdx.z;
+  for (int i = threadIdx.x; i < 16 * (RP / 4); i += 256) {
+    const int r = i / (RP / 4), c = i % (RP / 4);
+    if (r0 + r >= R) break;
+    float M = Lm[0][r];
+#pragma unroll
+    for (int w = 1; w < NW; w++) M = fmaxf(M, Lm[w][r]);
+    const float Mf = M == -INFINITY ? 0.f : M;
+    float S = 0.f;
+    f32x4 o{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const float f = exp2f(Lm[w][r] - Mf);
+      S += Ls[w][r] * f;
+      o += *reinterpret_cast<const f32x4*>(reinterpret_cast<float*>(buf[w]) + r * RP +
+                                           ((c ^ r) << 2)) * f;
     }
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-#pragma unroll
-      for (int t = 0; t < NT; t++)
-        a.part[(unit * 16 + 4 * hi + r) * RP + (wid * NT + t) * 16 + lo] = acc[t][r];
-    return;
-  }
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const float inv = 1.f / __shfl(sum, 4 * hi + r);
-    const int rr = r0 + 4 * hi + r;
-    if (rr >= R) continue;
-#pragma unroll
-    for (int t = 0; t < NT; t++)
-      stf(a.out + ((long)t0 * a.H + rr) * RP + (wid * NT + t) * 16 + lo, acc[t][r] * inv);
+    if (a.splits > 1) {
+      *reinterpret_cast<f32x4*>(a.part + (unit * 16 + r) * RP + 4 * c) = o;
+      if (c == 0) {
+        a.ms[(unit * 16 + r) * 2] = M;
+        a.ms[(unit * 16 + r) * 2 + 1] = S;
+      }
+    } else {
+      const float inv = 1.f / S, y[4] = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
+      stv<4>(a.out + ((long)t0 * a.H + r0 + r) * RP + 4 * c, y);
+    }
   }
 }
 
@@ -464,9 +469,9 @@ torch::Tensor latent_attn(torch::Tensor qa, torch::Tensor cache, c10::optional<t
   a.H = H;
   a.maxP = bt.size(1);
   a.scale = scale;
-  // enough workgroups for the chip, none with less than two tiles of context
+  // one workgroup per CU, none with less than two pages for every wave
   const long most = std::max<long>(1, bt.size(1) / 8);
-  a.splits = (int)std::min<long>(std::min<long>(most, 32), std::max<long>(1, 512 / units));
+  a.splits = (int)std::min<long>(std::min<long>(most, 64), std::max<long>(1, 256 / units));
   torch::Tensor part, ms;
   if (a.splits > 1) {
     auto f = qa.options().dtype(torch::kFloat32);
@@ -478,12 +483,11 @@ torch::Tensor latent_attn(torch::Tensor qa, torch::Tensor cache, c10::optional<t
   auto stream = at::hip::getCurrentHIPStream();
   TORCH_CHECK(B <= 65535, "too many sequences in a batch");
   const dim3 grid(units_x, B, a.splits);
-#define LAUNCH(RR, NW) \
-  hipLaunchKernelGGL((latent_attn_kernel<RR, NW>), grid, dim3(64 * NW), 0, stream, a)
-  if (RP == 64) LAUNCH(64, 4);
-  else if (RP == 128) LAUNCH(128, 4);
-  else if (RP == 256) LAUNCH(256, 8);
-  else if (RP == 512) LAUNCH(512, 8);
+#define LAUNCH(RR) hipLaunchKernelGGL((latent_attn_kernel<RR>), grid, dim3(256), 0, stream, a)
+  if (RP == 64) LAUNCH(64);
+  else if (RP == 128) LAUNCH(128);
+  else if (RP == 256) LAUNCH(256);
+  else if (RP == 512) LAUNCH(512);
   else TORCH_CHECK(false, "unsupported latent width ", RP);
 #undef LAUNCH
   if (a.splits > 1)

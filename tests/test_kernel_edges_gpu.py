@@ -198,3 +198,29 @@ def test_sampler_greedy_ties_and_odd_rows():
         assert g == [17, 3000, 0, 5, 9, 41]
         s = ops.sample_tokens(x.to(dtype).to(DEV), 1.0, 0.9, 1, 1).tolist()
         assert s[2] == 0 and s[3] == 5 and s[4] == 9 and 0 <= s[5] < 3001 and s[5] != 40
+
+
+# --------------------------------------------------------- latent attention
+@pytest.mark.parametrize("rp", [64, 128, 256, 512])
+@pytest.mark.parametrize("heads", [1, 12, 17])
+@pytest.mark.parametrize("lens,capacity", [
+    ([1, 15, 16, 17, 63, 64, 65, 128], 8), ([1000, 129, 4, 2047, 512], 200),
+    ([30 + i for i in range(300)], 40)])
+def test_latent_attention_page_edges(rp, heads, lens, capacity):
+    pages = [-(-n // 16) for n in lens]
+    order = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(1))
+    bt, at = torch.zeros(len(lens), capacity, dtype=torch.int32), 0
+    for i, n in enumerate(pages):
+        bt[i, :n] = order[at:at + n]
+        at += n
+    bt = bt.to(DEV)
+    cache = rnd(at, 16, rp, seed=1)
+    q = rnd(len(lens), heads, rp, seed=2)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    got = ops.serve_ext().latent_attn(q, cache, None, sl, bt, 1, rp ** -0.5)
+    want = torch.empty(got.shape, dtype=torch.float64, device=DEV)
+    for i, n in enumerate(lens):
+        c = cache[bt[i, :-(-n // 16)].long()].double().flatten(0, 1)[:n]
+        want[i] = torch.softmax(q[i].double() @ c.t() * rp ** -0.5, -1) @ c
+    # weights and result rounded to bf16 (0.0011 in the root mean square each)
+    assert rel(got, want) < 0.006
