@@ -148,6 +148,157 @@ __global__ void lora_gemm_kernel(const short* __restrict__ x,
   }
 }
 
+// ---- 256 x 256 tile, 8 waves -----------------------------------------------
+// For grids that fill most of the chip with one workgroup per CU.  Twice the
+// reuse of the 128-tile in both directions, LDS tiles without bank conflicts, the
+// next step's fragments read between the products, 16 neighbouring columns of y
+// per lane.  48720 x 17920 x 1536 + 64: 2.70 ms (1033 TFLOP/s) against 3.80, x 1536
+// x 17920: 2.37 (1136) against 3.30; 59% of the cycles are products, the rest
+// mostly waits at the tiles' barriers.  Four stages of 32 that land a barrier
+// ahead (974 TFLOP/s: rows of 64 bytes double the requests), 256 x 128 tiles twice
+// per CU (870) and four waves of 128 x 128 (999) were slower.
+typedef float f32x16_l __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8_m __attribute__((ext_vector_type(8)));
+
+constexpr int BIG = 256;
+
+// 16-byte chunk exchange (xor) of a tile row: rows are 128 bytes apart, so two
+// fill the banks.  Fragments take 16 rows in order from x, and from w rows
+// 0-3, 16-19, 4-7, 20-23 (see wrow).
+DEVINL int xswz(int row) { return (row >> 1) & 7; }
+DEVINL int wswz(int row) { return ((row >> 1) & 3) | ((row >> 4) & 1) << 2; }
+// the MFMA's row i of 32 is y's column wrow(i): a lane then holds 16 neighbours
+DEVINL int wrow(int i) { return 16 * ((i >> 2) & 1) + (i & 3) + 4 * (i >> 3); }
+
+template <bool HAS_LORA, bool HAS_BIAS, bool VEC>
+__global__ __launch_bounds__(512, 2)
+void lora_gemm_big_kernel(const short* __restrict__ x, const short* __restrict__ w,
+                          const short* __restrict__ u, const short* __restrict__ b,
+                          const float* __restrict__ bias, short* __restrict__ y, int M, int N,
+                          int K1, int grid_m, int grid_n) {
+  __shared__ __attribute__((aligned(16))) short lds[2][2][BIG * 64];   // [buffer][x, w]
+  int wg = blockIdx.x;
+  {
+    const int nwg = gridDim.x, q = nwg >> 3, r = nwg & 7;
+    const int xcd = wg & 7, i = wg >> 3;
+    wg = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + i;
+  }
+  constexpr int GM = 8;       // tiles that run together share rows and columns
+  const int group = wg / (GM * grid_n), first = group * GM;
+  const int rows_here = min(GM, grid_m - first);
+  const int bm = first + (wg - group * GM * grid_n) % rows_here;
+  const int bn = (wg - group * GM * grid_n) / rows_here;
+  const int m0 = bm * BIG, n0 = bn * BIG;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wid >> 2) * 128, wn = (wid & 3) * 64;
+  const int lo = lane & 31, hi = lane >> 5;
+  const int n_k1 = K1 >> 6, n_kt = n_k1 + (HAS_LORA ? 1 : 0);
+
+  // thread's rows of a tile: tid / 8 + 64 i; its chunk of each the same
+  unsigned xo[4], wo[4];
+  auto offsets = [&](int ld) {
+    const int r = tid >> 3;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      xo[i] = (unsigned)(min(r + 64 * i, M - 1 - m0) * ld + (((tid & 7) ^ xswz(r)) << 3)) * 2;
+      wo[i] = (unsigned)(min(r + 64 * i, N - 1 - n0) * ld + (((tid & 7) ^ wswz(r)) << 3)) * 2;
+    }
+  };
+  offsets(K1);
+  const short *xb = x + (long)m0 * K1, *wb = w + (long)n0 * K1;
+  auto stage = [&](int kt, int buf) {
+    const short *xs = xb + kt * 64, *ws = wb + kt * 64;
+    if (HAS_LORA && kt == n_k1) {
+      offsets(64);
+      xs = u + (long)m0 * 64;
+      ws = b + (long)n0 * 64;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) load_to_lds16(xs, xo[i], &lds[buf][0][(i * 512 + wid * 64) * 8]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) load_to_lds16(ws, wo[i], &lds[buf][1][(i * 512 + wid * 64) * 8]);
+  };
+  const int xr = wm + lo, wr = wn + wrow(lo);
+  auto xfrag = [&](int buf, int mt, int ks) {
+    return *reinterpret_cast<const bf16x8_m*>(
+        &lds[buf][0][(xr + 32 * mt) * 64 + (((2 * ks + hi) ^ xswz(xr)) << 3)]);
+  };
+  auto wfrag = [&](int buf, int nt, int ks) {
+    return *reinterpret_cast<const bf16x8_m*>(
+        &lds[buf][1][(wr + 32 * nt) * 64 + (((2 * ks + hi) ^ wswz(wr)) << 3)]);
+  };
+
+  f32x16_l acc[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[i][j] = f32x16_l{};
+
+  stage(0, 0);
+  for (int kt = 0; kt < n_kt; kt++) {
+    const int buf = kt & 1;
+    wait_loads<0>();
+    __syncthreads();
+    bf16x8_m xf[2][4], wf[2][2];
+    auto read = [&](int ks) {
+#pragma unroll
+      for (int j = 0; j < 2; j++) wf[ks & 1][j] = wfrag(buf, j, ks);
+#pragma unroll
+      for (int i = 0; i < 4; i++) xf[ks & 1][i] = xfrag(buf, i, ks);
+    };
+    read(0);
+    if (kt + 1 < n_kt) stage(kt + 1, buf ^ 1);
+    // the next step's fragments are read between this one's products
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++) {
+      if (ks < 3) read(ks + 1);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[ks & 1][j], xf[ks & 1][i],
+                                                              acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int g = 0; g < 6; g++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // product
+        if (ks < 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);      // LDS read
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+    }
+  }
+  // lane: row m0 + wm + 32 i + lo, columns n0 + wn + 32 j + 16 hi + 0..15
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int gn = n0 + wn + 32 * j + 16 * hi;
+    float bv[16];
+    if (HAS_BIAS) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) bv[r] = bias[min(gn + r, N - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int gm = m0 + wm + 32 * i + lo;
+      if (gm >= M) continue;
+      short* dst = y + (long)gm * N + gn;
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        s16x8 o;
+#pragma unroll
+        for (int r = 0; r < 8; r++)
+          o[r] = f2bf(acc[i][j][8 * h + r] + (HAS_BIAS ? bv[8 * h + r] : 0.f));
+        if (VEC) {
+          if (gn + 8 * h < N) *reinterpret_cast<s16x8*>(dst + 8 * h) = o;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 8; r++)
+            if (gn + 8 * h + r < N) dst[8 * h + r] = o[r];
+        }
+      }
+    }
+  }
+}
+
 torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
                         c10::optional<torch::Tensor> u,
                         c10::optional<torch::Tensor> b,
@@ -182,6 +333,24 @@ torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
   const short* bp = has_lora ? (const short*)b->data_ptr() : nullptr;
   const float* biasp = has_bias ? bias_f.data_ptr<float>() : nullptr;
 
+  // 4096 x 1536 x 1536 (96 tiles of 256): 38 us in big tiles, 42 in small ones;
+  // with fewer the small ones fill more of the chip
+  const int big_m = (int)((M + BIG - 1) / BIG), big_n = (int)((N + BIG - 1) / BIG);
+  if ((long)big_m * big_n >= 96) {
+#define LAUNCH(HL, HB, VEC)                                                               \
+  hipLaunchKernelGGL((lora_gemm_big_kernel<HL, HB, VEC>), dim3(big_m * big_n), dim3(512), 0, \
+                     stream, (const short*)x.data_ptr(), (const short*)w.data_ptr(), up, bp, \
+                     biasp, (short*)y.data_ptr(), (int)M, (int)N, (int)K1, big_m, big_n)
+#define LAUNCH_V(HL, HB) do { if (N % 8 == 0) LAUNCH(HL, HB, true); else LAUNCH(HL, HB, false); } while (0)
+    if (has_lora && has_bias) LAUNCH_V(true, true);
+    else if (has_lora) LAUNCH_V(true, false);
+    else if (has_bias) LAUNCH_V(false, true);
+    else LAUNCH_V(false, false);
+#undef LAUNCH_V
+#undef LAUNCH
+    HIP_CHECK_LAST();
+    return y;
+  }
 #define LAUNCH(HL, HB)                                                        \
   hipLaunchKernelGGL((lora_gemm_kernel<HL, HB>), grid, block, 0, stream,      \
                      (const short*)x.data_ptr(), (const short*)w.data_ptr(),  \
@@ -201,8 +370,16 @@ torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
 // B:[N,64]).  Used when hipBLASLt wins the base GEMM (deep-K shapes): the
 // adapter contribution is ONE custom MFMA pass over y instead of two skinny
 // library GEMMs + an eager add (3 launches + an extra y round trip).
+//
+// Bound by reading and writing y.  The product is made transposed (columns of y
+// as the MFMA's rows, four of which a lane holds), and the columns are dealt to
+// the MFMA's rows so that two tiles of 16 give a lane 8 neighbours: y moves in 16
+// bytes per lane and 64 per row.  All of a lane's y is asked for before the
+// product.  48720 x 17920: 2.33 ms (1.5 TB/s) with one element per access,
+// 0.81 ms now; 48720 x 1536: 0.128 to 0.053 ms (5.6 TB/s).
 // ---------------------------------------------------------------------------
-__launch_bounds__(256, 4)
+template <bool VEC>
+__launch_bounds__(256, 3)
 __global__ void lora_add_kernel(short* __restrict__ y,
                                 const short* __restrict__ u,
                                 const short* __restrict__ b,
@@ -218,55 +395,75 @@ __global__ void lora_add_kernel(short* __restrict__ y,
   const int m0 = (wg / grid_n) * 128, n0 = (wg % grid_n) * 128;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int wm = wid >> 1, wn = wid & 1;
+  const int lo = lane & 15, hi = lane >> 4;
 
+  // rows of 64 elements are 128 bytes apart: their 16-byte chunks are exchanged
+  // (xor) by row, so that 16 rows at one chunk meet all banks
 #pragma unroll
   for (int rnd = 0; rnd < 4; ++rnd) {
     const int c = rnd * 256 + tid;
-    const int row = c >> 3, col = (c & 7) << 3;
+    const int row = c >> 3, col = ((c & 7) ^ ((row >> 1) & 7)) << 3;
     GLDS16(u + (long)min(m0 + row, M - 1) * 64 + col, &lds[0][c << 3]);
     GLDS16(b + (long)min(n0 + row, N - 1) * 64 + col, &lds[1][c << 3]);
   }
+  // y rows m0 + wm*64 + 16 mf + lo, columns n0 + wn*64 + 32 h + 8 hi .. + 7
+  const int nb = n0 + wn * 64 + 8 * hi;
+  bf16x8_l yv[4][2];
+  if constexpr (VEC) {
+#pragma unroll
+    for (int mf = 0; mf < 4; ++mf)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        yv[mf][h] = *reinterpret_cast<const bf16x8_l*>(
+            y + (long)min(m0 + wm * 64 + mf * 16 + lo, M - 1) * N + min(nb + 32 * h, N - 8));
+  }
   __syncthreads();
 
-  const int fr = lane & 15, fk = (lane >> 4) << 3;
-  f32x4_l acc[4][4];
+  auto at = [&](const short* t, int row, int chunk) {
+    return *reinterpret_cast<const bf16x8_l*>(t + row * 64 + ((chunk ^ ((row >> 1) & 7)) << 3));
+  };
+  f32x4_l acc[4][4];      // [mf][nf]: column of y 32 (nf/2) + 8 hi + 4 (nf%2) + r, row lo
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_l{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
-    bf16x8_l af[4], bf[4];
+    bf16x8_l uf[4], bf[4];
 #pragma unroll
-    for (int mf = 0; mf < 4; ++mf)
-      af[mf] = *reinterpret_cast<const bf16x8_l*>(
-          lds[0] + ((wm * 64 + mf * 16 + fr) << 6) + kk * 32 + fk);
+    for (int mf = 0; mf < 4; ++mf) uf[mf] = at(lds[0], wm * 64 + mf * 16 + lo, kk * 4 + hi);
 #pragma unroll
     for (int nf = 0; nf < 4; ++nf)
-      bf[nf] = *reinterpret_cast<const bf16x8_l*>(
-          lds[1] + ((wn * 64 + nf * 16 + fr) << 6) + kk * 32 + fk);
+      bf[nf] = at(lds[1], wn * 64 + 32 * (nf >> 1) + 8 * (lo >> 2) + 4 * (nf & 1) + (lo & 3),
+                  kk * 4 + hi);
 #pragma unroll
     for (int mf = 0; mf < 4; ++mf)
 #pragma unroll
       for (int nf = 0; nf < 4; ++nf)
-        acc[mf][nf] = mfma16(af[mf], bf[nf], acc[mf][nf]);
+        acc[mf][nf] = mfma16(bf[nf], uf[mf], acc[mf][nf]);
   }
 
-  const int crow0 = (lane >> 4) << 2;
 #pragma unroll
-  for (int nf = 0; nf < 4; ++nf) {
-    const int gn = n0 + wn * 64 + nf * 16 + fr;
-    if (gn >= N) continue;
+  for (int mf = 0; mf < 4; ++mf) {
+    const int gm = m0 + wm * 64 + mf * 16 + lo;
+    if (gm >= M) continue;
 #pragma unroll
-    for (int mf = 0; mf < 4; ++mf)
+    for (int h = 0; h < 2; ++h) {
+      short* dst = y + (long)gm * N + nb + 32 * h;
+      if (VEC) {
+        if (nb + 32 * h >= N) continue;
+        bf16x8_l o;
 #pragma unroll
-      for (int reg = 0; reg < 4; ++reg) {
-        const int gm = m0 + wm * 64 + mf * 16 + crow0 + reg;
-        if (gm < M) {
-          const long idx = (long)gm * N + gn;
-          y[idx] = f2bf(bf2f(y[idx]) + acc[mf][nf][reg]);
-        }
+        for (int j = 0; j < 8; ++j)
+          o[j] = f2bf(bf2f(yv[mf][h][j]) + acc[mf][2 * h + (j >> 2)][j & 3]);
+        *reinterpret_cast<bf16x8_l*>(dst) = o;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (nb + 32 * h + j < N)
+            dst[j] = f2bf(bf2f(dst[j]) + acc[mf][2 * h + (j >> 2)][j & 3]);
       }
+    }
   }
 }
 
@@ -278,8 +475,12 @@ void lora_add_(torch::Tensor y, torch::Tensor u, torch::Tensor b) {
   TORCH_CHECK(b.size(0) == N && b.size(1) == 64);
   const int grid_m = (int)((M + 127) / 128), grid_n = (int)((N + 127) / 128);
   auto stream = at::hip::getCurrentHIPStream();
-  hipLaunchKernelGGL(lora_add_kernel, dim3(grid_m * grid_n), dim3(256), 0, stream,
-                     (short*)y.data_ptr(), (const short*)u.data_ptr(),
-                     (const short*)b.data_ptr(), (int)M, (int)N, grid_n);
+  const bool vec = N % 8 == 0 && (uintptr_t)y.data_ptr() % 16 == 0;
+#define LAUNCH(VEC)                                                                      \
+  hipLaunchKernelGGL(lora_add_kernel<VEC>, dim3(grid_m * grid_n), dim3(256), 0, stream,  \
+                     (short*)y.data_ptr(), (const short*)u.data_ptr(),                   \
+                     (const short*)b.data_ptr(), (int)M, (int)N, grid_n)
+  if (vec) LAUNCH(true); else LAUNCH(false);
+#undef LAUNCH
   HIP_CHECK_LAST();
 }

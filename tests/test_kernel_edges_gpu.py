@@ -224,3 +224,31 @@ def test_latent_attention_page_edges(rp, heads, lens, capacity):
         want[i] = torch.softmax(q[i].double() @ c.t() * rp ** -0.5, -1) @ c
     # weights and result rounded to bf16 (0.0011 in the root mean square each)
     assert rel(got, want) < 0.006
+
+
+# ------------------------------------------------------------- LoRA epilogue
+@pytest.mark.parametrize("M,N", [(1, 8), (1, 1), (127, 130), (128, 1536), (129, 1001), (300, 72),
+                                 (257, 2056), (5, 264)])
+@pytest.mark.parametrize("shift", [0, 1])        # elements the rows start off 16 bytes
+def test_lora_add_edges(M, N, shift):
+    y = rnd(M * N + 1, seed=1)[shift:M * N + shift].view(M, N)
+    u, b = rnd(M, 64, seed=2), rnd(N, 64, seed=3, scale=0.1)
+    want = y.double() + u.double() @ b.double().t()
+    ops.ext().lora_add_(y, u, b)
+    assert rel(y, want) < 0.003                  # one rounding to bf16: 0.0011
+
+
+@pytest.mark.parametrize("M,N,K", [(3073, 2040, 64), (4000, 1537, 128), (257, 24584, 192),
+                                   (24577, 8, 64), (3328, 2049, 320)])
+@pytest.mark.parametrize("lora,bias", [(True, False), (True, True), (False, True), (False, False)])
+def test_lora_gemm_big_tile_edges(M, N, K, lora, bias):
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=K ** -0.5)
+    u, b = (rnd(M, 64, seed=3), rnd(N, 64, seed=4, scale=0.1)) if lora else (None, None)
+    c = rnd(N, seed=5) if bias else None
+    got = ops.ext().lora_gemm(x, w, u, b, c)
+    want = x.float() @ w.float().t()
+    if lora:
+        want += u.float() @ b.float().t()
+    if bias:
+        want += c.float()
+    assert rel(got, want) < 0.003                # one rounding to bf16: 0.0011
