@@ -8,6 +8,11 @@ std::vector<torch::Tensor> rmsnorm_bwd(torch::Tensor dy, torch::Tensor x,
 std::vector<torch::Tensor> rmsnorm_addres_fwd(torch::Tensor x, torch::Tensor res,
                                               torch::Tensor w, double eps);
 torch::Tensor rope_fwd(torch::Tensor x, torch::Tensor table, torch::Tensor positions, double sign);
+std::vector<torch::Tensor> qkv_rope_fwd(torch::Tensor qkv, torch::Tensor table,
+                                        torch::Tensor positions, long Hq, long Hkv);
+torch::Tensor qkv_rope_bwd(c10::optional<torch::Tensor> dq, c10::optional<torch::Tensor> dk,
+                           c10::optional<torch::Tensor> dv, torch::Tensor table,
+                           torch::Tensor positions, long Hq, long Hkv);
 torch::Tensor swiglu_fwd(torch::Tensor gu);
 torch::Tensor swiglu_bwd(torch::Tensor dy, torch::Tensor gu);
 // logprob.hip
@@ -47,6 +52,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm_bwd", &rmsnorm_bwd);
   m.def("rmsnorm_addres_fwd", &rmsnorm_addres_fwd);
   m.def("rope_fwd", &rope_fwd);
+  m.def("qkv_rope_fwd", &qkv_rope_fwd);
+  m.def("qkv_rope_bwd", &qkv_rope_bwd);
   m.def("swiglu_fwd", &swiglu_fwd);
   m.def("swiglu_bwd", &swiglu_bwd);
   m.def("ce_rowstats", &ce_rowstats);

@@ -7,6 +7,7 @@
 
 #include "common.h"
 #include "checks.h"
+#include "qkv.h"
 
 // ------------------------------------------------------------- RMSNorm fwd
 // x [N, H] bf16 -> y [N, H] bf16, invrms [N] f32.  One 256-thread block/row.
@@ -257,6 +258,71 @@ torch::Tensor rope_fwd(torch::Tensor x, torch::Tensor table, torch::Tensor posit
                      positions.data_ptr<long>(), T, Hh, D, (float)sign);
   HIP_CHECK_LAST();
   return y;
+}
+
+static void check_rope(const torch::Tensor& table, const torch::Tensor& positions, long T, int D) {
+  on_gpu({table, positions});
+  TORCH_CHECK(table.scalar_type() == torch::kFloat32 && table.is_contiguous() &&
+              table.size(-1) == D, "rope table must be fp32 [positions, head_dim]");
+  TORCH_CHECK(positions.scalar_type() == torch::kLong && positions.is_contiguous() &&
+              positions.numel() == T, "positions must be int64, one per token");
+  TORCH_CHECK(D % 16 == 0, "head_dim must be divisible by 16");
+}
+
+// qkv [T, (Hq + 2 Hkv) D] -> q [T, Hq, D], k and v [T, Hkv, D], q and k rotated
+std::vector<torch::Tensor> qkv_rope_fwd(torch::Tensor qkv, torch::Tensor table,
+                                        torch::Tensor positions, long Hq, long Hkv) {
+  check_bf16(qkv, "qkv");
+  TORCH_CHECK(qkv.dim() == 2 && Hq > 0 && Hkv > 0 && qkv.size(1) % (Hq + 2 * Hkv) == 0);
+  const long T = qkv.size(0), D = qkv.size(1) / (Hq + 2 * Hkv);
+  check_rope(table, positions, T, (int)D);
+  if ((uintptr_t)qkv.data_ptr() % 16) qkv = qkv.clone();
+  auto q = torch::empty({T, Hq, D}, qkv.options());
+  auto k = torch::empty({T, Hkv, D}, qkv.options()), v = torch::empty_like(k);
+  auto stream = at::hip::getCurrentHIPStream();
+  by_tokens(T, (Hq + 2 * Hkv) * (D / 16), [&](long t0, unsigned units) {
+    QkvRope a{};
+    a.qkv = (const short*)qkv.data_ptr() + t0 * qkv.size(1);
+    a.q = (short*)q.data_ptr() + t0 * Hq * D;
+    a.k = (short*)k.data_ptr() + t0 * Hkv * D;
+    a.v = (short*)v.data_ptr() + t0 * Hkv * D;
+    a.table = table.data_ptr<float>();
+    a.pos = positions.data_ptr<long>() + t0;
+    a.Hq = Hq;
+    a.Hkv = Hkv;
+    a.D = D;
+    hipLaunchKernelGGL(qkv_rope_kernel<void>, dim3((units + 255) / 256), dim3(256), 0, stream, a,
+                       units);
+  });
+  HIP_CHECK_LAST();
+  return {q, k, v};
+}
+
+torch::Tensor qkv_rope_bwd(c10::optional<torch::Tensor> dq, c10::optional<torch::Tensor> dk,
+                           c10::optional<torch::Tensor> dv, torch::Tensor table,
+                           torch::Tensor positions, long Hq, long Hkv) {
+  const long T = positions.numel(), D = table.size(-1);
+  check_rope(table, positions, T, (int)D);
+  auto ptr = [&](c10::optional<torch::Tensor>& x, long H) -> const short* {
+    if (!x.has_value()) return nullptr;
+    check_bf16(*x, "gradient");
+    TORCH_CHECK(x->numel() == T * H * D, "gradient has another shape");
+    if ((uintptr_t)x->data_ptr() % 16) x = x->clone();
+    return (const short*)x->data_ptr();
+  };
+  const short *q = ptr(dq, Hq), *k = ptr(dk, Hkv), *v = ptr(dv, Hkv);
+  auto out = torch::empty({T, (Hq + 2 * Hkv) * D}, table.options().dtype(torch::kBFloat16));
+  auto stream = at::hip::getCurrentHIPStream();
+  by_tokens(T, (Hq + 2 * Hkv) * (D / 16), [&](long t0, unsigned units) {
+    auto from = [&](const short* p, long H) { return p ? p + t0 * H * D : nullptr; };
+    hipLaunchKernelGGL(qkv_rope_bwd_kernel, dim3((units + 255) / 256), dim3(256), 0, stream,
+                       from(q, Hq), from(k, Hkv), from(v, Hkv), table.data_ptr<float>(),
+                       positions.data_ptr<long>() + t0,
+                       (short*)out.data_ptr() + t0 * (Hq + 2 * Hkv) * D, (int)Hq, (int)Hkv, (int)D,
+                       units);
+  });
+  HIP_CHECK_LAST();
+  return out;
 }
 
 torch::Tensor swiglu_fwd(torch::Tensor gu) {

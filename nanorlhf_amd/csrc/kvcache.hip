@@ -16,6 +16,7 @@
 
 #include "common.h"
 #include "checks.h"
+#include "qkv.h"
 
 typedef __bf16 bf16x8k __attribute__((ext_vector_type(8)));
 typedef int i32x2k __attribute__((ext_vector_type(2)));
@@ -118,6 +119,58 @@ void kv_append(torch::Tensor k, torch::Tensor v, torch::Tensor slots,
     TORCH_CHECK(false, "kv cache must be bf16 or fp8_e4m3fn");
   }
   HIP_CHECK_LAST();
+}
+
+// qkv [T, (Hq + 2 Hkv) D]: q and k rotated, k and v into the cache at `slots`.
+// Returns q [T, Hq, D], and k and v [T, Hkv, D] if asked for.
+std::vector<torch::Tensor> qkv_rope_append(torch::Tensor qkv, torch::Tensor table,
+                                           torch::Tensor positions, torch::Tensor slots,
+                                           torch::Tensor k_cache, torch::Tensor v_cache, long Hq,
+                                           bool want_kv) {
+  on_gpu({qkv, table, positions, slots, k_cache, v_cache});
+  TORCH_CHECK(qkv.scalar_type() == torch::kBFloat16 && qkv.is_contiguous() && qkv.dim() == 2);
+  TORCH_CHECK(k_cache.dim() == 4 && k_cache.is_contiguous() && v_cache.is_contiguous() &&
+              v_cache.scalar_type() == k_cache.scalar_type());
+  const long T = qkv.size(0), ps = k_cache.size(1), Hkv = k_cache.size(2), D = k_cache.size(3);
+  TORCH_CHECK(Hq > 0 && qkv.size(1) == (Hq + 2 * Hkv) * D && D % 32 == 0);
+  TORCH_CHECK(v_cache.size(1) == Hkv && v_cache.size(2) == D && v_cache.size(3) == ps);
+  TORCH_CHECK(table.scalar_type() == torch::kFloat32 && table.is_contiguous() &&
+              table.size(-1) == D, "rope table must be fp32 [positions, head_dim]");
+  TORCH_CHECK(positions.scalar_type() == torch::kLong && positions.is_contiguous() &&
+              positions.numel() == T, "positions must be int64, one per token");
+  TORCH_CHECK(slots.scalar_type() == torch::kLong && slots.is_contiguous() && slots.numel() == T);
+  if ((uintptr_t)qkv.data_ptr() % 16) qkv = qkv.clone();
+  auto q = torch::empty({T, Hq, D}, qkv.options());
+  std::vector<torch::Tensor> out{q};
+  if (want_kv)
+    for (int i = 0; i < 2; i++) out.push_back(torch::empty({T, Hkv, D}, qkv.options()));
+  auto stream = at::hip::getCurrentHIPStream();
+  const bool fp8 = k_cache.scalar_type() == torch::kFloat8_e4m3fn;
+  TORCH_CHECK(fp8 || k_cache.scalar_type() == torch::kBFloat16,
+              "kv cache must be bf16 or fp8_e4m3fn");
+  by_tokens(T, (Hq + 2 * Hkv) * (D / 16), [&](long t0, unsigned units) {
+    QkvRope a{};
+    a.qkv = (const short*)qkv.data_ptr() + t0 * qkv.size(1);
+    a.q = (short*)q.data_ptr() + t0 * Hq * D;
+    if (want_kv) {
+      a.k = (short*)out[1].data_ptr() + t0 * Hkv * D;
+      a.v = (short*)out[2].data_ptr() + t0 * Hkv * D;
+    }
+    a.table = table.data_ptr<float>();
+    a.pos = positions.data_ptr<long>() + t0;
+    a.slots = slots.data_ptr<long>() + t0;
+    a.kc = k_cache.data_ptr();
+    a.vc = v_cache.data_ptr();
+    a.Hq = Hq;
+    a.Hkv = Hkv;
+    a.D = D;
+    a.ps = ps;
+    const dim3 grid((units + 255) / 256), block(256);
+    if (fp8) hipLaunchKernelGGL(qkv_rope_kernel<unsigned char>, grid, block, 0, stream, a, units);
+    else hipLaunchKernelGGL(qkv_rope_kernel<short>, grid, block, 0, stream, a, units);
+  });
+  HIP_CHECK_LAST();
+  return out;
 }
 
 // ------------------------------------------------------- decode attention

@@ -8,6 +8,10 @@ using OptTensor = c10::optional<torch::Tensor>;
 // kvcache.hip
 void kv_append(torch::Tensor k, torch::Tensor v, torch::Tensor slots,
                torch::Tensor k_cache, torch::Tensor v_cache);
+std::vector<torch::Tensor> qkv_rope_append(torch::Tensor qkv, torch::Tensor table,
+                                           torch::Tensor positions, torch::Tensor slots,
+                                           torch::Tensor k_cache, torch::Tensor v_cache, long Hq,
+                                           bool want_kv);
 torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor k_cache,
                                 torch::Tensor v_cache, torch::Tensor block_tables,
                                 torch::Tensor seq_lens, double scale);
@@ -84,6 +88,7 @@ torch::Tensor moe_down(torch::Tensor act, torch::Tensor down, torch::Tensor list
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_append", &kv_append);
+  m.def("qkv_rope_append", &qkv_rope_append);
   m.def("paged_attn_decode", &paged_attn_decode);
   m.def("paged_attn_decode_window", &paged_attn_decode_window);
   m.def("paged_attn_varlen", &paged_attn_varlen);

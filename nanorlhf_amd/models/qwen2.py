@@ -103,16 +103,13 @@ class Attention(nn.Module):
     def forward(self, x: torch.Tensor, rope_table: torch.Tensor, ctx: AttnContext):
         T = x.shape[0]
         qkv = self.qkv_proj(x)
-        q = qkv[:, : self.q_size].reshape(T, self.num_heads, self.head_dim)
-        k = qkv[:, self.q_size: self.q_size + self.kv_size].reshape(
-            T, self.num_kv_heads, self.head_dim)
-        v = qkv[:, self.q_size + self.kv_size:].reshape(T, self.num_kv_heads, self.head_dim)
-        q = ops.rope_apply(q, rope_table, ctx.positions)
-        k = ops.rope_apply(k, rope_table, ctx.positions)
-
         if ctx.mode != "train" and ctx.kv_caches is not None:
-            k_cache, v_cache = ctx.kv_caches[self.layer_idx]
-            ops.kv_append(k, v, ctx.slots, k_cache, v_cache)
+            q, k, v = ops.qkv_rope_append(qkv, rope_table, ctx.positions, self.num_heads,
+                                          ctx.slots, *ctx.kv_caches[self.layer_idx],
+                                          want_kv=ctx.mode not in ("decode", "step"))
+        else:
+            q, k, v = ops.qkv_rope(qkv, rope_table, ctx.positions, self.num_heads,
+                                   self.num_kv_heads)
 
         if ctx.mode == "decode":
             o = ops.paged_attn_decode(q, *ctx.kv_caches[self.layer_idx],

@@ -55,14 +55,14 @@ def ext_available() -> bool:
 
 from .rmsnorm import (add_rms_norm, gated_norm, residual_group_norm,  # noqa: E402,F401
                       rms_norm)
-from .rope import Rotation, build_rope_cache, rope_apply  # noqa: E402,F401
+from .rope import Rotation, build_rope_cache, qkv_rope, rope_apply  # noqa: E402,F401
 from .swiglu import gelu_glu, relu_squared_, swiglu  # noqa: E402,F401
 from .attention import flash_attn_varlen  # noqa: E402,F401
 from .logprob import token_logprob_entropy  # noqa: E402,F401
 from .adamw import FusedAdamW  # noqa: E402,F401
 from .sampling import sample_tokens  # noqa: E402,F401
 from .kvcache import (kv_append, paged_attn, paged_attn_decode,  # noqa: E402,F401
-                      pad_head_dim, rotary_qkv)
+                      pad_head_dim, qkv_rope_append, rotary_qkv)
 from .latent import latent_append, latent_attn, pad_latent  # noqa: E402,F401
 from .moe import group_linear, moe_experts, moe_route, stacked_linear  # noqa: E402,F401
 from .wkv import token_shift, wkv, wkv_decay  # noqa: E402,F401

@@ -19,7 +19,7 @@ from __future__ import annotations
 import torch
 
 from . import serve_ext
-from .rope import rotate_pairs
+from .rope import qkv_rope, rotate_pairs
 
 
 def kv_append(k: torch.Tensor, v: torch.Tensor, slots: torch.Tensor,
@@ -41,6 +41,20 @@ def kv_append(k: torch.Tensor, v: torch.Tensor, slots: torch.Tensor,
     offs = slots % ps
     # v_cache[page, h, d, off] = v[t, h, d]
     v_cache[pages, :, :, offs] = v
+
+
+def qkv_rope_append(qkv: torch.Tensor, table: torch.Tensor, positions: torch.Tensor, heads: int,
+                    slots: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                    want_kv: bool = True):
+    """qkv_rope, and kv_append of its k and v.  Returns (q, k, v), k and v None
+    unless wanted."""
+    if qkv.is_cuda and not (torch.is_grad_enabled() and qkv.requires_grad):
+        out = serve_ext().qkv_rope_append(qkv.contiguous(), table, positions, slots, k_cache,
+                                          v_cache, heads, want_kv)
+        return tuple(out) if want_kv else (out[0], None, None)
+    q, k, v = qkv_rope(qkv, table, positions, heads, k_cache.shape[2])
+    kv_append(k, v, slots, k_cache, v_cache)
+    return (q, k, v) if want_kv else (q, None, None)
 
 
 def _fp8_k_perm(D: int) -> torch.Tensor:

@@ -61,6 +61,37 @@ def rope_apply(x: torch.Tensor, table: torch.Tensor, positions: torch.Tensor) ->
     return _rope_ref(x, table, positions)
 
 
+class _QkvRopeFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, qkv, table, positions, heads, kv_heads):
+        ctx.save_for_backward(table, positions)
+        ctx.heads = heads, kv_heads
+        return tuple(ext().qkv_rope_fwd(qkv, table, positions, heads, kv_heads))
+
+    @staticmethod
+    def backward(ctx, *grads):
+        table, positions = ctx.saved_tensors
+        grads = [None if g is None else g.contiguous() for g in grads]
+        return ext().qkv_rope_bwd(*grads, table, positions, *ctx.heads), None, None, None, None
+
+
+def split_qkv(qkv: torch.Tensor, heads: int, kv_heads: int):
+    """q [T, heads, D], k and v [T, kv_heads, D] of a joint projection's rows."""
+    n = heads + 2 * kv_heads
+    parts = qkv.unflatten(1, (n, qkv.shape[1] // n))
+    return parts.split([heads, kv_heads, kv_heads], dim=1)
+
+
+def qkv_rope(qkv: torch.Tensor, table: torch.Tensor, positions: torch.Tensor, heads: int,
+             kv_heads: int):
+    """qkv [T, (heads + 2 kv_heads) D], the heads of q, then k's, then v's: split,
+    with q and k rotated as by rope_apply."""
+    if qkv.is_cuda and qkv.shape[1] // (heads + 2 * kv_heads) % 16 == 0:
+        return _QkvRopeFn.apply(qkv.contiguous(), table, positions, heads, kv_heads)
+    q, k, v = split_qkv(qkv, heads, kv_heads)
+    return (rope_apply(q, table, positions), rope_apply(k, table, positions), v)
+
+
 class Rotation:
     """Rotary positions over the first `dims` dimensions, in either layout of
     pairs: rotate-half (i with i + dims/2) or interleaved (2i with 2i + 1).

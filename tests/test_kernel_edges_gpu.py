@@ -252,3 +252,49 @@ def test_lora_gemm_big_tile_edges(M, N, K, lora, bias):
     if bias:
         want += c.float()
     assert rel(got, want) < 0.003                # one rounding to bf16: 0.0011
+
+
+# ------------------------------------------------- q, k, v of a projection
+@pytest.mark.parametrize("hq,hkv,d", [(12, 2, 128), (14, 2, 64), (4, 4, 32), (3, 1, 16)])
+@pytest.mark.parametrize("T", [1, 7, 500])
+def test_qkv_rope_matches_its_parts(hq, hkv, d, T):
+    from nanorlhf_amd.ops.rope import _rope_ref, split_qkv
+    table = ops.build_rope_cache(d, 600, device=DEV)
+    pos = torch.randint(0, 600, (T,), device=DEV)
+    x = rnd(T, (hq + 2 * hkv) * d, seed=T).requires_grad_(True)
+    got = ops.qkv_rope(x, table, pos, hq, hkv)
+    y = x.detach().float().requires_grad_(True)
+    q, k, v = split_qkv(y, hq, hkv)
+    want = (_rope_ref(q, table, pos), _rope_ref(k, table, pos), v)
+    grads = [rnd(*t.shape, seed=i) for i, t in enumerate(want)]
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and rel(a, b) < 0.003      # one rounding to bf16
+    torch.autograd.backward(got, grads)
+    torch.autograd.backward(want, [g.float() for g in grads])
+    assert rel(x.grad, y.grad) < 0.003
+    x.grad = None
+    ops.qkv_rope(x, table, pos, hq, hkv)[2].backward(grads[2])   # v alone
+    assert torch.equal(x.grad[:, (hq + hkv) * d:], grads[2].flatten(1))
+    assert not x.grad[:, :(hq + hkv) * d].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("hq,hkv,d", [(12, 2, 128), (14, 2, 64), (4, 4, 32)])
+def test_qkv_rope_append_fills_the_cache_as_kv_append_does(dtype, hq, hkv, d):
+    T, P = 100, 12
+    table = ops.build_rope_cache(d, 600, device=DEV)
+    pos = torch.randint(0, 600, (T,), device=DEV)
+    slots = torch.randperm(P * 16, device=DEV)[:T]
+    x = rnd(T, (hq + 2 * hkv) * d, seed=3)
+    kc, vc = (torch.zeros(P, 16, hkv, d, device=DEV).to(dtype),
+              torch.zeros(P, hkv, d, 16, device=DEV).to(dtype))
+    kr, vr = kc.clone(), vc.clone()
+    with torch.no_grad():
+        q, k, v = ops.qkv_rope_append(x, table, pos, hq, slots, kc, vc)
+        ref = ops.qkv_rope(x, table, pos, hq, hkv)
+        ops.kv_append(ref[1], ref[2], slots, kr, vr)
+        alone = ops.qkv_rope_append(x, table, pos, hq, slots, kc, vc, want_kv=False)
+    assert all(torch.equal(a, b) for a, b in zip((q, k, v), ref))
+    assert torch.equal(alone[0], q) and alone[1] is None
+    assert torch.equal(kc.view(torch.uint8), kr.view(torch.uint8))
+    assert torch.equal(vc.view(torch.uint8), vr.view(torch.uint8))
