@@ -8,6 +8,8 @@
 // rows and 96 tokens through 6 layers went from 95 to 86 ms.
 #pragma once
 
+#include <hip/hip_runtime.h>
+
 #include "common.h"
 
 struct QkvRope {
