@@ -4,7 +4,8 @@
 // elementwise.hip
 std::vector<torch::Tensor> rmsnorm_fwd(torch::Tensor x, torch::Tensor w, double eps);
 std::vector<torch::Tensor> rmsnorm_bwd(torch::Tensor dy, torch::Tensor x,
-                                       torch::Tensor w, torch::Tensor invrms);
+                                       torch::Tensor w, torch::Tensor invrms,
+                                       c10::optional<torch::Tensor> extra, bool want_dw);
 std::vector<torch::Tensor> rmsnorm_addres_fwd(torch::Tensor x, torch::Tensor res,
                                               torch::Tensor w, double eps);
 torch::Tensor rope_fwd(torch::Tensor x, torch::Tensor table, torch::Tensor positions, double sign);
@@ -49,7 +50,8 @@ std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm_fwd", &rmsnorm_fwd);
-  m.def("rmsnorm_bwd", &rmsnorm_bwd);
+  m.def("rmsnorm_bwd", &rmsnorm_bwd, py::arg("dy"), py::arg("x"), py::arg("w"),
+        py::arg("invrms"), py::arg("extra") = py::none(), py::arg("want_dw") = true);
   m.def("rmsnorm_addres_fwd", &rmsnorm_addres_fwd);
   m.def("rope_fwd", &rope_fwd);
   m.def("qkv_rope_fwd", &qkv_rope_fwd);

@@ -46,66 +46,112 @@ __global__ void rmsnorm_fwd_kernel(const short* __restrict__ x,
 }
 
 // ------------------------------------------------------------- RMSNorm bwd
-// dx = inv * (g - x_hat * mean(g * x_hat)),  g = dy*w,  x_hat = x*inv
-// Each block processes ROWS_PER_BLOCK rows; every thread owns fixed column
-// slices, accumulating its dw partial in REGISTERS across the block's rows
-// (no per-element atomics — the atomic version measured 1.0 ms/call from
-// contention), then one global atomicAdd per element per block.
-template <int BLOCK>
-__global__ void rmsnorm_bwd_kernel(const short* __restrict__ dy,
-                                   const short* __restrict__ x,
-                                   const short* __restrict__ w,
-                                   const float* __restrict__ invrms,
-                                   short* __restrict__ dx,
-                                   float* __restrict__ dw,  // [H]
-                                   long N, int H, int rows_per_block) {
-  __shared__ float scratch[BLOCK / 64];
-  constexpr int MAX_SLICES = 4;  // supports H up to BLOCK*8*4 = 8192
-  const int nvec = H / 8;
-  float dwacc[MAX_SLICES][8];
+// dx = inv * (g - x_hat * mean(g * x_hat)) [+ extra],  g = dy*w,  x_hat = x*inv
+// `extra` is what the residual stream's later consumers add to dx.  A row is held
+// in registers between the mean and dx: by one wave up to H = 2048 (no barrier),
+// else by the workgroup.  With DW, a workgroup sums dw over its rows and leaves
+// the sums in part [workgroups, H] for rmsnorm_dw_kernel: no atomics, one order.
+//
+// Bound by memory: three or four passes over [N, H].  48720 x 1536 without dw: 96 us
+// with the addition, where reading every row twice and 1024 workgroups'
+// atomics on dw took 306 and the addition 75 more.
+template <int WAVES, int SL, bool DW>     // waves of a row, vectors of 8 per lane
+__global__ __launch_bounds__(256)
+void rmsnorm_bwd_kernel(const short* __restrict__ dy,
+                        const short* __restrict__ x,
+                        const short* __restrict__ w,
+                        const float* __restrict__ invrms,
+                        const short* __restrict__ extra,   // or null
+                        short* __restrict__ dx,
+                        float* __restrict__ part,
+                        long N, int H) {
+  __shared__ float scratch[4];
+  __shared__ float sums[DW && WAVES == 1 ? 4 * 64 * SL * 8 : 1];
+  constexpr int LANES = 64 * WAVES, ROWS = 4 / WAVES;
+  const int nvec = H / 8, l = threadIdx.x % LANES;
+  float dwacc[SL][8];
+  s16x8 wv[SL];
 #pragma unroll
-  for (int sl = 0; sl < MAX_SLICES; sl++)
+  for (int k = 0; k < SL; k++) {
+    const int i = l + LANES * k;
+    wv[k] = i < nvec ? *reinterpret_cast<const s16x8*>(w + i * 8) : s16x8{};
 #pragma unroll
-    for (int j = 0; j < 8; j++) dwacc[sl][j] = 0.f;
-
-  const long row0 = (long)blockIdx.x * rows_per_block;
-  const long row1 = min(row0 + rows_per_block, N);
-  for (long row = row0; row < row1; row++) {
-    const short* dyr = dy + row * (long)H;
-    const short* xr = x + row * (long)H;
-    short* dxr = dx + row * (long)H;
-    const float inv = invrms[row];
+    for (int j = 0; j < 8; j++) dwacc[k][j] = 0.f;
+  }
+  for (long row = (long)blockIdx.x * ROWS + threadIdx.x / LANES;
+       WAVES > 1 ? row < N : row - threadIdx.x / LANES < N; row += (long)gridDim.x * ROWS) {
+    const bool ok = row < N;
+    const long at = min(row, N - 1) * H;
+    const float inv = invrms[min(row, N - 1)];
+    s16x8 dv[SL], xv[SL], ev[SL];
     float dot = 0.f;
-    for (int i = threadIdx.x; i < nvec; i += BLOCK) {
-      s16x8 dv = *reinterpret_cast<const s16x8*>(dyr + i * 8);
-      s16x8 xv = *reinterpret_cast<const s16x8*>(xr + i * 8);
-      s16x8 wv = *reinterpret_cast<const s16x8*>(w + i * 8);
 #pragma unroll
-      for (int j = 0; j < 8; j++)
-        dot += bf2f(dv[j]) * bf2f(wv[j]) * bf2f(xv[j]) * inv;
+    for (int k = 0; k < SL; k++) {
+      const int i = l + LANES * k;
+      if (i < nvec) {
+        dv[k] = *reinterpret_cast<const s16x8*>(dy + at + i * 8);
+        xv[k] = *reinterpret_cast<const s16x8*>(x + at + i * 8);
+        if (extra) ev[k] = *reinterpret_cast<const s16x8*>(extra + at + i * 8);
+      }
     }
-    dot = block_sum<BLOCK>(dot, scratch) / (float)H;
-    int sl = 0;
-    for (int i = threadIdx.x; i < nvec; i += BLOCK, sl++) {
-      s16x8 dv = *reinterpret_cast<const s16x8*>(dyr + i * 8);
-      s16x8 xv = *reinterpret_cast<const s16x8*>(xr + i * 8);
-      s16x8 wv = *reinterpret_cast<const s16x8*>(w + i * 8);
+#pragma unroll
+    for (int k = 0; k < SL; k++)
+      if (l + LANES * k < nvec)
+#pragma unroll
+        for (int j = 0; j < 8; j++) dot += bf2f(dv[k][j]) * bf2f(wv[k][j]) * bf2f(xv[k][j]) * inv;
+    dot = (WAVES == 1 ? wave_sum(dot) : block_sum<256>(dot, scratch)) / (float)H;
+    if (!ok) continue;
+#pragma unroll
+    for (int k = 0; k < SL; k++) {
+      const int i = l + LANES * k;
+      if (i >= nvec) continue;
       s16x8 o;
 #pragma unroll
       for (int j = 0; j < 8; j++) {
-        const float xh = bf2f(xv[j]) * inv;
-        const float g = bf2f(dv[j]) * bf2f(wv[j]);
-        o[j] = f2bf((g - xh * dot) * inv);
-        if (sl < MAX_SLICES) dwacc[sl][j] += bf2f(dv[j]) * bf2f(f2bf(xh));
+        const float xh = bf2f(xv[k][j]) * inv;
+        const float g = bf2f(dv[k][j]) * bf2f(wv[k][j]);
+        const float d = (g - xh * dot) * inv;
+        o[j] = f2bf(extra ? d + bf2f(ev[k][j]) : d);
+        if (DW) dwacc[k][j] += bf2f(dv[k][j]) * bf2f(f2bf(xh));
       }
-      *reinterpret_cast<s16x8*>(dxr + i * 8) = o;
+      *reinterpret_cast<s16x8*>(dx + at + i * 8) = o;
     }
   }
-  // drain register partials: one atomic per element per block
-  int sl = 0;
-  for (int i = threadIdx.x; i < nvec && sl < MAX_SLICES; i += BLOCK, sl++) {
+  if constexpr (DW) {
+    float* out = part + (long)blockIdx.x * H;
+    if constexpr (WAVES == 1) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) atomicAdd(&dw[i * 8 + j], dwacc[sl][j]);
+      for (int k = 0; k < SL; k++)
+#pragma unroll
+        for (int j = 0; j < 8; j++) sums[(threadIdx.x / 64 * SL + k) * 512 + j * 64 + l] = dwacc[k][j];
+      __syncthreads();
+      for (int i = threadIdx.x; i < H; i += 256) {
+        const int v = i / 8, at = v / 64 * 512 + i % 8 * 64 + v % 64;
+        float t = 0.f;
+        for (int q = 0; q < 4; q++) t += sums[q * SL * 512 + at];
+        out[i] = t;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < SL; k++)
+        if (l + LANES * k < nvec) stv<8>(out + (l + LANES * k) * 8, dwacc[k]);
+    }
+  }
+}
+
+// column sums of part [n, H]: 64 columns per workgroup, 16 rows at a time
+__global__ __launch_bounds__(1024) void rmsnorm_dw_kernel(const float* __restrict__ part,
+                                                          short* __restrict__ dw, int n, int H) {
+  __shared__ float sums[16][64];
+  const int c = blockIdx.x * 64 + (threadIdx.x & 63), r = threadIdx.x >> 6;
+  float t = 0.f;
+  if (c < H)
+    for (int i = r; i < n; i += 16) t += part[(long)i * H + c];
+  sums[r][threadIdx.x & 63] = t;
+  __syncthreads();
+  if (r == 0 && c < H) {
+    for (int i = 1; i < 16; i++) t += sums[i][threadIdx.x];
+    dw[c] = f2bf(t);
   }
 }
 
@@ -216,25 +262,49 @@ std::vector<torch::Tensor> rmsnorm_fwd(torch::Tensor x, torch::Tensor w, double 
   return {y, invrms};
 }
 
+// dx and, if wanted, dw (else an empty tensor).  extra: added to dx.
 std::vector<torch::Tensor> rmsnorm_bwd(torch::Tensor dy, torch::Tensor x,
-                                       torch::Tensor w, torch::Tensor invrms) {
+                                       torch::Tensor w, torch::Tensor invrms,
+                                       c10::optional<torch::Tensor> extra, bool want_dw) {
   check_bf16(dy, "dy"); check_bf16(x, "x"); check_bf16(w, "w");
   const int H = x.size(-1);
   const long N = x.numel() / H;
-  TORCH_CHECK(H <= 256 * 8 * 4, "hidden too large for rmsnorm_bwd slices");
+  TORCH_CHECK(H % 8 == 0 && H <= 256 * 8 * 4, "hidden too large for rmsnorm_bwd slices");
+  TORCH_CHECK(dy.sizes() == x.sizes() && w.numel() == H && invrms.numel() == N);
+  const short* ep = nullptr;
+  if (extra.has_value()) {
+    check_bf16(*extra, "extra");
+    TORCH_CHECK(extra->sizes() == x.sizes());
+    ep = (const short*)extra->data_ptr();
+  }
   auto dx = torch::empty_like(x);
-  auto dwf = torch::zeros({H}, x.options().dtype(torch::kFloat32));
+  auto dw = want_dw ? torch::empty({H}, x.options()) : torch::empty({0}, x.options());
+  if (N == 0) return {dx, want_dw ? dw.zero_() : dw};
   auto stream = at::hip::getCurrentHIPStream();
-  // ~4 blocks/CU worth of parallelism; more rows per block = fewer atomics
-  const int rows_per_block = (int)std::max<long>(1, (N + 1023) / 1024);
-  const long grid = (N + rows_per_block - 1) / rows_per_block;
-  hipLaunchKernelGGL((rmsnorm_bwd_kernel<256>), dim3(grid), dim3(256), 0, stream,
-                     (const short*)dy.data_ptr(), (const short*)x.data_ptr(),
-                     (const short*)w.data_ptr(), invrms.data_ptr<float>(),
-                     (short*)dx.data_ptr(), dwf.data_ptr<float>(), N, H,
-                     rows_per_block);
+  // without dw a workgroup per row (or four); with it, 512 share the rows
+  const long most = (N + (H <= 2048 ? 3 : 0)) / (H <= 2048 ? 4 : 1);
+  const long grid = want_dw ? std::min<long>(most, 512) : std::min<long>(most, 1 << 20);
+  torch::Tensor part;
+  if (want_dw) part = torch::empty({grid, H}, x.options().dtype(torch::kFloat32));
+  float* pp = want_dw ? part.data_ptr<float>() : nullptr;
+#define LAUNCH(WAVES, SL, DW)                                                             \
+  hipLaunchKernelGGL((rmsnorm_bwd_kernel<WAVES, SL, DW>), dim3(grid), dim3(256), 0, stream, \
+                     (const short*)dy.data_ptr(), (const short*)x.data_ptr(),             \
+                     (const short*)w.data_ptr(), invrms.data_ptr<float>(), ep,            \
+                     (short*)dx.data_ptr(), pp, N, H)
+#define LAUNCH_DW(WAVES, SL) do { if (want_dw) LAUNCH(WAVES, SL, true); else LAUNCH(WAVES, SL, false); } while (0)
+  if (H <= 512) LAUNCH_DW(1, 1);
+  else if (H <= 1024) LAUNCH_DW(1, 2);
+  else if (H <= 2048) LAUNCH_DW(1, 4);
+  else if (H <= 4096) LAUNCH_DW(4, 2);
+  else LAUNCH_DW(4, 4);
+#undef LAUNCH_DW
+#undef LAUNCH
+  if (want_dw)
+    hipLaunchKernelGGL(rmsnorm_dw_kernel, dim3((H + 63) / 64), dim3(1024), 0, stream, pp,
+                       (short*)dw.data_ptr(), (int)grid, H);
   HIP_CHECK_LAST();
-  return {dx, dwf.to(torch::kBFloat16)};
+  return {dx, dw};
 }
 
 torch::Tensor rope_fwd(torch::Tensor x, torch::Tensor table, torch::Tensor positions,

@@ -26,8 +26,9 @@ class _RMSNormFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, weight, invrms = ctx.saved_tensors
-        dx, dw = ext().rmsnorm_bwd(dy.contiguous(), x, weight, invrms)
-        return dx, dw, None
+        want_dw = ctx.needs_input_grad[1]      # not for a frozen weight, as under LoRA
+        dx, dw = ext().rmsnorm_bwd(dy.contiguous(), x, weight, invrms, want_dw=want_dw)
+        return dx, dw if want_dw else None, None
 
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
@@ -50,10 +51,11 @@ class _AddRMSNormFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy, dh_out):
         h, weight, invrms = ctx.saved_tensors
-        dh, dw = ext().rmsnorm_bwd(dy.contiguous(), h, weight, invrms)
+        want_dw = ctx.needs_input_grad[2]
         if dh_out is not None:
-            dh = dh + dh_out
-        return dh, dh, dw, None
+            dh_out = dh_out.contiguous()
+        dh, dw = ext().rmsnorm_bwd(dy.contiguous(), h, weight, invrms, dh_out, want_dw)
+        return dh, dh, dw if want_dw else None, None
 
 
 def add_rms_norm(x: torch.Tensor, res: torch.Tensor | None, weight: torch.Tensor,

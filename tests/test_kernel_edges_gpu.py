@@ -298,3 +298,32 @@ def test_qkv_rope_append_fills_the_cache_as_kv_append_does(dtype, hq, hkv, d):
     assert torch.equal(alone[0], q) and alone[1] is None
     assert torch.equal(kc.view(torch.uint8), kr.view(torch.uint8))
     assert torch.equal(vc.view(torch.uint8), vr.view(torch.uint8))
+
+
+# ------------------------------------------------------- norm, optimizer
+@pytest.mark.parametrize("N,H", [(1, 8), (3, 512), (5, 520), (1027, 1536), (7, 2048), (6, 2056),
+                                 (4000, 896), (33, 4096), (9, 8192)])
+@pytest.mark.parametrize("frozen", [True, False])
+@pytest.mark.parametrize("residual", [True, False])
+def test_rms_norm_backward_edges(N, H, frozen, residual):
+    x, r = rnd(N, H, seed=1), rnd(N, H, seed=2)
+    w = (1 + rnd(H, seed=3, scale=0.3, dtype=torch.float32)).bfloat16()
+    gy, gh = rnd(N, H, seed=4), rnd(N, H, seed=5)
+    leaves = [t.clone().requires_grad_(t is not w or not frozen) for t in (x, r, w)]
+    if residual:
+        y, h = ops.add_rms_norm(leaves[0], leaves[1], leaves[2])
+        torch.autograd.backward((y, h), (gy, gh))
+    else:
+        ops.rms_norm(leaves[0], leaves[2]).backward(gy)
+    e = [t.detach().double().requires_grad_(True) for t in (x, r, w)]
+    h64 = (x.float() + r.float()).bfloat16().double() - (x.double() + r.double()) + e[0] + e[1] \
+        if residual else e[0]               # the sum as rounded
+    y64 = h64 * torch.rsqrt(h64.pow(2).mean(-1, keepdim=True) + 1e-6) * e[2]
+    ((y64 * gy.double()).sum() + ((h64 * gh.double()).sum() if residual else 0)).backward()
+    assert rel(leaves[0].grad, e[0].grad) < 0.004        # one rounding to bf16
+    if residual:
+        assert torch.equal(leaves[0].grad, leaves[1].grad)
+    if frozen:
+        assert leaves[2].grad is None
+    else:
+        assert rel(leaves[2].grad, e[2].grad) < 0.006    # x_hat is rounded too
