@@ -24,6 +24,9 @@ void ce_backward_dlogits(torch::Tensor logits, torch::Tensor labels,
 // adamw.hip
 void adamw_step(torch::Tensor p, torch::Tensor g, torch::Tensor m, torch::Tensor v,
                 double lr, double b1, double b2, double eps, double wd, long step);
+void adamw_step_many(std::vector<torch::Tensor> p, std::vector<torch::Tensor> g,
+                     std::vector<torch::Tensor> m, std::vector<torch::Tensor> v, double lr,
+                     double b1, double b2, double eps, double wd, long step);
 // sampling.hip
 torch::Tensor sample_topp(torch::Tensor logits, double temperature, double top_p,
                           long seed, long step);
@@ -61,6 +64,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ce_rowstats", &ce_rowstats);
   m.def("ce_backward_dlogits", &ce_backward_dlogits);
   m.def("adamw_step", &adamw_step);
+  m.def("adamw_step_many", &adamw_step_many);
   m.def("sample_topp", &sample_topp);
   m.def("sample_topp_dev", &sample_topp_dev);
   m.def("masked_moments", &masked_moments);

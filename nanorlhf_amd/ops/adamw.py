@@ -3,7 +3,7 @@
 Replaces torch AdamW + the reference's blocking optimizer-state shuttles
 (GRPO/grpo_trainer.py:168-172 state_to_device, :475,:625).  States are fp32,
 params may be bf16 or fp32; the HIP kernel fuses the whole update (decoupled
-weight decay, bias correction) in one pass per tensor with vectorized loads.
+weight decay, bias correction) in one pass over up to 64 tensors per launch.
 Host-offload of states is a policy of utils.offload, not baked in here."""
 from __future__ import annotations
 
@@ -37,6 +37,8 @@ class FusedAdamW(torch.optim.Optimizer):
                 loss = closure()
         for group in self.param_groups:
             b1, b2 = group["betas"]
+            hyper = (group["lr"], b1, b2, group["eps"], group["weight_decay"])
+            together = {}       # GPU tensors that one launch may take, by device, dtype and step
             for p in group["params"]:
                 if p.grad is None:
                     continue
@@ -46,11 +48,11 @@ class FusedAdamW(torch.optim.Optimizer):
                     state["exp_avg"] = torch.zeros_like(p, dtype=torch.float32)
                     state["exp_avg_sq"] = torch.zeros_like(p, dtype=torch.float32)
                 state["step"] += 1
-                m, v = state["exp_avg"], state["exp_avg_sq"]
+                tensors = (p.data, p.grad, state["exp_avg"], state["exp_avg_sq"])
                 if p.is_cuda:
-                    ext().adamw_step(p.data, p.grad, m, v, group["lr"], b1, b2,
-                                     group["eps"], group["weight_decay"], state["step"])
+                    together.setdefault((p.device, p.dtype, state["step"]), []).append(tensors)
                 else:
-                    _adamw_ref(p.data, p.grad, m, v, group["lr"], b1, b2,
-                               group["eps"], group["weight_decay"], state["step"])
+                    _adamw_ref(*tensors, *hyper, state["step"])
+            for (_, _, step), rows in together.items():
+                ext().adamw_step_many(*map(list, zip(*rows)), *hyper, step)
         return loss

@@ -327,3 +327,24 @@ def test_rms_norm_backward_edges(N, H, frozen, residual):
         assert leaves[2].grad is None
     else:
         assert rel(leaves[2].grad, e[2].grad) < 0.006    # x_hat is rounded too
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_adamw_takes_many_tensors_at_once(dtype):
+    from nanorlhf_amd.ops.adamw import _adamw_ref
+    sizes = [1, 7, 8, 4095, 4096, 4097, 100003] + [64 + i for i in range(130)]
+    base = [rnd(n + 1, seed=i, dtype=dtype) for i, n in enumerate(sizes)]
+    p = [b[1:] if i % 5 == 4 else b[:-1] for i, b in enumerate(base)]     # some unaligned
+    g = [rnd(n, seed=1000 + i, dtype=dtype) for i, n in enumerate(sizes)]
+    m = [torch.zeros(n, device=DEV) for n in sizes]
+    v = [torch.zeros(n, device=DEV) for n in sizes]
+    want = [[t.cpu().clone() for t in ts] for ts in zip(p, g, m, v)]
+    guard = [b[0].clone() if i % 5 == 4 else b[-1].clone() for i, b in enumerate(base)]
+    for step in (1, 2):
+        ops.ext().adamw_step_many(p, g, m, v, 1e-2, 0.9, 0.95, 1e-8, 0.1, step)
+        for ts in want:
+            _adamw_ref(*ts, 1e-2, 0.9, 0.95, 1e-8, 0.1, step)
+    for i, ts in enumerate(want):
+        assert rel(p[i].cpu(), ts[0]) < (0.003 if dtype == torch.bfloat16 else 1e-6)
+        assert rel(m[i].cpu(), ts[2]) < 1e-6 and rel(v[i].cpu(), ts[3]) < 1e-6
+        assert torch.equal(guard[i], base[i][0] if i % 5 == 4 else base[i][-1])
