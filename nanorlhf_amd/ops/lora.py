@@ -83,12 +83,17 @@ def _dispatch_gemm(x, w, u, b, bias):
     return y
 
 
+def _scaled_mm(a: torch.Tensor, b: torch.Tensor, scale: float) -> torch.Tensor:
+    """scale * a b: the factor rides on the product's sums (beta 0 leaves the
+    first operand unread)."""
+    return torch.addmm(a.new_empty(1), a, b, beta=0, alpha=scale)
+
+
 class _FusedLoRAFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, bias, lora_A, lora_B, scaling, w_t_cache):
         # u = s·x·Aᵀ (skinny GEMM, r=64)
-        u = (x @ lora_A.t()) * scaling
-        u = u.to(x.dtype).contiguous()
+        u = _scaled_mm(x, lora_A.t(), scaling)
         y = _dispatch_gemm(x.contiguous(), w, u, lora_B.contiguous(),
                            bias if bias is not None else None)
         ctx.save_for_backward(x, u, lora_A, lora_B, w_t_cache)
@@ -101,8 +106,7 @@ class _FusedLoRAFn(torch.autograd.Function):
         scaling = ctx.scaling
         dy = dy.contiguous()
         # du = s·dy·B  [M, r]
-        du = (dy @ lora_B) * scaling
-        du = du.to(dy.dtype).contiguous()
+        du = _scaled_mm(dy, lora_B, scaling)
         dx = None
         if ctx.needs_input_grad[0]:
             # dx = dy·W + du·A → same dispatch on (dy, Wᵀ) + (du, Aᵀ)
