@@ -28,6 +28,10 @@ void adamw_step_many(std::vector<torch::Tensor> p, std::vector<torch::Tensor> g,
                      std::vector<torch::Tensor> m, std::vector<torch::Tensor> v, double lr,
                      double b1, double b2, double eps, double wd, long step);
 // sampling.hip
+std::vector<torch::Tensor> decode_inputs(torch::Tensor lens, torch::Tensor bt, long page_size);
+void decode_commit(torch::Tensor tokens, c10::optional<torch::Tensor> lps, torch::Tensor out,
+                   torch::Tensor lp, torch::Tensor count, torch::Tensor lens, torch::Tensor last,
+                   torch::Tensor finished, c10::optional<long> stop);
 torch::Tensor sample_topp(torch::Tensor logits, double temperature, double top_p,
                           long seed, long step);
 std::vector<torch::Tensor> sample_topp_dev(torch::Tensor logits, double temperature,
@@ -65,6 +69,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ce_backward_dlogits", &ce_backward_dlogits);
   m.def("adamw_step", &adamw_step);
   m.def("adamw_step_many", &adamw_step_many);
+  m.def("decode_inputs", &decode_inputs);
+  m.def("decode_commit", &decode_commit);
   m.def("sample_topp", &sample_topp);
   m.def("sample_topp_dev", &sample_topp_dev);
   m.def("masked_moments", &masked_moments);

@@ -457,3 +457,78 @@ std::vector<torch::Tensor> sample_topp_dev(torch::Tensor logits, double temperat
                  step.data_ptr<long>());
   return {out, lp};
 }
+
+// ------------------------------------------------------------ decode batch
+// What a decode step does to its rows beside the model: where each row's token
+// goes in the cache, and afterwards what the sampled token changes.  A thread a
+// row; bound by the launch, of which tensor operations took 26 a step: a rollout
+// of 64 rows and 96 tokens through 6 layers went from 85.2 to 78.5 ms.
+__global__ __launch_bounds__(256)
+void decode_inputs_kernel(const int* __restrict__ lens, const int* __restrict__ bt,
+                          long* __restrict__ pos, long* __restrict__ slots, int B, int P, int ps) {
+  const int b = blockIdx.x * 256 + threadIdx.x;
+  if (b >= B) return;
+  const int at = lens[b] - 1;
+  pos[b] = at;
+  slots[b] = (long)bt[(long)b * P + min(max(at, 0) / ps, P - 1)] * ps + max(at, 0) % ps;
+}
+
+__global__ __launch_bounds__(256)
+void decode_commit_kernel(const long* __restrict__ tokens, const float* __restrict__ lps,
+                          long* __restrict__ out, float* __restrict__ lp, int* __restrict__ count,
+                          int* __restrict__ lens, long* __restrict__ last,
+                          bool* __restrict__ finished, int B, int most, long stop,
+                          bool has_stop) {
+  const int b = blockIdx.x * 256 + threadIdx.x;
+  if (b >= B) return;
+  const int n = count[b];
+  if (finished[b] || n >= most) {
+    finished[b] = finished[b] || n >= most;
+    return;
+  }
+  const long tok = tokens[b];
+  out[(long)b * most + n] = tok;
+  if (lps) lp[(long)b * most + n] = lps[b];
+  count[b] = n + 1;
+  lens[b]++;
+  last[b] = tok;
+  finished[b] = (has_stop && tok == stop) || n + 1 >= most;
+}
+
+std::vector<torch::Tensor> decode_inputs(torch::Tensor lens, torch::Tensor bt, long page_size) {
+  const int B = lens.size(0);
+  TORCH_CHECK(lens.is_cuda() && bt.is_cuda() && bt.dim() == 2 && bt.size(0) == B &&
+              bt.size(1) > 0 && page_size > 0, "decode_inputs: lengths [B], pages [B, P]");
+  TORCH_CHECK(lens.scalar_type() == at::kInt && bt.scalar_type() == at::kInt &&
+              lens.is_contiguous() && bt.is_contiguous(), "decode_inputs: contiguous int32");
+  auto pos = torch::empty({B}, lens.options().dtype(at::kLong)), slots = torch::empty_like(pos);
+  if (B)
+    hipLaunchKernelGGL(decode_inputs_kernel, dim3((B + 255) / 256), dim3(256), 0,
+                       c10::hip::getCurrentHIPStream(), lens.data_ptr<int>(), bt.data_ptr<int>(),
+                       pos.data_ptr<long>(), slots.data_ptr<long>(), B, (int)bt.size(1),
+                       (int)page_size);
+  return {pos, slots};
+}
+
+void decode_commit(torch::Tensor tokens, c10::optional<torch::Tensor> lps, torch::Tensor out,
+                   torch::Tensor lp, torch::Tensor count, torch::Tensor lens, torch::Tensor last,
+                   torch::Tensor finished, c10::optional<long> stop) {
+  const int B = out.size(0), most = out.size(1);
+  for (const auto& t : {tokens, count, lens, last, finished})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.dim() == 1 && t.size(0) == B,
+                "decode_commit: one contiguous entry a row");
+  TORCH_CHECK(out.is_contiguous() && lp.is_contiguous() && lp.sizes() == out.sizes() &&
+              out.scalar_type() == at::kLong && lp.scalar_type() == at::kFloat &&
+              tokens.scalar_type() == at::kLong && last.scalar_type() == at::kLong &&
+              count.scalar_type() == at::kInt && lens.scalar_type() == at::kInt &&
+              finished.scalar_type() == at::kBool, "decode_commit: types");
+  TORCH_CHECK(!lps || (lps->is_cuda() && lps->is_contiguous() && lps->numel() == B &&
+                       lps->scalar_type() == at::kFloat), "decode_commit: log-probabilities");
+  if (B)
+    hipLaunchKernelGGL(decode_commit_kernel, dim3((B + 255) / 256), dim3(256), 0,
+                       c10::hip::getCurrentHIPStream(), tokens.data_ptr<long>(),
+                       lps ? lps->data_ptr<float>() : nullptr, out.data_ptr<long>(),
+                       lp.data_ptr<float>(), count.data_ptr<int>(), lens.data_ptr<int>(),
+                       last.data_ptr<long>(), finished.data_ptr<bool>(), B, most,
+                       stop.value_or(0), stop.has_value());
+}

@@ -2,8 +2,8 @@
 
 The per-token decode loop keeps ALL scheduling state (sequence lengths,
 block tables, slot mapping, generated-token buffer, finished mask) on the
-GPU as tensors: one decode step costs a handful of small index kernels +
-the model forward, with no per-sequence Python work and no host round trip
+GPU as tensors: one decode step costs two small kernels beside the model
+forward and the sampling, with no per-sequence Python work and no host round trip
 (the first bench profile showed list rebuilding at batch 2048 dominating
 rollout time).  Host synchronization happens only every `compact_interval`
 steps, when finished sequences are retired (pages freed) and queued
@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import torch
 
+from .. import ops
 from .cache import PagedKVCache, SeqState
 
 
@@ -84,6 +85,9 @@ class DecodeBatch:
     def step_inputs(self):
         """Tensors for the next decode forward (all on device, no sync)."""
         ps = self.pool.page_size
+        if self.seq_lens.is_cuda:
+            pos, slots = ops.ext().decode_inputs(self.seq_lens, self.bt, ps)
+            return self.last_tok, pos, slots, self.seq_lens, self.bt
         pos = (self.seq_lens - 1).long()
         page_idx = torch.div(pos, ps, rounding_mode="floor")
         page = self.bt.gather(1, page_idx.unsqueeze(1).int().long()).squeeze(1).long()
@@ -94,6 +98,10 @@ class DecodeBatch:
         """Record sampled tokens; advance lengths.  Fully IN-PLACE on the
         batch's state tensors so the whole step is hipGraph-capturable (no
         host sync, no tensor reassignment)."""
+        if tokens.is_cuda:
+            ops.ext().decode_commit(tokens, lps, self.out, self.lp, self.gen_count,
+                                    self.seq_lens, self.last_tok, self.finished, self.stop)
+            return
         write = (~self.finished) & (self.gen_count < self.max_tokens)
         idx = self.gen_count.clamp(max=self.max_tokens - 1).long().unsqueeze(1)
         cur = self.out.gather(1, idx).squeeze(1)

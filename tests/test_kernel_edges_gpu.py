@@ -348,3 +348,31 @@ def test_adamw_takes_many_tensors_at_once(dtype):
         assert rel(p[i].cpu(), ts[0]) < (0.003 if dtype == torch.bfloat16 else 1e-6)
         assert rel(m[i].cpu(), ts[2]) < 1e-6 and rel(v[i].cpu(), ts[3]) < 1e-6
         assert torch.equal(guard[i], base[i][0] if i % 5 == 4 else base[i][-1])
+
+
+# ------------------------------------------------------------ decode batch
+@pytest.mark.parametrize("B", [1, 255, 257])
+@pytest.mark.parametrize("stop", [None, 3])
+def test_decode_batch_matches_its_tensor_form(B, stop):
+    from types import SimpleNamespace
+    from nanorlhf_amd.sampler.decode_batch import DecodeBatch
+    pool, most, pages = SimpleNamespace(page_size=16), 5, 4
+    g = torch.Generator().manual_seed(B)
+    both = [DecodeBatch(pool, [], most, stop, d) for d in ("cpu", DEV)]
+    state = dict(bt=torch.randperm(B * pages, generator=g).view(B, pages).int(),
+                 seq_lens=torch.randint(1, 16 * pages - most, (B,), generator=g).int(),
+                 gen_count=torch.randint(0, most + 1, (B,), generator=g).int(),
+                 last_tok=torch.randint(0, 9, (B,), generator=g),
+                 finished=torch.rand(B, generator=g) < 0.2,
+                 out=torch.zeros(B, most, dtype=torch.long), lp=torch.zeros(B, most))
+    for db in both:
+        for k, v in state.items():
+            setattr(db, k, v.clone().to(db.device))
+    for step in range(most + 1):
+        for a, b in zip(both[0].step_inputs(), both[1].step_inputs()):
+            assert a.dtype == b.dtype and torch.equal(a, b.cpu())
+        tok, lp = torch.randint(0, 5, (B,), generator=g), torch.randn(B, generator=g)
+        for db in both:
+            db.commit(tok.to(db.device), None if step == 1 else lp.to(db.device))
+        for k in state:
+            assert torch.equal(getattr(both[0], k), getattr(both[1], k).cpu()), k
