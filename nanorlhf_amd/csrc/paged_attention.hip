@@ -5,11 +5,15 @@
 // kv-head, 128 query rows).  A "row" is a (token, query head) pair of the
 // kv-head's group, tokens outermost, so grouped heads share every K/V tile and
 // a short portion still fills the 32-row MFMA tiles.  Each of the 4 waves owns
-// 32 rows; KV walks in 64-token tiles (4 pages) double-buffered in LDS.  As in
-// the packed forward kernel, QK^T is computed swapped (S^T = K Q^T), which
-// leaves a row's 64 scores in one lane pair: online softmax without LDS, P
-// repacked to bf16 in registers, O^T = V^T P^T.  V pages are d-major, so a
-// V^T fragment (8 tokens of one d) is one 16-byte copy from page to LDS.
+// 32 rows; KV walks in 64-token tiles (4 pages) that two LDS buffers receive by
+// direct loads while the tile before is computed on.  As in the packed forward
+// kernel, QK^T is computed swapped (S^T = K Q^T), which leaves a row's 64 scores
+// in one lane pair: online softmax without LDS, weights converted to bf16 in
+// place, O^T = V^T P^T.  V pages are d-major, so a V^T fragment (8 tokens of one
+// d) is 16 bytes; the keys are read in the order that leaves a lane the scores
+// of those 8.  Bound by LDS reads, matrix products and exponentials together.
+// 4000 tokens after 0, 4000 and 8000, 12 heads of 128: 160 us each (920 TFLOP/s);
+// with tiles through registers and every head on every chiplet 309.
 //
 // The same kernel runs over a workspace (LIN) instead of pages: keys [rows, Hkv,
 // DK] and transposed values [Hkv * DV, rows] of whole contexts laid out one
@@ -50,25 +54,47 @@ struct VarlenArgs {
   const int* first;      // LIN: first workspace row of each sequence
   long ldv;              // LIN: row stride of vc
   int Hq, Hkv, maxP, V, size, keep;
+  int B, tiles;          // sequences, tiles of 128 rows of the longest portion
   float scale;
 };
+
+// ---- LDS tiles: rows of 16-byte chunks, the chunks exchanged (xor) by row so
+// that 16 rows' reads of one chunk touch every bank once.  V: [d][64 tokens] from
+// a workspace; from pages [page][d][16 tokens], as they lie.
+template <int D>
+DEVINL int row_swz(int row) {
+  return D >= 128 ? row & 15 : D == 64 ? (row >> 1) & 7 : (row >> 2) & 3;
+}
+DEVINL int half_swz(int d) { return (d >> 3) & 1; }
 
 template <int DK, int DV, bool LIN>
 __global__ __launch_bounds__(256, (DK > 128 || DV > 128) ? 1 : 2)
 void paged_varlen_kernel(VarlenArgs a) {
   constexpr int NDS = DK / 16, NDT = DV / 32, KV = 64;
-  constexpr int KROW = DK + 8;                 // padded LDS row: spreads the banks
   constexpr float THR = 11.54f;                // defer-max threshold (log2 units)
-  const int seq = blockIdx.y, kvh = blockIdx.z;
+  int seq, kvh, tile;
+  {
+    // From 8 kv heads on, a chiplet takes whole heads, whose keys then stay in its
+    // L2, long and short rows in turn; else the longest rows first.
+    int id = blockIdx.x;
+    const int n = gridDim.x;
+    if (a.Hkv >= 8) {
+      const int q = n >> 3, r = n & 7, xcd = id & 7;
+      id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (id >> 3);
+    }
+    const int t = id % a.tiles;
+    tile = a.Hkv >= 8 && (t & 1) ? t >> 1 : a.tiles - 1 - (a.Hkv >= 8 ? t >> 1 : t);
+    seq = id / a.tiles % a.B;
+    kvh = id / a.tiles / a.B;
+  }
   const int G = a.Hq / a.Hkv;
   const int t0 = a.cu[seq], nq = a.cu[seq + 1] - t0;
   const int L = a.seq_lens[seq];
   const int start = L - nq;                    // position of the portion's first token
   const int R = nq * G;
-  // LIN is plainly causal: the longest rows first
-  const int r0 = (LIN ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * 128;
+  const int r0 = tile * 128;
   if (r0 >= R) return;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 31, hi = lane >> 5;
   const int rw0 = r0 + wid * 32;
   const bool wave_active = rw0 < R;
@@ -77,8 +103,7 @@ void paged_varlen_kernel(VarlenArgs a) {
   const int tok = row / G, head = kvh * G + row % G;
   const int qpos = start + tok;
 
-  __shared__ __attribute__((aligned(16))) short Ks[2][KV * KROW];   // [tok][d]
-  __shared__ __attribute__((aligned(16))) short Vs[2][KV * DV];     // [tok/8][d][tok%8]
+  __shared__ __attribute__((aligned(16))) short Ks[2][KV * DK], Vs[2][KV * DV];
 
   bf16x8p qf[NDS];
   {
@@ -101,66 +126,53 @@ void paged_varlen_kernel(VarlenArgs a) {
   const int win_tile = max(0, pos_lo - a.size + 1) / KV;
   const int kept_tiles = min((a.keep + KV - 1) / KV, win_tile);
   const int ntiles = kept_tiles + pos_hi / KV + 1 - win_tile;
-  const int* btb = LIN ? nullptr : a.bt + (long)seq * a.maxP;
-  const int page0 = LIN ? a.first[seq] >> 4 : 0;
+  // scalar loads: a vector load would be waited for behind the tiles under way
+  typedef const __attribute__((address_space(4))) int* const_ints;
+  const const_ints btb = (const_ints)(size_t)(LIN ? nullptr : a.bt + (long)seq * a.maxP);
+  const long lin0 = LIN ? a.first[seq] : 0;
   const int last_page = (L - 1) >> 4;
-  auto page_of = [&](int p) { return LIN ? page0 + p : btb[min(p, last_page)]; };
-
-  constexpr int KCH = KV * DK / 8 / 256;   // 16-byte chunks per thread
-  constexpr int VCH = KV * DV / 8 / 256;
-  s16x8 kr[KCH], vr[VCH];
   auto tile_of = [&](int it) { return it < kept_tiles ? it : it - kept_tiles + win_tile; };
-  auto load_tile = [&](int tile) {
-#pragma unroll
-    for (int s = 0; s < KCH; s++) {
-      const int c = threadIdx.x + s * 256;
-      const int tk = c / (DK / 8), d0 = (c % (DK / 8)) * 8;
-      const int page = page_of(tile * 4 + (tk >> 4));
-      kr[s] = *reinterpret_cast<const s16x8*>(
-          a.kc + (((long)page * 16 + (tk & 15)) * a.Hkv + kvh) * DK + d0);
-    }
-#pragma unroll
-    for (int s = 0; s < VCH; s++) {
-      const int c = threadIdx.x + s * 256;
-      if constexpr (LIN) {                        // (d, 8 tokens) fastest last
-        vr[s] = *reinterpret_cast<const s16x8*>(
-            a.vc + ((long)kvh * DV + (c >> 3)) * a.ldv + (long)(page0 + tile * 4) * 16 +
-            (c & 7) * 8);
-      } else {                                    // (page, d, half) fastest last
-        const int half = c & 1, d = (c >> 1) % DV, pg = (c >> 1) / DV;
-        const int page = page_of(tile * 4 + pg);
-        vr[s] = *reinterpret_cast<const s16x8*>(
-            a.vc + (((long)page * a.Hkv + kvh) * DV + d) * 16 + half * 8);
-      }
-    }
-  };
-  auto store_tile = [&](int buf) {
-#pragma unroll
-    for (int s = 0; s < KCH; s++) {
-      const int c = threadIdx.x + s * 256;
-      const int tk = c / (DK / 8), d0 = (c % (DK / 8)) * 8;
-      *reinterpret_cast<s16x8*>(&Ks[buf][tk * KROW + d0]) = kr[s];
-    }
-#pragma unroll
-    for (int s = 0; s < VCH; s++) {
-      const int c = threadIdx.x + s * 256;
-      if constexpr (LIN) {
-        // d exchanged (xor) by token group: eight lanes store to eight banks' sets
-        const int g = c & 7, d = c >> 3;
-        *reinterpret_cast<s16x8*>(&Vs[buf][(g * DV + (d ^ g)) * 8]) = vr[s];
-      } else {
-        const int half = c & 1, d = (c >> 1) % DV, pg = (c >> 1) / DV;
-        *reinterpret_cast<s16x8*>(&Vs[buf][((pg * 2 + half) * DV + d) * 8]) = vr[s];
-      }
-    }
-  };
 
-  load_tile(tile_of(0));
+  // A wave's 64 chunks of one load are rows of one page (or 8 rows of V^T).
+  const int ldk = a.Hkv * DK;
+  auto stage = [&](int tile, int buf) {
+#pragma unroll
+    for (int i = 0; i < KV * DK / 8; i += 256) {
+      constexpr int PER = 64 / (DK / 8);                      // tokens of one load
+      const int row0 = i / (DK / 8) + wid * PER, r = row0 + lane / (DK / 8);
+      const int c = (lane % (DK / 8)) ^ row_swz<DK>(r);
+      const long at = LIN ? lin0 + tile * KV + row0
+                          : (long)btb[min(tile * 4 + (row0 >> 4), last_page)] * 16 + (row0 & 15);
+      load_to_lds16(a.kc + at * ldk + kvh * DK, (unsigned)((r - row0) * ldk + c * 8) * 2,
+                    &Ks[buf][(i + wid * 64) * 8]);
+    }
+#pragma unroll
+    for (int i = 0; i < KV * DV / 8; i += 256) {
+      if constexpr (LIN) {
+        const int d0 = i / 8 + wid * 8, d = d0 + (lane >> 3);
+        const int c = (lane & 7) ^ row_swz<64>(d);
+        load_to_lds16(a.vc + ((long)kvh * DV + d0) * a.ldv + lin0 + tile * KV,
+                      (unsigned)((lane >> 3) * a.ldv + c * 8) * 2, &Vs[buf][(i + wid * 64) * 8]);
+      } else {
+        const int d0 = (i / 2 + wid * 32) % DV, pg = (i / 2 + wid * 32) / DV;
+        const int d = d0 + (lane >> 1), c = (lane & 1) ^ half_swz(d);
+        load_to_lds16(a.vc + ((long)btb[min(tile * 4 + pg, last_page)] * a.Hkv + kvh) * DV * 16,
+                      (unsigned)(d * 16 + c * 8) * 2, &Vs[buf][(i + wid * 64) * 8]);
+      }
+    }
+  };
+  // Row i of a key fragment is the key with bits 2 and 3 of i exchanged, which
+  // leaves lane half `hi` with keys 16 ks + 8 hi + (0 .. 7) in registers 8 ks + ..
+  const int krow = (col & 19) | (col & 4) << 1 | (col & 8) >> 1;
+
+#pragma unroll
+  for (int ds = 0; ds < NDS; ds++) asm volatile("" : "+v"(qf[ds]));   // arrived
+  stage(tile_of(0), 0);
   for (int it = 0; it < ntiles; it++) {
     const int buf = it & 1, kv0 = tile_of(it) * KV;
-    store_tile(buf);          // readers of `buf` passed the previous barrier
-    __syncthreads();
-    if (it + 1 < ntiles) load_tile(tile_of(it + 1));
+    wait_loads<0>();
+    __syncthreads();          // the tile has arrived, the other buffer is free
+    if (it + 1 < ntiles) stage(tile_of(it + 1), buf ^ 1);
     // whole tile invisible to this wave?
     if (!wave_active || kv0 > wpos_hi ||
         (wpos_lo - (kv0 + KV - 1) >= a.size && kv0 >= a.keep))
@@ -170,31 +182,37 @@ void paged_varlen_kernel(VarlenArgs a) {
 #pragma unroll
     for (int sub = 0; sub < 2; sub++) {
       st[sub] = f32x16{};
+      const int r = sub * 32 + krow;
 #pragma unroll
       for (int ds = 0; ds < NDS; ds++) {
         const bf16x8p kf = *reinterpret_cast<const bf16x8p*>(
-            &Ks[buf][(sub * 32 + col) * KROW + 16 * ds + 8 * hi]);
+            &Ks[buf][r * DK + (((2 * ds + hi) ^ row_swz<DK>(r)) << 3)]);
         st[sub] = mfma32p(kf, qf[ds], st[sub]);
       }
     }
+    // scores meet scale * log2(e) in the exponent's fma, which needs a positive scale
     const float sl2 = a.scale * 1.4426950408889634f;
+    float mul = sl2;
+    if (!(sl2 > 0.f)) {
+#pragma unroll
+      for (int i = 0; i < 32; i++) st[i >> 4][i & 15] *= sl2;
+      mul = 1.f;
+    }
     const bool full = kv0 + KV - 1 <= wpos_lo &&
                       (wpos_hi - kv0 < a.size || kv0 + KV <= a.keep);
-    float p[32];
+    if (!full) {
 #pragma unroll
-    for (int i = 0; i < 32; i++) {
-      const int r = i & 15;
-      const int ki = kv0 + 32 * (i >> 4) + (r & 3) + 8 * (r >> 2) + 4 * hi;
-      const float s = st[i >> 4][r] * sl2;
-      p[i] = (full || (ki <= qpos && (qpos - ki < a.size || ki < a.keep))) ? s : -INFINITY;
+      for (int i = 0; i < 32; i++) {
+        const int ki = kv0 + 16 * (i >> 3) + 8 * hi + (i & 7);
+        if (!(ki <= qpos && (qpos - ki < a.size || ki < a.keep))) st[i >> 4][i & 15] = -INFINITY;
+      }
     }
-    float pmax = p[0];
+    float pmax = st[0][0];
 #pragma unroll
-    for (int i = 1; i < 32; i++) pmax = fmaxf(pmax, p[i]);
-    pmax = fmaxf(pmax, __shfl_xor(pmax, 32));
+    for (int i = 1; i < 32; i++) pmax = fmaxf(pmax, st[i >> 4][i & 15]);
+    pmax = fmaxf(pmax, __shfl_xor(pmax, 32)) * mul;
     float alpha = 1.f;
-    const bool need = !(pmax - m <= THR);      // also true while m is -inf
-    if (__any(need)) {
+    if (__any(!(pmax - m <= THR))) {           // also true while m is -inf
       const float mn = fmaxf(m, pmax);
       alpha = (m == -INFINITY) ? 0.f : exp2f(m - mn);
       m = mn;
@@ -203,44 +221,35 @@ void paged_varlen_kernel(VarlenArgs a) {
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[t][r] *= alpha;
     }
+    const float mm = m == -INFINITY ? 0.f : m;  // a row that sees nothing so far
     float rs = 0.f;
-#pragma unroll
-    for (int i = 0; i < 32; i++) {
-      p[i] = (p[i] > -INFINITY) ? exp2f(p[i] - m) : 0.f;
-      if constexpr (!LIN) rs += p[i];
-    }
-    // P^T fragments: lane holds P[row][16 ks + 8 hi + j]
     bf16x8p pf[4];
 #pragma unroll
     for (int ks = 0; ks < 4; ks++) {
-      const int b0 = ks * 8;
-      const unsigned w01 = pack2p(p[b0 + 0], p[b0 + 1]);
-      const unsigned w23 = pack2p(p[b0 + 2], p[b0 + 3]);
-      const unsigned w45 = pack2p(p[b0 + 4], p[b0 + 5]);
-      const unsigned w67 = pack2p(p[b0 + 6], p[b0 + 7]);
-      // LIN: normed by the sum of the weights as rounded, so that rounding a
-      // weight that stands out does not scale the result
-      if constexpr (LIN)
-        for (unsigned x : {w01, w23, w45, w67}) rs += bf2f((short)(x & 0xffff)) + bf2f((short)(x >> 16));
-      auto rA = __builtin_amdgcn_permlane32_swap(w01, w45, false, false);
-      auto rB = __builtin_amdgcn_permlane32_swap(w23, w67, false, false);
       union { unsigned u[4]; bf16x8p f; } fr;
-      fr.u[0] = (unsigned)rA[0];
-      fr.u[1] = (unsigned)rB[0];
-      fr.u[2] = (unsigned)rA[1];
-      fr.u[3] = (unsigned)rB[1];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int i = 8 * ks + 2 * j;
+        const float x = __builtin_amdgcn_exp2f(fmaf(st[i >> 4][i & 15], mul, -mm));
+        const float y = __builtin_amdgcn_exp2f(fmaf(st[i >> 4][(i & 15) + 1], mul, -mm));
+        fr.u[j] = pack2p(x, y);
+        // LIN: normed by the sum of the weights as rounded, so that rounding a
+        // weight that stands out does not scale the result
+        if constexpr (LIN) rs += __uint_as_float(fr.u[j] << 16) + __uint_as_float(fr.u[j] & 0xffff0000u);
+        else rs += x + y;
+      }
       pf[ks] = fr.f;
     }
     rs += __shfl_xor(rs, 32);
     sum = sum * alpha + rs;
 #pragma unroll
-    for (int t = 0; t < NDT; t++)
+    for (int ks = 0; ks < 4; ks++)
 #pragma unroll
-      for (int ks = 0; ks < 4; ks++) {
-        const int g = 2 * ks + hi, d = t * 32 + col;
-        const bf16x8p vf = *reinterpret_cast<const bf16x8p*>(
-            &Vs[buf][(g * DV + (LIN ? d ^ g : d)) * 8]);
-        acc[t] = mfma32p(vf, pf[ks], acc[t]);
+      for (int t = 0; t < NDT; t++) {
+        const int d = t * 32 + col;
+        const short* v = LIN ? &Vs[buf][d * 64 + (((2 * ks + hi) ^ row_swz<64>(d)) << 3)]
+                             : &Vs[buf][(ks * DV + d) * 16 + ((hi ^ half_swz(d)) << 3)];
+        acc[t] = mfma32p(*reinterpret_cast<const bf16x8p*>(v), pf[ks], acc[t]);
       }
   }
 
@@ -373,7 +382,10 @@ static void check_cache(const torch::Tensor& q, const torch::Tensor& kc, const t
 }
 
 template <bool LIN>
-static void launch_varlen(const VarlenArgs& a, int DK, int DV, dim3 grid, hipStream_t stream) {
+static void launch_varlen(VarlenArgs a, int DK, int DV, long max_rows, hipStream_t stream) {
+  a.tiles = (max_rows + 127) / 128;
+  if (!a.tiles) return;
+  const dim3 grid((unsigned)((long)a.tiles * a.B * a.Hkv));
 #define LAUNCH(KK, VV) \
   hipLaunchKernelGGL((paged_varlen_kernel<KK, VV, LIN>), grid, dim3(256), 0, stream, a)
 #define LAUNCH_V(KK)                                              \
@@ -425,9 +437,8 @@ void paged_attn_varlen(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torc
   a.keep = (int)std::min<long>(keep, 1 << 30);
   a.scale = scale;
   const int DK = q.size(2), DV = vc.size(2);
-  dim3 grid((max_q * (a.Hq / a.Hkv) + 127) / 128, B, a.Hkv);
-  auto stream = at::hip::getCurrentHIPStream();
-  launch_varlen<false>(a, DK, DV, grid, stream);
+  a.B = B;
+  launch_varlen<false>(a, DK, DV, max_q * (a.Hq / a.Hkv), at::hip::getCurrentHIPStream());
 }
 
 // Attention of portions over expanded contexts: q [T, Hq * DK] (any row
@@ -466,8 +477,8 @@ void expanded_attn_varlen(torch::Tensor q, torch::Tensor k, torch::Tensor vt, to
   a.scale = scale;
   const int DK = k.size(1) / heads, DV = vt.size(0) / heads;
   TORCH_CHECK(a.V <= DV);
-  launch_varlen<true>(a, DK, DV, dim3((max_q + 127) / 128, B, heads),
-                      at::hip::getCurrentHIPStream());
+  a.B = B;
+  launch_varlen<true>(a, DK, DV, max_q, at::hip::getCurrentHIPStream());
 }
 
 void paged_attn_plain(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Tensor row_seq,

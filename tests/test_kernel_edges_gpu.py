@@ -376,3 +376,57 @@ def test_decode_batch_matches_its_tensor_form(B, stop):
             db.commit(tok.to(db.device), None if step == 1 else lp.to(db.device))
         for k in state:
             assert torch.equal(getattr(both[0], k), getattr(both[1], k).cpu()), k
+
+
+# ----------------------------------------------- attention of prompt portions
+def _portions(held, new):
+    """cu, lengths, page table (pages in no order), row's sequence and position."""
+    lens = [h + n for h, n in zip(held, new)]
+    pages = [-(-l // 16) for l in lens]
+    order = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(1)).int()
+    bt, at = torch.zeros(len(lens), max(pages), dtype=torch.int32), 0
+    for i, n in enumerate(pages):
+        bt[i, :n] = order[at:at + n]
+        at += n
+    cu = torch.tensor([0] + new).cumsum(0).int()
+    seq = torch.repeat_interleave(torch.arange(len(new)), torch.tensor(new)).int()
+    pos = torch.cat([torch.arange(h, h + n) for h, n in zip(held, new)])
+    return lens, sum(pages), [t.to(DEV) for t in (cu, torch.tensor(lens).int(), bt, seq, pos)]
+
+
+@pytest.mark.parametrize("DK,DV,V", [(32, 32, 32), (64, 128, 100), (128, 64, 64), (128, 128, 128),
+                                     (256, 32, 30), (32, 256, 256), (256, 256, 256)])
+@pytest.mark.parametrize("H,G,size,keep", [(2, 2, 1 << 30, 0), (6, 1, 70, 3), (16, 8, 1 << 30, 0),
+                                           (9, 9, 64, 0)])
+def test_paged_portions_tile_edges(DK, DV, V, H, G, size, keep):
+    lens, P, (cu, sl, bt, seq, pos) = _portions([0, 63, 0, 200, 65], [1, 1, 129, 130, 0])
+    T = int(cu[-1])
+    q = rnd(T, H, DK, seed=1)
+    kc, vc = rnd(P, 16, G, DK, seed=2), rnd(P, G, DV, 16, seed=3)
+    out = torch.zeros(T, H * V, device=DEV, dtype=torch.bfloat16)
+    ops.serve_ext().paged_attn_varlen(q, kc, vc, cu, sl, bt, out, 130, DK ** -0.5, size, keep, None)
+    want = torch.zeros(T, H * V, device=DEV)
+    ops.serve_ext().paged_attn_plain(q.float(), kc.float(), vc.float(), seq, pos, bt, want,
+                                     DK ** -0.5, size, keep, None)
+    assert rel(out, want) < 0.004       # weights and result, each rounded by at most 2^-9
+
+
+@pytest.mark.parametrize("DK,DV", [(32, 64), (128, 128), (64, 256), (256, 32)])
+@pytest.mark.parametrize("H", [1, 12])
+def test_expanded_portions_tile_edges(DK, DV, H):
+    held, new = [0, 63, 100], [65, 129, 1]
+    lens, _, (cu, sl, _, seq, pos) = _portions(held, new)
+    first = torch.tensor([0] + [-(-l // 64) * 64 for l in lens]).cumsum(0).int().to(DEV)
+    rows, T = int(first[-1]), int(cu[-1])
+    q, k, vt = rnd(T, H * DK, seed=1), rnd(rows, H * DK, seed=2), rnd(H * DV, rows, seed=3)
+    out = torch.zeros(T, H * DV, device=DEV, dtype=torch.bfloat16)
+    ops.serve_ext().expanded_attn_varlen(q, k, vt, cu, sl, first, out, H, 129, DK ** -0.5)
+    for b, (h, n) in enumerate(zip(held, new)):
+        f, t = int(first[b]), int(cu[b])
+        qs = q[t:t + n].view(n, H, DK).transpose(0, 1).double().cpu()
+        ks = k[f:f + h + n].view(-1, H, DK).transpose(0, 1).double().cpu()
+        vs = vt.view(H, DV, rows)[:, :, f:f + h + n].transpose(1, 2).double().cpu()
+        s = qs @ ks.transpose(1, 2) * DK ** -0.5
+        s.masked_fill_(torch.arange(h + n)[None] > torch.arange(h, h + n)[:, None], -torch.inf)
+        want = (s.softmax(-1) @ vs).transpose(0, 1).reshape(n, -1)
+        assert rel(out[t:t + n].cpu(), want) < 0.004
