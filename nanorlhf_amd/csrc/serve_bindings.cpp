@@ -51,6 +51,9 @@ torch::Tensor rotary_qkv(torch::Tensor proj, long qoff, long koff, long voff, Op
                          torch::Tensor kc, torch::Tensor vc, long H, long G, long D, long V,
                          bool interleaved, double eps);
 
+// glu.hip
+void glu_linear(torch::Tensor x, torch::Tensor gate, torch::Tensor up, torch::Tensor out,
+                long act);
 // wkv.hip
 void token_shift(torch::Tensor h, torch::Tensor mu, OptTensor seq_lens, torch::Tensor slots,
                  OptTensor cu, OptTensor row_seq, OptTensor fresh, torch::Tensor last,
@@ -98,6 +101,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("residual_group_norm", &residual_group_norm);
   m.def("gated_norm", &gated_norm);
   m.def("gelu_glu", &gelu_glu);
+  m.def("glu_linear", &glu_linear);
   m.def("relu_squared_", &relu_squared_);
   m.def("token_shift", &token_shift);
   m.def("wkv_decay", &wkv_decay);

@@ -6,8 +6,10 @@ Block:  h = norm1(x);  x <- x + m (mixer(h) + ff(h)).
 Both sublayers read h and their outputs are added, so a block is two GEMMs:
 one input projection for all of the mixer's inputs and the feed-forward's gate
 and up, and one output projection over [mixer output | feed-forward output]
-side by side, whose sum over the columns is the addition.  The update of x is
-left pending and fused into the next norm.
+side by side, whose sum over the columns is the addition.  With many rows the
+feed-forward's half of the first is a product of its own, which ends in the
+activation (ops.linear_gelu_glu).  The update of x is left pending and fused into
+the next norm.
 """
 from __future__ import annotations
 
@@ -18,6 +20,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
+from .lora import plain_weight
 from .mixers import MIXERS
 
 ALIGN = 8   # columns of a segment start at multiples of 16 bytes (bf16)
@@ -104,8 +107,18 @@ class ParallelBlock(nn.Module):
                 p.copy_(take("mix." + name))
 
     def forward(self, h: torch.Tensor, ctx, cache) -> torch.Tensor:
-        proj = self.in_proj(h)
+        w = plain_weight(self.in_proj) if self.ff else None
         cat = torch.empty(h.shape[0], self.out_width, dtype=h.dtype, device=h.device)
+        if w is not None and ops.glu_fuses(h, w):
+            # the mixer's columns alone, gate and up straight into the output's input
+            (a, b), (c, d) = self.cols["gate"], self.cols["up"]
+            proj = F.linear(h, w[:a])
+            ops.linear_gelu_glu(h, w[a:b], w[c:d], cat[:, self.ff_start:self.ff_start + self.ff])
+            cat[:, self.mix_out:self.ff_start] = 0
+            cat[:, self.ff_start + self.ff:] = 0
+            self.mixer(self.cols, proj, ctx, cache, cat[:, :self.mix_out])
+            return self.out_proj(cat)
+        proj = self.in_proj(h)
         self.mixer(self.cols, proj, ctx, cache, cat[:, :self.mix_out])
         if self.ff:
             gate, up = (proj[:, slice(*self.cols[n])] for n in ("gate", "up"))

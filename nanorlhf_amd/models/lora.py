@@ -14,6 +14,7 @@ from dataclasses import dataclass
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+import torch.nn.modules.module as _module
 
 
 def quantize_fp8_weight(w_float: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
@@ -135,6 +136,24 @@ def apply_lora(model: nn.Module, cfg: LoraConfig) -> nn.Module:
             for p in module.parameters(recurse=True):
                 p.requires_grad_(True)
     return model
+
+
+def plain_weight(proj: nn.Module) -> torch.Tensor | None:
+    """The weight of a projection whose call is F.linear(x, weight) and nothing
+    else: no gradient wanted, no bias, nobody listening to the call.  Else None."""
+    if torch.is_grad_enabled() or proj.bias is not None or any(
+            (proj._forward_hooks, proj._forward_pre_hooks, proj._backward_hooks,
+             proj._backward_pre_hooks, _module._global_forward_hooks,
+             _module._global_forward_pre_hooks)):
+        return None
+    if type(proj) is nn.Linear and "forward" not in proj.__dict__:
+        w = proj.weight
+    elif type(proj) is LoRALinear and "forward" not in proj.__dict__ \
+            and proj._merged_fp8 is None:
+        w = proj._merged
+    else:
+        return None
+    return w if type(w) in (torch.Tensor, nn.Parameter) else None
 
 
 def merge_for_rollout(model: nn.Module, quant: str | None = None):

@@ -23,6 +23,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from .config import ModelConfig, get_config
+from .lora import plain_weight
 
 
 @dataclass
@@ -130,7 +131,9 @@ class MLP(nn.Module):
         self.down_proj = nn.Linear(cfg.intermediate_size, cfg.hidden_size, bias=False)
 
     def forward(self, x):
-        return self.down_proj(ops.swiglu(self.gate_up_proj(x)))
+        w = plain_weight(self.gate_up_proj)
+        act = ops.swiglu(self.gate_up_proj(x)) if w is None else ops.linear_swiglu(x, w)
+        return self.down_proj(act)
 
 
 class RMSNorm(nn.Module):

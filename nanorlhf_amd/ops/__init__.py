@@ -56,7 +56,8 @@ def ext_available() -> bool:
 from .rmsnorm import (add_rms_norm, gated_norm, residual_group_norm,  # noqa: E402,F401
                       rms_norm)
 from .rope import Rotation, build_rope_cache, qkv_rope, rope_apply  # noqa: E402,F401
-from .swiglu import gelu_glu, relu_squared_, swiglu  # noqa: E402,F401
+from .swiglu import (gelu_glu, glu_fuses, linear_gelu_glu, linear_swiglu,  # noqa: E402,F401
+                     relu_squared_, swiglu)
 from .attention import flash_attn_varlen  # noqa: E402,F401
 from .logprob import token_logprob_entropy  # noqa: E402,F401
 from .adamw import FusedAdamW  # noqa: E402,F401

@@ -31,12 +31,46 @@ def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
     return _swiglu_ref(gate_up)
 
 
+# Rows and depths from and up to which both products and the activation are one
+# kernel.  Library product and a pass against it, in us: 1024 x 4864 x 896 40 / 25,
+# 2048 x 4096 x 1024 68 / 33, 600 x 8960 x 1536 51 / 40, 16320 x 8960 x 1536 857 /
+# 786.  A few rows leave most of its 256-row tiles empty (300 x 8960 x 1536: 34 /
+# 37), and deep products have little to save (4096 x 18944 x 3584: 872 / 910).
+GLU_ROWS, GLU_DEPTH = 512, 2048
+
+
+def glu_fuses(x: torch.Tensor, gate: torch.Tensor) -> bool:
+    """Whether glu_linear takes (and is the faster way for) these operands."""
+    return (x.is_cuda and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
+            and x.dim() == 2 and x.dtype == gate.dtype == torch.bfloat16
+            and x.is_contiguous() and gate.is_contiguous() and gate.device == x.device
+            and x.shape[0] >= GLU_ROWS and x.shape[1] % 64 == 0 and x.shape[1] <= GLU_DEPTH
+            and x.data_ptr() % 16 == 0 and gate.data_ptr() % 16 == 0)
+
+
+def linear_swiglu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """swiglu of x [..., K] times weight [2 I, K] (gate rows, then up rows)."""
+    gate, up = weight.chunk(2)
+    if not glu_fuses(x, gate):
+        return swiglu(torch.nn.functional.linear(x, weight))
+    out = torch.empty(x.shape[0], gate.shape[0], dtype=x.dtype, device=x.device)
+    serve_ext().glu_linear(x, gate, up, out, 0)
+    return out
+
+
 def relu_squared_(x: torch.Tensor) -> torch.Tensor:
     """x <- relu(x)^2, in place."""
     if x.is_cuda:
         serve_ext().relu_squared_(x)
         return x
     return x.copy_(torch.relu(x.float()).pow(2))
+
+
+def linear_gelu_glu(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor,
+                    out: torch.Tensor) -> None:
+    """out = gelu_tanh(x gate^T) * (x up^T), where glu_fuses(x, gate); out may be
+    columns of a wider row."""
+    serve_ext().glu_linear(x, gate, up, out, 1)
 
 
 def gelu_glu(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor,

@@ -430,3 +430,48 @@ def test_expanded_portions_tile_edges(DK, DV, H):
         s.masked_fill_(torch.arange(h + n)[None] > torch.arange(h, h + n)[:, None], -torch.inf)
         want = (s.softmax(-1) @ vs).transpose(0, 1).reshape(n, -1)
         assert rel(out[t:t + n].cpu(), want) < 0.004
+
+
+# ------------------------------------------------------- gated feed-forward
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (255, 130, 128), (257, 128, 192), (300, 1000, 64),
+                                   (513, 260, 1536)])
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("strided", [False, True])
+def test_glu_linear_tile_edges(M, N, K, act, strided):
+    x, w = rnd(M, K, seed=1), rnd(2 * N, K, seed=2, scale=K ** -0.5)
+    whole = torch.full((M, N + 24), 7.0, device=DEV, dtype=torch.bfloat16)
+    out = whole[:, 8:8 + N] if strided else torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    ops.serve_ext().glu_linear(x, w[:N], w[N:], out, act)
+    g, u = (x.double() @ w.double().T).split(N, 1)
+    want = (torch.nn.functional.silu(g) if act == 0 else
+            torch.nn.functional.gelu(g, approximate="tanh")) * u
+    assert rel(out, want) < 0.002       # one rounding, 2^-9 at most
+    if strided:
+        assert (whole[:, :8] == 7).all() and (whole[:, 8 + N:] == 7).all()
+
+
+@pytest.mark.parametrize("rows", [511, 512])
+@pytest.mark.parametrize("form", ["plain", "merged", "hooked", "bias"])
+def test_gated_feed_forward_takes_both_ways(rows, form):
+    from nanorlhf_amd.models.config import get_config
+    from nanorlhf_amd.models.lora import LoRALinear
+    from nanorlhf_amd.models.qwen2 import MLP
+    mlp = MLP(get_config("tiny", hidden_size=128, intermediate_size=200)).to(DEV, torch.bfloat16)
+    calls = []
+    if form == "merged":
+        mlp.gate_up_proj = LoRALinear(mlp.gate_up_proj, 8, 16)
+        torch.nn.init.normal_(mlp.gate_up_proj.lora_B)
+        mlp.gate_up_proj.merge_for_rollout()
+    elif form == "hooked":
+        mlp.gate_up_proj.register_forward_hook(lambda *a: calls.append(1))
+    elif form == "bias":
+        mlp.gate_up_proj.bias = torch.nn.Parameter(torch.ones(400, device=DEV).bfloat16())
+    x = rnd(rows, 128, seed=1)
+    with torch.no_grad():
+        got = mlp(x)
+        p = mlp.gate_up_proj
+        w = p._merged if form == "merged" else p.weight
+        g, u = (x.double() @ w.double().T + (1 if form == "bias" else 0)).split(200, 1)
+        want = (torch.nn.functional.silu(g) * u) @ mlp.down_proj.weight.double().T
+    assert rel(got, want) < 0.006       # three roundings of 2^-9 at most
+    assert len(calls) == (form == "hooked")
