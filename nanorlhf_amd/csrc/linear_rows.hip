@@ -1,0 +1,276 @@
+// Linears of at most 64 rows (decoding): y = x w^T + bias, or the gated
+// feed-forward's silu(x Wg^T) * (x Wu^T).
+//
+// Bound by reading the weights and, with more than 16 rows, by fetching x into every
+// CU.  The waves of a workgroup share the depth: each walks 64 elements at a time
+// of its own part, which direct loads bring into a ring of its own in LDS, whole
+// 128-byte lines, so that nothing waits at a barrier; at the end they add up
+// through LDS.  (Fragments loaded straight into registers touch half a line at a
+// time: 64 rows of 8960 x 1536, gated, 34 us.)  Deep products of few columns are
+// also divided among workgroups, whose 32-bit parts rows_sum_kernel adds in order.
+//
+// us for 64 / 16 / 1 rows, library before -> now:
+//   2048 x 1536       7.6 -> 5.8    7.1 -> 3.8    6.9 -> 3.7
+//   1536 x 8960       24.8 -> 15.0  27.9 -> 10.6  27.7 -> 9.7
+//   8960 x 1536, GLU  23.1 -> 20.9  41.9 -> 14.5  41.5 -> 13.8
+//   151936 x 1536     115 -> 113    159 -> 89     158 -> 83     (467 MB: 5.6 TB/s)
+#include <torch/extension.h>
+#include <ATen/hip/HIPContext.h>
+
+#include "common.h"
+#include "checks.h"
+
+struct RowsArgs {
+  const short *x, *w;      // [M, K], [N, K] (GLU: w2 the up weights)
+  const short *w2, *bias;
+  short* y;                // [M, N]
+  float* parts;            // [splits, M, N] instead of y
+  int M, N, K;
+};
+
+// at most `left` chunks of L loads each are still under way
+template <int L, int R>
+DEVINL void chunk_ready(int left) {
+  if (left >= R - 1) wait_loads<L * (R - 1)>();
+  else if (R > 3 && left == 2) wait_loads<L * 2>();
+  else if (R > 2 && left == 1) wait_loads<L>();
+  else wait_loads<0>();
+}
+
+// MF * 16 rows, NF * 16 weight rows; R chunks of 64 elements in each wave's ring
+template <int MF, int NF, int WAVES, int R, bool GLU>
+__global__ __launch_bounds__(WAVES * 64)
+void linear_rows_kernel(RowsArgs a) {
+  constexpr int COLS = GLU ? NF * 8 : NF * 16;       // of y, of a workgroup
+  constexpr int CHUNK = (MF + NF) * 16 * 64, LOADS = (MF + NF) * 2;
+  static_assert(LOADS * (R - 1) < 64, "vmcnt");
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lo = lane & 15, hi = lane >> 4;
+  const int n0 = blockIdx.x * COLS;
+  __shared__ __attribute__((aligned(16))) short ring[WAVES][R][CHUNK];    // [w rows, x rows]
+
+  // A load of a wave is 8 rows of 128 bytes, their 16-byte chunks exchanged (xor)
+  // by row pair.
+  unsigned wo[NF * 2], xo[MF * 2];
+  const short* wb[GLU ? 2 : 1] = {a.w + (long)n0 * a.K};
+  if (GLU) wb[GLU ? 1 : 0] = a.w2 + (long)n0 * a.K;
+  auto spot = [&](int row, int most) {
+    return (unsigned)(min(row, most) * a.K + (((lane & 7) ^ ((lane >> 4) & 3)) << 3)) * 2;
+  };
+#pragma unroll
+  for (int i = 0; i < NF * 2; i++) {                 // GLU: 16 of gate and of up in turn
+    const int r = 8 * (i & 1) + (lane >> 3);
+    wo[i] = spot((GLU ? i / 4 : i / 2) * 16 + r, a.N - 1 - n0) ^ (i & 1) << 6;
+  }
+#pragma unroll
+  for (int i = 0; i < MF * 2; i++) xo[i] = spot(8 * i + (lane >> 3), a.M - 1) ^ (i & 1) << 6;
+  // this wave's share of the depth
+  const int steps = a.K / 64, shares = gridDim.y * WAVES, share = blockIdx.y * WAVES + wid;
+  const int first = (int)((long)steps * share / shares);
+  const int last = (int)((long)steps * (share + 1) / shares);
+  auto fetch = [&](int step, int slot) {
+    const int k0 = step * 64;
+    short* at = ring[wid][slot];
+#pragma unroll
+    for (int i = 0; i < NF * 2; i++)
+      load_to_lds16(wb[GLU ? (i / 2) & 1 : 0] + k0, wo[i], at + i * 512);
+#pragma unroll
+    for (int i = 0; i < MF * 2; i++) load_to_lds16(a.x + k0, xo[i], at + (NF * 2 + i) * 512);
+  };
+
+  f32x4 acc[NF][MF];
+#pragma unroll
+  for (int i = 0; i < NF; i++)
+#pragma unroll
+    for (int j = 0; j < MF; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < R; i++)
+    if (first + i < last) fetch(first + i, i);
+  int slot = 0;
+  for (int step = first; step < last; step++) {
+    chunk_ready<LOADS, R>(last - 1 - step);
+    const short* at = ring[wid][slot];
+    auto part = [&](int row16, int q) {
+      return frag(at + (row16 * 16 + lo) * 64 + (((4 * q + hi) ^ ((lo >> 1) & 7)) << 3));
+    };
+    bf16x8l wf[2][NF], xf[2][MF];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+#pragma unroll
+      for (int i = 0; i < NF; i++) wf[q][i] = part(i, q);
+#pragma unroll
+      for (int j = 0; j < MF; j++) xf[q][j] = part(NF + j, q);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // read before it is filled again
+    if (step + R < last) fetch(step + R, slot);
+    slot = slot + 1 == R ? 0 : slot + 1;
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+      for (int i = 0; i < NF; i++)
+#pragma unroll
+        for (int j = 0; j < MF; j++) acc[i][j] = mfma16l(wf[q][i], xf[q][j], acc[i][j]);
+  }
+  __syncthreads();
+  // halves of the waves add up, in the same order every time
+  typedef f32x4 Sums[NF][MF][64];
+  static_assert(sizeof(Sums) * (WAVES / 2) <= sizeof(ring), "room for the sums");
+  Sums* sums = reinterpret_cast<Sums*>(&ring[0][0][0]);
+#pragma unroll
+  for (int n = WAVES / 2; n > 0; n >>= 1) {
+    if (wid >= n && wid < 2 * n) {
+#pragma unroll
+      for (int i = 0; i < NF; i++)
+#pragma unroll
+        for (int j = 0; j < MF; j++) sums[wid - n][i][j][lane] = acc[i][j];
+    }
+    __syncthreads();
+    if (wid < n) {
+#pragma unroll
+      for (int i = 0; i < NF; i++)
+#pragma unroll
+        for (int j = 0; j < MF; j++) acc[i][j] += sums[wid][i][j][lane];
+    }
+    if (n > 1) __syncthreads();
+  }
+  if (wid > 0) return;
+  // lane: row 16 j + lo, columns 16 i + 4 hi .. + 3
+  const bool whole = a.N % 4 == 0;
+#pragma unroll
+  for (int j = 0; j < MF; j++) {
+    const int m = 16 * j + lo;
+    if (m >= a.M) continue;
+#pragma unroll
+    for (int i = 0; i < NF; i += GLU ? 2 : 1) {
+      const int n = n0 + (GLU ? i / 2 : i) * 16 + 4 * hi;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        v[r] = GLU ? silu_fast(acc[i][j][r]) * acc[GLU ? i + 1 : i][j][r] : acc[i][j][r];
+        if (!GLU && a.bias && n + r < a.N) v[r] += bf2f(a.bias[n + r]);
+      }
+      if (a.parts) {
+        float* p = a.parts + ((long)blockIdx.y * a.M + m) * a.N + n;
+        if (whole && n < a.N) stv<4>(p, v);
+        else
+          for (int r = 0; r < 4; r++)
+            if (n + r < a.N) p[r] = v[r];
+      } else {
+        short* p = a.y + (long)m * a.N + n;
+        if (whole && n < a.N) stv<4>(p, v);
+        else
+          for (int r = 0; r < 4; r++)
+            if (n + r < a.N) stf(p + r, v[r]);
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(256)
+void rows_sum_kernel(const float* __restrict__ parts, const short* __restrict__ bias,
+                     short* __restrict__ y, long n, int N, int splits) {
+  const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  f32x4 s = *reinterpret_cast<const f32x4*>(parts + i);
+  for (int k = 1; k < splits; k++) s += *reinterpret_cast<const f32x4*>(parts + k * n + i);
+  float v[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) v[r] = s[r] + (bias ? bf2f(bias[(i + r) % N]) : 0.f);
+  stv<4>(y + i, v);
+}
+
+static void check_rows(const torch::Tensor& x, const torch::Tensor& w) {
+  for (const auto& t : {x, w})
+    TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.scalar_type() == torch::kBFloat16 &&
+                (uintptr_t)t.data_ptr() % 16 == 0, "linear_rows: contiguous bf16 matrices");
+  TORCH_CHECK(x.size(0) <= 64 && x.size(1) == w.size(1) && x.size(1) % 64 == 0 &&
+              x.size(1) < (1L << 30) && w.size(0) < (1L << 30),
+              "linear_rows: at most 64 rows, depth a multiple of 64");
+}
+
+template <int NF, int WAVES, int R, bool GLU>
+static void launch_rows(const RowsArgs& a, int splits) {
+  constexpr int COLS = GLU ? NF * 8 : NF * 16;
+  const dim3 grid((a.N + COLS - 1) / COLS, splits);
+#define LAUNCH(MF)                                                                           \
+  hipLaunchKernelGGL((linear_rows_kernel<MF, NF, WAVES, R, GLU>), grid, dim3(WAVES * 64), 0, \
+                     c10::hip::getCurrentHIPStream(), a)
+  switch ((a.M + 15) / 16) {
+    case 1: LAUNCH(1); break;
+    case 2: LAUNCH(2); break;
+    case 3: LAUNCH(3); break;
+    default: LAUNCH(4);
+  }
+#undef LAUNCH
+}
+
+torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias) {
+  on_gpu({x, w, bias});
+  check_rows(x, w);
+  const long M = x.size(0), K = x.size(1), N = w.size(0);
+  if (bias)
+    TORCH_CHECK(bias->scalar_type() == torch::kBFloat16 && bias->is_contiguous() &&
+                bias->numel() == N, "linear_rows: bf16 bias");
+  auto y = torch::empty({M, N}, x.options());
+  if (M == 0 || N == 0) return y;
+  RowsArgs a{};
+  a.x = (const short*)x.data_ptr();
+  a.w = (const short*)w.data_ptr();
+  const short* b = bias ? (const short*)bias->data_ptr() : nullptr;
+  a.bias = b;
+  a.y = (short*)y.data_ptr();
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  // 16 columns each while that makes at most a workgroup per CU, since the rows of
+  // x are read by each; up to 64 for more columns.  A deep product of few columns is
+  // divided until about 224 workgroups share it, which has to pay for a second kernel
+  // of 3 us: 64 rows of 1536 x 8960 15 us in 4 parts, 24 in one; 1536 x 1536 6 us in
+  // one, 7 in 2.  More than 32 rows fill LDS with one chunk of four waves.
+  const bool deep = K > 2048;
+  const int nf = deep ? (N <= 1024 ? 1 : N < 3200 ? 2 : 4) : N <= 4096 ? 1 : N <= 8192 ? 2 : 4;
+  const long tiles = (N + 16 * nf - 1) / (16 * nf);
+  const int splits = deep && N % 4 == 0 ? (int)std::min(8L, std::max(1L, (224 + tiles / 2) / tiles)) : 1;
+  torch::Tensor parts;
+  if (splits > 1) {
+    parts = torch::empty({splits, M, N}, x.options().dtype(torch::kFloat32));
+    a.parts = parts.data_ptr<float>();
+    a.bias = nullptr;
+  }
+  if (nf == 1) launch_rows<1, 4, 3, false>(a, splits);
+  else if (nf == 2) launch_rows<2, 4, 3, false>(a, splits);
+  else if (splits > 1 || M <= 32) launch_rows<4, 2, 2, false>(a, splits);
+  else launch_rows<4, 4, 1, false>(a, splits);
+  if (splits > 1)
+    hipLaunchKernelGGL(rows_sum_kernel, dim3((M * N / 4 + 255) / 256), dim3(256), 0,
+                       c10::hip::getCurrentHIPStream(), a.parts, b, a.y, M * N, (int)N, splits);
+  HIP_CHECK_LAST();
+  return y;
+}
+
+// silu(x gate^T) * (x up^T)
+torch::Tensor glu_rows(torch::Tensor x, torch::Tensor gate, torch::Tensor up) {
+  on_gpu({x, gate, up});
+  check_rows(x, gate);
+  check_rows(x, up);
+  TORCH_CHECK(gate.sizes() == up.sizes(), "glu_rows: gate and up alike");
+  const long M = x.size(0), N = gate.size(0);
+  auto y = torch::empty({M, N}, x.options());
+  if (M == 0 || N == 0) return y;
+  RowsArgs a{};
+  a.x = (const short*)x.data_ptr();
+  a.w = (const short*)gate.data_ptr();
+  a.w2 = (const short*)up.data_ptr();
+  a.y = (short*)y.data_ptr();
+  a.M = M;
+  a.N = N;
+  a.K = x.size(1);
+  // 16 columns of each, or 32 where x's rows weigh more: 64 rows of 8960 x 1536 21
+  // us against 22, of 4864 x 896 8.5 against 7.3, 32 rows of 8960 x 1536 17.4
+  // against 15.5; 64 rows of 18944 x 3584 67 us with four waves, 72 with two
+  if (M <= 32 || N <= 6144) launch_rows<2, 2, 3, true>(a, 1);
+  else if (a.K <= 2048) launch_rows<4, 2, 2, true>(a, 1);
+  else launch_rows<4, 4, 1, true>(a, 1);
+  HIP_CHECK_LAST();
+  return y;
+}

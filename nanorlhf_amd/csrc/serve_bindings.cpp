@@ -54,6 +54,9 @@ torch::Tensor rotary_qkv(torch::Tensor proj, long qoff, long koff, long voff, Op
 // glu.hip
 void glu_linear(torch::Tensor x, torch::Tensor gate, torch::Tensor up, torch::Tensor out,
                 long act);
+// linear_rows.hip
+torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, OptTensor bias);
+torch::Tensor glu_rows(torch::Tensor x, torch::Tensor gate, torch::Tensor up);
 // wkv.hip
 void token_shift(torch::Tensor h, torch::Tensor mu, OptTensor seq_lens, torch::Tensor slots,
                  OptTensor cu, OptTensor row_seq, OptTensor fresh, torch::Tensor last,
@@ -102,6 +105,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gated_norm", &gated_norm);
   m.def("gelu_glu", &gelu_glu);
   m.def("glu_linear", &glu_linear);
+  m.def("linear_rows", &linear_rows);
+  m.def("glu_rows", &glu_rows);
   m.def("relu_squared_", &relu_squared_);
   m.def("token_shift", &token_shift);
   m.def("wkv_decay", &wkv_decay);

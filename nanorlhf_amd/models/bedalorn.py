@@ -199,7 +199,7 @@ class BedalornLM(nn.Module):
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """hidden carries the logit scale."""
-        return F.linear(hidden, self.embed)
+        return ops.linear(hidden, self.embed)
 
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -7,6 +7,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
+from .lora import project
 
 ALIGN = 8
 
@@ -24,7 +25,7 @@ class SquaredReluMLP(nn.Module):
         self.down.weight.copy_(take("down", (W, self.ff)))
 
     def forward(self, h):
-        return self.down(ops.relu_squared_(self.up(h)))
+        return project(self.down, ops.relu_squared_(project(self.up, h)))
 
 
 class MixtureOfExperts(nn.Module):

@@ -20,7 +20,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
-from .lora import plain_weight
+from .lora import plain_weight, project
 from .mixers import MIXERS
 
 ALIGN = 8   # columns of a segment start at multiples of 16 bytes (bf16)
@@ -109,7 +109,7 @@ class ParallelBlock(nn.Module):
     def forward(self, h: torch.Tensor, ctx, cache) -> torch.Tensor:
         w = plain_weight(self.in_proj) if self.ff else None
         cat = torch.empty(h.shape[0], self.out_width, dtype=h.dtype, device=h.device)
-        if w is not None and ops.glu_fuses(h, w):
+        if w is not None and self.in_proj.bias is None and ops.glu_fuses(h, w):
             # the mixer's columns alone, gate and up straight into the output's input
             (a, b), (c, d) = self.cols["gate"], self.cols["up"]
             proj = F.linear(h, w[:a])
@@ -117,15 +117,15 @@ class ParallelBlock(nn.Module):
             cat[:, self.mix_out:self.ff_start] = 0
             cat[:, self.ff_start + self.ff:] = 0
             self.mixer(self.cols, proj, ctx, cache, cat[:, :self.mix_out])
-            return self.out_proj(cat)
-        proj = self.in_proj(h)
+            return project(self.out_proj, cat)
+        proj = project(self.in_proj, h)
         self.mixer(self.cols, proj, ctx, cache, cat[:, :self.mix_out])
         if self.ff:
             gate, up = (proj[:, slice(*self.cols[n])] for n in ("gate", "up"))
             pad = self.ff_start - self.mix_out
             ops.gelu_glu(gate, up, cat[:, self.mix_out:], pad,
                          self.out_width - self.ff_start - self.ff)
-        return self.out_proj(cat)
+        return project(self.out_proj, cat)
 
 
 class GonuraxLM(nn.Module):
@@ -190,4 +190,4 @@ class GonuraxLM(nn.Module):
             ids=None if self.layers else input_ids)
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden, self.lm_head_weight)
+        return ops.linear(hidden, self.lm_head_weight)

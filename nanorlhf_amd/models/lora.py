@@ -16,6 +16,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 import torch.nn.modules.module as _module
 
+from .. import ops
+
 
 def quantize_fp8_weight(w_float: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """Per-tensor e4m3 quantization: returns (w8 [N,K], scale fp32 scalar)."""
@@ -139,9 +141,9 @@ def apply_lora(model: nn.Module, cfg: LoraConfig) -> nn.Module:
 
 
 def plain_weight(proj: nn.Module) -> torch.Tensor | None:
-    """The weight of a projection whose call is F.linear(x, weight) and nothing
-    else: no gradient wanted, no bias, nobody listening to the call.  Else None."""
-    if torch.is_grad_enabled() or proj.bias is not None or any(
+    """The weight of a projection whose call is F.linear(x, weight, proj.bias) and
+    nothing else: no gradient wanted, nobody listening to the call.  Else None."""
+    if torch.is_grad_enabled() or any(
             (proj._forward_hooks, proj._forward_pre_hooks, proj._backward_hooks,
              proj._backward_pre_hooks, _module._global_forward_hooks,
              _module._global_forward_pre_hooks)):
@@ -154,6 +156,12 @@ def plain_weight(proj: nn.Module) -> torch.Tensor | None:
     else:
         return None
     return w if type(w) in (torch.Tensor, nn.Parameter) else None
+
+
+def project(proj: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """proj(x), by the kernel for few rows where it is a plain linear."""
+    w = plain_weight(proj)
+    return proj(x) if w is None else ops.linear(x, w, proj.bias)
 
 
 def merge_for_rollout(model: nn.Module, quant: str | None = None):

@@ -21,6 +21,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from .config import KVSpec, LatentSpec, StateSpec
+from .lora import project
 
 
 class LinearMixer(nn.Module):
@@ -184,7 +185,7 @@ class WKV(nn.Module):
         mixed = ops.token_shift(h, self.mu, ctx, last)
         r, k, v, g = ops.stacked_linear(mixed[:4], self.proj)
         w = ops.wkv_decay(F.linear(mixed[4], self.w1), self.w2, self.w0)
-        return self.o(ops.wkv(r, k, v, w, self.u, ctx, state, g, self.norm, self.eps))
+        return project(self.o, ops.wkv(r, k, v, w, self.u, ctx, state, g, self.norm, self.eps))
 
 
 class LatentAttention(nn.Module):
@@ -221,13 +222,13 @@ class LatentAttention(nn.Module):
         self.o.weight.copy_(take("o", (W, H * V)))
 
     def forward(self, h, ctx, cache):
-        proj = self.in_proj(h)
+        proj = project(self.in_proj, h)
         ops.latent_append(proj[:, self.q_cols:self.q_cols + self.rank], self.dkv_norm, self.eps,
                           ctx.slots, cache)
         out = torch.empty(h.shape[0], self.heads * self.vdim, dtype=h.dtype, device=h.device)
         ops.latent_attn(proj[:, :self.q_cols], cache, ctx, self.uk, self.uk_t, self.uv, out,
                         self.scale)
-        return self.o(out)
+        return project(self.o, out)
 
 
 SUBLAYER_MIXERS = {"wkv": WKV, "latent_attention": LatentAttention}

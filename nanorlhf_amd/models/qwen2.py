@@ -7,7 +7,8 @@ Replaces the reference's transformers Qwen2 + flash_attention_2 stack
     collator packs, attention gets cu_seqlens (the reference instead builds
     pad masks in a local forward(), grpo_trainer.py:90-120);
   * hot ops route through nanorlhf_amd.ops (hand-written HIP on GPU);
-  * plain projections stay torch.nn.functional.linear → rocBLAS/hipBLASLt;
+  * plain projections of many rows stay torch.nn.functional.linear →
+    rocBLAS/hipBLASLt, few rows take ops.linear's kernel;
   * the SAME module graph serves training, prefill and paged decode — the
     in-process sampler passes an AttnContext instead of booting a separate
     engine (deletes the reference's disk round trip, grpo_trainer.py:122-166).
@@ -23,7 +24,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from .config import ModelConfig, get_config
-from .lora import plain_weight
+from .lora import plain_weight, project
 
 
 @dataclass
@@ -103,7 +104,7 @@ class Attention(nn.Module):
 
     def forward(self, x: torch.Tensor, rope_table: torch.Tensor, ctx: AttnContext):
         T = x.shape[0]
-        qkv = self.qkv_proj(x)
+        qkv = project(self.qkv_proj, x)
         if ctx.mode != "train" and ctx.kv_caches is not None:
             q, k, v = ops.qkv_rope_append(qkv, rope_table, ctx.positions, self.num_heads,
                                           ctx.slots, *ctx.kv_caches[self.layer_idx],
@@ -121,7 +122,7 @@ class Attention(nn.Module):
         else:
             o = ops.flash_attn_varlen(q, k, v, ctx.cu_seqlens, ctx.max_seqlen,
                                       self.scale, causal=ctx.causal)
-        return self.o_proj(o.reshape(T, -1))
+        return project(self.o_proj, o.reshape(T, -1))
 
 
 class MLP(nn.Module):
@@ -132,8 +133,11 @@ class MLP(nn.Module):
 
     def forward(self, x):
         w = plain_weight(self.gate_up_proj)
-        act = ops.swiglu(self.gate_up_proj(x)) if w is None else ops.linear_swiglu(x, w)
-        return self.down_proj(act)
+        if w is None or self.gate_up_proj.bias is not None:
+            act = ops.swiglu(self.gate_up_proj(x))
+        else:
+            act = ops.linear_swiglu(x, w)
+        return project(self.down_proj, act)
 
 
 class RMSNorm(nn.Module):
@@ -231,7 +235,7 @@ class CausalLM(nn.Module):
         return self.model(input_ids, ctx, checkpoint=self.gradient_checkpointing)
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden, self.lm_head_weight)
+        return ops.linear(hidden, self.lm_head_weight)
 
     @staticmethod
     def train_ctx(cu_seqlens: torch.Tensor, max_seqlen: int, positions: torch.Tensor,

@@ -56,6 +56,7 @@ def ext_available() -> bool:
 from .rmsnorm import (add_rms_norm, gated_norm, residual_group_norm,  # noqa: E402,F401
                       rms_norm)
 from .rope import Rotation, build_rope_cache, qkv_rope, rope_apply  # noqa: E402,F401
+from .linear import linear  # noqa: E402,F401
 from .swiglu import (gelu_glu, glu_fuses, linear_gelu_glu, linear_swiglu,  # noqa: E402,F401
                      relu_squared_, swiglu)
 from .attention import flash_attn_varlen  # noqa: E402,F401

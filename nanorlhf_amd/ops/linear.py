@@ -1,0 +1,29 @@
+"""Linears without gradients.  Few rows (decoding) take csrc/linear_rows.hip, which
+is bound by reading the weights; the rest is the library's."""
+from __future__ import annotations
+
+import torch
+import torch.nn.functional as F
+
+from . import serve_ext
+
+# Library against the kernel, in us: 64 rows of 3584 x 18944 91 / 36, of 4608 x 3584
+# 18.7 / 15.3, of 37888 x 3584 70 / 67, of 151936 x 1536 115 / 113; with more rows x
+# weighs as much as the weights and the library's tiles share it better.
+FEW_ROWS = 64
+
+
+def few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the kernels for few rows take x [M, K] and w [N, K]."""
+    return (x.is_cuda and x.dim() == 2 and x.shape[0] <= FEW_ROWS
+            and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
+            and x.dtype == w.dtype == torch.bfloat16 and x.shape[1] % 64 == 0
+            and x.is_contiguous() and w.is_contiguous() and w.device == x.device
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """x w^T + bias."""
+    if few_rows(x, w) and (bias is None or bias.dtype == x.dtype and bias.is_contiguous()):
+        return serve_ext().linear_rows(x, w, bias)
+    return F.linear(x, w, bias)

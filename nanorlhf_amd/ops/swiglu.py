@@ -6,6 +6,7 @@ from __future__ import annotations
 import torch
 
 from . import ext, serve_ext
+from .linear import few_rows
 
 
 def _swiglu_ref(gate_up: torch.Tensor) -> torch.Tensor:
@@ -51,6 +52,8 @@ def glu_fuses(x: torch.Tensor, gate: torch.Tensor) -> bool:
 def linear_swiglu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """swiglu of x [..., K] times weight [2 I, K] (gate rows, then up rows)."""
     gate, up = weight.chunk(2)
+    if few_rows(x, gate):
+        return serve_ext().glu_rows(x, gate, up)
     if not glu_fuses(x, gate):
         return swiglu(torch.nn.functional.linear(x, weight))
     out = torch.empty(x.shape[0], gate.shape[0], dtype=x.dtype, device=x.device)

@@ -24,7 +24,7 @@ EXTENSIONS = {
            "sampling.hip", "attention.hip", "masked.hip", "lora.hip"],
     "_serve": ["serve_bindings.cpp", "kvcache.hip", "paged_attention.hip",
                "linear_attn.hip", "stream.hip", "wkv.hip", "latent_attn.hip", "moe.hip",
-               "glu.hip"],
+               "glu.hip", "linear_rows.hip"],
 }
 
 wanted = [n for n in os.environ.get("NANORLHF_EXT", "").split(",") if n] or list(EXTENSIONS)

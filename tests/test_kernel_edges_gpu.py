@@ -475,3 +475,28 @@ def test_gated_feed_forward_takes_both_ways(rows, form):
         want = (torch.nn.functional.silu(g) * u) @ mlp.down_proj.weight.double().T
     assert rel(got, want) < 0.006       # three roundings of 2^-9 at most
     assert len(calls) == (form == "hooked")
+
+
+# ---------------------------------------------------------- linears of few rows
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,K", [(8, 64), (17, 128), (1536, 2112), (1000, 8960), (4100, 192),
+                                 (8204, 128), (3204, 2176), (3207, 2176)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_linear_of_few_rows(M, N, K, bias):
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=K ** -0.5)
+    b = rnd(N, seed=3) if bias else None
+    want = x.double() @ w.double().T + (b.double() if bias else 0)
+    with torch.no_grad():
+        got = ops.linear(x, w, b)
+        assert torch.equal(got, ops.serve_ext().linear_rows(x, w, b))
+    assert rel(got, want) < 0.002       # one rounding, 2^-9 at most
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 48, 64])
+@pytest.mark.parametrize("N,K", [(8, 64), (101, 192), (6200, 128), (6150, 2112)])
+def test_gated_linear_of_few_rows(M, N, K):
+    x, w = rnd(M, K, seed=1), rnd(2 * N, K, seed=2, scale=K ** -0.5)
+    g, u = (x.double() @ w.double().T).split(N, 1)
+    with torch.no_grad():
+        got = ops.serve_ext().glu_rows(x, w[:N], w[N:])
+    assert rel(got, torch.nn.functional.silu(g) * u) < 0.002
