@@ -506,16 +506,21 @@ void paged_decode_merge_kernel(const float* __restrict__ part, const float* __re
 }
 
 // How a batch of `units` workgroups with at most `tiles` tiles each is split:
-// until there is one per CU, each with at least two tiles for every wave.  Four
+// until there is about one per CU, each with at least two tiles for every wave.  Four
 // per sequence read 32 x 2000 tokens (12 heads over 2, bf16) in 17.4 us with the
 // merge, two in 22.5, eight in 22.4 (the first tile's page, key and value
 // latencies then outweigh the rest); unsplit it took 135.  At 256 sequences and
-// more nothing is split: 2048 x 850 in fp8 take 172 us, 5.1 TB/s.
-constexpr long DECODE_FILL = 256;
+// more nothing is split: 2048 x 850 in fp8 take 172 us, 5.1 TB/s.  Nor is a short
+// context, whose walk costs no more than the merge (in fp8: 64 x 170 tokens, 9
+// tiles, 5.6 us against 7.5, 8 x 400, 19 tiles, 7.1 against 7.5; from 21 tiles on in
+// bf16 9.5 against 8.5), nor a batch of which
+// part would get a second workgroup per CU (100 x 600: 10.3 against 13.2).
+constexpr long DECODE_FILL = 256, UNSPLIT = 20;
 struct Splits { int n, per; torch::Tensor part, ms; };
 static Splits decode_splits(long units, long tiles, int DV, const torch::Tensor& like) {
   Splits s{1, (int)std::max(tiles, 1L), {}, {}};
-  const long want = std::min((DECODE_FILL + units - 1) / units, (tiles + 7) / 8);
+  const long want = tiles > UNSPLIT ? std::min((DECODE_FILL + units / 2) / units, (tiles + 7) / 8)
+                                    : 1;
   if (want > 1) {
     s.per = (int)((tiles + want - 1) / want + 3) / 4 * 4;
     s.n = (int)((tiles + s.per - 1) / s.per);
