@@ -12,8 +12,8 @@
 // us for 64 / 16 / 1 rows, library before -> now:
 //   2048 x 1536       7.6 -> 5.8    7.1 -> 3.8    6.9 -> 3.7
 //   1536 x 8960       24.8 -> 15.0  27.9 -> 10.6  27.7 -> 9.7
-//   8960 x 1536, GLU  23.1 -> 20.9  41.9 -> 14.5  41.5 -> 13.8
-//   151936 x 1536     115 -> 113    159 -> 89     158 -> 83     (467 MB: 5.6 TB/s)
+//   8960 x 1536, GLU  20.6 -> 19.9  41.6 -> 14.1  42.1 -> 13.7
+//   151936 x 1536     115 -> 108    159 -> 89     158 -> 83     (467 MB: 5.6 TB/s)
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -37,11 +37,13 @@ DEVINL void chunk_ready(int left) {
   else wait_loads<0>();
 }
 
-// MF * 16 rows, NF * 16 weight rows; R chunks of 64 elements in each wave's ring
+// MF * 16 rows, NF * 16 weight rows; R chunks of 64 elements in each wave's ring.
+// GLU: tiles of gate's and up's rows in turn, or (NF odd) 8 rows of each in a tile.
 template <int MF, int NF, int WAVES, int R, bool GLU>
 __global__ __launch_bounds__(WAVES * 64)
 void linear_rows_kernel(RowsArgs a) {
   constexpr int COLS = GLU ? NF * 8 : NF * 16;       // of y, of a workgroup
+  constexpr bool HALVES = GLU && NF % 2;
   constexpr int CHUNK = (MF + NF) * 16 * 64, LOADS = (MF + NF) * 2;
   static_assert(LOADS * (R - 1) < 64, "vmcnt");
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -58,9 +60,9 @@ void linear_rows_kernel(RowsArgs a) {
     return (unsigned)(min(row, most) * a.K + (((lane & 7) ^ ((lane >> 4) & 3)) << 3)) * 2;
   };
 #pragma unroll
-  for (int i = 0; i < NF * 2; i++) {                 // GLU: 16 of gate and of up in turn
-    const int r = 8 * (i & 1) + (lane >> 3);
-    wo[i] = spot((GLU ? i / 4 : i / 2) * 16 + r, a.N - 1 - n0) ^ (i & 1) << 6;
+  for (int i = 0; i < NF * 2; i++) {
+    const int eight = HALVES ? i / 2 : GLU ? i / 4 * 2 + (i & 1) : i;
+    wo[i] = spot(eight * 8 + (lane >> 3), a.N - 1 - n0) ^ (i & 1) << 6;
   }
 #pragma unroll
   for (int i = 0; i < MF * 2; i++) xo[i] = spot(8 * i + (lane >> 3), a.M - 1) ^ (i & 1) << 6;
@@ -73,7 +75,7 @@ void linear_rows_kernel(RowsArgs a) {
     short* at = ring[wid][slot];
 #pragma unroll
     for (int i = 0; i < NF * 2; i++)
-      load_to_lds16(wb[GLU ? (i / 2) & 1 : 0] + k0, wo[i], at + i * 512);
+      load_to_lds16(wb[GLU ? (HALVES ? i : i / 2) & 1 : 0] + k0, wo[i], at + i * 512);
 #pragma unroll
     for (int i = 0; i < MF * 2; i++) load_to_lds16(a.x + k0, xo[i], at + (NF * 2 + i) * 512);
   };
@@ -134,21 +136,25 @@ void linear_rows_kernel(RowsArgs a) {
     if (n > 1) __syncthreads();
   }
   if (wid > 0) return;
-  // lane: row 16 j + lo, columns 16 i + 4 hi .. + 3
+  // lane: row 16 j + lo, columns 16 i + 4 hi .. + 3 (HALVES: 8 i + 4 hi .. + 3, up's
+  // in the wave's upper half)
   const bool whole = a.N % 4 == 0;
 #pragma unroll
   for (int j = 0; j < MF; j++) {
     const int m = 16 * j + lo;
-    if (m >= a.M) continue;
 #pragma unroll
-    for (int i = 0; i < NF; i += GLU ? 2 : 1) {
-      const int n = n0 + (GLU ? i / 2 : i) * 16 + 4 * hi;
+    for (int i = 0; i < NF; i += GLU && !HALVES ? 2 : 1) {
+      const int n = n0 + (GLU ? i * 8 : i * 16) + 4 * hi;
       float v[4];
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        v[r] = GLU ? silu_fast(acc[i][j][r]) * acc[GLU ? i + 1 : i][j][r] : acc[i][j][r];
-        if (!GLU && a.bias && n + r < a.N) v[r] += bf2f(a.bias[n + r]);
+        v[r] = acc[i][j][r];
+        if (GLU)
+          v[r] = silu_fast(v[r]) * (HALVES ? __shfl_xor(v[r], 32) : acc[GLU && !HALVES ? i + 1 : i][j][r]);
+        else if (a.bias && n + r < a.N)
+          v[r] += bf2f(a.bias[n + r]);
       }
+      if (m >= a.M || (HALVES && hi > 1)) continue;
       if (a.parts) {
         float* p = a.parts + ((long)blockIdx.y * a.M + m) * a.N + n;
         if (whole && n < a.N) stv<4>(p, v);
@@ -226,7 +232,8 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, c10::optional<torch:
   // x are read by each; up to 64 for more columns.  A deep product of few columns is
   // divided until about 224 workgroups share it, which has to pay for a second kernel
   // of 3 us: 64 rows of 1536 x 8960 15 us in 4 parts, 24 in one; 1536 x 1536 6 us in
-  // one, 7 in 2.  More than 32 rows fill LDS with one chunk of four waves.
+  // one, 7 in 2.  For more than 32 rows wider tiles share x better: 64 of 151936 x
+  // 1536 108 us, with 64 columns 113 to 118.
   const bool deep = K > 2048;
   const int nf = deep ? (N <= 1024 ? 1 : N < 3200 ? 2 : 4) : N <= 4096 ? 1 : N <= 8192 ? 2 : 4;
   const long tiles = (N + 16 * nf - 1) / (16 * nf);
@@ -240,7 +247,7 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, c10::optional<torch:
   if (nf == 1) launch_rows<1, 4, 3, false>(a, splits);
   else if (nf == 2) launch_rows<2, 4, 3, false>(a, splits);
   else if (splits > 1 || M <= 32) launch_rows<4, 2, 2, false>(a, splits);
-  else launch_rows<4, 4, 1, false>(a, splits);
+  else launch_rows<8, 2, 1, false>(a, splits);
   if (splits > 1)
     hipLaunchKernelGGL(rows_sum_kernel, dim3((M * N / 4 + 255) / 256), dim3(256), 0,
                        c10::hip::getCurrentHIPStream(), a.parts, b, a.y, M * N, (int)N, splits);
@@ -265,12 +272,11 @@ torch::Tensor glu_rows(torch::Tensor x, torch::Tensor gate, torch::Tensor up) {
   a.M = M;
   a.N = N;
   a.K = x.size(1);
-  // 16 columns of each, or 32 where x's rows weigh more: 64 rows of 8960 x 1536 21
-  // us against 22, of 4864 x 896 8.5 against 7.3, 32 rows of 8960 x 1536 17.4
-  // against 15.5; 64 rows of 18944 x 3584 67 us with four waves, 72 with two
-  if (M <= 32 || N <= 6144) launch_rows<2, 2, 3, true>(a, 1);
-  else if (a.K <= 2048) launch_rows<4, 2, 2, true>(a, 1);
-  else launch_rows<4, 4, 1, true>(a, 1);
+  // Up to 6144 columns 16 to a workgroup, else 40, which for 8960 makes one for each
+  // of 224 CUs: 64 rows of 8960 x 1536 18.7 us with 40, 21 with 32 (280 workgroups)
+  // and with 16; of 18944 x 3584 57 against 67; of 4864 x 896 7.3 with 16, 8.9 with 24
+  if (N <= 6144) launch_rows<2, 2, 3, true>(a, 1);
+  else launch_rows<5, 2, 2, true>(a, 1);
   HIP_CHECK_LAST();
   return y;
 }

@@ -8,7 +8,7 @@ import torch.nn.functional as F
 from . import serve_ext
 
 # Library against the kernel, in us: 64 rows of 3584 x 18944 91 / 36, of 4608 x 3584
-# 18.7 / 15.3, of 37888 x 3584 70 / 67, of 151936 x 1536 115 / 113; with more rows x
+# 18.7 / 15.3, of 37888 x 3584 70 / 57, of 151936 x 1536 115 / 108; with more rows x
 # weighs as much as the weights and the library's tiles share it better.
 FEW_ROWS = 64
 
