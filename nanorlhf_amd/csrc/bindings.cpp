@@ -55,6 +55,12 @@ std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
                                          torch::Tensor cu_seqlens, long max_seqlen,
                                          double scale, bool causal);
 
+// lora_grad.hip
+std::vector<torch::Tensor> lora_grads(c10::optional<torch::Tensor> x,
+                                      c10::optional<torch::Tensor> du,
+                                      c10::optional<torch::Tensor> dy,
+                                      c10::optional<torch::Tensor> u);
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm_fwd", &rmsnorm_fwd);
   m.def("rmsnorm_bwd", &rmsnorm_bwd, py::arg("dy"), py::arg("x"), py::arg("w"),
@@ -67,6 +73,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("swiglu_bwd", &swiglu_bwd);
   m.def("ce_rowstats", &ce_rowstats);
   m.def("ce_backward_dlogits", &ce_backward_dlogits);
+  m.def("lora_grads", &lora_grads);
   m.def("adamw_step", &adamw_step);
   m.def("adamw_step_many", &adamw_step_many);
   m.def("decode_inputs", &decode_inputs);

@@ -8,8 +8,8 @@ kernel does ≈(H+64)/H of the base GEMM's work in a single launch.
 Backward (W frozen under LoRA — no dW GEMM at all):
     du = s·(dy·B)            [M,r]   (skinny, hipBLASLt)
     dx = dy·W + du·A         = the SAME kernel on (dy, Wᵀ) + (du, Aᵀ)
-    dA = duᵀ·x               [r,H]   (skinny, hipBLASLt)
-    dB = dyᵀ·u               [N,r]   (skinny, hipBLASLt)
+    dA = duᵀ·x               [r,H]   } one launch of csrc/lora_grad.hip
+    dB = dyᵀ·u               [N,r]   }
 Wᵀ is cached once per linear (W never changes while LoRA trains).
 
 Constraints for the fused path: K % 64 == 0, rank == 64 (the reference
@@ -112,9 +112,17 @@ class _FusedLoRAFn(torch.autograd.Function):
             # dx = dy·W + du·A → same dispatch on (dy, Wᵀ) + (du, Aᵀ)
             a_t = lora_A.t().contiguous()
             dx = _dispatch_gemm(dy, w_t, du, a_t, None)
-        dA = du.t() @ x if ctx.needs_input_grad[3] else None
-        dB = dy.t() @ u if ctx.needs_input_grad[4] else None
-        return dx, None, None, dA, dB, None, None
+        want_A, want_B = ctx.needs_input_grad[3:5]
+        if not (want_A or want_B):
+            return dx, None, None, None, None, None, None
+        if dy.shape[1] % 8 == 0 and x.dtype == dy.dtype == torch.bfloat16:
+            dA, dB = ext().lora_grads(
+                *((x.contiguous(), du.contiguous()) if want_A else (None, None)),
+                *((dy, u.contiguous()) if want_B else (None, None)))
+        else:
+            dA, dB = (a.t() @ b if want else None
+                      for a, b, want in ((du, x, want_A), (dy, u, want_B)))
+        return dx, None, None, dA if want_A else None, dB if want_B else None, None, None
 
 
 def fused_lora_linear(x: torch.Tensor, w: torch.Tensor,

@@ -21,7 +21,8 @@ CSRC = os.path.join(ROOT, "nanorlhf_amd", "csrc")
 
 EXTENSIONS = {
     "_C": ["bindings.cpp", "elementwise.hip", "logprob.hip", "adamw.hip",
-           "sampling.hip", "attention.hip", "masked.hip", "lora.hip"],
+           "sampling.hip", "attention.hip", "masked.hip", "lora.hip",
+           "lora_grad.hip"],
     "_serve": ["serve_bindings.cpp", "kvcache.hip", "paged_attention.hip",
                "linear_attn.hip", "stream.hip", "wkv.hip", "latent_attn.hip", "moe.hip",
                "glu.hip", "linear_rows.hip"],

@@ -500,3 +500,16 @@ def test_gated_linear_of_few_rows(M, N, K):
     with torch.no_grad():
         got = ops.serve_ext().glu_rows(x, w[:N], w[N:])
     assert rel(got, torch.nn.functional.silu(g) * u) < 0.002
+
+
+# --------------------------------------------------------- adapter gradients
+@pytest.mark.parametrize("M", [1, 63, 64, 65, 511, 1023, 1025, 5000])
+@pytest.mark.parametrize("K,N", [(8, 120), (128, 136), (1536, 264), (200, 2000)])
+def test_adapter_gradients_tile_edges(M, K, N):
+    x, dy, u, du = (rnd(M, n, seed=i) for i, n in enumerate((K, N, 64, 64)))
+    dA, dB = ops.ext().lora_grads(x, du, dy, u)
+    wA, wB = du.double().T @ x.double(), dy.double().T @ u.double()
+    assert dA.shape == (64, K) and dB.shape == (N, 64)
+    assert rel(dA, wA) < 0.002 and rel(dB, wB) < 0.002      # one rounding, 2^-9 at most
+    assert torch.equal(ops.ext().lora_grads(x, du, None, None)[0], dA)
+    assert torch.equal(ops.ext().lora_grads(None, None, dy, u)[1], dB)
