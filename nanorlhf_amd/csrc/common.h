@@ -214,6 +214,11 @@ DEVINL void load_to_lds16(const void* base, unsigned offset, const void* at) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                ::"s"(lds_address(at)), "v"(offset), "s"(in_sgprs(base)) : "memory");
 }
+// the same with an address for every lane
+DEVINL void load_to_lds16(const void* p, const void* at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               ::"s"(lds_address(at)), "v"(p) : "memory");
+}
 DEVINL void load_to_lds4(const void* base, unsigned offset, const void* at) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                ::"s"(lds_address(at)), "v"(offset), "s"(in_sgprs(base)) : "memory");
@@ -225,6 +230,17 @@ DEVINL void wait_loads() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4) << 14 | 0x0f70);   // vmcnt alone
   asm volatile("" ::: "memory");
+}
+
+// The oldest of a ring of R chunks, L loads of this wave each, has arrived, if at
+// most `left` younger ones are under way.
+template <int L, int R>
+DEVINL void chunk_ready(int left) {
+  static_assert(R <= 4 && L * (R - 1) < 64, "vmcnt");
+  if (left >= R - 1) wait_loads<L * (R - 1)>();
+  else if (R > 3 && left == 2) wait_loads<L * 2>();
+  else if (R > 2 && left == 1) wait_loads<L>();
+  else wait_loads<0>();
 }
 
 // wave-private LDS write->read ordering (staging buffers written and read

@@ -28,15 +28,6 @@ struct RowsArgs {
   int M, N, K;
 };
 
-// at most `left` chunks of L loads each are still under way
-template <int L, int R>
-DEVINL void chunk_ready(int left) {
-  if (left >= R - 1) wait_loads<L * (R - 1)>();
-  else if (R > 3 && left == 2) wait_loads<L * 2>();
-  else if (R > 2 && left == 1) wait_loads<L>();
-  else wait_loads<0>();
-}
-
 // MF * 16 rows, NF * 16 weight rows; R chunks of 64 elements in each wave's ring.
 // GLU: tiles of gate's and up's rows in turn, or (NF odd) 8 rows of each in a tile.
 template <int MF, int NF, int WAVES, int R, bool GLU>
@@ -45,7 +36,6 @@ void linear_rows_kernel(RowsArgs a) {
   constexpr int COLS = GLU ? NF * 8 : NF * 16;       // of y, of a workgroup
   constexpr bool HALVES = GLU && NF % 2;
   constexpr int CHUNK = (MF + NF) * 16 * 64, LOADS = (MF + NF) * 2;
-  static_assert(LOADS * (R - 1) < 64, "vmcnt");
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lo = lane & 15, hi = lane >> 4;
   const int n0 = blockIdx.x * COLS;

@@ -513,3 +513,13 @@ def test_adapter_gradients_tile_edges(M, K, N):
     assert rel(dA, wA) < 0.002 and rel(dB, wB) < 0.002      # one rounding, 2^-9 at most
     assert torch.equal(ops.ext().lora_grads(x, du, None, None)[0], dA)
     assert torch.equal(ops.ext().lora_grads(None, None, dy, u)[1], dB)
+
+
+# ------------------------------------------------------- grouped products
+@pytest.mark.parametrize("T", [1, 12, 13, 32])
+@pytest.mark.parametrize("G,N,K", [(1, 24, 8), (3, 100, 72), (2, 1030, 200), (40, 700, 1000)])
+def test_grouped_product_of_few_rows(T, G, N, K):
+    x, w = rnd(T, G, K, seed=1), rnd(G, N, K, seed=2, scale=K ** -0.5)
+    got = ops.group_linear(x, w)
+    want = torch.einsum("tgk,gnk->tgn", x.double().cpu(), w.double().cpu())
+    assert rel(got.cpu(), want) < 0.002            # one rounding, 2^-9 at most
