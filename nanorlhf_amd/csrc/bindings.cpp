@@ -60,6 +60,7 @@ std::vector<torch::Tensor> lora_grads(c10::optional<torch::Tensor> x,
                                       c10::optional<torch::Tensor> du,
                                       c10::optional<torch::Tensor> dy,
                                       c10::optional<torch::Tensor> u);
+torch::Tensor lora_down(torch::Tensor z, torch::Tensor p, double scale, bool flat);
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm_fwd", &rmsnorm_fwd);
@@ -74,6 +75,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ce_rowstats", &ce_rowstats);
   m.def("ce_backward_dlogits", &ce_backward_dlogits);
   m.def("lora_grads", &lora_grads);
+  m.def("lora_down", &lora_down);
   m.def("adamw_step", &adamw_step);
   m.def("adamw_step_many", &adamw_step_many);
   m.def("decode_inputs", &decode_inputs);

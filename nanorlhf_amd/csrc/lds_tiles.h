@@ -60,8 +60,9 @@ DEVINL bf16x8 row_frag(const short* tile, int r0, int ds, int lane) {
       tile + row * D + (((2 * ds + (lane >> 5)) ^ swz<D>(row)) << 3));
 }
 
-// column d0 + lane % 32, rows r0 + {0-3, 8-11} + 4 * half (r0 a multiple of 16)
-template <int D>
+// column d0 + lane % 32, rows r0 + {0-3, 8-11} + 4 * half, the order of a result's
+// registers, or (IN_ORDER) r0 + 8 * half + {0-7}, that of row_frag (r0 a multiple of 16)
+template <int D, bool IN_ORDER = false>
 DEVINL bf16x8 col_frag(const short* tile, int r0, int d0, int lane) {
   typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
   const int i = lane & 15;
@@ -69,7 +70,7 @@ DEVINL bf16x8 col_frag(const short* tile, int r0, int d0, int lane) {
   union { s16x4 h[2]; bf16x8 f; } u;
 #pragma unroll
   for (int p = 0; p < 2; p++) {
-    const int row = r0 + 8 * p + 4 * (lane >> 5) + (i >> 2);
+    const int row = r0 + (IN_ORDER ? 4 : 8) * p + (IN_ORDER ? 8 : 4) * (lane >> 5) + (i >> 2);
     const short* a = tile + row * D + (((col >> 3) ^ swz<D>(row)) << 3) + (col & 7);
     u.h[p] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)a);
   }

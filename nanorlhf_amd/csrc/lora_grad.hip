@@ -167,3 +167,124 @@ std::vector<torch::Tensor> lora_grads(c10::optional<torch::Tensor> x,
   HIP_CHECK_LAST();
   return outs;
 }
+
+// ------------------------------------------------------- down to the rank
+// out [M, 64] = scale z p: p is A^T of A [64, C] (FLAT) or B [C, 64].  A workgroup
+// owns 64 rows and a part of the columns, 64 at a time through three LDS buffers.
+// Bound by reading z once; a few rows are divided among parts of the columns.  48720
+// x 1536 25 us (6 TB/s), library 29; 8000 x 1536 11, library 26; 240 x 896 8.5,
+// library 25, of which the host's calls are most.
+template <bool FLAT>
+__global__ __launch_bounds__(256, 3)
+void lora_down_kernel(const short* __restrict__ z, const short* __restrict__ p,
+                      short* __restrict__ out, float* __restrict__ parts, int M, int C, int splits,
+                      float scale) {
+  constexpr int R = 3, LOADS = 4;          // buffers, loads of a wave for one
+  const int tile = blockIdx.x / splits, split = blockIdx.x % splits;
+  const int m0 = tile * TILE, left = M - m0;
+  const int steps = (C + TILE - 1) / TILE;
+  const int first = (int)((long)steps * split / splits);
+  const int last = (int)((long)steps * (split + 1) / splits);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), hi = lane >> 5;
+  const int rows0 = 32 * (wid & 1), rank0 = 32 * (wid >> 1);
+  __shared__ __attribute__((aligned(16))) short zt[R][TILE * TILE], pt[R][TILE * RANK];
+
+  const short* zb = z + (long)m0 * C;
+  auto stage = [&](int step, int buf) {
+    const int k0 = step * TILE, wide = min(TILE, C - k0);
+#pragma unroll
+    for (int i = 0; i < TILE * TILE / 8; i += 256) {       // columns past the last: the first
+      const int idx = i + tid, row = idx >> 3, c = ((idx & 7) ^ swz<TILE>(row)) * 8;
+      load_to_lds16(zb + k0, (unsigned)(min(row, left - 1) * C + (c < wide ? c : 0)) * 2,
+                    &zt[buf][(i + wid * 64) * 8]);
+    }
+    if (FLAT) stage_tile<TILE>(p + k0, C, RANK, pt[buf]);
+    else stage_tile<RANK>(p + (long)k0 * RANK, RANK, wide, pt[buf]);
+  };
+  f32x16_t acc{};
+#pragma unroll
+  for (int i = 0; i < R - 1; i++)
+    if (first + i < last) stage(first + i, i);
+  int buf = 0;
+  for (int step = first; step < last; step++) {
+    if (step + 1 < last) wait_loads<LOADS>();
+    else wait_loads<0>();
+    __syncthreads();
+    if (step + R - 1 < last) stage(step + R - 1, buf + R - 1 >= R ? buf - 1 : buf + R - 1);
+    const int wide = C - step * TILE;
+    if (!FLAT && wide < TILE) {                            // the last: no columns past the end
+      for (int i = tid; i < TILE * TILE / 8; i += 256) {
+        const int row = i >> 3, c = ((i & 7) ^ swz<TILE>(row)) * 8;
+        if (c >= wide) *reinterpret_cast<s16x8*>(&zt[buf][i * 8]) = s16x8{};
+      }
+      for (int i = tid; i < (TILE - wide) * RANK / 8; i += 256)
+        *reinterpret_cast<s16x8*>(&pt[buf][wide * RANK + i * 8]) = s16x8{};
+      __syncthreads();
+    }
+#pragma unroll
+    for (int ks = 0; ks < TILE / 16; ks++) {
+      const bf16x8 zf = row_frag<TILE>(zt[buf], rows0, ks, lane);
+      const bf16x8 pf = FLAT ? row_frag<TILE>(pt[buf], rank0, ks, lane)
+                             : col_frag<RANK, true>(pt[buf], 16 * ks, rank0, lane);
+      acc = mfma32x32x16(pf, zf, acc);
+    }
+    buf = buf + 1 == R ? 0 : buf + 1;
+  }
+  // lane: row m0 + rows0 + lane % 32, ranks rank0 + crow(0 .. 15)
+  const int m = m0 + rows0 + (lane & 31);
+  if (m >= M) return;
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    const long at = (long)m * RANK + rank0 + crow(4 * g, hi);
+    float o[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) o[k] = acc[4 * g + k] * scale;
+    if (splits > 1) stv<4>(parts + (long)split * M * RANK + at, o);
+    else stv<4>(out + at, o);
+  }
+}
+
+__global__ __launch_bounds__(256)
+void lora_down_sum_kernel(const float* __restrict__ parts, short* __restrict__ out, long n,
+                          int splits) {
+  const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  f32x4 s = *reinterpret_cast<const f32x4*>(parts + i);
+#pragma unroll 4
+  for (int k = 1; k < splits; k++) s += *reinterpret_cast<const f32x4*>(parts + k * n + i);
+  float o[4] = {s[0], s[1], s[2], s[3]};
+  stv<4>(out + i, o);
+}
+
+// scale z A^T with A [64, C], or scale z B with B [C, 64] (`flat` tells which)
+torch::Tensor lora_down(torch::Tensor z, torch::Tensor p, double scale, bool flat) {
+  on_gpu({z, p});
+  for (const auto& t : {z, p})
+    TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.scalar_type() == torch::kBFloat16 &&
+                (uintptr_t)t.data_ptr() % 16 == 0, "lora_down: contiguous bf16 matrices");
+  const long M = z.size(0), C = z.size(1);
+  TORCH_CHECK(p.size(flat ? 0 : 1) == RANK && p.size(flat ? 1 : 0) == C, "lora_down: rank 64");
+  TORCH_CHECK(C > 0 && C % (flat ? TILE : 8) == 0 && C < (1L << 24) && M < (1L << 31) - TILE,
+              "lora_down: columns a multiple of ", flat ? TILE : 8);
+  auto out = torch::empty({M, RANK}, z.options());
+  if (M == 0) return out;
+  const long tiles = (M + TILE - 1) / TILE, steps = (C + TILE - 1) / TILE;
+  const int splits = (int)std::max(1L, std::min({384 / tiles, steps / 3, 16L}));
+  torch::Tensor parts;
+  if (splits > 1) parts = torch::empty({splits, M * RANK}, z.options().dtype(torch::kFloat32));
+  float* pp = splits > 1 ? parts.data_ptr<float>() : nullptr;
+  auto stream = c10::hip::getCurrentHIPStream();
+#define LAUNCH(FLAT)                                                                          \
+  hipLaunchKernelGGL((lora_down_kernel<FLAT>), dim3(tiles * splits), dim3(256), 0, stream,    \
+                     (const short*)z.data_ptr(), (const short*)p.data_ptr(),                  \
+                     (short*)out.data_ptr(), pp, (int)M, (int)C, splits, (float)scale)
+  if (flat) LAUNCH(true);
+  else LAUNCH(false);
+#undef LAUNCH
+  if (splits > 1)
+    hipLaunchKernelGGL(lora_down_sum_kernel, dim3((M * RANK / 4 + 255) / 256), dim3(256), 0,
+                       stream, pp, (short*)out.data_ptr(), M * RANK, splits);
+  HIP_CHECK_LAST();
+  return out;
+}

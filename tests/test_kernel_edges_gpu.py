@@ -523,3 +523,16 @@ def test_grouped_product_of_few_rows(T, G, N, K):
     got = ops.group_linear(x, w)
     want = torch.einsum("tgk,gnk->tgn", x.double().cpu(), w.double().cpu())
     assert rel(got.cpu(), want) < 0.002            # one rounding, 2^-9 at most
+
+
+@pytest.mark.parametrize("M", [1, 63, 64, 65, 240, 1537, 25000])
+@pytest.mark.parametrize("C", [8, 64, 120, 192, 1536, 1992])
+def test_product_down_to_the_rank(M, C):
+    z = rnd(M, C, seed=1)
+    for flat in (True, False):
+        if flat and C % 64:
+            continue
+        p = rnd(*((64, C) if flat else (C, 64)), seed=2, scale=C ** -0.5)
+        got = ops.ext().lora_down(z, p, 0.25, flat)
+        want = 0.25 * z.double() @ (p.T if flat else p).double()
+        assert rel(got, want) < 0.002              # one rounding, 2^-9 at most
