@@ -647,3 +647,45 @@ void paged_attn_decode_window(torch::Tensor q, torch::Tensor k_cache, torch::Ten
 #undef LAUNCH_KV
   HIP_CHECK_LAST();
 }
+
+// ----------------------------------------------------------- copies of pages
+// pages[dst[i]] = pages[src[i]] in every tensor, 64 of them per launch; a page is
+// contiguous.  What samples of one prompt share is computed for the first alone.
+struct PagePools {
+  char* base[64];
+  long bytes[64];        // of a page, multiples of 16
+};
+
+__global__ __launch_bounds__(256)
+void copy_pages_kernel(PagePools t, const int* __restrict__ src, const int* __restrict__ dst) {
+  const long bytes = t.bytes[blockIdx.y];
+  const char* from = t.base[blockIdx.y] + src[blockIdx.x] * bytes;
+  char* to = t.base[blockIdx.y] + dst[blockIdx.x] * bytes;
+  for (long i = threadIdx.x * 16L; i < bytes; i += 256 * 16)
+    *reinterpret_cast<uint4*>(to + i) = *reinterpret_cast<const uint4*>(from + i);
+}
+
+void copy_pages(std::vector<torch::Tensor> pools, torch::Tensor src, torch::Tensor dst) {
+  on_gpu({src, dst});
+  TORCH_CHECK(src.scalar_type() == torch::kInt && dst.scalar_type() == torch::kInt &&
+              src.is_contiguous() && dst.is_contiguous() && src.numel() == dst.numel(),
+              "copy_pages: int32 page numbers");
+  const long n = src.numel();
+  if (n == 0) return;
+  for (size_t i = 0; i < pools.size(); i += 64) {
+    PagePools t;
+    const size_t here = std::min<size_t>(64, pools.size() - i);
+    for (size_t k = 0; k < here; k++) {
+      const auto& p = pools[i + k];
+      on_gpu({p});
+      t.base[k] = (char*)p.data_ptr();
+      t.bytes[k] = p.size(0) ? p.numel() / p.size(0) * p.element_size() : 0;
+      TORCH_CHECK(p.is_contiguous() && t.bytes[k] % 16 == 0 && (uintptr_t)t.base[k] % 16 == 0,
+                  "copy_pages: contiguous pages of whole 16 bytes");
+    }
+    hipLaunchKernelGGL(copy_pages_kernel, dim3(n, here), dim3(256), 0,
+                       c10::hip::getCurrentHIPStream(), t, src.data_ptr<int>(),
+                       dst.data_ptr<int>());
+  }
+  HIP_CHECK_LAST();
+}

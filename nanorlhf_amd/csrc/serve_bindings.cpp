@@ -12,6 +12,7 @@ std::vector<torch::Tensor> qkv_rope_append(torch::Tensor qkv, torch::Tensor tabl
                                            torch::Tensor positions, torch::Tensor slots,
                                            torch::Tensor k_cache, torch::Tensor v_cache, long Hq,
                                            bool want_kv);
+void copy_pages(std::vector<torch::Tensor> pools, torch::Tensor src, torch::Tensor dst);
 torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor k_cache,
                                 torch::Tensor v_cache, torch::Tensor block_tables,
                                 torch::Tensor seq_lens, double scale);
@@ -94,6 +95,7 @@ torch::Tensor moe_down(torch::Tensor act, torch::Tensor down, torch::Tensor list
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_append", &kv_append);
+  m.def("copy_pages", &copy_pages);
   m.def("qkv_rope_append", &qkv_rope_append);
   m.def("paged_attn_decode", &paged_attn_decode);
   m.def("paged_attn_decode_window", &paged_attn_decode_window);

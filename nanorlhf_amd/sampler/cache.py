@@ -14,6 +14,7 @@ from __future__ import annotations
 import numpy as np
 import torch
 
+from ..ops import serve_ext
 from ..models.config import KVSpec, LatentSpec, StateSpec
 
 
@@ -66,6 +67,18 @@ class PagedKVCache:
 
     def free(self, pages: list[int]):
         self._free.extend(pages)
+
+    def copy_prompts(self, pairs: list[tuple["SeqState", "SeqState"]]):
+        """For each (have, want) the pages of have's tokens, copied to want's."""
+        n = [-(-len(a) // self.page_size) for a, _ in pairs]
+        src, dst = (torch.tensor([p for pair, k in zip(pairs, n) for p in pair[i].pages[:k]],
+                                 dtype=torch.int32, device=self.device) for i in (0, 1))
+        pools = [t for layer in self.layers for t in layer]
+        if src.is_cuda:
+            serve_ext().copy_pages(pools, src, dst)
+        else:
+            for t in pools:
+                t[dst.long()] = t[src.long()]
 
     def release(self, seq: "SeqState"):
         """Give back everything a sequence holds."""

@@ -223,20 +223,33 @@ class SamplerEngine:
                 total += len(seqs[i])
                 chunk.append(seqs[i])
                 i += 1
-            lens = [len(s) for s in chunk]
-            ids = torch.tensor([t for s in chunk for t in s.tokens], dtype=torch.long,
+            # samples of one prompt run it once
+            row, once, twins = {}, [], []
+            for s in chunk:
+                key = tuple(s.tokens)
+                if key in row:
+                    twins.append((once[row[key]], s))
+                else:
+                    row[key] = len(once)
+                    once.append(s)
+            lens = [len(s) for s in once]
+            ids = torch.tensor([t for s in once for t in s.tokens], dtype=torch.long,
                                device=self.device)
-            cu = torch.zeros(len(chunk) + 1, dtype=torch.int32, device=self.device)
+            cu = torch.zeros(len(once) + 1, dtype=torch.int32, device=self.device)
             cu[1:] = torch.cumsum(torch.tensor(lens, dtype=torch.int32, device=self.device), 0)
             pos = torch.cat([torch.arange(n, device=self.device) for n in lens])
             slots = torch.from_numpy(np.concatenate(
-                [s.slots_for(0, len(s), self.pool.page_size) for s in chunk])).to(self.device)
+                [s.slots_for(0, len(s), self.pool.page_size) for s in once])).to(self.device)
             ctx = AttnContext(mode="prefill", positions=pos, cu_seqlens=cu,
                               max_seqlen=max(lens), kv_caches=self.pool.layers, slots=slots)
-            hidden = self.model(ids, ctx)
+            hidden = self.model(ids, ctx)[cu[1:].long() - 1]
+            if twins:
+                self.pool.copy_prompts(twins)
+                hidden = hidden[torch.tensor([row[tuple(s.tokens)] for s in chunk],
+                                             device=self.device)]
             for s in chunk:
                 s.computed = len(s)
-            self._record_first(chunk, hidden[cu[1:].long() - 1], params)
+            self._record_first(chunk, hidden, params)
 
     # --------------------------------------------------------------- decode
     def _decode_step_eager(self, db: DecodeBatch, params: SamplingParams):

@@ -536,3 +536,17 @@ def test_product_down_to_the_rank(M, C):
         got = ops.ext().lora_down(z, p, 0.25, flat)
         want = 0.25 * z.double() @ (p.T if flat else p).double()
         assert rel(got, want) < 0.002              # one rounding, 2^-9 at most
+
+
+@pytest.mark.parametrize("tensors,n", [(1, 1), (2, 7), (64, 3), (67, 5)])
+def test_copies_of_pages(tensors, n):
+    g = torch.Generator().manual_seed(tensors)
+    pools = [torch.randint(0, 255, (2 * n + 3, 16 * (1 + i % 5) * (300 if i == 0 else 1)),
+                           generator=g, dtype=torch.uint8).to(DEV) for i in range(tensors)]
+    want = [p.clone() for p in pools]
+    order = torch.randperm(2 * n + 3, generator=g)
+    src, dst = order[:n], order[n:2 * n]
+    for p in want:
+        p[dst.to(DEV)] = p[src.to(DEV)]
+    ops.serve_ext().copy_pages(pools, src.int().to(DEV), dst.int().to(DEV))
+    assert all(torch.equal(a, b) for a, b in zip(pools, want))

@@ -86,3 +86,28 @@ def test_max_num_seqs_cap():
     out = eng.generate(prompts, params)
     big = SamplerEngine(m, kv_pool_tokens=8192, page_size=16)
     assert torch.equal(out, big.generate(prompts, params))
+
+
+def test_samples_of_one_prompt_are_as_if_run_alone():
+    """Prompts that occur more than once run once; every sample still draws for itself
+    and every page is its own."""
+    torch.manual_seed(0)
+    m = CausalLM.from_preset("tiny").eval()
+    p = [torch.randint(2, 1000, (n,)).tolist() for n in (15, 16, 17)]
+    eng = SamplerEngine(m, kv_pool_tokens=4096, page_size=16)
+    seen, forward = [], m.model.forward
+    m.model.forward = lambda ids, *a, **k: (seen.append(len(ids)), forward(ids, *a, **k))[1]
+    out, lp = eng.generate([p[0], p[1], p[0], p[2]], SamplingParams(
+        n=3, temperature=1.0, top_p=1.0, max_tokens=6, seed=4), return_logprobs=True)
+    m.model.forward = forward
+    assert seen[0] == 15 + 16 + 17
+    assert len({tuple(r) for r in out.tolist()}) > 4             # each draws for itself
+    for i, q in enumerate([p[0], p[1], p[0], p[2]]):
+        for j in range(3):
+            toks = q + out[3 * i + j].tolist()
+            ids, cu, mx, pos = pack_sequences([torch.tensor(toks)])
+            with torch.no_grad():
+                z = m.logits(m(ids, CausalLM.train_ctx(cu, mx, pos))).float().log_softmax(-1)
+            want = [float(z[len(q) - 1 + k, t]) for k, t in enumerate(toks[len(q):])]
+            assert torch.allclose(lp[3 * i + j], torch.tensor(want), atol=2e-3)
+    assert eng.pool.free_pages == eng.pool.num_pages
