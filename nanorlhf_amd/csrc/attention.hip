@@ -40,12 +40,6 @@
 #include "common.h"
 #include "lds_tiles.h"
 
-// pack two f32 into one dword of 2xbf16 (compiler emits v_cvt_pk_bf16_f32)
-DEVINL unsigned pack2bf(float lo, float hi) {
-  __hip_bfloat162 h2 = __float22bfloat162_rn(float2{lo, hi});
-  return *reinterpret_cast<unsigned*>(&h2);
-}
-
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr int ROWS = 128;    // rows that a workgroup owns, 32 per wave
 

@@ -22,12 +22,12 @@ DEVINL float bf2f(short x) {
   return c.f;
 }
 
-DEVINL short f2bf(float f) {
-  union { float f; unsigned int u; } c;
-  c.f = f;
-  unsigned int lsb = (c.u >> 16) & 1;
-  c.u += 0x7fff + lsb;  // round-to-nearest-even
-  return (short)(c.u >> 16);
+DEVINL short f2bf(float f) { return __builtin_bit_cast(short, (__bf16)f); }
+// two at once; as a vector, or the compiler converts each by itself and joins them
+DEVINL unsigned pack2bf(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 
 // ---- element access shared by kernels templated on bf16 (short) / float ----
@@ -80,15 +80,10 @@ DEVINL void stv(float* p, const float* v) {
 template <int VEC>
 DEVINL void stv(short* p, const float* v) {
   if constexpr (VEC == 8) {
-    s16x8 o;
-#pragma unroll
-    for (int j = 0; j < 8; j++) o[j] = f2bf(v[j]);
-    *reinterpret_cast<s16x8*>(p) = o;
+    *reinterpret_cast<uint4*>(p) = uint4{pack2bf(v[0], v[1]), pack2bf(v[2], v[3]),
+                                         pack2bf(v[4], v[5]), pack2bf(v[6], v[7])};
   } else if constexpr (VEC == 4) {
-    s16x4 o;
-#pragma unroll
-    for (int j = 0; j < 4; j++) o[j] = f2bf(v[j]);
-    *reinterpret_cast<s16x4*>(p) = o;
+    *reinterpret_cast<uint2*>(p) = uint2{pack2bf(v[0], v[1]), pack2bf(v[2], v[3])};
   } else {
 #pragma unroll
     for (int i = 0; i < VEC; i++) p[i] = f2bf(v[i]);

@@ -36,11 +36,6 @@ DEVINL f32x16 mfma32p(bf16x8p a, bf16x8p b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-DEVINL unsigned pack2p(float lo, float hi) {
-  __hip_bfloat162 h2 = __float22bfloat162_rn(float2{lo, hi});
-  return *reinterpret_cast<unsigned*>(&h2);
-}
-
 struct VarlenArgs {
   const short* q;        // [T, Hq, DK], row stride ldq
   const short* kc;       // [P, 16, Hkv, DK]
@@ -232,7 +227,7 @@ void paged_varlen_kernel(VarlenArgs a) {
         const int i = 8 * ks + 2 * j;
         const float x = __builtin_amdgcn_exp2f(fmaf(st[i >> 4][i & 15], mul, -mm));
         const float y = __builtin_amdgcn_exp2f(fmaf(st[i >> 4][(i & 15) + 1], mul, -mm));
-        fr.u[j] = pack2p(x, y);
+        fr.u[j] = pack2bf(x, y);
         // LIN: normed by the sum of the weights as rounded, so that rounding a
         // weight that stands out does not scale the result
         if constexpr (LIN) rs += __uint_as_float(fr.u[j] << 16) + __uint_as_float(fr.u[j] & 0xffff0000u);
