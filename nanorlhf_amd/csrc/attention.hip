@@ -16,14 +16,16 @@
 // has no atomics: dq, dk and dv are summed in registers in a fixed order and
 // written once.
 //
-// What bounds them: 16 MFMAs' worth of LDS reads (16 KB of fragments per 32 x 32
-// scores and two products) keep LDS as busy as the matrix cores, and the
-// exponentials take half as long as the products; two waves per SIMD overlap the
+// What bounds them: the matrix products' own rate under the power limit, the VALU
+// work between them (an exponential, a fused multiply-add, an addition and half a
+// conversion per score, and the fragments' addresses) and LDS reads (16 KB of
+// fragments per 32 x 32 scores and two products); two waves per SIMD overlap the
 // three.  5 causal sequences of about 6500 tokens, 12 heads over 2, width 128:
-// forward 1.1 ms (760 TFLOP/s), dq 1.3 ms, dk and dv 2.2 ms; before, with V
-// transposed by scalar LDS writes, 2.9 ms, and with dq added up by float atomics
-// over 32-row kv tiles, 21.5 ms for the backward.  Twice the rows per wave (half
-// the LDS reads, one wave per SIMD) was slower everywhere: forward 1.6 ms.
+// forward 0.89 ms (950 TFLOP/s), backward 2.75 ms; before, with V transposed by
+// scalar LDS writes, 2.9 ms, and with dq added up by float atomics over 32-row kv
+// tiles, 21.5 ms for the backward.  Twice the rows per wave (half the LDS reads, one
+// wave per SIMD) was slower everywhere, and so were chiplets that take whole heads
+// of one sequence after the other.
 //
 // Products contract over the MFMA's k index in any order as long as both
 // operands agree.  The C layout gives a lane the rows {0-3, 8-11} + 4 * half of
@@ -322,7 +324,7 @@ void fa_bwd_dkv_kernel(const short* __restrict__ dout, const short* __restrict__
   const int hi = lane >> 5;
   const int kw0 = kv0 + wid * 32, ki = kw0 + (lane & 31);
 
-  __shared__ short lds[2][2][TILE * D];   // [buffer][Q, dO]
+  __shared__ __attribute__((aligned(256))) short lds[2][2][TILE * D];   // [buffer][Q, dO]
   __shared__ float rows[2][2][TILE];      // [buffer][lse2, -sum(dO * O)]
 
   bf16x8 kf[NDS], vf[NDS];
@@ -346,6 +348,9 @@ void fa_bwd_dkv_kernel(const short* __restrict__ dout, const short* __restrict__
       load_to_lds4((wid ? drow : lse2) + (long)h * T + pl.s0 + r0, 4 * min(lane, len - r0 - 1),
                    rows[buf][wid]);
   };
+  constexpr unsigned BUFFER = sizeof(lds[0]);     // dO's tile lies TILE rows behind Q's
+  const unsigned base0 = lds_address(&lds[0][0][0]);
+  const unsigned row0 = base0 + row_at<D>(lane), col0 = base0 + col_at<D>(lane);
   stage(h0, qstart, 0);
   int h = h0, r0 = qstart, buf = 0;
   for (; h < h0 + heads; buf ^= 1) {
@@ -353,26 +358,26 @@ void fa_bwd_dkv_kernel(const short* __restrict__ dout, const short* __restrict__
     int hn = h, rn = r0 + TILE;
     if (rn >= len) { hn++; rn = qstart; }
     if (hn < h0 + heads) stage(hn, rn, buf ^ 1);
-    const short* Qt = lds[buf][0];
-    const short* Ot = lds[buf][1];
 #pragma unroll
     for (int sub = 0; sub < 2; sub++) {
       const int q1 = r0 + 32 * sub;
       if (!wave_active || q1 >= len || (CAUSAL && q1 + 31 < kw0)) continue;
       const bool whole = q1 + 32 <= len && (!CAUSAL || kw0 + 31 <= q1);
-      // K, V and the sums fill the registers: addresses are made anew each time
-      // and phases kept apart, or fragments of K and V go to scratch memory
-      int ln = lane;
-      asm volatile("" : "+v"(ln));
+      // K, V and the sums fill the registers: two addresses are kept, the others made
+      // from them each time and phases kept apart, or fragments go to scratch memory
+      unsigned ra = row0 + buf * BUFFER, ca = col0 + buf * BUFFER;
+      asm volatile("" : "+v"(ra), "+v"(ca));
       f32x16_t st{}, dp;
 #pragma unroll
       for (int g = 0; g < 4; g++)
 #pragma unroll
         for (int j = 0; j < 4; j++) dp[4 * g + j] = rows[buf][1][32 * sub + 8 * g + 4 * hi + j];
 #pragma unroll
-      for (int ds = 0; ds < NDS; ds++) st = mfma32x32x16(row_frag<D>(Qt, 32 * sub, ds, ln), kf[ds], st);
+      for (int ds = 0; ds < NDS; ds++)
+        st = mfma32x32x16(row_frag_at<D>(ra, 32 * sub, ds), kf[ds], st);
 #pragma unroll
-      for (int ds = 0; ds < NDS; ds++) dp = mfma32x32x16(row_frag<D>(Ot, 32 * sub, ds, ln), vf[ds], dp);
+      for (int ds = 0; ds < NDS; ds++)
+        dp = mfma32x32x16(row_frag_at<D>(ra, TILE + 32 * sub, ds), vf[ds], dp);
       __builtin_amdgcn_sched_barrier(0);
       float p[16], s[16];
 #pragma unroll
@@ -399,8 +404,9 @@ void fa_bwd_dkv_kernel(const short* __restrict__ dout, const short* __restrict__
         const bf16x8 pf = pack_frag(p + 8 * ks), sf = pack_frag(s + 8 * ks);
 #pragma unroll
         for (int c = 0; c < NDT; c++) {
-          adv[c] = mfma32x32x16(pf, col_frag<D>(Ot, 32 * sub + 16 * ks, 32 * c, ln), adv[c]);
-          adk[c] = mfma32x32x16(sf, col_frag<D>(Qt, 32 * sub + 16 * ks, 32 * c, ln), adk[c]);
+          const int r = 32 * sub + 16 * ks;
+          adv[c] = mfma32x32x16(pf, col_frag_at<D>(ca, TILE + r, 32 * c), adv[c]);
+          adk[c] = mfma32x32x16(sf, col_frag_at<D>(ca, r, 32 * c), adk[c]);
         }
       }
     }

@@ -76,3 +76,36 @@ DEVINL bf16x8 col_frag(const short* tile, int r0, int d0, int lane) {
   }
   return u.f;
 }
+
+// The same fragments from an address that all of a tile share: with `at` = the tile's
+// byte address + row_at<D>(lane) or col_at<D>(lane), another ds (or 32 columns) is an
+// xor of a constant, another 32 (16) rows an offset.  One register instead of one per
+// fragment.
+template <int D>
+DEVINL unsigned row_at(int lane) {
+  const int row = lane & 31;
+  return row * 2 * D + (((lane >> 5) ^ swz<D>(row)) << 4);
+}
+template <int D>
+DEVINL unsigned col_at(int lane) {
+  const int i = lane & 15, col = (lane & 16) + (i & 3) * 4;
+  const int row = 4 * (lane >> 5) + (i >> 2);
+  return row * 2 * D + (((col >> 3) ^ swz<D>(row)) << 4) + (col & 7) * 2;
+}
+template <int D>
+DEVINL bf16x8 row_frag_at(unsigned at, int r0, int ds) {
+  typedef __attribute__((address_space(3))) const char* lds_bytes;
+  typedef __attribute__((address_space(3))) const bf16x8* lds_frag;
+  return *(lds_frag)((lds_bytes)(at ^ ds << 5) + r0 * 2 * D);
+}
+template <int D>
+DEVINL bf16x8 col_frag_at(unsigned at, int r0, int d0) {
+  typedef __attribute__((address_space(3))) char* lds_bytes;
+  typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
+  union { s16x4 h[2]; bf16x8 f; } u;
+#pragma unroll
+  for (int p = 0; p < 2; p++)       // 8 rows on, the swizzle has its second bit changed
+    u.h[p] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_s16x4)((lds_bytes)(at ^ (d0 << 1 | p << 5)) + (r0 + 8 * p) * 2 * D));
+  return u.f;
+}
