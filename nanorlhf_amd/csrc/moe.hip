@@ -10,7 +10,7 @@
 // workgroup finds its group and rows from the counts, so the grid is made for
 // the worst case and surplus workgroups leave at once.
 //   tiles    bf16 MFMA, 128 x 128 tiles through LDS: groups of many rows
-//   stream   bf16 MFMA, 16 or 32 rows, every wave by itself through a ring in LDS:
+//   stream   bf16 MFMA, 16, 32 or 64 rows, every wave by itself through a ring in LDS:
 //            groups of few rows, bound by reading the weights
 //   plain    scalar products in 32-bit, any type and any size
 #include <torch/extension.h>
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(256, 2) void grouped_tiles_kernel(Grouped a, int ti
 // waves share the depth: each walks 64 elements at a time of its own part, which
 // direct loads bring into a ring of its own in LDS, whole 128-byte lines, without
 // barriers, and they add up through LDS.  16 experts of 1536 x 2240, 32 tokens with 4
-// each: gate and up 36 us (6.1 TB/s), down 20.5; 128 tokens 54 and 29.  Fragments
+// each: gate and up 36 us (6.1 TB/s), down 20.5; 128 tokens 50 and 26.  Fragments
 // loaded straight into registers, half a line at a time: 41 and 27, 102 and 52.
 template <int MF, int NF, int WAVES, int R, bool GLU>
 __global__ __launch_bounds__(WAVES * 64) void grouped_stream_kernel(Grouped a) {
@@ -509,12 +509,15 @@ static void launch_grouped(const Grouped& a, bool bf16) {
   if (mfma) {
     const long each = a.lists ? a.rows / a.G : a.rows;      // rows of a group, about
     const long tm = tiles_of(128), tn = (a.N + (GLU ? 63 : 127)) / (GLU ? 64 : 128);
-    if (each > 32 && (each > 512 || tm * tn >= 64)) {
+    // Up to 52 rows the weights are what counts: 160 tokens with 4 of 16 experts of 1536 x
+    // 2240 52 and 27 us in rows of 64, 60 and 33 in tiles; 256 tokens 75 and 38 against
+    // 64 and 40
+    if (each > 52 && (each > 512 || tm * tn >= 64)) {
       TORCH_CHECK(tm * tn < (1L << 31));
       hipLaunchKernelGGL((grouped_tiles_kernel<GLU>), dim3(tm * tn), dim3(256), 0, stream, a,
                          (int)tm, (int)tn);
     } else {
-      const int mf = each > 12 ? 2 : 1;
+      const int mf = each > 28 && each <= 52 ? 4 : each > 12 ? 2 : 1;
       // Four waves with a chunk of their own each.  Where 64 weight rows to a workgroup
       // leave CUs idle, 32 and two chunks: one token's 4 experts of 1536 x 2240 7.7 us
       // against 10.
@@ -525,8 +528,11 @@ static void launch_grouped(const Grouped& a, bool bf16) {
                                                  (NF * (GLU ? 8 : 16))),                       \
                      dim3(256), 0, stream, a)
       if (busy * ((a.N + (GLU ? 31 : 63)) / (GLU ? 32 : 64)) < 256) {
-        if (mf == 2) STREAM(2, 2, 2);
+        if (mf == 4) STREAM(4, 2, 2);
+        else if (mf == 2) STREAM(2, 2, 2);
         else STREAM(1, 2, 2);
+      } else if (mf == 4) {
+        STREAM(4, 4, 1);
       } else if (mf == 2) {
         STREAM(2, 4, 1);
       } else {
