@@ -166,8 +166,8 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
     top = fmaxf(top, __shfl_xor(top, 16));
     top = fmaxf(top, __shfl_xor(top, 32));
     float alpha = 1.f;
-    // rescale only when a row grew by 8 nats (or has no maximum yet)
-    if (__any(!(top - m <= 11.54f))) {
+    // a row's largest weight is 1 exactly, so that it is not rounded
+    if (__any(!(top <= m))) {
       const float mn = fmaxf(m, top);
       alpha = m == -INFINITY ? 0.f : exp2f(m - mn);
       m = mn;
