@@ -3,6 +3,7 @@ is bound by reading the weights; the rest is the library's."""
 from __future__ import annotations
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 import torch.nn.functional as F
 
 from . import serve_ext
@@ -13,10 +14,20 @@ from . import serve_ext
 FEW_ROWS = 64
 
 
+def plain_call(*tensors: torch.Tensor) -> bool:
+    """Whether a library call on these may be replaced by a kernel: no gradient of
+    either kind, no autocast, nobody tracing or transforming the call, no tensor that
+    overrides it."""
+    return not (torch.is_grad_enabled() or torch.is_autocast_enabled()
+                or forward_ad._current_level >= 0 or torch.jit.is_tracing()
+                or torch.compiler.is_compiling()
+                or torch._C._functorch.peek_interpreter_stack() is not None) \
+        and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+
+
 def few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the kernels for few rows take x [M, K] and w [N, K]."""
-    return (x.is_cuda and x.dim() == 2 and x.shape[0] <= FEW_ROWS
-            and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
+    return (x.is_cuda and x.dim() == 2 and x.shape[0] <= FEW_ROWS and plain_call(x, w)
             and x.dtype == w.dtype == torch.bfloat16 and x.shape[1] % 64 == 0
             and x.is_contiguous() and w.is_contiguous() and w.device == x.device
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)

@@ -1,8 +1,7 @@
 """Fused LoRA linear: y = x·Wᵀ + (α/r)·(x·Aᵀ)·Bᵀ + bias in ONE MFMA GEMM.
 
-Replaces the 3-launch F.linear chain (round-1 models/lora.py:60-65;
-reference peft call site GRPO/grpo.py:226-243).  The adapter contribution
-rides as one extra K-tile of the base GEMM (csrc/lora.hip), so the fused
+Replaces the 3-launch F.linear chain (reference peft call site
+GRPO/grpo.py:226-243).  The adapter contribution rides as one extra K-tile of the base GEMM (csrc/lora.hip), so the fused
 kernel does ≈(H+64)/H of the base GEMM's work in a single launch.
 
 Backward (W frozen under LoRA — no dW GEMM at all):
@@ -95,7 +94,8 @@ def _down(z: torch.Tensor, p: torch.Tensor, scale: float, flat: bool) -> torch.T
     on the product's sums."""
     C = z.shape[1]
     if (z.shape[0] <= DOWN_ROWS or z.numel() <= DOWN_SIZE) and C % (64 if flat else 8) == 0 \
-            and z.dtype == p.dtype == torch.bfloat16 and p.shape[0 if flat else 1] == 64:
+            and z.dtype == p.dtype == torch.bfloat16 and p.shape[0 if flat else 1] == 64 \
+            and not torch.is_grad_enabled():       # a backward that is itself recorded
         return ext().lora_down(z.contiguous(), p.contiguous(), scale, flat)
     return torch.addmm(z.new_empty(1), z, p.t() if flat else p, beta=0, alpha=scale)
 
@@ -126,7 +126,8 @@ class _FusedLoRAFn(torch.autograd.Function):
         want_A, want_B = ctx.needs_input_grad[3:5]
         if not (want_A or want_B):
             return dx, None, None, None, None, None, None
-        if dy.shape[1] % 8 == 0 and x.dtype == dy.dtype == torch.bfloat16:
+        if dy.shape[1] % 8 == 0 and x.dtype == dy.dtype == torch.bfloat16 \
+                and not torch.is_grad_enabled():
             dA, dB = ext().lora_grads(
                 *((x.contiguous(), du.contiguous()) if want_A else (None, None)),
                 *((dy, u.contiguous()) if want_B else (None, None)))

@@ -54,7 +54,11 @@ class _AddRMSNormFn(torch.autograd.Function):
         want_dw = ctx.needs_input_grad[2]
         if dh_out is not None:
             dh_out = dh_out.contiguous()
-        dh, dw = ext().rmsnorm_bwd(dy.contiguous(), h, weight, invrms, dh_out, want_dw)
+        recorded = torch.is_grad_enabled() and dh_out is not None    # a second derivative
+        dh, dw = ext().rmsnorm_bwd(dy.contiguous(), h, weight, invrms,
+                                   None if recorded else dh_out, want_dw)
+        if recorded:
+            dh = dh + dh_out
         return dh, dh, dw if want_dw else None, None
 
 

@@ -550,3 +550,16 @@ def test_copies_of_pages(tensors, n):
         p[dst.to(DEV)] = p[src.to(DEV)]
     ops.serve_ext().copy_pages(pools, src.int().to(DEV), dst.int().to(DEV))
     assert all(torch.equal(a, b) for a, b in zip(pools, want))
+
+
+def test_linear_leaves_transformed_calls_to_the_library():
+    import torch.autograd.forward_ad as fwd
+    x, t, w = rnd(4, 64, seed=1), rnd(4, 64, seed=2), rnd(24, 64, seed=3)
+    with torch.no_grad(), fwd.dual_level():
+        y = fwd.unpack_dual(ops.linear(fwd.make_dual(x, t), w))
+        assert torch.equal(y.tangent, torch.nn.functional.linear(t, w))
+    with torch.no_grad():
+        got = torch.func.vmap(lambda a: ops.linear(a, w))(x.view(2, 2, 64))
+    assert rel(got.view(4, 24), x.double() @ w.double().T) < 0.004
+    x.requires_grad_(True)
+    assert ops.linear(x, w).requires_grad
