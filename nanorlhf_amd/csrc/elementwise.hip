@@ -1,7 +1,6 @@
 // RMSNorm fwd/bwd, RoPE apply, SwiGLU fwd/bwd — fused memory-bound kernels
 // for gfx950.  All bf16 I/O with fp32 accumulation, bf16x8 (16 B) vector
-// loads per lane (cdna_hip_programming.md G13), one workgroup per row for
-// the norm reductions.
+// loads per lane; the norms reduce a row in one workgroup or wave.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 

@@ -1,6 +1,6 @@
 // Fused token-logprob + entropy row statistics over the vocab (V ~ 151k),
 // and the matching backward dlogits transform.  fp32 accumulation (bf16
-// logits over 151k need fp32 lse — SURVEY §7 hard part (c)).  Never
+// logits over 151k need fp32 lse).  Never
 // materializes log-softmax (the reference's memory pain point,
 // grpo_trainer.py:548-549,653-656,678-679).
 #include <torch/extension.h>

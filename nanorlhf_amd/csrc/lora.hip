@@ -1,7 +1,7 @@
 // Fused LoRA GEMM for gfx950 — y = x·Wᵀ [+ u·Bᵀ] [+ bias].
 //
 // The LoRA adapter matmul the reference delegates to peft/cuBLAS
-// (GRPO/grpo.py:226-243 call site; SURVEY §2.2 row 3).  MI355X-native
+// (GRPO/grpo.py:226-243 call site).  MI355X-native
 // design: instead of the 3-launch chain  y = F.linear(x,W) +
 // s·F.linear(F.linear(x,A),B), the adapter contribution is folded into the
 // base GEMM as ONE extra K-tile — the kernel consumes a "K-concat" operand
@@ -10,11 +10,11 @@
 // H+64 (≈4 % more FLOPs than the base GEMM, one launch, no y round trip).
 // Backward reuses the SAME kernel: dx = dy·W + du·A is the identical shape
 // with (dy, Wᵀ) and (du = s·dy·B, Aᵀ) as the operand pairs; W is frozen
-// under LoRA so Wᵀ is cached once.  dA/dB are skinny r-rank GEMMs left to
-// hipBLASLt (r/N of the FLOPs).
+// under LoRA so Wᵀ is cached once.  The products with 64 rows or columns of
+// result are lora_grad.hip's.
 //
-// Kernel structure (cdna_hip_programming.md §5 "step-3" ladder structure,
-// ~874 TF at 4096³ bf16): 128×128 output tile, BK=64, 4 waves (2×2 of
+// Large grids take gemm_big.h's 256-tile kernel; this file's own has a
+// 128×128 output tile, BK=64, 4 waves (2×2 of
 // 64×64), v_mfma_f32_16x16x32_bf16, double-buffered LDS filled by
 // global_load_lds dwordx4 (16 B/lane), one __syncthreads per K-step,
 // XCD-aware bijective block swizzle (8 XCDs, each with its own L2).
@@ -50,7 +50,7 @@ __global__ void lora_gemm_kernel(const short* __restrict__ x,
                                  const float* __restrict__ bias,
                                  short* __restrict__ y,
                                  int M, int N, int K1, int grid_n) {
-  // one __shared__ object only (§5 trap 4a): [buf][A/B][128][64]
+  // [buf][A/B][128][64]
   __shared__ short lds[2][2][128 * 64];
 
   // XCD-aware bijective swizzle (8 XCDs round-robin workgroup dispatch)

@@ -6,9 +6,9 @@ attn_implementation="flash_attention_2", GRPO/grpo.py:219,223).  Packed
 pad tokens ever enter the kernel, which is the MI355X-first version of the
 reference's de-padding/bucketing tricks (grpo_r1_trainer.py:571-579).
 
-GPU kernels: MFMA 16x16x32 bf16 QK^T / PV with online softmax, LDS-staged
-K/V tiles (XOR-swizzled, cdna_hip_programming.md §6 G4), fp32 accumulators;
-backward recomputes P from saved (o, lse).  GQA handled by head mapping.
+GPU kernels (csrc/attention.hip): 32x32x16 bf16 products, lane-local online softmax,
+K and V tiles by direct loads into LDS, fp32 accumulators; the backward recomputes P
+from the saved lse in two kernels without atomics.  GQA handled by head mapping.
 """
 from __future__ import annotations
 

@@ -1,11 +1,11 @@
 """Temperature / top-p token sampling.
 
 Replaces vLLM's sampler (SamplingParams(temperature, top_p=0.95, seed=...)
-at GRPO/grpo_trainer.py:127).  One HIP kernel per decode step: per row it
-(1) finds max and exp-sum at temperature, (2) locates the top-p probability
-threshold with an LDS histogram over exp-space (two refinement rounds — no
-full 151k sort), (3) draws inverse-CDF over the kept set with a counter-based
-philox-like hash of (seed, step, row), so replays are deterministic and the
+at GRPO/grpo_trainer.py:127).  One HIP kernel per decode step, a row in the registers
+of one workgroup: it (1) finds max and exp-sum at temperature, (2) locates the top-p
+probability threshold with a histogram over exp-space and its refinements (no
+full 151k sort), (3) draws inverse-CDF over the kept set with a counter hash
+of (seed, step, row), so replays are deterministic and the
 per-update reseed of the reference (random vLLM seed per update,
 grpo_trainer.py:127) is preserved at engine level.
 
