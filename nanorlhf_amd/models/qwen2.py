@@ -249,11 +249,13 @@ class CausalLM(nn.Module):
 
 
 def make_positions(cu_seqlens: torch.Tensor) -> torch.Tensor:
-    """position ids 0..len-1 per packed sequence."""
-    device = cu_seqlens.device
-    lens = (cu_seqlens[1:] - cu_seqlens[:-1]).long()
-    return torch.cat([torch.arange(int(n), device=device) for n in lens]) if len(lens) else \
-        torch.zeros(0, dtype=torch.long, device=device)
+    """position ids 0..len-1 per packed sequence (one wait for the device, for how
+    many there are)."""
+    first = cu_seqlens[:-1].long()
+    T = int(cu_seqlens[-1] - cu_seqlens[0]) if len(first) else 0
+    starts = torch.repeat_interleave(first - cu_seqlens[0].long() if T else first,
+                                     (cu_seqlens[1:] - cu_seqlens[:-1]).long(), output_size=T)
+    return torch.arange(T, device=cu_seqlens.device) - starts
 
 
 def pack_sequences(seqs: list[torch.Tensor], device="cpu"):
