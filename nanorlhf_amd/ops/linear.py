@@ -5,6 +5,7 @@ from __future__ import annotations
 import torch
 import torch.autograd.forward_ad as forward_ad
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from . import serve_ext
 
@@ -14,15 +15,24 @@ from . import serve_ext
 FEW_ROWS = 64
 
 
-def plain_call(*tensors: torch.Tensor) -> bool:
-    """Whether a library call on these may be replaced by a kernel: no gradient of
-    either kind, no autocast, nobody tracing or transforming the call, no tensor that
-    overrides it."""
-    return not (torch.is_grad_enabled() or torch.is_autocast_enabled()
-                or forward_ad._current_level >= 0 or torch.jit.is_tracing()
+def unwatched(*tensors: torch.Tensor) -> bool:
+    """Whether nobody traces, transforms or listens to calls on these: no forward-mode
+    derivative, no trace or transform, no mode of dispatch or of functions (but the one
+    that only gives new tensors their device), no tensor that overrides its calls."""
+    return not (forward_ad._current_level >= 0 or torch.jit.is_tracing()
                 or torch.compiler.is_compiling()
-                or torch._C._functorch.peek_interpreter_stack() is not None) \
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch._C._len_torch_dispatch_stack()
+                or torch._ops._len_torch_dispatch_stack_pre_dispatch()
+                or any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
+                       for i in range(torch._C._len_torch_function_stack()))) \
         and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+
+
+def plain_call(*tensors: torch.Tensor) -> bool:
+    """Whether a library call on these may be replaced by a kernel: no gradient, no
+    autocast, and unwatched."""
+    return not (torch.is_grad_enabled() or torch.is_autocast_enabled()) and unwatched(*tensors)
 
 
 def few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:

@@ -1,0 +1,37 @@
+"""Which calls take a kernel in a library call's place."""
+import torch
+import torch.autograd.forward_ad as fwd
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.overrides import TorchFunctionMode
+from torch.utils.flop_counter import FlopCounterMode
+
+from nanorlhf_amd.ops.linear import plain_call
+
+
+def test_plain_calls_are_those_that_nobody_sees():
+    x, seen = torch.randn(2, 2), []
+
+    class Listens(TorchFunctionMode):
+        def __torch_function__(self, fn, types, args=(), kwargs=None):
+            return fn(*args, **(kwargs or {}))
+
+    def call(a):
+        seen.append(plain_call(a))
+        return a + 1
+
+    assert not plain_call(x)                        # gradients are on
+    with torch.no_grad():
+        for pre_dispatch in (False, True):
+            make_fx(call, pre_dispatch=pre_dispatch)(x)
+        torch.jit.trace(call, x, check_trace=False)
+        torch.func.vmap(call)(x)
+        for mode in (FlopCounterMode(display=False), Listens()):
+            with mode:
+                call(x)
+        with fwd.dual_level():
+            call(x)
+        assert seen and not any(seen)
+        assert not plain_call(x.as_subclass(type("Sub", (torch.Tensor,), {})))
+        assert plain_call(x, torch.nn.Parameter(x))
+        with torch.device("cpu"):                   # only says where new tensors go
+            assert plain_call(x)
