@@ -19,6 +19,7 @@ from __future__ import annotations
 import torch
 
 from . import serve_ext
+from .linear import unwatched
 from .rope import qkv_rope, rotate_pairs
 
 
@@ -48,7 +49,7 @@ def qkv_rope_append(qkv: torch.Tensor, table: torch.Tensor, positions: torch.Ten
                     want_kv: bool = True):
     """qkv_rope, and kv_append of its k and v.  Returns (q, k, v), k and v None
     unless wanted."""
-    if qkv.is_cuda and not (torch.is_grad_enabled() and qkv.requires_grad):
+    if qkv.is_cuda and not (torch.is_grad_enabled() and qkv.requires_grad) and unwatched(qkv):
         out = serve_ext().qkv_rope_append(qkv.contiguous(), table, positions, slots, k_cache,
                                           v_cache, heads, want_kv)
         return tuple(out) if want_kv else (out[0], None, None)

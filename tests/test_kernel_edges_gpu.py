@@ -301,6 +301,18 @@ def test_qkv_rope_append_fills_the_cache_as_kv_append_does(dtype, hq, hkv, d):
 
 
 # ------------------------------------------------------- norm, optimizer
+def test_qkv_rope_append_drops_no_tangent():
+    import torch.autograd.forward_ad as fwd
+    T, table = 5, ops.build_rope_cache(64, 16, device=DEV)
+    qkv, pos = rnd(T, 4 * 64, seed=1), torch.arange(T, device=DEV)
+    kc = torch.zeros(1, 16, 1, 64, device=DEV, dtype=torch.bfloat16)
+    vc = torch.zeros(1, 1, 64, 16, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad(), fwd.dual_level():
+        dual = fwd.make_dual(qkv, rnd(T, 4 * 64, seed=2))
+        with pytest.raises(RuntimeError):        # a rotation has no forward derivative
+            ops.qkv_rope_append(dual, table, pos, 2, pos, kc, vc)
+
+
 @pytest.mark.parametrize("N,H", [(1, 8), (3, 512), (5, 520), (1027, 1536), (7, 2048), (6, 2056),
                                  (4000, 896), (33, 4096), (9, 8192)])
 @pytest.mark.parametrize("frozen", [True, False])
