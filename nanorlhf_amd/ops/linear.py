@@ -35,9 +35,15 @@ def plain_call(*tensors: torch.Tensor) -> bool:
     return not (torch.is_grad_enabled() or torch.is_autocast_enabled()) and unwatched(*tensors)
 
 
+def here(x: torch.Tensor) -> bool:
+    """Whether x is on the current GPU, on whose stream the kernels are launched; a
+    library call goes to its operands' GPU, whichever is the current."""
+    return x.is_cuda and x.device.index == torch.cuda.current_device()
+
+
 def few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the kernels for few rows take x [M, K] and w [N, K]."""
-    return (x.is_cuda and x.dim() == 2 and x.shape[0] <= FEW_ROWS and plain_call(x, w)
+    return (here(x) and x.dim() == 2 and x.shape[0] <= FEW_ROWS and plain_call(x, w)
             and x.dtype == w.dtype == torch.bfloat16 and x.shape[1] % 64 == 0
             and x.is_contiguous() and w.is_contiguous() and w.device == x.device
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
@@ -45,6 +51,8 @@ def few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """x w^T + bias."""
-    if few_rows(x, w) and (bias is None or bias.dtype == x.dtype and bias.is_contiguous()):
+    if few_rows(x, w) and (bias is None or plain_call(bias) and bias.dtype == x.dtype
+                           and bias.device == x.device and bias.shape == w.shape[:1]
+                           and bias.is_contiguous()):
         return serve_ext().linear_rows(x, w, bias)
     return F.linear(x, w, bias)

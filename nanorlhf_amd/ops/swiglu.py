@@ -6,7 +6,7 @@ from __future__ import annotations
 import torch
 
 from . import ext, serve_ext
-from .linear import few_rows, plain_call
+from .linear import few_rows, here, plain_call
 
 
 def _swiglu_ref(gate_up: torch.Tensor) -> torch.Tensor:
@@ -42,8 +42,9 @@ GLU_ROWS, GLU_DEPTH = 512, 2048
 
 def glu_fuses(x: torch.Tensor, gate: torch.Tensor) -> bool:
     """Whether glu_linear takes (and is the faster way for) these operands."""
-    return (x.is_cuda and plain_call(x, gate) and x.dim() == 2
-            and x.dtype == gate.dtype == torch.bfloat16 and x.is_contiguous() and gate.is_contiguous() and gate.device == x.device
+    return (here(x) and plain_call(x, gate) and x.dim() == 2
+            and x.dtype == gate.dtype == torch.bfloat16 and x.is_contiguous()
+            and gate.is_contiguous() and gate.device == x.device
             and x.shape[0] >= GLU_ROWS and x.shape[1] % 64 == 0 and x.shape[1] <= GLU_DEPTH
             and x.data_ptr() % 16 == 0 and gate.data_ptr() % 16 == 0)
 

@@ -575,3 +575,20 @@ def test_linear_leaves_transformed_calls_to_the_library():
     assert rel(got.view(4, 24), x.double() @ w.double().T) < 0.004
     x.requires_grad_(True)
     assert ops.linear(x, w).requires_grad
+
+
+def test_linears_of_another_gpu_are_the_library_s(monkeypatch):
+    from nanorlhf_amd.ops.linear import few_rows
+    x, w, big = rnd(4, 64, seed=1), rnd(24, 64, seed=2), rnd(4096, 64, seed=3)
+    with torch.no_grad():
+        assert few_rows(x, w) and ops.glu_fuses(big, big)
+        monkeypatch.setattr(torch.cuda, "current_device", lambda: x.device.index + 1)
+        assert not few_rows(x, w) and not ops.glu_fuses(big, big)
+
+
+def test_linear_leaves_other_biases_to_the_library():
+    x, w, one = rnd(4, 64, seed=1), rnd(24, 64, seed=2), rnd(1, seed=3)
+    with torch.no_grad():
+        assert rel(ops.linear(x, w, one), x.double() @ w.double().T + one.double()) < 0.004
+        with pytest.raises(RuntimeError, match="same device"):
+            ops.linear(x, w, torch.zeros(24, dtype=torch.bfloat16))
