@@ -21,6 +21,7 @@
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
+#include "checks.h"
 #include "common.h"
 #include "gemm_big.h"
 
@@ -168,6 +169,12 @@ torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
                 "adapter rank must be 64 for the fused kernel");
     TORCH_CHECK(b->size(0) == N && b->size(1) == 64);
     TORCH_CHECK(u->dtype() == torch::kBFloat16 && b->dtype() == torch::kBFloat16);
+  }
+  x = on16(x);
+  w = on16(w);
+  if (has_lora) {
+    u = on16(*u);
+    b = on16(*b);
   }
   torch::Tensor bias_f;
   const bool has_bias = bias.has_value();
@@ -323,6 +330,8 @@ void lora_add_(torch::Tensor y, torch::Tensor u, torch::Tensor b) {
   const long M = y.size(0), N = y.size(1);
   TORCH_CHECK(u.size(0) == M && u.size(1) == 64);
   TORCH_CHECK(b.size(0) == N && b.size(1) == 64);
+  u = on16(u);
+  b = on16(b);
   const int grid_m = (int)((M + 127) / 128), grid_n = (int)((N + 127) / 128);
   auto stream = at::hip::getCurrentHIPStream();
   const bool vec = N % 8 == 0 && (uintptr_t)y.data_ptr() % 16 == 0;

@@ -125,26 +125,28 @@ std::vector<torch::Tensor> lora_grads(c10::optional<torch::Tensor> x,
   GradJob jobs[2] = {};
   long blocks = 0, sums = 0;
   for (int k = 0; k < 2; k++) {
-    const auto& z = k ? dy : x;
-    const auto& v = k ? u : du;
+    const auto& given = k ? dy : x;
+    const auto& factor = k ? u : du;
     GradJob& j = jobs[k];
     j.splits = 1;
-    if (!z) {
+    if (!given) {
       outs.push_back(torch::empty({0}, options));
       continue;
     }
-    TORCH_CHECK(v.has_value(), "lora_grads: both factors");
-    const long C = z->size(1);
-    for (const auto& t : {*z, *v})
+    TORCH_CHECK(factor.has_value(), "lora_grads: both factors");
+    const long C = given->size(1);
+    for (const auto& t : {*given, *factor})
       TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.scalar_type() == torch::kBFloat16 &&
-                  t.size(0) == M && (uintptr_t)t.data_ptr() % 16 == 0,
-                  "lora_grads: contiguous bf16 matrices");
-    TORCH_CHECK(v->size(1) == RANK && C % 8 == 0 && C > 0 && C < (1L << 24),
+                  t.size(0) == M, "lora_grads: contiguous bf16 matrices");
+    TORCH_CHECK(factor->size(1) == RANK && C % 8 == 0 && C > 0 && C < (1L << 24),
                 "lora_grads: rank 64, columns a multiple of 8");
+    const auto z = on16(*given), v = on16(*factor);
+    keep.push_back(z);
+    keep.push_back(v);
     j.flat = k == 0;
     outs.push_back(torch::empty({j.flat ? RANK : C, j.flat ? C : RANK}, options));
-    j.z = (const short*)z->data_ptr();
-    j.v = (const short*)v->data_ptr();
+    j.z = (const short*)z.data_ptr();
+    j.v = (const short*)v.data_ptr();
     j.out = (short*)outs.back().data_ptr();
     j.C = C;
     j.tiles = (C + COLS - 1) / COLS;
@@ -261,14 +263,16 @@ void lora_down_sum_kernel(const float* __restrict__ parts, short* __restrict__ o
 torch::Tensor lora_down(torch::Tensor z, torch::Tensor p, double scale, bool flat) {
   on_gpu({z, p});
   for (const auto& t : {z, p})
-    TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.scalar_type() == torch::kBFloat16 &&
-                (uintptr_t)t.data_ptr() % 16 == 0, "lora_down: contiguous bf16 matrices");
+    TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.scalar_type() == torch::kBFloat16,
+                "lora_down: contiguous bf16 matrices");
   const long M = z.size(0), C = z.size(1);
   TORCH_CHECK(p.size(flat ? 0 : 1) == RANK && p.size(flat ? 1 : 0) == C, "lora_down: rank 64");
   TORCH_CHECK(C > 0 && C % (flat ? TILE : 8) == 0 && C < (1L << 24) && M < (1L << 31) - TILE,
               "lora_down: columns a multiple of ", flat ? TILE : 8);
   auto out = torch::empty({M, RANK}, z.options());
   if (M == 0) return out;
+  z = on16(z);
+  p = on16(p);
   const long tiles = (M + TILE - 1) / TILE, steps = (C + TILE - 1) / TILE;
   const int splits = (int)std::max(1L, std::min({384 / tiles, steps / 3, 16L}));
   torch::Tensor parts;

@@ -550,6 +550,29 @@ def test_product_down_to_the_rank(M, C):
         assert rel(got, want) < 0.002              # one rounding, 2^-9 at most
 
 
+@pytest.mark.parametrize("M,K,N", [(65, 128, 192), (3000, 2048, 2048)])    # small tiles, big
+@pytest.mark.parametrize("strategy", ["fused", "epilogue"])
+def test_adapter_operands_off_16_bytes(M, K, N, strategy, monkeypatch):
+    from nanorlhf_amd.ops import lora
+    monkeypatch.setattr(lora, "_choose_strategy", lambda *a: strategy)
+
+    def off(t):      # the same values, 2 bytes past a multiple of 16
+        return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+
+    x, w, dy = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=K ** -0.5), rnd(M, N, seed=3)
+    A, B = rnd(64, K, seed=4, scale=K ** -0.5), rnd(N, 64, seed=5, scale=0.1)
+    w_t = w.t().contiguous()
+    both = []
+    for move in (lambda t: t.clone(), off):
+        leaves = [move(t).requires_grad_(True) for t in (x, A, B)]
+        y = lora.fused_lora_linear(leaves[0], w, None, *leaves[1:], 0.25, w_t)
+        y.backward(move(dy))
+        both.append([y] + [t.grad for t in leaves])
+    # the library may choose by alignment: its sums' order, and so a rounding of each step
+    for a, b in zip(*both):
+        assert torch.equal(a, b) if strategy == "fused" else rel(a, b) < 0.004
+
+
 @pytest.mark.parametrize("tensors,n", [(1, 1), (2, 7), (64, 3), (67, 5)])
 def test_copies_of_pages(tensors, n):
     g = torch.Generator().manual_seed(tensors)
