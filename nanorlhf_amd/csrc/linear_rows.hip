@@ -179,9 +179,10 @@ static void check_rows(const torch::Tensor& x, const torch::Tensor& w) {
   for (const auto& t : {x, w})
     TORCH_CHECK(t.dim() == 2 && t.is_contiguous() && t.scalar_type() == torch::kBFloat16 &&
                 (uintptr_t)t.data_ptr() % 16 == 0, "linear_rows: contiguous bf16 matrices");
+  // a workgroup's offsets, of up to 128 rows, are 32-bit bytes
   TORCH_CHECK(x.size(0) <= 64 && x.size(1) == w.size(1) && x.size(1) % 64 == 0 &&
-              x.size(1) < (1L << 30) && w.size(0) < (1L << 30),
-              "linear_rows: at most 64 rows, depth a multiple of 64");
+              x.size(1) < (1L << 24) && w.size(0) < (1L << 30),
+              "linear_rows: at most 64 rows, depth a multiple of 64 below 2^24");
 }
 
 template <int NF, int WAVES, int R, bool GLU>

@@ -13,6 +13,7 @@ from . import serve_ext
 # 18.7 / 15.3, of 37888 x 3584 70 / 57, of 151936 x 1536 115 / 108; with more rows x
 # weighs as much as the weights and the library's tiles share it better.
 FEW_ROWS = 64
+DEPTH = 1 << 24         # from which on its 32-bit offsets would wrap
 
 
 def unwatched(*tensors: torch.Tensor) -> bool:
@@ -45,8 +46,8 @@ def few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the kernels for few rows take x [M, K] and w [N, K]."""
     return (here(x) and x.dim() == 2 and x.shape[0] <= FEW_ROWS and plain_call(x, w)
             and x.dtype == w.dtype == torch.bfloat16 and x.shape[1] % 64 == 0
-            and x.is_contiguous() and w.is_contiguous() and w.device == x.device
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+            and x.shape[1] < DEPTH and x.is_contiguous() and w.is_contiguous()
+            and w.device == x.device and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:

@@ -615,3 +615,14 @@ def test_linear_leaves_other_biases_to_the_library():
         assert rel(ops.linear(x, w, one), x.double() @ w.double().T + one.double()) < 0.004
         with pytest.raises(RuntimeError, match="same device"):
             ops.linear(x, w, torch.zeros(24, dtype=torch.bfloat16))
+
+
+def test_linear_of_few_rows_and_great_depth():
+    from nanorlhf_amd.ops.linear import few_rows
+    deep = 1 << 24
+    x, w = rnd(2, deep, seed=1), rnd(130, 64, seed=2).repeat(1, 4)
+    with torch.no_grad():
+        assert few_rows(x[:, :256].contiguous(), w) and not few_rows(x, x)
+        assert ops.linear(x, x).shape == (2, 2)
+    with pytest.raises(RuntimeError, match="2\\^24"):
+        ops.serve_ext().linear_rows(x, x, None)
