@@ -150,6 +150,13 @@ __global__ void lora_gemm_kernel(const short* __restrict__ x,
   }
 }
 
+// Whether lora_gemm takes the 256-tile kernel.  4096 x 1536 x 1536 (96 tiles of 256): 38 us
+// in big tiles, 42 in small ones; with fewer the small ones fill more of the chip.
+// From a depth of 2^22 on a big tile's 32-bit offsets come near their end.
+bool lora_gemm_big(long M, long N, long K) {
+  return ((M + BIG - 1) / BIG) * ((N + BIG - 1) / BIG) >= 96 && K < (1L << 22);
+}
+
 torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
                         c10::optional<torch::Tensor> u,
                         c10::optional<torch::Tensor> b,
@@ -190,10 +197,8 @@ torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
   const short* bp = has_lora ? (const short*)b->data_ptr() : nullptr;
   const float* biasp = has_bias ? bias_f.data_ptr<float>() : nullptr;
 
-  // 4096 x 1536 x 1536 (96 tiles of 256): 38 us in big tiles, 42 in small ones;
-  // with fewer the small ones fill more of the chip
   const int big_m = (int)((M + BIG - 1) / BIG), big_n = (int)((N + BIG - 1) / BIG);
-  if ((long)big_m * big_n >= 96) {
+  if (lora_gemm_big(M, N, K1)) {
 #define LAUNCH(HL, HB, VEC)                                                               \
   hipLaunchKernelGGL((gemm_big_kernel<HL, HB, VEC, 0>), dim3(big_m * big_n), dim3(512), 0, \
                      stream, (const short*)x.data_ptr(), (const short*)w.data_ptr(), up, bp, \

@@ -1,10 +1,12 @@
 """Which calls take a kernel in a library call's place."""
+import pytest
 import torch
 import torch.autograd.forward_ad as fwd
 from torch.fx.experimental.proxy_tensor import make_fx
 from torch.overrides import TorchFunctionMode
 from torch.utils.flop_counter import FlopCounterMode
 
+from nanorlhf_amd import ops
 from nanorlhf_amd.ops.linear import plain_call
 
 
@@ -35,3 +37,11 @@ def test_plain_calls_are_those_that_nobody_sees():
         assert plain_call(x, torch.nn.Parameter(x))
         with torch.device("cpu"):                   # only says where new tensors go
             assert plain_call(x)
+
+
+def test_big_tiles_of_the_adapter_product_stop_where_offsets_end():
+    if not ops.ext_available():
+        pytest.skip("extensions are not built")
+    big = ops.ext().lora_gemm_big
+    assert big(4096, 1536, 1536) and not big(4096, 1280, 1536)
+    assert big(24576, 256, (1 << 22) - 64) and not big(24576, 256, 1 << 22)
