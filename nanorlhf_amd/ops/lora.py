@@ -1,8 +1,9 @@
 """Fused LoRA linear: y = x·Wᵀ + (α/r)·(x·Aᵀ)·Bᵀ + bias in ONE MFMA GEMM.
 
 Replaces the 3-launch F.linear chain (reference peft call site
-GRPO/grpo.py:226-243).  The adapter contribution rides as one extra K-tile of the base GEMM (csrc/lora.hip), so the fused
-kernel does ≈(H+64)/H of the base GEMM's work in a single launch.
+GRPO/grpo.py:226-243).  The adapter contribution rides as one extra K-tile of the
+base GEMM (csrc/lora.hip), so the fused kernel does ≈(H+64)/H of the base GEMM's work
+in a single launch.
 
 Backward (W frozen under LoRA — no dW GEMM at all):
     du = s·(dy·B)            [M,r]   (_down)
@@ -33,15 +34,18 @@ def lora_gemm_ref(x, w, u=None, b=None, bias=None):
     return y.to(x.dtype)
 
 
-# Per-shape strategy cache: (N, K) -> "fused" | "epilogue".
+# Strategy cache: weight shape (N, K) -> {(whether lora_gemm takes its big tiles, whether
+# there is a bias, device): "fused" | "epilogue"}.
 # "fused"    = the single wide-K MFMA kernel (wins when our GEMM rate is
 #              within the fusion savings of hipBLASLt — e.g. N-heavy shapes);
 # "epilogue" = hipBLASLt base GEMM + the custom rank-64 lora_add_ MFMA pass
 #              (wins on deep-K shapes where the library GEMM is far ahead).
 # The fused kernel rounds y once, the epilogue twice, so the epilogue has to be
 # clearly faster.
-# Measured once per weight shape on first touch (events, ~1 ms).
-_TUNE: dict[tuple, str] = {}
+# Measured once per key on first touch (events, ~1 ms): a few rows say nothing about
+# many, for which lora_gemm is another kernel, nor a square weight's dx, which has no
+# bias, about its y.
+_TUNE: dict[tuple, dict] = {}
 
 
 def _time_cuda(fn, reps: int = 3) -> float:
@@ -56,8 +60,10 @@ def _time_cuda(fn, reps: int = 3) -> float:
 
 
 def _choose_strategy(x, w, u, b, bias) -> str:
-    key = (int(w.size(0)), int(w.size(1)))
-    st = _TUNE.get(key)
+    N, K = int(w.size(0)), int(w.size(1))
+    known = _TUNE.setdefault((N, K), {})
+    key = (ext().lora_gemm_big(x.shape[0], N, K), bias is not None, x.device)
+    st = known.get(key)
     if st is None:
         t_fused = _time_cuda(lambda: ext().lora_gemm(x, w, u, b, bias))
 
@@ -66,7 +72,7 @@ def _choose_strategy(x, w, u, b, bias) -> str:
             ext().lora_add_(y, u, b)
         t_ep = _time_cuda(ep)
         st = "fused" if t_fused <= 1.1 * t_ep else "epilogue"
-        _TUNE[key] = st
+        known[key] = st
     return st
 
 

@@ -45,3 +45,21 @@ def test_big_tiles_of_the_adapter_product_stop_where_offsets_end():
     big = ops.ext().lora_gemm_big
     assert big(4096, 1536, 1536) and not big(4096, 1280, 1536)
     assert big(24576, 256, (1 << 22) - 64) and not big(24576, 256, 1 << 22)
+
+
+def test_adapter_strategies_are_kept_by_what_the_kernels_depend_on(monkeypatch):
+    from types import SimpleNamespace
+    from nanorlhf_amd.ops import lora
+    monkeypatch.setattr(lora, "_TUNE", {})
+    monkeypatch.setattr(lora, "ext", lambda: SimpleNamespace(
+        lora_gemm_big=lambda M, N, K: M > 1000, lora_gemm=None, lora_add_=None))
+    times = iter([1.0, 3.0, 3.0, 1.0, 1.0, 3.0])            # fused, epilogue of each new key
+    monkeypatch.setattr(lora, "_time_cuda", lambda fn: next(times))
+    w, bias = torch.zeros(64, 64), torch.zeros(64)
+
+    def choose(rows, b=None):
+        return lora._choose_strategy(torch.zeros(rows, 64), w, None, None, b)
+
+    assert [choose(240), choose(4000), choose(240, bias)] == ["fused", "epilogue", "fused"]
+    assert [choose(17), choose(9000), choose(60, bias)] == ["fused", "epilogue", "fused"]
+    assert next(times, None) is None and len(lora._TUNE[64, 64]) == 3
