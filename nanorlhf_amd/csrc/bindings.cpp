@@ -63,6 +63,13 @@ std::vector<torch::Tensor> lora_grads(c10::optional<torch::Tensor> x,
                                       c10::optional<torch::Tensor> u);
 torch::Tensor lora_down(torch::Tensor z, torch::Tensor p, double scale, bool flat);
 
+// glu.hip
+void glu_linear(torch::Tensor x, torch::Tensor gate, torch::Tensor up, torch::Tensor out,
+                long act);
+// linear_rows.hip
+torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias);
+torch::Tensor glu_rows(torch::Tensor x, torch::Tensor gate, torch::Tensor up);
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm_fwd", &rmsnorm_fwd);
   m.def("rmsnorm_bwd", &rmsnorm_bwd, py::arg("dy"), py::arg("x"), py::arg("w"),
@@ -75,6 +82,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("swiglu_bwd", &swiglu_bwd);
   m.def("ce_rowstats", &ce_rowstats);
   m.def("ce_backward_dlogits", &ce_backward_dlogits);
+  m.def("glu_linear", &glu_linear);
+  m.def("linear_rows", &linear_rows);
+  m.def("glu_rows", &glu_rows);
   m.def("lora_grads", &lora_grads);
   m.def("lora_down", &lora_down);
   m.def("adamw_step", &adamw_step);

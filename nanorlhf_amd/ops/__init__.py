@@ -4,9 +4,9 @@ Every hot op has two paths:
   * GPU (``tensor.is_cuda``): the hand-written gfx950 HIP kernel from the
     in-tree extensions ``nanorlhf_amd/_C.so`` (training, scoring, sampling)
     and ``nanorlhf_amd/_serve.so`` (paged cache, attention over it, linear
-    attention, residual-stream kernels).  If an extension is missing on a
-    machine with a GPU this raises loudly — there is NO silent eager
-    fallback on GPU.
+    attention, residual-stream kernels); the linears without gradients are
+    in both.  If an extension is missing on a machine with a GPU this raises
+    loudly — there is NO silent eager fallback on GPU.
   * CPU: a plain-PyTorch fp32 reference used by the CPU test suite and as
     the numerics oracle for the kernels.
 """
@@ -47,6 +47,12 @@ def ext():
 def serve_ext():
     """The serving extension; raises loudly if unavailable."""
     return _require("_serve")
+
+
+def linear_ext():
+    """The linears without gradients, which scoring and serving both run: either
+    extension has them; raises loudly if neither is available."""
+    return _require("_serve" if _load("_serve")[0] is not None else "_C")
 
 
 def ext_available() -> bool:

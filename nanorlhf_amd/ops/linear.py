@@ -7,7 +7,7 @@ import torch.autograd.forward_ad as forward_ad
 import torch.nn.functional as F
 from torch.utils._device import DeviceContext
 
-from . import serve_ext
+from . import linear_ext
 
 # Library against the kernel, in us: 64 rows of 3584 x 18944 91 / 36, of 4608 x 3584
 # 18.7 / 15.3, of 37888 x 3584 70 / 57, of 151936 x 1536 115 / 108; with more rows x
@@ -55,5 +55,5 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -
     if few_rows(x, w) and (bias is None or plain_call(bias) and bias.dtype == x.dtype
                            and bias.device == x.device and bias.shape == w.shape[:1]
                            and bias.is_contiguous()):
-        return serve_ext().linear_rows(x, w, bias)
+        return linear_ext().linear_rows(x, w, bias)
     return F.linear(x, w, bias)

@@ -5,7 +5,7 @@ from __future__ import annotations
 
 import torch
 
-from . import ext, serve_ext
+from . import ext, linear_ext, serve_ext
 from .linear import few_rows, here, plain_call
 
 
@@ -53,11 +53,11 @@ def linear_swiglu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """swiglu of x [..., K] times weight [2 I, K] (gate rows, then up rows)."""
     gate, up = weight.chunk(2)
     if few_rows(x, gate):
-        return serve_ext().glu_rows(x, gate, up)
+        return linear_ext().glu_rows(x, gate, up)
     if not glu_fuses(x, gate):
         return swiglu(torch.nn.functional.linear(x, weight))
     out = torch.empty(x.shape[0], gate.shape[0], dtype=x.dtype, device=x.device)
-    serve_ext().glu_linear(x, gate, up, out, 0)
+    linear_ext().glu_linear(x, gate, up, out, 0)
     return out
 
 
@@ -73,7 +73,7 @@ def linear_gelu_glu(x: torch.Tensor, gate: torch.Tensor, up: torch.Tensor,
                     out: torch.Tensor) -> None:
     """out = gelu_tanh(x gate^T) * (x up^T), where glu_fuses(x, gate); out may be
     columns of a wider row."""
-    serve_ext().glu_linear(x, gate, up, out, 1)
+    linear_ext().glu_linear(x, gate, up, out, 1)
 
 
 def gelu_glu(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor,

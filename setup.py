@@ -19,13 +19,14 @@ from torch.utils.cpp_extension import BuildExtension, CUDAExtension  # noqa: E40
 ROOT = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(ROOT, "nanorlhf_amd", "csrc")
 
+LINEAR = ["glu.hip", "linear_rows.hip"]     # both have them, so that each serves alone
 EXTENSIONS = {
     "_C": ["bindings.cpp", "elementwise.hip", "logprob.hip", "adamw.hip",
            "sampling.hip", "attention.hip", "masked.hip", "lora.hip",
-           "lora_grad.hip"],
+           "lora_grad.hip", *LINEAR],
     "_serve": ["serve_bindings.cpp", "kvcache.hip", "paged_attention.hip",
                "linear_attn.hip", "stream.hip", "wkv.hip", "latent_attn.hip", "moe.hip",
-               "glu.hip", "linear_rows.hip"],
+               *LINEAR],
 }
 
 wanted = [n for n in os.environ.get("NANORLHF_EXT", "").split(",") if n] or list(EXTENSIONS)

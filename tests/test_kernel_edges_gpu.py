@@ -626,3 +626,28 @@ def test_linear_of_few_rows_and_great_depth():
         assert ops.linear(x, x).shape == (2, 2)
     with pytest.raises(RuntimeError, match="2\\^24"):
         ops.serve_ext().linear_rows(x, x, None)
+
+
+@pytest.mark.parametrize("absent", ["_serve", "_C"])
+def test_linears_need_one_extension(absent, monkeypatch):
+    monkeypatch.setitem(ops._LOADED, absent, (None, ImportError("not built")))
+    w, wide = rnd(48, 64, seed=1), rnd(400, 64, seed=2)
+    with torch.no_grad():
+        for rows in (4, 600):
+            x = rnd(rows, 64, seed=rows)
+            assert rel(ops.linear(x, w), x.double() @ w.double().T) < 0.004
+            g, u = (x.double() @ wide.double().T).split(200, 1)
+            assert rel(ops.linear_swiglu(x, wide), torch.nn.functional.silu(g) * u) < 0.004
+
+
+def test_scoring_needs_the_training_extension_alone(monkeypatch):
+    from nanorlhf_amd.models import CausalLM, get_config, pack_sequences
+    model = CausalLM(get_config("tiny")).to(DEV, torch.bfloat16).eval()
+    seqs = [torch.arange(3, 40), torch.arange(5, 600)]
+    ids, cu, longest, pos = pack_sequences(seqs, device=DEV)
+    monkeypatch.setitem(ops._LOADED, "_serve", (None, ImportError("not built")))
+    with torch.no_grad():
+        hidden = model(ids, CausalLM.train_ctx(cu, longest, pos))
+        lp, _ = ops.token_logprob_entropy(hidden[:-1], model.lm_head_weight, ids[1:])
+        few = model.logits(hidden[:60])
+    assert torch.isfinite(lp).all() and torch.isfinite(few).all()
