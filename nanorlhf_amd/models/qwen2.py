@@ -249,10 +249,13 @@ class CausalLM(nn.Module):
 
 
 def make_positions(cu_seqlens: torch.Tensor) -> torch.Tensor:
-    """position ids 0..len-1 per packed sequence (one wait for the device, for how
-    many there are)."""
+    """position ids 0..len-1 per packed sequence (one wait for the device, for the
+    boundaries: repeat_interleave would write past its output where they fall)."""
+    bounds = cu_seqlens.tolist()
+    if any(b < a for a, b in zip(bounds, bounds[1:])):
+        raise RuntimeError(f"sequence boundaries must not fall: {bounds}")
     first = cu_seqlens[:-1].long()
-    T = int(cu_seqlens[-1] - cu_seqlens[0]) if len(first) else 0
+    T = bounds[-1] - bounds[0] if len(bounds) > 1 else 0
     starts = torch.repeat_interleave(first - cu_seqlens[0].long() if T else first,
                                      (cu_seqlens[1:] - cu_seqlens[:-1]).long(), output_size=T)
     return torch.arange(T, device=cu_seqlens.device) - starts

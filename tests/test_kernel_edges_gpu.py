@@ -651,3 +651,12 @@ def test_scoring_needs_the_training_extension_alone(monkeypatch):
         lp, _ = ops.token_logprob_entropy(hidden[:-1], model.lm_head_weight, ids[1:])
         few = model.logits(hidden[:60])
     assert torch.isfinite(lp).all() and torch.isfinite(few).all()
+
+
+def test_positions_of_packed_sequences():
+    from nanorlhf_amd.models.qwen2 import make_positions
+    for cu in ([0, 3, 3, 8], [5, 6, 9], [0], [4, 4], []):
+        want = [i for a, b in zip(cu, cu[1:]) for i in range(b - a)]
+        assert make_positions(torch.tensor(cu, dtype=torch.int32, device=DEV)).tolist() == want
+    with pytest.raises(RuntimeError, match="fall"):
+        make_positions(torch.tensor([0, 20, 5, 6], dtype=torch.int32, device=DEV))
