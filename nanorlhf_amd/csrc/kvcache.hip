@@ -293,7 +293,10 @@ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
   const int G = EXT ? min(16, Gq - 16 * gc) : Gq;   // heads of this workgroup
   const int L = seq_lens[b];
   const TileRange tr = tile_range<EXT>(L, ext);
-  const int it0 = blockIdx.y * per_split, it1 = min(tr.n, it0 + per_split);
+  // a length past its page table (whose last page is then read again) may have more
+  // tiles than the splits were made for: the last takes them
+  const int it0 = blockIdx.y * per_split;
+  const int it1 = blockIdx.y + 1 == gridDim.y ? tr.n : min(tr.n, it0 + per_split);
   if (blockIdx.y > 0 && it0 >= tr.n) return;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -451,7 +454,7 @@ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
       o0 += Lacc[w][g * LD + d] * c;
       o1 += Lacc[w][g * LD + d + 1] * c;
     }
-    if (tr.n <= per_split) {      // nothing to merge
+    if (gridDim.y == 1 || tr.n <= per_split) {      // nothing to merge
       const float inv = S > 0.f ? 1.f / S : 0.f;
       write_pair<EXT>(out, o0 * inv, o1 * inv, b, h0 + g, d, Hq, DV, ext);
     } else {
@@ -472,7 +475,7 @@ void paged_decode_merge_kernel(const float* __restrict__ part, const float* __re
   const int unit = EXT ? x / ext.gchunks : x, gc = EXT ? x % ext.gchunks : 0;
   const int b = unit / Hkv, kvh = unit % Hkv;
   if (16 * gc + g >= Gq) return;
-  const int n = (tile_range<EXT>(seq_lens[b], ext).n + per_split - 1) / per_split;
+  const int n = min((tile_range<EXT>(seq_lens[b], ext).n + per_split - 1) / per_split, splits);
   if (n <= 1) return;
   const long row0 = (long)x * splits * 16 + g;
   const int lane = threadIdx.x;

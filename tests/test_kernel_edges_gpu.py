@@ -104,6 +104,22 @@ def test_paged_decode_split_edges(lens, capacity, hq, hkv, d, fp8):
     assert rel(got, want) < bound
 
 
+@pytest.mark.parametrize("capacity", [1, 2, 60, 61])       # in one part, in several
+@pytest.mark.parametrize("general", [False, True])
+def test_paged_decode_of_lengths_past_the_table(capacity, general):
+    n, more = 16 * capacity, 300
+    k, v, bt, _ = _paged([n, n], capacity, 2, 64, 64, torch.bfloat16, 31)
+    sl = torch.tensor([n, n + more], dtype=torch.int32, device=DEV)
+    q, out = rnd(2, 4, 64, seed=5), torch.empty(2, 256, device=DEV, dtype=torch.bfloat16)
+    if general:
+        ops.serve_ext().paged_attn_decode_window(q, k, v, bt, sl, out, 0.125, 1 << 30, 0, None)
+    else:
+        out = ops.paged_attn_decode(q, k, v, bt, sl, 0.125).flatten(1)
+    again = torch.cat([bt[1], bt[1, -1:].expand(more // 16 + 1)])      # its last page
+    assert rel(out[0], _attend64(q[0], k, v, bt[0], n, 0.125).flatten()) < 0.006
+    assert rel(out[1], _attend64(q[1], k, v, again, n + more, 0.125).flatten()) < 0.006
+
+
 @pytest.mark.parametrize("dk,dv,V", [(128, 128, 128), (64, 32, 24), (32, 256, 200)])
 @pytest.mark.parametrize("size,keep", [(1 << 30, 0), (70, 5), (1000, 40)])
 @pytest.mark.parametrize("hq,hkv", [(12, 2), (40, 2)])
