@@ -200,12 +200,16 @@ void fa_fwd_kernel(const short* __restrict__ q, const short* __restrict__ k,
 
 // =============================================================== BACKWARD ==
 // rows [Hq, T]: -sum(dO * O), which dP starts from in the matrix product's
-// accumulator, and lse in log2 units.  16 lanes per row.
+// accumulator, and lse in log2 units.  16 lanes per row.  Tokens ahead of the first
+// sequence and behind the last (padding) have no gradient: nobody else writes theirs.
+DEVINL bool outside(long t, const int* __restrict__ cu, int B) { return t < cu[0] || t >= cu[B]; }
 template <int D>
 __global__ __launch_bounds__(256)
 void fa_bwd_rows_kernel(const short* __restrict__ dout, const short* __restrict__ o,
                         const float* __restrict__ lse, float* __restrict__ drow,
-                        float* __restrict__ lse2, long T, int Hq) {
+                        float* __restrict__ lse2, const int* __restrict__ cu, int B,
+                        short* __restrict__ dq, short* __restrict__ dk, short* __restrict__ dv,
+                        long T, int Hq, int Hkv) {
   const long row = (long)blockIdx.x * 16 + (threadIdx.x >> 4);   // t * Hq + h
   const int i = threadIdx.x & 15;
   float acc = 0.f;
@@ -215,6 +219,16 @@ void fa_bwd_rows_kernel(const short* __restrict__ dout, const short* __restrict_
     ldv<D / 16>(o + row * D + i * (D / 16), b);
 #pragma unroll
     for (int j = 0; j < D / 16; j++) acc += a[j] * b[j];
+    const long t = row / Hq, h = row % Hq;
+    if (outside(t, cu, B)) {
+      const float zero[D / 16] = {};
+      stv<D / 16>(dq + row * D + i * (D / 16), zero);
+      if (h < Hkv) {
+        const long at = (t * Hkv + h) * D + i * (D / 16);
+        stv<D / 16>(dk + at, zero);
+        stv<D / 16>(dv + at, zero);
+      }
+    }
   }
 #pragma unroll
   for (int off = 8; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
@@ -431,11 +445,13 @@ void fa_bwd_dkv_kernel(const short* __restrict__ dout, const short* __restrict__
   }
 }
 
-// sums of the parts, in order; n elements each, 4 per thread; y = 0: dk, 1: dv
+// sums of the parts, in order; n elements each, 4 per thread, `width` per token; y = 0:
+// dk, 1: dv
 __global__ void fa_bwd_sum_kernel(const float* __restrict__ part, short* __restrict__ dk,
-                                  short* __restrict__ dv, long n, int parts) {
+                                  short* __restrict__ dv, const int* __restrict__ cu, int B,
+                                  long n, int width, int parts) {
   const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (i >= n) return;
+  if (i >= n || outside(i / width, cu, B)) return;
   const float* p = part + (blockIdx.y ? (long)parts * n : 0) + i;
   f32x4 s = *reinterpret_cast<const f32x4*>(p);
   for (int k = 1; k < parts; k++) s += *reinterpret_cast<const f32x4*>(p + k * n);
@@ -512,7 +528,9 @@ std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
   do {                                                                         \
     hipLaunchKernelGGL(fa_bwd_rows_kernel<DD>, dim3((T * Hq + 15) / 16), dim3(256), 0, stream, \
                        (const short*)dout.data_ptr(), (const short*)o.data_ptr(), \
-                       lse.data_ptr<float>(), drow, lse2, T, Hq);              \
+                       lse.data_ptr<float>(), drow, lse2, cu_seqlens.data_ptr<int>(), B, \
+                       (short*)dq.data_ptr(), (short*)dk.data_ptr(), (short*)dv.data_ptr(), T, \
+                       Hq, Hkv);                                               \
     hipLaunchKernelGGL((fa_bwd_dq_kernel<DD, CC>), dim3(B * Hq, row_tiles), dim3(256), 0, stream, \
                        (const short*)dout.data_ptr(), (const short*)q.data_ptr(), \
                        (const short*)k.data_ptr(), (const short*)v.data_ptr(), \
@@ -528,8 +546,8 @@ std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
 #undef CALL
   if (parts > 1)
     hipLaunchKernelGGL(fa_bwd_sum_kernel, dim3((n / 4 + 255) / 256, 2), dim3(256), 0, stream,
-                       sums.data_ptr<float>(), (short*)dk.data_ptr(), (short*)dv.data_ptr(), n,
-                       parts);
+                       sums.data_ptr<float>(), (short*)dk.data_ptr(), (short*)dv.data_ptr(),
+                       cu_seqlens.data_ptr<int>(), B, n, (int)(Hkv * D), parts);
   HIP_CHECK_LAST();
   return {dq, dk, dv};
 }

@@ -46,6 +46,25 @@ def test_flash_attention_tile_edges(lens, hq, hkv, d, causal):
         assert rel(got.grad, ref.grad) < FA_REL
 
 
+@pytest.mark.parametrize("rows", [90, 38700])         # dk and dv in several parts, in one
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_flash_attention_gives_padding_no_gradient(rows, d):
+    ahead, behind = 3, 70
+    T = ahead + rows + behind
+    lens = [rows // 90] * 90
+    cu = (torch.tensor([0] + lens, device=DEV).cumsum(0) + ahead).int()
+    leaves = [rnd(T, h, d, seed=h).requires_grad_(True) for h in (12, 2, 2)]
+    dirt = [torch.full((T, h, d), float("nan"), device=DEV, dtype=torch.bfloat16)
+            for h in (12, 12, 2, 2, 2, 2)]
+    del dirt                                          # what new tensors then hold
+    o = ops.flash_attn_varlen(*leaves, cu, lens[0])
+    do = rnd(T, 12, d, seed=4)
+    do[:ahead], do[ahead + rows:] = 0, 0
+    for g in torch.autograd.grad(o, leaves, do):
+        assert torch.isfinite(g).all()
+        assert (g[:ahead] == 0).all() and (g[ahead + rows:] == 0).all()
+
+
 def test_flash_attention_negative_and_zero_scale():
     lens = [70, 130]
     cu = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
