@@ -45,7 +45,7 @@ def glu_fuses(x: torch.Tensor, gate: torch.Tensor) -> bool:
     return (here(x) and plain_call(x, gate) and x.dim() == 2
             and x.dtype == gate.dtype == torch.bfloat16 and x.is_contiguous()
             and gate.is_contiguous() and gate.device == x.device
-            and x.shape[0] >= GLU_ROWS and x.shape[1] % 64 == 0 and x.shape[1] <= GLU_DEPTH
+            and x.shape[0] >= GLU_ROWS and x.shape[1] % 64 == 0 and 0 < x.shape[1] <= GLU_DEPTH
             and x.data_ptr() % 16 == 0 and gate.data_ptr() % 16 == 0)
 
 

@@ -695,3 +695,10 @@ def test_positions_of_packed_sequences():
         assert make_positions(torch.tensor(cu, dtype=torch.int32, device=DEV)).tolist() == want
     with pytest.raises(RuntimeError, match="fall"):
         make_positions(torch.tensor([0, 20, 5, 6], dtype=torch.int32, device=DEV))
+
+
+@pytest.mark.parametrize("rows", [3, 600])
+def test_gated_linear_of_no_depth(rows):
+    x, w = (torch.empty(n, 0, device=DEV, dtype=torch.bfloat16) for n in (rows, 64))
+    with torch.no_grad():
+        assert torch.equal(ops.linear_swiglu(x, w), x.new_zeros(rows, 32))
