@@ -507,6 +507,7 @@ std::vector<torch::Tensor> decode_inputs(torch::Tensor lens, torch::Tensor bt, l
                        c10::hip::getCurrentHIPStream(), lens.data_ptr<int>(), bt.data_ptr<int>(),
                        pos.data_ptr<long>(), slots.data_ptr<long>(), B, (int)bt.size(1),
                        (int)page_size);
+  HIP_CHECK_LAST();
   return {pos, slots};
 }
 
@@ -531,4 +532,5 @@ void decode_commit(torch::Tensor tokens, c10::optional<torch::Tensor> lps, torch
                        lp.data_ptr<float>(), count.data_ptr<int>(), lens.data_ptr<int>(),
                        last.data_ptr<long>(), finished.data_ptr<bool>(), B, most,
                        stop.value_or(0), stop.has_value());
+  HIP_CHECK_LAST();
 }
