@@ -376,6 +376,29 @@ def test_rms_norm_backward_edges(N, H, frozen, residual):
         assert rel(leaves[2].grad, e[2].grad) < 0.006    # x_hat is rounded too
 
 
+@pytest.mark.parametrize("residual", [True, False])
+def test_recorded_backward_of_the_norm(residual):
+    """A backward under create_graph: the same gradients, and the residual stream's part
+    of them can be differentiated (the norm's, a kernel, is a constant)."""
+    x, res = (rnd(5, 64, seed=i).requires_grad_(True) for i in (1, 2))
+    w = rnd(64, seed=3).requires_grad_(True)
+    a, c = rnd(5, 64, seed=4), rnd(5, 64, seed=5)
+
+    def loss():
+        if not residual:
+            return (ops.rms_norm(x, w, 1e-6) * a).sum()
+        y, h = ops.add_rms_norm(x, res, w, 1e-6)
+        return (y * a).sum() + (h * h * c).sum()
+
+    plain = torch.autograd.grad(loss(), (x, w))
+    kept = torch.autograd.grad(loss(), (x, w), create_graph=True)
+    # one more rounding where the residual's part is added by itself: 2^-9 of each term
+    assert rel(kept[0], plain[0]) < 0.006 and torch.equal(kept[1], plain[1])
+    if residual:
+        second, = torch.autograd.grad(kept[0].sum(), x)
+        assert rel(second, 2 * c) < 0.004
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_adamw_takes_many_tensors_at_once(dtype):
     from nanorlhf_amd.ops.adamw import _adamw_ref
@@ -583,6 +606,31 @@ def test_product_down_to_the_rank(M, C):
         got = ops.ext().lora_down(z, p, 0.25, flat)
         want = 0.25 * z.double() @ (p.T if flat else p).double()
         assert rel(got, want) < 0.002              # one rounding, 2^-9 at most
+
+
+def test_recorded_backward_of_the_adapter():
+    """A backward under create_graph: the same gradients, and those of the adapter can be
+    differentiated by dy, x and B (u and dx come from kernels and are constants)."""
+    from nanorlhf_amd.ops import lora
+    M, K, N, s = 65, 128, 192, 0.25
+    x, w = rnd(M, K, seed=1).requires_grad_(True), rnd(N, K, seed=2, scale=K ** -0.5)
+    A = rnd(64, K, seed=4, scale=K ** -0.5).requires_grad_(True)
+    B, c = rnd(N, 64, seed=5, scale=0.1).requires_grad_(True), rnd(M, N, seed=3).requires_grad_(True)
+    va, vb = rnd(64, K, seed=6), rnd(N, 64, seed=7)
+
+    def loss():
+        return (lora.fused_lora_linear(x, w, None, A, B, s, w.t().contiguous()) * c).sum()
+
+    plain = torch.autograd.grad(loss(), (x, A, B))
+    kept = torch.autograd.grad(loss(), (x, A, B), create_graph=True)
+    for got, want in zip(kept, plain):
+        assert rel(got, want) < 0.006              # another order of sums, roundings of 2^-9
+    got = torch.autograd.grad((kept[1] * va).sum() + (kept[2] * vb).sum(), (c, x, B))
+    X, Bd, C, Va, Vb = (t.detach().double() for t in (x, B, c, va, vb))
+    u = s * X @ A.detach().double().T
+    want = (s * X @ Va.T @ Bd.T + u @ Vb.T, s * C @ Bd @ Va, s * C.T @ (X @ Va.T))
+    for g, r in zip(got, want):
+        assert rel(g, r) < 0.012                   # up to four roundings of 2^-9
 
 
 @pytest.mark.parametrize("M,K,N", [(65, 128, 192), (3000, 2048, 2048)])    # small tiles, big
