@@ -448,6 +448,31 @@ def test_portions_and_decoding(dev, dtype, tol, name, sizes):
     close(got, oracle.forward(toks)[0], 4 * tol)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("fused", [False, True])     # one product, or gate and up by themselves
+@pytest.mark.parametrize("rows", [63, 511, 512])
+def test_feed_forward_of_many_rows_fills_its_columns(fused, rows, monkeypatch):
+    """Mixer outputs and feed-forwards whose ends are padded, in memory that holds NaN:
+    a column that nobody writes shows in the output projection."""
+    cfg = config(retention(heads=1, dim=6, vdim=10, rot=4), lightning(heads=2, dim=10, vdim=6),
+                 attention(heads=3, kv=3, dim=10, vdim=6, rot=10, size=5, keep=1),
+                 width=64, groups=1, vocab=97, ff=30)
+    model, oracle = make(cfg, "cuda", torch.bfloat16)
+    empty = torch.empty
+
+    def dirty(*args, **kwargs):
+        t = empty(*args, **kwargs)
+        return t.fill_(float("nan")) if t.is_floating_point() else t
+
+    seq = SeqState(0, tokens(cfg, rows), rows)
+    eng = engine(model, pool=1024)
+    monkeypatch.setattr(torch, "empty", dirty)
+    monkeypatch.setattr(ops, "glu_fuses", lambda x, w: fused)
+    got = run(eng, [[(seq, rows)]])[0]
+    monkeypatch.undo()
+    close(got, oracle.forward(seq.tokens)[0], 4 * 0.02)
+
+
 @kinds
 def test_mixed_batches_and_reused_slots(dev, dtype, tol):
     """Unequal requests in one batch, some left out of steps, more requests

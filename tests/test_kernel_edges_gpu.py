@@ -520,7 +520,7 @@ def test_glu_linear_tile_edges(M, N, K, act, strided):
         assert (whole[:, :8] == 7).all() and (whole[:, 8 + N:] == 7).all()
 
 
-@pytest.mark.parametrize("rows", [511, 512])
+@pytest.mark.parametrize("rows", [1, 64, 65, 511, 512])
 @pytest.mark.parametrize("form", ["plain", "merged", "hooked", "bias"])
 def test_gated_feed_forward_takes_both_ways(rows, form):
     from nanorlhf_amd.models.config import get_config
