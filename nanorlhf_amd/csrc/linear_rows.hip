@@ -12,7 +12,7 @@
 // us for 64 / 16 / 1 rows, library before -> now:
 //   2048 x 1536       7.6 -> 5.8    7.1 -> 3.8    6.9 -> 3.7
 //   1536 x 8960       24.8 -> 15.0  27.9 -> 10.6  27.7 -> 9.7
-//   8960 x 1536, GLU  20.6 -> 19.9  41.6 -> 14.1  42.1 -> 13.7
+//   8960 x 1536, GLU  20.6 -> 18.6  41.6 -> 14.1  42.1 -> 13.7
 //   151936 x 1536     115 -> 108    159 -> 89     158 -> 83     (467 MB: 5.6 TB/s)
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
@@ -220,15 +220,19 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, c10::optional<torch:
   a.N = N;
   a.K = K;
   // 16 columns each while that makes at most a workgroup per CU, since the rows of
-  // x are read by each; up to 64 for more columns.  A deep product of few columns is
-  // divided until about 224 workgroups share it, which has to pay for a second kernel
-  // of 3 us: 64 rows of 1536 x 8960 15 us in 4 parts, 24 in one; 1536 x 1536 6 us in
-  // one, 7 in 2.  For more than 32 rows wider tiles share x better: 64 of 151936 x
-  // 1536 108 us, with 64 columns 113 to 118.
-  const bool deep = K > 2048;
-  const int nf = deep ? (N <= 1024 ? 1 : N < 3200 ? 2 : 4) : N <= 4096 ? 1 : N <= 8192 ? 2 : 4;
+  // x are read by each; up to 64 for more columns, 128 for the widest with more than
+  // 32 rows, where that shares x better: 64 rows of 152064 x 1536 108 us, 119 with 64;
+  // of 32768 x 1536 32, 27 with 64.  A deep product of few columns is divided until about
+  // 224 workgroups share it, which has to pay for a second kernel of 3 us: 64 rows of
+  // 1536 x 8960 15 us in 4 parts, 24 in one; 1536 x 1536 6 us in one, 7 in 2.  A deep one
+  // of many columns wants many waves in flight on each: one row of 14336 x 4096 24 us
+  // with 32 columns and four waves, 32 with 64 and two.
+  const bool deep = K > 2048, shared = deep && N <= 5120;
+  const int nf = shared ? (N <= 1024 ? 1 : N < 3200 ? 2 : 4)
+                 : deep ? 2 : N <= 4096 ? 1 : N <= 8192 ? 2 : 4;
   const long tiles = (N + 16 * nf - 1) / (16 * nf);
-  const int splits = deep && N % 4 == 0 ? (int)std::min(8L, std::max(1L, (224 + tiles / 2) / tiles)) : 1;
+  const int splits =
+      shared && N % 4 == 0 ? (int)std::min(8L, std::max(1L, (224 + tiles / 2) / tiles)) : 1;
   torch::Tensor parts;
   if (splits > 1) {
     parts = torch::empty({splits, M, N}, x.options().dtype(torch::kFloat32));
@@ -237,7 +241,7 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, c10::optional<torch:
   }
   if (nf == 1) launch_rows<1, 4, 3, false>(a, splits);
   else if (nf == 2) launch_rows<2, 4, 3, false>(a, splits);
-  else if (splits > 1 || M <= 32) launch_rows<4, 2, 2, false>(a, splits);
+  else if (M <= 32 || N <= 65536) launch_rows<4, 2, 2, false>(a, splits);
   else launch_rows<8, 2, 1, false>(a, splits);
   if (splits > 1)
     hipLaunchKernelGGL(rows_sum_kernel, dim3((M * N / 4 + 255) / 256), dim3(256), 0,
@@ -263,11 +267,23 @@ torch::Tensor glu_rows(torch::Tensor x, torch::Tensor gate, torch::Tensor up) {
   a.M = M;
   a.N = N;
   a.K = x.size(1);
-  // Up to 6144 columns 16 to a workgroup, else 40, which for 8960 makes one for each
-  // of 224 CUs: 64 rows of 8960 x 1536 18.7 us with 40, 21 with 32 (280 workgroups)
-  // and with 16; of 18944 x 3584 57 against 67; of 4864 x 896 7.3 with 16, 8.9 with 24
-  if (N <= 6144) launch_rows<2, 2, 3, true>(a, 1);
-  else launch_rows<5, 2, 2, true>(a, 1);
+  // Of 16, 32, 40 and 48 columns to a workgroup those with which the 256 CUs, one workgroup
+  // each, are through soonest, more rather than fewer where it makes no difference: 64 rows
+  // of 7168 x 2048 16 us with 32, 20 with 40; 8960 x 1536 18.6 with 40, 25 with 16; 11008 x
+  // 2048 22 with 48, 31 with 40 (276 workgroups); 18944 x 3584 58 with 40, 61 and 80 with
+  // 48 and 32.
+  long best = 0, cost = 0;
+  for (long cols : {48L, 40L, 32L, 16L}) {
+    const long c = ((N + cols - 1) / cols + 255) / 256 * cols;
+    if (!best || c < cost) {
+      best = cols;
+      cost = c;
+    }
+  }
+  if (best == 16) launch_rows<2, 2, 3, true>(a, 1);
+  else if (best == 32) launch_rows<4, 2, 2, true>(a, 1);
+  else if (best == 40) launch_rows<5, 2, 2, true>(a, 1);
+  else launch_rows<6, 2, 2, true>(a, 1);
   HIP_CHECK_LAST();
   return y;
 }

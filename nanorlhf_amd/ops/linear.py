@@ -10,8 +10,8 @@ from torch.utils._device import DeviceContext
 from . import linear_ext
 
 # Library against the kernel, in us: 64 rows of 3584 x 18944 91 / 36, of 4608 x 3584
-# 18.7 / 15.3, of 37888 x 3584 70 / 57, of 151936 x 1536 115 / 108; with more rows x
-# weighs as much as the weights and the library's tiles share it better.
+# 18.7 / 15.3, of 151936 x 1536 115 / 108; with more rows x weighs as much as the weights
+# and the library's tiles share it better.
 FEW_ROWS = 64
 DEPTH = 1 << 24         # from which on its 32-bit offsets would wrap
 
@@ -42,8 +42,23 @@ def here(x: torch.Tensor) -> bool:
     return x.is_cuda and x.device.index == torch.cuda.current_device()
 
 
+def rows_pay(M: int, N: int, K: int) -> bool:
+    """Whether M <= FEW_ROWS rows of N x K are faster by the kernel.  Wide products are a
+    matter of how full the CUs' last round of 64 columns each is, and from some rows on of
+    x's fetch into every CU, which the library's tiles share; deep ones of a few columns
+    are divided, deep and wide ones are not.  Library / kernel in us: 32 rows of 18944 x
+    1536 16.8 / 19.3, of 32768 x 1536 24.1 / 23.5; 48 rows of 24576 x 1536 20 / 22, of
+    16384 x 1536 19.2 / 15; 64 rows of 12288 x 1536 13.6 / 15.3, of 12288 x 896 12 / 10.6;
+    16 rows of 14336 x 4096 31 / 25, 32 rows 27 / 30; 1 row of 6144 x 8192 24 / 30."""
+    if K > 2048 and N > 5120:
+        return M <= 16 and K <= 4096
+    tiles = -(-N // 64)
+    full = tiles / (256 * -(-tiles // 256)) >= 0.8
+    return N <= 16384 or N > 65536 or M <= (32 if full else 16)
+
+
 def few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether the kernels for few rows take x [M, K] and w [N, K]."""
+    """Whether the kernels for few rows can take x [M, K] and w [N, K]."""
     return (here(x) and x.dim() == 2 and x.shape[0] <= FEW_ROWS and plain_call(x, w)
             and x.dtype == w.dtype == torch.bfloat16 and x.shape[1] % 64 == 0
             and x.shape[1] < DEPTH and x.is_contiguous() and w.is_contiguous()
@@ -52,8 +67,8 @@ def few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """x w^T + bias."""
-    if few_rows(x, w) and (bias is None or plain_call(bias) and bias.dtype == x.dtype
-                           and bias.device == x.device and bias.shape == w.shape[:1]
-                           and bias.is_contiguous()):
+    if few_rows(x, w) and rows_pay(x.shape[0], *w.shape) and (
+            bias is None or plain_call(bias) and bias.dtype == x.dtype
+            and bias.device == x.device and bias.shape == w.shape[:1] and bias.is_contiguous()):
         return linear_ext().linear_rows(x, w, bias)
     return F.linear(x, w, bias)

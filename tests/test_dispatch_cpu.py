@@ -63,3 +63,12 @@ def test_adapter_strategies_are_kept_by_what_the_kernels_depend_on(monkeypatch):
     assert [choose(240), choose(4000), choose(240, bias)] == ["fused", "epilogue", "fused"]
     assert [choose(17), choose(9000), choose(60, bias)] == ["fused", "epilogue", "fused"]
     assert next(times, None) is None and len(lora._TUNE[64, 64]) == 3
+
+
+def test_linears_of_few_rows_leave_what_the_library_does_faster():
+    from nanorlhf_amd.ops.linear import rows_pay
+    for M, N, K in [(1, 1536, 1536), (64, 16384, 2048), (32, 32768, 1536), (16, 18944, 1536),
+                    (64, 151936, 1536), (64, 3584, 18944), (16, 14336, 4096)]:
+        assert rows_pay(M, N, K)
+    for M, N, K in [(33, 32768, 1536), (17, 18944, 1536), (17, 14336, 4096), (1, 6144, 8192)]:
+        assert not rows_pay(M, N, K)

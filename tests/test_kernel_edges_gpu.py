@@ -550,7 +550,7 @@ def test_gated_feed_forward_takes_both_ways(rows, form):
 # ---------------------------------------------------------- linears of few rows
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 48, 49, 64])
 @pytest.mark.parametrize("N,K", [(8, 64), (17, 128), (1536, 2112), (1000, 8960), (4100, 192),
-                                 (8204, 128), (3204, 2176), (3207, 2176)])
+                                 (8204, 128), (3204, 2176), (3207, 2176), (66004, 64)])
 @pytest.mark.parametrize("bias", [True, False])
 def test_linear_of_few_rows(M, N, K, bias):
     x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=K ** -0.5)
@@ -563,7 +563,8 @@ def test_linear_of_few_rows(M, N, K, bias):
 
 
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 48, 64])
-@pytest.mark.parametrize("N,K", [(8, 64), (101, 192), (6200, 128), (6150, 2112)])
+@pytest.mark.parametrize("N,K", [(8, 64), (101, 192), (6200, 128), (6150, 2112), (8204, 128),
+                                 (11003, 128)])
 def test_gated_linear_of_few_rows(M, N, K):
     x, w = rnd(M, K, seed=1), rnd(2 * N, K, seed=2, scale=K ** -0.5)
     g, u = (x.double() @ w.double().T).split(N, 1)
