@@ -109,9 +109,9 @@ class ParallelBlock(nn.Module):
     def forward(self, h: torch.Tensor, ctx, cache) -> torch.Tensor:
         w = plain_weight(self.in_proj) if self.ff else None
         cat = torch.empty(h.shape[0], self.out_width, dtype=h.dtype, device=h.device)
-        if w is not None and self.in_proj.bias is None and ops.glu_fuses(h, w):
+        (a, b), (c, d) = (self.cols[n] for n in ("gate", "up")) if self.ff else ((0, 0), (0, 0))
+        if w is not None and self.in_proj.bias is None and ops.glu_fuses(h, w[a:b]):
             # the mixer's columns alone, gate and up straight into the output's input
-            (a, b), (c, d) = self.cols["gate"], self.cols["up"]
             proj = F.linear(h, w[:a])
             ops.linear_gelu_glu(h, w[a:b], w[c:d], cat[:, self.ff_start:self.ff_start + self.ff])
             cat[:, self.mix_out:self.ff_start] = 0
@@ -121,9 +121,8 @@ class ParallelBlock(nn.Module):
         proj = project(self.in_proj, h)
         self.mixer(self.cols, proj, ctx, cache, cat[:, :self.mix_out])
         if self.ff:
-            gate, up = (proj[:, slice(*self.cols[n])] for n in ("gate", "up"))
             pad = self.ff_start - self.mix_out
-            ops.gelu_glu(gate, up, cat[:, self.mix_out:], pad,
+            ops.gelu_glu(proj[:, a:b], proj[:, c:d], cat[:, self.mix_out:], pad,
                          self.out_width - self.ff_start - self.ff)
         return project(self.out_proj, cat)
 

@@ -36,11 +36,22 @@ def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
 # kernel.  Library product and a pass against it, in us: 1024 x 4864 x 896 40 / 25,
 # 2048 x 4096 x 1024 68 / 33, 600 x 8960 x 1536 51 / 40, 16320 x 8960 x 1536 857 /
 # 786.  A few rows leave most of its 256-row tiles empty (300 x 8960 x 1536: 34 /
-# 37), and deep products have little to save (4096 x 18944 x 3584: 872 / 910).
+# 37), deep products have little to save (4096 x 18944 x 3584: 872 / 910), and its tiles
+# have to fill the CUs' rounds (glu_fills).
 GLU_ROWS, GLU_DEPTH = 512, 2048
 # The kernel of few rows does not divide the depth: 16 rows of 4128 x 8192 take the library
 # and a pass 36 us, it 45, of 4128 x 4096 28 and 23.
 FEW_DEPTH = 4096
+
+
+def glu_fills(M: int, I: int, K: int) -> bool:
+    """Whether M x I x K fills enough of the rounds that 256 CUs need for its tiles of 256 x
+    128, one each: a tile's time grows with the depth, an idle CU's share of it with that.
+    Library and pass / kernel in us: 512 x 1024 x 1536 13.5 / 31.6 (8 tiles), 1024 x 2240 x
+    1536 25.8 / 32 (72), 2000 x 2240 x 1536 43 / 34 (144), 600 x 11008 x 2048 70 / 88 (258);
+    512 x 4864 x 896 25 / 21 (76).  A shallow product is launches."""
+    tiles = -(-M // 256) * -(-I // 128)
+    return K <= 256 or tiles / (256 * -(-tiles // 256)) >= (0.25 if K <= 1024 else 0.6)
 
 
 def glu_fuses(x: torch.Tensor, gate: torch.Tensor) -> bool:
@@ -49,7 +60,8 @@ def glu_fuses(x: torch.Tensor, gate: torch.Tensor) -> bool:
             and x.dtype == gate.dtype == torch.bfloat16 and x.is_contiguous()
             and gate.is_contiguous() and gate.device == x.device
             and x.shape[0] >= GLU_ROWS and x.shape[1] % 64 == 0 and 0 < x.shape[1] <= GLU_DEPTH
-            and x.data_ptr() % 16 == 0 and gate.data_ptr() % 16 == 0)
+            and x.data_ptr() % 16 == 0 and gate.data_ptr() % 16 == 0
+            and glu_fills(x.shape[0], gate.shape[0], x.shape[1]))
 
 
 def linear_swiglu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:

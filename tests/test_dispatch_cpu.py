@@ -72,3 +72,11 @@ def test_linears_of_few_rows_leave_what_the_library_does_faster():
         assert rows_pay(M, N, K)
     for M, N, K in [(33, 32768, 1536), (17, 18944, 1536), (17, 14336, 4096), (1, 6144, 8192)]:
         assert not rows_pay(M, N, K)
+
+
+def test_gated_products_fuse_where_their_tiles_fill_the_gpu():
+    from nanorlhf_amd.ops.swiglu import glu_fills
+    for M, I, K in [(512, 4864, 896), (600, 8960, 1536), (16320, 8960, 1536), (512, 200, 128)]:
+        assert glu_fills(M, I, K)
+    for M, I, K in [(512, 1024, 1536), (1024, 2240, 1536), (600, 11008, 2048)]:
+        assert not glu_fills(M, I, K)
