@@ -510,14 +510,27 @@ static void launch_grouped(const Grouped& a, bool bf16) {
     const long each = a.lists ? a.rows / a.G : a.rows;      // rows of a group, about
     const long tm = tiles_of(128), tn = (a.N + (GLU ? 63 : 127)) / (GLU ? 64 : 128);
     // Up to 52 rows the weights are what counts: 160 tokens with 4 of 16 experts of 1536 x
-    // 2240 52 and 27 us in rows of 64, 60 and 33 in tiles; 256 tokens 75 and 38 against
-    // 64 and 40
-    if (each > 52 && (each > 512 || tm * tn >= 64)) {
+    // 2240 68 and 34 us in rows of 64, 79 and 39 in tiles; 288 tokens 84 and 51 against 80
+    // and 44.  Unless there are more than 32 rows to each and tiles enough for rounds of
+    // their own, the more the longer a tile takes: 40 rows of 128 experts of 512 x 1024 (1024
+    // tiles) 49 us against 58, of 16 experts of 4096 x 3584 (900) 253 against 207.
+    const bool many = tm * tn >= std::max<long>(256, a.K / 2);
+    if (each > 52 ? each > 512 || tm * tn >= 64 : each > 32 && many) {
       TORCH_CHECK(tm * tn < (1L << 31));
       hipLaunchKernelGGL((grouped_tiles_kernel<GLU>), dim3(tm * tn), dim3(256), 0, stream, a,
                          (int)tm, (int)tn);
     } else {
-      const int mf = each > 28 && each <= 52 ? 4 : each > 12 ? 2 : 1;
+      // 64 rows at a time read the weights once but leave half the workgroups: where there
+      // are enough for every CU all the same, and the depth is worth it.  8 experts of 1024 x
+      // 512, 40 rows each: 13 and 10 us with 32 rows, 18 and 14 with 64.  More than 52
+      // rows come here in small grids only: 12 heads of 512 x 128, 128 rows 6.2 us with 32, 7.6
+      // with 64.
+      constexpr long WIDE = GLU ? 32 : 64;
+      const bool full =
+          a.lists ? std::min<long>(tiles_of(64), a.rows) * ((a.N + WIDE - 1) / WIDE) >= 256
+                  : tiles_of(32) * ((a.N + WIDE / 2 - 1) / (WIDE / 2)) > 256;
+      const int mf = each > 28 && each <= 52 && a.K >= 1024 && !many && full ? 4
+                     : each > 12 ? 2 : 1;
       // Four waves with a chunk of their own each.  Where 64 weight rows to a workgroup
       // leave CUs idle, 32 and two chunks: one token's 4 experts of 1536 x 2240 7.7 us
       // against 10.

@@ -588,7 +588,8 @@ def test_adapter_gradients_tile_edges(M, K, N):
 
 # ------------------------------------------------------- grouped products
 @pytest.mark.parametrize("T", [1, 12, 13, 32, 33, 52, 53])
-@pytest.mark.parametrize("G,N,K", [(1, 24, 8), (3, 100, 72), (2, 1030, 200), (40, 700, 1000)])
+@pytest.mark.parametrize("G,N,K", [(1, 24, 8), (3, 100, 72), (2, 1030, 200), (40, 700, 1000),
+                                   (4, 1030, 1096), (40, 700, 1088), (70, 500, 72)])
 def test_grouped_product_of_few_rows(T, G, N, K):
     x, w = rnd(T, G, K, seed=1), rnd(G, N, K, seed=2, scale=K ** -0.5)
     got = ops.group_linear(x, w)
