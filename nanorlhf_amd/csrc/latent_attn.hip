@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
   constexpr int LOADS = PAGE / 512;                      // direct loads per page
   constexpr int NBUF = RP >= 512 ? 2 : 4;
   // pages of each wave; at the end its sums, 16 x RP floats
-  __shared__ __attribute__((aligned(16))) short buf[NW][NBUF * PAGE];
+  __shared__ __attribute__((aligned(1024))) short buf[NW][NBUF * PAGE];
   __shared__ float Lm[NW][16], Ls[NW][16];
   const int seq = blockIdx.y;
   const int t0 = a.cu ? a.cu[seq] : seq;
@@ -141,6 +141,15 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
 #pragma unroll
   for (int q = 0; q < NC; q++) asm volatile("" : "+v"(qf[q]));
 
+  // this lane's part of a page, by rows (scores) and turned around
+  typedef __attribute__((address_space(3))) char* lds_bytes;
+  typedef __attribute__((address_space(3))) const bf16x8l* lds_frag;
+  typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
+  const int tr = 4 * hi + (lo >> 2);
+  const unsigned buf0 = lds_address(buf[wid]);
+  const unsigned row_at = lo * 2 * RP + ((hi ^ page_swz<RP>(lo)) << 4);
+  const unsigned col_at = tr * 2 * RP + ((((lo & 3) >> 1) ^ page_swz<RP>(tr)) << 4) + (lo & 1) * 8;
+
   float m = -INFINITY, sum = 0.f;             // of row lo
   f32x4 acc[NT];                              // O^T: latent columns 16 t + 4 hi + r, row lo
 #pragma unroll
@@ -151,12 +160,27 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
     // pages behind this one that are on their way
     if (pg + NW * (NBUF - 1) < p1) wait_loads<LOADS * (NBUF - 1)>();
     else wait_loads<0>();
+    // Another fragment along the latent is an xor of its chunk, which has the bits below
+    // 256 bytes to itself, and an offset.  At 512 that makes a few addresses; one for each
+    // fragment would leave no registers to read ahead of the products (1 x 200 tokens
+    // of 12 heads 14.2 us, 15.5).  Narrower latents have them: 128 x 2000 of 256 38 us, 39.5.
+    const unsigned page = buf0 + slot * (PAGE * 2), ra = page + row_at, ca = page + col_at;
     const short* C = &buf[wid][slot * PAGE];
+    auto by_row = [&](int q) {
+      if constexpr (RP >= 512) return *(lds_frag)((lds_bytes)(ra ^ (q & 3) << 6) + (q >> 2) * 256);
+      else return frag(C + lo * RP + (((4 * q + hi) ^ page_swz<RP>(lo)) << 3));
+    };
+    auto turned = [&](int t) {
+      if constexpr (RP >= 512)
+        return (lds_s16x4)((lds_bytes)(ca ^ (t & 7) << 5) + (t >> 3) * 256);
+      else
+        return (lds_s16x4)(C + tr * RP + (((2 * t + ((lo & 3) >> 1)) ^ page_swz<RP>(tr)) << 3) +
+                           (lo & 1) * 4);
+    };
     f32x4 s2[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int q = 0; q < NC; q++)
-      s2[q & 1] = mfma16l(frag(C + lo * RP + (((4 * q + hi) ^ page_swz<RP>(lo)) << 3)), qf[q],
-                          s2[q & 1]);
+      s2[q & 1] = mfma16l(by_row(q), qf[q], s2[q & 1]);
     float x[4], top = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
@@ -185,16 +209,10 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
     rs += __shfl_xor(rs, 16);
     rs += __shfl_xor(rs, 32);
     sum = sum * alpha + rs;
-    {
-      typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-      const int tr = 4 * hi + (lo >> 2), sw = page_swz<RP>(tr);
 #pragma unroll
-      for (int t = 0; t < NT; t++) {
-        const short* at = C + tr * RP + (((2 * t + ((lo & 3) >> 1)) ^ sw) << 3) + (lo & 1) * 4;
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at), pf, acc[t], 0, 0, 0);
-      }
-    }
+    for (int t = 0; t < NT; t++)
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16(turned(t)), pf, acc[t], 0, 0, 0);
     if (ahead < p1) {
       lds_fence_wave_kv();                    // this page's reads are done
       fetch(ahead, slot);
@@ -212,30 +230,40 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
   if (hi == 0) { Lm[wid][lo] = m; Ls[wid][lo] = sum; }
   __syncthreads();
   const long unit = ((long)blockIdx.y * gridDim.x + blockIdx.x) * a.splits + blockIdx.z;
-  for (int i = threadIdx.x; i < 16 * (RP / 4); i += 256) {
-    const int r = i / (RP / 4), c = i % (RP / 4);
-    if (r0 + r >= R) break;
-    float M = Lm[0][r];
+  // four rows to a wave; all sums ahead of the first store, so that their reads overlap
+  constexpr int NK = RP / 64;
+  f32x4 o[NK];
+  float M[NK], S[NK];
 #pragma unroll
-    for (int w = 1; w < NW; w++) M = fmaxf(M, Lm[w][r]);
-    const float Mf = M == -INFINITY ? 0.f : M;
-    float S = 0.f;
-    f32x4 o{0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < NK; k++) {
+    const int i = lane + 64 * k, r = 4 * wid + i / (RP / 4), c = i % (RP / 4);
+    M[k] = Lm[0][r];
+#pragma unroll
+    for (int w = 1; w < NW; w++) M[k] = fmaxf(M[k], Lm[w][r]);
+    const float Mf = M[k] == -INFINITY ? 0.f : M[k];
+    S[k] = 0.f;
+    o[k] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < NW; w++) {
       const float f = exp2f(Lm[w][r] - Mf);
-      S += Ls[w][r] * f;
-      o += *reinterpret_cast<const f32x4*>(reinterpret_cast<float*>(buf[w]) + r * RP +
-                                           ((c ^ r) << 2)) * f;
+      S[k] += Ls[w][r] * f;
+      o[k] += *reinterpret_cast<const f32x4*>(reinterpret_cast<float*>(buf[w]) + r * RP +
+                                              ((c ^ r) << 2)) * f;
     }
+  }
+#pragma unroll
+  for (int k = 0; k < NK; k++) {
+    const int i = lane + 64 * k, r = 4 * wid + i / (RP / 4), c = i % (RP / 4);
+    if (r0 + r >= R) continue;
     if (a.splits > 1) {
-      *reinterpret_cast<f32x4*>(a.part + (unit * 16 + r) * RP + 4 * c) = o;
+      *reinterpret_cast<f32x4*>(a.part + (unit * 16 + r) * RP + 4 * c) = o[k];
       if (c == 0) {
-        a.ms[(unit * 16 + r) * 2] = M;
-        a.ms[(unit * 16 + r) * 2 + 1] = S;
+        a.ms[(unit * 16 + r) * 2] = M[k];
+        a.ms[(unit * 16 + r) * 2 + 1] = S[k];
       }
     } else {
-      const float inv = 1.f / S, y[4] = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
+      const float inv = 1.f / S[k];
+      const float y[4] = {o[k][0] * inv, o[k][1] * inv, o[k][2] * inv, o[k][3] * inv};
       stv<4>(a.out + ((long)t0 * a.H + r0 + r) * RP + 4 * c, y);
     }
   }
