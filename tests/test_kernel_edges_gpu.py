@@ -235,6 +235,20 @@ def test_sampler_greedy_ties_and_odd_rows():
         assert s[2] == 0 and s[3] == 5 and s[4] == 9 and 0 <= s[5] < 3001 and s[5] != 40
 
 
+@pytest.mark.parametrize("V", [8185, 8192, 8193, 20003])      # 256 threads to a row, 512
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_greedy_rows_of_both_widths(V, dtype):
+    x = rnd(5, V, seed=V, dtype=dtype)
+    x[0, V - 1], x[1, V // 2:V // 2 + 2], x[2, [V - 3, 1]] = 9.0, 9.0, 9.0
+    step = torch.ones(1, dtype=torch.long, device=DEV)
+    tok, lp = ops.ext().sample_topp_dev(x, 0.0, 1.0, 1, step)
+    top = x.double().max(1, keepdim=True)[0]
+    want = (x.double() == top).int().argmax(1)                # the lowest of equals
+    assert torch.equal(tok, want) and tok[:3].tolist() == [V - 1, V // 2, 1]
+    assert torch.allclose(lp.double(), x.double().log_softmax(1).gather(1, want[:, None])[:, 0],
+                          rtol=0, atol=1e-4)                  # 32-bit sums and exponentials
+
+
 # --------------------------------------------------------- latent attention
 @pytest.mark.parametrize("rp", [64, 128, 256, 512])
 @pytest.mark.parametrize("heads", [1, 12, 17])
