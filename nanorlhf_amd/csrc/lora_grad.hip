@@ -4,9 +4,9 @@
 // Bound by reading x and dy once.  A workgroup owns 128 of their columns and a part
 // of the tokens, 64 at a time, which two LDS buffers receive by direct loads; both
 // operands of the product are read transposed.  Few columns are divided among many
-// parts, whose 32-bit sums lora_grad_sum_kernel adds in order.  48720 tokens, K = N =
-// 1536: 81 us for both (floor 62), two library products 379; N = 17920 449 against
-// 578; 240 tokens 7.6 against 45, most of it the host's.
+// parts, whose 32-bit sums lora_grad_sum_kernel adds in order.  48720 tokens, dB of N =
+// 1536 54 us (floor 31), the library 150; of 17920 352 against 354; 8000 tokens of 1536 16
+// against 54; 240 7 against 8, and 7.6 against 45 with the host's part of both products.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -150,9 +150,10 @@ std::vector<torch::Tensor> lora_grads(c10::optional<torch::Tensor> x,
     j.out = (short*)outs.back().data_ptr();
     j.C = C;
     j.tiles = (C + COLS - 1) / COLS;
-    // about 512 workgroups, each with at least 8 steps
+    // at most 512 workgroups, two for each CU, of at least 8 steps: 48720 tokens of 17920
+    // columns 352 us in 3 parts (420 workgroups), 413 in 4; of 9728 193 in 6, 240 in 7
     const long steps = (M + TILE - 1) / TILE;
-    j.splits = (int)std::max(1L, std::min<long>((512 + j.tiles / 2) / j.tiles, steps / 8));
+    j.splits = (int)std::max(1L, std::min<long>(512 / j.tiles, steps / 8));
     if (j.splits > 1) {
       keep.push_back(torch::empty({j.splits, C * RANK}, options.dtype(torch::kFloat32)));
       j.part = keep.back().data_ptr<float>();
@@ -174,8 +175,8 @@ std::vector<torch::Tensor> lora_grads(c10::optional<torch::Tensor> x,
 // out [M, 64] = scale z p: p is A^T of A [64, C] (FLAT) or B [C, 64].  A workgroup
 // owns 64 rows and a part of the columns, 64 at a time through three LDS buffers.
 // Bound by reading z once; a few rows are divided among parts of the columns.  48720
-// x 1536 25 us (6 TB/s), library 29; 8000 x 1536 11, library 26; 240 x 896 8.5,
-// library 25, of which the host's calls are most.
+// x 1536 37 us, library 38; 4096 x 8960 26, library 43; 240 x 896 7, library 14, and with
+// the host's part 8.5 and 25.
 template <bool FLAT>
 __global__ __launch_bounds__(256, 3)
 void lora_down_kernel(const short* __restrict__ z, const short* __restrict__ p,
@@ -274,7 +275,21 @@ torch::Tensor lora_down(torch::Tensor z, torch::Tensor p, double scale, bool fla
   z = on16(z);
   p = on16(p);
   const long tiles = (M + TILE - 1) / TILE, steps = (C + TILE - 1) / TILE;
-  const int splits = (int)std::max(1L, std::min({384 / tiles, steps / 3, 16L}));
+  // Parts of the columns that make it shortest, in us: a step of a workgroup takes 0.31
+  // and the longer the more of them share the memory; a division costs another launch and
+  // the parts' way through memory.
+  // Measured in 1 / 2 / 4 parts: 240 x 1536 11.1 / 9.3 / 7.7, 4096 x 1536 11.4 / 10.5 / 10.6,
+  // 8000 x 1536 11.7 / 12.1 / 12.7, 8000 x 8960 59 / 42 / 39, 16000 x 3584 32.4 / 31.8 / 34.4.
+  int splits = 1;
+  double best = 0;
+  for (long n = 1; n <= std::min(16L, steps); n++) {
+    const double us = (double)((steps + n - 1) / n) * std::max(0.31, 0.25 + (double)(tiles * n) * 0.0012) +
+                      (n > 1 ? 2.2 + (double)(n * M) * 1e-4 : 0.0);
+    if (n == 1 || us < best) {
+      best = us;
+      splits = (int)n;
+    }
+  }
   torch::Tensor parts;
   if (splits > 1) parts = torch::empty({splits, M * RANK}, z.options().dtype(torch::kFloat32));
   float* pp = splits > 1 ? parts.data_ptr<float>() : nullptr;

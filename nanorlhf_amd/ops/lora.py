@@ -90,20 +90,31 @@ def _dispatch_gemm(x, w, u, b, bias):
 
 # Products down to the rank are csrc/lora_grad.hip's lora_down, unless both many rows
 # and many columns, where the library streams them 5 to 20% faster.  Library against
-# kernel, in us: 240 x 896 25 / 8.5, 8000 x 1536 26 / 11, 8000 x 17920 81 / 67, 48720 x
-# 1536 29 / 25, 64000 x 1536 33 / 32; 64000 x 2048 44 / 47, 24000 x 8960 86 / 103.
-DOWN_ROWS, DOWN_SIZE = 16384, 100_000_000
+# kernel, in us: 240 x 896 14 / 7, 4096 x 8960 43 / 25, 8000 x 3584 22 / 21, 48720 x 1536
+# 38 / 37; 16000 x 3584 28 / 32, 24000 x 8960 93 / 112, 64000 x 2048 58 / 65.
+DOWN_ROWS, DOWN_COLS, DOWN_SIZE = 8192, 2048, 100_000_000
+# Gradients of more columns than these leave no room to divide the tokens evenly: 16000
+# tokens of 37888 columns 247 / 284 us, 240 tokens 13.4 / 9.4.
+GRAD_COLS, GRAD_ROWS = 20480, 512
 
 
 def _down(z: torch.Tensor, p: torch.Tensor, scale: float, flat: bool) -> torch.Tensor:
     """scale * z pᵀ with p [r, C] (flat), or scale * z p with p [C, r]; the scale rides
     on the product's sums."""
     C = z.shape[1]
-    if (z.shape[0] <= DOWN_ROWS or z.numel() <= DOWN_SIZE) and C % (64 if flat else 8) == 0 \
-            and z.dtype == p.dtype == torch.bfloat16 and p.shape[0 if flat else 1] == 64 \
+    if (z.shape[0] <= DOWN_ROWS or C <= DOWN_COLS and z.numel() <= DOWN_SIZE) \
+            and C % (64 if flat else 8) == 0 and z.dtype == p.dtype == torch.bfloat16 \
+            and p.shape[0 if flat else 1] == 64 \
             and not torch.is_grad_enabled():       # a backward that is itself recorded
         return ext().lora_down(z.contiguous(), p.contiguous(), scale, flat)
     return torch.addmm(z.new_empty(1), z, p.t() if flat else p, beta=0, alpha=scale)
+
+
+def _fast_grad(z: torch.Tensor) -> bool:
+    """Whether csrc/lora_grad.hip's lora_grads takes the gradient with z [M, C] in it, and
+    not a backward that is itself recorded."""
+    return z.shape[1] % 8 == 0 and z.dtype == torch.bfloat16 and not torch.is_grad_enabled() \
+        and (z.shape[1] <= GRAD_COLS or z.shape[0] <= GRAD_ROWS)
 
 
 class _FusedLoRAFn(torch.autograd.Function):
@@ -132,14 +143,16 @@ class _FusedLoRAFn(torch.autograd.Function):
         want_A, want_B = ctx.needs_input_grad[3:5]
         if not (want_A or want_B):
             return dx, None, None, None, None, None, None
-        if dy.shape[1] % 8 == 0 and x.dtype == dy.dtype == torch.bfloat16 \
-                and not torch.is_grad_enabled():
+        fast_A, fast_B = want_A and _fast_grad(x), want_B and _fast_grad(dy)
+        dA = dB = None
+        if fast_A or fast_B:
             dA, dB = ext().lora_grads(
-                *((x.contiguous(), du.contiguous()) if want_A else (None, None)),
-                *((dy, u.contiguous()) if want_B else (None, None)))
-        else:
-            dA, dB = (a.t() @ b if want else None
-                      for a, b, want in ((du, x, want_A), (dy, u, want_B)))
+                *((x.contiguous(), du.contiguous()) if fast_A else (None, None)),
+                *((dy, u.contiguous()) if fast_B else (None, None)))
+        if want_A and not fast_A:
+            dA = du.t() @ x
+        if want_B and not fast_B:
+            dB = dy.t() @ u
         return dx, None, None, dA if want_A else None, dB if want_B else None, None, None
 
 

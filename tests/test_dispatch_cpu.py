@@ -80,3 +80,13 @@ def test_gated_products_fuse_where_their_tiles_fill_the_gpu():
         assert glu_fills(M, I, K)
     for M, I, K in [(512, 1024, 1536), (1024, 2240, 1536), (600, 11008, 2048)]:
         assert not glu_fills(M, I, K)
+
+
+def test_adapter_gradients_take_the_kernel_by_columns_and_rows():
+    from nanorlhf_amd.ops.lora import _fast_grad
+    z = torch.empty(1, dtype=torch.bfloat16)
+    with torch.no_grad():
+        assert _fast_grad(z.expand(50000, 17920)) and _fast_grad(z.expand(240, 37888))
+        assert not _fast_grad(z.expand(4096, 37888)) and not _fast_grad(z.expand(64, 36))
+        assert not _fast_grad(z.float().expand(64, 64))
+    assert not _fast_grad(z.expand(64, 64))            # a recorded backward
