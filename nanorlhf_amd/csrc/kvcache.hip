@@ -283,8 +283,8 @@ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
                          const int* __restrict__ seq_lens,
                          short* __restrict__ out,        // [B, Hq, DV]
                          float* __restrict__ part, float* __restrict__ ms,
-                         int Hq, int Hkv, int maxP, int Gq, int per_split, float scale,
-                         DecodeExt ext) {
+                         int Hq, int Hkv, int maxP, int Gq, int per_split, int splits,
+                         float scale, DecodeExt ext) {
   constexpr int NC = D / 32, NT = DV / 16;
   constexpr bool FP8 = sizeof(CT) == 1;
   const int unit = EXT ? blockIdx.x / ext.gchunks : blockIdx.x;
@@ -296,7 +296,7 @@ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
   // a length past its page table (whose last page is then read again) may have more
   // tiles than the splits were made for: the last takes them
   const int it0 = blockIdx.y * per_split;
-  const int it1 = blockIdx.y + 1 == gridDim.y ? tr.n : min(tr.n, it0 + per_split);
+  const int it1 = (int)blockIdx.y + 1 == splits ? tr.n : min(tr.n, it0 + per_split);
   if (blockIdx.y > 0 && it0 >= tr.n) return;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -454,11 +454,11 @@ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
       o0 += Lacc[w][g * LD + d] * c;
       o1 += Lacc[w][g * LD + d + 1] * c;
     }
-    if (gridDim.y == 1 || tr.n <= per_split) {      // nothing to merge
+    if (splits == 1 || tr.n <= per_split) {      // nothing to merge
       const float inv = S > 0.f ? 1.f / S : 0.f;
       write_pair<EXT>(out, o0 * inv, o1 * inv, b, h0 + g, d, Hq, DV, ext);
     } else {
-      const long row = ((long)blockIdx.x * gridDim.y + blockIdx.y) * 16 + g;
+      const long row = ((long)blockIdx.x * splits + blockIdx.y) * 16 + g;
       *reinterpret_cast<float2*>(part + row * DV + d) = make_float2(o0, o1);
       if (d == 0) *reinterpret_cast<float2*>(ms + row * 2) = make_float2(M, S);
     }
@@ -567,7 +567,7 @@ torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor k_cache,
                        (const short*)q.data_ptr(), (const CT*)k_cache.data_ptr(), \
                        (const CT*)v_cache.data_ptr(), block_tables.data_ptr<int>(), \
                        seq_lens.data_ptr<int>(), (short*)out.data_ptr(), part, ms, \
-                       Hq, Hkv, maxP, G, sp.per, (float)scale, DecodeExt{});    \
+                       Hq, Hkv, maxP, G, sp.per, sp.n, (float)scale, DecodeExt{}); \
     if (sp.n > 1)                                                               \
       hipLaunchKernelGGL((paged_decode_merge_kernel<DD, false>), dim3(B * Hkv, G), dim3(64), 0, \
                          stream, part, ms, seq_lens.data_ptr<int>(), (short*)out.data_ptr(), \
@@ -627,7 +627,7 @@ void paged_attn_decode_window(torch::Tensor q, torch::Tensor k_cache, torch::Ten
                        (const short*)q.data_ptr(), (const short*)k_cache.data_ptr(),       \
                        (const short*)v_cache.data_ptr(), block_tables.data_ptr<int>(),     \
                        seq_lens.data_ptr<int>(), (short*)out.data_ptr(), part, ms, Hq, Hkv, \
-                       maxP, G, sp.per, (float)scale, e);                                  \
+                       maxP, G, sp.per, sp.n, (float)scale, e);                            \
     if (sp.n > 1)                                                                          \
       hipLaunchKernelGGL((paged_decode_merge_kernel<VV, true>), dim3(units, std::min(G, 16)), \
                          dim3(64), 0, stream, part, ms, seq_lens.data_ptr<int>(),          \
