@@ -21,11 +21,11 @@
 // conversion per score, and the fragments' addresses) and LDS reads (16 KB of
 // fragments per 32 x 32 scores and two products); two waves per SIMD overlap the
 // three.  5 causal sequences of about 6500 tokens, 12 heads over 2, width 128:
-// forward 0.89 ms (950 TFLOP/s), backward 2.75 ms; before, with V transposed by
-// scalar LDS writes, 2.9 ms, and with dq added up by float atomics over 32-row kv
-// tiles, 21.5 ms for the backward.  Twice the rows per wave (half the LDS reads, one
-// wave per SIMD) was slower everywhere, and so were chiplets that take whole heads
-// of one sequence after the other.
+// forward 0.90 to 1.02 ms (830 to 940 TFLOP/s), backward 2.9; before, with V
+// transposed by scalar LDS writes, 2.9 ms, and with dq added up by float atomics over
+// 32-row kv tiles, 21.5 ms for the backward.  Twice the rows per wave (half the LDS
+// reads, one wave per SIMD) was slower everywhere, and so were chiplets that take whole
+// heads of one sequence after the other.
 //
 // Products contract over the MFMA's k index in any order as long as both
 // operands agree.  The C layout gives a lane the rows {0-3, 8-11} + 4 * half of
@@ -512,8 +512,8 @@ std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
   // A workgroup of dk and dv walks the group's q heads one after the other.
   // Where that leaves too few to fill 256 CUs twice, with spare to even out
   // causal tiles, they are divided among `parts`.  Whole backward, 12 heads over
-  // 2: 5 x 6500 tokens (518 workgroups undivided) 4.23 ms with 1 part, 3.15 with
-  // 2, 3.07 with 3; 56 x 870 (872) 0.77 with 1, 0.81 with 2, 0.95 with 6.
+  // 2: 5 x 6500 tokens (518 workgroups undivided) 3.95 ms with 1 part, 2.92 with
+  // 2, 2.87 with 3; 56 x 870 (872) 0.72 with 1, 0.77 with 2, 0.89 with 6.
   int parts = 1;
   const long tiles = (T / ROWS + B) * Hkv;
   while (parts < G && (G % parts || tiles * parts < 768)) parts++;

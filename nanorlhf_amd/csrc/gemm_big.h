@@ -12,8 +12,8 @@
 // For grids that fill most of the chip with one workgroup per CU.  Twice the
 // reuse of the 128-tile in both directions, LDS tiles without bank conflicts, the
 // next step's fragments read between the products, 16 neighbouring columns of y
-// per lane.  48720 x 17920 x 1536 + 64: 2.70 ms (1033 TFLOP/s) against 3.80, x 1536
-// x 17920: 2.37 (1136) against 3.30; 59% of the cycles are products, the rest
+// per lane.  48720 x 17920 x 1536 + 64: 2.65 ms (1056 TFLOP/s) against 3.80, x 1536
+// x 17920: 2.36 (1142) against 3.30; 59% of the cycles are products, the rest
 // mostly waits at the tiles' barriers.  Four stages of 32 that land a barrier
 // ahead (974 TFLOP/s: rows of 64 bytes double the requests), 256 x 128 tiles twice
 // per CU (870) and four waves of 128 x 128 (999) were slower.

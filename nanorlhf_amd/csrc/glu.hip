@@ -3,9 +3,9 @@
 // widths) and a pass over their results took three trips through memory for what
 // is written once here.
 //
-// The tile is gemm_big.h's, and so are its bounds.  16320 x 8960 x 1536: 0.79 ms
-// (1140 TFLOP/s), where the library's product of both widths took 0.66 and the pass
-// 0.19; 4096 x 4096 x 1024 0.062 against 0.081.
+// The tile is gemm_big.h's, and so are its bounds.  16320 x 8960 x 1536: 0.80 ms
+// (1120 TFLOP/s; 0.86 between a prompt's other kernels), where the library's product of
+// both widths takes 0.70 and the pass 0.16; 4096 x 4096 x 1024 0.062 against 0.077.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 

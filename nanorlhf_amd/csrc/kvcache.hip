@@ -513,7 +513,7 @@ void paged_decode_merge_kernel(const float* __restrict__ part, const float* __re
 // per sequence read 32 x 2000 tokens (12 heads over 2, bf16) in 17.4 us with the
 // merge, two in 22.5, eight in 22.4 (the first tile's page, key and value
 // latencies then outweigh the rest); unsplit it took 135.  At 256 sequences and
-// more nothing is split: 2048 x 850 in fp8 take 172 us, 5.1 TB/s.  Nor is a short
+// more nothing is split: 2048 x 850 in fp8 take 169 us, 5.3 TB/s.  Nor is a short
 // context, whose walk costs no more than the merge (in fp8: 64 x 170 tokens, 9
 // tiles, 5.6 us against 7.5, 8 x 400, 19 tiles, 7.1 against 7.5; from 21 tiles on in
 // bf16 9.5 against 8.5), nor a batch of which

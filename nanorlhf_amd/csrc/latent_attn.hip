@@ -90,10 +90,11 @@ DEVINL int page_swz(int row) {
 }
 
 // What bounds it: reading the latents, and their uneven lengths.  128 contexts of
-// about 2000 latents of 512, 12 heads: 65 us (4.3 TB/s) with two parts each, one
+// about 2000 latents of 512, 12 heads: 63 us (4.2 TB/s) with two parts each, one
 // workgroup per CU; with whole tiles of 64 tokens going through registers and
-// four barriers per tile it took 116.  Four parts took 74 us (a part costs about
-// 9 us beside its pages: first loads, sums), two waves per workgroup 67 at best.
+// four barriers per tile it took 116.  Before fragments were read ahead (72 us) four
+// parts took 9 us more than two (a part's first loads and sums), two waves per
+// workgroup 2 more.
 template <int RP>
 __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
   constexpr int NW = 4, NC = RP / 32, NT = RP / 16, CH = RP / 8;

@@ -238,7 +238,7 @@ torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
 // the MFMA's rows so that two tiles of 16 give a lane 8 neighbours: y moves in 16
 // bytes per lane and 64 per row.  All of a lane's y is asked for before the
 // product.  48720 x 17920: 2.33 ms (1.5 TB/s) with one element per access,
-// 0.81 ms now; 48720 x 1536: 0.128 to 0.053 ms (5.6 TB/s).
+// 0.77 ms now; 48720 x 1536: 0.128 to 0.052 ms (5.8 TB/s).
 // ---------------------------------------------------------------------------
 template <bool VEC>
 __launch_bounds__(256, 3)

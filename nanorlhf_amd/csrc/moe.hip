@@ -250,8 +250,8 @@ __global__ __launch_bounds__(256, 2) void grouped_tiles_kernel(Grouped a, int ti
 // waves share the depth: each walks 64 elements at a time of its own part, which
 // direct loads bring into a ring of its own in LDS, whole 128-byte lines, without
 // barriers, and they add up through LDS.  16 experts of 1536 x 2240, 32 tokens with 4
-// each: gate and up 36 us (6.1 TB/s), down 20.5; 128 tokens 50 and 26.  Fragments
-// loaded straight into registers, half a line at a time: 41 and 27, 102 and 52.
+// each: gate and up 43 us (5.1 TB/s), down 23; 128 tokens 61 and 31.  Fragments
+// loaded straight into registers, half a line at a time: 56 and 33, 129 and 65.
 template <int MF, int NF, int WAVES, int R, bool GLU>
 __global__ __launch_bounds__(WAVES * 64) void grouped_stream_kernel(Grouped a) {
   int g, m0, rows;
