@@ -59,11 +59,17 @@ def _time_cuda(fn, reps: int = 3) -> float:
     return s.elapsed_time(e) / reps
 
 
+def _capturing(x) -> bool:
+    return x.is_cuda and torch.cuda.is_current_stream_capturing()
+
+
 def _choose_strategy(x, w, u, b, bias) -> str:
     N, K = int(w.size(0)), int(w.size(1))
     known = _TUNE.setdefault((N, K), {})
     key = (ext().lora_gemm_big(x.shape[0], N, K), bias is not None, x.device)
     st = known.get(key)
+    if st is None and known and _capturing(x):
+        return next(iter(known.values()))       # nothing can be timed now
     if st is None:
         t_fused = _time_cuda(lambda: ext().lora_gemm(x, w, u, b, bias))
 

@@ -65,6 +65,21 @@ def test_adapter_strategies_are_kept_by_what_the_kernels_depend_on(monkeypatch):
     assert next(times, None) is None and len(lora._TUNE[64, 64]) == 3
 
 
+def test_a_capture_takes_the_strategy_that_is_known_of_its_weight(monkeypatch):
+    from types import SimpleNamespace
+    from nanorlhf_amd.ops import lora
+    monkeypatch.setattr(lora, "_TUNE", {})
+    monkeypatch.setattr(lora, "ext", lambda: SimpleNamespace(
+        lora_gemm_big=lambda M, N, K: M > 1000, lora_gemm=None, lora_add_=None))
+    times = iter([3.0, 1.0])
+    monkeypatch.setattr(lora, "_time_cuda", lambda fn: next(times))
+    w = torch.zeros(64, 64)
+    assert lora._choose_strategy(torch.zeros(240, 64), w, None, None, None) == "epilogue"
+    monkeypatch.setattr(lora, "_capturing", lambda x: True)
+    assert lora._choose_strategy(torch.zeros(4000, 64), w, None, None, None) == "epilogue"
+    assert len(lora._TUNE[64, 64]) == 1         # and leaves the timing for later
+
+
 def test_linears_of_few_rows_leave_what_the_library_does_faster():
     from nanorlhf_amd.ops.linear import rows_pay
     for M, N, K in [(1, 1536, 1536), (64, 16384, 2048), (32, 32768, 1536), (16, 18944, 1536),
