@@ -5,29 +5,15 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <ATen/hip/HIPContext.h>
+
+#include <type_traits>
 
 #include "common.h"
 
-// ---- 256 x 256 tile, 8 waves -----------------------------------------------
-// For grids that fill most of the chip with one workgroup per CU.  Twice the
-// reuse of the 128-tile in both directions, LDS tiles without bank conflicts, the
-// next step's fragments read between the products, 16 neighbouring columns of y
-// per lane.  48720 x 17920 x 1536 + 64: 2.65 ms (1056 TFLOP/s) against 3.80, x 1536
-// x 17920: 2.36 (1142) against 3.30; 59% of the cycles are products, the rest
-// mostly waits at the tiles' barriers.  Four stages of 32 that land a barrier
-// ahead (974 TFLOP/s: rows of 64 bytes double the requests), 256 x 128 tiles twice
-// per CU (870) and four waves of 128 x 128 (999) were slower.
 typedef __bf16 bf16x8_m __attribute__((ext_vector_type(8)));
 
 constexpr int BIG = 256;
-
-// 16-byte chunk exchange (xor) of a tile row: rows are 128 bytes apart, so two
-// fill the banks.  Fragments take 16 rows in order from x, and from w rows
-// 0-3, 16-19, 4-7, 20-23 (see wrow).
-DEVINL int xswz(int row) { return (row >> 1) & 7; }
-DEVINL int wswz(int row) { return ((row >> 1) & 3) | ((row >> 4) & 1) << 2; }
-// the MFMA's row i of 32 is y's column wrow(i): a lane then holds 16 neighbours
-DEVINL int wrow(int i) { return 16 * ((i >> 2) & 1) + (i & 3) + 4 * (i >> 3); }
 
 // ACT: a tile has 128 columns of y; of every 64 rows of its w tile the first half is
 // w's and the second the same columns of w2, and y = act(x w) * (x w2).
@@ -39,135 +25,371 @@ DEVINL float glu(float g, float up) {
   return g * __builtin_amdgcn_rcpf(1.f + __expf(-z)) * up;      // gelu_tanh: x sigmoid(2 ..)
 }
 
+struct Big {
+  const short *x, *w;            // [M, K], [N, K]
+  const short *u, *b;            // [M, 64], [N, 64]
+  const float* bias;
+  const short* w2;               // as w
+  short* y;
+  long ldy;
+  int M, N, K, grid_m, grid_n;
+  int whole, parts, units;       // tiles that are one unit of work, and units of the others
+};
+
+DEVINL void load_big(const void* base, unsigned offset, unsigned at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               ::"s"(at), "v"(offset), "s"(in_sgprs(base)) : "memory");
+}
+
+// One workgroup of 8 waves per CU walks over tiles; a wave has 128 rows and 64 columns
+// (or both weights' 32).  The two halves of the workgroup are half a phase apart: on every
+// SIMD one wave's 16 products run while the other one reads LDS and asks for memory,
+// and then they change places at a barrier.  A phase is a quarter of the wave's tile
+// and one step of 64 of the depth: x's rows and w's columns in halves, of which one
+// changes from phase to phase; what a phase multiplies was read a phase earlier.  LDS has
+// two steps, in quarters of 16 KB that are asked for again as soon as their last reader is
+// two phases away, so that a load has a whole step's time.
+//
+// Products are 16x16x32: by themselves they reach 1.88 PFLOP/s on normally distributed
+// data, 32x32x16 1.64 (the part runs into its power, and those move twice as much of the
+// sums).  x is the first operand and w's rows are dealt to LDS so that a lane
+// ends up with 4 neighbouring columns of y and 16 lanes with 128 bytes: stores of 16 bytes
+// to 64 rows' quarter lines cost up to 10%.  They leave past the caches' keeping,
+// for y is larger than those.  The next tile's first two steps are asked
+// for before the stores.
+//
+// 8192 x 8192 x 8192: 0.71 ms (1530 TFLOP/s), 48720 x 17920 x 1536 + 64: 2.13 (1310),
+// 48720 x 1536 x 8960 + 64: 1.01 (1340).  Lockstep waves that all read, then all
+// multiply 32x32x16, a barrier a step: 0.88 (1250), 2.70 (1030), 1.21 (1120).
 template <bool HAS_LORA, bool HAS_BIAS, bool VEC, int ACT>
-__global__ __launch_bounds__(512, 2)
-void gemm_big_kernel(const short* __restrict__ x, const short* __restrict__ w,
-                     const short* __restrict__ u, const short* __restrict__ b,
-                     const float* __restrict__ bias, const short* __restrict__ w2,
-                     short* __restrict__ y, long ldy, int M, int N, int K1, int grid_m,
-                     int grid_n) {
+__global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
   constexpr int TN = ACT ? BIG / 2 : BIG;
-  __shared__ __attribute__((aligned(16))) short lds[2][2][BIG * 64];   // [buffer][x, w]
-  int wg = blockIdx.x;
-  {
-    const int nwg = gridDim.x, q = nwg >> 3, r = nwg & 7;
-    const int xcd = wg & 7, i = wg >> 3;
-    wg = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + i;
-  }
-  constexpr int GM = 8;       // tiles that run together share rows and columns
-  const int group = wg / (GM * grid_n), first = group * GM;
-  const int rows_here = min(GM, grid_m - first);
-  const int bm = first + (wg - group * GM * grid_n) % rows_here;
-  const int bn = (wg - group * GM * grid_n) / rows_here;
-  const int m0 = bm * BIG, n0 = bn * TN;
+  constexpr int STORES = ACT ? 16 : 32;                                // of a wave and whole tile
+  constexpr int STEP = BIG * 128;                                      // bytes
+  __shared__ __attribute__((aligned(16))) short lds[2][2][BIG * 64];   // x's two steps, w's
+  __shared__ float biases[2][HAS_BIAS ? 2 * BIG : 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = (wid >> 2) * 128, wn = (wid & 3) * 64;
-  const int lo = lane & 31, hi = lane >> 5;
-  const int n_k1 = K1 >> 6, n_kt = n_k1 + (HAS_LORA ? 1 : 0);
+  const int wn = (wid & 3) * 64;
+  const int n_k1 = p.K >> 6, n_kt = n_k1 + (HAS_LORA ? 1 : 0);
 
-  // thread's rows of a tile: tid / 8 + 64 i; its chunk of each the same
+  // unit `at`: the tile's place, and which rows of it
+  int m0, n0, parts;
+  auto place = [&](int at) {
+    int wg = at, part = 0;
+    parts = 1;
+    if (at >= p.whole) {
+      parts = p.parts;
+      wg = p.whole + (at - p.whole) / parts;
+      part = (at - p.whole) % parts;
+    }
+    const int nwg = p.grid_m * p.grid_n, q = nwg >> 3, r = nwg & 7;
+    const int xcd = wg & 7, i = wg >> 3;
+    wg = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + i;
+    constexpr int GM = 8;       // tiles that run together share rows and columns
+    const int group = wg / (GM * p.grid_n), first = group * GM;
+    const int rows_here = min(GM, p.grid_m - first);
+    m0 = (first + (wg - group * GM * p.grid_n) % rows_here) * BIG + part * (BIG / parts);
+    n0 = (wg - group * GM * p.grid_n) / rows_here * TN;
+  };
+
+  // what follows from the lane, made again where it is needed: kept over the loop it
+  // would cost the loop's registers
+  auto fresh_tid = [&] {
+    int t = tid;
+    asm volatile("" : "+v"(t));
+    return t;
+  };
+  // A quarter is 128 rows of LDS: of x rows 0-63 and 128-191 (or 64 on), of w rows 0-31,
+  // 64-95, .. (or 32 on); a thread has one 16-byte chunk of two of them.  Chunks are
+  // exchanged (xor) by row pair, for two rows fill the banks.  Of a part of a tile only
+  // x's first half is there, 128 / parts rows for each half of the workgroup.
   unsigned xo[4], wo[4];
-  auto offsets = [&](int ld) {
-    const int r = tid >> 3;
+  auto x_offsets = [&](int ld) {
+    const int t = fresh_tid(), r = t >> 3, c = ((t & 7) ^ (r >> 1 & 7)) << 3;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      xo[i] = (unsigned)(min(r + 64 * i, M - 1 - m0) * ld + (((tid & 7) ^ xswz(r)) << 3)) * 2;
-      const int n = ACT ? (r & 31) + 32 * i : r + 64 * i;
-      wo[i] = (unsigned)(min(n, N - 1 - n0) * ld + (((tid & 7) ^ wswz(r)) << 3)) * 2;
+    for (int h = 0; h < 4; h++) {
+      const int m = parts == 1 ? r + 64 * (h >> 1) + 128 * (h & 1)
+                               : min(r, 128 / parts - 1) + 128 / parts * (h & 1);
+      xo[h] = (unsigned)(min(m, max(p.M - 1 - m0, 0)) * ld + c) * 2;
     }
   };
-  offsets(K1);
-  const short *xb = x + (long)m0 * K1, *wb = (ACT && wid >= 4 ? w2 : w) + (long)n0 * K1;
-  auto stage = [&](int kt, int buf) {
-    const short *xs = xb + kt * 64, *ws = wb + kt * 64;
-    if (HAS_LORA && kt == n_k1) {
-      offsets(64);
-      xs = u + (long)m0 * 64;
-      ws = b + (long)n0 * 64;
+  // LDS row 16 t + l of 64 is column 4 l + t, or 2 l + t % 2 of w (t < 2) or w2
+  auto w_offsets = [&](int ld) {
+    const int t = fresh_tid(), r = t >> 3 & 31, l = r & 15;
+    const int c = ((t & 7) ^ (r >> 1 & 7)) << 3;
+#pragma unroll
+    for (int h = 0; h < 4; h++) {
+      const int n = ACT ? 2 * l + (r >> 4) + (t >> 8) * 32 + 64 * (h & 1)
+                        : 4 * l + (r >> 4) + 2 * (h >> 1) + (t >> 8) * 64 + 128 * (h & 1);
+      wo[h] = (unsigned)(min(n, p.N - 1 - n0) * ld + c) * 2;
     }
-#pragma unroll
-    for (int i = 0; i < 4; i++) load_to_lds16(xs, xo[i], &lds[buf][0][(i * 512 + wid * 64) * 8]);
-#pragma unroll
-    for (int i = 0; i < 4; i++) load_to_lds16(ws, wo[i], &lds[buf][1][(i * 512 + wid * 64) * 8]);
   };
-  const int xr = wm + lo, wr = wn + wrow(lo);
-  auto xfrag = [&](int buf, int mt, int ks) {
-    return *reinterpret_cast<const bf16x8_m*>(
-        &lds[buf][0][(xr + 32 * mt) * 64 + (((2 * ks + hi) ^ xswz(xr)) << 3)]);
+  const short *xb, *wb, *w2b, *ub, *bb;
+  const unsigned base =
+      (unsigned)(size_t)(const __attribute__((address_space(3))) short*)&lds[0][0][0];
+  const unsigned xat = base + wid * 1024, wat = base + 2 * STEP + ((wid & 3) * 8 + (wid >> 2) * 64) * 128;
+  auto load_x = [&](int kt, int h) {
+    if (HAS_LORA && kt == n_k1 && h == 0) x_offsets(64);
+    const short* src = HAS_LORA && kt == n_k1 ? ub : xb + kt * 64;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      load_big(src, xo[2 * h + i], xat + (kt & 1) * STEP + (64 * h + 128 * i) * 128);
   };
-  auto wfrag = [&](int buf, int nt, int ks) {
-    return *reinterpret_cast<const bf16x8_m*>(
-        &lds[buf][1][(wr + 32 * nt) * 64 + (((2 * ks + hi) ^ wswz(wr)) << 3)]);
+  auto load_w = [&](int kt, int h, bool first) {
+    if (HAS_LORA && kt == n_k1 && first) w_offsets(64);
+    const short* src = HAS_LORA && kt == n_k1 ? bb : (h ? w2b : wb) + kt * 64;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      load_big(src, wo[2 * h + i], wat + (kt & 1) * STEP + (32 * h + 128 * i) * 128);
+  };
+  int side = 0;
+  auto begin = [&] {            // the first two steps of the unit at m0, n0
+    x_offsets(p.K);
+    w_offsets(p.K);
+    const int row = min(m0, p.M - 1);     // a part of the last tile may have none
+    xb = p.x + (long)row * p.K;
+    wb = p.w + (long)n0 * p.K;
+    w2b = ACT ? p.w2 + (long)n0 * p.K : wb;
+    if (HAS_LORA) {
+      ub = p.u + (long)row * 64;
+      bb = p.b + (long)n0 * 64;
+    }
+    if (HAS_BIAS)
+      load_to_lds4(p.bias, (unsigned)min(n0 + wn + lane, p.N - 1) * 4, &biases[side][wid * 64]);
+    load_x(0, 0);
+    load_w(0, 0, true);
+    load_w(0, 1, false);
+    load_x(0, 1);
+    if (n_kt > 1) {
+      load_x(1, 0);
+      load_w(1, 1, true);
+      load_w(1, 0, false);
+      load_x(1, 1);
+    }
   };
 
-  f32x16 acc[4][2];
+  unsigned xa[2], wa[2];        // of each 32 of a step's depth
 #pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++) acc[i][j] = f32x16{};
-
-  stage(0, 0);
-  for (int kt = 0; kt < n_kt; kt++) {
-    const int buf = kt & 1;
-    wait_loads<0>();
-    __syncthreads();
-    bf16x8_m xf[2][4], wf[2][2];
-    auto read = [&](int ks) {
-#pragma unroll
-      for (int j = 0; j < 2; j++) wf[ks & 1][j] = wfrag(buf, j, ks);
-#pragma unroll
-      for (int i = 0; i < 4; i++) xf[ks & 1][i] = xfrag(buf, i, ks);
-    };
-    read(0);
-    if (kt + 1 < n_kt) stage(kt + 1, buf ^ 1);
-    // the next step's fragments are read between this one's products
-#pragma unroll
-    for (int ks = 0; ks < 4; ks++) {
-      if (ks < 3) read(ks + 1);
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[ks & 1][j], xf[ks & 1][i],
-                                                              acc[i][j], 0, 0, 0);
-#pragma unroll
-      for (int g = 0; g < 6; g++) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // product
-        if (ks < 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);      // LDS read
-      }
-      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-    }
+  for (int ks = 0; ks < 2; ks++) {
+    const int lo = lane & 15, hi = lane >> 4, xr = (wid >> 2) * 128 + lo, wr = wn + lo;
+    xa[ks] = base + xr * 128 + (((4 * ks + hi) ^ (xr >> 1 & 7)) << 4);
+    wa[ks] = base + 2 * STEP + wr * 128 + (((4 * ks + hi) ^ (wr >> 1 & 7)) << 4);
   }
-  // lane: row m0 + wm + 32 i + lo, columns n0 + wn + 32 j + 16 hi + 0..15
+  auto lds_frag = [](unsigned at) {
+    typedef __attribute__((address_space(3))) const char* lds_bytes;
+    typedef __attribute__((address_space(3))) const bf16x8_m* lds_m;
+    return *(lds_m)((lds_bytes)0 + at);
+  };
+  bf16x8_m xf[2][2][4], wf[2][2][2];       // [half][32 of the depth][tile]
+  f32x4 acc[8][2][2];                      // [tile of rows][half of the columns][tile]
+  auto read_x = [&](int buf, int h, int ks, int t) {
+    xf[h][ks][t] = lds_frag(xa[ks] + buf * STEP + (4 * h + t) * 2048);
+  };
+  auto read_w = [&](int buf, int h) {
 #pragma unroll
-  for (int j = 0; j < (ACT ? 1 : 2); j++) {
-    const int gn = n0 + (ACT ? wn / 2 : wn + 32 * j) + 16 * hi;
-    float bv[16];
-    if (HAS_BIAS) {
+    for (int e = 0; e < 4; e++)
+      wf[h][e >> 1][e & 1] = lds_frag(wa[e >> 1] + buf * STEP + h * 4096 + (e & 1) * 2048);
+  };
+  auto barrier = [&] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto products = [&](int h, int j) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int r = 0; r < 16; r++) bv[r] = bias[min(gn + r, N - 1)];
+    for (int t2 = 0; t2 < 4; t2 += 2) {
+      if ((4 * h + t2) * parts >= 8) continue;
+#pragma unroll
+      for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+        for (int t = t2; t < t2 + 2; t++)
+#pragma unroll
+          for (int e = 0; e < 2; e++)
+            acc[4 * h + t][j][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                xf[h][ks][t], wf[j][ks][e], acc[4 * h + t][j][e], 0, 0, 0);
     }
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    barrier();
+  };
+  // Step kt of the depth.  F: which of w's halves comes first (the one that the step
+  // before had last), FIRST: the last tile's stores may be under way.  The waits are
+  // for the quarter that is read next, and leave the younger ones' loads (and stores) be.
+  auto step = [&](auto f, auto is_first, int kt) {
+    constexpr int F = decltype(f)::value, S = 1 - F;
+    constexpr bool FIRST = decltype(is_first)::value;
+    constexpr int E = FIRST ? STORES : 0;
+    const bool more = kt + 2 < n_kt, next = kt + 1 < n_kt;
+    read_w(F, S);
+    read_x(F, 1, 0, 0);
+    read_x(F, 1, 0, 1);
+    if (!FIRST && next) load_x(kt + 1, 1);
+    barrier();
+    products(0, F);
+
+    read_x(F, 1, 0, 2);
+    read_x(F, 1, 0, 3);
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int gm = m0 + wm + 32 * i + lo;
-      if (gm >= M) continue;
-      short* dst = y + gm * ldy + gn;
+    for (int t = 0; t < 4; t++) read_x(F, 1, 1, t);
+    if (more) {
+      load_x(kt + 2, 0);
+      wait_loads<8 + E>();
+    } else {
+      wait_loads<6 + E>();
+    }
+    barrier();
+    products(0, S);
+
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        s16x8 o;
+    for (int t = 0; t < 4; t++) read_x(S, 0, 0, t);
+    read_x(S, 0, 1, 0);
+    read_x(S, 0, 1, 1);
+    if (more) {
+      load_w(kt + 2, F, true);
+      wait_loads<8 + E>();
+    } else {
+      wait_loads<4 + E>();
+    }
+    barrier();
+    products(1, S);
+
+    read_x(S, 0, 1, 2);
+    read_x(S, 0, 1, 3);
+    read_w(S, S);
+    if (more) {
+      load_w(kt + 2, S, false);
+      wait_loads<6 + E>();
+    } else {
+      wait_loads<E>();
+    }
+    barrier();
+    products(1, F);
+  };
+  typedef std::integral_constant<int, 0> Zero;
+  typedef std::integral_constant<int, 1> One;
+
+  place(blockIdx.x);
+  begin();
+  wait_loads<0>();
+  for (int at = blockIdx.x;;) {
+    if (n_kt > 1) wait_loads<8 + STORES>();
+    else wait_loads<STORES>();
+    barrier();
 #pragma unroll
-        for (int r = 0; r < 8; r++)
-          o[r] = f2bf(ACT ? glu<ACT>(acc[i][0][8 * h + r], acc[i][1][8 * h + r])
-                          : acc[i][j][8 * h + r] + (HAS_BIAS ? bv[8 * h + r] : 0.f));
-        if (VEC) {
-          if (gn + 8 * h < N) *reinterpret_cast<s16x8*>(dst + 8 * h) = o;
-        } else {
+    for (int i = 0; i < 8; i++)
 #pragma unroll
-          for (int r = 0; r < 8; r++)
-            if (gn + 8 * h + r < N) dst[8 * h + r] = o[r];
+      for (int j = 0; j < 4; j++) acc[i][j >> 1][j & 1] = f32x4{};
+#pragma unroll
+    for (int t = 0; t < 8; t++) read_x(0, 0, t >> 2, t & 3);
+    read_w(0, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (wid >= 4) barrier();
+    step(Zero(), std::true_type(), 0);
+    for (int kt = 1; kt < n_kt; kt += 2) {
+      step(One(), std::false_type(), kt);
+      if (kt + 1 < n_kt) step(Zero(), std::false_type(), kt + 1);
+    }
+    if (wid < 4) barrier();
+
+    const int m1 = m0, n1 = n0, parts1 = parts, side1 = side;
+    at += gridDim.x;
+    const bool another = at < p.units;
+    if (another) {
+      place(at);
+      side ^= 1;
+      begin();
+    }
+    // lane: row 16 i + 4 hi + r of its half's, columns 4 (2) lo + 0 .. of the wave's
+    const int t = fresh_tid() & 63, lo = t & 15, hi = t >> 4;
+    const int gm0 = m1 + (wid >> 2) * (128 / parts1) + 4 * hi;
+    if constexpr (ACT == NO_ACT) {
+      const int gn = n1 + wn + 4 * lo;
+      float bv[4];
+      if (HAS_BIAS) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) bv[c] = biases[side1][(wid >> 2) * BIG + wn + 4 * lo + c];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        if (i * parts1 >= 8) continue;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int gm = gm0 + 16 * i + r;
+          float v[4];
+#pragma unroll
+          for (int c = 0; c < 4; c++) v[c] = acc[i][c >> 1][c & 1][r] + (HAS_BIAS ? bv[c] : 0.f);
+          if (gm >= p.M) continue;
+          short* dst = p.y + gm * p.ldy + gn;
+          if (VEC) {
+            typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+            if (gn < p.N)
+              __builtin_nontemporal_store(u32x2{pack2bf(v[0], v[1]), pack2bf(v[2], v[3])},
+                                          reinterpret_cast<u32x2*>(dst));
+          } else {
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+              if (gn + c < p.N) dst[c] = f2bf(v[c]);
+          }
+        }
+      }
+    } else {
+      // neighbouring lanes exchange a row, so that each has 4 columns of one
+      const bool odd = lo & 1;
+      const int gn = n1 + wn / 2 + 2 * lo;
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        if (i * parts1 >= 8) continue;
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+          float v[2][2];
+#pragma unroll
+          for (int q = 0; q < 2; q++)
+#pragma unroll
+            for (int c = 0; c < 2; c++)
+              v[q][c] = glu<ACT>(acc[i][0][c][r + q], acc[i][1][c][r + q]);
+          if (VEC) {
+            typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+            const unsigned a = pack2bf(v[0][0], v[0][1]), b = pack2bf(v[1][0], v[1][1]);
+            const unsigned mine = odd ? b : a;
+            const unsigned other = __builtin_amdgcn_mov_dpp(odd ? a : b, 0xb1, 0xf, 0xf, true);
+            const int gm = gm0 + 16 * i + r + odd, gn4 = gn - 2 * odd;
+            if (gm < p.M && gn4 < p.N)
+              __builtin_nontemporal_store(odd ? u32x2{other, mine} : u32x2{mine, other},
+                                          reinterpret_cast<u32x2*>(p.y + gm * p.ldy + gn4));
+          } else {
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+#pragma unroll
+              for (int c = 0; c < 2; c++)
+                if (gm0 + 16 * i + r + q < p.M && gn + c < p.N)
+                  p.y[(gm0 + 16 * i + r + q) * p.ldy + gn + c] = f2bf(v[q][c]);
+          }
         }
       }
     }
+    if (!another) break;
+    // a wave that stored less cannot count on its stores in the waits
+    if (!VEC || parts1 > 1 || m1 + BIG > p.M || n1 + TN > p.N) wait_loads<0>();
   }
+}
+
+// The tiles that are left after whole rounds of the CUs are divided by rows where that
+// still fits one round.
+template <bool HAS_LORA, bool HAS_BIAS, bool VEC, int ACT>
+void launch_big(Big p) {
+  const int cus = at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
+  constexpr int TN = ACT ? BIG / 2 : BIG;
+  p.grid_m = (p.M + BIG - 1) / BIG;
+  p.grid_n = (p.N + TN - 1) / TN;
+  const int tiles = p.grid_m * p.grid_n, left = tiles % cus;
+  p.parts = left == 0 || left * 2 > cus ? 1 : left * 4 > cus ? 2 : 4;
+  p.whole = p.parts > 1 ? tiles - left : tiles;
+  p.units = p.whole + (tiles - p.whole) * p.parts;
+  hipLaunchKernelGGL((gemm_big_kernel<HAS_LORA, HAS_BIAS, VEC, ACT>), dim3(std::min(p.units, cus)),
+                     dim3(512), 0, c10::hip::getCurrentHIPStream(), p);
 }

@@ -3,9 +3,8 @@
 // widths) and a pass over their results took three trips through memory for what
 // is written once here.
 //
-// The tile is gemm_big.h's, and so are its bounds.  16320 x 8960 x 1536: 0.80 ms
-// (1120 TFLOP/s; 0.86 between a prompt's other kernels), where the library's product of
-// both widths takes 0.70 and the pass 0.16; 4096 x 4096 x 1024 0.062 against 0.077.
+// The tile is gemm_big.h's, and so are its bounds.  16320 x 8960 x 1536: 0.66 ms
+// (1360 TFLOP/s), where the library's product of both widths takes 0.66 and the pass 0.16.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -33,13 +32,17 @@ void glu_linear(torch::Tensor x, torch::Tensor gate, torch::Tensor up, torch::Te
   const long gm = (M + BIG - 1) / BIG, gn = (N + BIG / 2 - 1) / (BIG / 2);
   TORCH_CHECK(gm * gn < (1L << 31) && K < (1L << 22), "glu_linear: too large");
   const long ldo = out.stride(0);
-  const bool vec = N % 8 == 0 && ldo % 8 == 0 && (uintptr_t)out.data_ptr() % 16 == 0;
-#define LAUNCH(VEC, ACT)                                                                     \
-  hipLaunchKernelGGL((gemm_big_kernel<false, false, VEC, ACT>), dim3(gm * gn), dim3(512), 0, \
-                     c10::hip::getCurrentHIPStream(), (const short*)x.data_ptr(),            \
-                     (const short*)gate.data_ptr(), nullptr, nullptr, nullptr,               \
-                     (const short*)up.data_ptr(), (short*)out.data_ptr(), ldo, (int)M,       \
-                     (int)N, (int)K, (int)gm, (int)gn)
+  const bool vec = N % 4 == 0 && ldo % 4 == 0 && (uintptr_t)out.data_ptr() % 8 == 0;
+  Big p{};
+  p.x = (const short*)x.data_ptr();
+  p.w = (const short*)gate.data_ptr();
+  p.w2 = (const short*)up.data_ptr();
+  p.y = (short*)out.data_ptr();
+  p.ldy = ldo;
+  p.M = M;
+  p.N = N;
+  p.K = K;
+#define LAUNCH(VEC, ACT) launch_big<false, false, VEC, ACT>(p)
   if (act == 0) { if (vec) LAUNCH(true, SILU_GLU); else LAUNCH(false, SILU_GLU); }
   else { if (vec) LAUNCH(true, GELU_GLU); else LAUNCH(false, GELU_GLU); }
 #undef LAUNCH

@@ -13,7 +13,7 @@
 // under LoRA so Wᵀ is cached once.  The products with 64 rows or columns of
 // result are lora_grad.hip's.
 //
-// Large grids take gemm_big.h's 256-tile kernel; this file's own has a
+// More than 128 rows take gemm_big.h's 256-tile kernel; this file's own has a
 // 128×128 output tile, BK=64, 4 waves (2×2 of
 // 64×64), v_mfma_f32_16x16x32_bf16, double-buffered LDS filled by
 // global_load_lds dwordx4 (16 B/lane), one __syncthreads per K-step,
@@ -150,12 +150,18 @@ __global__ void lora_gemm_kernel(const short* __restrict__ x,
   }
 }
 
-// Whether lora_gemm takes the 256-tile kernel.  4096 x 1536 x 1536 (96 tiles of 256): 38 us
-// in big tiles, 42 in small ones; with fewer the small ones fill more of the chip.
-// From a depth of 2^22 on a big tile's 32-bit offsets come near their end.
+// Whether a product has as many tiles of 256 as tell something about still larger ones, for
+// which a product of few says nothing: what its strategy is kept by.
 bool lora_gemm_big(long M, long N, long K) {
   return ((M + BIG - 1) / BIG) * ((N + BIG - 1) / BIG) >= 96 && K < (1L << 22);
 }
+
+// Up to 128 rows leave half of every other part of a 256-tile empty: 60 x 17920 x 1536 27 us in
+// tiles of 128, 30 in large ones; 130 x 17920 x 1536 36 and 30, 500 x 8960 x 1536 36 and 29,
+// 1000 x 4864 x 896 24 and 20, 4000 x 1536 x 1536 36 and 30; equal where a few tiles wait
+// for their loads (500 x 896 x 9728 139 and 140).  From a depth of 2^22 on a big tile's
+// 32-bit offsets come near their end.
+static bool takes_big(long M, long K) { return M > 128 && K < (1L << 22); }
 
 torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
                         c10::optional<torch::Tensor> u,
@@ -197,19 +203,25 @@ torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
   const short* bp = has_lora ? (const short*)b->data_ptr() : nullptr;
   const float* biasp = has_bias ? bias_f.data_ptr<float>() : nullptr;
 
-  const int big_m = (int)((M + BIG - 1) / BIG), big_n = (int)((N + BIG - 1) / BIG);
-  if (lora_gemm_big(M, N, K1)) {
-#define LAUNCH(HL, HB, VEC)                                                               \
-  hipLaunchKernelGGL((gemm_big_kernel<HL, HB, VEC, 0>), dim3(big_m * big_n), dim3(512), 0, \
-                     stream, (const short*)x.data_ptr(), (const short*)w.data_ptr(), up, bp, \
-                     biasp, nullptr, (short*)y.data_ptr(), (long)N, (int)M, (int)N, (int)K1, big_m, big_n)
-#define LAUNCH_V(HL, HB) do { if (N % 8 == 0) LAUNCH(HL, HB, true); else LAUNCH(HL, HB, false); } while (0)
+  if (takes_big(M, K1)) {
+    Big p{};
+    p.x = (const short*)x.data_ptr();
+    p.w = (const short*)w.data_ptr();
+    p.u = up;
+    p.b = bp;
+    p.bias = biasp;
+    p.y = (short*)y.data_ptr();
+    p.ldy = N;
+    p.M = M;
+    p.N = N;
+    p.K = K1;
+#define LAUNCH_V(HL, HB) \
+  do { if (N % 4 == 0) launch_big<HL, HB, true, NO_ACT>(p); else launch_big<HL, HB, false, NO_ACT>(p); } while (0)
     if (has_lora && has_bias) LAUNCH_V(true, true);
     else if (has_lora) LAUNCH_V(true, false);
     else if (has_bias) LAUNCH_V(false, true);
     else LAUNCH_V(false, false);
 #undef LAUNCH_V
-#undef LAUNCH
     HIP_CHECK_LAST();
     return y;
   }

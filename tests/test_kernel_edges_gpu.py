@@ -516,6 +516,39 @@ def test_expanded_portions_tile_edges(DK, DV, H):
         assert rel(out[t:t + n].cpu(), want) < 0.004
 
 
+# Rounds of 256 workgroups over the tiles, and what is left: whole tiles, halves and quarters
+# of their rows, before and after whole ones, and parts that have no rows at all
+@pytest.mark.parametrize("M,N,K", [(129, 40, 64), (300, 1000, 128), (16385, 1000, 64),
+                                   (16400, 1032, 192), (9000, 2100, 128), (11000, 1530, 320),
+                                   (12033, 3001, 64), (2305, 2052, 256)])
+@pytest.mark.parametrize("lora,bias", [(True, True), (False, False)])
+def test_big_products_in_rounds_and_parts(M, N, K, lora, bias):
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=K ** -0.5)
+    u, b = (rnd(M, 64, seed=3), rnd(N, 64, seed=4, scale=0.1)) if lora else (None, None)
+    c = rnd(N, seed=5) if bias else None
+    want = x.float() @ w.float().t()
+    if lora:
+        want += u.float() @ b.float().t()
+    if bias:
+        want += c.float()
+    for _ in range(2):
+        got = ops.ext().lora_gemm(x, w, u, b, c)
+        # one rounding, 2^-9 of the value at most, and sums of 32-bit
+        assert ((got.float() - want).abs() <= want.abs() / 256 + 1e-4).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(8200, 1100, 64), (4100, 1300, 128), (5000, 1000, 192),
+                                   (2305, 1150, 320), (9300, 1002, 64)])
+def test_gated_products_in_rounds_and_parts(M, N, K):
+    x, w = rnd(M, K, seed=1), rnd(2 * N, K, seed=2, scale=K ** -0.5)
+    g, u = (x.double() @ w.double().T).split(N, 1)
+    want = torch.nn.functional.silu(g) * u
+    for _ in range(2):
+        out = torch.full((M, N), torch.nan, device=DEV, dtype=torch.bfloat16)
+        ops.serve_ext().glu_linear(x, w[:N], w[N:], out, 0)
+        assert ((out.double() - want).abs() <= want.abs() / 256 + 1e-4).all()
+
+
 # ------------------------------------------------------- gated feed-forward
 @pytest.mark.parametrize("M,N,K", [(1, 8, 64), (255, 130, 128), (257, 128, 192), (300, 1000, 64),
                                    (513, 260, 1536)])
