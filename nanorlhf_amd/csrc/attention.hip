@@ -24,8 +24,9 @@
 // forward 0.90 to 1.02 ms (830 to 940 TFLOP/s), backward 2.9; before, with V
 // transposed by scalar LDS writes, 2.9 ms, and with dq added up by float atomics over
 // 32-row kv tiles, 21.5 ms for the backward.  Twice the rows per wave (half the LDS
-// reads, one wave per SIMD) was slower everywhere, and so were chiplets that take whole
-// heads of one sequence after the other.
+// reads, one wave per SIMD) and eight waves to a workgroup (half the loads) were slower
+// everywhere; the next tile's scores under this one's exponentials, a part of two products at
+// a time, took the same time.
 //
 // Products contract over the MFMA's k index in any order as long as both
 // operands agree.  The C layout gives a lane the rows {0-3, 8-11} + 4 * half of
@@ -80,17 +81,22 @@ DEVINL void store_row(short* __restrict__ dst, const f32x16_t* acc, float mul, i
     }
 }
 
-// Workgroups are ordered by tile first, the longest walks first: a causal
-// row tile's work grows with its index, a kv tile's shrinks.
+// Which sequence, head and tile a workgroup has.  `window` heads (of whichever sequences)
+// are taken at a time, and of these tile first, the longest walks first: a causal row
+// tile's work grows with its index, a kv tile's shrinks.  Workgroups go round the chiplets,
+// of which each has its own L2, so a head stays with one if the window is a multiple of 8.
 struct Place { int seq, head, s0, len, tile; };
 template <bool LAST_FIRST>
-DEVINL Place place(const int* __restrict__ cu, int heads) {
+DEVINL Place place(const int* __restrict__ cu, int heads, unsigned window) {
+  const unsigned n = gridDim.x, tiles = gridDim.y, at = blockIdx.y * n + blockIdx.x;
+  const unsigned begin = at / (window * tiles) * window, wide = min(window, n - begin);
+  const unsigned in = at - begin * tiles, x = begin + in % wide, y = in / wide;
   Place p;
-  p.seq = blockIdx.x / heads;
-  p.head = blockIdx.x % heads;
+  p.seq = x / heads;
+  p.head = x % heads;
   p.s0 = cu[p.seq];
   p.len = cu[p.seq + 1] - p.s0;
-  p.tile = LAST_FIRST ? gridDim.y - 1 - blockIdx.y : blockIdx.y;
+  p.tile = LAST_FIRST ? tiles - 1 - y : y;
   return p;
 }
 
@@ -99,10 +105,11 @@ template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256, 2)
 void fa_fwd_kernel(const short* __restrict__ q, const short* __restrict__ k,
                    const short* __restrict__ v, const int* __restrict__ cu,
-                   short* __restrict__ o, float* __restrict__ lse, int Hq, int Hkv, float scale) {
+                   short* __restrict__ o, float* __restrict__ lse, int Hq, int Hkv, float scale,
+                   unsigned window) {
   constexpr int NDS = D / 16, NDT = D / 32;
   constexpr float THR = 11.54f;       // rescale when a row grows past 8 nats (log2 units)
-  const Place pl = place<CAUSAL>(cu, Hq);
+  const Place pl = place<CAUSAL>(cu, Hq, window);
   const int len = pl.len, h = pl.head, kvh = h / (Hq / Hkv);
   const int q0 = pl.tile * ROWS;
   if (q0 >= len) return;
@@ -245,9 +252,9 @@ void fa_bwd_dq_kernel(const short* __restrict__ dout, const short* __restrict__ 
                       const short* __restrict__ k, const short* __restrict__ v,
                       const float* __restrict__ lse2, const float* __restrict__ drow,
                       const int* __restrict__ cu, short* __restrict__ dq, long T, int Hq,
-                      int Hkv, float scale) {
+                      int Hkv, float scale, unsigned window) {
   constexpr int NDS = D / 16, NDT = D / 32;
-  const Place pl = place<CAUSAL>(cu, Hq);
+  const Place pl = place<CAUSAL>(cu, Hq, window);
   const int len = pl.len, h = pl.head, kvh = h / (Hq / Hkv);
   const int q0 = pl.tile * ROWS;
   if (q0 >= len) return;
@@ -327,9 +334,10 @@ void fa_bwd_dkv_kernel(const short* __restrict__ dout, const short* __restrict__
                        const short* __restrict__ k, const short* __restrict__ v,
                        const float* __restrict__ lse2, const float* __restrict__ drow,
                        const int* __restrict__ cu, void* __restrict__ dk,
-                       void* __restrict__ dv, long T, int Hq, int Hkv, int parts, float scale) {
+                       void* __restrict__ dv, long T, int Hq, int Hkv, int parts, float scale,
+                       unsigned window) {
   constexpr int NDS = D / 16, NDT = D / 32;
-  const Place pl = place<false>(cu, Hkv * parts);
+  const Place pl = place<false>(cu, Hkv * parts, window);
   const int len = pl.len, kvh = pl.head / parts, part = pl.head % parts;
   const int heads = Hq / Hkv / parts, h0 = kvh * (Hq / Hkv) + part * heads;
   const int kv0 = pl.tile * ROWS;
@@ -462,6 +470,20 @@ __global__ void fa_bwd_sum_kernel(const float* __restrict__ part, short* __restr
 }
 
 // ======================================================== host wrappers ==
+// Heads that workgroups are taken from at a time.  As many as fill every chiplet's 32 CUs
+// twice: what runs there together then shares the tiles that its L2 holds.  Or all, so that
+// the longest walks of all come first, which a causal grid needs to end evenly unless it is
+// several rounds of the workgroups that run at a time.  Forward, all heads / a window, us:
+// 80 x 800 not causal, 16 heads of 64 456 / 371 (70% of the tiles' requests missed the L2);
+// causal, 12 heads over 2 of 128: 56 x 870 256 / 221, 8 x 3000 354 / 280, 16 x 6000 2550 /
+// 2050, 5 x 6500 896 / 880; 3.5 rounds, 28 heads over 4, 4 x 2000 139 / 146; 2.8 rounds, 14
+// heads of 64, 20 x 1200 102 / 121.  Backward of the first 1354 / 1118.  The walks of dk and dv
+// are few and long: causal, 40 x 1200 1041 / 1291.
+static unsigned head_window(long heads, long tiles, long rounds, bool causal) {
+  if (causal && rounds < 4) return heads;
+  return 8 * std::max(64 / std::max(tiles, 1L), 1L);
+}
+
 #define FA_BY_WIDTH(CALL)                                                  \
   do {                                                                     \
     if (D == 128) { if (causal) CALL(128, true); else CALL(128, false); }  \
@@ -483,11 +505,13 @@ std::vector<torch::Tensor> fa_fwd_varlen(torch::Tensor q, torch::Tensor k,
   if (T == 0) return {o, lse};
   auto stream = at::hip::getCurrentHIPStream();
   const dim3 grid(B * Hq, (max_seqlen + ROWS - 1) / ROWS);
+  const long rounds = (T / ROWS + B) * Hq / (D > 64 ? 512 : 1024);
 #define CALL(DD, CC)                                                           \
   hipLaunchKernelGGL((fa_fwd_kernel<DD, CC>), grid, dim3(256), 0, stream,      \
                      (const short*)q.data_ptr(), (const short*)k.data_ptr(),   \
                      (const short*)v.data_ptr(), cu_seqlens.data_ptr<int>(),   \
-                     (short*)o.data_ptr(), lse.data_ptr<float>(), Hq, Hkv, (float)scale)
+                     (short*)o.data_ptr(), lse.data_ptr<float>(), Hq, Hkv, (float)scale,     \
+                     head_window(grid.x, grid.y, rounds, causal))
   FA_BY_WIDTH(CALL);
 #undef CALL
   HIP_CHECK_LAST();
@@ -524,6 +548,7 @@ std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
   void* dvp = parts > 1 ? (void*)(sums.data_ptr<float>() + parts * n) : dv.data_ptr();
   auto stream = at::hip::getCurrentHIPStream();
   const int row_tiles = (max_seqlen + ROWS - 1) / ROWS;
+  const long rounds = (T / ROWS + B) * Hq / (D > 64 ? 512 : 1024);
 #define CALL(DD, CC)                                                           \
   do {                                                                         \
     hipLaunchKernelGGL(fa_bwd_rows_kernel<DD>, dim3((T * Hq + 15) / 16), dim3(256), 0, stream, \
@@ -535,12 +560,14 @@ std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
                        (const short*)dout.data_ptr(), (const short*)q.data_ptr(), \
                        (const short*)k.data_ptr(), (const short*)v.data_ptr(), \
                        lse2, drow, cu_seqlens.data_ptr<int>(), (short*)dq.data_ptr(), \
-                       T, Hq, Hkv, (float)scale);                              \
+                       T, Hq, Hkv, (float)scale,                               \
+                       head_window(B * Hq, row_tiles, rounds, causal));        \
     hipLaunchKernelGGL((fa_bwd_dkv_kernel<DD, CC>), dim3(B * Hkv * parts, row_tiles), dim3(256), \
                        0, stream, (const short*)dout.data_ptr(),               \
                        (const short*)q.data_ptr(), (const short*)k.data_ptr(), \
                        (const short*)v.data_ptr(), lse2, drow,                 \
-                       cu_seqlens.data_ptr<int>(), dkp, dvp, T, Hq, Hkv, parts, (float)scale); \
+                       cu_seqlens.data_ptr<int>(), dkp, dvp, T, Hq, Hkv, parts, (float)scale, \
+                       head_window(B * Hkv * parts, row_tiles, 0, causal));    \
   } while (0)
   FA_BY_WIDTH(CALL);
 #undef CALL

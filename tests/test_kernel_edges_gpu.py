@@ -46,6 +46,26 @@ def test_flash_attention_tile_edges(lens, hq, hkv, d, causal):
         assert rel(got.grad, ref.grad) < FA_REL
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("hq,hkv,d", [(12, 2, 128), (20, 4, 64)])
+def test_flash_attention_windows_of_heads(hq, hkv, d, causal):
+    """Grids of several rounds, of which the last window of heads is not a whole one."""
+    from nanorlhf_amd.ops.attention import _sdpa_ref_autograd
+    lens = [1 + 37 * i % 300 for i in range(121)]
+    cu = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
+    T = sum(lens)
+    leaves = [rnd(T, h, d, seed=h).requires_grad_(True) for h in (hq, hkv, hkv)]
+    do = rnd(T, hq, d, seed=4)
+    o = ops.flash_attn_varlen(*leaves, cu, max(lens), causal=causal)
+    o.backward(do)
+    exact = [t.detach().float().requires_grad_(True) for t in leaves]
+    want = _sdpa_ref_autograd(*exact, cu.cpu(), d ** -0.5, causal=causal)
+    want.backward(do.float())
+    assert rel(o, want) < FA_REL
+    for got, ref in zip(leaves, exact):
+        assert rel(got.grad, ref.grad) < FA_REL
+
+
 @pytest.mark.parametrize("rows", [90, 38700])         # dk and dv in several parts, in one
 @pytest.mark.parametrize("d", [32, 64, 128])
 def test_flash_attention_gives_padding_no_gradient(rows, d):
