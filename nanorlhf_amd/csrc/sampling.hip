@@ -64,6 +64,7 @@ struct Row {
   const LT* p;
   int nvec, V;
   Vec8<LT> c[NV ? NV : 1];
+  float most[NV ? NV : 1];      // each one's largest element
 
   DEVINL void load() {
     if (nvec == 0) {
@@ -77,6 +78,22 @@ struct Row {
 #pragma unroll
     for (int k = 0; k < NV; k++)
       if ((int)threadIdx.x + SBLOCK * k >= nvec) fill8(c[k]);
+  }
+  // f(the largest of 8 logits)
+  template <typename F> DEVINL void maxima(F f) {
+    if constexpr (NV > 0) {
+#pragma unroll
+      for (int k = 0; k < NV; k++) {
+        float v[8];
+        anew(c[k]);
+        get8(c[k], v);
+        most[k] = max8(v);
+        f(most[k]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      vectors([&](int, const float* v) { f(max8(v)); });
+    }
   }
   // f(first element's index, 8 logits, -inf where there are none)
   template <typename F> DEVINL void vectors(F f) {
@@ -97,6 +114,24 @@ struct Row {
         get8(w, v);
         f(8 * i, v);
       }
+    }
+  }
+  // of those only that some lane of the wave has an element in which is worth it
+  template <typename W, typename F> DEVINL void vectors(W worth, F f) {
+    if constexpr (NV > 0) {
+#pragma unroll
+      for (int k = 0; k < NV; k++) {
+        if (!__any(worth(most[k]))) continue;
+        float v[8];
+        anew(c[k]);
+        get8(c[k], v);
+        f(v);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      vectors([&](int, const float* v) {
+        if (__any(worth(max8(v)))) f(v);
+      });
     }
   }
   DEVINL bool has_tail() const { return 8 * nvec + (int)threadIdx.x < V; }
@@ -244,7 +279,7 @@ void sample_topp_kernel(const LT* __restrict__ logits,
 
   // ---- 1: row maximum ---------------------------------------------------
   float top = -INFINITY;
-  r.vectors([&](int, const float* v) { top = fmaxf(top, max8(v)); });
+  r.maxima([&](float m) { top = fmaxf(top, m); });
   if (r.has_tail()) top = fmaxf(top, r.tail());
   top = block_max<SBLOCK>(top, s.red);
 
@@ -278,8 +313,7 @@ void sample_topp_kernel(const LT* __restrict__ logits,
       const float u = l * invT - M;
       if (u >= lo && u < lo + width) add_hist(s, (u - lo) * scale, __expf(u));
     };
-    r.vectors([&](int, const float* v) {
-      if (!__any(max8(v) * invT - M >= lo)) return;
+    r.vectors([&](float most) { return most * invT - M >= lo; }, [&](const float* v) {
 #pragma unroll
       for (int j = 0; j < 8; j++) fine(v[j]);
     });
@@ -295,8 +329,7 @@ void sample_topp_kernel(const LT* __restrict__ logits,
     return u >= lowest ? __expf(u) : 0.f;
   };
   float own = 0.f;
-  r.vectors([&](int, const float* v) {
-    if (!__any(max8(v) * invT - M >= lowest)) return;
+  r.vectors([&](float most) { return most * invT - M >= lowest; }, [&](const float* v) {
 #pragma unroll
     for (int j = 0; j < 8; j++) own += kept(v[j]);
   });
@@ -392,7 +425,10 @@ void sample_topp_kernel(const LT* __restrict__ logits,
 // on one CU.  151936 bf16 logits at T = 0.7, top-p 0.95, us: 8 rows 29 (with 256
 // threads, five passes over memory and histograms in registers 215), 256 rows 56
 // (325), 2048 rows 299 (1608); LDS float atomics in place of the private
-// columns' plain adds took 221 for 8 rows.
+// columns' plain adds took 221 for 8 rows.  With each vector's maximum kept, so that the
+// passes after the histogram unpack only the few that matter, 8 rows 27.8 (31.0 in the same
+// process), 256 rows 37.5 (40.4); four elements' histogram entries read before the first is
+// written 30.5 for 8 rows: the passes are bound by the VALU of one CU.
 static void launch_sampler(const torch::Tensor& logits, torch::Tensor& out, float* lp,
                            double temperature, double top_p, long seed, long step,
                            const long* step_ptr) {
