@@ -6,6 +6,8 @@ std::vector<torch::Tensor> rmsnorm_fwd(torch::Tensor x, torch::Tensor w, double 
 std::vector<torch::Tensor> rmsnorm_bwd(torch::Tensor dy, torch::Tensor x,
                                        torch::Tensor w, torch::Tensor invrms,
                                        c10::optional<torch::Tensor> extra, bool want_dw);
+std::vector<torch::Tensor> rmsnorm_parts_fwd(torch::Tensor parts, torch::Tensor res,
+                                             torch::Tensor w, double eps);
 std::vector<torch::Tensor> rmsnorm_addres_fwd(torch::Tensor x, torch::Tensor res,
                                               torch::Tensor w, double eps);
 torch::Tensor rope_fwd(torch::Tensor x, torch::Tensor table, torch::Tensor positions, double sign);
@@ -68,6 +70,8 @@ void glu_linear(torch::Tensor x, torch::Tensor gate, torch::Tensor up, torch::Te
                 long act);
 // linear_rows.hip
 torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias);
+torch::Tensor linear_rows_parts(torch::Tensor x, torch::Tensor w,
+                                c10::optional<torch::Tensor> bias);
 torch::Tensor glu_rows(torch::Tensor x, torch::Tensor gate, torch::Tensor up);
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -75,6 +79,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm_bwd", &rmsnorm_bwd, py::arg("dy"), py::arg("x"), py::arg("w"),
         py::arg("invrms"), py::arg("extra") = py::none(), py::arg("want_dw") = true);
   m.def("rmsnorm_addres_fwd", &rmsnorm_addres_fwd);
+  m.def("rmsnorm_parts_fwd", &rmsnorm_parts_fwd);
   m.def("rope_fwd", &rope_fwd);
   m.def("qkv_rope_fwd", &qkv_rope_fwd);
   m.def("qkv_rope_bwd", &qkv_rope_bwd);
@@ -84,6 +89,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ce_backward_dlogits", &ce_backward_dlogits);
   m.def("glu_linear", &glu_linear);
   m.def("linear_rows", &linear_rows);
+  m.def("linear_rows_parts", &linear_rows_parts);
   m.def("glu_rows", &glu_rows);
   m.def("lora_grads", &lora_grads);
   m.def("lora_down", &lora_down);

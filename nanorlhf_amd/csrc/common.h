@@ -90,6 +90,27 @@ DEVINL void stv(short* p, const float* v) {
   }
 }
 
+// 8 elements of the sum of `splits` (at most 8) parts of a product's depth, `stride` elements
+// apart, and its bias if there is one, rounded as the product's output is
+DEVINL s16x8 sum_parts8(const float* p, long stride, int splits, const short* bias) {
+  float v[8][8];
+#pragma unroll
+  for (int k = 0; k < 8; k++)
+    if (k < splits) ldv<8>(p + k * stride, v[k]);
+  float b[8] = {};
+  if (bias) ldv<8>(bias, b);
+#pragma unroll
+  for (int k = 1; k < 8; k++)
+    if (k < splits) {
+#pragma unroll
+      for (int j = 0; j < 8; j++) v[0][j] += v[k][j];
+    }
+  s16x8 o;
+#pragma unroll
+  for (int j = 0; j < 8; j++) o[j] = f2bf(v[0][j] + b[j]);
+  return o;
+}
+
 // ---- activations (32-bit) -------------------------------------------------
 DEVINL float act_sigmoid(float x) { return 1.f / (1.f + expf(-x)); }
 DEVINL float act_silu(float x) { return x / (1.f + expf(-x)); }

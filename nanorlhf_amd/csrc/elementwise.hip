@@ -431,17 +431,36 @@ torch::Tensor swiglu_bwd(torch::Tensor dy, torch::Tensor gu) {
 // h slice in registers across both phases (read x,res; write h,y — the
 // unfused pair costs an extra h read plus a launch).  invrms saved for the
 // backward, which reuses rmsnorm_bwd on h (d h = d x = d res).
+//
+// Where few rows decode it is a chain of latencies: the weight is asked for with the rows
+// and the sum crosses the waves with one barrier.  With `splits` x is 32-bit parts of the
+// depth of the product before ([splits][rows][H]) that are added up here, for which that
+// product took another launch: 64 rows of 1536 in 5 parts 4.5 us, where the sum took 4.6
+// and this 4.7.
 template <int BLOCK>
-__global__ void rmsnorm_addres_fwd_kernel(const short* __restrict__ x,
+DEVINL float block_sum_once(float v, float* scratch) {
+  static_assert(BLOCK == 256, "four waves");
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return (scratch[0] + scratch[2]) + (scratch[1] + scratch[3]);
+}
+template <int BLOCK, bool PARTS>
+__global__ void rmsnorm_addres_fwd_kernel(const void* __restrict__ x,
                                           const short* __restrict__ res,
                                           const short* __restrict__ w,
                                           short* __restrict__ h,
                                           short* __restrict__ y,
                                           float* __restrict__ invrms,
-                                          int H, float eps) {
+                                          int H, float eps, int splits) {
   __shared__ float scratch[BLOCK / 64];
-  const long row = blockIdx.x;
-  const short* xr = x + row * (long)H;
+  const long row = blockIdx.x, part = (long)gridDim.x * H;
+  auto load_x = [&](int i) {
+    if constexpr (PARTS)
+      return sum_parts8((const float*)x + row * (long)H + i * 8, part, splits, nullptr);
+    else
+      return *reinterpret_cast<const s16x8*>((const short*)x + row * (long)H + i * 8);
+  };
   const short* rr = res + row * (long)H;
   short* hr = h + row * (long)H;
   short* yr = y + row * (long)H;
@@ -449,11 +468,12 @@ __global__ void rmsnorm_addres_fwd_kernel(const short* __restrict__ x,
   float ss = 0.f;
   if (nvec <= BLOCK) {
     // register-resident path (H <= BLOCK*8)
-    s16x8 hv{};
+    s16x8 hv{}, wv{};
     const int i = threadIdx.x;
     if (i < nvec) {
-      s16x8 xv = *reinterpret_cast<const s16x8*>(xr + i * 8);
       s16x8 rv = *reinterpret_cast<const s16x8*>(rr + i * 8);
+      wv = *reinterpret_cast<const s16x8*>(w + i * 8);
+      s16x8 xv = load_x(i);
 #pragma unroll
       for (int j = 0; j < 8; j++) {
         const float f = bf2f(xv[j]) + bf2f(rv[j]);
@@ -462,11 +482,10 @@ __global__ void rmsnorm_addres_fwd_kernel(const short* __restrict__ x,
         ss += fb * fb;
       }
     }
-    ss = block_sum<BLOCK>(ss, scratch);
+    ss = block_sum_once<BLOCK>(ss, scratch);
     const float inv = rsqrtf(ss / (float)H + eps);
-    if (threadIdx.x == 0) invrms[row] = inv;
+    if (invrms && threadIdx.x == 0) invrms[row] = inv;
     if (i < nvec) {
-      s16x8 wv = *reinterpret_cast<const s16x8*>(w + i * 8);
       s16x8 o;
 #pragma unroll
       for (int j = 0; j < 8; j++) {
@@ -480,8 +499,8 @@ __global__ void rmsnorm_addres_fwd_kernel(const short* __restrict__ x,
   }
   // general path: write h in pass 1, re-read (L2-hot) in pass 2
   for (int i = threadIdx.x; i < nvec; i += BLOCK) {
-    s16x8 xv = *reinterpret_cast<const s16x8*>(xr + i * 8);
     s16x8 rv = *reinterpret_cast<const s16x8*>(rr + i * 8);
+    s16x8 xv = load_x(i);
     s16x8 hv;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
@@ -493,7 +512,7 @@ __global__ void rmsnorm_addres_fwd_kernel(const short* __restrict__ x,
   }
   ss = block_sum<BLOCK>(ss, scratch);
   const float inv = rsqrtf(ss / (float)H + eps);
-  if (threadIdx.x == 0) invrms[row] = inv;
+  if (invrms && threadIdx.x == 0) invrms[row] = inv;
   for (int i = threadIdx.x; i < nvec; i += BLOCK) {
     s16x8 hv = *reinterpret_cast<const s16x8*>(hr + i * 8);
     s16x8 wv = *reinterpret_cast<const s16x8*>(w + i * 8);
@@ -521,10 +540,34 @@ std::vector<torch::Tensor> rmsnorm_addres_fwd(torch::Tensor x, torch::Tensor res
   auto invrms = torch::empty({N}, x.options().dtype(torch::kFloat32));
   if (N == 0) return {y, h, invrms};
   auto stream = at::hip::getCurrentHIPStream();
-  hipLaunchKernelGGL(rmsnorm_addres_fwd_kernel<256>, dim3(N), dim3(256), 0, stream,
-                     (const short*)x.data_ptr(), (const short*)res.data_ptr(),
+  hipLaunchKernelGGL((rmsnorm_addres_fwd_kernel<256, false>), dim3(N), dim3(256), 0, stream,
+                     x.data_ptr(), (const short*)res.data_ptr(),
                      (const short*)w.data_ptr(), (short*)h.data_ptr(),
-                     (short*)y.data_ptr(), invrms.data_ptr<float>(), H, (float)eps);
+                     (short*)y.data_ptr(), invrms.data_ptr<float>(), H, (float)eps, 0);
   HIP_CHECK_LAST();
   return {y, h, invrms};
+}
+
+// parts [splits, N, H] float32, res [N, H]: (rmsnorm(h) * w, h), h = sum of the parts + res
+std::vector<torch::Tensor> rmsnorm_parts_fwd(torch::Tensor parts, torch::Tensor res,
+                                             torch::Tensor w, double eps) {
+  on_gpu({parts, res, w});
+  TORCH_CHECK(parts.dim() == 3 && parts.scalar_type() == torch::kFloat32 &&
+              parts.is_contiguous() && parts.size(0) > 0 && parts.size(0) <= 8,
+              "rmsnorm_parts: float32 parts [1 to 8, rows, width]");
+  const long N = parts.size(1), H = parts.size(2);
+  TORCH_CHECK(res.scalar_type() == torch::kBFloat16 && res.is_contiguous() && res.dim() == 2 &&
+              res.size(0) == N && res.size(1) == H && w.scalar_type() == torch::kBFloat16 &&
+              w.is_contiguous() && w.numel() == H && H % 8 == 0, "rmsnorm_parts: bf16 [N, H]");
+  for (const auto& t : {parts, res, w})
+    TORCH_CHECK((uintptr_t)t.data_ptr() % 16 == 0, "rmsnorm_parts: operands on 16 bytes");
+  auto h = torch::empty_like(res), y = torch::empty_like(res);
+  if (N == 0) return {y, h};
+  hipLaunchKernelGGL((rmsnorm_addres_fwd_kernel<256, true>), dim3(N), dim3(256), 0,
+                     at::hip::getCurrentHIPStream(), parts.data_ptr(),
+                     (const short*)res.data_ptr(), (const short*)w.data_ptr(),
+                     (short*)h.data_ptr(), (short*)y.data_ptr(), nullptr, (int)H, (float)eps,
+                     (int)parts.size(0));
+  HIP_CHECK_LAST();
+  return {y, h};
 }

@@ -122,17 +122,25 @@ void kv_append(torch::Tensor k, torch::Tensor v, torch::Tensor slots,
 }
 
 // qkv [T, (Hq + 2 Hkv) D]: q and k rotated, k and v into the cache at `slots`.
-// Returns q [T, Hq, D], and k and v [T, Hkv, D] if asked for.
+// Returns q [T, Hq, D], and k and v [T, Hkv, D] if asked for.  Or qkv float32 [splits, T, ..],
+// parts of a projection that this adds up, with its bias.
 std::vector<torch::Tensor> qkv_rope_append(torch::Tensor qkv, torch::Tensor table,
                                            torch::Tensor positions, torch::Tensor slots,
                                            torch::Tensor k_cache, torch::Tensor v_cache, long Hq,
-                                           bool want_kv) {
-  on_gpu({qkv, table, positions, slots, k_cache, v_cache});
-  TORCH_CHECK(qkv.scalar_type() == torch::kBFloat16 && qkv.is_contiguous() && qkv.dim() == 2);
+                                           bool want_kv, c10::optional<torch::Tensor> bias) {
+  on_gpu({qkv, table, positions, slots, k_cache, v_cache, bias});
+  const bool parts = qkv.dim() == 3;
+  TORCH_CHECK(qkv.is_contiguous() &&
+              (parts ? qkv.scalar_type() == torch::kFloat32 && qkv.size(0) > 0 && qkv.size(0) <= 8
+                     : qkv.scalar_type() == torch::kBFloat16 && qkv.dim() == 2 && !bias));
   TORCH_CHECK(k_cache.dim() == 4 && k_cache.is_contiguous() && v_cache.is_contiguous() &&
               v_cache.scalar_type() == k_cache.scalar_type());
-  const long T = qkv.size(0), ps = k_cache.size(1), Hkv = k_cache.size(2), D = k_cache.size(3);
-  TORCH_CHECK(Hq > 0 && qkv.size(1) == (Hq + 2 * Hkv) * D && D % 32 == 0);
+  const long T = qkv.size(-2), N = qkv.size(-1), ps = k_cache.size(1), Hkv = k_cache.size(2),
+             D = k_cache.size(3);
+  TORCH_CHECK(Hq > 0 && N == (Hq + 2 * Hkv) * D && D % 32 == 0);
+  if (bias)
+    TORCH_CHECK(bias->scalar_type() == torch::kBFloat16 && bias->is_contiguous() &&
+                bias->numel() == N, "bias must be bf16, one per column");
   TORCH_CHECK(v_cache.size(1) == Hkv && v_cache.size(2) == D && v_cache.size(3) == ps);
   TORCH_CHECK(table.scalar_type() == torch::kFloat32 && table.is_contiguous() &&
               table.size(-1) == D, "rope table must be fp32 [positions, head_dim]");
@@ -140,17 +148,26 @@ std::vector<torch::Tensor> qkv_rope_append(torch::Tensor qkv, torch::Tensor tabl
               positions.numel() == T, "positions must be int64, one per token");
   TORCH_CHECK(slots.scalar_type() == torch::kLong && slots.is_contiguous() && slots.numel() == T);
   if ((uintptr_t)qkv.data_ptr() % 16) qkv = qkv.clone();
-  auto q = torch::empty({T, Hq, D}, qkv.options());
+  if (bias && (uintptr_t)bias->data_ptr() % 16) bias = bias->clone();
+  const auto opt = qkv.options().dtype(torch::kBFloat16);
+  auto q = torch::empty({T, Hq, D}, opt);
   std::vector<torch::Tensor> out{q};
   if (want_kv)
-    for (int i = 0; i < 2; i++) out.push_back(torch::empty({T, Hkv, D}, qkv.options()));
+    for (int i = 0; i < 2; i++) out.push_back(torch::empty({T, Hkv, D}, opt));
   auto stream = at::hip::getCurrentHIPStream();
   const bool fp8 = k_cache.scalar_type() == torch::kFloat8_e4m3fn;
   TORCH_CHECK(fp8 || k_cache.scalar_type() == torch::kBFloat16,
               "kv cache must be bf16 or fp8_e4m3fn");
   by_tokens(T, (Hq + 2 * Hkv) * (D / 16), [&](long t0, unsigned units) {
     QkvRope a{};
-    a.qkv = (const short*)qkv.data_ptr() + t0 * qkv.size(1);
+    if (parts) {
+      a.parts = qkv.data_ptr<float>() + t0 * N;
+      a.part = T * N;
+      a.splits = qkv.size(0);
+      a.bias = bias ? (const short*)bias->data_ptr() : nullptr;
+    } else {
+      a.qkv = (const short*)qkv.data_ptr() + t0 * N;
+    }
     a.q = (short*)q.data_ptr() + t0 * Hq * D;
     if (want_kv) {
       a.k = (short*)out[1].data_ptr() + t0 * Hkv * D;
@@ -166,8 +183,10 @@ std::vector<torch::Tensor> qkv_rope_append(torch::Tensor qkv, torch::Tensor tabl
     a.D = D;
     a.ps = ps;
     const dim3 grid((units + 255) / 256), block(256);
-    if (fp8) hipLaunchKernelGGL(qkv_rope_kernel<unsigned char>, grid, block, 0, stream, a, units);
-    else hipLaunchKernelGGL(qkv_rope_kernel<short>, grid, block, 0, stream, a, units);
+#define LAUNCH(CT, P) hipLaunchKernelGGL((qkv_rope_kernel<CT, P>), grid, block, 0, stream, a, units)
+    if (fp8) { if (parts) LAUNCH(unsigned char, true); else LAUNCH(unsigned char, false); }
+    else { if (parts) LAUNCH(short, true); else LAUNCH(short, false); }
+#undef LAUNCH
   });
   HIP_CHECK_LAST();
   return out;

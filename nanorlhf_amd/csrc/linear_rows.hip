@@ -201,21 +201,21 @@ static void launch_rows(const RowsArgs& a, int splits) {
 #undef LAUNCH
 }
 
-torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias) {
+// y [M, N], or with `deferred`, where the depth is divided, its 32-bit parts [splits, M, N],
+// which the next kernel adds up
+static torch::Tensor rows_product(torch::Tensor x, torch::Tensor w,
+                                  c10::optional<torch::Tensor> bias, bool deferred) {
   on_gpu({x, w, bias});
   check_rows(x, w);
   const long M = x.size(0), K = x.size(1), N = w.size(0);
   if (bias)
     TORCH_CHECK(bias->scalar_type() == torch::kBFloat16 && bias->is_contiguous() &&
                 bias->numel() == N, "linear_rows: bf16 bias");
-  auto y = torch::empty({M, N}, x.options());
-  if (M == 0 || N == 0) return y;
+  if (M == 0 || N == 0) return torch::empty({M, N}, x.options());
   RowsArgs a{};
   a.x = (const short*)x.data_ptr();
   a.w = (const short*)w.data_ptr();
   const short* b = bias ? (const short*)bias->data_ptr() : nullptr;
-  a.bias = b;
-  a.y = (short*)y.data_ptr();
   a.M = M;
   a.N = N;
   a.K = K;
@@ -224,30 +224,49 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, c10::optional<torch:
   // 32 rows, where that shares x better: 64 rows of 152064 x 1536 108 us, 119 with 64;
   // of 32768 x 1536 32, 27 with 64.  A deep product of few columns is divided until about
   // 224 workgroups share it, which has to pay for a second kernel of 3 us: 64 rows of
-  // 1536 x 8960 15 us in 4 parts, 24 in one; 1536 x 1536 6 us in one, 7 in 2.  A deep one
+  // 1536 x 8960 15 us in 4 parts, 24 in one; 1536 x 1536 6 us in one, 7 in 2.  Without
+  // that kernel a shallow one is divided by two where it leaves half of the CUs idle: 64 rows
+  // of 2048 x 1536 7.1 us, 5.4 in 2 parts, 16 rows 4.6 and 3.9, one 4.1 and 3.7; 64 of 896 x
+  // 896 4.6 and 3.9.  A deep one
   // of many columns wants many waves in flight on each: one row of 14336 x 4096 24 us
   // with 32 columns and four waves, 32 with 64 and two.
   const bool deep = K > 2048, shared = deep && N <= 5120;
   const int nf = shared ? (N <= 1024 ? 1 : N < 3200 ? 2 : 4)
                  : deep ? 2 : N <= 4096 ? 1 : N <= 8192 ? 2 : 4;
   const long tiles = (N + 16 * nf - 1) / (16 * nf);
-  const int splits =
-      shared && N % 4 == 0 ? (int)std::min(8L, std::max(1L, (224 + tiles / 2) / tiles)) : 1;
-  torch::Tensor parts;
+  int splits = 1;
+  if (N % 4 == 0 && shared) splits = (int)std::min(8L, std::max(1L, (224 + tiles / 2) / tiles));
+  else if (N % 4 == 0 && deferred && !deep && tiles <= 128 && K >= 512) splits = 2;
+  torch::Tensor y, parts;
   if (splits > 1) {
     parts = torch::empty({splits, M, N}, x.options().dtype(torch::kFloat32));
     a.parts = parts.data_ptr<float>();
-    a.bias = nullptr;
+  } else {
+    a.bias = b;
+  }
+  if (splits == 1 || !deferred) {
+    y = torch::empty({M, N}, x.options());
+    a.y = (short*)y.data_ptr();
   }
   if (nf == 1) launch_rows<1, 4, 3, false>(a, splits);
   else if (nf == 2) launch_rows<2, 4, 3, false>(a, splits);
   else if (M <= 32 || N <= 65536) launch_rows<4, 2, 2, false>(a, splits);
   else launch_rows<8, 2, 1, false>(a, splits);
-  if (splits > 1)
+  if (splits > 1 && !deferred)
     hipLaunchKernelGGL(rows_sum_kernel, dim3((M * N / 4 + 255) / 256), dim3(256), 0,
                        c10::hip::getCurrentHIPStream(), a.parts, b, a.y, M * N, (int)N, splits);
   HIP_CHECK_LAST();
-  return y;
+  return y.defined() ? y : parts;
+}
+
+torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> bias) {
+  return rows_product(x, w, bias, false);
+}
+
+// x w^T + bias as bf16 [M, N], or float32 [parts, M, N] that add up to x w^T alone
+torch::Tensor linear_rows_parts(torch::Tensor x, torch::Tensor w,
+                                c10::optional<torch::Tensor> bias) {
+  return rows_product(x, w, bias, true);
 }
 
 // silu(x gate^T) * (x up^T)

@@ -20,6 +20,11 @@ struct QkvRope {
   const long* slots;     // [T] flat cache slots, with a cache
   void *kc, *vc;         // [P, ps, Hkv, D], [P, Hkv, D, ps]
   int Hq, Hkv, D, ps;
+  // instead of qkv: 32-bit sums of parts of the projection's depth [splits][T, ..] and bias
+  const float* parts;
+  const short* bias;     // may be null
+  long part;             // elements of one
+  int splits;
 };
 
 DEVINL void rotate8(const s16x8& x1, const s16x8& x2, const float* tb, int D, float sign, s16x8& o1,
@@ -41,7 +46,7 @@ DEVINL unsigned fp8x4(const s16x8& x, int at) {
 }
 
 // CT: element of the cache, or void
-template <typename CT>
+template <typename CT, bool PARTS = false>
 __global__ __launch_bounds__(256) void qkv_rope_kernel(QkvRope a, unsigned units) {
   const unsigned idx = blockIdx.x * 256u + threadIdx.x;
   if (idx >= units) return;
@@ -49,10 +54,18 @@ __global__ __launch_bounds__(256) void qkv_rope_kernel(QkvRope a, unsigned units
   const unsigned g = idx % G, row = idx / G;       // row = t * H + h
   const unsigned h = row % H;
   const long t = row / H;
-  const short* src = a.qkv + (long)row * a.D;
   const int d1 = 8 * g, d2 = a.D / 2 + 8 * g;
-  s16x8 x1 = *reinterpret_cast<const s16x8*>(src + d1);
-  s16x8 x2 = *reinterpret_cast<const s16x8*>(src + d2);
+  s16x8 x1, x2;
+  if constexpr (PARTS) {
+    const float* src = a.parts + (long)row * a.D;
+    const short* bias = a.bias ? a.bias + h * a.D : nullptr;
+    x1 = sum_parts8(src + d1, a.part, a.splits, bias ? bias + d1 : nullptr);
+    x2 = sum_parts8(src + d2, a.part, a.splits, bias ? bias + d2 : nullptr);
+  } else {
+    const short* src = a.qkv + (long)row * a.D;
+    x1 = *reinterpret_cast<const s16x8*>(src + d1);
+    x2 = *reinterpret_cast<const s16x8*>(src + d2);
+  }
   const bool is_v = h >= (unsigned)(a.Hq + a.Hkv), is_q = h < (unsigned)a.Hq;
   if (!is_v) rotate8(x1, x2, a.table + a.pos[t] * a.D + d1, a.D, 1.f, x1, x2);
   const int kvh = is_v ? h - a.Hq - a.Hkv : (int)h - a.Hq;

@@ -11,7 +11,7 @@ void kv_append(torch::Tensor k, torch::Tensor v, torch::Tensor slots,
 std::vector<torch::Tensor> qkv_rope_append(torch::Tensor qkv, torch::Tensor table,
                                            torch::Tensor positions, torch::Tensor slots,
                                            torch::Tensor k_cache, torch::Tensor v_cache, long Hq,
-                                           bool want_kv);
+                                           bool want_kv, OptTensor bias);
 void copy_pages(std::vector<torch::Tensor> pools, torch::Tensor src, torch::Tensor dst);
 torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor k_cache,
                                 torch::Tensor v_cache, torch::Tensor block_tables,
@@ -57,6 +57,7 @@ void glu_linear(torch::Tensor x, torch::Tensor gate, torch::Tensor up, torch::Te
                 long act);
 // linear_rows.hip
 torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, OptTensor bias);
+torch::Tensor linear_rows_parts(torch::Tensor x, torch::Tensor w, OptTensor bias);
 torch::Tensor glu_rows(torch::Tensor x, torch::Tensor gate, torch::Tensor up);
 // wkv.hip
 void token_shift(torch::Tensor h, torch::Tensor mu, OptTensor seq_lens, torch::Tensor slots,
@@ -96,7 +97,9 @@ torch::Tensor moe_down(torch::Tensor act, torch::Tensor down, torch::Tensor list
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("kv_append", &kv_append);
   m.def("copy_pages", &copy_pages);
-  m.def("qkv_rope_append", &qkv_rope_append);
+  m.def("qkv_rope_append", &qkv_rope_append, py::arg("qkv"), py::arg("table"),
+        py::arg("positions"), py::arg("slots"), py::arg("k_cache"), py::arg("v_cache"),
+        py::arg("heads"), py::arg("want_kv"), py::arg("bias") = py::none());
   m.def("paged_attn_decode", &paged_attn_decode);
   m.def("paged_attn_decode_window", &paged_attn_decode_window);
   m.def("paged_attn_varlen", &paged_attn_varlen);
@@ -108,6 +111,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gelu_glu", &gelu_glu);
   m.def("glu_linear", &glu_linear);
   m.def("linear_rows", &linear_rows);
+  m.def("linear_rows_parts", &linear_rows_parts);
   m.def("glu_rows", &glu_rows);
   m.def("relu_squared_", &relu_squared_);
   m.def("token_shift", &token_shift);

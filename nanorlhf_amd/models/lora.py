@@ -140,13 +140,17 @@ def apply_lora(model: nn.Module, cfg: LoraConfig) -> nn.Module:
     return model
 
 
+def unheard(m: nn.Module) -> bool:
+    """Whether nobody listens to calls of this module."""
+    return not any((m._forward_hooks, m._forward_pre_hooks, m._backward_hooks,
+                    m._backward_pre_hooks, _module._global_forward_hooks,
+                    _module._global_forward_pre_hooks))
+
+
 def plain_weight(proj: nn.Module) -> torch.Tensor | None:
     """The weight of a projection whose call is F.linear(x, weight, proj.bias) and
     nothing else: no gradient wanted, nobody listening to the call.  Else None."""
-    if torch.is_grad_enabled() or any(
-            (proj._forward_hooks, proj._forward_pre_hooks, proj._backward_hooks,
-             proj._backward_pre_hooks, _module._global_forward_hooks,
-             _module._global_forward_pre_hooks)):
+    if torch.is_grad_enabled() or not unheard(proj):
         return None
     if type(proj) is nn.Linear and "forward" not in proj.__dict__:
         w = proj.weight
@@ -158,10 +162,13 @@ def plain_weight(proj: nn.Module) -> torch.Tensor | None:
     return w if type(w) in (torch.Tensor, nn.Parameter) else None
 
 
-def project(proj: nn.Module, x: torch.Tensor) -> torch.Tensor:
-    """proj(x), by the kernel for few rows where it is a plain linear."""
+def project(proj: nn.Module, x: torch.Tensor, parts: bool = False) -> torch.Tensor:
+    """proj(x), by the kernel for few rows where it is a plain linear; with `parts` as
+    ops.linear_parts gives it."""
     w = plain_weight(proj)
-    return proj(x) if w is None else ops.linear(x, w, proj.bias)
+    if w is None:
+        return proj(x)
+    return (ops.linear_parts if parts else ops.linear)(x, w, proj.bias)
 
 
 def merge_for_rollout(model: nn.Module, quant: str | None = None):

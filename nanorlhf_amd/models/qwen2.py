@@ -24,7 +24,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from .config import ModelConfig, get_config
-from .lora import plain_weight, project
+from .lora import plain_weight, project, unheard
 
 
 @dataclass
@@ -102,13 +102,16 @@ class Attention(nn.Module):
         self.o_proj = nn.Linear(cfg.num_heads * cfg.head_dim, H, bias=False)
         self.scale = cfg.head_dim ** -0.5
 
-    def forward(self, x: torch.Tensor, rope_table: torch.Tensor, ctx: AttnContext):
+    def forward(self, x: torch.Tensor, rope_table: torch.Tensor, ctx: AttnContext,
+                parts: bool = False):
         T = x.shape[0]
-        qkv = project(self.qkv_proj, x)
-        if ctx.mode != "train" and ctx.kv_caches is not None:
+        cached = ctx.mode != "train" and ctx.kv_caches is not None
+        qkv = project(self.qkv_proj, x, parts=cached)
+        if cached:
             q, k, v = ops.qkv_rope_append(qkv, rope_table, ctx.positions, self.num_heads,
                                           ctx.slots, *ctx.kv_caches[self.layer_idx],
-                                          want_kv=ctx.mode not in ("decode", "step"))
+                                          want_kv=ctx.mode not in ("decode", "step"),
+                                          bias=getattr(self.qkv_proj, "bias", None))
         else:
             q, k, v = ops.qkv_rope(qkv, rope_table, ctx.positions, self.num_heads,
                                    self.num_kv_heads)
@@ -122,7 +125,8 @@ class Attention(nn.Module):
         else:
             o = ops.flash_attn_varlen(q, k, v, ctx.cu_seqlens, ctx.max_seqlen,
                                       self.scale, causal=ctx.causal)
-        return project(self.o_proj, o.reshape(T, -1))
+        return project(self.o_proj, o.reshape(T, -1),
+                       parts and getattr(self.o_proj, "bias", None) is None)
 
 
 class MLP(nn.Module):
@@ -131,13 +135,14 @@ class MLP(nn.Module):
         self.gate_up_proj = nn.Linear(cfg.hidden_size, 2 * cfg.intermediate_size, bias=False)
         self.down_proj = nn.Linear(cfg.intermediate_size, cfg.hidden_size, bias=False)
 
-    def forward(self, x):
+    def forward(self, x, parts: bool = False):
         w = plain_weight(self.gate_up_proj)
         if w is None or self.gate_up_proj.bias is not None:
             act = ops.swiglu(self.gate_up_proj(x))
         else:
             act = ops.linear_swiglu(x, w)
-        return project(self.down_proj, act)
+        return project(self.down_proj, act,
+                       parts and getattr(self.down_proj, "bias", None) is None)
 
 
 class RMSNorm(nn.Module):
@@ -150,6 +155,12 @@ class RMSNorm(nn.Module):
         return ops.rms_norm(x, self.weight, self.eps)
 
 
+def _parts(m: nn.Module, cls: type) -> dict:
+    """What lets a module that nobody watches return parts."""
+    plain = not torch.is_grad_enabled() and type(m) is cls and "forward" not in m.__dict__
+    return dict(parts=True) if plain and unheard(m) else {}
+
+
 class Block(nn.Module):
     def __init__(self, cfg: ModelConfig, layer_idx: int):
         super().__init__()
@@ -158,16 +169,18 @@ class Block(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_eps)
         self.mlp = MLP(cfg)
 
-    def forward(self, delta, res, rope_table, ctx):
+    def forward(self, delta, res, rope_table, ctx, parts: bool = False):
         """Carries the residual stream as (delta, res) with hidden =
         delta + res: the pending add fuses into the NEXT norm's kernel
-        (ops.add_rms_norm), so no standalone residual-add kernels run."""
+        (ops.add_rms_norm), so no standalone residual-add kernels run.  So does the sum
+        of a decoding projection's parts (ops.linear_parts), of this layer's last one
+        only if the caller asks for `parts`."""
         eps = self.input_layernorm.eps
-        a_in, h = ops.add_rms_norm(delta, res, self.input_layernorm.weight, eps)
-        attn_delta = self.self_attn(a_in, rope_table, ctx)
-        m_in, h2 = ops.add_rms_norm(attn_delta, h,
-                                    self.post_attention_layernorm.weight, eps)
-        return self.mlp(m_in), h2
+        a_in, h = ops.add_parts_rms_norm(delta, res, self.input_layernorm.weight, eps)
+        attn_delta = self.self_attn(a_in, rope_table, ctx, **_parts(self.self_attn, Attention))
+        m_in, h2 = ops.add_parts_rms_norm(attn_delta, h,
+                                          self.post_attention_layernorm.weight, eps)
+        return self.mlp(m_in, **(_parts(self.mlp, MLP) if parts else {})), h2
 
 
 class Transformer(nn.Module):
@@ -194,8 +207,8 @@ class Transformer(nn.Module):
                 delta, res = torch.utils.checkpoint.checkpoint(
                     layer, delta, res, self.rope_table, ctx, use_reentrant=False)
             else:
-                delta, res = layer(delta, res, self.rope_table, ctx)
-        y, _ = ops.add_rms_norm(delta, res, self.norm.weight, self.norm.eps)
+                delta, res = layer(delta, res, self.rope_table, ctx, **_parts(layer, Block))
+        y, _ = ops.add_parts_rms_norm(delta, res, self.norm.weight, self.norm.eps)
         return y
 
 

@@ -59,10 +59,10 @@ def ext_available() -> bool:
     return all(_load(n)[0] is not None for n in ("_C", "_serve"))
 
 
-from .rmsnorm import (add_rms_norm, gated_norm, residual_group_norm,  # noqa: E402,F401
-                      rms_norm)
+from .rmsnorm import (add_parts_rms_norm, add_rms_norm, gated_norm,  # noqa: E402,F401
+                      residual_group_norm, rms_norm)
 from .rope import Rotation, build_rope_cache, qkv_rope, rope_apply  # noqa: E402,F401
-from .linear import linear  # noqa: E402,F401
+from .linear import linear, linear_parts, sum_parts  # noqa: E402,F401
 from .swiglu import (gelu_glu, glu_fuses, linear_gelu_glu, linear_swiglu,  # noqa: E402,F401
                      relu_squared_, swiglu)
 from .attention import flash_attn_varlen  # noqa: E402,F401

@@ -19,7 +19,7 @@ from __future__ import annotations
 import torch
 
 from . import serve_ext
-from .linear import unwatched
+from .linear import sum_parts, unwatched
 from .rope import qkv_rope, rotate_pairs
 
 
@@ -46,13 +46,16 @@ def kv_append(k: torch.Tensor, v: torch.Tensor, slots: torch.Tensor,
 
 def qkv_rope_append(qkv: torch.Tensor, table: torch.Tensor, positions: torch.Tensor, heads: int,
                     slots: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
-                    want_kv: bool = True):
+                    want_kv: bool = True, bias: torch.Tensor | None = None):
     """qkv_rope, and kv_append of its k and v.  Returns (q, k, v), k and v None
-    unless wanted."""
+    unless wanted.  qkv may be linear_parts' result for this bias."""
     if qkv.is_cuda and not (torch.is_grad_enabled() and qkv.requires_grad) and unwatched(qkv):
         out = serve_ext().qkv_rope_append(qkv.contiguous(), table, positions, slots, k_cache,
-                                          v_cache, heads, want_kv)
+                                          v_cache, heads, want_kv,
+                                          bias if qkv.dim() == 3 else None)
         return tuple(out) if want_kv else (out[0], None, None)
+    if qkv.dim() == 3:
+        qkv = sum_parts(qkv, torch.bfloat16, bias)
     q, k, v = qkv_rope(qkv, table, positions, heads, k_cache.shape[2])
     kv_append(k, v, slots, k_cache, v_cache)
     return (q, k, v) if want_kv else (q, None, None)

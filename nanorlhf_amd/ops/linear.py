@@ -65,10 +65,34 @@ def few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
             and w.device == x.device and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+def _rows(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
+    return few_rows(x, w) and rows_pay(x.shape[0], *w.shape) and (
+        bias is None or plain_call(bias) and bias.dtype == x.dtype
+        and bias.device == x.device and bias.shape == w.shape[:1] and bias.is_contiguous())
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """x w^T + bias."""
-    if few_rows(x, w) and rows_pay(x.shape[0], *w.shape) and (
-            bias is None or plain_call(bias) and bias.dtype == x.dtype
-            and bias.device == x.device and bias.shape == w.shape[:1] and bias.is_contiguous()):
+    if _rows(x, w, bias):
         return linear_ext().linear_rows(x, w, bias)
     return F.linear(x, w, bias)
+
+
+def linear_parts(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None):
+    """x w^T + bias for a kernel that can add up parts as it reads them: [M, N], or, where
+    the depth is divided among workgroups, float32 parts [parts, M, N] of x w^T without the
+    bias.  See sum_parts for what they stand for."""
+    if _rows(x, w, bias):
+        return linear_ext().linear_rows_parts(x, w, bias)
+    return F.linear(x, w, bias)
+
+
+def sum_parts(y: torch.Tensor, dtype: torch.dtype,
+              bias: torch.Tensor | None = None) -> torch.Tensor:
+    """What linear_parts' result stands for."""
+    if y.dim() == 2:
+        return y
+    s = y[0]
+    for p in y[1:]:
+        s = s + p
+    return (s if bias is None else s + bias.float()).to(dtype)

@@ -7,6 +7,7 @@ from __future__ import annotations
 import torch
 
 from . import ext, serve_ext
+from .linear import plain_call, sum_parts
 
 
 def _rms_norm_ref(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
@@ -72,6 +73,19 @@ def add_rms_norm(x: torch.Tensor, res: torch.Tensor | None, weight: torch.Tensor
         return _AddRMSNormFn.apply(x.contiguous(), res.contiguous(), weight, eps)
     h = x + res
     return rms_norm(h, weight, eps), h
+
+
+def add_parts_rms_norm(x: torch.Tensor, res: torch.Tensor | None, weight: torch.Tensor,
+                       eps: float = 1e-6):
+    """add_rms_norm, of linear_parts' result."""
+    if x.dim() != 3 or x.dtype != torch.float32 or res is None or res.dim() != 2:
+        return add_rms_norm(x, res, weight, eps)
+    if x.is_cuda and plain_call(x, res, weight) and x.shape[0] <= 8 and x.shape[2] % 8 == 0 \
+            and res.dtype == weight.dtype == torch.bfloat16 \
+            and weight.device == res.device == x.device and weight.is_contiguous() \
+            and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (x, res, weight)):
+        return tuple(ext().rmsnorm_parts_fwd(x, res, weight, eps))
+    return add_rms_norm(sum_parts(x, res.dtype), res, weight, eps)
 
 
 def _group_rms(x: torch.Tensor, groups: int, eps: float) -> torch.Tensor:

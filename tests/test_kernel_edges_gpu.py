@@ -370,6 +370,41 @@ def test_qkv_rope_append_fills_the_cache_as_kv_append_does(dtype, hq, hkv, d):
 
 
 # ------------------------------------------------------- norm, optimizer
+@pytest.mark.parametrize("rows", [1, 16, 17, 64])
+@pytest.mark.parametrize("N,K", [(2048, 1536), (896, 512), (896, 4864), (1536, 8960), (3584, 3584),
+                                 (2112, 1536), (1002, 1536)])
+def test_parts_of_a_product_are_summed_by_the_next_kernel(rows, N, K):
+    """Sums of small whole numbers are the same in any order."""
+    g = torch.Generator(device=DEV).manual_seed(rows + N)
+    x, w = (torch.randint(-3, 4, (n, K), generator=g, device=DEV).bfloat16() for n in (rows, N))
+    bias, weight = rnd(N, seed=1), rnd(N, seed=2)
+    res = rnd(rows, N, seed=3, scale=30.0)
+    with torch.no_grad():
+        y = ops.linear(x, w)
+        parts = ops.linear_parts(x, w)
+        assert (parts.dim() == 3) == (N in (2048, 896, 1536, 3584))
+        assert torch.equal(ops.sum_parts(parts, x.dtype), y)
+        if N % 8:
+            return
+        want = ops.add_rms_norm(y, res, weight)
+        got = ops.add_parts_rms_norm(parts, res, weight)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        if N != 2048:
+            return
+        table, pos = ops.build_rope_cache(128, 64).to(DEV), torch.arange(rows, device=DEV) % 64
+        slots = torch.randperm(128, generator=g, device=DEV)[:rows]
+        for dtype in (torch.bfloat16, torch.float8_e4m3fn):
+            kc = torch.zeros(8, 16, 2, 128, dtype=dtype, device=DEV)
+            vc = torch.zeros(8, 2, 128, 16, dtype=dtype, device=DEV)
+            kc2, vc2 = kc.clone(), vc.clone()
+            a = ops.qkv_rope_append(ops.linear(x, w, bias), table, pos, 12, slots, kc, vc)
+            b = ops.qkv_rope_append(ops.linear_parts(x, w, bias), table, pos, 12, slots, kc2, vc2,
+                                    bias=bias)
+            assert all(torch.equal(s, t) for s, t in zip(a, b))
+            assert torch.equal(kc.view(torch.uint8), kc2.view(torch.uint8))
+            assert torch.equal(vc.view(torch.uint8), vc2.view(torch.uint8))
+
+
 def test_qkv_rope_append_drops_no_tangent():
     import torch.autograd.forward_ad as fwd
     T, table = 5, ops.build_rope_cache(64, 16, device=DEV)
