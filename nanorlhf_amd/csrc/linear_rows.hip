@@ -10,10 +10,14 @@
 // also divided among workgroups, whose 32-bit parts rows_sum_kernel adds in order.
 //
 // us for 64 / 16 / 1 rows, library before -> now:
-//   2048 x 1536       7.6 -> 5.8    7.1 -> 3.8    6.9 -> 3.7
-//   1536 x 8960       24.8 -> 15.0  27.9 -> 10.6  27.7 -> 9.7
-//   8960 x 1536, GLU  20.6 -> 18.6  41.6 -> 14.1  42.1 -> 13.7
-//   151936 x 1536     115 -> 108    159 -> 89     158 -> 83     (467 MB: 5.6 TB/s)
+//   2048 x 1536       7.6 -> 6.8    7.1 -> 4.6    6.9 -> 4.1    (in two parts 5.2, 3.8, 3.6)
+//   1536 x 8960       24.8 -> 10.7  27.9 -> 7.5   27.7 -> 7.2   (in five parts, without
+//                                                               their sum: 4.6 by itself)
+//   8960 x 1536, GLU  20.6 -> 16.4  41.6 -> 13.2  42.1 -> 13.0
+//   151936 x 1536     115 -> 108    159 -> 90     158 -> 82     (467 MB: 5.7 TB/s)
+// With 64 rows, the sums and stores of all tiles by one wave took as long as fetching x:
+// 5.4, 11.8, 18.3 and 110 us.  Addresses made in the loads' own assembly, products between
+// the loads, deeper rings and walks that start at different depths changed nothing.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -104,60 +108,67 @@ void linear_rows_kernel(RowsArgs a) {
         for (int j = 0; j < MF; j++) acc[i][j] = mfma16l(wf[q][i], xf[q][j], acc[i][j]);
   }
   __syncthreads();
-  // halves of the waves add up, in the same order every time
-  typedef f32x4 Sums[NF][MF][64];
-  static_assert(sizeof(Sums) * (WAVES / 2) <= sizeof(ring), "room for the sums");
-  Sums* sums = reinterpret_cast<Sums*>(&ring[0][0][0]);
+  // Each wave adds up and stores its share of the tiles, always in the same order, so that
+  // one barrier is all and no wave is left with the stores of all: with 64 rows that
+  // took longer than fetching x.  A unit is a tile, or a gate's and its up's.
+  constexpr int TILES = GLU && !HALVES ? 2 : 1, UNITS = NF / TILES * MF;
+  typedef f32x4 Tile[64];
+  static_assert(sizeof(Tile) * UNITS * TILES * (WAVES - 1) <= sizeof(ring), "room for the sums");
+  Tile* sums = reinterpret_cast<Tile*>(&ring[0][0][0]);
 #pragma unroll
-  for (int n = WAVES / 2; n > 0; n >>= 1) {
-    if (wid >= n && wid < 2 * n) {
+  for (int u = 0; u < UNITS; u++) {
+    const int owner = u % WAVES;
+    if (wid == owner) continue;
 #pragma unroll
-      for (int i = 0; i < NF; i++)
-#pragma unroll
-        for (int j = 0; j < MF; j++) sums[wid - n][i][j][lane] = acc[i][j];
-    }
-    __syncthreads();
-    if (wid < n) {
-#pragma unroll
-      for (int i = 0; i < NF; i++)
-#pragma unroll
-        for (int j = 0; j < MF; j++) acc[i][j] += sums[wid][i][j][lane];
-    }
-    if (n > 1) __syncthreads();
+    for (int e = 0; e < TILES; e++)
+      sums[(u * TILES + e) * (WAVES - 1) + wid - (wid > owner)][lane] =
+          acc[u / MF * TILES + e][u % MF];
   }
-  if (wid > 0) return;
+  __syncthreads();
   // lane: row 16 j + lo, columns 16 i + 4 hi .. + 3 (HALVES: 8 i + 4 hi .. + 3, up's
   // in the wave's upper half)
   const bool whole = a.N % 4 == 0;
 #pragma unroll
-  for (int j = 0; j < MF; j++) {
-    const int m = 16 * j + lo;
+  for (int u = 0; u < UNITS; u++) {
+    const int owner = u % WAVES, i = u / MF * TILES, j = u % MF;
+    if (wid != owner) continue;
+    f32x4 sum[TILES];
 #pragma unroll
-    for (int i = 0; i < NF; i += GLU && !HALVES ? 2 : 1) {
-      const int n = n0 + (GLU ? i * 8 : i * 16) + 4 * hi;
-      float v[4];
+    for (int e = 0; e < TILES; e++) {
+      f32x4 w[WAVES];
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        v[r] = acc[i][j][r];
-        if (GLU)
-          v[r] = silu_fast(v[r]) * (HALVES ? __shfl_xor(v[r], 32) : acc[GLU && !HALVES ? i + 1 : i][j][r]);
-        else if (a.bias && n + r < a.N)
-          v[r] += bf2f(a.bias[n + r]);
-      }
-      if (m >= a.M || (HALVES && hi > 1)) continue;
-      if (a.parts) {
-        float* p = a.parts + ((long)blockIdx.y * a.M + m) * a.N + n;
-        if (whole && n < a.N) stv<4>(p, v);
-        else
-          for (int r = 0; r < 4; r++)
-            if (n + r < a.N) p[r] = v[r];
-      } else {
-        short* p = a.y + (long)m * a.N + n;
-        if (whole && n < a.N) stv<4>(p, v);
-        else
-          for (int r = 0; r < 4; r++)
-            if (n + r < a.N) stf(p + r, v[r]);
-      }
+      for (int k = 0; k < WAVES; k++)
+        w[k] = k == owner ? acc[i + e][j]
+                          : sums[(u * TILES + e) * (WAVES - 1) + k - (k > owner)][lane];
+#pragma unroll
+      for (int n = WAVES / 2; n > 0; n >>= 1)
+#pragma unroll
+        for (int k = 0; k < n; k++) w[k] += w[k + n];
+      sum[e] = w[0];
+    }
+    const int m = 16 * j + lo, n = n0 + (GLU ? i * 8 : i * 16) + 4 * hi;
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      v[r] = sum[0][r];
+      if (GLU)
+        v[r] = silu_fast(v[r]) * (HALVES ? __shfl_xor(v[r], 32) : sum[TILES - 1][r]);
+      else if (a.bias && n + r < a.N)
+        v[r] += bf2f(a.bias[n + r]);
+    }
+    if (m >= a.M || (HALVES && hi > 1)) continue;
+    if (a.parts) {
+      float* p = a.parts + ((long)blockIdx.y * a.M + m) * a.N + n;
+      if (whole && n < a.N) stv<4>(p, v);
+      else
+        for (int r = 0; r < 4; r++)
+          if (n + r < a.N) p[r] = v[r];
+    } else {
+      short* p = a.y + (long)m * a.N + n;
+      if (whole && n < a.N) stv<4>(p, v);
+      else
+        for (int r = 0; r < 4; r++)
+          if (n + r < a.N) stf(p + r, v[r]);
     }
   }
 }
@@ -220,9 +231,9 @@ static torch::Tensor rows_product(torch::Tensor x, torch::Tensor w,
   a.N = N;
   a.K = K;
   // 16 columns each while that makes at most a workgroup per CU, since the rows of
-  // x are read by each; up to 64 for more columns, 128 for the widest with more than
-  // 32 rows, where that shares x better: 64 rows of 152064 x 1536 108 us, 119 with 64;
-  // of 32768 x 1536 32, 27 with 64.  A deep product of few columns is divided until about
+  // x are read by each; up to 64 for more columns, 96 and four waves for the widest
+  // with more than 32 rows, where that shares x better: 64 rows of 151936 x 1536 108 us, 113
+  // with 64 and two, of x 896 65.8 and 71.7; 32 rows 97.6 and 95.6.  A deep product of few columns is divided until about
   // 224 workgroups share it, which has to pay for a second kernel of 3 us: 64 rows of
   // 1536 x 8960 15 us in 4 parts, 24 in one; 1536 x 1536 6 us in one, 7 in 2.  Without
   // that kernel a shallow one is divided by two where it leaves half of the CUs idle: 64 rows
@@ -251,7 +262,7 @@ static torch::Tensor rows_product(torch::Tensor x, torch::Tensor w,
   if (nf == 1) launch_rows<1, 4, 3, false>(a, splits);
   else if (nf == 2) launch_rows<2, 4, 3, false>(a, splits);
   else if (M <= 32 || N <= 65536) launch_rows<4, 2, 2, false>(a, splits);
-  else launch_rows<8, 2, 1, false>(a, splits);
+  else launch_rows<6, 4, 1, false>(a, splits);
   if (splits > 1 && !deferred)
     hipLaunchKernelGGL(rows_sum_kernel, dim3((M * N / 4 + 255) / 256), dim3(256), 0,
                        c10::hip::getCurrentHIPStream(), a.parts, b, a.y, M * N, (int)N, splits);
@@ -300,7 +311,12 @@ torch::Tensor glu_rows(torch::Tensor x, torch::Tensor gate, torch::Tensor up) {
     }
   }
   if (best == 16) launch_rows<2, 2, 3, true>(a, 1);
+  // twice the waves where there is as much to do for each: 64 rows of 8960 x 1536 16.4 us, 18.4
+  // with two, 48 of 18944 x 3584 53.8 and 52.2; with 32 columns 64 rows of 14336 x 4096 50.6 and
+  // 55.2, one to 16 41 and 50, 64 of 7168 x 2048 15.9 and 15.1
+  else if (best == 32 && a.K > 2048) launch_rows<4, 4, 2, true>(a, 1);
   else if (best == 32) launch_rows<4, 2, 2, true>(a, 1);
+  else if (best == 40 && M > 48) launch_rows<5, 4, 2, true>(a, 1);
   else if (best == 40) launch_rows<5, 2, 2, true>(a, 1);
   else launch_rows<6, 2, 2, true>(a, 1);
   HIP_CHECK_LAST();

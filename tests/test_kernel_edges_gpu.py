@@ -370,6 +370,25 @@ def test_qkv_rope_append_fills_the_cache_as_kv_append_does(dtype, hq, hkv, d):
 
 
 # ------------------------------------------------------- norm, optimizer
+@pytest.mark.parametrize("rows", [1, 16, 33, 48, 49, 64])
+def test_rows_of_many_waves_and_tiles(rows):
+    """The widest products, and gated ones of 32 deep and of 40 columns a workgroup, whose
+    tiles the waves share; sums of small whole numbers are exact."""
+    g = torch.Generator(device=DEV).manual_seed(rows)
+
+    def whole(n, k):
+        return torch.randint(-2, 3, (n, k), generator=g, device=DEV).bfloat16()
+
+    with torch.no_grad():
+        x, w = whole(rows, 192), whole(65539, 192)
+        assert torch.equal(ops.linear(x, w), (x.float() @ w.float().t()).bfloat16())
+        for N, K in ((8190, 2112), (10236, 64)):
+            x, w = whole(rows, K) * 0.125, whole(2 * N, K)
+            gate, up = (x.float() @ w.float().t()).chunk(2, 1)
+            want = torch.nn.functional.silu(gate) * up
+            assert rel(ops.linear_swiglu(x, w), want) < 0.003     # rounded once, 2^-9
+
+
 @pytest.mark.parametrize("rows", [1, 16, 17, 64])
 @pytest.mark.parametrize("N,K", [(2048, 1536), (896, 512), (896, 4864), (1536, 8960), (3584, 3584),
                                  (2112, 1536), (1002, 1536)])
