@@ -34,6 +34,12 @@ struct Big {
   long ldy;
   int M, N, K, grid_m, grid_n;
   int whole, parts, units;       // tiles that are one unit of work, and units of the others
+  // grouped: G <= 64 products, of the rows that lists [G, cap] name (of x a row / div) or of
+  // M each; their results go to the same rows of y, times scale [rows]
+  const int *lists, *counts;
+  const float* scale;
+  int cap, div, G;
+  long ldx, ldw, gx, gw, gy;     // row and group strides
 };
 
 DEVINL void load_big(const void* base, unsigned offset, unsigned at) {
@@ -61,36 +67,66 @@ DEVINL void load_big(const void* base, unsigned offset, unsigned at) {
 // 8192 x 8192 x 8192: 0.71 ms (1530 TFLOP/s), 48720 x 17920 x 1536 + 64: 2.13 (1310),
 // 48720 x 1536 x 8960 + 64: 1.01 (1340).  Lockstep waves that all read, then all
 // multiply 32x32x16, a barrier a step: 0.88 (1250), 2.70 (1030), 1.21 (1120).
-template <bool HAS_LORA, bool HAS_BIAS, bool VEC, int ACT>
+template <bool HAS_LORA, bool HAS_BIAS, bool VEC, int ACT, bool GROUPED = false>
 __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
   constexpr int TN = ACT ? BIG / 2 : BIG;
   constexpr int STORES = ACT ? 16 : 32;                                // of a wave and whole tile
   constexpr int STEP = BIG * 128;                                      // bytes
   __shared__ __attribute__((aligned(16))) short lds[2][2][BIG * 64];   // x's two steps, w's
   __shared__ float biases[2][HAS_BIAS ? 2 * BIG : 1];
+  // of groups: tiles of rows before each, and its rows; of a unit's rows: where they go
+  __shared__ int starts[GROUPED ? 65 : 1], sizes[GROUPED ? 64 : 1], ids[2][GROUPED ? BIG : 1];
+  __shared__ float scales[2][GROUPED ? BIG : 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = (wid & 3) * 64;
   const int n_k1 = p.K >> 6, n_kt = n_k1 + (HAS_LORA ? 1 : 0);
+
+  int grid_m = p.grid_m, units = p.units, whole = p.whole, M = p.M, g = 0;
+  if constexpr (GROUPED) {
+    if (wid == 0) {
+      const int c = lane >= p.G ? 0 : p.counts ? p.counts[lane] : p.M;
+      int s = (c + BIG - 1) / BIG;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(s, off);
+        if (lane >= off) s += y;
+      }
+      sizes[lane] = c;
+      starts[lane + 1] = s;
+      if (lane == 0) starts[0] = 0;
+    }
+    __syncthreads();
+    grid_m = __builtin_amdgcn_readfirstlane(starts[64]);
+    units = whole = grid_m * p.grid_n;
+    if (blockIdx.x >= units) return;
+  }
 
   // unit `at`: the tile's place, and which rows of it
   int m0, n0, parts;
   auto place = [&](int at) {
     int wg = at, part = 0;
     parts = 1;
-    if (at >= p.whole) {
+    if (at >= whole) {
       parts = p.parts;
-      wg = p.whole + (at - p.whole) / parts;
-      part = (at - p.whole) % parts;
+      wg = whole + (at - whole) / parts;
+      part = (at - whole) % parts;
     }
-    const int nwg = p.grid_m * p.grid_n, q = nwg >> 3, r = nwg & 7;
+    const int nwg = grid_m * p.grid_n, q = nwg >> 3, r = nwg & 7;
     const int xcd = wg & 7, i = wg >> 3;
     wg = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + i;
     constexpr int GM = 8;       // tiles that run together share rows and columns
     const int group = wg / (GM * p.grid_n), first = group * GM;
-    const int rows_here = min(GM, p.grid_m - first);
-    m0 = (first + (wg - group * GM * p.grid_n) % rows_here) * BIG + part * (BIG / parts);
+    const int rows_here = min(GM, grid_m - first);
+    const int tile = first + (wg - group * GM * p.grid_n) % rows_here;
+    m0 = tile * BIG + part * (BIG / parts);
     n0 = (wg - group * GM * p.grid_n) / rows_here * TN;
+    if constexpr (GROUPED) {
+      const int l = threadIdx.x & 63;
+      g = __ffsll((unsigned long long)__ballot(tile >= starts[l] && tile < starts[l + 1])) - 1;
+      m0 = (tile - __builtin_amdgcn_readfirstlane(starts[g])) * BIG;
+      M = __builtin_amdgcn_readfirstlane(sizes[g]);
+    }
   };
 
   // what follows from the lane, made again where it is needed: kept over the loop it
@@ -105,13 +141,24 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
   // exchanged (xor) by row pair, for two rows fill the banks.  Of a part of a tile only
   // x's first half is there, 128 / parts rows for each half of the workgroup.
   unsigned xo[4], wo[4];
+  int side = 0;
   auto x_offsets = [&](int ld) {
     const int t = fresh_tid(), r = t >> 3, c = ((t & 7) ^ (r >> 1 & 7)) << 3;
 #pragma unroll
     for (int h = 0; h < 4; h++) {
       const int m = parts == 1 ? r + 64 * (h >> 1) + 128 * (h & 1)
                                : min(r, 128 / parts - 1) + 128 / parts * (h & 1);
-      xo[h] = (unsigned)(min(m, max(p.M - 1 - m0, 0)) * ld + c) * 2;
+      if constexpr (GROUPED) {
+        const int row = min(m0 + m, M - 1);
+        const int id = p.lists ? p.lists[(long)g * p.cap + row] : row;
+        if ((t & 7) == 0) {
+          ids[side][m] = id;
+          scales[side][m] = p.scale ? p.scale[id] : 1.f;
+        }
+        xo[h] = ((unsigned)(p.div > 1 ? id / p.div : id) * (unsigned)ld + c) * 2;
+      } else {
+        xo[h] = (unsigned)(min(m, max(M - 1 - m0, 0)) * ld + c) * 2;
+      }
     }
   };
   // LDS row 16 t + l of 64 is column 4 l + t, or 2 l + t % 2 of w (t < 2) or w2
@@ -143,14 +190,14 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
     for (int i = 0; i < 2; i++)
       load_big(src, wo[2 * h + i], wat + (kt & 1) * STEP + (32 * h + 128 * i) * 128);
   };
-  int side = 0;
   auto begin = [&] {            // the first two steps of the unit at m0, n0
-    x_offsets(p.K);
-    w_offsets(p.K);
-    const int row = min(m0, p.M - 1);     // a part of the last tile may have none
-    xb = p.x + (long)row * p.K;
-    wb = p.w + (long)n0 * p.K;
-    w2b = ACT ? p.w2 + (long)n0 * p.K : wb;
+    x_offsets(GROUPED ? p.ldx : p.K);
+    w_offsets(GROUPED ? p.ldw : p.K);
+    const int row = min(m0, M - 1);       // a part of the last tile may have none
+    xb = GROUPED ? p.x + g * p.gx : p.x + (long)row * p.K;
+    const long first_w = GROUPED ? g * p.gw + n0 * p.ldw : (long)n0 * p.K;
+    wb = p.w + first_w;
+    w2b = ACT ? p.w2 + first_w : wb;
     if (HAS_LORA) {
       ub = p.u + (long)row * 64;
       bb = p.b + (long)n0 * 64;
@@ -296,9 +343,10 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
     }
     if (wid < 4) barrier();
 
-    const int m1 = m0, n1 = n0, parts1 = parts, side1 = side;
+    const int m1 = m0, n1 = n0, parts1 = parts, side1 = side, M1 = M;
+    short* const y1 = GROUPED ? p.y + g * p.gy : p.y;
     at += gridDim.x;
-    const bool another = at < p.units;
+    const bool another = at < units;
     if (another) {
       place(at);
       side ^= 1;
@@ -307,6 +355,9 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
     // lane: row 16 i + 4 hi + r of its half's, columns 4 (2) lo + 0 .. of the wave's
     const int t = fresh_tid() & 63, lo = t & 15, hi = t >> 4;
     const int gm0 = m1 + (wid >> 2) * (128 / parts1) + 4 * hi;
+    // row gm of y, and what it is multiplied by
+    auto row_of = [&](int gm) { return y1 + (GROUPED ? ids[side1][gm - m1] : gm) * p.ldy; };
+    auto scale_of = [&](int gm) { return GROUPED ? scales[side1][gm - m1] : 1.f; };
     if constexpr (ACT == NO_ACT) {
       const int gn = n1 + wn + 4 * lo;
       float bv[4];
@@ -323,8 +374,13 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
           float v[4];
 #pragma unroll
           for (int c = 0; c < 4; c++) v[c] = acc[i][c >> 1][c & 1][r] + (HAS_BIAS ? bv[c] : 0.f);
-          if (gm >= p.M) continue;
-          short* dst = p.y + gm * p.ldy + gn;
+          if (gm >= M1) continue;
+          short* dst = row_of(gm) + gn;
+          if (GROUPED) {
+            const float sc = scale_of(gm);
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] *= sc;
+          }
           if (VEC) {
             typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
             if (gn < p.N)
@@ -351,30 +407,31 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
           for (int q = 0; q < 2; q++)
 #pragma unroll
             for (int c = 0; c < 2; c++)
-              v[q][c] = glu<ACT>(acc[i][0][c][r + q], acc[i][1][c][r + q]);
+              v[q][c] = glu<ACT>(acc[i][0][c][r + q], acc[i][1][c][r + q]) *
+                        (GROUPED ? scale_of(gm0 + 16 * i + r + q) : 1.f);
           if (VEC) {
             typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
             const unsigned a = pack2bf(v[0][0], v[0][1]), b = pack2bf(v[1][0], v[1][1]);
             const unsigned mine = odd ? b : a;
             const unsigned other = __builtin_amdgcn_mov_dpp(odd ? a : b, 0xb1, 0xf, 0xf, true);
             const int gm = gm0 + 16 * i + r + odd, gn4 = gn - 2 * odd;
-            if (gm < p.M && gn4 < p.N)
+            if (gm < M1 && gn4 < p.N)
               __builtin_nontemporal_store(odd ? u32x2{other, mine} : u32x2{mine, other},
-                                          reinterpret_cast<u32x2*>(p.y + gm * p.ldy + gn4));
+                                          reinterpret_cast<u32x2*>(row_of(gm) + gn4));
           } else {
 #pragma unroll
             for (int q = 0; q < 2; q++)
 #pragma unroll
               for (int c = 0; c < 2; c++)
-                if (gm0 + 16 * i + r + q < p.M && gn + c < p.N)
-                  p.y[(gm0 + 16 * i + r + q) * p.ldy + gn + c] = f2bf(v[q][c]);
+                if (gm0 + 16 * i + r + q < M1 && gn + c < p.N)
+                  row_of(gm0 + 16 * i + r + q)[gn + c] = f2bf(v[q][c]);
           }
         }
       }
     }
     if (!another) break;
     // a wave that stored less cannot count on its stores in the waits
-    if (!VEC || parts1 > 1 || m1 + BIG > p.M || n1 + TN > p.N) wait_loads<0>();
+    if (!VEC || parts1 > 1 || m1 + BIG > M1 || n1 + TN > p.N) wait_loads<0>();
   }
 }
 
@@ -392,4 +449,19 @@ void launch_big(Big p) {
   p.units = p.whole + (tiles - p.whole) * p.parts;
   hipLaunchKernelGGL((gemm_big_kernel<HAS_LORA, HAS_BIAS, VEC, ACT>), dim3(std::min(p.units, cus)),
                      dim3(512), 0, c10::hip::getCurrentHIPStream(), p);
+}
+
+// Grouped products of whole steps of the depth, N and the strides of y multiples of 4: `most`
+// tiles of rows at most.  A workgroup counts the groups' tiles at its start and finds the
+// group of each as it comes to it; which rows of x and y they are is kept in LDS.  16
+// experts of 1536 x 2240, 1000 rows each, gate and up 193 us (1140 TFLOP/s), down 100; in
+// tiles of 128 that wait at a barrier a step 299 and 145.
+template <int ACT>
+void launch_big_grouped(Big p, long most) {
+  const int cus = at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
+  constexpr int TN = ACT ? BIG / 2 : BIG;
+  p.grid_n = (p.N + TN - 1) / TN;
+  hipLaunchKernelGGL((gemm_big_kernel<false, false, true, ACT, true>),
+                     dim3(std::min<long>(most * p.grid_n, cus)), dim3(512), 0,
+                     c10::hip::getCurrentHIPStream(), p);
 }

@@ -9,7 +9,8 @@
 // all rows at an offset of their own per group) by its own weights [N][K].  A
 // workgroup finds its group and rows from the counts, so the grid is made for
 // the worst case and surplus workgroups leave at once.
-//   tiles    bf16 MFMA, 128 x 128 tiles through LDS: groups of many rows
+//   big      gemm_big.h's kernel of 256 x 256 tiles: groups of many rows
+//   tiles    bf16 MFMA, 128 x 128 tiles through LDS: fewer, or sizes that are not its
 //   stream   bf16 MFMA, 16, 32 or 64 rows, every wave by itself through a ring in LDS:
 //            groups of few rows, bound by reading the weights
 //   plain    scalar products in 32-bit, any type and any size
@@ -18,6 +19,7 @@
 
 #include "common.h"
 #include "checks.h"
+#include "gemm_big.h"
 
 struct Grouped {
   const void *a, *w;
@@ -496,6 +498,21 @@ __global__ __launch_bounds__(1024) void expert_lists_kernel(
 }
 
 // ======================================================== host wrappers ==
+// Whether gemm_big.h's kernel takes these, with `tm` tiles of rows at most: that is what its
+// 32-bit offsets, whole steps and stores of four columns can do, and where its tiles of 256
+// fill the CUs and their columns.  us, tiles of 128 / it: 16 experts of 1536 x 2240, gate and
+// up, 140 rows each (432 tiles) 76 / 67, 1000 rows 299 / 193, down 180 rows (162) 41 / 44, 256
+// (192) 68 / 46; 4 experts, 300 rows (144) 33 / 36, 400 (180) 50 / 34; 12 heads of 512 x 128,
+// 4000 rows 16.4 / 18.3.  Up to 128 rows half of a tile is empty and it takes a long product:
+// 110 rows of 1536 x 2240 65 / 66, 80 of 2048 x 2752 133 / 99, 56 of 3584 x 4096 143 / 95.
+static bool takes_big(const Grouped& a, long each, long tm, int width) {
+  const long tn = (a.N + width - 1) / width;
+  return a.G <= 64 && a.K > 0 && a.K % 64 == 0 && a.N % 4 == 0 && (a.ldo | a.go) % 4 == 0 &&
+         (uintptr_t)a.out % 8 == 0 && a.K < 1L << 22 && a.ldw < 1L << 22 &&
+         (a.rows / a.div + 1) * a.lda < 1L << 31 && tm * tn < 1L << 31 &&
+         a.N * 4L >= tn * width * 3 && (each > 128 ? tm * tn >= 176 : tm * tn * a.K >= 800000);
+}
+
 template <bool GLU>
 static void launch_grouped(const Grouped& a, bool bf16) {
   if (a.rows == 0 || a.N == 0) return;
@@ -515,6 +532,32 @@ static void launch_grouped(const Grouped& a, bool bf16) {
     // their own, the more the longer a tile takes: 40 rows of 128 experts of 512 x 1024 (1024
     // tiles) 49 us against 58, of 16 experts of 4096 x 3584 (900) 253 against 207.
     const bool many = tm * tn >= std::max<long>(256, a.K / 2);
+    const long big = tiles_of(BIG);
+    if (each > 52 && takes_big(a, each, big, GLU ? BIG / 2 : BIG)) {
+      Big p{};
+      p.x = (const short*)a.a;
+      p.w = (const short*)a.w;
+      p.w2 = p.w + a.up;
+      p.y = (short*)a.out;
+      p.ldy = a.ldo;
+      p.M = a.rows;
+      p.N = a.N;
+      p.K = a.K;
+      p.lists = a.lists;
+      p.counts = a.lists ? a.counts : nullptr;
+      p.scale = a.scale;
+      p.cap = a.cap;
+      p.div = a.div;
+      p.G = a.G;
+      p.ldx = a.lda;
+      p.ldw = a.ldw;
+      p.gx = a.ga;
+      p.gw = a.gw;
+      p.gy = a.go;
+      launch_big_grouped<GLU ? SILU_GLU : NO_ACT>(p, big);
+      HIP_CHECK_LAST();
+      return;
+    }
     if (each > 52 ? each > 512 || tm * tn >= 64 : each > 32 && many) {
       TORCH_CHECK(tm * tn < (1L << 31));
       hipLaunchKernelGGL((grouped_tiles_kernel<GLU>), dim3(tm * tn), dim3(256), 0, stream, a,

@@ -718,6 +718,43 @@ def test_grouped_product_of_few_rows(T, G, N, K):
     assert rel(got.cpu(), want) < 0.002            # one rounding, 2^-9 at most
 
 
+@pytest.mark.parametrize("W,ff", [(2880, 1344), (64, 1356)])      # both products, gated alone
+@pytest.mark.parametrize("skew", [True, False])
+def test_experts_of_many_rows(W, ff, skew):
+    """Tiles of 256 rows: groups that fill one, miss it by one or are empty."""
+    counts = [0, 1, 255, 256, 257, 0, 512, 600, 3, 0] if skew else [190] * 10
+    T, E = sum(counts), len(counts)
+    order = torch.randperm(T, generator=torch.Generator().manual_seed(W)).to(DEV)
+    chosen = torch.empty(T, 1, dtype=torch.int32, device=DEV)
+    lists = torch.full((E, T), -1, dtype=torch.int32, device=DEV)      # only counted ones count
+    rows, first = [], 0
+    for e, n in enumerate(counts):
+        r = order[first:first + n].sort().values
+        chosen[r, 0], lists[e, :n] = e, r.int()
+        rows.append(r)
+        first += n
+    weights = torch.rand(T, 1, generator=torch.Generator(device=DEV).manual_seed(5), device=DEV)
+    h, gate_up, down = rnd(T, W, seed=1), rnd(E, 2, ff, W, seed=2, scale=W ** -0.5), \
+        rnd(E, W, ff, seed=3, scale=ff ** -0.5)
+    got = ops.moe_experts(h, gate_up, down, (chosen, weights, lists,
+                                             torch.tensor(counts, dtype=torch.int32, device=DEV)))
+    want = torch.empty(T, 1, W, dtype=torch.float64, device=DEV)
+    for e, r in enumerate(rows):
+        x = h[r].double()
+        act = torch.nn.functional.silu(x @ gate_up[e, 0].double().t()) \
+            * (x @ gate_up[e, 1].double().t())
+        want[r, 0] = weights[r].double() * (act @ down[e].double().t())
+    assert rel(got, want) < 0.004                  # two roundings, 2^-9 at most each
+
+
+@pytest.mark.parametrize("T", [257, 512])
+@pytest.mark.parametrize("G,N,K", [(12, 2060, 192), (64, 772, 64)])
+def test_grouped_product_of_many_rows(T, G, N, K):
+    x, w = rnd(T, G, K, seed=1), rnd(G, N, K, seed=2, scale=K ** -0.5)
+    want = torch.stack([x[:, g].double() @ w[g].double().t() for g in range(G)], 1)
+    assert rel(ops.group_linear(x, w), want) < 0.002       # one rounding, 2^-9 at most
+
+
 @pytest.mark.parametrize("M", [1, 63, 64, 65, 240, 1537, 25000])
 @pytest.mark.parametrize("C", [8, 64, 120, 192, 1536, 1992])
 def test_product_down_to_the_rank(M, C):
