@@ -252,7 +252,7 @@ __global__ __launch_bounds__(256, 2) void grouped_tiles_kernel(Grouped a, int ti
 // waves share the depth: each walks 64 elements at a time of its own part, which
 // direct loads bring into a ring of its own in LDS, whole 128-byte lines, without
 // barriers, and they add up through LDS.  16 experts of 1536 x 2240, 32 tokens with 4
-// each: gate and up 43 us (5.1 TB/s), down 23; 128 tokens 61 and 31.  Fragments
+// each: gate and up 42 us (5.2 TB/s), down 23; 100 tokens 51 and 31.  Fragments
 // loaded straight into registers, half a line at a time: 56 and 33, 129 and 65.
 template <int MF, int NF, int WAVES, int R, bool GLU>
 __global__ __launch_bounds__(WAVES * 64) void grouped_stream_kernel(Grouped a) {
@@ -334,44 +334,47 @@ __global__ __launch_bounds__(WAVES * 64) void grouped_stream_kernel(Grouped a) {
         for (int j = 0; j < MF; j++) acc[i][j] = mfma16l(wf[q][i], af[q][j], acc[i][j]);
   }
   __syncthreads();
-  typedef f32x4 Sums[NF][MF][64];
-  static_assert(sizeof(Sums) * (WAVES / 2) <= sizeof(ring), "room for the sums");
-  Sums* sums = reinterpret_cast<Sums*>(&ring[0][0][0]);
+  // Each wave adds up and stores its share of the tiles, as in linear_rows.hip.  A unit is a
+  // tile, or a gate's and its up's.
+  constexpr int TILES = GLU ? 2 : 1, UNITS = NF / TILES * MF;
+  typedef f32x4 Tile[64];
+  static_assert(sizeof(Tile) * UNITS * TILES * (WAVES - 1) <= sizeof(ring), "room for the sums");
+  Tile* sums = reinterpret_cast<Tile*>(&ring[0][0][0]);
 #pragma unroll
-  for (int n = WAVES / 2; n > 0; n >>= 1) {
-    if (wid >= n && wid < 2 * n) {
+  for (int u = 0; u < UNITS; u++) {
+    const int owner = u % WAVES;
+    if (wid == owner) continue;
 #pragma unroll
-      for (int i = 0; i < NF; i++)
-#pragma unroll
-        for (int j = 0; j < MF; j++) sums[wid - n][i][j][lane] = acc[i][j];
-    }
-    __syncthreads();
-    if (wid < n) {
-#pragma unroll
-      for (int i = 0; i < NF; i++)
-#pragma unroll
-        for (int j = 0; j < MF; j++) acc[i][j] += sums[wid][i][j][lane];
-    }
-    if (n > 1) __syncthreads();
+    for (int e = 0; e < TILES; e++)
+      sums[(u * TILES + e) * (WAVES - 1) + wid - (wid > owner)][lane] =
+          acc[u / MF * TILES + e][u % MF];
   }
-  if (wid > 0) return;
+  __syncthreads();
   const bool wide = ((a.ldo | a.go) & 3) == 0 && ((size_t)a.out & 7) == 0;
 #pragma unroll
-  for (int j = 0; j < MF; j++) {
+  for (int u = 0; u < UNITS; u++) {
+    const int owner = u % WAVES, i = u / MF * TILES, j = u % MF;
+    if (wid != owner) continue;
+    f32x4 sum[TILES];
+#pragma unroll
+    for (int e = 0; e < TILES; e++) {
+      f32x4 w[WAVES];
+#pragma unroll
+      for (int k = 0; k < WAVES; k++)
+        w[k] = k == owner ? acc[i + e][j]
+                          : sums[(u * TILES + e) * (WAVES - 1) + k - (k > owner)][lane];
+#pragma unroll
+      for (int n = WAVES / 2; n > 0; n >>= 1)
+#pragma unroll
+        for (int k = 0; k < n; k++) w[k] += w[k + n];
+      sum[e] = w[0];
+    }
     const int m = m0 + 16 * j + lo;
     if (m >= rows) continue;
     const int id = list ? list[m] : m;
     const float sc = a.scale ? a.scale[id] : 1.f;
     short* o = (short*)a.out + g * a.go + (long)id * a.ldo;
-    if constexpr (GLU) {
-#pragma unroll
-      for (int i = 0; i < NF; i += 2)
-        store_row<true>(a, o, n0 + i * 8 + 4 * hi, acc[i][j], acc[i + 1][j], sc, wide);
-    } else {
-#pragma unroll
-      for (int i = 0; i < NF; i++)
-        store_row<false>(a, o, n0 + i * 16 + 4 * hi, acc[i][j], acc[i][j], sc, wide);
-    }
+    store_row<GLU>(a, o, n0 + (GLU ? i * 8 : i * 16) + 4 * hi, sum[0], sum[TILES - 1], sc, wide);
   }
 }
 
@@ -435,12 +438,13 @@ __global__ __launch_bounds__(256) void route_plain_kernel(
   if (wid == 0) choose<64>(z, E, top, chosen + t * top, weight + t * top, true);
 }
 
-// 16 tokens per workgroup; the waves share the depth.  ET tiles of 16 experts.
-template <int ET>
-__global__ __launch_bounds__(256) void route_mfma_kernel(
+// 16 tokens per workgroup; the waves share the depth.  ET tiles of 16 experts.  A few tokens
+// are a chain of loads: 32 of 1536 with 16 experts 9.9 us with four waves, 7.6 with 16.
+template <int ET, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void route_mfma_kernel(
     const short* __restrict__ h, const short* __restrict__ wr, const short* __restrict__ bias,
     int* __restrict__ chosen, float* __restrict__ weight, long T, int W, int E, int top) {
-  __shared__ float z[4][16][ET * 16 + 1];
+  __shared__ float z[WAVES][16][ET * 16 + 1];
   const long t0 = blockIdx.x * 16L;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int lo = lane & 15, hi = lane >> 4;
@@ -449,7 +453,7 @@ __global__ __launch_bounds__(256) void route_mfma_kernel(
 #pragma unroll
   for (int i = 0; i < ET; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-  for (int k0 = wid * 32; k0 < W; k0 += 128) {
+  for (int k0 = wid * 32; k0 < W; k0 += WAVES * 32) {
     const bool in = k0 + 8 * hi < W;
     const s16x8 x = in ? *reinterpret_cast<const s16x8*>(hp + k0) : s16x8{};
 #pragma unroll
@@ -464,12 +468,15 @@ __global__ __launch_bounds__(256) void route_mfma_kernel(
 #pragma unroll
     for (int r = 0; r < 4; r++) z[wid][4 * hi + r][16 * i + lo] = acc[i][r];
   __syncthreads();
-  for (int i = threadIdx.x; i < 16 * E; i += 256) {
+  for (int i = threadIdx.x; i < 16 * E; i += WAVES * 64) {
     const int t = i / E, e = i % E;
-    z[0][t][e] = z[0][t][e] + z[1][t][e] + z[2][t][e] + z[3][t][e] + bf2f(bias[e]);
+    float x = z[0][t][e];
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) x += z[w][t][e];
+    z[0][t][e] = x + bf2f(bias[e]);
   }
   __syncthreads();
-  constexpr int L = ET == 1 ? 16 : ET == 2 ? 32 : 64, AT_ONCE = 256 / L;
+  constexpr int L = ET == 1 ? 16 : ET == 2 ? 32 : 64, AT_ONCE = WAVES * 64 / L;
   for (int t = threadIdx.x / L; t < 16; t += AT_ONCE)
     choose<L>(z[0][t], E, top, chosen + (t0 + t) * top, weight + (t0 + t) * top, t0 + t < T);
 }
@@ -576,7 +583,8 @@ static void launch_grouped(const Grouped& a, bool bf16) {
                      : each > 12 ? 2 : 1;
       // Four waves with a chunk of their own each.  Where 64 weight rows to a workgroup
       // leave CUs idle, 32 and two chunks: one token's 4 experts of 1536 x 2240 7.7 us
-      // against 10.
+      // against 10; and for a few rows' gate and up: 16 experts of 1536 x 2240 42.4 us, 43.9
+      // with 64 rows, of 4096 x 3584 138 and 143, down 24.5 and 22.9.
       const long busy = std::min<long>(tiles_of(16 * mf), a.rows);
 #define STREAM(MF, NF, R)                                                                      \
   hipLaunchKernelGGL((grouped_stream_kernel<MF, NF, 4, R, GLU>),                               \
@@ -591,6 +599,8 @@ static void launch_grouped(const Grouped& a, bool bf16) {
         STREAM(4, 4, 1);
       } else if (mf == 2) {
         STREAM(2, 4, 1);
+      } else if (GLU) {
+        STREAM(1, 2, 2);
       } else {
         STREAM(1, 4, 1);
       }
@@ -656,18 +666,18 @@ std::vector<torch::Tensor> moe_route(torch::Tensor h, torch::Tensor router, torc
   auto counts = torch::empty({E}, ints);
   TORCH_CHECK(T > 0 && T * top < (1L << 31));
   auto stream = at::hip::getCurrentHIPStream();
-#define ROUTE(ET)                                                                            \
-  hipLaunchKernelGGL((route_mfma_kernel<ET>), dim3((T + 15) / 16), dim3(256), 0, stream,     \
+#define ROUTE(ET, WAVES)                                                                     \
+  hipLaunchKernelGGL((route_mfma_kernel<ET, WAVES>), dim3((T + 15) / 16), dim3(WAVES * 64), 0, stream, \
                      (const short*)h.data_ptr(), (const short*)router.data_ptr(),            \
                      (const short*)bias.data_ptr(), chosen.data_ptr<int>(),                  \
                      weight.data_ptr<float>(), T, (int)W, (int)E, (int)top)
   if (is_bf16(h) && W % 8 == 0 && E <= 256 && (uintptr_t)h.data_ptr() % 16 == 0 &&
       (uintptr_t)router.data_ptr() % 16 == 0) {
-    if (E <= 16) ROUTE(1);
-    else if (E <= 32) ROUTE(2);
-    else if (E <= 64) ROUTE(4);
-    else if (E <= 128) ROUTE(8);
-    else ROUTE(16);
+    if (E <= 16) ROUTE(1, 16);
+    else if (E <= 32) ROUTE(2, 4);
+    else if (E <= 64) ROUTE(4, 4);
+    else if (E <= 128) ROUTE(8, 4);
+    else ROUTE(16, 4);
   } else if (is_bf16(h))
     hipLaunchKernelGGL((route_plain_kernel<short>), dim3(T), dim3(256), 4 * E, stream,
                        (const short*)h.data_ptr(), (const short*)router.data_ptr(),
