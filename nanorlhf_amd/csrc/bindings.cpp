@@ -33,11 +33,13 @@ void adamw_step_many(std::vector<torch::Tensor> p, std::vector<torch::Tensor> g,
 std::vector<torch::Tensor> decode_inputs(torch::Tensor lens, torch::Tensor bt, long page_size);
 void decode_commit(torch::Tensor tokens, c10::optional<torch::Tensor> lps, torch::Tensor out,
                    torch::Tensor lp, torch::Tensor count, torch::Tensor lens, torch::Tensor last,
-                   torch::Tensor finished, c10::optional<long> stop);
+                   torch::Tensor finished, c10::optional<long> stop,
+                   c10::optional<torch::Tensor> step);
 torch::Tensor sample_topp(torch::Tensor logits, double temperature, double top_p,
                           long seed, long step);
 std::vector<torch::Tensor> sample_topp_dev(torch::Tensor logits, double temperature,
-                                           double top_p, long seed, torch::Tensor step);
+                                           double top_p, long seed, torch::Tensor step,
+                                           long ahead);
 // masked.hip
 std::vector<torch::Tensor> masked_moments(torch::Tensor v, torch::Tensor mask);
 torch::Tensor whiten_apply(torch::Tensor v, double mean, double invstd, double shift);
@@ -96,9 +98,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("adamw_step", &adamw_step);
   m.def("adamw_step_many", &adamw_step_many);
   m.def("decode_inputs", &decode_inputs);
-  m.def("decode_commit", &decode_commit);
+  m.def("decode_commit", &decode_commit, py::arg("tokens"), py::arg("lps"), py::arg("out"),
+        py::arg("lp"), py::arg("count"), py::arg("lens"), py::arg("last"), py::arg("finished"),
+        py::arg("stop"), py::arg("step") = py::none());
   m.def("sample_topp", &sample_topp);
-  m.def("sample_topp_dev", &sample_topp_dev);
+  m.def("sample_topp_dev", &sample_topp_dev, py::arg("logits"), py::arg("temperature"),
+        py::arg("top_p"), py::arg("seed"), py::arg("step"), py::arg("ahead") = 0);
   m.def("masked_moments", &masked_moments);
   m.def("whiten_apply", &whiten_apply);
   m.def("lora_gemm_big", &lora_gemm_big);

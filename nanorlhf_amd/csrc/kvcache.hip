@@ -182,7 +182,7 @@ std::vector<torch::Tensor> qkv_rope_append(torch::Tensor qkv, torch::Tensor tabl
     a.Hkv = Hkv;
     a.D = D;
     a.ps = ps;
-    const dim3 grid((units + 255) / 256), block(256);
+    const dim3 block(qkv_block(units)), grid((units + block.x - 1) / block.x);
 #define LAUNCH(CT, P) hipLaunchKernelGGL((qkv_rope_kernel<CT, P>), grid, block, 0, stream, a, units)
     if (fp8) { if (parts) LAUNCH(unsigned char, true); else LAUNCH(unsigned char, false); }
     else { if (parts) LAUNCH(short, true); else LAUNCH(short, false); }

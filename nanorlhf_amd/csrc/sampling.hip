@@ -268,7 +268,7 @@ void sample_topp_kernel(const LT* __restrict__ logits,
                         unsigned long long step_imm,
                         const long* __restrict__ step_ptr) {
   __shared__ Scratch s;
-  const unsigned long long step = step_ptr ? (unsigned long long)*step_ptr : step_imm;
+  const unsigned long long step = step_imm + (step_ptr ? (unsigned long long)*step_ptr : 0);
   const long row = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   Row<LT, NV> r;
@@ -480,8 +480,9 @@ torch::Tensor sample_topp(torch::Tensor logits, double temperature, double top_p
 }
 
 std::vector<torch::Tensor> sample_topp_dev(torch::Tensor logits, double temperature,
-                                           double top_p, long seed, torch::Tensor step) {
-  // step: int64 [1] device tensor, read inside the kernel — safe under
+                                           double top_p, long seed, torch::Tensor step,
+                                           long ahead) {
+  // step: int64 [1] device tensor, read inside the kernel, and `ahead` more — safe under
   // hipGraph capture/replay (the immediate-arg form would freeze the step).
   // Also returns the chosen token's logprob (vLLM logprobs parity).
   TORCH_CHECK(logits.dim() == 2 && logits.is_contiguous());
@@ -492,14 +493,15 @@ std::vector<torch::Tensor> sample_topp_dev(torch::Tensor logits, double temperat
   auto out = torch::empty({B}, logits.options().dtype(torch::kLong));
   auto lp = torch::empty({B}, logits.options().dtype(torch::kFloat32));
   if (B == 0) return {out, lp};
-  launch_sampler(logits, out, lp.data_ptr<float>(), temperature, top_p, seed, 0,
+  launch_sampler(logits, out, lp.data_ptr<float>(), temperature, top_p, seed, ahead,
                  step.data_ptr<long>());
   return {out, lp};
 }
 
 // ------------------------------------------------------------ decode batch
 // What a decode step does to its rows beside the model: where each row's token
-// goes in the cache, and afterwards what the sampled token changes.  A thread a
+// goes in the cache, and afterwards what the sampled token changes, the counter of the
+// sampling among it.  A thread a
 // row; bound by the launch, of which tensor operations took 26 a step: a rollout
 // of 64 rows and 96 tokens through 6 layers went from 85.2 to 78.5 ms.
 __global__ __launch_bounds__(256)
@@ -517,8 +519,9 @@ void decode_commit_kernel(const long* __restrict__ tokens, const float* __restri
                           long* __restrict__ out, float* __restrict__ lp, int* __restrict__ count,
                           int* __restrict__ lens, long* __restrict__ last,
                           bool* __restrict__ finished, int B, int most, long stop,
-                          bool has_stop) {
+                          bool has_stop, long* __restrict__ step) {
   const int b = blockIdx.x * 256 + threadIdx.x;
+  if (b == 0 && step) *step += 1;
   if (b >= B) return;
   const int n = count[b];
   if (finished[b] || n >= most) {
@@ -552,8 +555,11 @@ std::vector<torch::Tensor> decode_inputs(torch::Tensor lens, torch::Tensor bt, l
 
 void decode_commit(torch::Tensor tokens, c10::optional<torch::Tensor> lps, torch::Tensor out,
                    torch::Tensor lp, torch::Tensor count, torch::Tensor lens, torch::Tensor last,
-                   torch::Tensor finished, c10::optional<long> stop) {
+                   torch::Tensor finished, c10::optional<long> stop,
+                   c10::optional<torch::Tensor> step) {
   const int B = out.size(0), most = out.size(1);
+  TORCH_CHECK(!step || (step->is_cuda() && step->scalar_type() == at::kLong && step->numel() == 1),
+              "decode_commit: an int64 step");
   for (const auto& t : {tokens, count, lens, last, finished})
     TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.dim() == 1 && t.size(0) == B,
                 "decode_commit: one contiguous entry a row");
@@ -570,6 +576,7 @@ void decode_commit(torch::Tensor tokens, c10::optional<torch::Tensor> lps, torch
                        lps ? lps->data_ptr<float>() : nullptr, out.data_ptr<long>(),
                        lp.data_ptr<float>(), count.data_ptr<int>(), lens.data_ptr<int>(),
                        last.data_ptr<long>(), finished.data_ptr<bool>(), B, most,
-                       stop.value_or(0), stop.has_value());
+                       stop.value_or(0), stop.has_value(),
+                       step ? step->data_ptr<long>() : nullptr);
   HIP_CHECK_LAST();
 }

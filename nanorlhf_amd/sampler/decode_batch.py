@@ -94,14 +94,18 @@ class DecodeBatch:
         slots = page * ps + pos % ps
         return self.last_tok, pos, slots, self.seq_lens, self.bt
 
-    def commit(self, tokens: torch.Tensor, lps: torch.Tensor | None = None):
-        """Record sampled tokens; advance lengths.  Fully IN-PLACE on the
+    def commit(self, tokens: torch.Tensor, lps: torch.Tensor | None = None,
+               step: torch.Tensor | None = None):
+        """Record sampled tokens; advance lengths, and `step` by one.  Fully IN-PLACE on the
         batch's state tensors so the whole step is hipGraph-capturable (no
         host sync, no tensor reassignment)."""
         if tokens.is_cuda:
             ops.ext().decode_commit(tokens, lps, self.out, self.lp, self.gen_count,
-                                    self.seq_lens, self.last_tok, self.finished, self.stop)
+                                    self.seq_lens, self.last_tok, self.finished, self.stop,
+                                    step)
             return
+        if step is not None:
+            step.add_(1)
         write = (~self.finished) & (self.gen_count < self.max_tokens)
         idx = self.gen_count.clamp(max=self.max_tokens - 1).long().unsqueeze(1)
         cur = self.out.gather(1, idx).squeeze(1)

@@ -82,18 +82,21 @@ class SamplerEngine:
 
     # ----------------------------------------------------------------- utils
     def _sample_from_hidden(self, hidden_last: torch.Tensor,
-                            params: SamplingParams):
+                            params: SamplingParams, counts: bool = True):
         """Returns (tokens [B], logprobs [B] fp32) — the chosen token's
         logprob under the temperature-scaled softmax (vLLM logprobs parity;
         matches the scoring pass's logits/temperature quirk)."""
         logits = self.model.logits(hidden_last)
         if self._step_dev is not None:
-            # device-side step counter: correct under hipGraph replay
-            self._step_dev.add_(1)
+            # device-side step counter: correct under hipGraph replay; a decode step's
+            # commit counts it
+            if counts:
+                self._step_dev.add_(1)
             tok, lp = ops.ext().sample_topp_dev(logits.contiguous(),
                                                 float(params.temperature),
                                                 float(params.top_p),
-                                                int(params.seed), self._step_dev)
+                                                int(params.seed), self._step_dev,
+                                                0 if counts else 1)
             return tok, lp
         self._sample_step += 1
         tok = ops.sample_tokens(logits, params.temperature, params.top_p,
@@ -259,8 +262,8 @@ class SamplerEngine:
                           block_tables=bt, seq_lens=seq_lens,
                           state_slots=db.state_slots)
         hidden = self.model(ids, ctx)
-        tokens, lps = self._sample_from_hidden(hidden, params)
-        db.commit(tokens, lps)
+        tokens, lps = self._sample_from_hidden(hidden, params, counts=False)
+        db.commit(tokens, lps, self._step_dev)
 
     def _run_decode_step(self, db: DecodeBatch, params: SamplingParams) -> int:
         """One decode step; hipGraph-captured and replayed when the batch

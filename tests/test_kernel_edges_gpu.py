@@ -526,14 +526,27 @@ def test_decode_batch_matches_its_tensor_form(B, stop):
     for db in both:
         for k, v in state.items():
             setattr(db, k, v.clone().to(db.device))
+    counts = [torch.zeros(1, dtype=torch.long, device=db.device) for db in both]
     for step in range(most + 1):
         for a, b in zip(both[0].step_inputs(), both[1].step_inputs()):
             assert a.dtype == b.dtype and torch.equal(a, b.cpu())
         tok, lp = torch.randint(0, 5, (B,), generator=g), torch.randn(B, generator=g)
-        for db in both:
-            db.commit(tok.to(db.device), None if step == 1 else lp.to(db.device))
+        for db, n in zip(both, counts):
+            db.commit(tok.to(db.device), None if step == 1 else lp.to(db.device),
+                      None if step == 2 else n)
         for k in state:
             assert torch.equal(getattr(both[0], k), getattr(both[1], k).cpu()), k
+    assert [int(n) for n in counts] == [most, most]
+
+
+@pytest.mark.parametrize("temperature", [0.0, 0.7])
+def test_sampling_ahead_of_its_counter(temperature):
+    x = rnd(8, 1000, seed=1, scale=3.0)
+    for n in range(20):
+        step, before = (torch.full((1,), k, device=DEV) for k in (n + 1, n))
+        want = ops.ext().sample_topp_dev(x, temperature, 0.95, 5, step)
+        got = ops.ext().sample_topp_dev(x, temperature, 0.95, 5, before, 1)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)) and int(before) == n
 
 
 # ----------------------------------------------- attention of prompt portions
