@@ -407,8 +407,9 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
           for (int q = 0; q < 2; q++)
 #pragma unroll
             for (int c = 0; c < 2; c++)
-              v[q][c] = glu<ACT>(acc[i][0][c][r + q], acc[i][1][c][r + q]) *
-                        (GROUPED ? scale_of(gm0 + 16 * i + r + q) : 1.f);
+              v[q][c] = GROUPED ? act_silu(acc[i][0][c][r + q]) * acc[i][1][c][r + q] *
+                                      scale_of(gm0 + 16 * i + r + q)
+                                : glu<ACT>(acc[i][0][c][r + q], acc[i][1][c][r + q]);
           if (VEC) {
             typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
             const unsigned a = pack2bf(v[0][0], v[0][1]), b = pack2bf(v[1][0], v[1][1]);
@@ -454,10 +455,12 @@ void launch_big(Big p) {
 // Grouped products of whole steps of the depth, N and the strides of y multiples of 4: `most`
 // tiles of rows at most.  A workgroup counts the groups' tiles at its start and finds the
 // group of each as it comes to it; which rows of x and y they are is kept in LDS.  16
-// experts of 1536 x 2240, 1000 rows each, gate and up 193 us (1140 TFLOP/s), down 100; in
-// tiles of 128 that wait at a barrier a step 299 and 145.
+// experts of 1536 x 2240, 1000 rows each, gate and up 211 us (1050 TFLOP/s), down 100; in
+// tiles of 128 that wait at a barrier a step 299 and 145.  Silu is divided, as those have it,
+// which takes 17 us of the 211: the bits are theirs, on which a router's near ties hang.
 template <int ACT>
 void launch_big_grouped(Big p, long most) {
+  static_assert(ACT == NO_ACT || ACT == SILU_GLU, "silu alone is divided");
   const int cus = at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
   constexpr int TN = ACT ? BIG / 2 : BIG;
   p.grid_n = (p.N + TN - 1) / TN;

@@ -439,7 +439,8 @@ __global__ __launch_bounds__(256) void route_plain_kernel(
 }
 
 // 16 tokens per workgroup; the waves share the depth.  ET tiles of 16 experts.  A few tokens
-// are a chain of loads: 32 of 1536 with 16 experts 9.9 us with four waves, 7.6 with 16.
+// are a chain of loads: 32 of 1536 with 16 experts 9.9 us with four waves, 7.6 with 16.  Many
+// fill the CUs anyway: 4000 tokens and their lists 25.5 us with either.
 template <int ET, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void route_mfma_kernel(
     const short* __restrict__ h, const short* __restrict__ wr, const short* __restrict__ bias,
@@ -481,7 +482,9 @@ __global__ __launch_bounds__(WAVES * 64) void route_mfma_kernel(
     choose<L>(z[0][t], E, top, chosen + (t0 + t) * top, weight + (t0 + t) * top, t0 + t < T);
 }
 
-// One workgroup per expert: the rows that chose it, in order.
+// One workgroup per expert: the rows that chose it, in order.  Four choices to a thread at a
+// time, for every round waits for its loads and twice at a barrier: 16000 choices of 16
+// experts 13.2 us with one each, 5.8 now.
 __global__ __launch_bounds__(1024) void expert_lists_kernel(
     const int* __restrict__ chosen, int* __restrict__ lists, int* __restrict__ counts, long n,
     int cap) {
@@ -489,16 +492,34 @@ __global__ __launch_bounds__(1024) void expert_lists_kernel(
   const int e = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   int* list = lists + (long)e * cap;
   int total = 0;
-  for (long base = 0; base < n; base += 1024) {
-    const long i = base + threadIdx.x;
-    const bool hit = i < n && chosen[i] == e;
-    const unsigned long long mask = __ballot(hit);
-    if (lane == 0) wave_n[wid] = __popcll(mask);
+  for (long base = 0; base < n; base += 4096) {
+    const long i = base + 4 * threadIdx.x;
+    int c[4];
+    if (i + 4 <= n) {
+      *reinterpret_cast<int4*>(c) = *reinterpret_cast<const int4*>(chosen + i);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) c[j] = i + j < n ? chosen[i + j] : -1;
+    }
+    int mine = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) mine += c[j] == e;
+    int upto = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int x = __shfl_up(upto, off);
+      if (lane >= off) upto += x;
+    }
+    if (lane == 63) wave_n[wid] = upto;
     __syncthreads();
-    int at = total;
-    for (int w = 0; w < wid; w++) at += wave_n[w];
-    for (int w = 0; w < 16; w++) total += wave_n[w];
-    if (hit) list[at + __popcll(mask & ((1ull << lane) - 1))] = (int)i;
+    int at = total + upto - mine;
+    for (int w = 0; w < 16; w++) {
+      if (w < wid) at += wave_n[w];
+      total += wave_n[w];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (c[j] == e) list[at++] = (int)(i + j);
     __syncthreads();
   }
   if (threadIdx.x == 0) counts[e] = total;
@@ -508,10 +529,10 @@ __global__ __launch_bounds__(1024) void expert_lists_kernel(
 // Whether gemm_big.h's kernel takes these, with `tm` tiles of rows at most: that is what its
 // 32-bit offsets, whole steps and stores of four columns can do, and where its tiles of 256
 // fill the CUs and their columns.  us, tiles of 128 / it: 16 experts of 1536 x 2240, gate and
-// up, 140 rows each (432 tiles) 76 / 67, 1000 rows 299 / 193, down 180 rows (162) 41 / 44, 256
+// up, 250 rows each (576 tiles) 102 / 82, 1000 rows 299 / 211, down 180 rows (162) 41 / 44, 256
 // (192) 68 / 46; 4 experts, 300 rows (144) 33 / 36, 400 (180) 50 / 34; 12 heads of 512 x 128,
 // 4000 rows 16.4 / 18.3.  Up to 128 rows half of a tile is empty and it takes a long product:
-// 110 rows of 1536 x 2240 65 / 66, 80 of 2048 x 2752 133 / 99, 56 of 3584 x 4096 143 / 95.
+// 110 rows of 1536 x 2240 65 / 66, 100 of 2048 x 2752 139 / 108, 56 of 3584 x 4096 143 / 95.
 static bool takes_big(const Grouped& a, long each, long tm, int width) {
   const long tn = (a.N + width - 1) / width;
   return a.G <= 64 && a.K > 0 && a.K % 64 == 0 && a.N % 4 == 0 && (a.ldo | a.go) % 4 == 0 &&
@@ -673,7 +694,8 @@ std::vector<torch::Tensor> moe_route(torch::Tensor h, torch::Tensor router, torc
                      weight.data_ptr<float>(), T, (int)W, (int)E, (int)top)
   if (is_bf16(h) && W % 8 == 0 && E <= 256 && (uintptr_t)h.data_ptr() % 16 == 0 &&
       (uintptr_t)router.data_ptr() % 16 == 0) {
-    if (E <= 16) ROUTE(1, 16);
+    if (E <= 16 && T <= 512) ROUTE(1, 16);
+    else if (E <= 16) ROUTE(1, 4);
     else if (E <= 32) ROUTE(2, 4);
     else if (E <= 64) ROUTE(4, 4);
     else if (E <= 128) ROUTE(8, 4);

@@ -13,8 +13,13 @@ import torch
 import torch.nn.functional as F
 
 from . import serve_ext
+from .linear import here, plain_call
 
-STACKED_ROWS = 256     # rows up to which separate GEMMs cost more than one launch
+# Rows up to which separate GEMMs cost more than one launch, whatever the sizes.  With more
+# one launch of whole steps of the depth: 4 products of 1536 x 1536, 1000 rows 30 us, four
+# library calls 74 (and 20 us each on the host), 4000 rows 71 / 87, 12000 186 / 229; of 4096 x
+# 4096, 4000 rows 366 / 365.
+STACKED_ROWS = 256
 
 
 def group_linear(x: torch.Tensor, w: torch.Tensor,
@@ -29,10 +34,20 @@ def group_linear(x: torch.Tensor, w: torch.Tensor,
     return out.copy_(torch.einsum("tgk,gnk->tgn", x.float(), w.float()))
 
 
+def _stacks(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (here(x) and plain_call(x, w) and x.dim() == w.dim() == 3 and x.dtype == w.dtype
+            and w.device == x.device and x.shape[0] == w.shape[0] <= 64
+            and x.shape[2] == w.shape[2] and x.shape[2] % 64 == 0 and w.shape[1] % 4 == 0
+            and w.shape[1] >= 256 and x.is_contiguous() and w.is_contiguous()
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and x.shape[1] * x.shape[2] < 1 << 30)
+
+
 def stacked_linear(x: torch.Tensor, w: torch.Tensor):
     """x [G, T, K], w [G, N, K] -> G results [T, N]: one launch while the rows
-    are few."""
-    if x.is_cuda and x.dtype == torch.bfloat16 and x.shape[1] <= STACKED_ROWS:
+    are few, or the kernel for many takes them."""
+    if x.is_cuda and x.dtype == torch.bfloat16 and (
+            x.shape[1] <= STACKED_ROWS or _stacks(x, w)):
         out = torch.empty(x.shape[0], x.shape[1], w.shape[1], dtype=x.dtype, device=x.device)
         group_linear(x.transpose(0, 1), w, out.transpose(0, 1))
         return out

@@ -768,6 +768,23 @@ def test_grouped_product_of_many_rows(T, G, N, K):
     assert rel(ops.group_linear(x, w), want) < 0.002       # one rounding, 2^-9 at most
 
 
+@pytest.mark.parametrize("T", [300, 512])
+def test_stacked_products_of_many_rows(T):
+    x, w = rnd(4, T, 192, seed=1), rnd(4, 516, 192, seed=2, scale=192 ** -0.5)
+    with torch.no_grad():
+        for got, a, b in zip(ops.stacked_linear(x, w), x, w):
+            assert rel(got, a.double() @ b.double().t()) < 0.002       # one rounding, 2^-9
+
+
+@pytest.mark.parametrize("n", [1, 4095, 4096, 4099, 9000])
+def test_lists_of_a_route_are_in_order(n):
+    h, router = rnd(n, 64, seed=1), rnd(5, 64, seed=2)
+    chosen, _, lists, counts = ops.moe_route(h, router, rnd(5, seed=3), 2)
+    for e in range(5):
+        rows = (chosen.flatten() == e).nonzero(as_tuple=True)[0]
+        assert int(counts[e]) == len(rows) and torch.equal(lists[e, :len(rows)].long(), rows)
+
+
 @pytest.mark.parametrize("M", [1, 63, 64, 65, 240, 1537, 25000])
 @pytest.mark.parametrize("C", [8, 64, 120, 192, 1536, 1992])
 def test_product_down_to_the_rank(M, C):
