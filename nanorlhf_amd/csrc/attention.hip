@@ -473,15 +473,17 @@ __global__ void fa_bwd_sum_kernel(const float* __restrict__ part, short* __restr
 // Heads that workgroups are taken from at a time.  As many as fill every chiplet's 32 CUs
 // twice: what runs there together then shares the tiles that its L2 holds.  Or all, so that
 // the longest walks of all come first, which a causal grid needs to end evenly unless it is
-// several rounds of the workgroups that run at a time.  Forward, all heads / a window, us:
+// several rounds of the workgroups that run at a time and the last window, which may hold the
+// longest sequence, is a small part of it.  Forward, all heads / a window, us:
 // 80 x 800 not causal, 16 heads of 64 456 / 371 (70% of the tiles' requests missed the L2);
-// causal, 12 heads over 2 of 128: 56 x 870 256 / 221, 8 x 3000 354 / 280, 16 x 6000 2550 /
-// 2050, 5 x 6500 896 / 880; 3.5 rounds, 28 heads over 4, 4 x 2000 139 / 146; 2.8 rounds, 14
-// heads of 64, 20 x 1200 102 / 121.  Backward of the first 1354 / 1118.  The walks of dk and dv
-// are few and long: causal, 40 x 1200 1041 / 1291.
+// causal, 12 heads over 2 of 128: 56 x 870 256 / 221, 16 x 1500 194 / 167, 16 x 6000 2550 /
+// 2050; 3.5 rounds, 28 heads over 4, 4 x 2000 139 / 146; 2.8 rounds, 14 heads of 64, 20 x
+// 1200 102 / 121; 7.5 windows, 5 x 6500 896 / 880 with the longest sequence ahead, but forward
+// and backward 3811 / 3997 with it behind.  Backward of the first 1354 / 1118.  The walks of
+// dk and dv are few and long: causal, 40 x 1200 1041 / 1291.
 static unsigned head_window(long heads, long tiles, long rounds, bool causal) {
-  if (causal && rounds < 4) return heads;
-  return 8 * std::max(64 / std::max(tiles, 1L), 1L);
+  const long window = 8 * std::max(64 / std::max(tiles, 1L), 1L);
+  return causal && (rounds < 4 || heads < 8 * window) ? heads : window;
 }
 
 #define FA_BY_WIDTH(CALL)                                                  \
