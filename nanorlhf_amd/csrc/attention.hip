@@ -88,9 +88,14 @@ DEVINL void store_row(short* __restrict__ dst, const f32x16_t* acc, float mul, i
 struct Place { int seq, head, s0, len, tile; };
 template <bool LAST_FIRST>
 DEVINL Place place(const int* __restrict__ cu, int heads, unsigned window) {
-  const unsigned n = gridDim.x, tiles = gridDim.y, at = blockIdx.y * n + blockIdx.x;
-  const unsigned begin = at / (window * tiles) * window, wide = min(window, n - begin);
-  const unsigned in = at - begin * tiles, x = begin + in % wide, y = in / wide;
+  const unsigned n = gridDim.x, tiles = gridDim.y;
+  unsigned x = blockIdx.x, y = blockIdx.y;
+  if (window < n) {
+    const unsigned at = y * n + x, begin = at / (window * tiles) * window;
+    const unsigned wide = min(window, n - begin), in = at - begin * tiles;
+    x = begin + in % wide;
+    y = in / wide;
+  }
   Place p;
   p.seq = x / heads;
   p.head = x % heads;
@@ -537,12 +542,15 @@ std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
   float* lse2 = drow + (long)Hq * T;
   // A workgroup of dk and dv walks the group's q heads one after the other.
   // Where that leaves too few to fill 256 CUs twice, with spare to even out
-  // causal tiles, they are divided among `parts`.  Whole backward, 12 heads over
-  // 2: 5 x 6500 tokens (518 workgroups undivided) 3.95 ms with 1 part, 2.92 with
-  // 2, 2.87 with 3; 56 x 870 (872) 0.72 with 1, 0.77 with 2, 0.89 with 6.
+  // causal tiles, they are divided among `parts`, the finer the longer the longest of
+  // those walks is.  Whole backward, 12 heads over
+  // 2: 5 x 6500 tokens (518 workgroups undivided) 3.95 ms with 1 part, 2.87 with
+  // 2, 2.83 with 3; 6 x 4000 (400) 1.51 with 2, 1.36 with 3, 3 x 6000 (290) 1.22 with 3, 1.13
+  // with 6; 8 x 3000 (390) 1.13 with 2, 1.16 with 3; 56 x 870 (872) 0.72 with 1, 0.77 with
+  // 2, 0.89 with 6.
   int parts = 1;
-  const long tiles = (T / ROWS + B) * Hkv;
-  while (parts < G && (G % parts || tiles * parts < 768)) parts++;
+  const long tiles = (T / ROWS + B) * Hkv, wanted = max_seqlen >= 6000 ? 1100 : 768;
+  while (parts < G && (G % parts || tiles * parts < wanted)) parts++;
   const long n = T * Hkv * D;
   torch::Tensor sums;
   if (parts > 1) sums = torch::empty({2, (long)parts, n}, f32);
