@@ -539,6 +539,29 @@ def test_decode_batch_matches_its_tensor_form(B, stop):
     assert [int(n) for n in counts] == [most, most]
 
 
+@pytest.mark.parametrize("rows", [5, 40])
+def test_listeners_get_sums_and_no_parts(rows):
+    """Few rows pass on parts of the projections' depth, but not where somebody listens."""
+    from nanorlhf_amd.models import CausalLM, get_config, pack_sequences
+    torch.manual_seed(0)
+    model = CausalLM(get_config("qwen2.5-1.5b", num_layers=2, vocab_size=512)).to(DEV).bfloat16()
+    ids, cu, mx, pos = pack_sequences([torch.arange(rows)], device=DEV)
+    seen = []
+
+    def listen(module, args, out):
+        seen.extend(out if isinstance(out, tuple) else (out,))
+
+    with torch.no_grad():
+        alone = model(ids, CausalLM.train_ctx(cu, mx, pos))
+        layer = model.model.layers
+        for m in (layer[0], layer[0].self_attn, layer[0].mlp, layer[1].self_attn, layer[1].mlp):
+            m.register_forward_hook(listen)
+        heard = model(ids, CausalLM.train_ctx(cu, mx, pos))
+    assert len(seen) == 6
+    assert all(t.shape == (rows, 1536) and t.dtype == torch.bfloat16 for t in seen)
+    assert rel(alone, heard) < 0.01        # the same sums in another order, rounded to 2^-9
+
+
 @pytest.mark.parametrize("temperature", [0.0, 0.7])
 def test_sampling_ahead_of_its_counter(temperature):
     x = rnd(8, 1000, seed=1, scale=3.0)
