@@ -39,13 +39,19 @@ def lora_gemm_ref(x, w, u=None, b=None, bias=None):
 # "fused"    = the single wide-K MFMA kernel (wins when our GEMM rate is
 #              within the fusion savings of hipBLASLt — e.g. N-heavy shapes);
 # "epilogue" = hipBLASLt base GEMM + the custom rank-64 lora_add_ MFMA pass
-#              (wins on deep-K shapes where the library GEMM is far ahead).
-# The fused kernel rounds y once, the epilogue twice, so the epilogue has to be
-# clearly faster.
+#              (wins on deep K: few rows, which the library divides, by far).
+# They round y differently (the fused kernel once, the epilogue twice), so a choice that
+# the timer's noise could turn would give a step other bits in another process.  One of them
+# is the rule and the other has to be clearly faster: the fused kernel up to DEEP, where
+# the epilogue's pass over y costs more than a tenth of the product (448 / K of it: y twice
+# at 5.8 TB/s, the product at 1.3 PFLOP/s), the epilogue beyond, where they come close.
+# 46673 rows, fused / epilogue in us: 1536 x 1536 241 / 296, 2048 x 1536 250 / 330, 17920 x
+# 1536 2205 / 2610; 1536 x 8960 1020 / 1069, 1536 x 17920 1990 / 2015.
 # Measured once per key on first touch (events, ~1 ms): a few rows say nothing about
 # many, for which lora_gemm is another kernel, nor a square weight's dx, which has no
 # bias, about its y.
 _TUNE: dict[tuple, dict] = {}
+DEEP = 4096
 
 
 def _time_cuda(fn, reps: int = 3) -> float:
@@ -77,7 +83,7 @@ def _choose_strategy(x, w, u, b, bias) -> str:
             y = torch.nn.functional.linear(x, w, bias)
             ext().lora_add_(y, u, b)
         t_ep = _time_cuda(ep)
-        st = "fused" if t_fused <= 1.1 * t_ep else "epilogue"
+        st = "fused" if t_fused <= (1.1 if K <= DEEP else 0.9) * t_ep else "epilogue"
         known[key] = st
     return st
 

@@ -65,6 +65,22 @@ def test_adapter_strategies_are_kept_by_what_the_kernels_depend_on(monkeypatch):
     assert next(times, None) is None and len(lora._TUNE[64, 64]) == 3
 
 
+@pytest.mark.parametrize("K,rule", [(64, "fused"), (4096, "fused"), (4160, "epilogue"),
+                                    (8960, "epilogue")])
+def test_near_ties_of_the_adapter_strategies_do_not_hang_on_the_timer(monkeypatch, K, rule):
+    from types import SimpleNamespace
+    from nanorlhf_amd.ops import lora
+    monkeypatch.setattr(lora, "ext", lambda: SimpleNamespace(
+        lora_gemm_big=lambda M, N, K: True, lora_gemm=None, lora_add_=None))
+    w, x = torch.zeros(64, K), torch.zeros(300, K)
+    # fused against epilogue
+    for ratio, want in [(0.95, rule), (1.0, rule), (1.05, rule), (0.5, "fused"), (2.0, "epilogue")]:
+        monkeypatch.setattr(lora, "_TUNE", {})
+        times = iter([ratio, 1.0])
+        monkeypatch.setattr(lora, "_time_cuda", lambda fn: next(times))
+        assert lora._choose_strategy(x, w, None, None, None) == want
+
+
 def test_a_capture_takes_the_strategy_that_is_known_of_its_weight(monkeypatch):
     from types import SimpleNamespace
     from nanorlhf_amd.ops import lora
