@@ -45,6 +45,7 @@ std::vector<torch::Tensor> masked_moments(torch::Tensor v, torch::Tensor mask);
 torch::Tensor whiten_apply(torch::Tensor v, double mean, double invstd, double shift);
 // lora.hip
 bool lora_gemm_big(long M, long N, long K);
+long lora_gemm_tiles(long M, long K);
 torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
                         c10::optional<torch::Tensor> u,
                         c10::optional<torch::Tensor> b,
@@ -107,6 +108,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("masked_moments", &masked_moments);
   m.def("whiten_apply", &whiten_apply);
   m.def("lora_gemm_big", &lora_gemm_big);
+  m.def("lora_gemm_tiles", &lora_gemm_tiles);
   m.def("lora_gemm", &lora_gemm, py::arg("x"), py::arg("w"),
         py::arg("u") = py::none(), py::arg("b") = py::none(),
         py::arg("bias") = py::none());

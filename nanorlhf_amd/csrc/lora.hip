@@ -151,7 +151,7 @@ __global__ void lora_gemm_kernel(const short* __restrict__ x,
 }
 
 // Whether a product has as many tiles of 256 as tell something about still larger ones, for
-// which a product of few says nothing: what its strategy is kept by.
+// which a product of few says nothing: what its strategy is kept by, beside its kernel.
 bool lora_gemm_big(long M, long N, long K) {
   return ((M + BIG - 1) / BIG) * ((N + BIG - 1) / BIG) >= 96 && K < (1L << 22);
 }
@@ -162,6 +162,7 @@ bool lora_gemm_big(long M, long N, long K) {
 // for their loads (500 x 896 x 9728 139 and 140).  From a depth of 2^22 on a big tile's
 // 32-bit offsets come near their end.
 static bool takes_big(long M, long K) { return M > 128 && K < (1L << 22); }
+long lora_gemm_tiles(long M, long K) { return takes_big(M, K) ? BIG : 128; }
 
 torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
                         c10::optional<torch::Tensor> u,

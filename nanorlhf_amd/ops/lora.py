@@ -34,8 +34,8 @@ def lora_gemm_ref(x, w, u=None, b=None, bias=None):
     return y.to(x.dtype)
 
 
-# Strategy cache: weight shape (N, K) -> {(whether lora_gemm takes its big tiles, whether
-# there is a bias, device): "fused" | "epilogue"}.
+# Strategy cache: weight shape (N, K) -> {(edge of lora_gemm's tiles, whether they are many,
+# whether there is a bias, device): "fused" | "epilogue"}.
 # "fused"    = the single wide-K MFMA kernel (wins when our GEMM rate is
 #              within the fusion savings of hipBLASLt — e.g. N-heavy shapes);
 # "epilogue" = hipBLASLt base GEMM + the custom rank-64 lora_add_ MFMA pass
@@ -47,9 +47,9 @@ def lora_gemm_ref(x, w, u=None, b=None, bias=None):
 # at 5.8 TB/s, the product at 1.3 PFLOP/s), the epilogue beyond, where they come close.
 # 46673 rows, fused / epilogue in us: 1536 x 1536 241 / 296, 2048 x 1536 250 / 330, 17920 x
 # 1536 2205 / 2610; 1536 x 8960 1020 / 1069, 1536 x 17920 1990 / 2015.
-# Measured once per key on first touch (events, ~1 ms): a few rows say nothing about
-# many, for which lora_gemm is another kernel, nor a square weight's dx, which has no
-# bias, about its y.
+# Measured once per key on first touch (events, ~1 ms): up to 128 rows, which run in
+# another kernel, say nothing about more, nor do a few tiles about many that fill the CUs, nor
+# a square weight's dx, which has no bias, about its y.
 _TUNE: dict[tuple, dict] = {}
 DEEP = 4096
 
@@ -71,8 +71,9 @@ def _capturing(x) -> bool:
 
 def _choose_strategy(x, w, u, b, bias) -> str:
     N, K = int(w.size(0)), int(w.size(1))
+    M = x.shape[0]
     known = _TUNE.setdefault((N, K), {})
-    key = (ext().lora_gemm_big(x.shape[0], N, K), bias is not None, x.device)
+    key = (ext().lora_gemm_tiles(M, K), ext().lora_gemm_big(M, N, K), bias is not None, x.device)
     st = known.get(key)
     if st is None and known and _capturing(x):
         return next(iter(known.values()))       # nothing can be timed now

@@ -45,6 +45,10 @@ def test_big_tiles_of_the_adapter_product_stop_where_offsets_end():
     big = ops.ext().lora_gemm_big
     assert big(4096, 1536, 1536) and not big(4096, 1280, 1536)
     assert big(24576, 256, (1 << 22) - 64) and not big(24576, 256, 1 << 22)
+    tiles = ops.ext().lora_gemm_tiles                   # of the kernel that runs
+    for rows in (129, 24576):
+        assert tiles(rows, 64) == tiles(rows, (1 << 22) - 64) == 256
+        assert tiles(rows, 1 << 22) == tiles(128, 64) == 128
 
 
 def test_adapter_strategies_are_kept_by_what_the_kernels_depend_on(monkeypatch):
@@ -52,8 +56,10 @@ def test_adapter_strategies_are_kept_by_what_the_kernels_depend_on(monkeypatch):
     from nanorlhf_amd.ops import lora
     monkeypatch.setattr(lora, "_TUNE", {})
     monkeypatch.setattr(lora, "ext", lambda: SimpleNamespace(
+        lora_gemm_tiles=lambda M, K: 256 if M > 128 else 128,
         lora_gemm_big=lambda M, N, K: M > 1000, lora_gemm=None, lora_add_=None))
-    times = iter([1.0, 3.0, 3.0, 1.0, 1.0, 3.0])            # fused, epilogue of each new key
+    # fused, epilogue of each new key
+    times = iter([1.0, 3.0, 3.0, 1.0, 1.0, 3.0, 3.0, 1.0, 3.0, 1.0])
     monkeypatch.setattr(lora, "_time_cuda", lambda fn: next(times))
     w, bias = torch.zeros(64, 64), torch.zeros(64)
 
@@ -61,8 +67,12 @@ def test_adapter_strategies_are_kept_by_what_the_kernels_depend_on(monkeypatch):
         return lora._choose_strategy(torch.zeros(rows, 64), w, None, None, b)
 
     assert [choose(240), choose(4000), choose(240, bias)] == ["fused", "epilogue", "fused"]
-    assert [choose(17), choose(9000), choose(60, bias)] == ["fused", "epilogue", "fused"]
-    assert next(times, None) is None and len(lora._TUNE[64, 64]) == 3
+    assert [choose(129), choose(9000), choose(500, bias)] == ["fused", "epilogue", "fused"]
+    assert len(lora._TUNE[64, 64]) == 3
+    # up to 128 rows are another kernel's, whose time is its own
+    assert [choose(60), choose(60, bias)] == ["epilogue", "epilogue"]
+    assert [choose(17), choose(128, bias), choose(240)] == ["epilogue", "epilogue", "fused"]
+    assert next(times, None) is None and len(lora._TUNE[64, 64]) == 5
 
 
 @pytest.mark.parametrize("K,rule", [(64, "fused"), (4096, "fused"), (4160, "epilogue"),
@@ -71,7 +81,8 @@ def test_near_ties_of_the_adapter_strategies_do_not_hang_on_the_timer(monkeypatc
     from types import SimpleNamespace
     from nanorlhf_amd.ops import lora
     monkeypatch.setattr(lora, "ext", lambda: SimpleNamespace(
-        lora_gemm_big=lambda M, N, K: True, lora_gemm=None, lora_add_=None))
+        lora_gemm_tiles=lambda M, K: 256, lora_gemm_big=lambda M, N, K: True, lora_gemm=None,
+        lora_add_=None))
     w, x = torch.zeros(64, K), torch.zeros(300, K)
     # fused against epilogue
     for ratio, want in [(0.95, rule), (1.0, rule), (1.05, rule), (0.5, "fused"), (2.0, "epilogue")]:
@@ -86,6 +97,7 @@ def test_a_capture_takes_the_strategy_that_is_known_of_its_weight(monkeypatch):
     from nanorlhf_amd.ops import lora
     monkeypatch.setattr(lora, "_TUNE", {})
     monkeypatch.setattr(lora, "ext", lambda: SimpleNamespace(
+        lora_gemm_tiles=lambda M, K: 256 if M > 128 else 128,
         lora_gemm_big=lambda M, N, K: M > 1000, lora_gemm=None, lora_add_=None))
     times = iter([3.0, 1.0])
     monkeypatch.setattr(lora, "_time_cuda", lambda fn: next(times))
