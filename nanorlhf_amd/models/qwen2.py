@@ -155,10 +155,15 @@ class RMSNorm(nn.Module):
         return ops.rms_norm(x, self.weight, self.eps)
 
 
+def _plain(m: nn.Module, cls: type) -> bool:
+    """Whether a call of this module is what this file says of `cls`, and nobody watches it."""
+    return (type(m) is cls and cls.forward is _FORWARDS[cls] and "forward" not in m.__dict__
+            and m._compiled_call_impl is None and unheard(m))
+
+
 def _parts(m: nn.Module, cls: type) -> dict:
     """What lets a module that nobody watches return parts."""
-    plain = not torch.is_grad_enabled() and type(m) is cls and "forward" not in m.__dict__
-    return dict(parts=True) if plain and unheard(m) else {}
+    return dict(parts=True) if not torch.is_grad_enabled() and _plain(m, cls) else {}
 
 
 class Block(nn.Module):
@@ -181,6 +186,9 @@ class Block(nn.Module):
         m_in, h2 = ops.add_parts_rms_norm(attn_delta, h,
                                           self.post_attention_layernorm.weight, eps)
         return self.mlp(m_in, **(_parts(self.mlp, MLP) if parts else {})), h2
+
+
+_FORWARDS = {cls: cls.forward for cls in (Attention, MLP, Block)}
 
 
 class Transformer(nn.Module):

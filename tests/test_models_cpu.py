@@ -131,3 +131,37 @@ def test_rope_table_follows_the_default_device():
     with torch.device("meta"):
         assert build_rope_cache(32, 64).device.type == "meta"
         assert torch.equal(build_rope_cache(32, 64, device="cpu"), want)
+
+
+@pytest.fixture
+def in_parts(monkeypatch):
+    """Projections of float32 rows return two parts of their depth where they may."""
+    from nanorlhf_amd import ops
+
+    def linear_parts(x, w, bias=None):
+        half = w.shape[1] // 2
+        return torch.stack([x[:, :half] @ w[:, :half].T, x[:, half:] @ w[:, half:].T])
+
+    monkeypatch.setattr(ops, "linear_parts", linear_parts)
+
+
+@pytest.mark.parametrize("name", ["Attention", "MLP", "Block"])
+def test_replaced_forwards_of_a_class_are_called_as_they_were(monkeypatch, in_parts, name):
+    """What a program puts in a class's place knows nothing of parts and gets none."""
+    from nanorlhf_amd.models import qwen2
+    m, s = CausalLM.from_preset("tiny").eval(), torch.arange(2, 9)
+    cls, shapes = getattr(qwen2, name), []
+    own = cls.forward
+
+    def forward(self, *args):
+        shapes.extend(tuple(a.shape) for a in args[:2 if name == "Block" else 1] if a is not None)
+        out = own(self, *args)
+        shapes.extend(tuple(t.shape) for t in (out if isinstance(out, tuple) else (out,)))
+        return out
+
+    with torch.no_grad():
+        want = _fwd(m, [s])
+        monkeypatch.setattr(cls, "forward", forward)
+        got = _fwd(m, [s])
+    assert set(shapes) == {(7, m.cfg.hidden_size)}
+    assert torch.allclose(got, want, atol=1e-5)
