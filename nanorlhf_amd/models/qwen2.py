@@ -210,12 +210,16 @@ class Transformer(nn.Module):
             self.rope_table = self.rope_table.float()
         delta = self.embed_tokens(input_ids)
         res = None
-        for layer in self.layers:
+        layers = list(self.layers)
+        for i, layer in enumerate(layers):
             if checkpoint and torch.is_grad_enabled():
                 delta, res = torch.utils.checkpoint.checkpoint(
                     layer, delta, res, self.rope_table, ctx, use_reentrant=False)
             else:
-                delta, res = layer(delta, res, self.rope_table, ctx, **_parts(layer, Block))
+                # parts only for a next layer that knows of them, or the norm below
+                knows = i + 1 == len(layers) or _plain(layers[i + 1], Block)
+                delta, res = layer(delta, res, self.rope_table, ctx,
+                                   **(_parts(layer, Block) if knows else {}))
         y, _ = ops.add_parts_rms_norm(delta, res, self.norm.weight, self.norm.eps)
         return y
 

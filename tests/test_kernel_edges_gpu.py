@@ -562,6 +562,19 @@ def test_listeners_get_sums_and_no_parts(rows):
     assert rel(alone, heard) < 0.01        # the same sums in another order, rounded to 2^-9
 
 
+@pytest.mark.parametrize("rows", [5, 40])
+def test_a_listening_layer_is_given_sums_and_no_parts(rows):
+    """Nor does the layer before one where somebody listens pass on parts."""
+    from nanorlhf_amd.models import CausalLM, get_config, pack_sequences
+    model = CausalLM(get_config("qwen2.5-1.5b", num_layers=2, vocab_size=512)).to(DEV).bfloat16()
+    ids, cu, mx, pos = pack_sequences([torch.arange(rows)], device=DEV)
+    seen = []
+    model.model.layers[1].register_forward_pre_hook(lambda mod, args: seen.extend(args[:2]))
+    with torch.no_grad():
+        model(ids, CausalLM.train_ctx(cu, mx, pos))
+    assert [(t.shape, t.dtype) for t in seen] == [((rows, 1536), torch.bfloat16)] * 2
+
+
 @pytest.mark.parametrize("temperature", [0.0, 0.7])
 def test_sampling_ahead_of_its_counter(temperature):
     x = rnd(8, 1000, seed=1, scale=3.0)

@@ -165,3 +165,43 @@ def test_replaced_forwards_of_a_class_are_called_as_they_were(monkeypatch, in_pa
         got = _fwd(m, [s])
     assert set(shapes) == {(7, m.cfg.hidden_size)}
     assert torch.allclose(got, want, atol=1e-5)
+
+
+@pytest.mark.parametrize("how", ["pre-hook", "hook", "subclass", "instance", "wrapped"])
+def test_a_layer_that_is_not_plain_is_given_sums_and_no_parts(monkeypatch, in_parts, how):
+    from nanorlhf_amd import ops
+    from nanorlhf_amd.models.qwen2 import Block
+    m, s = CausalLM.from_preset("tiny", num_layers=3).eval(), torch.arange(2, 9)
+    layers, normed, seen = m.model.layers, [], []
+    plain, norm = layers[1], ops.add_parts_rms_norm
+    monkeypatch.setattr(ops, "add_parts_rms_norm",
+                        lambda x, *args: (normed.append(x.dim()), norm(x, *args))[1])
+    with torch.no_grad():
+        want = _fwd(m, [s])
+    assert normed == [2] + [3] * 6          # but the embedding all of them are parts
+
+    class Sub(Block):
+        def forward(self, delta, res, *args):
+            seen.append(delta.shape)
+            return super().forward(delta, res, *args)
+
+    class Wrapped(torch.nn.Module):
+        def forward(self, delta, res, *args):
+            seen.append(delta.shape)
+            return plain(delta, res, *args)
+
+    if how == "pre-hook":
+        plain.register_forward_pre_hook(lambda mod, args: seen.append(args[0].shape))
+    elif how == "hook":
+        plain.register_forward_hook(lambda mod, args, out: seen.append(args[0].shape))
+    elif how == "subclass":
+        plain.__class__ = Sub
+    elif how == "wrapped":
+        layers[1] = Wrapped()
+    else:
+        own = plain.forward
+        plain.forward = lambda delta, *args: (seen.append(delta.shape), own(delta, *args))[1]
+    with torch.no_grad():
+        got = _fwd(m, [s])
+    assert seen == [(7, m.cfg.hidden_size)]
+    assert torch.allclose(got, want, atol=1e-5)
