@@ -526,19 +526,28 @@ __global__ __launch_bounds__(1024) void expert_lists_kernel(
 }
 
 // ======================================================== host wrappers ==
-// Whether gemm_big.h's kernel takes these, with `tm` tiles of rows at most: that is what its
-// 32-bit offsets, whole steps and stores of four columns can do, and where its tiles of 256
+// Whether gemm_big.h's kernel pays with `tm` tiles of rows at most: where its tiles of 256
 // fill the CUs and their columns.  us, tiles of 128 / it: 16 experts of 1536 x 2240, gate and
 // up, 250 rows each (576 tiles) 102 / 82, 1000 rows 299 / 211, down 180 rows (162) 41 / 44, 256
 // (192) 68 / 46; 4 experts, 300 rows (144) 33 / 36, 400 (180) 50 / 34; 12 heads of 512 x 128,
 // 4000 rows 16.4 / 18.3.  Up to 128 rows half of a tile is empty and it takes a long product:
 // 110 rows of 1536 x 2240 65 / 66, 100 of 2048 x 2752 139 / 108, 56 of 3584 x 4096 143 / 95.
+static bool fills_big(long each, long tm, long N, long K, int width) {
+  const long tn = (N + width - 1) / width;
+  return tm * tn < 1L << 31 && N * 4 >= tn * width * 3 &&
+         (each > 128 ? tm * tn >= 176 : tm * tn * K >= 800000);
+}
+
+// ... and takes them: what its 32-bit offsets, whole steps and stores of four columns can do
 static bool takes_big(const Grouped& a, long each, long tm, int width) {
-  const long tn = (a.N + width - 1) / width;
   return a.G <= 64 && a.K > 0 && a.K % 64 == 0 && a.N % 4 == 0 && (a.ldo | a.go) % 4 == 0 &&
          (uintptr_t)a.out % 8 == 0 && a.K < 1L << 22 && a.ldw < 1L << 22 &&
-         (a.rows / a.div + 1) * a.lda < 1L << 31 && tm * tn < 1L << 31 &&
-         a.N * 4L >= tn * width * 3 && (each > 128 ? tm * tn >= 176 : tm * tn * a.K >= 800000);
+         (a.rows / a.div + 1) * a.lda < 1L << 31 && fills_big(each, tm, a.N, a.K, width);
+}
+
+// Whether T rows of each of G products fill gemm_big.h's tiles
+bool group_linear_fills(long T, long G, long N, long K) {
+  return fills_big(T, G * ((T + BIG - 1) / BIG), N, K, BIG);
 }
 
 template <bool GLU>

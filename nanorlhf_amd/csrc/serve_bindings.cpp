@@ -87,6 +87,7 @@ void expanded_attn_varlen(torch::Tensor q, torch::Tensor k, torch::Tensor vt, to
                           long heads, long max_q, double scale);
 // moe.hip
 void group_linear(torch::Tensor x, torch::Tensor w, torch::Tensor out);
+bool group_linear_fills(long T, long G, long N, long K);
 std::vector<torch::Tensor> moe_route(torch::Tensor h, torch::Tensor router, torch::Tensor bias,
                                      long top);
 torch::Tensor moe_gate_up(torch::Tensor h, torch::Tensor gate_up, torch::Tensor lists,
@@ -124,6 +125,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("latent_attn_plain", &latent_attn_plain);
   m.def("expanded_attn_varlen", &expanded_attn_varlen);
   m.def("group_linear", &group_linear);
+  m.def("group_linear_fills", &group_linear_fills);
   m.def("moe_route", &moe_route);
   m.def("moe_gate_up", &moe_gate_up);
   m.def("moe_down", &moe_down);

@@ -16,10 +16,19 @@ from . import serve_ext
 from .linear import here, plain_call
 
 # Rows up to which separate GEMMs cost more than one launch, whatever the sizes.  With more
-# one launch of whole steps of the depth: 4 products of 1536 x 1536, 1000 rows 30 us, four
-# library calls 74 (and 20 us each on the host), 4000 rows 71 / 87, 12000 186 / 229; of 4096 x
-# 4096, 4000 rows 366 / 365.
+# one launch of whole steps of the depth, if there are a few products of them, and either not
+# too deep, for without enough tiles for the CUs the library divides the depth, or filling
+# csrc/gemm_big.h's tiles.  us, one launch / library calls (and 20 us each on the host):
+#   4 of 1536 x 1536   300 rows 23 / 33   700 28 / 48   1200 30 / 54   4000 67 / 83   12000 182 / 221
+#   4 of 512 x 512     300 rows 6 / 20    4 of 320 x 2048   700 rows 27 / 34, 12000 88 / 92
+#   4 of 4096 x 4096   300 rows 60 / 84 (not filled)   700 78 / 112   4000 373 / 350   12000 1158 / 1772
+#   4 of 256 x 4096    700 rows 48 / 41   8 of 320 x 4096   300 rows 48 / 72, 12000 375 / 421
+#   4 of 1536 x 6144   260 rows 73 / 72   2 of 512 x 2048   700 rows 27 / 19
+#   2 of 1536 x 1536   260 rows 21 / 15   2 of 256 x 4096   700 rows 48 / 21
+#   1 of 4096 x 4096   260 rows 48 / 21, 4000 94 / 89
 STACKED_ROWS = 256
+STACKED_PRODUCTS = 4
+STACKED_DEPTH = 512         # for each product
 
 
 def group_linear(x: torch.Tensor, w: torch.Tensor,
@@ -36,11 +45,13 @@ def group_linear(x: torch.Tensor, w: torch.Tensor,
 
 def _stacks(x: torch.Tensor, w: torch.Tensor) -> bool:
     return (here(x) and plain_call(x, w) and x.dim() == w.dim() == 3 and x.dtype == w.dtype
-            and w.device == x.device and x.shape[0] == w.shape[0] <= 64
+            and w.device == x.device and STACKED_PRODUCTS <= x.shape[0] == w.shape[0] <= 64
             and x.shape[2] == w.shape[2] and x.shape[2] % 64 == 0 and w.shape[1] % 4 == 0
             and w.shape[1] >= 256 and x.is_contiguous() and w.is_contiguous()
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and x.shape[1] * x.shape[2] < 1 << 30)
+            and x.shape[1] * x.shape[2] < 1 << 30
+            and (x.shape[2] <= STACKED_DEPTH * x.shape[0] or serve_ext().group_linear_fills(
+                x.shape[1], x.shape[0], w.shape[1], x.shape[2])))
 
 
 def stacked_linear(x: torch.Tensor, w: torch.Tensor):

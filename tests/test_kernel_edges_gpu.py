@@ -804,12 +804,20 @@ def test_grouped_product_of_many_rows(T, G, N, K):
     assert rel(ops.group_linear(x, w), want) < 0.002       # one rounding, 2^-9 at most
 
 
-@pytest.mark.parametrize("T", [300, 512])
-def test_stacked_products_of_many_rows(T):
-    x, w = rnd(4, T, 192, seed=1), rnd(4, 516, 192, seed=2, scale=192 ** -0.5)
+# rows at a time, tiles of 128, and of 256 (12 * 2 * 9 of them, 4 * 3 * 16, 5 * 6 * 6)
+@pytest.mark.parametrize("G,T,N,K,own", [
+    (4, 300, 516, 192, True), (4, 512, 516, 192, True), (12, 300, 2060, 192, True),
+    (4, 700, 4096, 2112, True), (5, 1500, 1288, 2624, True),
+    (4, 300, 516, 2112, False), (2, 512, 256, 192, False), (3, 4096, 4096, 64, False)])
+def test_stacked_products_of_many_rows(G, T, N, K, own, monkeypatch):
+    """In one launch where that is faster than the library."""
+    x, w = rnd(G, T, K, seed=1), rnd(G, N, K, seed=2, scale=K ** -0.5)
+    seen, launch = [], ops.moe.group_linear
+    monkeypatch.setattr(ops.moe, "group_linear", lambda *a: (seen.append(1), launch(*a))[1])
     with torch.no_grad():
         for got, a, b in zip(ops.stacked_linear(x, w), x, w):
             assert rel(got, a.double() @ b.double().t()) < 0.002       # one rounding, 2^-9
+    assert bool(seen) == own
 
 
 @pytest.mark.parametrize("n", [1, 4095, 4096, 4099, 9000])
