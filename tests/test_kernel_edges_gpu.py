@@ -820,6 +820,21 @@ def test_stacked_products_of_many_rows(G, T, N, K, own, monkeypatch):
     assert bool(seen) == own
 
 
+@pytest.mark.parametrize("E", [5, 16, 17])
+@pytest.mark.parametrize("W", [8, 72, 1528, 1536, 1544, 4096])
+def test_a_token_is_routed_alike_in_any_company(W, E):
+    """The same bits, whatever the number of tokens beside it: near ties hang on them."""
+    h, router, bias = rnd(4000, W, seed=1), rnd(E, W, seed=2, scale=W ** -0.5), rnd(E, seed=3)
+    chosen, weights, _, _ = ops.moe_route(h, router, bias, 4)
+    for n in (1, 32, 511, 512, 513):
+        few = ops.moe_route(h[:n], router, bias, 4)
+        assert torch.equal(few[0], chosen[:n]) and torch.equal(few[1], weights[:n])
+    z = h.double() @ router.double().t() + bias.double()
+    v = z.gather(1, chosen.long())
+    assert (v - z.topk(4).values).abs().max() < 1e-5      # 32-bit sums of about 1
+    assert rel(weights, torch.softmax(v, 1)) < 1e-5
+
+
 @pytest.mark.parametrize("n", [1, 4095, 4096, 4099, 9000])
 def test_lists_of_a_route_are_in_order(n):
     h, router = rnd(n, 64, seed=1), rnd(5, 64, seed=2)
