@@ -40,6 +40,8 @@
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
+#include <algorithm>
+
 #include "common.h"
 #include "lds_tiles.h"
 
@@ -525,6 +527,32 @@ std::vector<torch::Tensor> fa_fwd_varlen(torch::Tensor q, torch::Tensor k,
   return {o, lse};
 }
 
+// A workgroup of dk and dv walks the group's q heads one after the other.  Where that leaves
+// too few to fill 256 CUs twice, with spare to even out causal tiles, they are divided among
+// `parts`.  Long sequences want more of them the shorter the others are, for a walk of the
+// longest then is more of the whole, and with heads of 64, of which a CU runs more
+// at a time.  From 1100 undivided ones on there is one part, which bounds the parts'
+// memory.  Whole backward, us by parts, undivided workgroups in brackets:
+//   12 heads over 2   56 x 870 (872) 1: 720, 2: 770, 6: 890   8 x 3000 (390) 2: 1130, 3: 1160
+//     equal lengths   2 x 6000 (190) 3: 854, 6: 762   3 x 6000 (286) 2: 1260, 3: 1114, 6: 1131
+//                     4 x 6000 (382) 2: 1485, 3: 1450   5 x 6000 (478) 2: 1845, 3: 1848
+//     mixed           8000 2 x, 3000 6 x (546) 2: 3021, 3: 2071   7900, 600 30 x (466) 2: 1441, 3: 1238
+//     up to 10000     5 of 6900 (546) 1: 3971, 2: 2888, 3: 2887
+//   28 heads over 4   5 x 6000 (956) 1: 4319, 7: 4555   4 x 8000 (1016) 1: 6019, 7: 6146
+//     mixed           4 of 6200 (796) 1: 5743, 7: 4601   7900, 600 30 x (932) 1: 3179, 7: 2239
+//     up to 10000     5 of 6900 (1092) 1: 6782, 7: 7134
+//   14 over 2 of 64   9 x 6000 (860) 1: 2265, 7: 2092   8 x 8000 (1016) 1: 3241, 7: 3153
+//                     12 x 6000 (1148) 1: 2652, 7: 2758
+long fa_bwd_parts(long T, long B, long Hq, long Hkv, long D, long max_seqlen) {
+  const long G = Hq / Hkv, tiles = (T / ROWS + B) * Hkv;
+  const long wanted = max_seqlen < 6000 ? 768
+                      : D <= 64         ? 1100
+                                        : std::clamp(720 * max_seqlen * B / T, 768L, 1100L);
+  long parts = 1;
+  while (parts < G && (G % parts || tiles * parts < wanted)) parts++;
+  return parts;
+}
+
 std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
                                          torch::Tensor k, torch::Tensor v,
                                          torch::Tensor o, torch::Tensor lse,
@@ -540,17 +568,7 @@ std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
   auto rows = torch::empty({2, (long)Hq, T}, f32);    // -sum(dO * O), lse in log2 units
   float* drow = rows.data_ptr<float>();
   float* lse2 = drow + (long)Hq * T;
-  // A workgroup of dk and dv walks the group's q heads one after the other.
-  // Where that leaves too few to fill 256 CUs twice, with spare to even out
-  // causal tiles, they are divided among `parts`, the finer the longer the longest of
-  // those walks is.  Whole backward, 12 heads over
-  // 2: 5 x 6500 tokens (518 workgroups undivided) 3.95 ms with 1 part, 2.87 with
-  // 2, 2.83 with 3; 6 x 4000 (400) 1.51 with 2, 1.36 with 3, 3 x 6000 (290) 1.22 with 3, 1.13
-  // with 6; 8 x 3000 (390) 1.13 with 2, 1.16 with 3; 56 x 870 (872) 0.72 with 1, 0.77 with
-  // 2, 0.89 with 6.
-  int parts = 1;
-  const long tiles = (T / ROWS + B) * Hkv, wanted = max_seqlen >= 6000 ? 1100 : 768;
-  while (parts < G && (G % parts || tiles * parts < wanted)) parts++;
+  const int parts = fa_bwd_parts(T, B, Hq, Hkv, D, max_seqlen);
   const long n = T * Hkv * D;
   torch::Tensor sums;
   if (parts > 1) sums = torch::empty({2, (long)parts, n}, f32);

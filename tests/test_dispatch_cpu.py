@@ -133,3 +133,27 @@ def test_adapter_gradients_take_the_kernel_by_columns_and_rows():
         assert not _fast_grad(z.expand(4096, 37888)) and not _fast_grad(z.expand(64, 36))
         assert not _fast_grad(z.float().expand(64, 64))
     assert not _fast_grad(z.expand(64, 64))            # a recorded backward
+
+
+def test_gradients_of_keys_and_values_are_divided_where_that_pays():
+    if not ops.ext_available():
+        pytest.skip("extensions are not built")
+
+    def parts(heads, lens, D=128):
+        return ops.ext().fa_bwd_parts(sum(lens), len(lens), *heads, D, max(lens))
+
+    small, large = (12, 2), (28, 4)
+    assert parts(small, [870] * 56) == 1 and parts(small, [3000] * 8) == 2
+    assert [parts(small, [6000] * n) for n in (2, 3, 4, 5)] == [6, 3, 3, 2]
+    assert parts(small, [8000] * 2 + [3000] * 6) == parts(small, [7900] + [600] * 30) == 3
+    assert parts(large, [6000] * 5) == parts(large, [8000] * 4) == 1
+    assert parts(large, [10000, 4000, 5000, 7000, 8300]) == 1        # 1088 workgroups undivided
+    assert parts(large, [8500, 4500, 5000, 6900]) == parts(large, [7900] + [600] * 30) == 7
+    assert [parts((14, 2), [6000] * n, 64) for n in (9, 12)] == [7, 1]
+    assert parts((16, 16), [6000]) == 1 and parts(large, [6000] + [1] * 300000) == 1
+    # what the parts take: float32 sums of both for every token and part
+    for n in range(1, 200):
+        for heads in (small, large, (32, 8), (40, 8)):
+            lens = [8000] + [100 * n] * n
+            p = parts(heads, lens)
+            assert p == 1 or 2 * p * sum(lens) * heads[1] * 128 * 4 <= 7 * 1100 * 128 * 128 * 8

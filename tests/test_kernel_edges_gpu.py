@@ -66,6 +66,21 @@ def test_flash_attention_windows_of_heads(hq, hkv, d, causal):
         assert rel(got.grad, ref.grad) < FA_REL
 
 
+@pytest.mark.parametrize("lens", [[5999, 257], [6000, 257], [6000, 1, 6001, 130]])
+@pytest.mark.parametrize("hq,hkv,d", [(7, 1, 128), (6, 2, 128), (7, 1, 64)])
+def test_flash_attention_of_long_sequences(lens, hq, hkv, d):
+    """dk and dv in one part to seven; lengths at which their number changes."""
+    from nanorlhf_amd.ops.attention import _sdpa_ref_autograd
+    cu = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
+    leaves = [rnd(sum(lens), h, d, seed=h).requires_grad_(True) for h in (hq, hkv, hkv)]
+    do = rnd(sum(lens), hq, d, seed=4)
+    ops.flash_attn_varlen(*leaves, cu, max(lens), causal=True).backward(do)
+    exact = [t.detach().float().requires_grad_(True) for t in leaves]
+    _sdpa_ref_autograd(*exact, cu.cpu(), d ** -0.5, causal=True).backward(do.float())
+    for got, ref in zip(leaves, exact):
+        assert rel(got.grad, ref.grad) < FA_REL
+
+
 @pytest.mark.parametrize("rows", [90, 38700])         # dk and dv in several parts, in one
 @pytest.mark.parametrize("d", [32, 64, 128])
 def test_flash_attention_gives_padding_no_gradient(rows, d):
