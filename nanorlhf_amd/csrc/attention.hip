@@ -487,10 +487,11 @@ __global__ void fa_bwd_sum_kernel(const float* __restrict__ part, short* __restr
 // 2050; 3.5 rounds, 28 heads over 4, 4 x 2000 139 / 146; 2.8 rounds, 14 heads of 64, 20 x
 // 1200 102 / 121; 7.5 windows, 5 x 6500 896 / 880 with the longest sequence ahead, but forward
 // and backward 3811 / 3997 with it behind.  Backward of the first 1354 / 1118.  The walks of
-// dk and dv are few and long: causal, 40 x 1200 1041 / 1291.
-static unsigned head_window(long heads, long tiles, long rounds, bool causal) {
+// dk and dv are few and long: causal, 40 x 1200 1041 / 1291.  A window's place is found from
+// the workgroup's number, which has to fit 32 bits.
+long fa_head_window(long heads, long tiles, long rounds, bool causal) {
   const long window = 8 * std::max(64 / std::max(tiles, 1L), 1L);
-  return causal && (rounds < 4 || heads < 8 * window) ? heads : window;
+  return causal && (rounds < 4 || heads < 8 * window) || heads * tiles >= 1L << 32 ? heads : window;
 }
 
 #define FA_BY_WIDTH(CALL)                                                  \
@@ -520,7 +521,7 @@ std::vector<torch::Tensor> fa_fwd_varlen(torch::Tensor q, torch::Tensor k,
                      (const short*)q.data_ptr(), (const short*)k.data_ptr(),   \
                      (const short*)v.data_ptr(), cu_seqlens.data_ptr<int>(),   \
                      (short*)o.data_ptr(), lse.data_ptr<float>(), Hq, Hkv, (float)scale,     \
-                     head_window(grid.x, grid.y, rounds, causal))
+                     fa_head_window(grid.x, grid.y, rounds, causal))
   FA_BY_WIDTH(CALL);
 #undef CALL
   HIP_CHECK_LAST();
@@ -589,13 +590,13 @@ std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
                        (const short*)k.data_ptr(), (const short*)v.data_ptr(), \
                        lse2, drow, cu_seqlens.data_ptr<int>(), (short*)dq.data_ptr(), \
                        T, Hq, Hkv, (float)scale,                               \
-                       head_window(B * Hq, row_tiles, rounds, causal));        \
+                       fa_head_window(B * Hq, row_tiles, rounds, causal));     \
     hipLaunchKernelGGL((fa_bwd_dkv_kernel<DD, CC>), dim3(B * Hkv * parts, row_tiles), dim3(256), \
                        0, stream, (const short*)dout.data_ptr(),               \
                        (const short*)q.data_ptr(), (const short*)k.data_ptr(), \
                        (const short*)v.data_ptr(), lse2, drow,                 \
                        cu_seqlens.data_ptr<int>(), dkp, dvp, T, Hq, Hkv, parts, (float)scale, \
-                       head_window(B * Hkv * parts, row_tiles, 0, causal));    \
+                       fa_head_window(B * Hkv * parts, row_tiles, 0, causal)); \
   } while (0)
   FA_BY_WIDTH(CALL);
 #undef CALL

@@ -55,6 +55,7 @@ void lora_add_(torch::Tensor y, torch::Tensor u, torch::Tensor b);
 std::vector<torch::Tensor> fa_fwd_varlen(torch::Tensor q, torch::Tensor k,
                                          torch::Tensor v, torch::Tensor cu_seqlens,
                                          long max_seqlen, double scale, bool causal);
+long fa_head_window(long heads, long tiles, long rounds, bool causal);
 long fa_bwd_parts(long T, long B, long Hq, long Hkv, long D, long max_seqlen);
 std::vector<torch::Tensor> fa_bwd_varlen(torch::Tensor dout, torch::Tensor q,
                                          torch::Tensor k, torch::Tensor v,
@@ -117,4 +118,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fa_fwd_varlen", &fa_fwd_varlen);
   m.def("fa_bwd_varlen", &fa_bwd_varlen);
   m.def("fa_bwd_parts", &fa_bwd_parts);
+  m.def("fa_head_window", &fa_head_window);
 }

@@ -157,3 +157,17 @@ def test_gradients_of_keys_and_values_are_divided_where_that_pays():
             lens = [8000] + [100 * n] * n
             p = parts(heads, lens)
             assert p == 1 or 2 * p * sum(lens) * heads[1] * 128 * 4 <= 7 * 1100 * 128 * 128 * 8
+
+
+def test_windows_of_heads_have_places_that_fit_32_bits():
+    """The kernels number heads * tiles workgroups in unsigned."""
+    if not ops.ext_available():
+        pytest.skip("extensions are not built")
+    window = ops.ext().fa_head_window
+    assert window(1280, 7, 30, False) == 72 and window(672, 12, 10, True) == 40
+    assert window(60, 51, 6, True) == 60 and window(80, 16, 3, True) == 80
+    for heads in (1 << 20, 16_000_000):
+        most = ((1 << 32) - 1) // heads
+        for causal in (False, True):
+            assert window(heads, most, 100, causal) < heads
+            assert window(heads, most + 1, 100, causal) == heads
