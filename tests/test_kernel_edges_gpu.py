@@ -784,31 +784,34 @@ def test_grouped_product_of_few_rows(T, G, N, K):
 
 @pytest.mark.parametrize("W,ff", [(2880, 1344), (64, 1356)])      # both products, gated alone
 @pytest.mark.parametrize("skew", [True, False])
-def test_experts_of_many_rows(W, ff, skew):
-    """Tiles of 256 rows: groups that fill one, miss it by one or are empty."""
-    counts = [0, 1, 255, 256, 257, 0, 512, 600, 3, 0] if skew else [190] * 10
-    T, E = sum(counts), len(counts)
-    order = torch.randperm(T, generator=torch.Generator().manual_seed(W)).to(DEV)
-    chosen = torch.empty(T, 1, dtype=torch.int32, device=DEV)
+@pytest.mark.parametrize("top", [1, 3])
+def test_experts_of_many_rows(W, ff, skew, top):
+    """Tiles of 256 rows: groups that fill one, miss it by one or are empty; a token's choices
+    are rows of their own, which share its row of h."""
+    counts = [0, 1, 255, 256, 257, 0, 512, 600, 3, 0] if skew else [192] * 10
+    R, E = sum(counts), len(counts)
+    T = R // top
+    order = torch.randperm(R, generator=torch.Generator().manual_seed(W)).to(DEV)
+    chosen = torch.empty(T, top, dtype=torch.int32, device=DEV)
     lists = torch.full((E, T), -1, dtype=torch.int32, device=DEV)      # only counted ones count
     rows, first = [], 0
     for e, n in enumerate(counts):
         r = order[first:first + n].sort().values
-        chosen[r, 0], lists[e, :n] = e, r.int()
+        chosen.view(-1)[r], lists[e, :n] = e, r.int()
         rows.append(r)
         first += n
-    weights = torch.rand(T, 1, generator=torch.Generator(device=DEV).manual_seed(5), device=DEV)
+    weights = torch.rand(T, top, generator=torch.Generator(device=DEV).manual_seed(5), device=DEV)
     h, gate_up, down = rnd(T, W, seed=1), rnd(E, 2, ff, W, seed=2, scale=W ** -0.5), \
         rnd(E, W, ff, seed=3, scale=ff ** -0.5)
     got = ops.moe_experts(h, gate_up, down, (chosen, weights, lists,
                                              torch.tensor(counts, dtype=torch.int32, device=DEV)))
-    want = torch.empty(T, 1, W, dtype=torch.float64, device=DEV)
+    want = torch.empty(R, W, dtype=torch.float64, device=DEV)
     for e, r in enumerate(rows):
-        x = h[r].double()
+        x = h[r // top].double()
         act = torch.nn.functional.silu(x @ gate_up[e, 0].double().t()) \
             * (x @ gate_up[e, 1].double().t())
-        want[r, 0] = weights[r].double() * (act @ down[e].double().t())
-    assert rel(got, want) < 0.004                  # two roundings, 2^-9 at most each
+        want[r] = weights.view(-1, 1)[r].double() * (act @ down[e].double().t())
+    assert rel(got, want.view(T, top, W)) < 0.004          # two roundings, 2^-9 at most each
 
 
 @pytest.mark.parametrize("T", [257, 512])
