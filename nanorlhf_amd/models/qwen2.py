@@ -23,6 +23,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
+from ..ops.linear import FEW_ROWS
 from .config import ModelConfig, get_config
 from .lora import plain_weight, project, unheard
 
@@ -161,9 +162,14 @@ def _plain(m: nn.Module, cls: type) -> bool:
             and m._compiled_call_impl is None and unheard(m))
 
 
+def _few(rows: int) -> bool:
+    """Whether a projection of so many rows may come in parts at all."""
+    return rows <= FEW_ROWS and not torch.is_grad_enabled()
+
+
 def _parts(m: nn.Module, cls: type) -> dict:
     """What lets a module that nobody watches return parts."""
-    return dict(parts=True) if not torch.is_grad_enabled() and _plain(m, cls) else {}
+    return dict(parts=True) if _plain(m, cls) else {}
 
 
 class Block(nn.Module):
@@ -180,12 +186,13 @@ class Block(nn.Module):
         (ops.add_rms_norm), so no standalone residual-add kernels run.  So does the sum
         of a decoding projection's parts (ops.linear_parts), of this layer's last one
         only if the caller asks for `parts`."""
-        eps = self.input_layernorm.eps
+        eps, few = self.input_layernorm.eps, _few(delta.shape[-2])
         a_in, h = ops.add_parts_rms_norm(delta, res, self.input_layernorm.weight, eps)
-        attn_delta = self.self_attn(a_in, rope_table, ctx, **_parts(self.self_attn, Attention))
+        attn_delta = self.self_attn(a_in, rope_table, ctx,
+                                    **(_parts(self.self_attn, Attention) if few else {}))
         m_in, h2 = ops.add_parts_rms_norm(attn_delta, h,
                                           self.post_attention_layernorm.weight, eps)
-        return self.mlp(m_in, **(_parts(self.mlp, MLP) if parts else {})), h2
+        return self.mlp(m_in, **(_parts(self.mlp, MLP) if parts and few else {})), h2
 
 
 _FORWARDS = {cls: cls.forward for cls in (Attention, MLP, Block)}
@@ -210,16 +217,18 @@ class Transformer(nn.Module):
             self.rope_table = self.rope_table.float()
         delta = self.embed_tokens(input_ids)
         res = None
-        layers = list(self.layers)
+        layers, few = list(self.layers), _few(delta.shape[0])
+        plain = few and layers and _plain(layers[0], Block)
         for i, layer in enumerate(layers):
             if checkpoint and torch.is_grad_enabled():
                 delta, res = torch.utils.checkpoint.checkpoint(
                     layer, delta, res, self.rope_table, ctx, use_reentrant=False)
             else:
                 # parts only for a next layer that knows of them, or the norm below
-                knows = i + 1 == len(layers) or _plain(layers[i + 1], Block)
+                then = few and (i + 1 == len(layers) or _plain(layers[i + 1], Block))
                 delta, res = layer(delta, res, self.rope_table, ctx,
-                                   **(_parts(layer, Block) if knows else {}))
+                                   **(dict(parts=True) if plain and then else {}))
+                plain = then
         y, _ = ops.add_parts_rms_norm(delta, res, self.norm.weight, self.norm.eps)
         return y
 
