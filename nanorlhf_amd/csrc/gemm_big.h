@@ -57,11 +57,13 @@ DEVINL void load_big(const void* base, unsigned offset, unsigned at) {
 // two phases away, so that a load has a whole step's time.
 //
 // Products are 16x16x32: by themselves they reach 1.88 PFLOP/s on normally distributed
-// data, 32x32x16 1.64 (the part runs into its power, and those move twice as much of the
-// sums).  x is the first operand and w's rows are dealt to LDS so that a lane
+// data, 32x32x16 1.64 (the part lowers its clock, to 1.9 GHz where zeros keep 2.4, and those
+// move twice as much of the sums).  x is the first operand and w's rows are dealt to LDS so that a lane
 // ends up with 4 neighbouring columns of y and 16 lanes with 128 bytes: stores of 16 bytes
-// to 64 rows' quarter lines cost up to 10%.  They leave past the caches' keeping,
-// for y is larger than those.  The next tile's first two steps are asked
+// to 64 rows' quarter lines cost up to 10%.  They are marked as not to be kept, which makes
+// no difference, neither to a large y nor to a small one that the next kernel reads at once:
+// with SwiGLU behind it 212 x 1152 x 896 19.8 us and 19.7 without the mark, 500 x 17920 x 1536
+// 41.8 and 41.9, 46673 x 17920 x 1536 2529 and 2521.  The next tile's first two steps are asked
 // for before the stores.
 //
 // 8192 x 8192 x 8192: 0.71 ms (1530 TFLOP/s), 48720 x 17920 x 1536 + 64: 2.13 (1310),
