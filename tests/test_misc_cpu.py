@@ -165,3 +165,26 @@ def test_mathcheck_pathological_timeout_fast():
     out = answers_equal("x**x**x**x**99999 + y", "z", 0.3)
     assert out is False
     assert time.time() - t0 < 5.0
+
+
+def test_a_changed_header_compiles_every_source_again(tmp_path, monkeypatch):
+    """Sources are compiled again when their command changes; headers are not tracked."""
+    import runpy
+    import shutil
+    from types import SimpleNamespace
+    import setuptools
+    import torch.utils.cpp_extension as cpp
+    seen = []
+    monkeypatch.setattr(cpp, "CUDAExtension", lambda **k: SimpleNamespace(**k))
+    monkeypatch.setattr(setuptools, "setup", lambda **k: seen.append(
+        [e.extra_compile_args for e in k["ext_modules"]]))
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    shutil.copy(os.path.join(root, "setup.py"), tmp_path)
+    csrc = tmp_path / "nanorlhf_amd" / "csrc"
+    csrc.mkdir(parents=True)
+    for text in ("one", "one", "two"):
+        (csrc / "common.h").write_text(text)
+        runpy.run_path(str(tmp_path / "setup.py"))
+    assert seen[0] == seen[1]
+    for before, after in zip(seen[1], seen[2]):
+        assert all(before[kind] != after[kind] for kind in ("cxx", "nvcc"))
