@@ -625,8 +625,10 @@ static void launch_grouped(const Grouped& a, bool bf16) {
                      : each > 12 ? 2 : 1;
       // Four waves with a chunk of their own each.  Where 64 weight rows to a workgroup
       // leave CUs idle, 32 and two chunks: one token's 4 experts of 1536 x 2240 7.7 us
-      // against 10; and for a few rows' gate and up: 16 experts of 1536 x 2240 42.4 us, 43.9
-      // with 64 rows, of 4096 x 3584 138 and 143, down 24.5 and 22.9.
+      // against 10; and for a few rows' gate and up of some depth: 16 experts of 1536 x 2240
+      // 42.4 us, 43.9 with 64 rows, of 4096 x 3584 138 and 143, down 24.5 and 22.9.  Both products,
+      // 12 rows each: 64 experts of 512 x 1408 72 and 62, 32 of 1024 x 1024 44.0 and 43.8, 64 of
+      // 1536 x 512 58.1 and 59.5, 16 of 4096 x 3584 279 and 291.
       const long busy = std::min<long>(tiles_of(16 * mf), a.rows);
 #define STREAM(MF, NF, R)                                                                      \
   hipLaunchKernelGGL((grouped_stream_kernel<MF, NF, 4, R, GLU>),                               \
@@ -641,7 +643,7 @@ static void launch_grouped(const Grouped& a, bool bf16) {
         STREAM(4, 4, 1);
       } else if (mf == 2) {
         STREAM(2, 4, 1);
-      } else if (GLU) {
+      } else if (GLU && a.K >= 1536) {
         STREAM(1, 2, 2);
       } else {
         STREAM(1, 4, 1);

@@ -814,6 +814,18 @@ def test_experts_of_many_rows(W, ff, skew, top):
     assert rel(got, want.view(T, top, W)) < 0.004          # two roundings, 2^-9 at most each
 
 
+@pytest.mark.parametrize("T", [20, 40])
+@pytest.mark.parametrize("W", [72, 1472, 1536])        # 64 weight rows to a workgroup, then 32
+def test_experts_of_few_rows(T, W):
+    h, router, bias = rnd(T, W, seed=1), rnd(16, W, seed=2, scale=W ** -0.5), rnd(16, seed=3)
+    gate_up, down = rnd(16, 2, 530, W, seed=4, scale=W ** -0.5), rnd(16, W, 530, seed=5, scale=0.04)
+    routing = ops.moe_route(h, router, bias, 4)
+    got, chosen = ops.moe_experts(h, gate_up, down, routing), routing[0].long()
+    g, u = (torch.einsum("tw,tefw->tef", h.float(), gate_up[chosen, i].float()) for i in (0, 1))
+    want = torch.einsum("tef,tewf->tew", torch.nn.functional.silu(g) * u, down[chosen].float())
+    assert rel(got, want * routing[1][..., None]) < 0.004          # two roundings, 2^-9 each
+
+
 @pytest.mark.parametrize("T", [257, 512])
 @pytest.mark.parametrize("G,N,K", [(12, 2060, 192), (64, 772, 64)])
 def test_grouped_product_of_many_rows(T, G, N, K):
