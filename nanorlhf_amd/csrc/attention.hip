@@ -487,7 +487,9 @@ __global__ void fa_bwd_sum_kernel(const float* __restrict__ part, short* __restr
 // 2050; 3.5 rounds, 28 heads over 4, 4 x 2000 139 / 146; 2.8 rounds, 14 heads of 64, 20 x
 // 1200 102 / 121; 7.5 windows, 5 x 6500 896 / 880 with the longest sequence ahead, but forward
 // and backward 3811 / 3997 with it behind.  Backward of the first 1354 / 1118.  The walks of
-// dk and dv are few and long: causal, 40 x 1200 1041 / 1291.  A window's place is found from
+// dk and dv are few and long: causal, 40 x 1200 1041 / 1291.  The forward of up to two tiles
+// has little to share before it ends: not causal, 16 heads of 64, 64 x 100 18.7 / 20.5, 12 of
+// 128 27.8 / 28.8; with 3.9 rounds, 128 x 120, 40.0 / 37.5.  A window's place is found from
 // the workgroup's number, which has to fit 32 bits.
 long fa_head_window(long heads, long tiles, long rounds, bool causal) {
   const long window = 8 * std::max(64 / std::max(tiles, 1L), 1L);
@@ -516,12 +518,13 @@ std::vector<torch::Tensor> fa_fwd_varlen(torch::Tensor q, torch::Tensor k,
   auto stream = at::hip::getCurrentHIPStream();
   const dim3 grid(B * Hq, (max_seqlen + ROWS - 1) / ROWS);
   const long rounds = (T / ROWS + B) * Hq / (D > 64 ? 512 : 1024);
+  const bool short_walks = grid.y <= 2 && rounds < 3;
 #define CALL(DD, CC)                                                           \
   hipLaunchKernelGGL((fa_fwd_kernel<DD, CC>), grid, dim3(256), 0, stream,      \
                      (const short*)q.data_ptr(), (const short*)k.data_ptr(),   \
                      (const short*)v.data_ptr(), cu_seqlens.data_ptr<int>(),   \
                      (short*)o.data_ptr(), lse.data_ptr<float>(), Hq, Hkv, (float)scale,     \
-                     fa_head_window(grid.x, grid.y, rounds, causal))
+                     fa_head_window(grid.x, grid.y, rounds, causal || short_walks))
   FA_BY_WIDTH(CALL);
 #undef CALL
   HIP_CHECK_LAST();
