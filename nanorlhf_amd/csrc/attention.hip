@@ -16,12 +16,13 @@
 // has no atomics: dq, dk and dv are summed in registers in a fixed order and
 // written once.
 //
-// What bounds them: the matrix products' own rate under the power limit, the VALU
-// work between them (an exponential, a fused multiply-add, an addition and half a
-// conversion per score, and the fragments' addresses) and LDS reads (16 KB of
-// fragments per 32 x 32 scores and two products); two waves per SIMD overlap the
-// three.  5 causal sequences of about 6500 tokens, 12 heads over 2, width 128:
-// forward 0.90 to 1.02 ms (830 to 940 TFLOP/s), backward 2.9; before, with V
+// What bounds them: the matrix products (0.47 of the forward's cycles, 0.58 of dq's, 0.51 of
+// dk's and dv's, at 1.9 of 2.4 GHz), the VALU
+// work between them (0.46, 0.37 and 0.28: an exponential, a fused multiply-add, an addition and
+// half a conversion per score, and the fragments' addresses) and LDS reads (16 KB of
+// fragments per 32 x 32 scores and two products).  Two waves per SIMD overlap the reads, but
+// hardly the first two, whose shares add up to one in the forward of 64-wide heads.  5 causal sequences of about 6500 tokens, 12 heads over 2, width 128:
+// forward 0.90 to 1.02 ms (830 to 940 TFLOP/s), backward 2.83; before, with V
 // transposed by scalar LDS writes, 2.9 ms, and with dq added up by float atomics over
 // 32-row kv tiles, 21.5 ms for the backward.  Twice the rows per wave (half the LDS
 // reads, one wave per SIMD) and eight waves to a workgroup (half the loads) were slower
