@@ -27,7 +27,9 @@ enum { NO_BIAS, BIAS_F32, BIAS_BF16 };    // bf16: of an even N, on 4 bytes
 
 template <int ACT>
 DEVINL float glu(float g, float up) {
-  const float z = ACT != GELU_GLU ? g : 1.5957691216057308f * (g + 0.044715f * g * g * g);
+  // swiglu_fwd_kernel's steps, bit by bit: the exact quotient, which its backward has too
+  if (ACT == SILU_KEEP) return g * (1.f / (1.f + __expf(-g))) * up;
+  const float z = ACT == SILU_GLU ? g : 1.5957691216057308f * (g + 0.044715f * g * g * g);
   return g * __builtin_amdgcn_rcpf(1.f + __expf(-z)) * up;      // gelu_tanh: x sigmoid(2 ..)
 }
 
