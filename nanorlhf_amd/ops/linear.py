@@ -34,12 +34,14 @@ def unwatched(*tensors: torch.Tensor) -> bool:
 
 def differentiated(*tensors: torch.Tensor) -> bool:
     """Whether an autograd function of these has anything to do: a gradient, a forward-mode
-    derivative or a transform."""
+    derivative, a transform, or a trace, which records the function to run it again, but of a
+    kernel's call only the memory that its result got."""
     if torch.is_grad_enabled():
         for t in tensors:
             if t.requires_grad:
                 return True
-    return (forward_ad._current_level >= 0
+    return (forward_ad._current_level >= 0 or torch.jit.is_tracing()
+            or torch.compiler.is_compiling()
             or torch._C._functorch.peek_interpreter_stack() is not None)
 
 

@@ -128,6 +128,9 @@ def test_what_an_autograd_function_has_to_see():
     seen = []
     torch.func.vmap(lambda t: seen.append(differentiated(t)) or t)(torch.zeros(3, 2))
     assert seen == [True]
+    with torch.no_grad():                            # a trace keeps functions, not kernels' calls
+        torch.jit.trace(lambda t: seen.append(differentiated(t)) or t + 1, x, check_trace=False)
+    assert seen == [True] * 2
 
 
 def test_products_in_blocks_are_one_round_and_deep_ones_full():
