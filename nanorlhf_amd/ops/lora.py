@@ -80,8 +80,8 @@ def _choose_strategy(x, w, u, b, bias) -> str:
     known = _TUNE.setdefault((N, K), {})
     key = _strategy_key(M, N, K, bias, x.device)
     st = known.get(key)
-    if st is None and known and _capturing(x):
-        return next(iter(known.values()))       # nothing can be timed now
+    if st is None and _capturing(x):            # nothing can be timed now
+        return next(iter(known.values()), "fused" if K <= DEEP else "epilogue")
     if st is None:
         t_fused = _time_cuda(lambda: ext().lora_gemm(x, w, u, b, bias))
 
@@ -120,13 +120,12 @@ def _dispatch_gemm(x, w, u, b, bias):
 
 
 def _known_strategy(x, w, bias) -> str | None:
-    """The strategy that a rule says or an earlier call measured, None if neither does."""
+    """The strategy that a rule says or an earlier call measured, None if neither does.  A
+    rule's answer is not put among the measured ones: its sizes have no key of their own."""
     M, (N, K) = x.shape[0], w.shape
-    edge = 64 if blocks_fill(M, N) else 128 if _mid(M, N, K) else 0
-    if edge:
-        _TUNE.setdefault((N, K), {})[edge, False, bias is not None, x.device] = "fused"
+    known = _TUNE.setdefault((N, K), {})
+    if blocks_fill(M, N) or _mid(M, N, K):
         return "fused"
-    known = _TUNE.get((N, K))
     return known.get(_strategy_key(M, N, K, bias, x.device)) if known else None
 
 

@@ -108,6 +108,32 @@ def test_a_capture_takes_the_strategy_that_is_known_of_its_weight(monkeypatch):
     assert len(lora._TUNE[64, 64]) == 1         # and leaves the timing for later
 
 
+def test_a_rule_s_strategy_is_not_taken_for_a_measured_one(monkeypatch):
+    from types import SimpleNamespace
+    from nanorlhf_amd.ops import lora
+    monkeypatch.setattr(lora, "_TUNE", {})
+    monkeypatch.setattr(lora, "ext", lambda: SimpleNamespace(
+        lora_gemm_tiles=lambda M, K: 256 if M > 128 else 128,
+        lora_gemm_big=lambda M, N, K: M > 1000, lora_gemm=None, lora_add_=None))
+    w = torch.empty(1, dtype=torch.bfloat16)
+
+    def known(rows, N, K):
+        return lora._known_strategy(w.expand(rows, K), w.expand(N, K), None)
+
+    # blocks, tiles of 128, and more rows of the weight whose 100 rows are timed
+    for rows, N, K in [(64, 3000, 8960), (1024, 1536, 17920), (300, 9216, 2048)]:
+        assert known(rows, N, K) == "fused"
+    assert known(100, 9216, 12288) is None
+    known(200, 9216, 12288)
+    assert known(100, 9216, 12288) is None and not any(lora._TUNE.values())
+    # nor does a capture that has nothing measured try to time: it takes the rule of the depth
+    monkeypatch.setattr(lora, "_capturing", lambda x: True)
+    for K, want in [(2048, "fused"), (8960, "epilogue")]:
+        x = w.expand(4000, K)
+        assert known(64, 3000, K) == "fused"
+        assert lora._choose_strategy(x, w.expand(3000, K), None, None, None) == want
+
+
 def test_linears_of_few_rows_leave_what_the_library_does_faster():
     from nanorlhf_amd.ops.linear import rows_pay
     for M, N, K in [(1, 1536, 1536), (64, 16384, 2048), (32, 32768, 1536), (16, 18944, 1536),
