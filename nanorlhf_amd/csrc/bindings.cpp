@@ -50,6 +50,7 @@ torch::Tensor whiten_apply(torch::Tensor v, double mean, double invstd, double s
 // lora.hip
 bool lora_gemm_big(long M, long N, long K);
 long lora_gemm_tiles(long M, long K);
+long lora_gemm_round(long M, long N, long K);
 torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
                         c10::optional<torch::Tensor> u,
                         c10::optional<torch::Tensor> b,
@@ -142,6 +143,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("whiten_apply", &whiten_apply);
   m.def("lora_gemm_big", &lora_gemm_big);
   m.def("lora_gemm_tiles", &lora_gemm_tiles);
+  m.def("lora_gemm_round", &lora_gemm_round);
   m.def("lora_gemm", &lora_gemm, py::arg("x"), py::arg("w"),
         py::arg("u") = py::none(), py::arg("b") = py::none(),
         py::arg("bias") = py::none());

@@ -176,6 +176,12 @@ static bool takes_mid(long M, long N, long K) {
   return tiles <= 256 && K < (1L << 22) && (K <= 2048 || (K >= 10240 && tiles >= 96));
 }
 
+// the edge of what takes a product with an adapter in one round: 64 or 128, 0 neither
+// (ops/lora.py one_round)
+long lora_gemm_round(long M, long N, long K) {
+  return takes_blocks(M, N, K) ? 64 : takes_mid(M, N, K) ? 128 : 0;
+}
+
 // Up to 128 rows leave half of every other part of a 256-tile empty: 60 x 17920 x 1536 27 us in
 // tiles of 128, 30 in large ones; 130 x 17920 x 1536 36 and 30, 500 x 8960 x 1536 36 and 29,
 // 1000 x 4864 x 896 24 and 20, 4000 x 1536 x 1536 36 and 30; equal where a few tiles wait

@@ -22,7 +22,7 @@ from typing import Optional
 import torch
 
 from . import ext
-from .linear import blocks_fill, mid_fills
+from .linear import DEPTH, blocks_fill, mid_fills
 
 
 def lora_gemm_ref(x, w, u=None, b=None, bias=None):
@@ -103,6 +103,12 @@ def _mid(M: int, N: int, K: int) -> bool:
     return mid_fills(M, N, 0.0 if K <= 2048 else 0.375) and (K <= 2048 or 10240 <= K < 1 << 22)
 
 
+def one_round(M: int, N: int, K: int) -> int:
+    """The edge of the tiles, 64 or 128, in which lora_gemm takes the product in one round of the
+    CUs; 0 where it does not.  csrc/lora.hip lora_gemm_round is the same rule."""
+    return 64 if blocks_fill(M, N) and K < DEPTH else 128 if _mid(M, N, K) else 0
+
+
 def _dispatch_gemm(x, w, u, b, bias):
     """y = x·wᵀ + u·bᵀ (+bias) via the per-shape-tuned strategy, or in blocks of 64 rows
     (csrc/linear_rows.hip) while they are one round of the CUs.  212 rows, library and
@@ -124,7 +130,7 @@ def _known_strategy(x, w, bias) -> str | None:
     rule's answer is not put among the measured ones: its sizes have no key of their own."""
     M, (N, K) = x.shape[0], w.shape
     known = _TUNE.setdefault((N, K), {})
-    if blocks_fill(M, N) or _mid(M, N, K):
+    if one_round(M, N, K):
         return "fused"
     return known.get(_strategy_key(M, N, K, bias, x.device)) if known else None
 
@@ -223,8 +229,7 @@ def glu_keeps(M: int, N: int, K: int) -> bool:
     """Whether a gate/up product of these sizes writes its activation too (csrc/lora.hip
     lora_glu): where its kernel is the one of 256-tiles anyway, which is to say more than 128
     rows that are neither blocks of 64 nor tiles of 128 (_dispatch_gemm)."""
-    return (M > 128 and N % 8 == 0 and K < 1 << 22
-            and not blocks_fill(M, N) and not _mid(M, N, K))
+    return M > 128 and N % 8 == 0 and K < 1 << 22 and not one_round(M, N, K)
 
 
 class _LoRAGluFn(torch.autograd.Function):

@@ -51,6 +51,21 @@ def test_big_tiles_of_the_adapter_product_stop_where_offsets_end():
         assert tiles(rows, 1 << 22) == tiles(128, 64) == 128
 
 
+def test_adapter_products_of_one_round_by_one_rule():
+    """What is called "fused" without a timing is what the kernel's own choice makes of it."""
+    if not ops.ext_available():
+        pytest.skip("extensions are not built")
+    from nanorlhf_amd.ops.lora import one_round
+    seen = set()
+    for M in (1, 64, 65, 128, 129, 896, 897, 1000, 1152, 1153, 2048, 2049, 4000, 16384, 16385, 32769):
+        for N in (8, 64, 65, 128, 129, 896, 1024, 1025, 1536, 2048, 8192, 16384, 16385, 32768, 32769):
+            for K in (64, 2048, 2112, 4864, 9728, 10176, 10240, 16384, 16448, 17920, (1 << 22) - 64,
+                      1 << 22, (1 << 24) - 64, 1 << 24):
+                assert one_round(M, N, K) == ops.ext().lora_gemm_round(M, N, K), (M, N, K)
+                seen.add(one_round(M, N, K))
+    assert seen == {0, 64, 128} and one_round(4000, 64, 1536) == 128
+
+
 def test_adapter_strategies_are_kept_by_what_the_kernels_depend_on(monkeypatch):
     from types import SimpleNamespace
     from nanorlhf_amd.ops import lora
