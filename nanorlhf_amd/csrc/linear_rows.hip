@@ -297,10 +297,7 @@ torch::Tensor linear_rows(torch::Tensor x, torch::Tensor w, c10::optional<torch:
   return rows_product(x, w, bias, false);
 }
 
-// ops/linear.py blocks_fill
-bool linear_blocks_fill(long M, long N) {
-  return M <= 1152 && (M + 63) / 64 * ((N + 63) / 64) <= 256;
-}
+bool linear_blocks_fill(long M, long N) { return (M + 63) / 64 * ((N + 63) / 64) <= 256; }
 
 template <bool LORA>
 static void launch_blocks(const RowsArgs& a) {

@@ -75,10 +75,15 @@ def rows_pay(M: int, N: int, K: int) -> bool:
 BLOCK_ROWS = 1152
 
 
+def one_round_of_blocks(M: int, N: int) -> bool:
+    """Whether M rows and N columns are at most one round of 256 CUs in blocks of 64 x 64."""
+    return -(-M // 64) * -(-N // 64) <= 256
+
+
 def blocks_fill(M: int, N: int) -> bool:
-    """Whether M rows and N columns are at most one round of 256 CUs in blocks of 64 x 64;
-    many rows of a few columns are the library's (4000 of 64 x 1536 7 us, in blocks 10)."""
-    return M <= BLOCK_ROWS and -(-M // 64) * -(-N // 64) <= 256
+    """Of plain products; many rows of a few columns are the library's (4000 of 64 x 1536 7 us,
+    in blocks 10)."""
+    return M <= BLOCK_ROWS and one_round_of_blocks(M, N)
 
 
 def blocks_pay(M: int, N: int, K: int) -> bool:

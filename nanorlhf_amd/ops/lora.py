@@ -22,7 +22,7 @@ from typing import Optional
 import torch
 
 from . import ext
-from .linear import DEPTH, blocks_fill, mid_fills
+from .linear import DEPTH, mid_fills, one_round_of_blocks
 
 
 def lora_gemm_ref(x, w, u=None, b=None, bias=None):
@@ -105,8 +105,11 @@ def _mid(M: int, N: int, K: int) -> bool:
 
 def one_round(M: int, N: int, K: int) -> int:
     """The edge of the tiles, 64 or 128, in which lora_gemm takes the product in one round of the
-    CUs; 0 where it does not.  csrc/lora.hip lora_gemm_round is the same rule."""
-    return 64 if blocks_fill(M, N) and K < DEPTH else 128 if _mid(M, N, K) else 0
+    CUs; 0 where it does not.  csrc/lora.hip lora_gemm_round is the same rule.  Blocks of 64 also
+    of many rows of a few columns, for which the library needs a pass more: library and
+    lora_add_ / tiles of 128 / blocks in us, of a depth of 896: 1200 x 64 11.8 / 10.5 / 5.0, 16384 x
+    64 18.4 / 12.6 / 11.6, 2048 x 512 13.6 / 11.2 / 9.7; of 2048 4000 x 128 20 / 23 / 13."""
+    return 64 if one_round_of_blocks(M, N) and K < DEPTH else 128 if _mid(M, N, K) else 0
 
 
 def _dispatch_gemm(x, w, u, b, bias):
