@@ -167,13 +167,14 @@ static bool takes_blocks(long M, long N, long K) {
   return linear_blocks_fill(M, N) && K < (1L << 24);
 }
 
-// linear_mid.hip: up to one round of the CUs in tiles of 128, but for the depths and rows that
+// linear_mid.hip: up to one round of the CUs in tiles of 128, but for the depths and sizes that
 // the library divides better (ops/lora.py has the figures)
 torch::Tensor linear_mid(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> u,
                          c10::optional<torch::Tensor> b, c10::optional<torch::Tensor> bias);
 static bool takes_mid(long M, long N, long K) {
   const long tiles = (M + 127) / 128 * ((N + 127) / 128);
-  return tiles <= 256 && K < (1L << 22) && (K <= 2048 || (K >= 10240 && tiles >= 96));
+  return tiles <= 256 && K < (1L << 22) &&
+         (K <= 2048 || (K > 16384 && M >= 1000 && N >= 1024 && tiles >= 96));
 }
 
 // the edge of what takes a product with an adapter in one round: 64 or 128, 0 neither

@@ -97,10 +97,17 @@ def _choose_strategy(x, w, u, b, bias) -> str:
 def _mid(M: int, N: int, K: int) -> bool:
     """Whether lora_gemm takes csrc/linear_mid.hip's tiles of 128.  Library and lora_add_ / these in
     us, over operands that no cache holds: 1000 rows of 896 x 896 13.3 / 11.4, 2667 17.5 / 11.7,
-    1800 of 2048 x 1536 25.5 / 19.4, 2667 of 1536 x 2048 31 / 24 (tiles of 256 27 to 33); 1000
-    of 1536 x 17920 199 / 160, 2667 214 / 161, but 500 139 / 158; between those depths the library
-    divides what is no round: 1300 of 896 x 4864 34 / 47, 1800 of 1536 x 8960 73 / 81."""
-    return mid_fills(M, N, 0.0 if K <= 2048 else 0.375) and (K <= 2048 or 10240 <= K < 1 << 22)
+    1800 of 2048 x 1536 25.5 / 19.4, 2667 of 1536 x 2048 31 / 24 (tiles of 256 27 to 33), 100 of
+    17920 x 1536 30 / 22; the slowest 2667 of 512 x 2048 20.9 / 22.7.  Deeper the library divides
+    what is no round, 1300 of 896 x 4864 34 / 47, 1800 of 1536 x 8960 73 / 81, 1000 and 2667 of
+    1536 x 12288 74 / 113 and 121 / 119, of 1536 x 16384 91 / 138 and 152 / 149, up to a depth from
+    which it takes kernels of half the rate: of 1536 x 17920 200 / 160 and 214 / 161, of 2048 x
+    18944 199 / 165 (1800 rows 219 / 169), 1300 of 1536 x 37888 312 / 323, 1152 of 3584 x
+    18944 225 / 174; but 800 of 2048 x 17920 133 / 157 and 1800 of 896 x 17920 130 / 158.  What is
+    left between is timed."""
+    if K <= 2048:
+        return mid_fills(M, N, 0.0)
+    return 16384 < K < 1 << 22 and M >= 1000 and N >= 1024 and mid_fills(M, N, 0.375)
 
 
 def one_round(M: int, N: int, K: int) -> int:

@@ -57,7 +57,7 @@ def test_adapter_products_of_one_round_by_one_rule():
         pytest.skip("extensions are not built")
     from nanorlhf_amd.ops.lora import one_round
     seen = set()
-    for M in (1, 64, 65, 128, 129, 896, 897, 1000, 1152, 1153, 2048, 2049, 4000, 16384, 16385, 32769):
+    for M in (1, 64, 65, 128, 129, 896, 897, 999, 1000, 1152, 1153, 2048, 2049, 4000, 16384, 16385, 32769):
         for N in (8, 64, 65, 128, 129, 896, 1024, 1025, 1536, 2048, 8192, 16384, 16385, 32768, 32769):
             for K in (64, 2048, 2112, 4864, 9728, 10176, 10240, 16384, 16448, 17920, (1 << 22) - 64,
                       1 << 22, (1 << 24) - 64, 1 << 24):
@@ -197,6 +197,10 @@ def test_products_in_tiles_of_128_are_half_a_round_to_one():
         assert _mid(M, N, K)
     for M, N, K in [(896, 1536, 17920), (1800, 1536, 8960), (3585, 1152, 896)]:
         assert not _mid(M, N, K)
+    # deep ones only where the library's kernels were seen to be slow
+    for M, N, K in [(1300, 1536, 10240), (2667, 1536, 16384), (999, 3584, 17920), (1800, 896, 17920)]:
+        assert not _mid(M, N, K)
+    assert _mid(1000, 3584, 18944) and _mid(1000, 1536, 16448)
 
 
 def test_large_products_by_rounds_and_depth():
