@@ -153,31 +153,45 @@ def _plain_bias(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> 
             and bias.device == x.device and bias.shape == w.shape[:1] and bias.is_contiguous())
 
 
-def _rows(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
-    return few_rows(x, w) and rows_pay(x.shape[0], *w.shape) and _plain_bias(x, w, bias)
+def linear_route(M: int, N: int, K: int) -> str | None:
+    """Which of the extension's products is the faster way for x [M, K] and w [N, K]; None where
+    the library is."""
+    if M <= FEW_ROWS and rows_pay(M, N, K):
+        return "linear_rows"
+    if M > FEW_ROWS and blocks_pay(M, N, K):
+        return "linear_blocks"
+    if mid_pays(M, N, K):
+        return "linear_mid"
+    return "linear_big" if N % 4 == 0 and K < 1 << 22 and big_pays(M, N, K) else None
 
 
-def _blocks(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
-    return (x.dim() == w.dim() == 2 and x.shape[0] > FEW_ROWS
-            and blocks_pay(x.shape[0], *w.shape)
-            and _plain_operands(x, w) and _plain_bias(x, w, bias))
+def linear_kernel(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> str | None:
+    """Which of the extension's products takes these, None where it is the library."""
+    if x.dim() != 2 or w.dim() != 2:
+        return None
+    name = linear_route(x.shape[0], *w.shape)
+    if name is None or not _plain_operands(x, w) or not _plain_bias(x, w, bias):
+        return None
+    if name in ("linear_mid", "linear_big") and x.shape[1] == 0:
+        return None
+    if name == "linear_big" and bias is not None and bias.data_ptr() % 4:
+        return None
+    return name
 
 
-def _mid(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
-    return (x.dim() == w.dim() == 2 and mid_pays(x.shape[0], *w.shape) and x.shape[1] > 0
-            and _plain_operands(x, w) and _plain_bias(x, w, bias))
-
-
-def _big(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
-    return (x.dim() == w.dim() == 2 and w.shape[0] % 4 == 0 and big_pays(x.shape[0], *w.shape)
-            and 0 < x.shape[1] < 1 << 22 and _plain_operands(x, w) and _plain_bias(x, w, bias)
-            and (bias is None or bias.data_ptr() % 4 == 0))
+def linear_by(name: str | None, x: torch.Tensor, w: torch.Tensor,
+              bias: torch.Tensor | None) -> torch.Tensor:
+    """x w^T + bias by what linear_kernel said of them."""
+    if name is None:
+        return F.linear(x, w, bias)
+    if name == "linear_mid":
+        return linear_ext().linear_mid(x, w, None, None, bias)
+    return getattr(linear_ext(), name)(x, w, bias)
 
 
 def linear_takes_big(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None) -> bool:
     """Whether linear takes these to linear_big."""
-    return (not (_rows(x, w, bias) or _blocks(x, w, bias) or _mid(x, w, bias))
-            and _big(x, w, bias))
+    return linear_kernel(x, w, bias) == "linear_big"
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None,
@@ -186,26 +200,20 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None,
     near ties of the router's logits, and another kernel's last bits turn one of them in a
     token of some thousand (a prompt's logits 0.046 off in place of 0.015), so such a product
     stays where it was rounded before: more rows than few are the library's."""
-    if _rows(x, w, bias):
-        return linear_ext().linear_rows(x, w, bias)
-    if routed:
-        return F.linear(x, w, bias)
-    if _blocks(x, w, bias):
-        return linear_ext().linear_blocks(x, w, bias)
-    if _mid(x, w, bias):
-        return linear_ext().linear_mid(x, w, None, None, bias)
-    if _big(x, w, bias):
-        return linear_ext().linear_big(x, w, bias)
-    return F.linear(x, w, bias)
+    name = linear_kernel(x, w, bias)
+    if routed and name != "linear_rows":
+        name = None
+    return linear_by(name, x, w, bias)
 
 
 def linear_parts(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None):
     """x w^T + bias for a kernel that can add up parts as it reads them: [M, N], or, where
     the depth is divided among workgroups, float32 parts [parts, M, N] of x w^T without the
     bias.  See sum_parts for what they stand for."""
-    if _rows(x, w, bias):
+    name = linear_kernel(x, w, bias)
+    if name == "linear_rows":
         return linear_ext().linear_rows_parts(x, w, bias)
-    return linear(x, w, bias)
+    return linear_by(name, x, w, bias)
 
 
 def sum_parts(y: torch.Tensor, dtype: torch.dtype,

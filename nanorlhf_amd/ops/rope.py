@@ -9,7 +9,7 @@ from __future__ import annotations
 import torch
 
 from . import ext, linear_ext, serve_ext
-from .linear import differentiated, linear, linear_takes_big, unwatched
+from .linear import differentiated, linear_by, linear_kernel, unwatched
 
 
 def build_rope_cache(head_dim: int, max_pos: int, theta: float = 1e6,
@@ -98,15 +98,16 @@ def qkv_rope(qkv: torch.Tensor, table: torch.Tensor, positions: torch.Tensor, he
 def linear_qkv_rope(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None,
                     table: torch.Tensor, positions: torch.Tensor, heads: int, kv_heads: int):
     """qkv_rope of linear(x, w, bias), in one kernel where that product is linear_big's."""
-    if w.shape[0] in [(heads + 2 * kv_heads) * d for d in (64, 128)] \
-            and linear_takes_big(x, w, bias) and unwatched(table, positions) \
+    name = linear_kernel(x, w, bias)
+    if name == "linear_big" and w.shape[0] in [(heads + 2 * kv_heads) * d for d in (64, 128)] \
+            and unwatched(table, positions) \
             and table.dim() == 2 and table.shape[1] * (heads + 2 * kv_heads) == w.shape[0] \
             and table.dtype == torch.float32 and table.is_contiguous() \
             and table.data_ptr() % 8 == 0 and table.device == positions.device == x.device \
             and positions.dtype == torch.int64 and positions.is_contiguous() \
             and positions.numel() == x.shape[0] < 1 << 28:
         return tuple(linear_ext().linear_big_rope(x, w, bias, table, positions, heads, kv_heads))
-    return qkv_rope(linear(x, w, bias), table, positions, heads, kv_heads)
+    return qkv_rope(linear_by(name, x, w, bias), table, positions, heads, kv_heads)
 
 
 class Rotation:

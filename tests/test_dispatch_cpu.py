@@ -158,6 +158,22 @@ def test_linears_of_few_rows_leave_what_the_library_does_faster():
         assert not rows_pay(M, N, K)
 
 
+def test_operands_of_a_product_are_looked_at_once(monkeypatch):
+    import sys
+    linear = sys.modules["nanorlhf_amd.ops.linear"]
+    asked = []
+    monkeypatch.setattr(linear, "_plain_operands", lambda x, w: asked.append(x.shape[0]))
+    table, w = ops.build_rope_cache(64, 10), torch.zeros(192, 896)
+    # few rows, blocks of 64, tiles of 128 and of 256, and sizes that the library takes anyway
+    rows = [4, 130, 8192, 60000]
+    with torch.no_grad():
+        for M in (*rows, 1500):
+            x = torch.zeros(M, 896)
+            ops.linear(x, w), ops.linear_parts(x, w)
+            ops.linear_qkv_rope(x, w, None, table, torch.zeros(M, dtype=torch.int64), 1, 1)
+    assert asked == [M for M in rows for _ in range(3)]
+
+
 def test_what_an_autograd_function_has_to_see():
     from nanorlhf_amd.ops.linear import differentiated
     x, y = torch.zeros(2), torch.zeros(2, requires_grad=True)
