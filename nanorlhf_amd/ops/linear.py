@@ -113,26 +113,54 @@ def mid_pays(M: int, N: int, K: int) -> bool:
     Library / kernel in us: 2667 rows of 1152 x 896 13.2 / 11.5, 1000 of 3072 x 1024 14.2 /
     12.4, 1500 of 2048 x 1536 15.3 / 15.8, 2667 of 1536 x 1536 18.0 / 17.8, with some 14 us less
     of the host's time; half a round or less 1500 of 1152 x 896 9.3 / 10.9, deeper 2667 of
-    896 x 4864 35.7 / 35.3, more than a round 4000 of 1152 x 896 13.8 / 20.8."""
-    return K <= 2048 and mid_fills(M, N, 0.5)
+    896 x 4864 35.7 / 35.3, more than a round 4000 of 1152 x 896 13.8 / 20.8.  Few rows of many
+    columns and many rows of few, whose tiles are in part empty, over operands that no cache
+    holds: up to a depth of 1024 17 to 64 rows of 18944 x 896 15.0 to 13.6 / 11.2 to 12.3, 128 of
+    32768 x 1024 20.2 / 18.3, 30000 of 64 x 896 16.5 / 15.3; up to 1536 33 rows of 18944 19.3 / 19.9,
+    but 65 25.2 / 22.0, 30000 of 128 26.1 / 28.9, but 9000 of 256 23.6 / 20.7; up to 2048 129 of 8960
+    17.8 / 22.0, 128 of 16384 22.5 / 25.9, but 192 of 8960 25.1 / 22.0 (320 of 6144 17.8 / 21.4, as
+    the only one of those)."""
+    if not mid_fills(M, N, 0.5) or K > 2048:
+        return False
+    return K <= 1024 or N > 128 and M > (FEW_ROWS if K <= 1536 else 160)
+
+
+def big_rows(M: int, N: int, K: int) -> bool:
+    """Whether M rows are worth tiles of 256: up to three rows of tiles whose last one is more
+    than half there, or a few rows of so many columns that they are nearly a round.  Library /
+    kernel in us, over operands that no cache holds: 160 rows of 151936 x 1536 141 / 120, 65 122 /
+    110, 65 of 65536 54 / 47, 130 of 49152 49 / 44, but of 32768 x 1024 21.4 / 27.1; 257 rows of
+    128100 x 1536 152 / 165, 340 of 16640 x 1024 20.6 / 24.0, 513 of 24576 x 1536 54 / 61, but 385 of
+    128100 233 / 186, 385 of 16640 23.2 / 24.2, 700 of 18944 x 1024 30.5 / 28.4; 770 of 32768 x 1536
+    86 / 75, of 24576 63 / 68."""
+    tiles = -(-M // 256) * -(-N // 256)
+    if M <= FEW_ROWS:
+        return K <= 1024 and tiles >= 256
+    return M > 768 or (tiles >= 192 if M <= 256 else (M - 1) % 256 >= 128)
 
 
 def big_pays(M: int, N: int, K: int) -> bool:
     """Whether csrc/gemm_big.h's tiles of 256 x 256 are the faster way for many rows, by rounds
     of the 256 CUs.  Library / kernel, geometric means over some 20 numbers of rows (lowest,
     highest): from 0.45 rounds on 1.33 (0.99, 1.88) for 1152 x 896, 1.27 for 896 x 896, 1.03
-    for 3072 x 1024, 1.01 for 1024 x 1024; with fewer rounds its few tiles' latencies count:
-    2500 of 1152 x 896 10.6 / 14.6 us.  From one round on 1.05 (0.95, 1.23) for 2048 x 1536,
+    for 3072 x 1024; with fewer rounds its few tiles' latencies count: 2500 of 1152 x 896 10.6 /
+    14.6 us.  Columns that are 256 or a few times as many fit the library's own tiles: 1024 x 896
+    and x 1024 0.97 (0.88, 1.33) and 0.92 (0.88, 1.00), 512 x 896 0.91 (0.87, 0.96), but 640 1.26
+    (0.99, 1.59), 1280 1.07 (0.91, 1.45); up to 128 columns leave half of each tile empty: 46673
+    of 64 x 896 22.3 / 27.2.  From one round on 1.05 (0.95, 1.23) for 2048 x 1536,
     1.04 for 1536 x 1536, 1.03 for 6144 x 1536 and 8960 x 1536.  Up to a depth of 9000 the library
     divides what is no whole round (1536 x 8960 0.98); deeper its choice falls at random on a
-    kernel of half its rate: beyond one round and up to five 1.14 (0.91, 1.53) for 1536 x 10496,
-    1.16 for 2048 x 13056, 1.20 for 3584 x 18944; 19235 rows of 1536 x 10496 729 / 489 us."""
+    kernel of half its rate: beyond one round and up to five 1.14 (0.85, 1.59) for 1536 x 10496,
+    1.16 for 2048 x 13056, 1.20 for 3584 x 18944; 19235 rows of 1536 x 10496 729 / 489 us.  It does
+    so below 10240 too, where the library is left what it had: over seven numbers of
+    rows of 1536 and 2048 columns 8960 1.08 (0.92, 1.54), 9728 1.09 (0.88, 1.50), 10240 1.11 (0.88,
+    1.57), 12288 1.18 (0.96, 1.57)."""
     tiles = -(-M // 256) * -(-N // 256)
-    if K <= 1024:
-        return tiles >= 115
-    if K <= 2048:
-        return tiles >= 256
-    return K >= 10240 and 256 < tiles <= 1280
+    if not big_rows(M, N, K):
+        return False
+    if K > 2048:
+        return K >= 10240 and 256 < tiles <= 1280
+    return tiles >= (115 if K <= 1024 else 256) and N > 128 and (N > 1024 or N % 256 > 0)
 
 
 def _plain_operands(x: torch.Tensor, w: torch.Tensor) -> bool:

@@ -201,6 +201,29 @@ def test_products_in_blocks_are_one_round_and_deep_ones_full():
     assert blocks_fill(130, 1536) and not blocks_fill(897, 1152)
 
 
+def test_a_linear_s_route_where_tiles_are_in_part_empty():
+    """What is the library's by one rule is not taken by the next one."""
+    from nanorlhf_amd.ops.linear import linear_route
+    for sizes, want in [
+            # few rows of many columns
+            ([(1, 1536, 1536), (64, 16384, 2048), (64, 151936, 2048)], "linear_rows"),
+            ([(33, 32768, 1536), (17, 18944, 1536), (33, 65536, 1536), (64, 40960, 896)], None),
+            ([(33, 32768, 1024), (17, 18944, 896), (65, 18944, 1536)], "linear_mid"),
+            ([(65, 151936, 1536), (255, 128100, 2048), (33, 65536, 896), (96, 49152, 1024)], "linear_big"),
+            ([(129, 32768, 1024), (256, 32768, 896), (129, 8960, 2048), (100, 16384, 2048)], None),
+            # a last row of tiles that is half there or less, and more
+            ([(257, 151936, 1536), (384, 65536, 896), (513, 24576, 1536), (640, 128100, 2048)], None),
+            ([(385, 65536, 896), (641, 128100, 2048), (769, 32768, 1536)], "linear_big"),
+            # many rows of few columns
+            ([(46673, 4, 896), (46673, 128, 1024), (64000, 1024, 1024), (64000, 512, 896),
+              (16400, 4, 2048), (30000, 128, 1536)], None),
+            ([(16400, 4, 896), (30000, 128, 1024), (9000, 256, 1536)], "linear_mid"),
+            ([(46673, 192, 896), (46673, 1152, 896), (64000, 3072, 1024), (64000, 640, 1536)],
+             "linear_big")]:
+        for M, N, K in sizes:
+            assert linear_route(M, N, K) == want, (M, N, K)
+
+
 def test_products_in_tiles_of_128_are_half_a_round_to_one():
     from nanorlhf_amd.ops.linear import mid_fills, mid_pays
     for M, N, K in [(1921, 1152, 896), (3584, 1152, 896), (2048, 2048, 2048)]:
