@@ -41,11 +41,13 @@ def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
 # 37), deep products have little to save (4096 x 18944 x 3584: 872 / 910), and its tiles
 # have to fill the CUs' rounds (glu_fills).
 GLU_ROWS, GLU_DEPTH = 512, 2048
-# Fewer rows are as fast by it, and a library call (19 us of the host's time) and a launch
-# less, where 36 tiles of columns or more keep CUs at work and, in the deeper ones, the last
-# 256 rows are more than half there: 212 x 4864 x 896 16.2 / 15.5, 400 19.1 / 17.0, 212 x
-# 8960 x 1536 26.3 / 25.5, 400 32.8 / 31.1, 212 x 11008 x 2048 33.2 / 32.6; but 128 x 4864 x 896
-# 12.2 / 15.7, 212 x 4096 x 1024 13.5 / 16.8, 328 x 8960 x 1536 28.6 / 31.3.
+# Fewer rows are about as fast by it, and a library call (19 us of the host's time) and a launch
+# less, where 36 tiles of columns or more keep CUs at work and, in the deeper ones, 70 tiles do and
+# the last 256 rows are more than half there.  In us, over operands that no cache holds: 212 x 4864
+# x 896 17.4 / 17.9, 400 21.1 / 18.9, 192 x 8192 x 896 as the slowest 0.86 of the rate; 212 x 8960
+# x 1536 32.9 / 33.2, 385 37.0 / 35.3, 212 x 11008 x 2048 41.6 / 40.4; but 192 x 6144 x 1536, of 48
+# tiles, 23.0 / 29.4, 288 x 7168 x 1536 0.95, 257 x 4608 x 1536 0.83, and with the weights in
+# caches 128 x 4864 x 896 12.2 / 15.7, 212 x 4096 x 1024 13.5 / 16.8, 328 x 8960 x 1536 28.6 / 31.3.
 GLU_FEWER, GLU_WIDE = 192, 36 * 128
 # The kernel of few rows does not divide the depth: 16 rows of 4128 x 8192 take the library
 # and a pass 36 us, it 45, of 4128 x 4096 28 and 23.
@@ -65,7 +67,8 @@ def glu_fills(M: int, I: int, K: int) -> bool:
 def glu_pays(M: int, I: int, K: int) -> bool:
     if M >= GLU_ROWS:
         return glu_fills(M, I, K)
-    return M >= GLU_FEWER and I >= GLU_WIDE and (K <= 1024 or (M - 1) % 256 >= 143)
+    return M >= GLU_FEWER and I >= GLU_WIDE and (
+        K <= 1024 or (M - 1) % 256 >= 128 and -(-M // 256) * -(-I // 128) >= 70)
 
 
 def glu_fuses(x: torch.Tensor, gate: torch.Tensor) -> bool:

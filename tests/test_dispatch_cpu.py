@@ -256,7 +256,12 @@ def test_gated_products_of_fewer_rows():
     for M, I, K in [(192, 4608, 896), (212, 8960, 1536), (300, 4864, 896), (400, 8960, 1536),
                     (600, 8960, 1536)]:
         assert glu_pays(M, I, K)
-    for M, I, K in [(191, 4864, 896), (212, 4096, 1024), (328, 8960, 1536), (399, 8960, 1536)]:
+    for M, I, K in [(191, 4864, 896), (212, 4096, 1024), (328, 8960, 1536), (384, 8960, 1536)]:
+        assert not glu_pays(M, I, K)
+    # the last 256 rows of deeper ones more than half there, and tiles enough
+    for M, I, K in [(385, 8960, 1536), (511, 6144, 2048), (192, 8960, 2048), (500, 4608, 1536)]:
+        assert glu_pays(M, I, K)
+    for M, I, K in [(192, 6144, 1536), (256, 8832, 1536), (256, 4608, 1088)]:
         assert not glu_pays(M, I, K)
 
 
