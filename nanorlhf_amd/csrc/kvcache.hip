@@ -466,7 +466,6 @@ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
     take_q();
   }
 
-
   for (; it < it1; it += 4) {
     const int t0 = tile_of(it) * 32;
     // V^T fragments: row d = 16t + lo, tokens 8hi .. + 7 of the two pages
@@ -482,12 +481,15 @@ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
       }
     }
     if constexpr (NEW) {
-      const int at = L - 1 - t0;
-      if (at < 32 && at >= 0) {              // the newest token's tile
-        if (lo == (at & 15)) {
+      // The newest token's place in the tiles that have its page: the last one or, of a length past
+      // its table, all that read the table's last page again, where it was put.
+      const int own = min((L - 1) >> 4, maxP - 1), at = (L - 1) & 15, first = 2 * tile_of(it);
+      if (first + 1 >= own) {
+        const bool has[2] = {min(first, maxP - 1) == own, min(first + 1, maxP - 1) == own};
+        if (lo == at) {
 #pragma unroll
           for (int n = 0; n < 2; n++) {
-            if (n != at >> 4) continue;
+            if (!has[n]) continue;
 #pragma unroll
             for (int c = 0; c < KTile<D, CT>::NV; c++) {
               if constexpr (!FP8) {
@@ -501,7 +503,7 @@ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
             }
           }
         }
-        if (hi == at >> 3) {
+        if ((hi < 2 ? has[0] : has[1]) && (hi & 1) == at >> 3) {
           const int bits = FP8 ? 8 * (at & 3) : 16 * (at & 1), word = FP8 ? (at & 7) >> 2
                                                                           : (at & 7) >> 1;
           const unsigned mask = (FP8 ? 0xffu : 0xffffu) << bits;
