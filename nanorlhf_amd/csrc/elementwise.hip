@@ -684,7 +684,7 @@ void embedding_grad_kernel(const long* __restrict__ ids, const short* __restrict
   __shared__ unsigned long long same[EMBED_MOST / 64];
   __shared__ unsigned short list[EMBED_MOST];
   __shared__ int count;
-  __shared__ float sums[EMBED_BLOCK][8];
+  __shared__ __attribute__((aligned(16))) float sums[EMBED_BLOCK][8];
   const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const long id = ids[t];
   if (id < 0 || id >= V) return;

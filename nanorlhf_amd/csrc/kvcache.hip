@@ -307,7 +307,7 @@ DEVINL void write_pair(short* out, float o0, float o1, int b, int h, int d, int 
 // were two, in us: 64 x 170 tokens of 12 over 2 heads in fp8 9.0 -> 6.8, one sequence of 60
 // tokens 7.4 -> 5.7, 32 x 2000 in bf16 17.9 -> 15.4, 256 x 600 24.8 -> 22.4.
 template <int D, typename CT>
-struct NewToken {
+struct alignas(16) NewToken {         // read and written 16 bytes at a time
   short q[16][D], k[D], v[D];
   unsigned char k8[D], v8[D];       // of an fp8 cache; k8 fragment-major, as the cache has it
 
@@ -414,6 +414,7 @@ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
   // an fp8 cache, whose bytes feed the MFMA directly
   bf16x8k qf[NC];
   long qf8[NC];
+  static_assert(!NEW || (alignof(NewToken<D, CT>) >= 16 && D % 16 == 0));
   __shared__ std::conditional_t<NEW, NewToken<D, CT>, NoToken> now;
   auto take_q = [&] {
 #pragma unroll
@@ -437,7 +438,7 @@ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
 
   constexpr int LD = DV + 4;               // rows of 16 lanes start at different banks
   __shared__ float Lm[4][16], Ls[4][16];   // per-wave (m, s) of each head
-  __shared__ float Lacc[4][16 * LD];       // per-wave sums
+  __shared__ __attribute__((aligned(16))) float Lacc[4][16 * LD];      // per-wave sums
 
   float m = -INFINITY, sum = 0.f;          // log2 units; of head lo
   f32x4 acc[NT];                           // O^T: rows d = 16t + 4hi + r, column lo
