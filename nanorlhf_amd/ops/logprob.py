@@ -69,7 +69,8 @@ class _TokenLogprobFn(torch.autograd.Function):
             # in-place: logits <- bf16( g * (softmax(logits*inv_t) - onehot) * inv_t )
             ext().ce_backward_dlogits(logits, labels[s:e], lse[s:e],
                                       g_lp[s:e].contiguous().float(), float(ctx.inv_temp))
-            if torch.is_grad_enabled():          # a recorded backward
+            # a recorded backward, or one whose products are cast, cannot write in place
+            if torch.is_grad_enabled() or torch.is_autocast_enabled():
                 dh[s:e] = torch.mm(logits, weight)
             else:
                 torch.mm(logits, weight, out=dh[s:e])
