@@ -13,6 +13,7 @@ from __future__ import annotations
 import torch
 
 from .. import ops
+from ..models.qwen2 import AttnContext, DecodeContext
 from .cache import PagedKVCache, SeqState
 
 
@@ -90,17 +91,21 @@ class DecodeBatch:
         return max(self.due, default=self.clock) - self.clock
 
     # ------------------------------------------------------------------ step
-    def step_inputs(self):
-        """Tensors for the next decode forward (all on device, no sync)."""
-        ps = self.pool.page_size
+    def context(self, kv_caches) -> AttnContext:
+        """What the next decode forward is told of the batch (all on device, no sync)."""
+        ps, fields = self.pool.page_size, dict(kv_caches=kv_caches, state_slots=self.state_slots)
         if self.seq_lens.is_cuda:
-            pos, slots = ops.ext().decode_inputs(self.seq_lens, self.bt, ps)
-            return self.last_tok, pos, slots, self.seq_lens, self.bt
+            return DecodeContext((self.seq_lens, self.bt, ps), **fields)
         pos = (self.seq_lens - 1).long()
         page_idx = torch.div(pos, ps, rounding_mode="floor")
         page = self.bt.gather(1, page_idx.unsqueeze(1).int().long()).squeeze(1).long()
-        slots = page * ps + pos % ps
-        return self.last_tok, pos, slots, self.seq_lens, self.bt
+        return AttnContext(mode="decode", positions=pos, slots=page * ps + pos % ps,
+                           block_tables=self.bt, seq_lens=self.seq_lens, **fields)
+
+    def step_inputs(self):
+        """Tensors for the next decode forward: tokens, and what its context says."""
+        ctx = self.context(None)
+        return self.last_tok, ctx.positions, ctx.slots, ctx.seq_lens, ctx.block_tables
 
     def commit(self, tokens: torch.Tensor, lps: torch.Tensor | None = None,
                step: torch.Tensor | None = None):

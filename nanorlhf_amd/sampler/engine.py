@@ -20,7 +20,7 @@ import numpy as np
 import torch
 
 from .. import ops
-from ..models.qwen2 import AttnContext, DecodeContext, Portions
+from ..models.qwen2 import AttnContext, Portions
 from ..models.lora import merge_for_rollout, unmerge
 from .cache import PagedKVCache, SeqState
 from .decode_batch import DecodeBatch
@@ -256,15 +256,7 @@ class SamplerEngine:
 
     # --------------------------------------------------------------- decode
     def _decode_step_eager(self, db: DecodeBatch, params: SamplingParams):
-        fields = dict(kv_caches=self.pool.layers, state_slots=db.state_slots)
-        if db.seq_lens.is_cuda:
-            ids = db.last_tok
-            ctx = DecodeContext((db.seq_lens, db.bt, self.pool.page_size), **fields)
-        else:
-            ids, pos, slots, seq_lens, bt = db.step_inputs()
-            ctx = AttnContext(mode="decode", positions=pos, slots=slots, block_tables=bt,
-                              seq_lens=seq_lens, **fields)
-        hidden = self.model(ids, ctx)
+        hidden = self.model(db.last_tok, db.context(self.pool.layers))
         tokens, lps = self._sample_from_hidden(hidden, params, counts=False)
         db.commit(tokens, lps, self._step_dev)
 
