@@ -225,9 +225,10 @@ def linear_takes_big(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None,
            routed: bool = False) -> torch.Tensor:
     """x w^T + bias.  `routed`: a router reads what becomes of it.  A token's experts hang on
-    near ties of the router's logits, and another kernel's last bits turn one of them in a
-    token of some thousand (a prompt's logits 0.046 off in place of 0.015), so such a product
-    stays where it was rounded before: more rows than few are the library's."""
+    near ties of the router's logits, and other last bits turn one of them in a token of some
+    thousand (a prompt's logits 0.046 off in place of 0.015), so more rows than few are left to
+    the library, with whose bits such models were checked.  It is no nearer to 64 bits than the
+    kernels, and other numbers of rows, as of a prompt in portions, have other bits by it too."""
     name = linear_kernel(x, w, bias)
     if routed and name != "linear_rows":
         name = None
