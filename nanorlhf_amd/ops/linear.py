@@ -229,10 +229,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None,
     thousand (a prompt's logits 0.046 off in place of 0.015), so more rows than few are left to
     the library, with whose bits such models were checked.  It is no nearer to 64 bits than the
     kernels, and other numbers of rows, as of a prompt in portions, have other bits by it too."""
+    if routed and (x.dim() != 2 or x.shape[0] > FEW_ROWS):
+        return F.linear(x, w, bias)
     name = linear_kernel(x, w, bias)
-    if routed and name != "linear_rows":
-        name = None
-    return linear_by(name, x, w, bias)
+    return linear_by(None if routed and name != "linear_rows" else name, x, w, bias)
 
 
 def linear_parts(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None):

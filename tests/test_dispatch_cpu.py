@@ -172,6 +172,10 @@ def test_operands_of_a_product_are_looked_at_once(monkeypatch):
             ops.linear(x, w), ops.linear_parts(x, w)
             ops.linear_qkv_rope(x, w, None, table, torch.zeros(M, dtype=torch.int64), 1, 1)
     assert asked == [M for M in rows for _ in range(3)]
+    with torch.no_grad():
+        for M in rows[1:]:
+            ops.linear(torch.zeros(M, 896), w, None, routed=True)      # the library's anyway
+    assert len(asked) == 12
 
 
 def test_what_an_autograd_function_has_to_see():
