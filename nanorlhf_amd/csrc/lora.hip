@@ -285,13 +285,13 @@ torch::Tensor lora_gemm(torch::Tensor x, torch::Tensor w,
 // (act, gate | up): silu(gate) * up of both halves of y = x w^T + u b^T [M, 2 I], which are
 // rounded first and stored too.  A pass over y, which read what the product had just written, took
 // 428 us of 46673 x 17920 beside 2.2 ms for the product.  Product and pass / this in us, y [M, 2 I],
-// over operands that no cache holds: 46673 x 17920 x 1536 2513 / 2420, 13000 714 / 664, 2667 176 /
-// 168, 1000 79.6 / 77.3, 130 33.6 / 32.8; 13000 x 9728 x 896 271 / 261, 512 27.1 / 25.0; 13000 x
-// 37888 x 3584 2907 / 2913, 2667 653 / 656; but 300 x 9728 x 896, which tiles of 128 take, 16.5 /
-// 20.8.  The activation has the pass's exact quotient and with it the pass's bits: with an
-// approximate reciprocal 46673 x 17920 took 2304, and two values in 100 000 were another one.  Bound
-// by the matrix cores as the product is; both stores go past the caches, nothing here reads them
-// again.
+// over operands that no cache holds: 46673 x 17920 x 1536 2450 / 2357, 13000 692 / 643, 2667 171 /
+// 163, 1000 77.9 / 76.2, 130 33.4 / 32.6; 13000 x 9728 x 896 266 / 240, 512 27.8 / 24.9; 13000 x
+// 22016 x 2048 1068 / 1046; deeper there is nothing in it, 13000 x 37888 x 3584 2850 / 2875, 2667
+// 638 / 638 (ops/lora.py glu_keeps); nor is there for 300 x 9728 x 896, which tiles of 128 take, 16.5
+// / 20.8.  The activation has the pass's exact quotient and with it the pass's bits: an approximate
+// reciprocal took 2290 of the 2357, and two values in 100 000 were other ones.  Bound by the matrix
+// cores as the product is; both stores go past the caches, nothing here reads them again.
 std::vector<torch::Tensor> lora_glu(torch::Tensor x, torch::Tensor w, torch::Tensor u,
                                     torch::Tensor b) {
   on_gpu({x, w, u, b});

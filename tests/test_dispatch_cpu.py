@@ -66,6 +66,16 @@ def test_adapter_products_of_one_round_by_one_rule():
     assert seen == {0, 64, 128} and one_round(4000, 64, 1536) == 64
 
 
+def test_activations_behind_an_adapter_s_product_by_rows_and_depth():
+    from nanorlhf_amd.ops.lora import glu_keeps
+    for M, N, K in [(129, 17920, 1536), (46673, 17920, 1536), (13000, 9728, 896), (700, 22016, 2048)]:
+        assert glu_keeps(M, N, K)
+    # another kernel's rows, blocks, tiles of 128, odd columns, and depths where a pass is as fast
+    for M, N, K in [(128, 37888, 1536), (212, 4096, 896), (300, 9728, 896), (13000, 17924, 1536),
+                    (13000, 37888, 3584), (2667, 17920, 2112)]:
+        assert not glu_keeps(M, N, K)
+
+
 def test_adapter_strategies_are_kept_by_what_the_kernels_depend_on(monkeypatch):
     from types import SimpleNamespace
     from nanorlhf_amd.ops import lora
