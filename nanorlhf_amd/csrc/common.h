@@ -119,57 +119,58 @@ DEVINL float act_gelu_tanh(float x) {
 }
 
 // ---- wave (64-lane) reductions ------------------------------------------
-DEVINL float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
+// All lanes get the result, exchanged between halves, rows of 16 and within a row by
+// the VALU itself: through LDS (__shfl_xor), which 16 waves of a workgroup share, an
+// exchange takes 107 cycles, a swap of rows 62 and a rotation in a row 27.  Pairs are
+// 32, 16, 8, 4, 2 and 1 lanes apart; from 8 on every row holds the same, so that a
+// rotation by 4 is that exchange too.
+template <int CTRL>
+DEVINL float row_move(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
-
-DEVINL float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-  return v;
+template <typename F>
+DEVINL float wave_reduce(float v, F f) {
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(h[0]), __uint_as_float(h[1]));
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  v = f(v, row_move<0x128>(v));     // row_ror:8
+  v = f(v, row_move<0x124>(v));     // row_ror:4
+  v = f(v, row_move<0x4e>(v));      // quad_perm:[2,3,0,1]
+  return f(v, row_move<0xb1>(v));   // quad_perm:[1,0,3,2]
 }
+DEVINL float wave_sum(float v) { return wave_reduce(v, [](float a, float b) { return a + b; }); }
+DEVINL float wave_max(float v) { return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); }); }
 
-// block reduction via LDS (block size multiple of 64)
+// block reduction via LDS (block size a multiple of 64, up to 1024): every thread reduces
+// the waves' results, in pairs of 8, 4, 2 and 1 waves apart.  1024 threads: 2700 cycles
+// with exchanges through LDS and the first wave reducing for all.
+template <int BLOCK, typename F>
+DEVINL float block_reduce(float v, float* lds_scratch /* BLOCK/64 floats */, F f) {
+  constexpr int W = BLOCK / 64;
+  static_assert((W & (W - 1)) == 0 && W <= 16, "a power of two of waves");
+  v = wave_reduce(v, f);
+  if constexpr (W == 1) return v;
+  if ((threadIdx.x & 63) == 0) lds_scratch[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float x[W];
+#pragma unroll
+  for (int w = 0; w < W; w++) x[w] = lds_scratch[w];
+#pragma unroll
+  for (int off = W / 2; off > 0; off >>= 1)
+#pragma unroll
+    for (int w = 0; w < off; w++) x[w] = f(x[w], x[w + off]);
+  __syncthreads();
+  return x[0];
+}
 template <int BLOCK>
-DEVINL float block_sum(float v, float* lds_scratch /* BLOCK/64 floats */) {
-  const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  v = wave_sum(v);
-  if (lane == 0) lds_scratch[wid] = v;
-  __syncthreads();
-  float out = 0.f;
-  if (wid == 0) {
-    float x = (lane < BLOCK / 64) ? lds_scratch[lane] : 0.f;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
-    out = x;
-    if (lane == 0) lds_scratch[0] = out;
-  }
-  __syncthreads();
-  out = lds_scratch[0];
-  __syncthreads();
-  return out;
+DEVINL float block_sum(float v, float* lds_scratch) {
+  return block_reduce<BLOCK>(v, lds_scratch, [](float a, float b) { return a + b; });
 }
-
 template <int BLOCK>
 DEVINL float block_max(float v, float* lds_scratch) {
-  const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
-  v = wave_max(v);
-  if (lane == 0) lds_scratch[wid] = v;
-  __syncthreads();
-  if (wid == 0) {
-    float x = (lane < BLOCK / 64) ? lds_scratch[lane] : -INFINITY;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x = fmaxf(x, __shfl_xor(x, off));
-    if (lane == 0) lds_scratch[0] = x;
-  }
-  __syncthreads();
-  float out = lds_scratch[0];
-  __syncthreads();
-  return out;
+  return block_reduce<BLOCK>(v, lds_scratch, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // ---- counter-based RNG (deterministic replay) ----------------------------
