@@ -10,8 +10,14 @@
 //      elements (counter-hash uniform: deterministic in (seed, step, row),
 //      replay-safe via a device-side step counter for hipGraphs).
 // Rows too long for the registers are read again for every pass.
+//
+// Few rows leave most CUs idle: sample_slices_kernel divides 1 and the sum of 2 among
+// workgroups, and sample_row_kernel goes on with the row's few likely elements, or, where
+// they are many, with a pass around the bin that a sample of the row names.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -418,6 +424,475 @@ void sample_topp_kernel(const LT* __restrict__ logits,
   }
 }
 
+// Every element once, by workgroups of 256 threads, 8 vectors a thread: `part` [B, slices],
+// a slice's largest logit and its sum of exp((l - that) / T), and `runs` [B, RBLOCK, RUN], the
+// vectors' largest elements, where a thread of the row's workgroup finds a run of RUN vectors
+// of one owner next to each other (half the owner's).  A slice without anything above -inf has a sum of 0, or a
+// not-a-number if it holds one.
+constexpr int RBLOCK = 512, RWAVES = RBLOCK / 64;
+constexpr int SLICE_VECS = 8, SLICE = OWNERS * SLICE_VECS;
+template <typename LT, int RUN>
+__global__ __launch_bounds__(OWNERS)
+void sample_slices_kernel(const LT* __restrict__ logits, float2* __restrict__ part,
+                          LT* __restrict__ runs, int V, float invT) {
+  static_assert(RUN % SLICE_VECS == 0, "a slice's vectors of an owner are of one run");
+  __shared__ float red[OWNERS / 64];
+  const long row = blockIdx.y;
+  const int nvec = V / 8, at = blockIdx.x * SLICE + threadIdx.x;
+  const LT* p = logits + row * (long)V;
+  Vec8<LT> c[SLICE_VECS];
+#pragma unroll
+  for (int k = 0; k < SLICE_VECS; k++)
+    load8(p + 8L * min(at + OWNERS * k, nvec - 1), c[k]);
+  // the last elements belong to the last slice
+  const int t = 8 * nvec + threadIdx.x;
+  const float tail = blockIdx.x == gridDim.x - 1 && t < V ? ldf(p + t) : -INFINITY;
+  float top = tail, m[SLICE_VECS];
+#pragma unroll
+  for (int k = 0; k < SLICE_VECS; k++) {
+    if (at + OWNERS * k >= nvec) fill8(c[k]);
+    float v[8];
+    get8(c[k], v);
+    m[k] = max8(v);
+    top = fmaxf(top, m[k]);
+  }
+  const int j = blockIdx.x * SLICE_VECS;
+  stv<SLICE_VECS>(runs + ((row * OWNERS + threadIdx.x) * 2 + j / RUN) * RUN + j % RUN, m);
+  top = block_max<OWNERS>(top, red);
+  const float M = top == -INFINITY ? 0.f : top * invT;
+  float sum = __expf(tail * invT - M);
+#pragma unroll
+  for (int k = 0; k < SLICE_VECS; k++) {
+    float v[8];
+    get8(c[k], v);
+#pragma unroll
+    for (int j = 0; j < 8; j++) sum += __expf(v[j] * invT - M);
+  }
+  sum = block_sum<OWNERS>(sum, red);
+  if (threadIdx.x == 0) part[row * gridDim.x + blockIdx.x] = float2{top, sum};
+}
+
+// inclusive sums over the lanes before
+template <typename T>
+DEVINL T lanes_before(T v) {
+  static_assert(sizeof(T) == 4, "");
+  auto shift = [&](auto ctrl) {
+    v += __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                           decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  shift(std::integral_constant<int, 0x111>{});    // row_shr:1, 2, 4, 8
+  shift(std::integral_constant<int, 0x112>{});
+  shift(std::integral_constant<int, 0x114>{});
+  shift(std::integral_constant<int, 0x118>{});
+  auto of = [&](int lane) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+  };
+  const T a = of(15), b = a + of(31), c = b + of(47);
+  const int r = (threadIdx.x & 63) >> 4;
+  return r == 0 ? v : v + (r == 1 ? a : r == 2 ? b : c);
+}
+template <typename T>
+DEVINL T of_lane(T v, int lane) {     // a lane that all agree on
+  return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+
+// The row's workgroup behind sample_slices_kernel, with the same bins, thresholds, categories
+// and order of them as sample_topp_kernel.  Bound by a chain of some 15 dependent steps where
+// the nucleus is small (8 rows of 151936: 11.2 us with the slices, of which each kernel's
+// start and first loads are half; one kernel 26.0), and else by reading, adding and writing
+// back the columns of the bins on one CU.
+constexpr int LIKELY = 4096;
+struct RowScratch {
+  union {
+    float hist[RWAVES][2 * BINS + 1][64];   // columns private to a lane, as Scratch's
+    struct {
+      float u[LIKELY];
+      int id[LIKELY];
+    } likely;
+  };
+  // Masses of bins in multiples of 2^-42: exact for an exp(u) of at least exp(-12), which has
+  // 24 bits, whatever the order; and integers are added up in LDS much faster than floats
+  // (67 and 3073 cycles for 16 waves; reading, adding and writing back takes 130).
+  unsigned long long exact[BINS];
+  float bin[2 * BINS], red[RWAVES];
+  int count[RWAVES];
+  int pick;
+};
+DEVINL unsigned long long exactly(float e) { return (unsigned long long)(e * 0x1p42f); }
+
+// Of 64 lanes' masses, from the top: the first lane at which `above` and they reach the target
+// (-1: none), and the mass above it.
+DEVINL int reach(float mass, float above, float target, float& before) {
+  const float incl = lanes_before(mass);
+  const unsigned long long hit = __ballot(above + incl >= target);
+  const int at = hit ? __ffsll(hit) - 1 : -1;
+  before = above + of_lane(incl - mass, max(at, 0));
+  return at;
+}
+// the sum over the lanes and waves ahead, for all threads, and that of all
+template <typename T>
+DEVINL T block_before(T v, T* scratch, T& total) {
+  const int wid = threadIdx.x >> 6;
+  const T incl = lanes_before(v);
+  if ((threadIdx.x & 63) == 63) scratch[wid] = incl;
+  __syncthreads();
+  T base{};
+  total = T{};
+#pragma unroll
+  for (int w = 0; w < RWAVES; w++) {
+    if (w < wid) base += scratch[w];
+    total += scratch[w];
+  }
+  __syncthreads();
+  return base + incl - v;
+}
+
+template <typename LT, int RUN>
+__global__ __launch_bounds__(RBLOCK)
+void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
+                       float* __restrict__ out_lp, int V, float invT, float top_p,
+                       unsigned long long seed, unsigned long long step_imm,
+                       const long* __restrict__ step_ptr, const float2* __restrict__ part,
+                       const LT* __restrict__ runs, int slices) {
+  __shared__ __attribute__((aligned(16))) RowScratch s;
+  const unsigned long long step = step_imm + (step_ptr ? (unsigned long long)*step_ptr : 0);
+  const long row = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nvec = V / 8;
+  const LT* p = logits + row * (long)V;
+  const float uniform = of_lane(hash_uniform(seed, step, (unsigned long long)row), 0);
+
+  // Two threads an owner, so that what they find has the order of the categories; the
+  // owner's element of the V % 8 last ones behind its vectors.
+  const int owner = tid >> 1, first = owner + OWNERS * RUN * (tid & 1);
+  const int t = (tid & 1) ? 8 * nvec + owner : V;
+  float most[RUN];
+#pragma unroll
+  for (int k = 0; k < RUN; k += 8) ldv<8>(runs + (row * RBLOCK + tid) * RUN + k, most + k);
+  const float tail = t < V ? ldf(p + t) : -INFINITY;
+  const float2 w = lane < slices ? part[row * slices + lane] : float2{-INFINITY, 0.f};
+  const float top = wave_max(w.x);
+  const float M = of_lane(top * invT, 0);
+  const float S = of_lane(wave_sum(w.x == top ? w.y : w.y * __expf(w.x * invT - M)), 0);
+  const float target = top_p * S;
+  const auto scaled = [&](float l) { return l * invT - M; };
+#pragma unroll
+  for (int k = 0; k < RUN; k++)       // past the row's end is whatever the memory held
+    most[k] = first + OWNERS * k < nvec ? scaled(most[k]) : -INFINITY;
+
+  // logprob of the chosen token under the temperature-scaled softmax
+  // (matches the scoring pass's logits/temperature quirk, grpo_trainer.py:547)
+  const auto put = [&](int pick) {
+    out[row] = pick;
+    if (out_lp) out_lp[row] = ldf(p + pick) * invT - (M + __logf(S));
+  };
+  // f(8 u, the first one's index) of this thread's vectors with one at `least` or above, and
+  // of the tail's element, with -inf behind it
+  const auto each = [&](float least, auto f) {
+    unsigned long long ones = 0;
+#pragma unroll
+    for (int k = 0; k < RUN; k++) ones |= (most[k] >= least ? 1ull : 0ull) << k;
+    while (__any(ones != 0)) {
+      constexpr int FEW = 4;           // loads in flight
+      Vec8<LT> c[FEW];
+      int at[FEW];
+#pragma unroll
+      for (int i = 0; i < FEW; i++) {
+        at[i] = ones ? first + OWNERS * (__ffsll(ones) - 1) : -1;
+        ones &= ones - 1;
+        fill8(c[i]);
+        if (at[i] >= 0) load8(p + 8L * at[i], c[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < FEW; i++) {
+        if (!__any(at[i] >= 0)) break;
+        float v[8];
+        get8(c[i], v);
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = scaled(v[j]);
+        f(v, 8 * at[i]);
+      }
+    }
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = j ? -INFINITY : scaled(tail);
+    if (__any(t < V)) f(v, t);
+  };
+
+  // ---- few likely elements ------------------------------------------------
+  // A language model's logits fall with the rank's logarithm: few are within some nats of
+  // the maximum and hold the nucleus, 8 at a temperature of 0.7 and 12 at 1.  `upper`: what
+  // is at `from` or above.
+  float from = 0.f, upper = 0.f;
+  bool few = S > 0.f;
+  for (float near = 8.f; few && near <= 12.f; near += 4.f) {
+    // rows of many are known by their vectors
+    int n = 0, total;
+#pragma unroll
+    for (int k = 0; k < RUN; k++) n += most[k] >= -near;
+    block_before(n, s.count, total);
+    if (total > LIKELY) break;
+    n = 0;
+    each(-near, [&](const float* u, int) {
+#pragma unroll
+      for (int j = 0; j < 8; j++) n += u[j] >= -near;
+    });
+    int at = block_before(n, s.count, total);
+    if (total > LIKELY) break;
+    each(-near, [&](const float* u, int i) {
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if (u[j] >= -near) {
+          s.likely.u[at] = u[j];
+          s.likely.id[at++] = i + j;
+        }
+    });
+    // the bin at which the mass reaches the target, and its refinements
+    float lo = -URANGE, width = 1.f, above = 0.f;
+    bool done = false;
+    for (int it = 0; it < 3 && !done; it++) {
+      if (tid < BINS) s.exact[tid] = 0;
+      __syncthreads();
+      const float scale = 1.f / width;
+      for (int i = tid; i < total; i += RBLOCK) {
+        const float u = s.likely.u[i];
+        if (it == 0 || (u >= lo && u < lo + BINS * width))
+          atomicAdd(&s.exact[max(0, min(BINS - 1, (int)((u - lo) * scale)))], exactly(__expf(u)));
+      }
+      __syncthreads();
+      const float mass = lane < BINS ? (float)s.exact[BINS - 1 - lane] * 0x1p-42f : 0.f;
+      __syncthreads();
+      float before;
+      const int hit = reach(mass, above, target, before);
+      const int at = hit < 0 || hit >= BINS ? BINS - 1 : hit;
+      if (it == 0 && !(hit >= 0 && lo + (float)(BINS - 1 - at) >= -near)) {
+        from = -near;
+        upper = wave_sum(lane < (int)near ? mass : 0.f);
+        lo = -INFINITY;
+        break;
+      }
+      above = hit < 0 ? above + wave_sum(lane < BINS - 1 ? mass : 0.f) : before;
+      lo += (float)(BINS - 1 - at) * width;
+      // over-keeping a sliver of the boundary bin changes the nucleus by < 2% of S
+      done = it > 0 && of_lane(mass, at) <= 0.02f * S;
+      width /= BINS;
+    }
+    if (lo == -INFINITY) continue;
+    const auto kept = [&](int i) {
+      const float u = s.likely.u[i];
+      return u >= lo ? __expf(u) : 0.f;
+    };
+    const int share = (total + RBLOCK - 1) / RBLOCK, i0 = min(tid * share, total);
+    const int i1 = min(i0 + share, total);
+    float own = 0.f, all;
+    for (int i = i0; i < i1; i++) own += kept(i);
+    if (tid == 0) s.pick = RBLOCK;
+    float sum = block_before(own, s.red, all);
+    const float goal = uniform * all;
+    // rounding may leave two at a border: the first
+    const bool mine = own > 0.f && goal >= sum && goal < sum + own;
+    if (mine) atomicMin(&s.pick, tid);
+    __syncthreads();
+    const int chosen = s.pick;
+    if (chosen == RBLOCK) break;        // rounding: none
+    if (tid == chosen) {
+      int pick = -1;
+      for (int i = i0; i < i1; i++) {
+        const float e = kept(i);
+        sum += e;
+        if (e > 0.f) {
+          pick = s.likely.id[i];
+          if (goal < sum) break;
+        }
+      }
+      put(pick);
+    }
+    return;
+  }
+
+  // ---- many: a pass over two bins at a time, which leaves every thread the mass of each of
+  // their refined bins (as hist's columns), and so its own kept mass -----------
+  const auto clear = [&](int bins) {
+    for (int i = tid; i < RWAVES * bins * 16; i += RBLOCK)
+      reinterpret_cast<f32x4*>(&s.hist[i / (bins * 16)][0][0])[i % (bins * 16)] = f32x4{};
+    __syncthreads();
+  };
+  const auto sum_bins = [&] {         // of all columns, 8 threads a bin
+    __syncthreads();
+    float x = 0.f;
+#pragma unroll
+    for (int w = 0; w < RWAVES; w++)
+#pragma unroll
+      for (int c = 0; c < 8; c++) x += s.hist[w][tid >> 3][8 * c + (tid & 7)];
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1) x += __shfl_xor(x, off);
+    if ((tid & 7) == 0) s.bin[tid >> 3] = x;
+    __syncthreads();
+  };
+  const auto columns = [&](int a, int b) {      // this lane's, of bins [a, b)
+    float x = 0.f;
+    for (int i = a; i < b; i++) x += s.hist[wid][i][lane];
+    return x;
+  };
+  float own = 0.f, lowest = -URANGE;
+  if (few) {       // S is a number
+    __syncthreads();
+    clear(BINS);
+    {
+      Vec8<LT> c;
+      float v[8];
+      load8(p + 8L * ((long)tid * nvec / RBLOCK), c);
+      get8(c, v);
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const float u = scaled(v[j]);
+        if (u < from || from == 0.f)
+          s.hist[wid][max(0, min(BINS - 1, (int)(u + URANGE)))][lane] += __expf(u);
+      }
+    }
+    sum_bins();
+    // bins from the top; what is left of S is divided as the sample is
+    const float some = lane < BINS ? s.bin[BINS - 1 - lane] : 0.f, rest = wave_sum(some);
+    const float mass = rest > 0.f ? some * ((S - upper) / rest) : 0.f;
+    float before;
+    const int at = reach(mass, upper, target, before);
+    const float in = of_lane(mass, max(at, 0));
+    float hi = at < 0 ? 2.f - URANGE : target - before < 0.5f * in ? 1.f - at : (float)-at;
+    hi = fmaxf(fminf(hi, 0.f), 2.f - URANGE);
+    float A, m1, m2;
+    for (int moved = 0;;) {
+      __syncthreads();
+      clear(2 * BINS);
+      const float bottom = hi - 2.f;
+      own = 0.f;
+      // In pairs, whose columns are read before either is written: half the reads' latency,
+      // which is what the pass takes.  Elements of neither bin go to one behind them.
+      each(bottom, [&](const float* u, int) {
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+          float e[2];
+          int k[2];
+#pragma unroll
+          for (int i = 0; i < 2; i++) {
+            e[i] = __expf(u[j + i]);
+            own += u[j + i] >= hi ? e[i] : 0.f;
+            k[i] = u[j + i] >= bottom && u[j + i] < hi ? (int)((u[j + i] - bottom) * BINS) : 2 * BINS;
+          }
+          if (!__any(min(k[0], k[1]) < 2 * BINS)) continue;
+          float *h0 = &s.hist[wid][k[0]][lane], *h1 = &s.hist[wid][k[1]][lane];
+          const float x = *h0 + e[0], y = *h1;
+          *h0 = x;
+          *h1 = (k[0] == k[1] ? x : y) + e[1];
+        }
+      });
+      sum_bins();
+      block_before(own, s.red, A);
+      m2 = wave_sum(lane < BINS ? s.bin[lane] : 0.f);
+      m1 = wave_sum(lane < BINS ? s.bin[BINS + lane] : 0.f);
+      if (A >= target && hi < 0.f && moved >= 0) {
+        hi = fminf(hi + 2.f, 0.f);
+        moved = 1;
+      } else if (A + (m1 + m2) < target && bottom > -URANGE && moved <= 0) {
+        hi = fmaxf(bottom, 2.f - URANGE);
+        moved = -1;
+      } else {
+        break;
+      }
+    }
+    const int b = A + m1 >= target ? BINS : 0;        // the upper of the two, or the lower
+    if (!b) own += columns(BINS, 2 * BINS);
+    lowest = hi - (b ? 1.f : 2.f);
+    // the maximum itself is of no refined bin
+    float above = lowest == -1.f ? 0.f : b ? A : A + m1;
+    const float x = lane < BINS ? s.bin[b + BINS - 1 - lane] : 0.f;
+    int fine = reach(x, above, target, before);
+    if (fine < 0 || fine >= BINS) {
+      fine = BINS - 1;
+      before = above + wave_sum(lane < fine ? x : 0.f);
+    }
+    above = before;
+    fine = BINS - 1 - fine;
+    lowest += fine * (1.f / BINS);
+    own += columns(b + fine + 1, b + BINS);
+    // over-keeping a sliver of the boundary bin changes the nucleus by < 2% of S
+    if (s.bin[b + fine] <= 0.02f * S) {
+      own += s.hist[wid][b + fine][lane];
+    } else {
+      __syncthreads();
+      clear(BINS);
+      const float lo = lowest;
+      each(lo, [&](const float* u, int) {
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          if (u[j] >= lo && u[j] < lo + 1.f / BINS)
+            s.hist[wid][(int)((u[j] - lo) * (BINS * BINS))][lane] += __expf(u[j]);
+      });
+      sum_bins();
+      const float y = lane < BINS ? s.bin[BINS - 1 - lane] : 0.f;
+      fine = reach(y, above, target, before);
+      fine = fine < 0 || fine >= BINS ? 0 : BINS - 1 - fine;
+      lowest += fine * (1.f / (BINS * BINS));
+      own += columns(fine, BINS);
+    }
+  } else {
+    each(lowest, [&](const float* u, int) {
+#pragma unroll
+      for (int j = 0; j < 8; j++) own += u[j] >= lowest ? __expf(u[j]) : 0.f;
+    });
+  }
+
+  // ---- scan and walk ---------------------------------------------------------
+  const auto kept = [&](float u) { return u >= lowest ? __expf(u) : 0.f; };
+  float all;
+  if (tid == 0) s.pick = RBLOCK;
+  const float sum = block_before(own, s.red, all), goal = uniform * all;
+  if (own > 0.f && goal >= sum && goal < sum + own) atomicMin(&s.pick, tid);
+  __syncthreads();
+  const int chosen = s.pick;
+  if (tid == chosen) s.bin[0] = sum;
+  __syncthreads();
+  if (tid == 0) s.pick = -1;
+  __syncthreads();
+  if (wid == 0 && chosen < RBLOCK) {
+    // its vectors in order, one per lane, and the tail's element in the last
+    static_assert(RUN < 64, "a run and one");
+    const int run = (chosen >> 1) + OWNERS * RUN * (chosen & 1);
+    const int i = run + OWNERS * lane, last = (chosen & 1) ? 8 * nvec + (chosen >> 1) : V;
+    Vec8<LT> c;
+    fill8(c);
+    if (lane < RUN && i < nvec) load8(p + 8L * i, c);
+    float e[8], m = 0.f;
+    get8(c, e);
+    if (lane == RUN && last < V) e[0] = ldf(p + last);
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      e[j] = kept(scaled(e[j]));
+      m += e[j];
+    }
+    const float base = s.bin[0] + lanes_before(m) - m;
+    const unsigned long long hit = __ballot(m > 0.f && goal < base + m);
+    const unsigned long long any = __ballot(m > 0.f);
+    // rounding may leave the goal behind all of them: the last
+    const int owner = hit ? __ffsll(hit) - 1 : any ? 63 - __clzll(any) : -1;
+    if (lane == owner) {
+      float at = base;
+      int pick = -1;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        if (e[j] > 0.f && !(pick >= 0 && goal < at)) pick = lane == RUN ? last : 8 * i + j;
+        at += e[j];
+      }
+      s.pick = pick;
+    }
+  }
+  __syncthreads();
+  int pick = s.pick;
+  if (pick < 0) {                     // nothing is above -inf
+    float best;
+    pick = row_argmax<RBLOCK>(p, V, best, s.red, s.count);
+  }
+  if (tid == 0) put(pick);
+}
+
 // Vectors per thread that are held in registers; 1024 threads have 128 each, so
 // 19 of bf16 (155648 logits) and 8 of float32 (65536) fit beside the rest.
 //
@@ -446,6 +921,45 @@ static void launch_sampler(const torch::Tensor& logits, torch::Tensor& out, floa
     if (half) { if (V <= 8192) GREEDY(short, 256); else GREEDY(short, 512); }
     else { if (V <= 8192) GREEDY(float, 256); else GREEDY(float, 512); }
 #undef GREEDY
+    HIP_CHECK_LAST();
+    return;
+  }
+  // A CU that has a row to itself takes the time of its VALU and LDS over the whole row: few
+  // rows are divided for the first half of it.  A nucleus of few elements, as a language
+  // model's, then is a few us; of rows that are flat (normal logits of deviation 1) every
+  // element has to be put into a bin all the same.  us, T = 0.7 and top-p 0.95, one kernel /
+  // divided, logits of a language model | flat:
+  //   bf16 of 151936   1 row 25.5 / 10.6 | 43.8 / 43.5    8 rows 26.0 / 11.2 | 44.4 / 44.0
+  //                    32    28.1 / 12.8 | 44.6 / 46.0    64     28.2 / 14.6 | 44.8 / 49.9
+  //                    128   30.7 / 19.8 | 48.0 / 54.7    512    70.6 / 52.4 | 107 / 125
+  //   bf16, 64 rows    128100 24.5 / 13.7 | 38.1 / 42.3   70000  24.3 / 12.6 | 30.5 / 40.1
+  //   32 bits, 152064  4     31.9 / 12.6 | 47.2 / 44.2    64     47.4 / 18.8 | 57.6 / 53.3
+  //                    512   175 / 91 | 171 / 172
+  // At T = 1, where the nucleus has a thousand elements, 8 rows 38.5 / 30.5, 64 39.3 / 37.5.
+  // A top-p of 1 has no bin to look for.
+  if (n > 12 && n <= 20 && B <= (half ? 64 : 512) && top_p < 1.) {
+    const int slices = (V / 8 + SLICE - 1) / SLICE;
+    const int run = n <= 16 ? 32 : 40;          // half of an owner's vectors, n * 4
+    const long ahead = (B * slices * 8 + 63) / 64 * 64;
+    auto work = torch::empty({ahead + B * RBLOCK * run * (half ? 2 : 4)},
+                             logits.options().dtype(torch::kByte));
+    auto* part = (float2*)work.data_ptr();
+    void* runs = (char*)work.data_ptr() + ahead;
+    const float invT = temperature > 0. ? 1.f / (float)temperature : 1.f;
+#define LAUNCH(LT, RUN)                                                                       \
+  do {                                                                                       \
+    hipLaunchKernelGGL((sample_slices_kernel<LT, RUN>), dim3(slices, B), dim3(OWNERS), 0,    \
+                       stream, (const LT*)logits.data_ptr(), part, (LT*)runs, V, invT);      \
+    hipLaunchKernelGGL((sample_row_kernel<LT, RUN>), dim3(B), dim3(RBLOCK), 0, stream,       \
+                       (const LT*)logits.data_ptr(), out.data_ptr<long>(), lp, V, invT,      \
+                       (float)top_p, (unsigned long long)seed, (unsigned long long)step,     \
+                       step_ptr, part, (const LT*)runs, slices);                             \
+  } while (0)
+    if (half && run == 32) LAUNCH(short, 32);
+    else if (half) LAUNCH(short, 40);
+    else if (run == 32) LAUNCH(float, 32);
+    else LAUNCH(float, 40);
+#undef LAUNCH
     HIP_CHECK_LAST();
     return;
   }
