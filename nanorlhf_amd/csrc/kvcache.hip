@@ -625,8 +625,11 @@ void paged_decode_kernel(const short* __restrict__ q,    // [B, Hq, D]
   }
 }
 
-// one wave per (sequence, kv head, head group, head): the splits' sums into out
-template <int DV, bool EXT>
+// One wave per (sequence, kv head, head group, head): the splits' sums into out.  A chain of
+// latencies: length, maxima, sums.  Up to MOST splits everything is asked for at once, whether
+// the sequence has that many or not (what it has not is whatever the memory held): 32 x 2000
+// tokens, 12 heads over 2, 17.4 us with the splits one after the other, 15.9.
+template <int DV, bool EXT, int MOST>
 __global__ __launch_bounds__(64)
 void paged_decode_merge_kernel(const float* __restrict__ part, const float* __restrict__ ms,
                                const int* __restrict__ seq_lens, short* __restrict__ out, int Hq,
@@ -635,27 +638,64 @@ void paged_decode_merge_kernel(const float* __restrict__ part, const float* __re
   const int unit = EXT ? x / ext.gchunks : x, gc = EXT ? x % ext.gchunks : 0;
   const int b = unit / Hkv, kvh = unit % Hkv;
   if (16 * gc + g >= Gq) return;
-  const int n = min((tile_range<EXT>(seq_lens[b], ext).n + per_split - 1) / per_split, splits);
-  if (n <= 1) return;
   const long row0 = (long)x * splits * 16 + g;
   const int lane = threadIdx.x;
-  float M = -INFINITY;
-  for (int k = lane; k < n; k += 64) M = fmaxf(M, ms[(row0 + 16L * k) * 2]);
-  M = wave_max(M);
-  if (M == -INFINITY) M = 0.f;
   constexpr int NP = DV > 128 ? 2 : 1;      // pairs per lane
   float S = 0.f, o[NP][2] = {};
-#pragma unroll 8
-  for (int k = 0; k < n; k++) {
-    const long row = row0 + 16L * k;
-    const float c = exp2f(ms[row * 2] - M);
-    S += ms[row * 2 + 1] * c;
+  if constexpr (MOST > 0) {
+    const int len = seq_lens[b];
+    float2 w[MOST], v[MOST][NP];
 #pragma unroll
-    for (int j = 0; j < NP; j++) {
-      const int d = 2 * (lane + 64 * j);
-      if (d < DV) {
-        o[j][0] += part[row * DV + d] * c;
-        o[j][1] += part[row * DV + d + 1] * c;
+    for (int k = 0; k < MOST; k++) {
+      const long row = row0 + 16L * min(k, splits - 1);
+      w[k] = *reinterpret_cast<const float2*>(ms + row * 2);
+#pragma unroll
+      for (int j = 0; j < NP; j++)
+        v[k][j] = *reinterpret_cast<const float2*>(part + row * DV + min(2 * (lane + 64 * j), DV - 2));
+    }
+    // (asked for before the first of them is needed)
+#pragma unroll
+    for (int k = 0; k < MOST; k++) {
+      asm volatile("" : "+v"(w[k].x), "+v"(w[k].y));
+#pragma unroll
+      for (int j = 0; j < NP; j++) asm volatile("" : "+v"(v[k][j].x), "+v"(v[k][j].y));
+    }
+    const int n = min((tile_range<EXT>(len, ext).n + per_split - 1) / per_split, splits);
+    if (n <= 1) return;
+    float M = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < MOST; k++) M = k < n ? fmaxf(M, w[k].x) : M;
+    if (M == -INFINITY) M = 0.f;
+#pragma unroll
+    for (int k = 0; k < MOST; k++) {
+      if (k >= n) break;
+      const float c = exp2f(w[k].x - M);
+      S += w[k].y * c;
+#pragma unroll
+      for (int j = 0; j < NP; j++) {
+        o[j][0] += v[k][j].x * c;
+        o[j][1] += v[k][j].y * c;
+      }
+    }
+  } else {
+    const int n = min((tile_range<EXT>(seq_lens[b], ext).n + per_split - 1) / per_split, splits);
+    if (n <= 1) return;
+    float M = -INFINITY;
+    for (int k = lane; k < n; k += 64) M = fmaxf(M, ms[(row0 + 16L * k) * 2]);
+    M = wave_max(M);
+    if (M == -INFINITY) M = 0.f;
+#pragma unroll 8
+    for (int k = 0; k < n; k++) {
+      const long row = row0 + 16L * k;
+      const float c = exp2f(ms[row * 2] - M);
+      S += ms[row * 2 + 1] * c;
+#pragma unroll
+      for (int j = 0; j < NP; j++) {
+        const int d = 2 * (lane + 64 * j);
+        if (d < DV) {
+          o[j][0] += part[row * DV + d] * c;
+          o[j][1] += part[row * DV + d + 1] * c;
+        }
       }
     }
   }
@@ -670,8 +710,8 @@ void paged_decode_merge_kernel(const float* __restrict__ part, const float* __re
 
 // How a batch of `units` workgroups with at most `tiles` tiles each is split:
 // until there is about one per CU, each with at least two tiles for every wave.  Four
-// per sequence read 32 x 2000 tokens (12 heads over 2, bf16) in 17.4 us with the
-// merge, two in 22.5, eight in 22.4 (the first tile's page, key and value
+// per sequence read 32 x 2000 tokens (12 heads over 2, bf16) in 15.9 us with the
+// merge, and, with a merge that took 1.5 more, 17.4, two in 22.5, eight in 22.4 (the first tile's page, key and value
 // latencies then outweigh the rest); unsplit it took 135.  At 256 sequences and
 // more nothing is split: 2048 x 850 in fp8 take 169 us, 5.3 TB/s.  Nor is a short
 // context, whose walk costs no more than the merge (in fp8: 64 x 170 tokens, 9
@@ -694,6 +734,20 @@ static Splits decode_splits(long units, long tiles, int DV, const torch::Tensor&
     s.ms = torch::empty({units * s.n * 16, 2L}, f32);
   }
   return s;
+}
+
+template <int DV, bool EXT>
+static void launch_merge(dim3 grid, const Splits& sp, const torch::Tensor& seq_lens,
+                         torch::Tensor& out, int Hq, int Hkv, int Gq, const DecodeExt& ext) {
+#define MERGE(MOST)                                                                          \
+  hipLaunchKernelGGL((paged_decode_merge_kernel<DV, EXT, MOST>), grid, dim3(64), 0,          \
+                     at::hip::getCurrentHIPStream(), sp.part.data_ptr<float>(),              \
+                     sp.ms.data_ptr<float>(), seq_lens.data_ptr<int>(), (short*)out.data_ptr(), \
+                     Hq, Hkv, Gq, sp.per, sp.n, ext)
+  if (sp.n <= 4) MERGE(4);
+  else if (sp.n <= 8) MERGE(8);
+  else MERGE(0);
+#undef MERGE
 }
 
 torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor k_cache,
@@ -729,9 +783,7 @@ torch::Tensor paged_attn_decode(torch::Tensor q, torch::Tensor k_cache,
                        seq_lens.data_ptr<int>(), (short*)out.data_ptr(), part, ms, \
                        Hq, Hkv, maxP, G, sp.per, sp.n, (float)scale, DecodeExt{}, NoToken{}); \
     if (sp.n > 1)                                                               \
-      hipLaunchKernelGGL((paged_decode_merge_kernel<DD, false>), dim3(B * Hkv, G), dim3(64), 0, \
-                         stream, part, ms, seq_lens.data_ptr<int>(), (short*)out.data_ptr(), \
-                         Hq, Hkv, G, sp.per, sp.n, DecodeExt{});                \
+      launch_merge<DD, false>(dim3(B * Hkv, G), sp, seq_lens, out, Hq, Hkv, G, DecodeExt{}); \
   } while (0)
   if (D == 128) { if (fp8) LAUNCH_D(128, unsigned char); else LAUNCH_D(128, short); }
   else if (D == 64) { if (fp8) LAUNCH_D(64, unsigned char); else LAUNCH_D(64, short); }
@@ -792,9 +844,7 @@ torch::Tensor paged_attn_decode_new(torch::Tensor qkv, torch::Tensor table, torc
                        seq_lens.data_ptr<int>(), (short*)out.data_ptr(), part, ms, (int)Hq,    \
                        (int)Hkv, maxP, G, sp.per, sp.n, (float)scale, DecodeExt{}, a);         \
     if (sp.n > 1)                                                                              \
-      hipLaunchKernelGGL((paged_decode_merge_kernel<DD, false>), dim3(B * Hkv, G), dim3(64), 0, \
-                         stream, part, ms, seq_lens.data_ptr<int>(), (short*)out.data_ptr(),   \
-                         (int)Hq, (int)Hkv, G, sp.per, sp.n, DecodeExt{});                     \
+      launch_merge<DD, false>(dim3(B * Hkv, G), sp, seq_lens, out, Hq, Hkv, G, DecodeExt{}); \
   } while (0)
   const bool fp8 = k_cache.scalar_type() == torch::kFloat8_e4m3fn;
   if (D == 128) { if (fp8) LAUNCH_N(128, unsigned char); else LAUNCH_N(128, short); }
@@ -852,9 +902,7 @@ void paged_attn_decode_window(torch::Tensor q, torch::Tensor k_cache, torch::Ten
                        seq_lens.data_ptr<int>(), (short*)out.data_ptr(), part, ms, Hq, Hkv, \
                        maxP, G, sp.per, sp.n, (float)scale, e, NoToken{});                 \
     if (sp.n > 1)                                                                          \
-      hipLaunchKernelGGL((paged_decode_merge_kernel<VV, true>), dim3(units, std::min(G, 16)), \
-                         dim3(64), 0, stream, part, ms, seq_lens.data_ptr<int>(),          \
-                         (short*)out.data_ptr(), Hq, Hkv, G, sp.per, sp.n, e);             \
+      launch_merge<VV, true>(dim3(units, std::min(G, 16)), sp, seq_lens, out, Hq, Hkv, G, e); \
   } while (0)
 #define LAUNCH_V(KK)                                                                       \
   do {                                                                                     \

@@ -270,35 +270,55 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
   }
 }
 
-// One workgroup per (16-row unit, row): the parts of a split context joined.
+// One workgroup per (16-row unit, row): the parts of a split context joined.  A chain of
+// latencies, so up to MOST parts are asked for at once with their shares.
+template <int MOST>
 __global__ __launch_bounds__(128) void latent_merge_kernel(LatentArgs a, int RP, int units_x) {
-  __shared__ float part_of[64];               // each split's share of the result
   const int unit = blockIdx.x, rr = blockIdx.y;
   const int seq = unit / units_x, r0 = unit % units_x * 16;
+  const int z = threadIdx.x & 63;
+  const float* ms = a.ms + ((long)unit * a.splits * 16 + rr) * 2;
+  const float* p = a.part + ((long)unit * a.splits * 16 + rr) * RP;
+  const float2 w = z < a.splits ? *reinterpret_cast<const float2*>(ms + z * 32)
+                                : float2{-INFINITY, 0.f};
+  f32x4 x[MOST ? MOST : 1];
+#pragma unroll
+  for (int i = 0; i < MOST; i++)
+    x[i] = *reinterpret_cast<const f32x4*>(p + (long)min(i, a.splits - 1) * 16 * RP +
+                                           min((int)threadIdx.x * 4, RP - 4));
+#pragma unroll
+  for (int i = 0; i < MOST; i++) asm volatile("" : "+v"(x[i]));
   const int t0 = a.cu ? a.cu[seq] : seq;
   const int nq = a.cu ? a.cu[seq + 1] - t0 : 1;
   if (r0 + rr >= nq * a.H) return;
-  const float* ms = a.ms + ((long)unit * a.splits * 16 + rr) * 2;
-  if (threadIdx.x < 64) {
-    const int z = threadIdx.x;
-    const bool ok = z < a.splits;
-    const float mz = ok ? ms[z * 32] : -INFINITY, sz = ok ? ms[z * 32 + 1] : 0.f;
-    const float f = exp2f(mz - wave_max(mz));
-    part_of[z] = f / wave_sum(sz * f);
-  }
-  __syncthreads();
-  const float* p = a.part + ((long)unit * a.splits * 16 + rr) * RP;
+  const float f = exp2f(w.x - wave_max(w.x));
+  float share = f / wave_sum(w.y * f);
+  asm volatile("" : "+v"(share));         // of every lane, those too that have no column below
+  auto of = [&](int i) {                  // part i's share of the result
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(share), i));
+  };
+  short* out = a.out + ((long)t0 * a.H + r0 + rr) * RP;
   for (int d = threadIdx.x * 4; d < RP; d += 512) {
     float o[4] = {};
-#pragma unroll 4
-    for (int z = 0; z < a.splits; z++) {
-      const float f = part_of[z];
-      float x[4];
-      ldv<4>(p + (long)z * 16 * RP + d, x);
+    if (MOST) {
 #pragma unroll
-      for (int j = 0; j < 4; j++) o[j] += f * x[j];
+      for (int i = 0; i < MOST; i++)
+        if (i < a.splits) {
+          const float g = of(i);
+#pragma unroll
+          for (int j = 0; j < 4; j++) o[j] += g * x[i][j];
+        }
+    } else {
+#pragma unroll 4
+      for (int i = 0; i < a.splits; i++) {
+        const float g = of(i);
+        float y[4];
+        ldv<4>(p + (long)i * 16 * RP + d, y);
+#pragma unroll
+        for (int j = 0; j < 4; j++) o[j] += g * y[j];
+      }
     }
-    stv<4>(a.out + ((long)t0 * a.H + r0 + rr) * RP + d, o);
+    stv<4>(out + d, o);
   }
 }
 
@@ -519,9 +539,12 @@ torch::Tensor latent_attn(torch::Tensor qa, torch::Tensor cache, c10::optional<t
   else if (RP == 512) LAUNCH(512);
   else TORCH_CHECK(false, "unsupported latent width ", RP);
 #undef LAUNCH
-  if (a.splits > 1)
-    hipLaunchKernelGGL(latent_merge_kernel, dim3(units, 16), dim3(128), 0, stream, a, (int)RP,
-                       (int)units_x);
+#define MERGE(MOST)                                                                           \
+  hipLaunchKernelGGL(latent_merge_kernel<MOST>, dim3(units, 16), dim3(128), 0, stream, a,     \
+                     (int)RP, (int)units_x)
+  if (a.splits > 4) MERGE(0);
+  else if (a.splits > 1) MERGE(4);
+#undef MERGE
   HIP_CHECK_LAST();
   return out;
 }
