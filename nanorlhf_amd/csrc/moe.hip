@@ -379,45 +379,84 @@ __global__ __launch_bounds__(WAVES * 64) void grouped_stream_kernel(Grouped a) {
 }
 
 // ---------------------------------------------------------------- routing
-// Top choices of one token's logits z[0..E) in LDS, by L neighbouring lanes; the
-// lower index wins a tie.  Not stored unless `store`.  top <= L.
+// The largest of L neighbouring lanes' values, in all of them: 8, 4, 2 and 1 lanes apart by
+// row_ror:8, row_ror:4 and two quad_perm
 template <int L>
-DEVINL void choose(const float* z, int E, int top, int* chosen, float* weight, bool store) {
+DEVINL float lanes_max(float v) {
+  if constexpr (L == 64) {
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
+  }
+  if constexpr (L >= 32) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  v = fmaxf(v, row_move<0x128>(v));
+  v = fmaxf(v, row_move<0x124>(v));
+  v = fmaxf(v, row_move<0x4e>(v));
+  return fmaxf(v, row_move<0xb1>(v));
+}
+
+// Top choices of one token's logits z[0..E) in LDS, by L neighbouring lanes; the
+// lower index wins a tie.  Not stored unless `store`.  top <= L.  With an expert a lane a
+// round is a maximum and a ballot: 16 tokens' 4 of 16 experts 600 cycles, 5000 with the
+// lanes' values and indexes exchanged through LDS.
+template <int L>
+DEVINL void choose(const float* z, int E, int top, int* chosen, float* weight, bool store,
+                   int* also = nullptr) {
   const int lane = threadIdx.x & (L - 1);
-  unsigned long long taken = 0;         // of this lane's experts lane, lane + 64, ..
   float first = 0.f, sum = 0.f, mine = 0.f;
   int pick = 0;
-  for (int i = 0; i < top; i++) {
-    float best = -INFINITY;
-    int at = 1 << 30;
-    for (int e = lane, q = 0; e < E; e += L, q++) {
-      const float x = z[e] == z[e] ? z[e] : -INFINITY;     // every lane must agree
-      if (!(taken >> q & 1) && (x > best || at == 1 << 30)) {
-        best = x;
-        at = e;
-      }
-    }
-#pragma unroll
-    for (int off = L / 2; off > 0; off >>= 1) {
-      const float b = __shfl_xor(best, off);
-      const int o = __shfl_xor(at, off);
-      if (o != 1 << 30 && (at == 1 << 30 || b > best || (b == best && o < at))) {
-        best = b;
-        at = o;
-      }
-    }
+  auto take = [&](int i, float best, int at) {
     if (i == 0) first = best;
     const float p = expf(best - first);
     sum += p;
-    if ((at & (L - 1)) == lane) taken |= 1ull << (at / L);
     if (lane == i) {
       mine = p;
       pick = at;
+    }
+  };
+  if (E <= L) {
+    const int group = threadIdx.x & 63 & ~(L - 1);      // its first lane
+    float v = lane < E ? z[lane] : -INFINITY;
+    v = v == v ? v : -INFINITY;                         // every lane must agree
+    bool left = lane < E;
+    for (int i = 0; i < top; i++) {
+      const float best = lanes_max<L>(left ? v : -INFINITY);
+      const unsigned long long all = __ballot(left && v == best) >> group;
+      const int at = __ffsll(L == 64 ? all : all & ((1ull << (L & 63)) - 1)) - 1;
+      left &= lane != at;
+      take(i, best, at);
+    }
+  } else {
+    unsigned long long taken = 0;         // of this lane's experts lane, lane + L, ..
+    for (int i = 0; i < top; i++) {
+      float best = -INFINITY;
+      int at = 1 << 30;
+      for (int e = lane, q = 0; e < E; e += L, q++) {
+        const float x = z[e] == z[e] ? z[e] : -INFINITY;
+        if (!(taken >> q & 1) && (x > best || at == 1 << 30)) {
+          best = x;
+          at = e;
+        }
+      }
+#pragma unroll
+      for (int off = L / 2; off > 0; off >>= 1) {
+        const float b = __shfl_xor(best, off);
+        const int o = __shfl_xor(at, off);
+        if (o != 1 << 30 && (at == 1 << 30 || b > best || (b == best && o < at))) {
+          best = b;
+          at = o;
+        }
+      }
+      if ((at & (L - 1)) == lane) taken |= 1ull << (at / L);
+      take(i, best, at);
     }
   }
   if (store && lane < top) {
     chosen[lane] = pick;
     weight[lane] = mine / sum;
+    if (also) also[lane] = pick;
   }
 }
 
@@ -438,6 +477,19 @@ __global__ __launch_bounds__(256) void route_plain_kernel(
   if (wid == 0) choose<64>(z, E, top, chosen + t * top, weight + t * top, true);
 }
 
+// the rows that chose expert e of n choices, in order, by one wave
+DEVINL void list_expert(const int* choices, int n, int e, int* list, int* count) {
+  const int lane = threadIdx.x & 63;
+  int total = 0;
+  for (int base = 0; base < n; base += 64) {
+    const bool mine = base + lane < n && choices[base + lane] == e;
+    const unsigned long long all = __ballot(mine);
+    if (mine) list[total + __popcll(all & ((1ull << lane) - 1))] = base + lane;
+    total += __popcll(all);
+  }
+  if (lane == 0) *count = total;
+}
+
 // 16 tokens per workgroup; the waves share the depth.  ET tiles of 16 experts.  A few tokens
 // are a chain of loads, so up to 16 experts those of AT steps are asked for at once.  The order
 // of the sums is the same for any number of tokens: on it hangs which expert a token at a near
@@ -445,11 +497,16 @@ __global__ __launch_bounds__(256) void route_plain_kernel(
 // them, 81.1 us with 4 steps as the compiler has them, 77.3 with 4, 77.0 with 12; 16 waves in
 // place of four, which add up in another order, 76.6.  4000 tokens and their lists 13.7 us
 // with any of these.  With more experts the compiler's 4 steps are 12 to 68 loads by themselves.
-template <int ET>
+// ALL: one workgroup has all tokens, and writes the experts' lists too, for which another
+// launch takes 4 us (1, 8 and 16 tokens' experts of 1536 x 2240 29.6 -> 25.9, 58.6 -> 54.6, 68.1
+// -> 64.9 us).  Not of more than 16 tokens, whose rows one CU would have to fetch: 32 tokens
+// 20500 cycles with the lists, 10300 without them where each 16 have a workgroup.
+template <int ET, bool ALL>
 __global__ __launch_bounds__(256) void route_mfma_kernel(
     const short* __restrict__ h, const short* __restrict__ wr, const short* __restrict__ bias,
-    int* __restrict__ chosen, float* __restrict__ weight, long T, int W, int E, int top) {
-  constexpr int AT = ET == 1 ? 12 : 1;
+    int* __restrict__ chosen, float* __restrict__ weight, int* __restrict__ lists,
+    int* __restrict__ counts, long T, int W, int E, int top) {
+  constexpr int AT = ET > 1 ? 1 : 12;
   __shared__ float z[4][16][ET * 16 + 1];
   const long t0 = blockIdx.x * 16L;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -490,8 +547,15 @@ __global__ __launch_bounds__(256) void route_mfma_kernel(
   }
   __syncthreads();
   constexpr int L = ET == 1 ? 16 : ET == 2 ? 32 : 64, AT_ONCE = 256 / L;
+  __shared__ int picks[ALL ? 16 * (ET > 4 ? 64 : ET * 16) : 1];      // [tokens, top]
   for (int t = threadIdx.x / L; t < 16; t += AT_ONCE)
-    choose<L>(z[0][t], E, top, chosen + (t0 + t) * top, weight + (t0 + t) * top, t0 + t < T);
+    choose<L>(z[0][t], E, top, chosen + (t0 + t) * top, weight + (t0 + t) * top, t0 + t < T,
+              ALL ? picks + t * top : nullptr);
+  if constexpr (ALL) {
+    __syncthreads();
+    for (int e = wid; e < E; e += 4)
+      list_expert(picks, (int)T * top, e, lists + (long)e * T, counts + e);
+  }
 }
 
 // One workgroup per expert: the rows that chose it, in order.  Four choices to a thread at a
@@ -710,11 +774,19 @@ std::vector<torch::Tensor> moe_route(torch::Tensor h, torch::Tensor router, torc
   auto counts = torch::empty({E}, ints);
   TORCH_CHECK(T > 0 && T * top < (1L << 31));
   auto stream = at::hip::getCurrentHIPStream();
-#define ROUTE(ET)                                                                            \
-  hipLaunchKernelGGL((route_mfma_kernel<ET>), dim3((T + 15) / 16), dim3(256), 0, stream,     \
-                     (const short*)h.data_ptr(), (const short*)router.data_ptr(),            \
-                     (const short*)bias.data_ptr(), chosen.data_ptr<int>(),                  \
-                     weight.data_ptr<float>(), T, (int)W, (int)E, (int)top)
+#define ROUTE_OF(ET, ALL)                                                                      \
+  hipLaunchKernelGGL((route_mfma_kernel<ET, ALL>), dim3((T + 15) / 16), dim3(256), 0, stream,  \
+                     (const short*)h.data_ptr(), (const short*)router.data_ptr(),              \
+                     (const short*)bias.data_ptr(), chosen.data_ptr<int>(),                    \
+                     weight.data_ptr<float>(), lists.data_ptr<int>(), counts.data_ptr<int>(),  \
+                     T, (int)W, (int)E, (int)top)
+#define ROUTE(ET)                      \
+  do {                                 \
+    listed = T <= 16;                  \
+    if (listed) ROUTE_OF(ET, true);    \
+    else ROUTE_OF(ET, false);          \
+  } while (0)
+  bool listed = false;
   if (is_bf16(h) && W % 8 == 0 && E <= 256 && (uintptr_t)h.data_ptr() % 16 == 0 &&
       (uintptr_t)router.data_ptr() % 16 == 0) {
     if (E <= 16) ROUTE(1);
@@ -733,8 +805,11 @@ std::vector<torch::Tensor> moe_route(torch::Tensor h, torch::Tensor router, torc
                        (const float*)bias.data_ptr(), chosen.data_ptr<int>(),
                        weight.data_ptr<float>(), (int)W, (int)E, (int)top);
 #undef ROUTE
-  hipLaunchKernelGGL(expert_lists_kernel, dim3(E), dim3(1024), 0, stream, chosen.data_ptr<int>(),
-                     lists.data_ptr<int>(), counts.data_ptr<int>(), T * top, (int)T);
+#undef ROUTE_OF
+  if (!listed)
+    hipLaunchKernelGGL(expert_lists_kernel, dim3(E), dim3(1024), 0, stream,
+                       chosen.data_ptr<int>(), lists.data_ptr<int>(), counts.data_ptr<int>(),
+                       T * top, (int)T);
   HIP_CHECK_LAST();
   return {chosen, weight, lists, counts};
 }
