@@ -11,9 +11,17 @@
 // in one lane pair: online softmax without LDS, weights converted to bf16 in
 // place, O^T = V^T P^T.  V pages are d-major, so a V^T fragment (8 tokens of one
 // d) is 16 bytes; the keys are read in the order that leaves a lane the scores
-// of those 8.  Bound by LDS reads, matrix products and exponentials together.
-// 4000 tokens after 0, 4000 and 8000, 12 heads of 128: 160 us each (920 TFLOP/s);
-// with tiles through registers and every head on every chiplet 309.
+// of those 8.
+//
+// What bounds it: of the portions that fill the chip once, a wave's instructions.  A wave
+// alone on its SIMD issues one in 5 cycles, whichever unit it is for, so the matrix products
+// of a tile (32, 1024 cycles) are hidden only if what else it takes (some 450 instructions)
+// lies between them: a tile's scores are computed under the exponentials of the tile before,
+// an LDS read and six VALU instructions to a product, which leaves 2750 cycles of 3330 a tile.
+// Of more workgroups, products, VALU and LDS reads (as many cycles as the products) together.
+// 12 heads of 128, one tile after the other / now, us: 128 rows over 8064 keys 175 / 145;
+// 2048 tokens, 8 times 180 / 166 over a workspace, over pages of 2 heads 178 / 162; 16384
+// 1069 / 941 and 873 / 817; a window of 1024 over 8 of 693 to 3380 137 / 130.
 //
 // The same kernel runs over a workspace (LIN) instead of pages: keys [rows, Hkv,
 // DK] and transposed values [Hkv * DV, rows] of whole contexts laid out one
@@ -62,23 +70,54 @@ DEVINL int row_swz(int row) {
 }
 DEVINL int half_swz(int d) { return (d >> 3) & 1; }
 
+#define INLINE __attribute__((always_inline))
+
+DEVINL float other_half(float x, int hi) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(hi ? r[0] : r[1]);
+}
+
 template <int DK, int DV, bool LIN>
 __global__ __launch_bounds__(256, (DK > 128 || DV > 128) ? 1 : 2)
 void paged_varlen_kernel(VarlenArgs a) {
   constexpr int NDS = DK / 16, NDT = DV / 32, KV = 64;
   constexpr float THR = 11.54f;                // defer-max threshold (log2 units)
+  constexpr bool PAIRS = DK <= 128 && DV <= 128;   // two workgroups fit a CU
   int seq, kvh, tile;
   {
     // From 8 kv heads on, a chiplet takes whole heads, whose keys then stay in its
     // L2, long and short rows in turn; else the longest rows first.
-    int id = blockIdx.x;
     const int n = gridDim.x;
+    int id = blockIdx.x;
     if (a.Hkv >= 8) {
-      const int q = n >> 3, r = n & 7, xcd = id & 7;
-      id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (id >> 3);
+      const int q = n >> 3, r = n & 7, xcd = id & 7, mine = id >> 3, all = q + (xcd < r);
+      const int first = xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q;
+      if (PAIRS && a.B == 1 && n > 256 && n <= 512 && a.size >= a.seq_lens[0]) {
+        // One sequence without a window, whose workgroups are more than the CUs, but at most
+        // twice as many: some CUs run two, which are the first that a chiplet is given and
+        // those after its 32nd.  These are the shortest rows, two neighbours in length each;
+        // the longest, alone, come first among the others.  2708 rows of 12 heads after 0, 2708
+        // and 5416 (264 workgroups): 60, 115 and 165 us; long and short in turn 65, 134 and 195.
+        const int over = max(all - 32, 0);
+        int rank = mine < over ? 2 * mine + 1
+                   : mine >= 32 ? 2 * (mine - 32) : 2 * over + (all - over - 1 - mine);
+        for (tile = 0;; tile++) {    // the rank'th shortest: a tile's heads are `tiles` ids apart
+          const int off = (tile - first % a.tiles + a.tiles) % a.tiles;
+          const int same = all / a.tiles + (off < all % a.tiles);
+          if (rank < same) {
+            id = first + off + rank * a.tiles;
+            break;
+          }
+          rank -= same;
+        }
+      } else {
+        id = first + mine;
+        const int t = id % a.tiles;
+        tile = t & 1 ? t >> 1 : a.tiles - 1 - (t >> 1);
+      }
+    } else {
+      tile = a.tiles - 1 - id % a.tiles;
     }
-    const int t = id % a.tiles;
-    tile = a.Hkv >= 8 && (t & 1) ? t >> 1 : a.tiles - 1 - (a.Hkv >= 8 ? t >> 1 : t);
     seq = id / a.tiles % a.B;
     kvh = id / a.tiles / a.B;
   }
@@ -98,7 +137,7 @@ void paged_varlen_kernel(VarlenArgs a) {
   const int tok = row / G, head = kvh * G + row % G;
   const int qpos = start + tok;
 
-  __shared__ __attribute__((aligned(16))) short Ks[2][KV * DK], Vs[2][KV * DV];
+  __shared__ __attribute__((aligned(512))) short Ks[2][KV * DK], Vs[2][KV * DV];
 
   bf16x8p qf[NDS];
   {
@@ -128,31 +167,57 @@ void paged_varlen_kernel(VarlenArgs a) {
   const int last_page = (L - 1) >> 4;
   auto tile_of = [&](int it) { return it < kept_tiles ? it : it - kept_tiles + win_tile; };
 
-  // A wave's 64 chunks of one load are rows of one page (or 8 rows of V^T).
+  // A wave's 64 chunks of one load are rows of one page (or 8 rows of V^T).  What does not
+  // change from tile to tile is prepared, for a wave alone on its SIMD waits for every
+  // scalar instruction; pages are looked up a step before they are needed.
+  constexpr int NK = KV * DK / 8 / 256, NV = KV * DV / 8 / 256, PER = 64 / (DK / 8);
   const int ldk = a.Hkv * DK;
-  auto stage = [&](int tile, int buf) {
+  const short* kw = a.kc + kvh * DK + (LIN ? (lin0 + wid * PER) * ldk : (long)(wid * PER % 16) * ldk);
+  const short* vw = LIN ? a.vc + ((long)kvh * DV + wid * 8) * a.ldv + lin0
+                        : a.vc + ((long)kvh * DV + wid * 32 % DV) * 16;
+  auto key_page = [&](int tile, int i) INLINE {
+    return btb[min(tile * 4 + ((i * 256 / (DK / 8) + wid * PER) >> 4), last_page)];
+  };
+  auto value_page = [&](int tile, int i) INLINE {
+    return btb[min(tile * 4 + (i * 128 + wid * 32) / DV, last_page)];
+  };
+  int kpage[NK], vpage[NV];             // of the tiles that are asked for next
+  auto key_pages = [&](int tile) INLINE {
+    if constexpr (!LIN)
 #pragma unroll
-    for (int i = 0; i < KV * DK / 8; i += 256) {
-      constexpr int PER = 64 / (DK / 8);                      // tokens of one load
-      const int row0 = i / (DK / 8) + wid * PER, r = row0 + lane / (DK / 8);
+      for (int i = 0; i < NK; i++) kpage[i] = key_page(tile, i);
+  };
+  auto value_pages = [&](int tile) INLINE {
+    if constexpr (!LIN)
+#pragma unroll
+      for (int i = 0; i < NV; i++) vpage[i] = value_page(tile, i);
+  };
+  auto stage_keys = [&](int tile, int buf) INLINE {
+    const short* at = kw + (LIN ? (long)tile * KV * ldk : 0);
+#pragma unroll
+    for (int i = 0; i < NK; i++) {
+      const int row0 = i * 256 / (DK / 8) + wid * PER, r = row0 + lane / (DK / 8);
       const int c = (lane % (DK / 8)) ^ row_swz<DK>(r);
-      const long at = LIN ? lin0 + tile * KV + row0
-                          : (long)btb[min(tile * 4 + (row0 >> 4), last_page)] * 16 + (row0 & 15);
-      load_to_lds16(a.kc + at * ldk + kvh * DK, (unsigned)((r - row0) * ldk + c * 8) * 2,
-                    &Ks[buf][(i + wid * 64) * 8]);
+      const long off = LIN ? (long)(i * 256 / (DK / 8)) * ldk
+                           : ((long)kpage[i] * 16 + i * 256 / (DK / 8) % 16) * ldk;
+      load_to_lds16(at + off, (unsigned)((r - row0) * ldk + c * 8) * 2,
+                    &Ks[buf][(i * 256 + wid * 64) * 8]);
     }
+  };
+  auto stage_values = [&](int tile, int buf) INLINE {
 #pragma unroll
-    for (int i = 0; i < KV * DV / 8; i += 256) {
+    for (int i = 0; i < NV; i++) {
       if constexpr (LIN) {
-        const int d0 = i / 8 + wid * 8, d = d0 + (lane >> 3);
-        const int c = (lane & 7) ^ row_swz<64>(d);
-        load_to_lds16(a.vc + ((long)kvh * DV + d0) * a.ldv + lin0 + tile * KV,
-                      (unsigned)((lane >> 3) * a.ldv + c * 8) * 2, &Vs[buf][(i + wid * 64) * 8]);
+        const int d = wid * 8 + (lane >> 3), c = (lane & 7) ^ row_swz<64>(d);
+        load_to_lds16(vw + tile * KV + (long)(i * 32) * a.ldv,
+                      (unsigned)((lane >> 3) * a.ldv + c * 8) * 2,
+                      &Vs[buf][(i * 256 + wid * 64) * 8]);
       } else {
-        const int d0 = (i / 2 + wid * 32) % DV, pg = (i / 2 + wid * 32) / DV;
+        const int d0 = (i * 128 + wid * 32) % DV;
         const int d = d0 + (lane >> 1), c = (lane & 1) ^ half_swz(d);
-        load_to_lds16(a.vc + ((long)btb[min(tile * 4 + pg, last_page)] * a.Hkv + kvh) * DV * 16,
-                      (unsigned)(d * 16 + c * 8) * 2, &Vs[buf][(i + wid * 64) * 8]);
+        load_to_lds16(vw + ((long)vpage[i] * a.Hkv * DV + (d0 - wid * 32 % DV)) * 16,
+                      (unsigned)((lane >> 1) * 16 + c * 8) * 2,
+                      &Vs[buf][(i * 256 + wid * 64) * 8]);
       }
     }
   };
@@ -160,65 +225,51 @@ void paged_varlen_kernel(VarlenArgs a) {
   // leaves lane half `hi` with keys 16 ks + 8 hi + (0 .. 7) in registers 8 ks + ..
   const int krow = (col & 19) | (col & 4) << 1 | (col & 8) >> 1;
 
+  // scores meet scale * log2(e) in the exponent's fma, which needs a positive scale
+  const float sl2 = a.scale * 1.4426950408889634f;
+  const float mul = sl2 > 0.f ? sl2 : 1.f;
+  // does any of this wave's rows see any of the tile?
+  auto visible = [&](int kv0) {
+    return wave_active && kv0 <= wpos_hi &&
+           !(wpos_lo - (kv0 + KV - 1) >= a.size && kv0 >= a.keep);
+  };
+  // A fragment's address is that of its tile's first, which two registers keep, with a
+  // constant exchanged (xor) into the chunk and another added.
+  typedef __attribute__((address_space(3))) const char* lds_bytes;
+  typedef __attribute__((address_space(3))) const bf16x8p* lds_frag;
+  const unsigned k0 = lds_address(&Ks[0][0]) + krow * 2 * DK + ((hi ^ row_swz<DK>(krow)) << 4);
+  const unsigned v0 = lds_address(&Vs[0][0]) +
+                      (LIN ? col * 128 + ((hi ^ row_swz<64>(col)) << 4)
+                           : col * 32 + ((hi ^ half_swz(col)) << 4));
+  constexpr int AHEAD = 2;              // of a product's fragments, read before it starts
+  auto key_frag = [&](unsigned at, int buf, int i) INLINE {
+    return *(lds_frag)((lds_bytes)(at ^ (i >> 1) << 5) + (buf * KV + (i & 1) * 32) * 2 * DK);
+  };
+  auto first_keys = [&](int buf, bf16x8p* f) INLINE {
+    unsigned at = k0;
+    asm volatile("" : "+v"(at));
 #pragma unroll
-  for (int ds = 0; ds < NDS; ds++) asm volatile("" : "+v"(qf[ds]));   // arrived
-  stage(tile_of(0), 0);
-  for (int it = 0; it < ntiles; it++) {
-    const int buf = it & 1, kv0 = tile_of(it) * KV;
-    wait_loads<0>();
-    __syncthreads();          // the tile has arrived, the other buffer is free
-    if (it + 1 < ntiles) stage(tile_of(it + 1), buf ^ 1);
-    // whole tile invisible to this wave?
-    if (!wave_active || kv0 > wpos_hi ||
-        (wpos_lo - (kv0 + KV - 1) >= a.size && kv0 >= a.keep))
-      continue;
-
-    f32x16 st[2];
+    for (int i = 0; i < 2 * AHEAD; i++) f[i] = key_frag(at, buf, i);
+  };
+  auto scores = [&](int buf, f32x16* st, const bf16x8p* first) INLINE {
+    unsigned at = k0;
+    asm volatile("" : "+v"(at));      // the others made anew each time, or they fill registers
+    st[0] = st[1] = f32x16{};
 #pragma unroll
-    for (int sub = 0; sub < 2; sub++) {
-      st[sub] = f32x16{};
-      const int r = sub * 32 + krow;
+    for (int i = 0; i < 2 * NDS; i++)
+      st[i & 1] = mfma32p(i < 2 * AHEAD ? first[i] : key_frag(at, buf, i), qf[i >> 1], st[i & 1]);
+  };
+  auto top_of = [&](const f32x16* st) INLINE {
+    float top = st[0][0];
 #pragma unroll
-      for (int ds = 0; ds < NDS; ds++) {
-        const bf16x8p kf = *reinterpret_cast<const bf16x8p*>(
-            &Ks[buf][r * DK + (((2 * ds + hi) ^ row_swz<DK>(r)) << 3)]);
-        st[sub] = mfma32p(kf, qf[ds], st[sub]);
-      }
-    }
-    // scores meet scale * log2(e) in the exponent's fma, which needs a positive scale
-    const float sl2 = a.scale * 1.4426950408889634f;
-    float mul = sl2;
-    if (!(sl2 > 0.f)) {
-#pragma unroll
-      for (int i = 0; i < 32; i++) st[i >> 4][i & 15] *= sl2;
-      mul = 1.f;
-    }
-    const bool full = kv0 + KV - 1 <= wpos_lo &&
-                      (wpos_hi - kv0 < a.size || kv0 + KV <= a.keep);
-    if (!full) {
-#pragma unroll
-      for (int i = 0; i < 32; i++) {
-        const int ki = kv0 + 16 * (i >> 3) + 8 * hi + (i & 7);
-        if (!(ki <= qpos && (qpos - ki < a.size || ki < a.keep))) st[i >> 4][i & 15] = -INFINITY;
-      }
-    }
-    float pmax = st[0][0];
-#pragma unroll
-    for (int i = 1; i < 32; i++) pmax = fmaxf(pmax, st[i >> 4][i & 15]);
-    pmax = fmaxf(pmax, __shfl_xor(pmax, 32)) * mul;
-    float alpha = 1.f;
-    if (__any(!(pmax - m <= THR))) {           // also true while m is -inf
-      const float mn = fmaxf(m, pmax);
-      alpha = (m == -INFINITY) ? 0.f : exp2f(m - mn);
-      m = mn;
-#pragma unroll
-      for (int t = 0; t < NDT; t++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[t][r] *= alpha;
-    }
+    for (int i = 1; i < 32; i++) top = fmaxf(top, st[i >> 4][i & 15]);
+    return top;
+  };
+  auto weigh = [&](int buf, const f32x16* st, float alpha) INLINE {
     const float mm = m == -INFINITY ? 0.f : m;  // a row that sees nothing so far
     float rs = 0.f;
-    bf16x8p pf[4];
+    unsigned at = v0;
+    asm volatile("" : "+v"(at));
 #pragma unroll
     for (int ks = 0; ks < 4; ks++) {
       union { unsigned u[4]; bf16x8p f; } fr;
@@ -233,19 +284,141 @@ void paged_varlen_kernel(VarlenArgs a) {
         if constexpr (LIN) rs += __uint_as_float(fr.u[j] << 16) + __uint_as_float(fr.u[j] & 0xffff0000u);
         else rs += x + y;
       }
-      pf[ks] = fr.f;
+#pragma unroll
+      for (int t = 0; t < NDT; t++)
+        acc[t] = mfma32p(LIN ? *(lds_frag)((lds_bytes)(at ^ ks << 5) + (buf * DV + t * 32) * 128)
+                             : *(lds_frag)((lds_bytes)at + ((buf * 4 + ks) * DV + t * 32) * 32),
+                         fr.f, acc[t]);
     }
-    rs += __shfl_xor(rs, 32);
-    sum = sum * alpha + rs;
+    sum = sum * alpha + (rs + other_half(rs, hi));
+  };
+
+  // V(it) and K(it + 1) have arrived, K(it) and V(it - 1) are read: the next two are asked for
+  auto arrive = [&](int it, int buf, bf16x8p* first) INLINE {
+    wait_loads<0>();
+    __syncthreads();
+    first_keys(buf ^ 1, first);
+    if (it + 2 < ntiles) stage_keys(tile_of(it + 2), buf);
+    if (it + 1 < ntiles) stage_values(tile_of(it + 1), buf ^ 1);
+    key_pages(tile_of(it + 3));
+    value_pages(tile_of(it + 2));
+  };
+  // mask and maximum of a tile's scores, of which `top` is a lane's largest; rescales if needed
+  auto settle = [&](int kv0, f32x16* st, float top) INLINE {
+    if (!(sl2 > 0.f)) {
 #pragma unroll
-    for (int ks = 0; ks < 4; ks++)
+      for (int i = 0; i < 32; i++) st[i >> 4][i & 15] *= sl2;
+      top = top_of(st);
+    }
+    const bool full = kv0 + KV - 1 <= wpos_lo &&
+                      (wpos_hi - kv0 < a.size || kv0 + KV <= a.keep);
+    if (!full) {
+      int see = qpos - kv0 - 8 * hi;                      // counted from the lane's first key
+      int kept = a.keep - kv0 - 8 * hi;
+      asm volatile("" : "+v"(see), "+v"(kept));
 #pragma unroll
-      for (int t = 0; t < NDT; t++) {
-        const int d = t * 32 + col;
-        const short* v = LIN ? &Vs[buf][d * 64 + (((2 * ks + hi) ^ row_swz<64>(d)) << 3)]
-                             : &Vs[buf][(ks * DV + d) * 16 + ((hi ^ half_swz(d)) << 3)];
-        acc[t] = mfma32p(*reinterpret_cast<const bf16x8p*>(v), pf[ks], acc[t]);
+      for (int i = 0; i < 32; i++) {
+        const int ki = 16 * (i >> 3) + (i & 7);
+        if (!(ki <= see && (see - ki < a.size || ki < kept))) st[i >> 4][i & 15] = -INFINITY;
       }
+      top = top_of(st);
+    }
+    const float pmax = fmaxf(top, other_half(top, hi)) * mul;
+    float alpha = 1.f;
+    if (__any(!(pmax - m <= THR))) {           // also true while m is -inf
+      const float mn = fmaxf(m, pmax);
+      alpha = (m == -INFINITY) ? 0.f : exp2f(m - mn);
+      m = mn;
+#pragma unroll
+      for (int t = 0; t < NDT; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[t][r] *= alpha;
+    }
+    return alpha;
+  };
+  // one tile, the next one's scores under its exponentials
+  auto both = [&](int it, int buf, f32x16* cur, float top, f32x16* next, float& ntop) INLINE {
+    bf16x8p first[2 * AHEAD];
+    arrive(it, buf, first);
+    const float alpha = settle(tile_of(it) * KV, cur, top);
+    __builtin_amdgcn_sched_barrier(0);
+    scores(buf ^ 1, next, first);
+    weigh(buf, cur, alpha);
+    ntop = top_of(next);
+    asm volatile("" : "+v"(ntop));
+    // a product, six VALU instructions and the read of the product after the next, in turn
+    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+    for (int i = 0; i < 2 * NDS + 4 * NDT; i++) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x402, 6, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  f32x16 s0[2], s1[2];
+  float top0 = 0.f, top1 = 0.f;
+  auto one = [&](int it, int buf) INLINE {
+    bf16x8p first[2 * AHEAD];
+    arrive(it, buf, first);
+    const int kv0 = tile_of(it) * KV;
+    if (visible(kv0)) weigh(buf, s0, settle(kv0, s0, top0));
+    if (it + 1 < ntiles && visible(tile_of(it + 1) * KV)) {
+      scores(buf ^ 1, s0, first);
+      top0 = top_of(s0);
+    }
+  };
+
+#pragma unroll
+  for (int ds = 0; ds < NDS; ds++) asm volatile("" : "+v"(qf[ds]));   // arrived
+  key_pages(tile_of(0));
+  value_pages(tile_of(0));
+  stage_keys(tile_of(0), 0);
+  if constexpr (PAIRS) {
+    key_pages(tile_of(1));
+    wait_loads<0>();
+    __syncthreads();
+    if (ntiles > 1) stage_keys(tile_of(1), 1);
+    stage_values(tile_of(0), 0);
+    key_pages(tile_of(2));
+    value_pages(tile_of(1));
+    if (visible(tile_of(0) * KV)) {
+      bf16x8p first[2 * AHEAD];
+      first_keys(0, first);
+      scores(0, s0, first);
+      top0 = top_of(s0);
+    }
+    for (int it = 0; it < ntiles; it += 2) {
+      // (a loop of its own, or the scores change registers in every round)
+      for (; it + 2 < ntiles && visible(tile_of(it) * KV) && visible(tile_of(it + 1) * KV) &&
+             visible(tile_of(it + 2) * KV); it += 2) {
+        both(it, 0, s0, top0, s1, top1);
+        both(it + 1, 1, s1, top1, s0, top0);
+      }
+      one(it, 0);
+      if (it + 1 < ntiles) one(it + 1, 1);
+    }
+  } else {
+    // Wider rows leave no registers for two tiles' scores: these would pass through the
+    // accumulation registers (1500 rows of 8 heads over 1 of 256 100 us, this way 85).
+    stage_values(tile_of(0), 0);
+    for (int it = 0; it < ntiles; it++) {
+      const int buf = it & 1, kv0 = tile_of(it) * KV;
+      wait_loads<0>();
+      __syncthreads();
+      if (it + 1 < ntiles) {
+        key_pages(tile_of(it + 1));
+        value_pages(tile_of(it + 1));
+        stage_keys(tile_of(it + 1), buf ^ 1);
+        stage_values(tile_of(it + 1), buf ^ 1);
+      }
+      if (!visible(kv0)) continue;
+      bf16x8p first[2 * AHEAD];
+      f32x16 st[2];
+      first_keys(buf, first);
+      scores(buf, st, first);
+      weigh(buf, st, settle(kv0, st, top_of(st)));
+    }
   }
 
   if (!wave_active || !row_ok) return;
