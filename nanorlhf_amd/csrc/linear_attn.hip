@@ -9,6 +9,8 @@
 //                   sequence's slot (or zero) and back into it;
 //   3. chunk_out:   decayed (q k^T) v inside a chunk plus q times the state
 //                   ahead of it, in parallel.
+// bf16 rows that can be read four elements at a time, of heads up to 128 wide, run the same by
+// segments of several chunks (below).
 // Products run on the matrix cores.  float32 inputs use float32 MFMA.  bf16
 // inputs use bf16 MFMA on split operands: whatever is 32-bit (rotated and
 // decayed q and k, decayed scores, the state) is the sum of two bf16 numbers,
@@ -19,6 +21,8 @@
 // (sequence, head) streams S once through registers.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
+
+#include <algorithm>
 
 #include "common.h"
 #include "checks.h"
@@ -236,6 +240,37 @@ __global__ __launch_bounds__(256) void chunk_out_kernel(
 // ===================================================== bf16: split operands
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
+// SiLU and rotation of two runs that hold whole pairs
+DEVINL void shape_runs(float* a, float* b, const Source& s, bool rot, const float* c,
+                       const float* sn) {
+  if (s.silu) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      a[j] = silu_fast(a[j]);
+      b[j] = silu_fast(b[j]);
+    }
+  }
+  if (!rot) return;
+  if (s.interleaved) {
+#pragma unroll
+    for (int j = 0; j < 4; j += 2) {
+      const float u = a[j], v = a[j + 1];
+      a[j] = u * c[j / 2] - v * sn[j / 2];
+      a[j + 1] = v * c[j / 2] + u * sn[j / 2];
+      const float x = b[j], y = b[j + 1];
+      b[j] = x * c[2 + j / 2] - y * sn[2 + j / 2];
+      b[j + 1] = y * c[2 + j / 2] + x * sn[2 + j / 2];
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float u = a[j], v = b[j];
+      a[j] = u * c[j] - v * sn[j];
+      b[j] = v * c[j] + u * sn[j];
+    }
+  }
+}
+
 // Eight elements of one q or k row, as two runs of four: a at element ea, b at
 // eb.  Run g holds whole rotation pairs (with `vec`; without it, elements 8g..
 // 8g+7 one by one).  Elements past D are 0.
@@ -264,35 +299,12 @@ DEVINL void load_runs(const short* row, int g, const Source& s, const float* cs,
   for (int j = 0; j < 4; j++) a[j] = b[j] = 0.f;
   if (ea < s.D) ldv<4>(row + ea, a);
   if (eb < s.D) ldv<4>(row + eb, b);
-  if (s.silu) {
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      a[j] = silu_fast(a[j]);
-      b[j] = silu_fast(b[j]);
-    }
-  }
-  if (!rot) return;
   float c[4], sn[4];
-  ldv<4>(cs + p, c);
-  ldv<4>(cs + half + p, sn);
-  if (s.interleaved) {
-#pragma unroll
-    for (int j = 0; j < 4; j += 2) {
-      const float u = a[j], v = a[j + 1];
-      a[j] = u * c[j / 2] - v * sn[j / 2];
-      a[j + 1] = v * c[j / 2] + u * sn[j / 2];
-      const float x = b[j], y = b[j + 1];
-      b[j] = x * c[2 + j / 2] - y * sn[2 + j / 2];
-      b[j + 1] = y * c[2 + j / 2] + x * sn[2 + j / 2];
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const float u = a[j], v = b[j];
-      a[j] = u * c[j] - v * sn[j];
-      b[j] = v * c[j] + u * sn[j];
-    }
+  if (rot) {
+    ldv<4>(cs + p, c);
+    ldv<4>(cs + half + p, sn);
   }
+  shape_runs(a, b, s, rot, c, sn);
 }
 
 constexpr int TS = CHUNK + 8;    // LDS row of a [feature][token] tile
@@ -610,6 +622,394 @@ __global__ __launch_bounds__(512, DP > 128 ? 2 : 4) void chunk_out_split_kernel(
   }
 }
 
+// ---------------------------------------------- the same by segments
+// A segment is `per` chunks of one sequence.  A workgroup walks it in steps of STEP tokens and
+// keeps the state S [D, VB] in its registers, so that states pass through memory once a segment
+// and not once a chunk:
+//   1. linear_walk<false>: what each segment adds to the state, and its decay;
+//   2. segment_scan:       the state ahead of each segment;
+//   3. linear_walk<true>:  the outputs, the state going along.
+// Eight waves own 16 columns of v each (64 columns: the two halves of a step's tokens besides).
+// S lies as the matrix product leaves it: 4 * hi + (0 .. 3) of 16 features of one column to a
+// lane, which is a fragment of two such tiles for the product with q, if q's features are read
+// in that order.  The tokens of decayed k and of v, whose products need them along a lane, are
+// read transposed (ds_read_tr16_b64), rows 4 * hi + (0 .. 3) and 16 on.
+// Bound by instructions of all kinds, some 850 to a wave's step (SiLU, rotation, the division
+// into hi and lo of q, twice k and S): a CU with two workgroups takes 7.9 us for a step of both,
+// with one 4.9.  Hence no exec branches around loads, offsets of 32 bits from a step's first
+// token, and no exact quotient or root in the norm (9.5 and 6.0 us with those).
+// 8 sequences of 2404 tokens on average, 12 heads of 128, norm and gate in it: 242 us, by chunks
+// 434 (133 + 112 + 187 us at 16300 tokens; the states of 305 chunks are 240 MB); 16 of 696 160
+// and 234; 4 of 499 48 and 52; of 32 heads, 8 of 2048, 470 and 925.
+constexpr int STEP = 32;
+
+// Sequence b's segments have the numbers first[b] / per + b on, some of which stay unused.
+DEVINL bool segment(const Chunks& ch, int B, int per, int g, int& c0, int& c1) {
+  int b = 0, last = B - 1;
+  while (b < last) {
+    const int mid = (b + last + 1) / 2;
+    if (ch.first[mid] / per + mid <= g) b = mid;
+    else last = mid - 1;
+  }
+  c0 = ch.first[b] + (g - (ch.first[b] / per + b)) * per;
+  c1 = min(c0 + per, ch.first[b + 1]);
+  return c0 < c1;
+}
+
+// tokens 4 * hi + (0 .. 3) and 16 on of columns c0 + lane % 16 of a [STEP][ld] tile
+DEVINL bf16x8l tokens_frag(const short* tile, int ld, int c0, int lane) {
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  const short* a = tile + ((lane >> 4) * 4 + ((lane & 15) >> 2)) * ld + c0 + (lane & 3) * 4;
+  union { s16x4 h[2]; bf16x8l f; } u;
+  u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)a);
+  u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(a + 16 * ld));
+  return u.f;
+}
+// elements 4 * hi + (0 .. 3) and 16 on of a row
+DEVINL bf16x8l spread_frag(const short* row, int hi) {
+  union { s16x4 h[2]; bf16x8l f; } u;
+  u.h[0] = *reinterpret_cast<const s16x4*>(row + 4 * hi);
+  u.h[1] = *reinterpret_cast<const s16x4*>(row + 16 + 4 * hi);
+  return u.f;
+}
+
+struct Hilo { unsigned hi[2], lo[2]; };        // four numbers as hi + lo
+DEVINL Hilo divide(const float* x) {
+  Hilo r;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    r.hi[j] = pack2bf(x[2 * j], x[2 * j + 1]);
+    r.lo[j] = pack2bf(x[2 * j] - __uint_as_float(r.hi[j] << 16),
+                      x[2 * j + 1] - __uint_as_float(r.hi[j] & 0xffff0000u));
+  }
+  return r;
+}
+DEVINL void put(short* hi, short* lo, const float* x) {
+  const Hilo r = divide(x);
+  *reinterpret_cast<unsigned long long*>(hi) = (unsigned long long)r.hi[1] << 32 | r.hi[0];
+  *reinterpret_cast<unsigned long long*>(lo) = (unsigned long long)r.lo[1] << 32 | r.lo[0];
+}
+
+template <int DP, int VB, bool OUT>
+__global__ __launch_bounds__(512, 4) void linear_walk_kernel(
+    const short* __restrict__ q, const short* __restrict__ k, const short* __restrict__ v,
+    Source s, Chunks ch, int B, int per, const float* __restrict__ pw, float* __restrict__ ws,
+    float* __restrict__ decays, const short* __restrict__ gate, long ldg, float eps,
+    short* __restrict__ o, long ldo) {
+  constexpr int QS = DP + 8, TS2 = DP + 16, VS = VB + 16, PS = STEP + 8;   // LDS rows
+  constexpr int DT = DP / 16, CT = VB / 16, RW = CT / 4;
+  __shared__ __attribute__((aligned(16))) short qt[2][OUT ? STEP * QS : 8];
+  __shared__ __attribute__((aligned(16))) short kt[2][OUT ? STEP * QS : 8];
+  __shared__ __attribute__((aligned(16))) short kd[2][STEP * TS2], vt[STEP * VS];
+  __shared__ __attribute__((aligned(16))) short pt[2][OUT ? STEP * PS : 8];
+  __shared__ float pws[CHUNK + 1], red[OUT ? CT : 1][STEP];
+  const int h = blockIdx.y, v0 = blockIdx.z * VB;
+  int c, c1;
+  if (!segment(ch, B, per, blockIdx.x, c, c1)) return;
+  if (threadIdx.x <= CHUNK) pws[threadIdx.x] = pw[h * (CHUNK + 1) + threadIdx.x];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lo = lane & 15, hi = lane >> 4;
+  const int ct = w % CT, r0 = (w / CT) * RW;
+  const int e0 = v0 + 16 * ct;
+
+  // the state ahead: column e0 + lo, features 16 * dt + 4 * hi + (0 .. 3)
+  float* u = ws + (((long)blockIdx.x * s.H + h) * s.V + min(e0 + lo, s.V - 1)) * DP + 4 * hi;
+  f32x4 S[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++) {
+    S[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (OUT && e0 + lo < s.V) S[dt] = *reinterpret_cast<const f32x4*>(u + 16 * dt);
+  }
+
+  // what this thread stages: two runs of a token's q and k, eight columns of a token's v
+  const int qj = threadIdx.x / (DP / 8), qg = threadIdx.x % (DP / 8);
+  const int vj = threadIdx.x / (VB / 8), ve = threadIdx.x % (VB / 8) * 8;
+  const int half = s.rdims >> 1;
+  const bool rot = 4 * qg < half;
+  int ea, eb;
+  if (s.interleaved || !rot) {
+    ea = rot || s.interleaved ? 8 * qg : s.rdims + 2 * (4 * qg - half);
+    eb = ea + 4;
+  } else {
+    ea = 4 * qg;
+    eb = half + 4 * qg;
+  }
+  // Offsets in bytes from a step's first token, which is the same for all threads.  Threads
+  // past a tile or a row's end read its first.
+  const bool mine = STEP * DP / 8 == 512 || qj < STEP, myv = STEP * VB / 8 == 512 || vj < STEP;
+  const bool la = mine && ea < s.D, lb = mine && eb < s.D;
+  const bool va = myv && v0 + ve < s.V, vb = myv && v0 + ve + 4 < s.V;
+  const bool whole = s.D == DP && v0 + VB <= s.V && STEP * DP / 8 == 512 && STEP * VB / 8 == 512;
+  const unsigned ld2 = (unsigned)s.ld * 2;
+  const s16x4 none{0, 0, 0, 0};
+  s16x4 raw[6];
+  f32x4 cs{}, sn{};
+  auto fetch = [&](long t0, int n) __attribute__((always_inline)) {
+    const char* kb = (const char*)(k + t0 * s.ld + h * s.D);
+    const char* qb = (const char*)(q + t0 * s.ld + h * s.D);
+    const char* vp = (const char*)(v + t0 * s.ld + h * s.V + v0);
+    const char* cb = (const char*)(s.cs + t0 * s.rdims);
+    const bool full = whole && n == STEP;
+    const unsigned j = full || qj < n ? qj : 0, jv = full || vj < n ? vj : 0;
+    const unsigned oa = j * ld2 + (full || la ? ea : 0) * 2, ob = j * ld2 + (full || lb ? eb : 0) * 2;
+    const unsigned xa = jv * ld2 + (full || va ? ve : 0) * 2;
+    const unsigned xb = jv * ld2 + (full || vb ? ve + 4 : 0) * 2;
+    raw[2] = *reinterpret_cast<const s16x4*>(kb + oa);
+    raw[3] = *reinterpret_cast<const s16x4*>(kb + ob);
+    if constexpr (OUT) {
+      raw[0] = *reinterpret_cast<const s16x4*>(qb + oa);
+      raw[1] = *reinterpret_cast<const s16x4*>(qb + ob);
+    }
+    if (half) {
+      const unsigned oc = (j * s.rdims + (rot ? 4 * qg : 0)) * 4;
+      cs = *reinterpret_cast<const f32x4*>(cb + oc);
+      sn = *reinterpret_cast<const f32x4*>(cb + oc + half * 4);
+    }
+    raw[4] = *reinterpret_cast<const s16x4*>(vp + xa);
+    raw[5] = *reinterpret_cast<const s16x4*>(vp + xb);
+  };
+  // what was read of other tokens or columns
+  auto clear = [&](int n) __attribute__((always_inline)) {
+    if (whole && n == STEP) return;
+    if (!(la && qj < n)) raw[0] = raw[2] = none;
+    if (!(lb && qj < n)) raw[1] = raw[3] = none;
+    if (!(va && vj < n)) raw[4] = none;
+    if (!(vb && vj < n)) raw[5] = none;
+  };
+  auto runs = [&](int i, float* a, float* b) {
+    float cc[4], ss[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      a[j] = bf2f(raw[2 * i][j]);
+      b[j] = bf2f(raw[2 * i + 1][j]);
+      cc[j] = cs[j];
+      ss[j] = sn[j];
+    }
+    shape_runs(a, b, s, rot, cc, ss);
+  };
+
+  const bool col_ok = e0 + 4 * hi < s.V;
+  const float invV = 1.f / (float)s.V;
+  int at = 0, len = ch.len[c];
+  long row = ch.row[c];
+  float decay = 1.f;
+  fetch(row, min(STEP, len));
+  __syncthreads();                              // pws
+  for (bool more = true; more;) {
+    const long t0 = row + at;
+    const int n = min(STEP, len - at);
+    clear(n);
+    if (mine) {
+      float a[4], b[4];
+      if constexpr (OUT) {
+        runs(0, a, b);
+        put(&qt[0][qj * QS + ea], &qt[1][qj * QS + ea], a);
+        put(&qt[0][qj * QS + eb], &qt[1][qj * QS + eb], b);
+      }
+      runs(1, a, b);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        a[j] *= s.kscale;
+        b[j] *= s.kscale;
+      }
+      if constexpr (OUT) {
+        put(&kt[0][qj * QS + ea], &kt[1][qj * QS + ea], a);
+        put(&kt[0][qj * QS + eb], &kt[1][qj * QS + eb], b);
+      }
+      const float m = pws[max(n - 1 - qj, 0)];   // tokens past n are zero
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        a[j] *= m;
+        b[j] *= m;
+      }
+      put(&kd[0][qj * TS2 + ea], &kd[1][qj * TS2 + ea], a);
+      put(&kd[0][qj * TS2 + eb], &kd[1][qj * TS2 + eb], b);
+    }
+    if (myv) {
+      if (s.silu) {
+#pragma unroll
+        for (int i = 4; i < 6; i++) {
+          union { unsigned u[2]; s16x4 x; } y;
+#pragma unroll
+          for (int j = 0; j < 2; j++)
+            y.u[j] = pack2bf(silu_fast(bf2f(raw[i][2 * j])), silu_fast(bf2f(raw[i][2 * j + 1])));
+          raw[i] = y.x;
+        }
+      }
+      *reinterpret_cast<s16x4*>(&vt[vj * VS + ve]) = raw[4];
+      *reinterpret_cast<s16x4*>(&vt[vj * VS + ve + 4]) = raw[5];
+    }
+    at += STEP;
+    if (at >= len) {
+      at = 0;
+      more = ++c < c1;
+      if (more) {
+        len = ch.len[c];
+        row = ch.row[c];
+      }
+    }
+    if (more) fetch(row + at, min(STEP, len - at));
+    s16x4 gr[RW];
+    if constexpr (OUT) {
+      if (gate) {
+        const char* gb = (const char*)(gate + t0 * ldg + h * s.V);
+#pragma unroll
+        for (int r = 0; r < RW; r++) {           // past the end: the first token's, not used
+          const int i = 16 * (r0 + r) + lo;
+          gr[r] = *reinterpret_cast<const s16x4*>(
+              gb + ((unsigned)(i < n ? i : 0) * (unsigned)ldg + (col_ok ? e0 + 4 * hi : 0)) * 2);
+        }
+      }
+    }
+    __syncthreads();                            // staged
+    f32x4 acc[RW];
+    if constexpr (OUT) {
+      // scores of one of four tiles, of tokens it with keys jt, to each of the first waves
+      if (w < 4) {
+        const int it = w >> 1, jt = w & 1;
+        f32x4 sc{0.f, 0.f, 0.f, 0.f};
+        if (jt <= it)
+#pragma unroll
+          for (int ks = 0; ks < DP / 32; ks++) {
+            const int qa = (16 * it + lo) * QS + 32 * ks + 8 * hi;
+            const int ka = (16 * jt + lo) * QS + 32 * ks + 8 * hi;
+            const bf16x8l qh = frag(&qt[0][qa]), ql = frag(&qt[1][qa]);
+            const bf16x8l kh = frag(&kt[0][ka]), kl = frag(&kt[1][ka]);
+            sc = mfma16l(kl, qh, sc);
+            sc = mfma16l(kh, ql, sc);
+            sc = mfma16l(kh, qh, sc);
+          }
+        const int i = 16 * it + lo, j = 16 * jt + 4 * hi;
+        float p[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) p[r] = i >= j + r ? sc[r] * pws[max(i - j - r, 0)] : 0.f;
+        put(&pt[0][i * PS + j], &pt[1][i * PS + j], p);
+      }
+      // the state ahead of the step, times q
+#pragma unroll
+      for (int r = 0; r < RW; r++) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int x = 0; x < DP / 32; x++) {
+        const float a[4] = {S[2 * x][0], S[2 * x][1], S[2 * x][2], S[2 * x][3]};
+        const float b[4] = {S[2 * x + 1][0], S[2 * x + 1][1], S[2 * x + 1][2], S[2 * x + 1][3]};
+        const Hilo ha = divide(a), hb = divide(b);
+        union { unsigned u[4]; bf16x8l f; } sh, sl;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          sh.u[j] = ha.hi[j];
+          sh.u[2 + j] = hb.hi[j];
+          sl.u[j] = ha.lo[j];
+          sl.u[2 + j] = hb.lo[j];
+        }
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+          const int qa = (16 * (r0 + r) + lo) * QS + 32 * x;
+          const bf16x8l qh = spread_frag(&qt[0][qa], hi), ql = spread_frag(&qt[1][qa], hi);
+          acc[r] = mfma16l(sl.f, qh, acc[r]);
+          acc[r] = mfma16l(sh.f, ql, acc[r]);
+          acc[r] = mfma16l(sh.f, qh, acc[r]);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < RW; r++) acc[r] *= pws[16 * (r0 + r) + lo + 1];
+      __syncthreads();                          // scores
+    }
+    const bf16x8l vf = tokens_frag(vt, VS, 16 * ct, lane);
+    if constexpr (OUT) {
+#pragma unroll
+      for (int r = 0; r < RW; r++) {
+        const int pa = (16 * (r0 + r) + lo) * PS;
+        acc[r] = mfma16l(vf, spread_frag(&pt[1][pa], hi), acc[r]);
+        acc[r] = mfma16l(vf, spread_frag(&pt[0][pa], hi), acc[r]);
+      }
+    }
+    if (!OUT || more) {                         // the state behind it
+      const float f = pws[n];
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) {
+        S[dt] *= f;
+        S[dt] = mfma16l(tokens_frag(kd[1], TS2, 16 * dt, lane), vf, S[dt]);
+        S[dt] = mfma16l(tokens_frag(kd[0], TS2, 16 * dt, lane), vf, S[dt]);
+      }
+      decay *= f;
+    }
+    if constexpr (OUT) {
+      if (gate) {
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+          float ss = acc[r][0] * acc[r][0] + acc[r][1] * acc[r][1] + acc[r][2] * acc[r][2] +
+                     acc[r][3] * acc[r][3];
+          ss += __shfl_xor(ss, 16);
+          ss += __shfl_xor(ss, 32);
+          if (hi == 0) red[ct][16 * (r0 + r) + lo] = ss;
+        }
+      }
+    }
+    __syncthreads();                            // read, and the sums of squares
+    if constexpr (OUT) {
+      char* ob = (char*)(o + t0 * ldo + h * s.V);
+#pragma unroll
+      for (int r = 0; r < RW; r++) {
+        const int i = 16 * (r0 + r) + lo;
+        float x[4] = {acc[r][0], acc[r][1], acc[r][2], acc[r][3]};
+        if (gate) {
+          float ss = 0.f;
+#pragma unroll
+          for (int y = 0; y < CT; y++) ss += red[y][i];
+          ss = ss * invV + eps;                 // its inverse root, with a step of Newton's
+          float inv = __builtin_amdgcn_rsqf(ss);
+          inv = inv * (1.5f - 0.5f * ss * inv * inv);
+#pragma unroll
+          for (int j = 0; j < 4; j++) x[j] *= inv * silu_fast(bf2f(gr[r][j]));
+        }
+        if (i < n && col_ok) {
+          const unsigned long long y =
+              (unsigned long long)pack2bf(x[2], x[3]) << 32 | pack2bf(x[0], x[1]);
+          *reinterpret_cast<unsigned long long*>(ob + ((unsigned)i * (unsigned)ldo + e0 + 4 * hi) * 2) = y;
+        }
+      }
+    }
+  }
+  if constexpr (!OUT) {
+    if (e0 + lo < s.V && r0 == 0)
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) *reinterpret_cast<f32x4*>(u + 16 * dt) = S[dt];
+    if (threadIdx.x == 0 && blockIdx.z == 0) decays[(long)blockIdx.x * s.H + h] = decay;
+  }
+}
+
+// in place: what a segment adds -> the state ahead of it; the slot is [D][V]
+__global__ __launch_bounds__(256) void segment_scan_kernel(
+    float* __restrict__ ws, const float* __restrict__ decays, float* __restrict__ state, Chunks ch,
+    int per, const int* __restrict__ slots, const int* __restrict__ fresh, int H, int D, int V,
+    int DP) {
+  constexpr int AHEAD = 8;
+  const int b = blockIdx.x, h = blockIdx.y;
+  const int e = blockIdx.z * 256 + threadIdx.x;
+  if (e >= V * DP) return;
+  const int vi = e / DP, d = e % DP;
+  const bool real = d < D;
+  float* st = state + (((long)slots[b] * H + h) * D + (real ? d : 0)) * V + vi;
+  float s = (fresh[b] || !real) ? 0.f : *st;
+  const int g0 = ch.first[b] / per + b, n = (ch.first[b + 1] - ch.first[b] + per - 1) / per;
+  const long step = (long)H * V * DP;
+  float* p = ws + ((long)g0 * H + h) * V * DP + e;
+  const float* f = decays + (long)g0 * H + h;
+  for (int g = 0; g < n; g += AHEAD) {
+    float x[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++) x[i] = g + i < n ? p[i * step] : 0.f;
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++) {
+      if (g + i >= n) break;
+      p[i * step] = s;
+      s = f[(g + i) * H] * s + x[i];
+    }
+    p += AHEAD * step;
+  }
+  if (real) *st = s;
+}
+
 // ------------------------------------------------------------- one token
 // One workgroup per (sequence, head).  With a gate, the head's output is
 // divided by its root mean square and multiplied by silu(gate) on the way out.
@@ -742,14 +1142,13 @@ void linear_attn_chunked(torch::Tensor q, torch::Tensor k, torch::Tensor v, torc
   if (n == 0) return;
   const int DP = s.D <= 32 ? 32 : s.D <= 64 ? 64 : s.D <= 128 ? 128 : 256;
   const bool split = q.scalar_type() == torch::kBFloat16;
-  auto ws = torch::empty({n, s.H, s.V, split ? DP : s.D}, state.options());
   int* cp = chunks.data_ptr<int>();
   const Chunks ch{cp, cp + n, cp + 2 * n, first.data_ptr<int>()};
   auto stream = at::hip::getCurrentHIPStream();
   const dim3 grid(n, s.H, (s.V + VBLK - 1) / VBLK);
   const int DV = s.D * s.V;
   const float* pwp = pw.data_ptr<float>();
-  float* wsp = ws.data_ptr<float>();
+  torch::Tensor ws;
   if (split) {
     auto al = [](const void* p) { return ((uintptr_t)p % 8) == 0; };
     const bool vec = s.D % 4 == 0 && s.V % 4 == 0 && s.rdims % 8 == 0 && s.ld % 4 == 0 &&
@@ -758,6 +1157,43 @@ void linear_attn_chunked(torch::Tensor q, torch::Tensor k, torch::Tensor v, torc
                      (!gate.has_value() || (gate->stride(0) % 4 == 0 && al(gate->data_ptr())));
     const short* gp = gate.has_value() ? (const short*)gate->data_ptr() : nullptr;
     const long ldg = gate.has_value() ? gate->stride(0) : 0;
+    auto short_rows = [](long ld) { return ld >= 0 && ld < 1L << 24; };   // a step's offsets: 32 bits
+    if (vec && DP <= 128 && short_rows(s.ld) && short_rows(ldg) && short_rows(o.stride(0)) &&
+        s.rdims < 1 << 24) {
+      // As many chunks to a segment as leave each CU two workgroups, which is one round.
+      const long across = (long)s.H * ((s.V + (s.V <= 64 ? 63 : 127)) / (s.V <= 64 ? 64 : 128));
+      const int per = std::clamp((n * across + 511) / 512, 1L, 16L);
+      const long G = n / per + B;
+      auto parts = torch::empty({G, s.H, s.V, DP}, state.options());
+      auto decays = torch::empty({G, s.H}, state.options());
+      float* wp = parts.data_ptr<float>();
+      float* dp = decays.data_ptr<float>();
+#define WALK(DD, VB)                                                                            \
+  do {                                                                                          \
+    const dim3 sg(G, s.H, (s.V + VB - 1) / VB);                                                 \
+    hipLaunchKernelGGL((linear_walk_kernel<DD, VB, false>), sg, dim3(512), 0, stream,           \
+                       (const short*)q.data_ptr(), (const short*)k.data_ptr(),                  \
+                       (const short*)v.data_ptr(), s, ch, (int)B, per, pwp, wp, dp, nullptr,    \
+                       0L, 0.f, nullptr, 0L);                                                   \
+    hipLaunchKernelGGL(segment_scan_kernel, dim3(B, s.H, (s.V * DD + 255) / 256), dim3(256), 0, \
+                       stream, wp, dp, state.data_ptr<float>(), ch, per, slots.data_ptr<int>(), \
+                       fresh.data_ptr<int>(), s.H, s.D, s.V, DD);                               \
+    hipLaunchKernelGGL((linear_walk_kernel<DD, VB, true>), sg, dim3(512), 0, stream,            \
+                       (const short*)q.data_ptr(), (const short*)k.data_ptr(),                  \
+                       (const short*)v.data_ptr(), s, ch, (int)B, per, pwp, wp, dp, gp, ldg,    \
+                       (float)eps, (short*)o.data_ptr(), (long)o.stride(0));                    \
+  } while (0)
+#define WALK_V(DD) do { if (s.V <= 64) WALK(DD, 64); else WALK(DD, 128); } while (0)
+      if (DP == 32) WALK_V(32);
+      else if (DP == 64) WALK_V(64);
+      else WALK_V(128);
+#undef WALK_V
+#undef WALK
+      HIP_CHECK_LAST();
+      return;
+    }
+    ws = torch::empty({n, s.H, s.V, DP}, state.options());
+    float* wsp = ws.data_ptr<float>();
 #define SPLIT(DD, VB)                                                                           \
   do {                                                                                          \
     const dim3 sg(n, s.H, (s.V + VB - 1) / VB);                                                 \
@@ -783,6 +1219,8 @@ void linear_attn_chunked(torch::Tensor q, torch::Tensor k, torch::Tensor v, torc
     return;
   }
   TORCH_CHECK(q.scalar_type() == torch::kFloat32);
+  ws = torch::empty({n, s.H, s.V, s.D}, state.options());
+  float* wsp = ws.data_ptr<float>();
 #define PHASES(DD)                                                                             \
   do {                                                                                         \
     hipLaunchKernelGGL((chunk_state_kernel<float, DD>), grid, dim3(256), 0, stream,            \
