@@ -33,6 +33,12 @@ DEVINL float glu(float g, float up) {
   return g * __builtin_amdgcn_rcpf(1.f + __expf(-z)) * up;      // gelu_tanh: x sigmoid(2 ..)
 }
 
+// Into how many units of fewer rows the tiles are divided that are left after whole rounds of
+// the CUs: where they still fit one round.
+__host__ __device__ inline int parts_of(int left, int cus) {
+  return left == 0 || left * 2 > cus ? 1 : left * 4 > cus ? 2 : 4;
+}
+
 struct Big {
   const short *x, *w;            // [M, K], [N, K]
   const short *u, *b;            // [M, 64], [N, 64]
@@ -47,6 +53,7 @@ struct Big {
   int half, Hq, Hkv;
   int M, N, K, grid_m, grid_n;
   int whole, parts, units;       // tiles that are one unit of work, and units of the others
+  int cus;                       // grouped: what these are divided for
   // grouped: G <= 64 products, of the rows that lists [G, cap] name (of x a row / div) or of
   // M each; their results go to the same rows of y, times scale [rows]
   const int *lists, *counts;
@@ -100,7 +107,7 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
   const int wn = (wid & 3) * 64;
   const int n_k1 = p.K >> 6, n_kt = n_k1 + (HAS_LORA ? 1 : 0);
 
-  int grid_m = p.grid_m, units = p.units, whole = p.whole, M = p.M, g = 0;
+  int grid_m = p.grid_m, units = p.units, whole = p.whole, left_parts = p.parts, M = p.M, g = 0;
   if constexpr (GROUPED) {
     if (wid == 0) {
       const int c = lane >= p.G ? 0 : p.counts ? p.counts[lane] : p.M;
@@ -116,7 +123,10 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
     }
     __syncthreads();
     grid_m = __builtin_amdgcn_readfirstlane(starts[64]);
-    units = whole = grid_m * p.grid_n;
+    const int tiles = grid_m * p.grid_n, left = tiles % p.cus;
+    left_parts = parts_of(left, p.cus);
+    whole = left_parts > 1 ? tiles - left : tiles;
+    units = whole + (tiles - whole) * left_parts;
     if (blockIdx.x >= units) return;
   }
 
@@ -126,7 +136,7 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
     int wg = at, part = 0;
     parts = 1;
     if (at >= whole) {
-      parts = p.parts;
+      parts = left_parts;
       wg = whole + (at - whole) / parts;
       part = (at - whole) % parts;
     }
@@ -142,8 +152,10 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
     if constexpr (GROUPED) {
       const int l = threadIdx.x & 63;
       g = __ffsll((unsigned long long)__ballot(tile >= starts[l] && tile < starts[l + 1])) - 1;
-      m0 = (tile - __builtin_amdgcn_readfirstlane(starts[g])) * BIG;
+      m0 = (tile - __builtin_amdgcn_readfirstlane(starts[g])) * BIG + part * (BIG / parts);
       M = __builtin_amdgcn_readfirstlane(sizes[g]);
+      // a group's last rows: of a tile's parts the first has all of them
+      if (parts == 1 && M - m0 <= BIG / 2) parts = M - m0 <= BIG / 4 ? 4 : 2;
     }
   };
 
@@ -562,8 +574,6 @@ __global__ __launch_bounds__(512, 2) void gemm_big_kernel(Big p) {
   }
 }
 
-// The tiles that are left after whole rounds of the CUs are divided by rows where that
-// still fits one round.
 template <bool HAS_LORA, int BIAS, bool VEC, int ACT>
 void launch_big(Big p) {
   const int cus = at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
@@ -571,7 +581,7 @@ void launch_big(Big p) {
   p.grid_m = (p.M + BIG - 1) / BIG;
   p.grid_n = (p.N + TN - 1) / TN;
   const int tiles = p.grid_m * p.grid_n, left = tiles % cus;
-  p.parts = left == 0 || left * 2 > cus ? 1 : left * 4 > cus ? 2 : 4;
+  p.parts = parts_of(left, cus);
   p.whole = p.parts > 1 ? tiles - left : tiles;
   p.units = p.whole + (tiles - p.whole) * p.parts;
   hipLaunchKernelGGL((gemm_big_kernel<HAS_LORA, BIAS, VEC, ACT>), dim3(std::min(p.units, cus)),
@@ -582,7 +592,10 @@ void launch_big(Big p) {
 // tiles of rows at most.  A workgroup counts the groups' tiles at its start and finds the
 // group of each as it comes to it; which rows of x and y they are is kept in LDS.  16
 // experts of 1536 x 2240, 1000 rows each, gate and up 211 us (1050 TFLOP/s), down 100; in
-// tiles of 128 that wait at a barrier a step 299 and 145.  Silu is divided, as those have it,
+// tiles of 128 that wait at a barrier a step 299 and 145.  The tiles left after whole rounds are
+// divided as those of a single product, and a group's last tile takes as many rows as it has
+// (64, 128 or all): 4 products of 2708 x 1536 x 1536 (264 tiles) 72 us, divided 63; the experts
+// of 1536 x 2240 with 300 rows each 148 and 132 us, 677 300 and 286; the bits stay.  Silu is divided, as those have it,
 // which takes 17 us of the 211: the bits are theirs, on which a router's near ties hang.
 template <int ACT>
 void launch_big_grouped(Big p, long most) {
@@ -590,7 +603,8 @@ void launch_big_grouped(Big p, long most) {
   const int cus = at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
   constexpr int TN = ACT ? BIG / 2 : BIG;
   p.grid_n = (p.N + TN - 1) / TN;
+  p.cus = cus;
   hipLaunchKernelGGL((gemm_big_kernel<false, NO_BIAS, true, ACT, true>),
-                     dim3(std::min<long>(most * p.grid_n, cus)), dim3(512), 0,
+                     dim3(std::min<long>(most * p.grid_n * 4, cus)), dim3(512), 0,
                      c10::hip::getCurrentHIPStream(), p);
 }

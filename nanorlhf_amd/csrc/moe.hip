@@ -608,22 +608,29 @@ __global__ __launch_bounds__(1024) void expert_lists_kernel(
 // (192) 68 / 46; 4 experts, 300 rows (144) 33 / 36, 400 (180) 50 / 34; 12 heads of 512 x 128,
 // 4000 rows 16.4 / 18.3.  Up to 128 rows half of a tile is empty and it takes a long product:
 // 110 rows of 1536 x 2240 65 / 66, 100 of 2048 x 2752 139 / 108, 56 of 3584 x 4096 143 / 95.
-static bool fills_big(long each, long tm, long N, long K, int width) {
+// Since what is left after whole rounds is divided, `least` tiles are 96 where all groups have
+// as many rows (4 products of 1536 x 1536, 800 rows 30.2 / 29.1, 1300 50 / 37, 600 (72) 24.7 / 28.2;
+// of 1024 x 4096, 1500 rows 68.3 / 67.4).  Where they are counted, and fewer than `tm`, 150 down (both
+// products, 16 experts of 1536 x 2240, 150 rows 146 / 126), but 176 for gate and up (4 experts of
+// 2048 x 2752, 200 rows (154) 77 / 86).
+static bool fills_big(long each, long tm, long N, long K, int width, long least) {
   const long tn = (N + width - 1) / width;
   return tm * tn < 1L << 31 && N * 4 >= tn * width * 3 &&
-         (each > 128 ? tm * tn >= 176 : tm * tn * K >= 800000);
+         (each > 128 ? tm * tn >= least : tm * tn * K >= 800000);
 }
 
 // ... and takes them: what its 32-bit offsets, whole steps and stores of four columns can do
 static bool takes_big(const Grouped& a, long each, long tm, int width) {
   return a.G <= 64 && a.K > 0 && a.K % 64 == 0 && a.N % 4 == 0 && (a.ldo | a.go) % 4 == 0 &&
          (uintptr_t)a.out % 8 == 0 && a.K < 1L << 22 && a.ldw < 1L << 22 &&
-         (a.rows / a.div + 1) * a.lda < 1L << 31 && fills_big(each, tm, a.N, a.K, width);
+         (a.rows / a.div + 1) * a.lda < 1L << 31 &&
+         fills_big(each, tm, a.N, a.K, width, !a.lists ? 96 : width < BIG ? 176 : 150);
 }
 
-// Whether T rows of each of G products fill gemm_big.h's tiles
+// Whether T rows of each of G products fill gemm_big.h's tiles, for those that are the library's
+// else
 bool group_linear_fills(long T, long G, long N, long K) {
-  return fills_big(T, G * ((T + BIG - 1) / BIG), N, K, BIG);
+  return fills_big(T, G * ((T + BIG - 1) / BIG), N, K, BIG, 176);
 }
 
 template <bool GLU>
