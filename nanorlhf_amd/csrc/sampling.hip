@@ -14,6 +14,8 @@
 // Few rows leave most CUs idle: sample_slices_kernel divides 1 and the sum of 2 among
 // workgroups, and sample_row_kernel goes on with the row's few likely elements, or, where
 // they are many, with a pass around the bin that a sample of the row names.
+//
+// A top-p of 1 keeps every token, which needs no bins and no row in registers: sample_all_kernel.
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -893,6 +895,203 @@ void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
   if (tid == 0) put(pick);
 }
 
+// ------------------------------------------------------ top-p of 1: no bins
+// Every token stays: a maximum and the owners' masses are all that sampling needs, in one pass
+// that keeps no row.  A workgroup of a thread to an owner takes a row, or a slice of it where
+// these are fewer than 2048, which fill the CUs with waves; a second kernel then adds up the
+// slices' masses.  Bound by reading the logits (2048 rows of 151936: 113 us, 5.5 TB/s), for few
+// rows by two launches and their chains of latencies.  bf16 at T = 1, through the bins / so, us:
+//   151936   1 row 36.7 / 8.8   64 44.2 / 12.8   512 99.5 / 32.4   2048 371 / 113
+//   32768    1 row 14.7 / 8.2   64 16.2 / 8.4    512 32.6 / 13.5   2048 121 / 24.3
+//   1000     1 row 12.2 / 5.1   64 13.0 / 5.6    512 25.5 / 6.0    2048 94 / 8.9
+// 32 bits of 151936: 64 rows 54.3 / 14.5, 2048 679 / 207.
+constexpr int ALL_VECS = 4;       // of a thread, asked for together
+
+struct PickScratch {
+  float red[OWNERS / 64], excl;
+  int index[OWNERS / 64], owner, found;
+};
+
+// A category by the owners' masses exp(l / T - top / T), of which each thread has one, and its
+// log-probability.
+template <typename LT>
+DEVINL void pick_of_all(PickScratch& s, const LT* __restrict__ p, int V, float invT, float top,
+                        float own, float uniform, long* __restrict__ out,
+                        float* __restrict__ out_lp) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nvec = V / 8;
+  const float M = top * invT;
+  float incl = own;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const float x = __shfl_up(incl, off);
+    if (lane >= off) incl += x;
+  }
+  if (lane == 63) s.red[wid] = incl;
+  if (tid == 0) { s.owner = OWNERS; s.found = -1; }
+  __syncthreads();
+  float base = 0.f, total = 0.f;
+#pragma unroll
+  for (int w = 0; w < OWNERS / 64; w++) {
+    if (w < wid) base += s.red[w];
+    total += s.red[w];
+  }
+  const float goal = uniform * total, excl = base + incl - own;
+  // rounding may leave two at a border: the first
+  if (own > 0.f && goal >= excl && goal < excl + own) atomicMin(&s.owner, tid);
+  __syncthreads();
+  if (tid == s.owner) s.excl = excl;
+  __syncthreads();
+  if (wid == 0 && s.owner < OWNERS) {
+    // the owner's vectors in order, 64 at a time, one per lane; behind them its last element
+    float acc = s.excl;
+    int last = -1;                  // of a mass, should rounding let no element cross the goal
+    bool found = false;
+    for (int i0 = s.owner; i0 < nvec && !found; i0 += OWNERS * 64) {
+      const int i = i0 + OWNERS * lane;
+      float e[8], m = 0.f;
+      Vec8<LT> w;
+      if (i < nvec) load8(p + 8L * i, w);
+      else fill8(w);
+      get8(w, e);
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        e[j] = __expf(e[j] * invT - M);
+        m += e[j];
+      }
+      float upto = m;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const float x = __shfl_up(upto, off);
+        if (lane >= off) upto += x;
+      }
+      const unsigned long long hit = __ballot(m > 0.f && goal < acc + upto);
+      const unsigned long long some = __ballot(m > 0.f);
+      found = hit != 0;
+      if (some) {
+        const int of = found ? __ffsll(hit) - 1 : 63 - __clzll((long long)some);
+        if (lane == of) {
+          float at = acc + (upto - m);
+          int pick = -1;
+#pragma unroll
+          for (int j = 0; j < 8; j++) {
+            at += e[j];
+            if (e[j] > 0.f) last = 8 * i + j;
+            if (pick < 0 && e[j] > 0.f && goal < at) pick = 8 * i + j;
+          }
+          if (found && pick >= 0) last = pick;
+        }
+        last = __shfl(last, of);
+      }
+      acc += __shfl(upto, 63);
+    }
+    const int t = 8 * nvec + s.owner;
+    if (!found && t < V && __expf(ldf(p + t) * invT - M) > 0.f) last = t;
+    if (lane == 0) s.found = last;
+  }
+  __syncthreads();
+  int pick = s.found;
+  if (pick < 0) {                   // no masses, or not-a-numbers among them
+    float best;
+    pick = row_argmax<OWNERS>(p, V, best, s.red, s.index);
+  }
+  if (tid == 0) {
+    *out = pick;
+    if (out_lp) *out_lp = ldf(p + pick) * invT - (M + __logf(total));
+  }
+}
+
+// Chunks of ALL_VECS vectors a thread, `per` of them to a workgroup.  ONE: the whole row, whose
+// category is chosen at once; else tops [B, slices] and masses [B, slices, OWNERS, ALL_VECS].
+// Every vector of a chunk has a sum of its own, and sums, scans and walk have the order of
+// sample_topp_kernel: of 151936 categories at T = 1 a border lies every 7e-6 of the mass, and
+// 32-bit sums choose another of two neighbours than 64-bit ones 4 times in 1000, there and here,
+// 6 times with sums in one chain.
+template <typename LT, bool ONE>
+__global__ __launch_bounds__(OWNERS)
+void sample_all_kernel(const LT* __restrict__ logits, long* __restrict__ out,
+                       float* __restrict__ out_lp, float* __restrict__ tops,
+                       float* __restrict__ masses, int V, int chunks, int per, int slices,
+                       float invT,
+                       unsigned long long seed, unsigned long long step_imm,
+                       const long* __restrict__ step_ptr) {
+  __shared__ PickScratch s;
+  const long row = blockIdx.x / slices;
+  const int slice = blockIdx.x % slices, tid = threadIdx.x, nvec = V / 8;
+  const LT* p = logits + row * (long)V;
+  const int c1 = min(chunks, (slice + 1) * per);
+  static_assert(ALL_VECS * OWNERS == SBLOCK, "a thread's vectors there");
+  float top = -INFINITY;                   // this thread's
+  f32x4 sum{0.f, 0.f, 0.f, 0.f};
+  auto grow = [&](float most) {            // the exponent's subtrahend from here on
+    const float now = fmaxf(top, most), M = now == -INFINITY ? 0.f : now * invT;
+    sum *= __expf(top * invT - M);
+    top = now;
+    return M;
+  };
+  for (int c = slice * per; c < c1; c++) {
+    const int at = c * ALL_VECS * OWNERS + tid;
+    Vec8<LT> v[ALL_VECS];
+#pragma unroll
+    for (int k = 0; k < ALL_VECS; k++) load8(p + 8L * min(at + OWNERS * k, nvec - 1), v[k]);
+    float most = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < ALL_VECS; k++) {
+      if (at + OWNERS * k >= nvec) fill8(v[k]);
+      float x[8];
+      get8(v[k], x);
+      most = fmaxf(most, max8(x));
+    }
+    const float M = grow(most);
+#pragma unroll
+    for (int k = 0; k < ALL_VECS; k++) {
+      float x[8];
+      get8(v[k], x);
+#pragma unroll
+      for (int j = 0; j < 8; j++) sum[k] += __expf(x[j] * invT - M);
+    }
+  }
+  // the last elements belong to the first owners, behind their vectors
+  if (c1 == chunks && 8 * nvec + tid < V) {
+    const float x = ldf(p + 8 * nvec + tid);
+    const float M = grow(x);
+    sum[0] += __expf(x * invT - M);
+  }
+  const float best = block_max<OWNERS>(top, s.red);
+  if (best != -INFINITY) sum *= __expf((top - best) * invT);
+  if constexpr (ONE) {
+    const unsigned long long step = step_imm + (step_ptr ? (unsigned long long)*step_ptr : 0);
+    __syncthreads();
+    pick_of_all(s, p, V, invT, best, ((sum[0] + sum[1]) + sum[2]) + sum[3],
+                hash_uniform(seed, step, (unsigned long long)row), out + row, out_lp ? out_lp + row : nullptr);
+  } else {
+    const long part = blockIdx.x;
+    if (tid == 0) tops[part] = best;
+    reinterpret_cast<f32x4*>(masses)[part * OWNERS + tid] = sum;
+  }
+}
+
+template <typename LT>
+__global__ __launch_bounds__(OWNERS)
+void sample_all_pick_kernel(const LT* __restrict__ logits, long* __restrict__ out,
+                            float* __restrict__ out_lp, const float* __restrict__ tops,
+                            const float* __restrict__ masses, int V, int slices, float invT,
+                            unsigned long long seed, unsigned long long step_imm,
+                            const long* __restrict__ step_ptr) {
+  __shared__ PickScratch s;
+  const long row = blockIdx.x;
+  const unsigned long long step = step_imm + (step_ptr ? (unsigned long long)*step_ptr : 0);
+  float best = -INFINITY;
+  f32x4 sum{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < slices; i++) best = fmaxf(best, tops[row * slices + i]);
+#pragma unroll 4
+  for (int i = 0; i < slices; i++)
+    sum += reinterpret_cast<const f32x4*>(masses)[(row * slices + i) * OWNERS + threadIdx.x] *
+           __expf((tops[row * slices + i] - best) * invT);
+  pick_of_all(s, logits + row * (long)V, V, invT, best, ((sum[0] + sum[1]) + sum[2]) + sum[3],
+              hash_uniform(seed, step, (unsigned long long)row), out + row,
+              out_lp ? out_lp + row : nullptr);
+}
+
 // Vectors per thread that are held in registers; 1024 threads have 128 each, so
 // 19 of bf16 (155648 logits) and 8 of float32 (65536) fit beside the rest.
 //
@@ -924,6 +1123,43 @@ static void launch_sampler(const torch::Tensor& logits, torch::Tensor& out, floa
     HIP_CHECK_LAST();
     return;
   }
+  if (top_p >= 1.) {
+    const int chunks = (V / 8 + ALL_VECS * OWNERS - 1) / (ALL_VECS * OWNERS);
+    const int want = std::max(1L, std::min<long>(chunks, (2047 + B) / B));
+    const int per = std::max(1, (chunks + want - 1) / want);
+    const int slices = std::max(1, (chunks + per - 1) / per);
+    const float invT = temperature > 0. ? 1.f / (float)temperature : 1.f;
+    TORCH_CHECK(B * slices < 1L << 31, "sampling: too many rows");
+    torch::Tensor work;
+    float *tops = nullptr, *masses = nullptr;
+    if (slices > 1) {
+      work = torch::empty({B * slices * (SBLOCK + 1)}, logits.options().dtype(torch::kFloat32));
+      masses = work.data_ptr<float>();
+      tops = masses + B * slices * SBLOCK;
+    }
+#define LAUNCH(LT, ONE)                                                                       \
+  hipLaunchKernelGGL((sample_all_kernel<LT, ONE>), dim3(B * slices), dim3(OWNERS), 0, stream, \
+                     (const LT*)logits.data_ptr(), out.data_ptr<long>(), lp, tops, masses, V, \
+                     chunks, per, slices, invT, (unsigned long long)seed,                     \
+                     (unsigned long long)step, step_ptr)
+#define PICK(LT)                                                                              \
+  hipLaunchKernelGGL((sample_all_pick_kernel<LT>), dim3(B), dim3(OWNERS), 0, stream,          \
+                     (const LT*)logits.data_ptr(), out.data_ptr<long>(), lp, tops, masses, V, \
+                     slices, invT, (unsigned long long)seed, (unsigned long long)step, step_ptr)
+    if (slices == 1) {
+      if (half) LAUNCH(short, true); else LAUNCH(float, true);
+    } else if (half) {
+      LAUNCH(short, false);
+      PICK(short);
+    } else {
+      LAUNCH(float, false);
+      PICK(float);
+    }
+#undef PICK
+#undef LAUNCH
+    HIP_CHECK_LAST();
+    return;
+  }
   // A CU that has a row to itself takes the time of its VALU and LDS over the whole row: few
   // rows are divided for the first half of it.  A nucleus of few elements, as a language
   // model's, then is a few us; of rows that are flat (normal logits of deviation 1) every
@@ -936,7 +1172,6 @@ static void launch_sampler(const torch::Tensor& logits, torch::Tensor& out, floa
   //   32 bits, 152064  4     31.9 / 12.6 | 47.2 / 44.2    64     47.4 / 18.8 | 57.6 / 53.3
   //                    512   175 / 91 | 171 / 172
   // At T = 1, where the nucleus has a thousand elements, 8 rows 38.5 / 30.5, 64 39.3 / 37.5.
-  // A top-p of 1 has no bin to look for.
   if (n > 12 && n <= 20 && B <= (half ? 64 : 512) && top_p < 1.) {
     const int slices = (V / 8 + SLICE - 1) / SLICE;
     const int run = n <= 16 ? 32 : 40;          // half of an owner's vectors, n * 4
