@@ -638,8 +638,8 @@ __global__ __launch_bounds__(512, DP > 128 ? 2 : 4) void chunk_out_split_kernel(
 // into hi and lo of q, twice k and S): a CU with two workgroups takes 7.9 us for a step of both,
 // with one 4.9.  Hence no exec branches around loads, offsets of 32 bits from a step's first
 // token, and no exact quotient or root in the norm (9.5 and 6.0 us with those).
-// 8 sequences of 2404 tokens on average, 12 heads of 128, norm and gate in it: 242 us, by chunks
-// 434 (133 + 112 + 187 us at 16300 tokens; the states of 305 chunks are 240 MB); 16 of 696 160
+// 8 sequences of 2404 tokens on average, 12 heads of 128, norm and gate in it: 200 us, by chunks
+// 434 (133 + 112 + 187 us at 16300 tokens; the states of 305 chunks are 240 MB); 16 of 696 136
 // and 234; 4 of 499 48 and 52; of 32 heads, 8 of 2048, 470 and 925.
 constexpr int STEP = 32;
 
@@ -1158,11 +1158,18 @@ void linear_attn_chunked(torch::Tensor q, torch::Tensor k, torch::Tensor v, torc
     const short* gp = gate.has_value() ? (const short*)gate->data_ptr() : nullptr;
     const long ldg = gate.has_value() ? gate->stride(0) : 0;
     auto short_rows = [](long ld) { return ld >= 0 && ld < 1L << 24; };   // a step's offsets: 32 bits
-    if (vec && DP <= 128 && short_rows(s.ld) && short_rows(ldg) && short_rows(o.stride(0)) &&
-        s.rdims < 1 << 24) {
-      // As many chunks to a segment as leave each CU two workgroups, which is one round.
-      const long across = (long)s.H * ((s.V + (s.V <= 64 ? 63 : 127)) / (s.V <= 64 ? 64 : 128));
-      const int per = std::clamp((n * across + 511) / 512, 1L, 16L);
+    // Of a few workgroups the steps of 32 tokens follow each other where a chunk has one of 64: 36
+    // tokens of 12 heads 23.0 us by segments, 21.6 by chunks; 536 (108 workgroups) 29.2 and 28.8, 4
+    // times 499 47.9 and 52.
+    const long across = (long)s.H * ((s.V + (s.V <= 64 ? 63 : 127)) / (s.V <= 64 ? 64 : 128));
+    if (vec && DP <= 128 && n * across >= 128 && short_rows(s.ld) && short_rows(ldg) &&
+        short_rows(o.stride(0)) && s.rdims < 1 << 24) {
+      // As many chunks to a segment as leave each CU two workgroups, which is one round, if three
+      // quarters of a segment are lost at each sequence's end (half of one is, most times).  16
+      // sequences of 696 tokens on average (183 chunks), 12 heads: 5 chunks (some 540 workgroups)
+      // 160 us, 6 136; 8 of 2404 (305 chunks) 240 with 8, 200 with 9.
+      int per = 1;
+      while (per < 16 && across * (4 * n + 3 * B * (per - 1)) > 2048L * per) per++;
       const long G = n / per + B;
       auto parts = torch::empty({G, s.H, s.V, DP}, state.options());
       auto decays = torch::empty({G, s.H}, state.options());
