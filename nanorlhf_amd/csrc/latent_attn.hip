@@ -77,7 +77,78 @@ struct LatentArgs {
   float* ms;             // [units, splits, 16, 2] maximum (log2) and weight
   int H, maxP, splits;
   float scale;
+  int B, budget;         // one token each: workgroups to divide all pages among, or 0
+  int2* plan;            // [B] a sequence's first workgroup, and how many it has
 };
+
+// Which part of which sequence workgroup w of a.budget has: every sequence is divided into as
+// many parts of at most `per` pages as it takes, `per` being about the least (to a sixteenth)
+// with which all parts are at most the budget.  A wave's lane looks at four sequences; all waves
+// come to the same.
+struct LatentPart { int seq, z, per, parts; };
+DEVINL bool latent_part(const LatentArgs& a, int w, LatentPart& out) {
+  const int lane = threadIdx.x & 63;
+  int pages[4];
+  float sum = 0.f, longest = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int b = 4 * lane + i;
+    pages[i] = b < a.B ? max((a.seq_lens[b] - 1) / 16 + 1, 1) : 0;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    sum += (float)pages[i];
+    longest = fmaxf(longest, (float)pages[i]);
+  }
+  const float total = wave_sum(sum);
+  const int most = (int)wave_max(longest);
+  auto parts = [&](int n, int per, float inv) {      // n / per, rounded up
+    int q = (int)((float)(n + per - 1) * inv);
+    if (q * per > n + per - 1) q--;
+    if ((q + 1) * per <= n + per - 1) q++;
+    return q;
+  };
+  // two pages to a wave at least, and what the merge's lanes can hold
+  int low = max(max(8, (most + 63) / 64), (int)(total / (float)a.budget));
+  int per = max(low, min(most, (int)(total / (float)(a.budget - a.B)) + 1));
+  while (per - low > low / 16) {
+    const int mid = (low + per) / 2;
+    const float inv = 1.f / (float)mid;
+    float n = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) n += (float)parts(pages[i], mid, inv);
+    if (wave_sum(n) <= (float)a.budget) per = mid;
+    else low = mid + 1;
+  }
+  int c[4], mine = 0;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    c[i] = parts(pages[i], per, 1.f / (float)per);
+    mine += c[i];
+  }
+  int upto = mine;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int x = __shfl_up(upto, off);
+    if (lane >= off) upto += x;
+  }
+  const unsigned long long hit = __ballot(w >= upto - mine && w < upto);
+  if (!hit) return false;
+  const int at = __ffsll(hit) - 1;
+  int z = w - __builtin_amdgcn_readlane(upto - mine, at), seq = 4 * at, n = 0;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int here = __builtin_amdgcn_readlane(c[i], at);
+    if (n == 0 && z < here) {
+      n = here;
+      seq = 4 * at + i;
+    } else if (n == 0) {
+      z -= here;
+    }
+  }
+  out = {seq, z, per, n};
+  return true;
+}
 
 // A page's 16-byte chunks are exchanged (xor) by row, so that 16 rows at one
 // column (scores) and 4 rows at 4 columns (turned around) meet all banks.
@@ -95,7 +166,7 @@ DEVINL int page_swz(int row) {
 // four barriers per tile it took 116.  Before fragments were read ahead (72 us) four
 // parts took 9 us more than two (a part's first loads and sums), two waves per
 // workgroup 2 more.
-template <int RP>
+template <int RP, bool ALL>
 __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
   constexpr int NW = 4, NC = RP / 32, NT = RP / 16, CH = RP / 8;
   constexpr int PAGE = 16 * RP;                          // elements
@@ -104,7 +175,16 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
   // pages of each wave; at the end its sums, 16 x RP floats
   __shared__ __attribute__((aligned(1024))) short buf[NW][NBUF * PAGE];
   __shared__ float Lm[NW][16], Ls[NW][16];
-  const int seq = blockIdx.y;
+  int seq = blockIdx.y, z = blockIdx.z, splits = a.splits, per = 0;
+  if constexpr (ALL) {
+    LatentPart mine;
+    if (!latent_part(a, blockIdx.y, mine)) return;
+    seq = mine.seq;
+    z = mine.z;
+    splits = mine.parts;
+    per = mine.per;
+    if (z == 0 && blockIdx.x == 0 && threadIdx.x == 0) a.plan[seq] = int2{(int)blockIdx.y, splits};
+  }
   const int t0 = a.cu ? a.cu[seq] : seq;
   const int nq = a.cu ? a.cu[seq + 1] - t0 : 1;
   const int R = nq * a.H, r0 = blockIdx.x * 16;
@@ -115,8 +195,8 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
   const int row = min(r0 + lo, R - 1);
   const int qpos = start + row / a.H;         // of this lane's row
   const int npages = (start + min(r0 + 15, R - 1) / a.H) / 16 + 1;
-  const int per = (npages + a.splits - 1) / a.splits;
-  const int p0 = blockIdx.z * per, p1 = min(npages, p0 + per);
+  if (!ALL) per = (npages + splits - 1) / splits;
+  const int p0 = z * per, p1 = min(npages, p0 + per);
   // scalar loads: a vector load would be waited for behind the pages under way
   typedef const __attribute__((address_space(4))) int* const_ints;
   const const_ints btb = (const_ints)(size_t)(a.bt + (long)seq * a.maxP);
@@ -230,7 +310,8 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
     *reinterpret_cast<f32x4*>(own + lo * RP + (((4 * t + hi) ^ lo) << 2)) = acc[t];
   if (hi == 0) { Lm[wid][lo] = m; Ls[wid][lo] = sum; }
   __syncthreads();
-  const long unit = ((long)blockIdx.y * gridDim.x + blockIdx.x) * a.splits + blockIdx.z;
+  const long unit = ALL ? (long)blockIdx.y * gridDim.x + blockIdx.x
+                        : ((long)blockIdx.y * gridDim.x + blockIdx.x) * splits + z;
   // four rows to a wave; all sums ahead of the first store, so that their reads overlap
   constexpr int NK = RP / 64;
   f32x4 o[NK];
@@ -256,7 +337,7 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
   for (int k = 0; k < NK; k++) {
     const int i = lane + 64 * k, r = 4 * wid + i / (RP / 4), c = i % (RP / 4);
     if (r0 + r >= R) continue;
-    if (a.splits > 1) {
+    if (splits > 1) {
       *reinterpret_cast<f32x4*>(a.part + (unit * 16 + r) * RP + 4 * c) = o[k];
       if (c == 0) {
         a.ms[(unit * 16 + r) * 2] = M[k];
@@ -272,19 +353,28 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
 
 // One workgroup per (16-row unit, row): the parts of a split context joined.  A chain of
 // latencies, so up to MOST parts are asked for at once with their shares.
-template <int MOST>
+template <int MOST, bool ALL>
 __global__ __launch_bounds__(128) void latent_merge_kernel(LatentArgs a, int RP, int units_x) {
   const int unit = blockIdx.x, rr = blockIdx.y;
   const int seq = unit / units_x, r0 = unit % units_x * 16;
   const int z = threadIdx.x & 63;
-  const float* ms = a.ms + ((long)unit * a.splits * 16 + rr) * 2;
-  const float* p = a.part + ((long)unit * a.splits * 16 + rr) * RP;
-  const float2 w = z < a.splits ? *reinterpret_cast<const float2*>(ms + z * 32)
-                                : float2{-INFINITY, 0.f};
+  int splits = a.splits, step = 1;
+  long first = (long)unit * splits;                    // of parts
+  if constexpr (ALL) {
+    const int2 has = a.plan[seq];
+    splits = has.y;
+    if (splits < 2) return;                            // written as it is
+    first = (long)has.x * units_x + unit % units_x;
+    step = units_x;
+  }
+  const float* ms = a.ms + (first * 16 + rr) * 2;
+  const float* p = a.part + (first * 16 + rr) * RP;
+  const float2 w = z < splits ? *reinterpret_cast<const float2*>(ms + z * step * 32)
+                              : float2{-INFINITY, 0.f};
   f32x4 x[MOST ? MOST : 1];
 #pragma unroll
   for (int i = 0; i < MOST; i++)
-    x[i] = *reinterpret_cast<const f32x4*>(p + (long)min(i, a.splits - 1) * 16 * RP +
+    x[i] = *reinterpret_cast<const f32x4*>(p + (long)min(i, splits - 1) * step * 16 * RP +
                                            min((int)threadIdx.x * 4, RP - 4));
 #pragma unroll
   for (int i = 0; i < MOST; i++) asm volatile("" : "+v"(x[i]));
@@ -294,29 +384,34 @@ __global__ __launch_bounds__(128) void latent_merge_kernel(LatentArgs a, int RP,
   const float f = exp2f(w.x - wave_max(w.x));
   float share = f / wave_sum(w.y * f);
   asm volatile("" : "+v"(share));         // of every lane, those too that have no column below
-  auto of = [&](int i) {                  // part i's share of the result
-    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(share), i));
+  // Part i's share of the result.  Of many parts through LDS: 16 x 8000 latents, in 16 parts, took
+  // 48.5 us so and 51.3 with a lane read for each.
+  __shared__ float shares[MOST ? 1 : 64];
+  if constexpr (MOST == 0) {
+    if (threadIdx.x < 64) shares[z] = share;
+    __syncthreads();
+  }
+  auto of = [&](int i) {
+    if constexpr (MOST == 0) return shares[i];
+    else return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(share), i));
   };
   short* out = a.out + ((long)t0 * a.H + r0 + rr) * RP;
   for (int d = threadIdx.x * 4; d < RP; d += 512) {
     float o[4] = {};
-    if (MOST) {
 #pragma unroll
-      for (int i = 0; i < MOST; i++)
-        if (i < a.splits) {
-          const float g = of(i);
-#pragma unroll
-          for (int j = 0; j < 4; j++) o[j] += g * x[i][j];
-        }
-    } else {
-#pragma unroll 4
-      for (int i = 0; i < a.splits; i++) {
+    for (int i = 0; i < MOST; i++)
+      if (i < splits) {
         const float g = of(i);
-        float y[4];
-        ldv<4>(p + (long)i * 16 * RP + d, y);
 #pragma unroll
-        for (int j = 0; j < 4; j++) o[j] += g * y[j];
+        for (int j = 0; j < 4; j++) o[j] += g * x[i][j];
       }
+#pragma unroll 4
+    for (int i = MOST; i < splits; i++) {
+      const float g = of(i);
+      float y[4];
+      ldv<4>(p + (long)i * step * 16 * RP + d, y);
+#pragma unroll
+      for (int j = 0; j < 4; j++) o[j] += g * y[j];
     }
     stv<4>(out + d, o);
   }
@@ -518,32 +613,53 @@ torch::Tensor latent_attn(torch::Tensor qa, torch::Tensor cache, c10::optional<t
   a.H = H;
   a.maxP = bt.size(1);
   a.scale = scale;
-  // one workgroup per CU, none with less than two pages for every wave
-  const long most = std::max<long>(1, bt.size(1) / 8);
+  // One workgroup per CU, none with less than two pages for every wave, all sequences with as
+  // many parts.  Single tokens of long and uneven contexts divide all pages instead, which leaves
+  // no CU idle and no context's parts longer than others; that takes a workgroup 1 us to find
+  // out, and parts that are not full.  us, as many parts / all pages, of rows x mean of 512, lengths
+  // a third to five thirds of it: 32 x 8000 69.5 / 58.9, 64 x 4000 73.5 / 65.0, 100 x 2600 83.7 /
+  // 70.3, but 128 x 2000 76.2 / 77.6, 16 x 8000 48.4 / 48.2, 128 x 700 42.8 / 42.2, 64 x 1000 of
+  // 256 27.0 / 27.9.
+  const long most = std::max<long>(1, bt.size(1) / 8), budget = 256 / units_x;
   a.splits = (int)std::min<long>(std::min<long>(most, 64), std::max<long>(1, 256 / units));
-  torch::Tensor part, ms;
-  if (a.splits > 1) {
+  a.B = B;
+  a.budget = !cu.has_value() && B > 1 && 5 * B <= 2 * budget && B * units_x * bt.size(1) >= 16384
+                 ? (int)budget : 0;
+  torch::Tensor part, ms, plan;
+  if (a.splits > 1 || a.budget) {
     auto f = qa.options().dtype(torch::kFloat32);
-    part = torch::empty({units, a.splits, 16, RP}, f);
-    ms = torch::empty({units, a.splits, 16, 2}, f);
+    const long n = a.budget ? budget * units_x : units * a.splits;
+    part = torch::empty({n, 16, RP}, f);
+    ms = torch::empty({n, 16, 2}, f);
     a.part = part.data_ptr<float>();
     a.ms = ms.data_ptr<float>();
   }
+  if (a.budget) {
+    plan = torch::empty({B, 2}, qa.options().dtype(torch::kInt));
+    a.plan = (int2*)plan.data_ptr<int>();
+  }
   auto stream = at::hip::getCurrentHIPStream();
   TORCH_CHECK(B <= 65535, "too many sequences in a batch");
-  const dim3 grid(units_x, B, a.splits);
-#define LAUNCH(RR) hipLaunchKernelGGL((latent_attn_kernel<RR>), grid, dim3(256), 0, stream, a)
+  const dim3 grid = a.budget ? dim3(units_x, budget) : dim3(units_x, B, a.splits);
+#define LAUNCH(RR)                                                                            \
+  do {                                                                                        \
+    if (a.budget)                                                                             \
+      hipLaunchKernelGGL((latent_attn_kernel<RR, true>), grid, dim3(256), 0, stream, a);      \
+    else                                                                                      \
+      hipLaunchKernelGGL((latent_attn_kernel<RR, false>), grid, dim3(256), 0, stream, a);     \
+  } while (0)
   if (RP == 64) LAUNCH(64);
   else if (RP == 128) LAUNCH(128);
   else if (RP == 256) LAUNCH(256);
   else if (RP == 512) LAUNCH(512);
   else TORCH_CHECK(false, "unsupported latent width ", RP);
 #undef LAUNCH
-#define MERGE(MOST)                                                                           \
-  hipLaunchKernelGGL(latent_merge_kernel<MOST>, dim3(units, 16), dim3(128), 0, stream, a,     \
+#define MERGE(MOST, ALL)                                                                      \
+  hipLaunchKernelGGL((latent_merge_kernel<MOST, ALL>), dim3(units, 16), dim3(128), 0, stream, a,     \
                      (int)RP, (int)units_x)
-  if (a.splits > 4) MERGE(0);
-  else if (a.splits > 1) MERGE(4);
+  if (a.budget) MERGE(8, true);
+  else if (a.splits > 4) MERGE(0, false);
+  else if (a.splits > 1) MERGE(4, false);
 #undef MERGE
   HIP_CHECK_LAST();
   return out;
