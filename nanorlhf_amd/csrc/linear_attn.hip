@@ -640,7 +640,7 @@ __global__ __launch_bounds__(512, DP > 128 ? 2 : 4) void chunk_out_split_kernel(
 // token, and no exact quotient or root in the norm (9.5 and 6.0 us with those).
 // 8 sequences of 2404 tokens on average, 12 heads of 128, norm and gate in it: 200 us, by chunks
 // 434 (133 + 112 + 187 us at 16300 tokens; the states of 305 chunks are 240 MB); 16 of 696 136
-// and 234; 4 of 499 48 and 52; of 32 heads, 8 of 2048, 470 and 925.
+// and 234; 4 of 499 48 and 52; of 32 heads, 8 of 2048, 412 to 435 and 925.
 constexpr int STEP = 32;
 
 // Sequence b's segments have the numbers first[b] / per + b on, some of which stay unused.
@@ -1167,9 +1167,18 @@ void linear_attn_chunked(torch::Tensor q, torch::Tensor k, torch::Tensor v, torc
       // As many chunks to a segment as leave each CU two workgroups, which is one round, if three
       // quarters of a segment are lost at each sequence's end (half of one is, most times).  16
       // sequences of 696 tokens on average (183 chunks), 12 heads: 5 chunks (some 540 workgroups)
-      // 160 us, 6 136; 8 of 2404 (305 chunks) 240 with 8, 200 with 9.
+      // 160 us, 6 136; 8 of 2404 (305 chunks) 240 with 8, 200 with 9.  Where 16 chunks are more
+      // than a round and sequences long, the number with which the rounds are through soonest: 32
+      // heads, 8 of 2048 tokens 468 with 16 (two rounds), 412 to 435 so; but 16 of 464 tokens
+      // of 12 heads, chosen so, 129 and not 107.
+      auto groups = [&](long i) { return across * (4 * n + 3 * B * (i - 1)) / (4 * i); };
       int per = 1;
-      while (per < 16 && across * (4 * n + 3 * B * (per - 1)) > 2048L * per) per++;
+      while (per < 16 && groups(per) > 512) per++;
+      if (groups(per) > 512 && n >= 24 * B) {
+        auto cost = [&](long i) { return (groups(i) + 511) / 512 * (2 * i + 1); };
+        for (int i = 8; i <= 24; i++)
+          if (cost(i) < cost(per)) per = i;
+      }
       const long G = n / per + B;
       auto parts = torch::empty({G, s.H, s.V, DP}, state.options());
       auto decays = torch::empty({G, s.H}, state.options());
