@@ -767,7 +767,10 @@ void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
       const float bottom = hi - 2.f;
       own = 0.f;
       // In pairs, whose columns are read before either is written: half the reads' latency,
-      // which is what the pass takes.  Elements of neither bin go to one behind them.
+      // which is what the pass takes.  Elements of neither bin go to one behind them.  The bin
+      // by u's floor, which is exact, as kept's comparison is: u - bottom is rounded, and an
+      // element just below a bin's upper border would be in the next, the largest behind them.
+      const int first_bin = (int)bottom * BINS;
       each(bottom, [&](const float* u, int) {
 #pragma unroll
         for (int j = 0; j < 8; j += 2) {
@@ -777,7 +780,8 @@ void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
           for (int i = 0; i < 2; i++) {
             e[i] = __expf(u[j + i]);
             own += u[j + i] >= hi ? e[i] : 0.f;
-            k[i] = u[j + i] >= bottom && u[j + i] < hi ? (int)((u[j + i] - bottom) * BINS) : 2 * BINS;
+            k[i] = u[j + i] >= bottom && u[j + i] < hi
+                       ? (int)floorf(u[j + i] * BINS) - first_bin : 2 * BINS;
           }
           if (!__any(min(k[0], k[1]) < 2 * BINS)) continue;
           float *h0 = &s.hist[wid][k[0]][lane], *h1 = &s.hist[wid][k[1]][lane];
@@ -822,11 +826,12 @@ void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
       __syncthreads();
       clear(BINS);
       const float lo = lowest;
+      const int first_bin = (int)(lo * (BINS * BINS));
       each(lo, [&](const float* u, int) {
 #pragma unroll
         for (int j = 0; j < 8; j++)
           if (u[j] >= lo && u[j] < lo + 1.f / BINS)
-            s.hist[wid][(int)((u[j] - lo) * (BINS * BINS))][lane] += __expf(u[j]);
+            s.hist[wid][(int)floorf(u[j] * (BINS * BINS)) - first_bin][lane] += __expf(u[j]);
       });
       sum_bins();
       const float y = lane < BINS ? s.bin[BINS - 1 - lane] : 0.f;
