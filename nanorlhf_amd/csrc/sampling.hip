@@ -426,6 +426,11 @@ void sample_topp_kernel(const LT* __restrict__ logits,
   }
 }
 
+// A part of a row may hold nothing but a mask, -1e10 or the type's lowest value, and so far from 0
+// top / T is no subtrahend of l / T: its rounding alone is a large exponent, or it is -inf.  There
+// the exponents are (l - top) / T.
+DEVINL bool far_below(float top, float invT) { return top * invT < -1e6f && top > -INFINITY; }
+
 // Every element once, by workgroups of 256 threads, 8 vectors a thread: `part` [B, slices],
 // a slice's largest logit and its sum of exp((l - that) / T), and `runs` [B, RBLOCK, RUN], the
 // vectors' largest elements, where a thread of the row's workgroup finds a run of RUN vectors
@@ -461,15 +466,20 @@ void sample_slices_kernel(const LT* __restrict__ logits, float2* __restrict__ pa
   const int j = blockIdx.x * SLICE_VECS;
   stv<SLICE_VECS>(runs + ((row * OWNERS + threadIdx.x) * 2 + j / RUN) * RUN + j % RUN, m);
   top = block_max<OWNERS>(top, red);
+  float sum = 0.f;
+  const auto add = [&](auto e) {
+    sum = e(tail);
+#pragma unroll
+    for (int k = 0; k < SLICE_VECS; k++) {
+      float v[8];
+      get8(c[k], v);
+#pragma unroll
+      for (int j = 0; j < 8; j++) sum += e(v[j]);
+    }
+  };
   const float M = top == -INFINITY ? 0.f : top * invT;
-  float sum = __expf(tail * invT - M);
-#pragma unroll
-  for (int k = 0; k < SLICE_VECS; k++) {
-    float v[8];
-    get8(c[k], v);
-#pragma unroll
-    for (int j = 0; j < 8; j++) sum += __expf(v[j] * invT - M);
-  }
+  if (far_below(top, invT)) add([&](float l) { return __expf((l - top) * invT); });
+  else add([&](float l) { return __expf(l * invT - M); });
   sum = block_sum<OWNERS>(sum, red);
   if (threadIdx.x == 0) part[row * gridDim.x + blockIdx.x] = float2{top, sum};
 }
@@ -1028,10 +1038,10 @@ void sample_all_kernel(const LT* __restrict__ logits, long* __restrict__ out,
   float top = -INFINITY;                   // this thread's
   f32x4 sum{0.f, 0.f, 0.f, 0.f};
   auto grow = [&](float most) {            // the exponent's subtrahend from here on
-    const float now = fmaxf(top, most), M = now == -INFINITY ? 0.f : now * invT;
-    sum *= __expf(top * invT - M);
+    const float now = fmaxf(top, most);
+    if (now > top) sum *= __expf((top - now) * invT);
     top = now;
-    return M;
+    return now == -INFINITY ? 0.f : now * invT;
   };
   for (int c = slice * per; c < c1; c++) {
     const int at = c * ALL_VECS * OWNERS + tid;
@@ -1047,19 +1057,23 @@ void sample_all_kernel(const LT* __restrict__ logits, long* __restrict__ out,
       most = fmaxf(most, max8(x));
     }
     const float M = grow(most);
+    const auto add = [&](auto e) {
 #pragma unroll
-    for (int k = 0; k < ALL_VECS; k++) {
-      float x[8];
-      get8(v[k], x);
+      for (int k = 0; k < ALL_VECS; k++) {
+        float x[8];
+        get8(v[k], x);
 #pragma unroll
-      for (int j = 0; j < 8; j++) sum[k] += __expf(x[j] * invT - M);
-    }
+        for (int j = 0; j < 8; j++) sum[k] += e(x[j]);
+      }
+    };
+    if (far_below(top, invT)) add([&](float l) { return __expf((l - top) * invT); });
+    else add([&](float l) { return __expf(l * invT - M); });
   }
   // the last elements belong to the first owners, behind their vectors
   if (c1 == chunks && 8 * nvec + tid < V) {
     const float x = ldf(p + 8 * nvec + tid);
     const float M = grow(x);
-    sum[0] += __expf(x * invT - M);
+    sum[0] += __expf(far_below(top, invT) ? (x - top) * invT : x * invT - M);
   }
   const float best = block_max<OWNERS>(top, s.red);
   if (best != -INFINITY) sum *= __expf((top - best) * invT);
