@@ -516,7 +516,7 @@ DEVINL T of_lane(T v, int lane) {     // a lane that all agree on
 constexpr int LIKELY = 4096;
 struct RowScratch {
   union {
-    float hist[RWAVES][2 * BINS + 1][64];   // columns private to a lane, as Scratch's
+    float hist[RWAVES][2 * BINS + 2][64];   // columns private to a lane, as Scratch's
     struct {
       float u[LIKELY];
       int id[LIKELY];
@@ -728,13 +728,13 @@ void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
       reinterpret_cast<f32x4*>(&s.hist[i / (bins * 16)][0][0])[i % (bins * 16)] = f32x4{};
     __syncthreads();
   };
-  const auto sum_bins = [&] {         // of all columns, 8 threads a bin
+  const auto sum_bins = [&](int from) {         // of all columns, 8 threads a bin
     __syncthreads();
     float x = 0.f;
 #pragma unroll
     for (int w = 0; w < RWAVES; w++)
 #pragma unroll
-      for (int c = 0; c < 8; c++) x += s.hist[w][tid >> 3][8 * c + (tid & 7)];
+      for (int c = 0; c < 8; c++) x += s.hist[w][from + (tid >> 3)][8 * c + (tid & 7)];
 #pragma unroll
     for (int off = 4; off > 0; off >>= 1) x += __shfl_xor(x, off);
     if ((tid & 7) == 0) s.bin[tid >> 3] = x;
@@ -761,7 +761,7 @@ void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
           s.hist[wid][max(0, min(BINS - 1, (int)(u + URANGE)))][lane] += __expf(u);
       }
     }
-    sum_bins();
+    sum_bins(0);
     // bins from the top; what is left of S is divided as the sample is
     const float some = lane < BINS ? s.bin[BINS - 1 - lane] : 0.f, rest = wave_sum(some);
     const float mass = rest > 0.f ? some * ((S - upper) / rest) : 0.f;
@@ -773,14 +773,15 @@ void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
     float A, m1, m2;
     for (int moved = 0;;) {
       __syncthreads();
-      clear(2 * BINS);
+      clear(2 * BINS + 1);
       const float bottom = hi - 2.f;
       own = 0.f;
       // In pairs, whose columns are read before either is written: half the reads' latency,
-      // which is what the pass takes.  Elements of neither bin go to one behind them.  The bin
-      // by u's floor, which is exact, as kept's comparison is: u - bottom is rounded, and an
-      // element just below a bin's upper border would be in the next, the largest behind them.
-      const int first_bin = (int)bottom * BINS;
+      // which is what the pass takes.  Elements of neither bin go to one below or above, for
+      // asking whether a wave has others takes more: 64 flat rows of 151936 48.2 us so, 44.8 now.
+      // The bin by u's floor, which is exact, as kept's comparison is: u - bottom is rounded, and
+      // an element just below a bin's upper border would be in the next.
+      const int below = (int)bottom * BINS - 1;
       each(bottom, [&](const float* u, int) {
 #pragma unroll
         for (int j = 0; j < 8; j += 2) {
@@ -790,17 +791,16 @@ void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
           for (int i = 0; i < 2; i++) {
             e[i] = __expf(u[j + i]);
             own += u[j + i] >= hi ? e[i] : 0.f;
-            k[i] = u[j + i] >= bottom && u[j + i] < hi
-                       ? (int)floorf(u[j + i] * BINS) - first_bin : 2 * BINS;
+            k[i] = (int)floorf(__builtin_amdgcn_fmed3f(u[j + i] * BINS, below,
+                                                       below + 2.f * BINS + 1.f)) - below;
           }
-          if (!__any(min(k[0], k[1]) < 2 * BINS)) continue;
           float *h0 = &s.hist[wid][k[0]][lane], *h1 = &s.hist[wid][k[1]][lane];
           const float x = *h0 + e[0], y = *h1;
           *h0 = x;
           *h1 = (k[0] == k[1] ? x : y) + e[1];
         }
       });
-      sum_bins();
+      sum_bins(1);
       block_before(own, s.red, A);
       m2 = wave_sum(lane < BINS ? s.bin[lane] : 0.f);
       m1 = wave_sum(lane < BINS ? s.bin[BINS + lane] : 0.f);
@@ -815,7 +815,7 @@ void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
       }
     }
     const int b = A + m1 >= target ? BINS : 0;        // the upper of the two, or the lower
-    if (!b) own += columns(BINS, 2 * BINS);
+    if (!b) own += columns(1 + BINS, 1 + 2 * BINS);
     lowest = hi - (b ? 1.f : 2.f);
     // the maximum itself is of no refined bin
     float above = lowest == -1.f ? 0.f : b ? A : A + m1;
@@ -828,10 +828,10 @@ void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
     above = before;
     fine = BINS - 1 - fine;
     lowest += fine * (1.f / BINS);
-    own += columns(b + fine + 1, b + BINS);
+    own += columns(1 + b + fine + 1, 1 + b + BINS);
     // over-keeping a sliver of the boundary bin changes the nucleus by < 2% of S
     if (s.bin[b + fine] <= 0.02f * S) {
-      own += s.hist[wid][b + fine][lane];
+      own += s.hist[wid][1 + b + fine][lane];
     } else {
       __syncthreads();
       clear(BINS);
@@ -843,7 +843,7 @@ void sample_row_kernel(const LT* __restrict__ logits, long* __restrict__ out,
           if (u[j] >= lo && u[j] < lo + 1.f / BINS)
             s.hist[wid][(int)floorf(u[j] * (BINS * BINS)) - first_bin][lane] += __expf(u[j]);
       });
-      sum_bins();
+      sum_bins(0);
       const float y = lane < BINS ? s.bin[BINS - 1 - lane] : 0.f;
       fine = reach(y, above, target, before);
       fine = fine < 0 || fine >= BINS ? 0 : BINS - 1 - fine;
@@ -1182,16 +1182,21 @@ static void launch_sampler(const torch::Tensor& logits, torch::Tensor& out, floa
   // A CU that has a row to itself takes the time of its VALU and LDS over the whole row: few
   // rows are divided for the first half of it.  A nucleus of few elements, as a language
   // model's, then is a few us; of rows that are flat (normal logits of deviation 1) every
-  // element has to be put into a bin all the same.  us, T = 0.7 and top-p 0.95, one kernel /
-  // divided, logits of a language model | flat:
-  //   bf16 of 151936   1 row 25.5 / 10.6 | 43.8 / 43.5    8 rows 26.0 / 11.2 | 44.4 / 44.0
-  //                    32    28.1 / 12.8 | 44.6 / 46.0    64     28.2 / 14.6 | 44.8 / 49.9
-  //                    128   30.7 / 19.8 | 48.0 / 54.7    512    70.6 / 52.4 | 107 / 125
-  //   bf16, 64 rows    128100 24.5 / 13.7 | 38.1 / 42.3   70000  24.3 / 12.6 | 30.5 / 40.1
-  //   32 bits, 152064  4     31.9 / 12.6 | 47.2 / 44.2    64     47.4 / 18.8 | 57.6 / 53.3
-  //                    512   175 / 91 | 171 / 172
-  // At T = 1, where the nucleus has a thousand elements, 8 rows 38.5 / 30.5, 64 39.3 / 37.5.
-  if (n > 12 && n <= 20 && B <= (half ? 64 : 512) && top_p < 1.) {
+  // element has to be put into a bin all the same.  Taken where neither is slower.  us, top-p 0.95,
+  // one kernel / divided, logits of a language model at T = 0.7, at T = 1, where the nucleus has a
+  // thousand elements | flat ones:
+  //   bf16     151936   1 row  25.1 / 10.7, 37.5 / 28.9 | 43.8 / 38.3
+  //                     64     28.1 / 15.1, 39.9 / 36.8 | 45.1 / 44.8
+  //            128100   32     24.0 / 12.0, 34.3 / 32.6 | 38.2 / 35.5
+  //                     64     25.4 / 13.7, 33.8 / 35.1 | 38.4 / 39.0   not divided
+  //            107000   32     24.6 / 11.6, 33.1 / 30.7 | 35.7 / 34.9
+  //             98312   32     24.3 / 11.6, 32.2 / 30.0 | 34.5 / 35.2   not divided
+  //   32 bits  151936   64     48.5 / 18.9, 52.4 / 42.9 | 58.2 / 49.1
+  //                     512     173 / 92,    170 / 140  |  172 / 166
+  //            107000   16     26.7 / 13.0, 34.2 / 30.1 | 37.4 / 37.1
+  //                     32     30.3 / 13.3, 34.9 / 33.5 | 37.5 / 38.5   not divided
+  const long most = half ? (n >= 19 ? 64 : 32) : (n >= 16 ? 512 : 16);
+  if (n >= 14 && n <= 20 && B <= most) {
     const int slices = (V / 8 + SLICE - 1) / SLICE;
     const int run = n <= 16 ? 32 : 40;          // half of an owner's vectors, n * 4
     const long ahead = (B * slices * 8 + 63) / 64 * 64;
