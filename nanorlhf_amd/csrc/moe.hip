@@ -500,7 +500,9 @@ DEVINL void list_expert(const int* choices, int n, int e, int* list, int* count)
 // ALL: one workgroup has all tokens, and writes the experts' lists too, for which another
 // launch takes 4 us (1, 8 and 16 tokens' experts of 1536 x 2240 29.6 -> 25.9, 58.6 -> 54.6, 68.1
 // -> 64.9 us).  Not of more than 16 tokens, whose rows one CU would have to fetch: 32 tokens
-// 20500 cycles with the lists, 10300 without them where each 16 have a workgroup.
+// 20500 cycles with the lists, 10300 without them where each 16 have a workgroup.  Nor of
+// more than 64 experts, whose lists are too many for four waves: 16 tokens' 8 of 64 of width 1536
+// 36.1 -> 19.5 us, but of 128 44.6 -> 50.1, of 256 60.9 -> 74.6.
 template <int ET, bool ALL>
 __global__ __launch_bounds__(256) void route_mfma_kernel(
     const short* __restrict__ h, const short* __restrict__ wr, const short* __restrict__ bias,
@@ -547,7 +549,7 @@ __global__ __launch_bounds__(256) void route_mfma_kernel(
   }
   __syncthreads();
   constexpr int L = ET == 1 ? 16 : ET == 2 ? 32 : 64, AT_ONCE = 256 / L;
-  __shared__ int picks[ALL ? 16 * (ET > 4 ? 64 : ET * 16) : 1];      // [tokens, top]
+  __shared__ int picks[ALL ? 16 * ET * 16 : 1];      // [tokens, top]
   for (int t = threadIdx.x / L; t < 16; t += AT_ONCE)
     choose<L>(z[0][t], E, top, chosen + (t0 + t) * top, weight + (t0 + t) * top, t0 + t < T,
               ALL ? picks + t * top : nullptr);
@@ -787,11 +789,11 @@ std::vector<torch::Tensor> moe_route(torch::Tensor h, torch::Tensor router, torc
                      (const short*)bias.data_ptr(), chosen.data_ptr<int>(),                    \
                      weight.data_ptr<float>(), lists.data_ptr<int>(), counts.data_ptr<int>(),  \
                      T, (int)W, (int)E, (int)top)
-#define ROUTE(ET)                      \
-  do {                                 \
-    listed = T <= 16;                  \
-    if (listed) ROUTE_OF(ET, true);    \
-    else ROUTE_OF(ET, false);          \
+#define ROUTE(ET)                              \
+  do {                                         \
+    listed = T <= 16 && ET <= 4;               \
+    if (listed) ROUTE_OF(ET, (ET <= 4));       \
+    else ROUTE_OF(ET, false);                  \
   } while (0)
   bool listed = false;
   if (is_bf16(h) && W % 8 == 0 && E <= 256 && (uintptr_t)h.data_ptr() % 16 == 0 &&
