@@ -635,9 +635,10 @@ __global__ __launch_bounds__(512, DP > 128 ? 2 : 4) void chunk_out_split_kernel(
 // in that order.  The tokens of decayed k and of v, whose products need them along a lane, are
 // read transposed (ds_read_tr16_b64), rows 4 * hi + (0 .. 3) and 16 on.
 // Bound by instructions of all kinds, some 850 to a wave's step (SiLU, rotation, the division
-// into hi and lo of q, twice k and S): a CU with two workgroups takes 7.9 us for a step of both,
-// with one 4.9.  Hence no exec branches around loads, offsets of 32 bits from a step's first
-// token, and no exact quotient or root in the norm (9.5 and 6.0 us with those).
+// into hi and lo of q, twice k and S).  Hence no exec branches around loads and offsets of 32 bits
+// from a step's first token.  The norm's exact quotient and root, as decoding has them, take 2 to 3
+// % (16 sequences of 696 tokens on average, 12 heads, 136 -> 139 us): an approximate root is
+// not-a-number where the squares' sum is infinite or below the smallest normal number.
 // 8 sequences of 2404 tokens on average, 12 heads of 128, norm and gate in it: 200 us, by chunks
 // 434 (133 + 112 + 187 us at 16300 tokens; the states of 305 chunks are 240 MB); 16 of 696 136
 // and 234; 4 of 499 48 and 52; of 32 heads, 8 of 2048, 412 to 435 and 925.
@@ -789,7 +790,6 @@ __global__ __launch_bounds__(512, 4) void linear_walk_kernel(
   };
 
   const bool col_ok = e0 + 4 * hi < s.V;
-  const float invV = 1.f / (float)s.V;
   int at = 0, len = ch.len[c];
   long row = ch.row[c];
   float decay = 1.f;
@@ -956,9 +956,7 @@ __global__ __launch_bounds__(512, 4) void linear_walk_kernel(
           float ss = 0.f;
 #pragma unroll
           for (int y = 0; y < CT; y++) ss += red[y][i];
-          ss = ss * invV + eps;                 // its inverse root, with a step of Newton's
-          float inv = __builtin_amdgcn_rsqf(ss);
-          inv = inv * (1.5f - 0.5f * ss * inv * inv);
+          const float inv = 1.f / sqrtf(ss / (float)s.V + eps);
 #pragma unroll
           for (int j = 0; j < 4; j++) x[j] *= inv * silu_fast(bf2f(gr[r][j]));
         }
