@@ -1115,6 +1115,44 @@ static void check_ints(const torch::Tensor& t, long n) {
   TORCH_CHECK(t.is_cuda() && t.scalar_type() == torch::kInt && t.is_contiguous() && t.numel() == n);
 }
 
+// How many of n chunks of B sequences make a segment; 0: chunk by chunk.  Both counts are known
+// here, but not how long each sequence is, so that the lines lie where neither even sequences nor
+// one long one among short ones is slower than by chunks.  A workgroup's steps follow each other:
+// segments stay near the time that all of them take (`work` chunks on 512 workgroups, two to a CU),
+// for one long sequence takes its segment's steps however many CUs are idle (200 of 20 tokens and
+// one of 2560, 12 heads: 645 us with 3 chunks, 621 with 4, 790 with 24, by chunks 725).  Up to that
+// as many as leave one round, if three quarters of a segment are lost at each sequence's end (half
+// of one is, most times): 16 sequences of 696 on average, 12 heads, 147 us with 3, 140 with 6; 8 of
+// 2139 198 with 3, 170 with 8.  Where these are more rounds, 6, or of long sequences the number
+// with which the rounds are through soonest: 32 heads, 190 chunks of one 281 with 6, 268 with 12.
+//
+// By chunks / so, us, heads of 128: with a CU to each workgroup, 12 heads, one of 1004 tokens
+// 37 / 32; without, but no more than two, which leaves no round to save, one of 2028 (384) 48 / 46,
+// 32 heads, one of 1004 (512) 51 / 55; 12 heads, one of 2693 (516) 71 / 58, of 6124 113 / 82.  Of
+// fewer than 2.5 chunks to a sequence there is little to save, and only many of them save it: 32
+// heads, 48 of 108 tokens 604 / 378, 33 of 100 (32 of 40) 291 / 261, but 12 heads 109 / 118.  Heads
+// of 64, whose states are a quarter: 16 heads, one of 1004 22 / 27, of 3052 42 / 38.  Of 32, 16 heads,
+// 16 of 172 tokens 28 / 36, 32 of 40 and one of 4096 57 / 58 to 62: by chunks.
+long linear_attn_segment(long n, long B, long H, long D, long V) {
+  if (D <= 32 || D > 128) return 0;
+  const long columns = V <= 64 ? 64 : 128, across = H * ((V + columns - 1) / columns);
+  const long work = n * across;
+  if (2 * n < 5 * B) return D > 64 && 4 * n >= 5 * B && work >= 2048 ? 4 : 0;
+  if (D <= 64 ? work < 640 : work <= 512 && (work < 144 || work + B * across > 256)) return 0;
+  auto groups = [&](long i) { return across * (4 * n + 3 * B * (i - 1)) / (4 * i); };
+  const long most = std::min(12L, (5 * work + 2047) / 2048);
+  long per = 1;
+  while (per < most && groups(per) > 512) per++;
+  if (groups(per) > 512) {
+    per = std::min(per, 6L);
+    auto cost = [&](long i) { return (groups(i) + 511) / 512 * (2 * i + 1); };
+    if (n >= 24 * B)
+      for (long i = 6; i <= 24; i++)
+        if (cost(i) < cost(per)) per = i;
+  }
+  return per;
+}
+
 // o [T, H * V] (any row stride) <- portions described by chunks (int32 [3, n]:
 // sequence, first row, length), first (int32 [B + 1]), slots and fresh (int32
 // [B]).  With a gate, each head's output is divided by its root mean square and
@@ -1156,27 +1194,9 @@ void linear_attn_chunked(torch::Tensor q, torch::Tensor k, torch::Tensor v, torc
     const short* gp = gate.has_value() ? (const short*)gate->data_ptr() : nullptr;
     const long ldg = gate.has_value() ? gate->stride(0) : 0;
     auto short_rows = [](long ld) { return ld >= 0 && ld < 1L << 24; };   // a step's offsets: 32 bits
-    // Of a few workgroups the steps of 32 tokens follow each other where a chunk has one of 64: 36
-    // tokens of 12 heads 23.0 us by segments, 21.6 by chunks; 536 (108 workgroups) 29.2 and 28.8, 4
-    // times 499 47.9 and 52.
-    const long across = (long)s.H * ((s.V + (s.V <= 64 ? 63 : 127)) / (s.V <= 64 ? 64 : 128));
-    if (vec && DP <= 128 && n * across >= 128 && short_rows(s.ld) && short_rows(ldg) &&
-        short_rows(o.stride(0)) && s.rdims < 1 << 24) {
-      // As many chunks to a segment as leave each CU two workgroups, which is one round, if three
-      // quarters of a segment are lost at each sequence's end (half of one is, most times).  16
-      // sequences of 696 tokens on average (183 chunks), 12 heads: 5 chunks (some 540 workgroups)
-      // 160 us, 6 136; 8 of 2404 (305 chunks) 240 with 8, 200 with 9.  Where 16 chunks are more
-      // than a round and sequences long, the number with which the rounds are through soonest: 32
-      // heads, 8 of 2048 tokens 468 with 16 (two rounds), 412 to 435 so; but 16 of 464 tokens
-      // of 12 heads, chosen so, 129 and not 107.
-      auto groups = [&](long i) { return across * (4 * n + 3 * B * (i - 1)) / (4 * i); };
-      int per = 1;
-      while (per < 16 && groups(per) > 512) per++;
-      if (groups(per) > 512 && n >= 24 * B) {
-        auto cost = [&](long i) { return (groups(i) + 511) / 512 * (2 * i + 1); };
-        for (int i = 8; i <= 24; i++)
-          if (cost(i) < cost(per)) per = i;
-      }
+    const int per = linear_attn_segment(n, B, s.H, s.D, s.V);
+    if (vec && per && short_rows(s.ld) && short_rows(ldg) && short_rows(o.stride(0)) &&
+        s.rdims < 1 << 24) {
       const long G = n / per + B;
       auto parts = torch::empty({G, s.H, s.V, DP}, state.options());
       auto decays = torch::empty({G, s.H}, state.options());
@@ -1198,8 +1218,7 @@ void linear_attn_chunked(torch::Tensor q, torch::Tensor k, torch::Tensor v, torc
                        (float)eps, (short*)o.data_ptr(), (long)o.stride(0));                    \
   } while (0)
 #define WALK_V(DD) do { if (s.V <= 64) WALK(DD, 64); else WALK(DD, 128); } while (0)
-      if (DP == 32) WALK_V(32);
-      else if (DP == 64) WALK_V(64);
+      if (DP == 64) WALK_V(64);
       else WALK_V(128);
 #undef WALK_V
 #undef WALK

@@ -32,6 +32,7 @@ void paged_attn_plain(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch
                       torch::Tensor positions, torch::Tensor bt, torch::Tensor out, double scale,
                       long size, long keep, OptTensor uncs);
 // linear_attn.hip
+long linear_attn_segment(long n, long B, long H, long D, long V);
 void linear_attn_chunked(torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor pw,
                          OptTensor cs, bool interleaved, bool silu, double kscale,
                          torch::Tensor chunks, torch::Tensor first, torch::Tensor slots,
@@ -118,6 +119,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_attn_varlen", &paged_attn_varlen);
   m.def("paged_attn_plain", &paged_attn_plain);
   m.def("linear_attn_chunked", &linear_attn_chunked);
+  m.def("linear_attn_segment", &linear_attn_segment);
   m.def("linear_attn_decode", &linear_attn_decode);
   m.def("residual_group_norm", &residual_group_norm);
   m.def("gated_norm", &gated_norm);
