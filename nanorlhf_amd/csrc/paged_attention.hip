@@ -233,6 +233,13 @@ void paged_varlen_kernel(VarlenArgs a) {
     return wave_active && kv0 <= wpos_hi &&
            !(wpos_lo - (kv0 + KV - 1) >= a.size && kv0 >= a.keep);
   };
+  // ... and some of every wave's that has rows?  The same for all waves, and so are the barriers
+  // that follow from it.
+  const int all_lo = start + min(r0 + 96, R - 1) / G, all_hi = start + min(r0 + 31, R - 1) / G;
+  auto visible_to_all = [&](int it) {
+    const int kv0 = tile_of(it) * KV;
+    return kv0 <= all_hi && !(all_lo - (kv0 + KV - 1) >= a.size && kv0 >= a.keep);
+  };
   // A fragment's address is that of its tile's first, which two registers keep, with a
   // constant exchanged (xor) into the chunk and another added.
   typedef __attribute__((address_space(3))) const char* lds_bytes;
@@ -340,6 +347,7 @@ void paged_varlen_kernel(VarlenArgs a) {
   auto both = [&](int it, int buf, f32x16* cur, float top, f32x16* next, float& ntop) INLINE {
     bf16x8p first[2 * AHEAD];
     arrive(it, buf, first);
+    if (!wave_active) return;
     const float alpha = settle(tile_of(it) * KV, cur, top);
     __builtin_amdgcn_sched_barrier(0);
     scores(buf ^ 1, next, first);
@@ -356,7 +364,7 @@ void paged_varlen_kernel(VarlenArgs a) {
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  f32x16 s0[2], s1[2];
+  f32x16 s0[2] = {}, s1[2];
   float top0 = 0.f, top1 = 0.f;
   auto one = [&](int it, int buf) INLINE {
     bf16x8p first[2 * AHEAD];
@@ -390,8 +398,8 @@ void paged_varlen_kernel(VarlenArgs a) {
     }
     for (int it = 0; it < ntiles; it += 2) {
       // (a loop of its own, or the scores change registers in every round)
-      for (; it + 2 < ntiles && visible(tile_of(it) * KV) && visible(tile_of(it + 1) * KV) &&
-             visible(tile_of(it + 2) * KV); it += 2) {
+      for (; it + 2 < ntiles && visible_to_all(it) && visible_to_all(it + 1) &&
+             visible_to_all(it + 2); it += 2) {
         both(it, 0, s0, top0, s1, top1);
         both(it + 1, 1, s1, top1, s0, top0);
       }
