@@ -95,12 +95,14 @@ void paged_varlen_kernel(VarlenArgs a) {
       if (PAIRS && a.B == 1 && n > 256 && n <= 512 && a.size >= a.seq_lens[0]) {
         // One sequence without a window, whose workgroups are more than the CUs, but at most
         // twice as many: some CUs run two, which are the first that a chiplet is given and
-        // those after its 32nd.  These are the shortest rows, two neighbours in length each;
-        // the longest, alone, come first among the others.  2708 rows of 12 heads after 0, 2708
-        // and 5416 (264 workgroups): 60, 115 and 165 us; long and short in turn 65, 134 and 195.
+        // those after its 32nd.  These are the shortest rows, the longest of them with the
+        // shortest and so on; those that are longer, alone, come first among the others.  2708
+        // rows of 12 heads after 0, 2708 and 5416 (264 workgroups): 60, 115 and 165 us; long and
+        // short in turn 65, 134 and 195.  1500 rows of 40 heads over 8 (472): 50 us, and
+        // with two neighbours in length on such a CU 57, long and short in turn 51.
         const int over = max(all - 32, 0);
-        int rank = mine < over ? 2 * mine + 1
-                   : mine >= 32 ? 2 * (mine - 32) : 2 * over + (all - over - 1 - mine);
+        int rank = mine < over ? 2 * over - 1 - mine
+                   : mine >= 32 ? mine - 32 : 2 * over + (all - over - 1 - mine);
         for (tile = 0;; tile++) {    // the rank'th shortest: a tile's heads are `tiles` ids apart
           const int off = (tile - first % a.tiles + a.tiles) % a.tiles;
           const int same = all / a.tiles + (off < all % a.tiles);
