@@ -13,15 +13,20 @@
 // d) is 16 bytes; the keys are read in the order that leaves a lane the scores
 // of those 8.
 //
-// What bounds it: of the portions that fill the chip once, a wave's instructions.  A wave
-// alone on its SIMD issues one in 5 cycles, whichever unit it is for, so the matrix products
-// of a tile (32, 1024 cycles) are hidden only if what else it takes (some 450 instructions)
-// lies between them: a tile's scores are computed under the exponentials of the tile before,
-// an LDS read and six VALU instructions to a product, which leaves 2750 cycles of 3330 a tile.
-// Of more workgroups, products, VALU and LDS reads (as many cycles as the products) together.
-// 12 heads of 128, one tile after the other / now, us: 128 rows over 8064 keys 175 / 145;
-// 2048 tokens, 8 times 180 / 166 over a workspace, over pages of 2 heads 178 / 162; 16384
-// 1069 / 941 and 873 / 817; a window of 1024 over 8 of 693 to 3380 137 / 130.
+// What bounds it: of the portions that fill the chip once, a wave's instructions.  A wave alone on
+// its SIMD issues one at a time, whichever unit it is for, so the matrix products of a tile (32)
+// are hidden only if what else it takes (some 450 instructions) lies between them: a tile's scores
+// are computed under the exponentials of the tile before, an LDS read and six VALU instructions to
+// a product, which leaves 1.14 us of 1.38 a tile.  Of more workgroups, products, VALU and LDS reads
+// together.  12 heads of 128, one tile after the other / now, us: 128 rows over 8064 keys 175 / 145;
+// 2048 tokens, 8 times 178 / 162 over a workspace, over pages of 2 heads 177 / 160; 16384 1062 / 950
+// and 862 / 805; a window of 1024 over 8 of 693 to 3380 140 / 130.
+//
+// It takes registers for a second tile's scores, which heads of 128 have: no more than two
+// workgroups fit a CU either way.  Narrower ones have up to six, of which three would be left, and
+// are overlapped only where there are no more workgroups than CUs (12 heads of 64, 1500 tokens 32.0
+// / 27.8, but 40 sequences of 400 in a window of 100 42.9 / 50.5), or, with one width of 128, twice
+// as many (16 heads of 128 and 64, 2000 tokens 50 / 40, 16 times 300 20.7 / 26.9).
 //
 // The same kernel runs over a workspace (LIN) instead of pages: keys [rows, Hkv,
 // DK] and transposed values [Hkv * DV, rows] of whole contexts laid out one
@@ -72,12 +77,17 @@ DEVINL int half_swz(int d) { return (d >> 3) & 1; }
 
 #define INLINE __attribute__((always_inline))
 
+// From so many tiles on a tile's scores are computed under the exponentials of the one before:
+// of fewer, what that takes to start outweighs it (64 sequences of 200 tokens, 12 heads over 2 of
+// 128, 40.7 us, overlapped 43.2; 16 of 300 31.2 and 31.0).
+constexpr int OVERLAPPED = 6;
+
 DEVINL float other_half(float x, int hi) {
   auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(hi ? r[0] : r[1]);
 }
 
-template <int DK, int DV, bool LIN>
+template <int DK, int DV, bool LIN, bool PIPE>
 __global__ __launch_bounds__(256, (DK > 128 || DV > 128) ? 1 : 2)
 void paged_varlen_kernel(VarlenArgs a) {
   constexpr int NDS = DK / 16, NDT = DV / 32, KV = 64;
@@ -384,12 +394,14 @@ void paged_varlen_kernel(VarlenArgs a) {
   key_pages(tile_of(0));
   value_pages(tile_of(0));
   stage_keys(tile_of(0), 0);
-  if constexpr (PAIRS) {
+  stage_values(tile_of(0), 0);
+  bool piped = false;
+  if constexpr (PIPE) piped = ntiles >= OVERLAPPED;
+  if (piped) {
     key_pages(tile_of(1));
-    wait_loads<0>();
+    wait_loads<NV>();         // the keys
     __syncthreads();
-    if (ntiles > 1) stage_keys(tile_of(1), 1);
-    stage_values(tile_of(0), 0);
+    stage_keys(tile_of(1), 1);
     key_pages(tile_of(2));
     value_pages(tile_of(1));
     if (visible(tile_of(0) * KV)) {
@@ -409,9 +421,6 @@ void paged_varlen_kernel(VarlenArgs a) {
       if (it + 1 < ntiles) one(it + 1, 1);
     }
   } else {
-    // Wider rows leave no registers for two tiles' scores: these would pass through the
-    // accumulation registers (1500 rows of 8 heads over 1 of 256 100 us, this way 85).
-    stage_values(tile_of(0), 0);
     for (int it = 0; it < ntiles; it++) {
       const int buf = it & 1, kv0 = tile_of(it) * KV;
       wait_loads<0>();
@@ -564,8 +573,17 @@ static void launch_varlen(VarlenArgs a, int DK, int DV, long max_rows, hipStream
   a.tiles = (max_rows + 127) / 128;
   if (!a.tiles) return;
   const dim3 grid((unsigned)((long)a.tiles * a.B * a.Hkv));
-#define LAUNCH(KK, VV) \
-  hipLaunchKernelGGL((paged_varlen_kernel<KK, VV, LIN>), grid, dim3(256), 0, stream, a)
+  const long longest = LIN ? a.ldv : 16L * a.maxP;      // a context, at most
+  const bool pipe = longest > 64 * (OVERLAPPED - 1) &&
+                    ((DK == 128 && DV == 128) || grid.x <= (DK + DV > 128 ? 512 : 256));
+#define LAUNCH(KK, VV)                                                                           \
+  do {                                                                                           \
+    if (pipe && KK <= 128 && VV <= 128)                                                          \
+      hipLaunchKernelGGL((paged_varlen_kernel<KK, VV, LIN, (KK <= 128 && VV <= 128)>), grid,     \
+                         dim3(256), 0, stream, a);                                               \
+    else                                                                                         \
+      hipLaunchKernelGGL((paged_varlen_kernel<KK, VV, LIN, false>), grid, dim3(256), 0, stream, a); \
+  } while (0)
 #define LAUNCH_V(KK)                                              \
   do {                                                            \
     if (DV == 32) LAUNCH(KK, 32);                                 \
