@@ -16,6 +16,8 @@
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "checks.h"
 
@@ -85,15 +87,17 @@ struct LatentArgs {
 // many parts of at most `per` pages as it takes, `per` being about the least (to a sixteenth)
 // with which all parts are at most the budget.  A wave's lane looks at four sequences; all waves
 // come to the same.
-struct LatentPart { int seq, z, per, parts; };
+struct LatentPart { int seq, z, per, parts, length; };
 DEVINL bool latent_part(const LatentArgs& a, int w, LatentPart& out) {
   const int lane = threadIdx.x & 63;
-  int pages[4];
+  int lens[4], pages[4];
   float sum = 0.f, longest = 0.f;
 #pragma unroll
+  for (int i = 0; i < 4; i++) lens[i] = a.seq_lens[min(4 * lane + i, a.B - 1)];
+#pragma unroll
   for (int i = 0; i < 4; i++) {
-    const int b = 4 * lane + i;
-    pages[i] = b < a.B ? max((a.seq_lens[b] - 1) / 16 + 1, 1) : 0;
+    asm volatile("" : "+v"(lens[i]));        // asked for together
+    pages[i] = 4 * lane + i < a.B ? max((lens[i] - 1) / 16 + 1, 1) : 0;
   }
 #pragma unroll
   for (int i = 0; i < 4; i++) {
@@ -126,27 +130,35 @@ DEVINL bool latent_part(const LatentArgs& a, int w, LatentPart& out) {
     c[i] = parts(pages[i], per, 1.f / (float)per);
     mine += c[i];
   }
-  int upto = mine;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int x = __shfl_up(upto, off);
-    if (lane >= off) upto += x;
+  int upto = mine;           // sums over the lanes before: row_shr:1, 2, 4, 8, then the rows'
+  auto shift = [&](auto ctrl) {
+    upto += __builtin_amdgcn_update_dpp(0, upto, decltype(ctrl)::value, 0xf, 0xf, true);
+  };
+  shift(std::integral_constant<int, 0x111>{});
+  shift(std::integral_constant<int, 0x112>{});
+  shift(std::integral_constant<int, 0x114>{});
+  shift(std::integral_constant<int, 0x118>{});
+  {
+    const int r0 = __builtin_amdgcn_readlane(upto, 15), r1 = r0 + __builtin_amdgcn_readlane(upto, 31);
+    const int r2 = r1 + __builtin_amdgcn_readlane(upto, 47), r = lane >> 4;
+    upto += r == 0 ? 0 : r == 1 ? r0 : r == 2 ? r1 : r2;
   }
   const unsigned long long hit = __ballot(w >= upto - mine && w < upto);
   if (!hit) return false;
   const int at = __ffsll(hit) - 1;
-  int z = w - __builtin_amdgcn_readlane(upto - mine, at), seq = 4 * at, n = 0;
+  int z = w - __builtin_amdgcn_readlane(upto - mine, at), seq = 4 * at, n = 0, length = 0;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int here = __builtin_amdgcn_readlane(c[i], at);
     if (n == 0 && z < here) {
       n = here;
       seq = 4 * at + i;
+      length = __builtin_amdgcn_readlane(lens[i], at);
     } else if (n == 0) {
       z -= here;
     }
   }
-  out = {seq, z, per, n};
+  out = {seq, z, per, n, length};
   return true;
 }
 
@@ -175,7 +187,7 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
   // pages of each wave; at the end its sums, 16 x RP floats
   __shared__ __attribute__((aligned(1024))) short buf[NW][NBUF * PAGE];
   __shared__ float Lm[NW][16], Ls[NW][16];
-  int seq = blockIdx.y, z = blockIdx.z, splits = a.splits, per = 0;
+  int seq = blockIdx.y, z = blockIdx.z, splits = a.splits, per = 0, length = 0;
   if constexpr (ALL) {
     LatentPart mine;
     if (!latent_part(a, blockIdx.y, mine)) return;
@@ -183,13 +195,14 @@ __global__ __launch_bounds__(256) void latent_attn_kernel(LatentArgs a) {
     z = mine.z;
     splits = mine.parts;
     per = mine.per;
+    length = mine.length;
     if (z == 0 && blockIdx.x == 0 && threadIdx.x == 0) a.plan[seq] = int2{(int)blockIdx.y, splits};
   }
-  const int t0 = a.cu ? a.cu[seq] : seq;
-  const int nq = a.cu ? a.cu[seq + 1] - t0 : 1;
+  const int t0 = !ALL && a.cu ? a.cu[seq] : seq;
+  const int nq = !ALL && a.cu ? a.cu[seq + 1] - t0 : 1;
   const int R = nq * a.H, r0 = blockIdx.x * 16;
   if (r0 >= R) return;
-  const int start = a.seq_lens[seq] - nq;
+  const int start = (ALL ? length : a.seq_lens[seq]) - nq;
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lo = lane & 15, hi = lane >> 4;
   const int row = min(r0 + lo, R - 1);
@@ -385,7 +398,8 @@ __global__ __launch_bounds__(128) void latent_merge_kernel(LatentArgs a, int RP,
   float share = f / wave_sum(w.y * f);
   asm volatile("" : "+v"(share));         // of every lane, those too that have no column below
   // Part i's share of the result.  Of many parts through LDS: 16 x 8000 latents, in 16 parts, took
-  // 48.5 us so and 51.3 with a lane read for each.
+  // 48.5 us so and 51.3 with a lane read for each; 8 x 4000 of 256 by pages, in some 28, the merge
+  // alone 3.9 and 12.0.
   __shared__ float shares[MOST ? 1 : 64];
   if constexpr (MOST == 0) {
     if (threadIdx.x < 64) shares[z] = share;
@@ -615,28 +629,25 @@ torch::Tensor latent_attn(torch::Tensor qa, torch::Tensor cache, c10::optional<t
   a.scale = scale;
   // One workgroup per CU, none with less than two pages for every wave, all sequences with as
   // many parts.  Single tokens of long and uneven contexts divide all pages instead, which leaves
-  // no CU idle and no context's parts longer than others; that takes a workgroup 1 us to find
-  // out, and parts that are not full.  us, as many parts / all pages, of rows x mean of 512, lengths
-  // a third to five thirds of it: 32 x 8000 69.5 / 58.9, 64 x 4000 73.5 / 65.0, 100 x 2600 83.7 /
-  // 70.3, but 128 x 2000 76.2 / 77.6, 16 x 8000 48.4 / 48.2, 128 x 700 42.8 / 42.2, 64 x 1000 of
-  // 256 27.0 / 27.9.
+  // no CU idle and no context's parts longer than others.  How long they are is not known here, but
+  // how many pages the table holds.  us, as many parts / all pages, of rows x mean of 512, lengths a
+  // third to five thirds of it: 32 x 8000 64.6 / 55.4, 64 x 4000 64.0 / 58.5, 100 x 2600 74.2 / 56.8;
+  // 100 of 60 and two of 16000 203 / 26, 48 of which 8 have 5000 41.1 / 40.9.  To find out takes a
+  // workgroup 2 us and the merge 1, which short contexts in a wide table do not get back (2048
+  // pages a row: 64 x 1000 23.9 / 24.4, 64 x 500 17.8 / 19.2, 32 x 500 12.4 / 15.5, 16 x 500 11.5 /
+  // 14.7): up to 16 rows, which have 16 parts each anyway, only with 65536 pages.
   const long most = std::max<long>(1, bt.size(1) / 8), budget = 256 / units_x;
   a.splits = (int)std::min<long>(std::min<long>(most, 64), std::max<long>(1, 256 / units));
   a.B = B;
-  a.budget = !cu.has_value() && B > 1 && 5 * B <= 2 * budget && B * units_x * bt.size(1) >= 16384
-                 ? (int)budget : 0;
-  torch::Tensor part, ms, plan;
+  a.budget = !cu.has_value() && B > 1 && 5 * B <= 2 * budget &&
+                     B * units_x * bt.size(1) >= (B <= 16 ? 65536 : 16384) ? (int)budget : 0;
+  torch::Tensor work;      // one allocation: the calls of small batches wait for the host
   if (a.splits > 1 || a.budget) {
-    auto f = qa.options().dtype(torch::kFloat32);
     const long n = a.budget ? budget * units_x : units * a.splits;
-    part = torch::empty({n, 16, RP}, f);
-    ms = torch::empty({n, 16, 2}, f);
-    a.part = part.data_ptr<float>();
-    a.ms = ms.data_ptr<float>();
-  }
-  if (a.budget) {
-    plan = torch::empty({B, 2}, qa.options().dtype(torch::kInt));
-    a.plan = (int2*)plan.data_ptr<int>();
+    work = torch::empty({n * 16 * (RP + 2) + 2 * B}, qa.options().dtype(torch::kFloat32));
+    a.part = work.data_ptr<float>();
+    a.ms = a.part + n * 16 * RP;
+    a.plan = (int2*)(a.ms + n * 32);
   }
   auto stream = at::hip::getCurrentHIPStream();
   TORCH_CHECK(B <= 65535, "too many sequences in a batch");
@@ -657,7 +668,7 @@ torch::Tensor latent_attn(torch::Tensor qa, torch::Tensor cache, c10::optional<t
 #define MERGE(MOST, ALL)                                                                      \
   hipLaunchKernelGGL((latent_merge_kernel<MOST, ALL>), dim3(units, 16), dim3(128), 0, stream, a,     \
                      (int)RP, (int)units_x)
-  if (a.budget) MERGE(8, true);
+  if (a.budget) MERGE(0, true);
   else if (a.splits > 4) MERGE(0, false);
   else if (a.splits > 1) MERGE(4, false);
 #undef MERGE
