@@ -639,9 +639,8 @@ __global__ __launch_bounds__(512, DP > 128 ? 2 : 4) void chunk_out_split_kernel(
 // from a step's first token.  The norm's exact quotient and root, as decoding has them, take 2 to 3
 // % (16 sequences of 696 tokens on average, 12 heads, 136 -> 139 us): an approximate root is
 // not-a-number where the squares' sum is infinite or below the smallest normal number.
-// 8 sequences of 2404 tokens on average, 12 heads of 128, norm and gate in it: 200 us, by chunks
-// 434 (133 + 112 + 187 us at 16300 tokens; the states of 305 chunks are 240 MB); 16 of 696 136
-// and 234; 4 of 499 48 and 52; of 32 heads, 8 of 2048, 412 to 435 and 925.
+// 8 sequences of 2139 tokens on average, 12 heads of 128, norm and gate in it: 170 us, by chunks 389
+// (the states of 272 chunks are 214 MB); 16 of 696 140 and 233; of 32 heads, 8 of 2139, 448 and 1036.
 constexpr int STEP = 32;
 
 // Sequence b's segments have the numbers first[b] / per + b on, some of which stay unused.
