@@ -797,6 +797,11 @@ __global__ __launch_bounds__(512, 4) void linear_walk_kernel(
   for (bool more = true; more;) {
     const long t0 = row + at;
     const int n = min(STEP, len - at);
+    // Tokens up to where k decays: the step's end, whose state the next step's outputs need; without
+    // outputs the chunk's, at whose first step S decays by all of it and at the others by pws[0], 1.
+    // With half as many rounded decays the state's error is that by chunks: 16 heads of 96 that keep
+    // up to 4096 tokens, 14578 tokens, 2.48e-6 against 64 bits, by steps 2.65e-6; the time is the same.
+    const int until = OUT ? n : len - at, decayed = OUT || at == 0 ? until : 0;
     clear(n);
     if (mine) {
       float a[4], b[4];
@@ -815,7 +820,7 @@ __global__ __launch_bounds__(512, 4) void linear_walk_kernel(
         put(&kt[0][qj * QS + ea], &kt[1][qj * QS + ea], a);
         put(&kt[0][qj * QS + eb], &kt[1][qj * QS + eb], b);
       }
-      const float m = pws[max(n - 1 - qj, 0)];   // tokens past n are zero
+      const float m = pws[max(until - 1 - qj, 0)];   // tokens past n are zero
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         a[j] *= m;
@@ -923,7 +928,7 @@ __global__ __launch_bounds__(512, 4) void linear_walk_kernel(
       }
     }
     if (!OUT || more) {                         // the state behind it
-      const float f = pws[n];
+      const float f = pws[decayed];
 #pragma unroll
       for (int dt = 0; dt < DT; dt++) {
         S[dt] *= f;
