@@ -16,7 +16,7 @@ from nanorlhf_amd.rewards import ModelReward
 ON_GPU = torch.cuda.is_available()
 config = RLOOConfig(
     exp_name="rloo_default", output_dir="runs/rloo", seed=2434,
-    # BASELINE config #4 runs this at qwen2.5-7b, DP=8 (torchrun, one rank/GPU)
+    # larger: qwen2.5-7b, DP=8 (torchrun, one rank/GPU)
     model_preset="qwen2.5-1.5b" if ON_GPU else "tiny",
     reward_preset="rm-large" if ON_GPU else "rm-tiny",
     dtype="bfloat16" if ON_GPU else "float32",

@@ -1,11 +1,10 @@
 """Pure algorithm math shared by every trainer.
 
 Each function is a semantics-preserving re-implementation of the math the
-reference inlines inside its six ``<algo>_trainer.py`` ``train()`` bodies
-(see SURVEY.md §2.1/§3.1).  Reference call sites cited per function so the
-judge can check parity.  Everything here is device-agnostic torch; the hot
-token-level pieces have HIP-fused twins in ``nanorlhf_amd.ops`` which these
-functions dispatch to on GPU where it pays.
+reference inlines inside its six ``<algo>_trainer.py`` ``train()`` bodies,
+whose call sites each function cites.  Everything here is device-agnostic
+torch; the hot token-level pieces have HIP-fused twins in ``nanorlhf_amd.ops``
+which these functions dispatch to on GPU where it pays.
 """
 from __future__ import annotations
 

@@ -7,7 +7,7 @@ KL-shaped sequence reward (:564-585), pick the BEST per prompt (torch.max
 Reference quirk (raft_trainer.py:588): the snapshot OVERWRITES the argmax
 with torch.randint, making best-of-K selection dead code.  We default to the
 intended argmax; set cfg.random_keep_quirk=True to reproduce the reference
-exactly (SURVEY.md "quirks to preserve vs fix")."""
+exactly."""
 from __future__ import annotations
 
 from dataclasses import dataclass

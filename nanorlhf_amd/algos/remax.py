@@ -16,7 +16,7 @@ from .trainer import AlgoSpec, Rollout, RLHFTrainer, TrainData
 
 @dataclass
 class RemaxConfig(RLHFConfig):
-    sample_n: int = 1  # n=1 + greedy baseline (SURVEY §2.1 ReMax row)
+    sample_n: int = 1  # n=1 + greedy baseline
 
 
 class ReMax(AlgoSpec):

@@ -2,8 +2,8 @@
 
 One engine; each algorithm (GRPO/PPO/RLOO/ReMax/RAFT/REINFORCE) reduces to
 an AlgoSpec plug-in providing its advantage construction and loss — exactly
-the delta SURVEY.md §2.1 shows between the reference's six forked 700-800
-line trainer files.  Per-update pipeline mirrors the reference's train()
+the difference between the reference's six forked 700-800 line
+trainer files.  Per-update pipeline mirrors the reference's train()
 (GRPO/grpo_trainer.py:406-778):
 
   rollout (in-process sampler) → reward → [algo row selection] → scoring
@@ -608,8 +608,7 @@ class RLHFTrainer:
                     upd_stats = self._update(td)
             except Exception:
                 # crash recovery: persist what we have before surfacing the
-                # error (the reference loses the run past the last save —
-                # SURVEY §5 "Failure detection: none")
+                # error (the reference loses the run past the last save)
                 if self.global_step > 0:
                     self.save()
                 raise
@@ -684,7 +683,7 @@ class RLHFTrainer:
     def load_checkpoint(self, ckpt_dir: str):
         """Resume policy adapter + optimizer + RNG from a checkpoint dir
         (an improvement over the reference, whose custom train() never wires
-        resume_from_checkpoint — SURVEY.md §5 Checkpoint/resume)."""
+        resume_from_checkpoint)."""
         import json
         import os
         from ..utils.checkpoint import CheckpointManager, load_rng_state

@@ -100,7 +100,7 @@ class RLHFConfig:
     # synthetic bench is balanced).  When on, whole sample-groups are
     # re-assigned across ranks after reward so per-rank token totals are
     # near-equal (LPT greedy, deterministic).  Off by default: it is an
-    # opt-in for real-data DP runs (SURVEY §7 hard part (d)).
+    # opt-in for real-data DP runs.
     dp_rebalance_rollout: bool = False
 
     # ---- eval (r1 mode: greedy accuracy pass, grpo_r1_trainer.py:824-825) ----

@@ -1,4 +1,4 @@
-// Fused masked-moments + whitening (trl masked_whiten,
+// Fused masked-moments + whitening (trl's masked_whiten,
 // GRPO/grpo_trainer.py:607,619).  fp32 advantage tensors [N] with a 0/1
 // mask: pass 1 reduces per-block (sum, sumsq, count) partials; the host
 // combines the tiny partial array; pass 2 applies (x-mean)*invstd (+mean).

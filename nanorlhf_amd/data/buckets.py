@@ -5,7 +5,7 @@ Re-implements the reference's `_create_batches` packer
 greedily while max_len_in_bucket * count <= token_budget.  Used for both
 the scoring pass (rollout budget) and the update pass (train budget) — it is
 a throughput feature (pad-free GEMMs), kept even though 288 GB HBM removes
-the memory pressure that motivated it on A100-40G (SURVEY.md §5)."""
+the memory pressure that motivated it on A100-40G."""
 from __future__ import annotations
 
 

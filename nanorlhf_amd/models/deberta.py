@@ -1,9 +1,8 @@
 """DeBERTa-v2/v3 sequence-classification reward model (own implementation).
 
 The reference's reward model is microsoft/deberta-v3-large loaded through
-AutoModelForSequenceClassification (GRPO/grpo.py:162-198).  Round 1 shipped
-a same-shape Qwen-style encoder that could never host the real weights
-(VERDICT missing #4); this module implements the actual architecture —
+AutoModelForSequenceClassification (GRPO/grpo.py:162-198).
+This module implements that architecture —
 disentangled attention with log-bucketed relative positions (c2p + p2c,
 shared q/k projections for the position embeddings), LayerNorm/GELU
 encoder, context pooler + classifier head — and imports real HF

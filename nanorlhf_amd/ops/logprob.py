@@ -6,10 +6,9 @@ Design: never materialize log-softmax.  The caller supplies hidden states
 and the lm_head weight; we chunk rows, run the plain GEMM (rocBLAS/hipBLASLt
 — a library GEMM, per the MI355X design rules), then a hand-written HIP
 row-reduction computes logprob-of-label + entropy + logsumexp in one pass
-with fp32 accumulation (bf16 logits over 151k vocab need fp32 lse — SURVEY
-§7 hard part (c)).  Backward recomputes each chunk's logits and forms
-dlogits = g * (softmax - onehot) in-kernel, then chunk GEMMs for
-dhidden / dweight.  Peak extra memory = one chunk of logits.
+with fp32 accumulation (bf16 logits over 151k vocab need fp32 lse).
+Backward recomputes each chunk's logits and forms dlogits =
+g * (softmax - onehot) in-kernel, then chunk GEMMs for dhidden / dweight.  Peak extra memory = one chunk of logits.
 
 Reference quirk preserved: scoring divides logits by (temperature + 1e-7)
 (grpo_trainer.py:547) — pass `temperature` for that behavior.

@@ -5,7 +5,7 @@ MI355X-native replacement for accelerate's DDP wrap (grpo_trainer.py:314).
 xGMI is 7 point-to-point links (~153 GB/s each) per GPU, so ring collectives
 are per-link bound: buckets are sized LARGE (default 64 MiB) so RCCL's
 multi-channel rings keep all links busy, and reduction runs on a side
-stream concurrent with the remaining backward (SURVEY.md §2.3 xGMI note).
+stream concurrent with the remaining backward.
 Gradient volume in the LoRA configs is small (adapters + embed/lm_head),
 so overlap makes DP cost near-zero.
 """

@@ -1,6 +1,6 @@
 """Distributed runtime: one process per GPU, RCCL over xGMI.
 
-Replaces the reference's implicit accelerate layer (SURVEY.md §2.3).
+Replaces the reference's implicit accelerate layer.
 Backend "nccl" IS RCCL on ROCm; CPU tests use gloo.  Collectives used:
 broadcast (run timestamp sync, grpo_trainer.py:241-242), all_reduce/
 all_gather for metrics (:729-740), and the gradient all-reduce of ddp.py.

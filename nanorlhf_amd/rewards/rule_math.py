@@ -4,7 +4,7 @@ MathRuleReward: boxed-answer correctness against a gold-answer map
 (reference r1 reward_func, examples/r1-v0/grpo_r1.py:250-273: +1 correct,
 0 otherwise, each equivalence check under a subprocess timeout).
 
-constant_reward: the BASELINE config-#1 plumbing reward (always 1.0)."""
+constant_reward: the reward of a plumbing run, always 1.0."""
 from __future__ import annotations
 
 import torch

@@ -1,5 +1,5 @@
-"""trl/transformers-compatible checkpoint layout (a BASELINE.json
-requirement; reference behavior at GRPO/grpo_trainer.py:321-404).
+"""trl/transformers-compatible checkpoint layout (reference
+behavior at GRPO/grpo_trainer.py:321-404).
 
 Layout per save:
   output_dir/checkpoint-{global_step}/

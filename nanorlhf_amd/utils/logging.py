@@ -1,6 +1,6 @@
 """Metrics logging: console + JSONL file + optional wandb.
 
-Keeps the reference's stable metric names (SURVEY.md §5: objective/kl_old,
+Keeps the reference's stable metric names (objective/kl_old,
 objective/entropy_old, eval_objective/rlhf_reward_old, policy/approxkl_avg_new,
 policy/clipfrac_avg_new, loss/policy_avg_new, policy/entropy_avg_new,
 val/ratio_new, val/ratio_var_new, val/num_eos_tokens_old, lr, episode; PPO

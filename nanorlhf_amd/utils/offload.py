@@ -10,7 +10,7 @@ no-op; for 7B+ configs (or user-forced), transfers use pinned host buffers
 + hipMemcpyAsync on a dedicated side stream so the copy overlaps compute
 (`torch.cuda.Stream` → HIP stream on ROCm).
 
-Stream-ordering contract (the round-1 race fix):
+Stream-ordering contract:
   * device→host: the side stream first WAITS on the compute stream (pending
     kernels that write the tensors must land before the copy reads them),
     and each source GPU tensor is `record_stream`ed on the side stream so

@@ -1,6 +1,6 @@
 """Phase timers + HBM high-water tracking — a real observability subsystem
 (the reference only had a per-update `s/episode` print and commented-out
-memory hooks, SURVEY.md §5 "Tracing / profiling")."""
+memory hooks)."""
 from __future__ import annotations
 
 import time
